@@ -480,6 +480,58 @@ def test_sample_respects_filters_statistically():
         assert probs[3, tok[3]] >= 0.2 * sp[3, 0] - 1e-7
 
 
+@pytest.mark.parametrize("V,dtype,spread,offset", [
+    (1, torch.float32, 2.0, 0), (2, torch.bfloat16, 2.0, 1), (7, torch.float16, 2.0, 3),
+    (1023, torch.float32, 2.0, 1), (4097, torch.bfloat16, 0.0, 0),           # more equal weights than the list holds
+    (50257, torch.bfloat16, 2.5, 1), (50257, torch.float32, 0.02, 2),        # misaligned rows; bins cut twice and three times
+    (128256, torch.bfloat16, 0.3, 0), (151936, torch.float32, 30.0, 0)])
+def test_sample_draws_inside_the_interval_of_the_kept_distribution(V, dtype, spread, offset):
+    """The drawn entry's stretch of the descending cumulative distribution (64-bit) holds ``u`` times the kept mass.
+    A weight's relative error is under 1e-5 (an fp32 exponent of at most a hundred, rounded) and the filter's border
+    may move by one entry."""
+    B = 40
+    logits = (_rand(B, V + offset, dtype=torch.float32, scale=spread) + 0.0).to(dtype)[:, offset:]
+    masked = torch.rand(B, V, device=DEV) < 0.3
+    masked[:, V // 2] = False
+    masked[B // 2:] = False
+    logits = logits.masked_fill(masked, float("-inf")) if offset != 1 else logits     # (the fill packs the rows again)
+    i = torch.arange(B, device=DEV)
+    temperature = torch.where(i % 8 == 7, 0.0, 0.4 + 1.5 * torch.rand(B, device=DEV))
+    top_k = torch.where(i % 3 == 0, 50, torch.where(i % 3 == 1, 0, int(0.7 * V) + 1)).to(torch.int32)
+    top_p = torch.where(i % 4 == 0, 1.0, torch.where(i % 4 == 1, 0.3, 0.95)).float()
+    min_p = torch.where(i % 5 == 0, 0.05, 0.0).float()
+    u = torch.rand(B, device=DEV).clamp(1e-6, 1 - 1e-6)
+    got = ops.sample(logits, temperature, top_k, top_p, min_p, u).long()
+    greedy = temperature == 0
+    assert torch.equal(got[greedy], logits[greedy].float().argmax(-1))
+    p = torch.softmax(logits.double() / torch.where(greedy, 1.0, temperature).double().unsqueeze(1), -1)
+    sp, si = p.sort(dim=-1, descending=True, stable=True)
+    cum = sp.cumsum(-1)
+    keep = torch.arange(V, device=DEV).unsqueeze(0) < torch.where(top_k <= 0, V, top_k).unsqueeze(1)
+    keep &= ((cum - sp) < top_p.double().unsqueeze(1)) | (top_p >= 1).unsqueeze(1)
+    keep &= sp >= min_p.double().unsqueeze(1) * sp[:, :1]
+    keep[:, 0] = True
+    kept = keep.sum(-1)
+    total = cum.gather(1, (kept - 1).unsqueeze(1)).squeeze(1)
+    border = torch.where(kept < V, sp.gather(1, (kept - 1).unsqueeze(1)).squeeze(1), 0.0)
+    rank = (si == got.unsqueeze(1)).to(torch.int8).argmax(-1)
+    hi = cum.gather(1, rank.unsqueeze(1)).squeeze(1)
+    lo = hi - sp.gather(1, rank.unsqueeze(1)).squeeze(1)
+    slack, target = 1e-5 + border, u.double() * total
+    ok = (target >= lo - slack) & (target <= hi + slack) & (rank <= kept)
+    assert (ok | greedy).all(), (got[~ok].tolist(), rank[~ok].tolist(), kept[~ok].tolist())
+
+
+def test_sample_of_rows_without_a_distribution_is_entry_zero():
+    """Rows of nothing but minus infinity, with a NaN or with an infinity: token 0, no hang, neighbours unharmed."""
+    logits = _rand(4, 5000, dtype=torch.float32, scale=2.0)
+    logits[0], logits[1, 77], logits[2, 4999] = float("-inf"), float("nan"), float("inf")
+    one, k = torch.ones(4, device=DEV), torch.zeros(4, device=DEV, dtype=torch.int32)
+    got = ops.sample(logits, one, k, one, 0 * one, 0.5 * one).tolist()
+    assert got[:3] == [0, 0, 0]
+    assert got[3] == torch_ref.sample(logits[3:], one[3:], k[3:], one[3:], 0 * one[3:], 0.5 * one[3:]).item()
+
+
 @pytest.mark.parametrize("sp", ["0", "force"])
 def test_microbatch_overlap_path_matches_plain_decode(monkeypatch, sp):
     """The two-stream micro-batch schedule (forced on at TP=1, where the
