@@ -1,0 +1,891 @@
+// Prompt portions of the recurrent mixers in chunks of 64 rows on the matrix cores, all in 32-bit floats, gfx950:
+//
+//   linear      S <- g S + k v^T ; o = S^T q                            (decayed linear attention, the state-space scan)
+//   delta rule  S <- g S ; u = b (v - S^T k) ; S <- S + k u^T ; o = S^T q
+//
+// per (sequence, head), S [dim, vdim], with a decay g per head, or per head and key channel.  With b_i the product of the
+// chunk's decays up to row i, S_0 the state in front of the chunk and G_ij the product of the decays behind row j up to
+// row i, a chunk is
+//   linear      o_i = (b_i q_i)^T S_0 + sum_(j <= i) A_ij v_j,  A_ij = q_i^T G_ij k_j ;  S = b_64 S_0 + sum_j (G_64,j k_j) v_j^T
+//   delta rule  the same with u for v, where (I + diag(beta) L) u = diag(beta) (v - (b k)^T S_0), L_ij = k_i^T G_ij k_j (j < i):
+//               u = U - W S_0 with U and W, the solutions for beta v and for beta (b k), known without the state
+//
+//   chunk_prep  a workgroup per (chunk, head), all chunks at once: A, b q, G k, U and W (everything without S)
+//   chunk_walk  a workgroup per (sequence, head, 32 value columns): the chunks one after the other, three products each
+//
+// The walk row by row (delta_rule.hip, linear_latent.hip, state_space.hip) is bound by a chain of dependent steps per
+// row; here the chain has a link per 64 rows and the sums are 16x16x4 fp32 matrix instructions (a fused multiply-add per
+// term like the vector unit's: no input is narrowed).  Products of decays are formed directly, never as differences of
+// logarithms: a product between two rows of different groups of 16 is (from the start of i's group up to i) * (whole groups
+// between) * (behind j to the end of its group), each at most 1 where decays are, so nothing overflows; inside a group it
+// is the quotient of two products from the group's start, unless one of those is smaller than 2^-96 or larger than 2^96,
+// where the group's 120 pairs are multiplied out (diag_exact).
+#include "common.h"
+#include <math.h>
+#include <type_traits>
+
+namespace {
+
+constexpr int C = 64;                              // rows of a chunk
+
+enum { LINEAR_HEAD = 0, LINEAR_CHANNEL = 1, STATE_SPACE = 2, DELTA_CHANNEL = 3, DELTA_HEAD = 4 };
+
+struct ChunkArgs {
+  const void* x;                                   // [T, x_stride]: q, k, v of head 0 (group 0) at the three columns
+  long x_stride;
+  int q_off, k_off, v_off;
+  const void* beta;                                // [T, beta_stride], raw (delta rule)
+  long beta_stride;
+  const void* dt;                                  // [T, dt_stride], raw (state space, delta rule)
+  long dt_stride;
+  const float* dt_bias;
+  const float* a_log;
+  const float* decay;                              // [H] (LINEAR_HEAD) or [T, H * dim] (LINEAR_CHANNEL)
+  float* ws;                                       // per (chunk, head of the launch): A | b q | G k, transposed | b_64 | U, transposed | -W
+  long ws_stride;
+  const int* qsl;
+  int B, H, G, dim, vdim, VP;                      // VP: vdim up to a multiple of 32
+  int h0, nh;                                      // the launch's heads
+  int silu, vec, vvec;                             // rows of q, k and the decays / of v can be read 16 bytes at a time
+  float eps;
+};
+
+// What crosses from one kernel to the other lies in pieces of 16x16 as the matrix instruction's operands: 64 lanes of four
+// floats, (lane % 16, 4 (lane / 16) + e) = (row, reduction index) of a left operand, (column, row) of U: a wave's load is one
+// run of 1 KB.  A[4][4] and b q, -W [4][KB] by (rows, reduction); G k, transposed, [KB][4]; U [tiles][4] by (columns, rows).
+struct Layout { int q, kt, bc, u, w, total; };
+__device__ __forceinline__ int piece(int index, int lane) { return (index * 64 + lane) * 4; }
+__host__ __device__ constexpr Layout layout_of(int DP, int VP, bool delta) {
+  Layout l{};
+  l.q = C * C;
+  l.kt = l.q + C * DP;
+  l.bc = l.kt + DP * C;
+  l.u = l.bc + DP;
+  l.w = l.u + VP * C;
+  l.total = l.w + (delta ? C * DP : 0);
+  return l;
+}
+
+template <typename T> __device__ __forceinline__ float ldf(const T* p) { return (float)(*p); }
+__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The product over 16 reduction indices.  Every product here is summed up in such pieces, each from zero, that are then
+// added in turns to two sums: one accumulator running through 192 terms loses twice the digits that the row by row kernels
+// lose (relative error in norm of the delta rule's output against 64 bits 4.1e-7; so 2.2e-7, row by row 2.2e-7).
+__device__ __forceinline__ f32x4 dot16(f32x4 a, f32x4 b) {
+  f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = mfma4(a[e], b[e], c);
+  return c;
+}
+
+// N such products side by side: a matrix instruction of these takes 32 cycles and its result another few, which the others fill
+template <int N> __device__ __forceinline__ void dots16(const f32x4* const (&a)[N], const f32x4* const (&b)[N], f32x4 (&c)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int i = 0; i < N; ++i) c[i] = mfma4((*a[i])[e], (*b[i])[e], c[i]);
+}
+
+// p[0 .. 3], `fill` from `left` on
+template <typename T> __device__ __forceinline__ f32x4 ld4(const T* p, int left, float fill) {
+  f32x4 o = {fill, fill, fill, fill};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) if (e < left) o[e] = ldf(p + e);
+  return o;
+}
+
+// one step of a running product over the 16 lanes of a row; lanes without a source multiply by one
+// Sixteen rows of a wave, `cols` values each, on their way into LDS: a row is read by neighbouring lanes, 16 bytes each, whole
+// lines at a time (read as operands, four lanes to a row, every line is asked for again while it is on its way: the kernel then
+// spends 65 % of its time in such stalls of the vector cache).
+template <typename T, int DP> struct RowLoad {
+  static constexpr int N = 16 / (int)sizeof(T), PER = DP / N, ROWS = 64 / PER, NI = 16 / ROWS;
+  typedef T Vec __attribute__((ext_vector_type(N)));
+  Vec v[NI];
+  // rows first .. first + valid - 1 of p exist; lanes past `cols` and rows past `valid` get `fill`
+  __device__ __forceinline__ void fetch(const T* p, long stride, int valid, int cols, float fill) {
+    const int lane = threadIdx.x & 63, j = (lane % PER) * N;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int rr = i * ROWS + lane / PER;
+      if (rr < valid && j < cols) v[i] = *reinterpret_cast<const Vec*>(p + (long)rr * stride + j);
+      else
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[i][e] = (T)fill;
+    }
+  }
+  __device__ __forceinline__ void stash(float* dst, int ld) const {
+    const int lane = threadIdx.x & 63, j = (lane % PER) * N;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      float* d = dst + (i * ROWS + lane / PER) * ld + j;
+#pragma unroll
+      for (int e = 0; e < N; e += 4)
+        *reinterpret_cast<f32x4*>(d + e) = f32x4{(float)v[i][e], (float)v[i][e + 1], (float)v[i][e + 2], (float)v[i][e + 3]};
+    }
+  }
+};
+// between one wave's LDS writes and its other lanes' reads of them (a wave's LDS accesses are carried out in order)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int CTRL> __device__ __forceinline__ float dpp_mul(float v) {
+  return v * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float prefix_product(float v) {       // lanes up to and including this one
+  v = dpp_mul<0x111>(v);
+  v = dpp_mul<0x112>(v);
+  v = dpp_mul<0x114>(v);
+  return dpp_mul<0x118>(v);
+}
+__device__ __forceinline__ float suffix_product(float v) {       // lanes behind this one
+  v = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), 0x101, 0xf, 0xf, false));
+  v = dpp_mul<0x101>(v);
+  v = dpp_mul<0x102>(v);
+  v = dpp_mul<0x104>(v);
+  return dpp_mul<0x108>(v);
+}
+
+__device__ __forceinline__ int chunks_of(const int* qsl, int B, int s) {
+  const int n = s < B ? qsl[s + 1] - qsl[s] : 0;
+  return n > 0 ? (n + C - 1) / C : 0;
+}
+
+// the sequence and its chunk that the batch's chunk `want` is (false: there are fewer); a wave's work
+__device__ __forceinline__ bool locate(const int* qsl, int B, int want, int& seq, int& c) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int s0 = 0; s0 < B; s0 += 64) {
+    const int cnt = chunks_of(qsl, B, s0 + lane);
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
+    const unsigned long long past = __ballot(base + incl > want);
+    if (past) {
+      const int l = __ffsll(past) - 1;
+      seq = s0 + l;
+      c = want - base - (__shfl(incl, l, 64) - __shfl(cnt, l, 64));
+      return true;
+    }
+    base += __shfl(incl, 63, 64);
+  }
+  return false;
+}
+
+__device__ __forceinline__ int chunks_before(const int* qsl, int B, int seq) {
+  const int lane = threadIdx.x & 63;
+  int sum = 0;
+  for (int s0 = 0; s0 < seq; s0 += 64) sum += s0 + lane < seq ? chunks_of(qsl, B, s0 + lane) : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  return sum;
+}
+
+// the sequence that is place `rank` of the batch by length, longest first (up to 64 sequences; beyond, in their order): what is
+// started first is what takes longest
+__device__ __forceinline__ int by_length(const int* qsl, int B, int rank) {
+  if (B > 64) return rank;
+  const int lane = threadIdx.x & 63, n = lane < B ? qsl[lane + 1] - qsl[lane] : -1;
+  int place = 0;
+  for (int o = 0; o < B; ++o) {
+    const int other = __shfl(n, o, 64);
+    place += other > n || (other == n && o < lane);
+  }
+  return __ffsll(__ballot(lane < B && place == rank)) - 1;
+}
+
+// grid (bound on the batch's chunks, heads of the launch), 4 waves; wave w has rows 16 w .. 16 w + 15 of the chunk: lane (kh =
+// lane / 16, lane % 16) holds channels 16 kb + 4 kh + e of row lane % 16 in registers, which is at once the left operand
+// (row, reduction index 4 kh + e) and the right one of the matrix instruction and the lane layout of the products
+// over rows (DPP).  Only G k and, in the solve, M and beta b k cross waves, through LDS.
+// Bound by what it writes (112 KB per chunk and head, the delta rule 144: linear attention's 6007 rows x 16 heads, 170 MB,
+// in 74 us) and, with a decay per channel under the delta rule, by their exponentials (200 us for 8017 rows x 16 heads).
+template <typename T, int KIND, int DP>
+__global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
+  constexpr bool DELTA = KIND >= DELTA_CHANNEL, CHAN = KIND == LINEAR_CHANNEL || KIND == DELTA_CHANNEL;
+  constexpr int KB = DP / 16, NP = CHAN ? KB * 4 : 1, LD = DP + 4, LM = C + 4;
+  constexpr Layout L0 = layout_of(DP, 0, false);
+  __shared__ __attribute__((aligned(16))) float ks[C * LD];
+  __shared__ __attribute__((aligned(16))) float tl[CHAN ? 4 * DP : 4];
+  __shared__ __attribute__((aligned(16))) float mn[DELTA ? C * LM : 4];      // -beta L
+  __shared__ __attribute__((aligned(16))) float ti[DELTA ? 4 * 16 * 20 : 4]; // inverses of the diagonal blocks
+  __shared__ float bl[C];
+  __shared__ double td[4];
+  int seq, c;
+  if (!locate(a.qsl, a.B, blockIdx.x, seq, c)) return;           // (the same for every wave)
+  const int hh = blockIdx.y, h = a.h0 + hh, g = h / (a.H / a.G);
+  const int q0 = a.qsl[seq], n = a.qsl[seq + 1] - q0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;
+  const int r = 16 * wave + lr;
+  const bool ok = c * C + r < n;
+  const long row = q0 + (ok ? c * C + r : 0);
+  const T* xr = (const T*)a.x + row * a.x_stride;
+  float* ws = a.ws + ((long)hh * gridDim.x + blockIdx.x) * a.ws_stride;   // (a head's chunks side by side: the walk stays in a page)
+
+  // ---- the wave's rows: q, k, the decays
+  f32x4 q[KB], k[KB], dk[CHAN ? KB : 1];           // dk: the row's decays (raw dt for the delta rule, until below)
+  float p[NP], s[NP];
+  const int valid = min(16, n - (c * C + 16 * wave));            // rows of the wave that exist (none: <= 0)
+  const long row0 = q0 + c * C + 16 * wave;
+  float* mine = ks + 16 * wave * LD;               // the wave's rows of ks, free until it writes G k there
+  const float* fr = mine + lr * LD + 4 * kh;
+  if (a.vec) {
+    RowLoad<T, DP> lq, lk;
+    lq.fetch((const T*)a.x + row0 * a.x_stride + a.q_off + (long)g * a.dim, a.x_stride, valid, a.dim, 0.f);
+    lk.fetch((const T*)a.x + row0 * a.x_stride + a.k_off + (long)g * a.dim, a.x_stride, valid, a.dim, 0.f);
+    using D = std::conditional_t<KIND == LINEAR_CHANNEL, float, T>;
+    RowLoad<D, DP> ld;
+    if constexpr (KIND == LINEAR_CHANNEL)
+      ld.fetch(a.decay + (row0 * a.H + h) * (long)a.dim, (long)a.H * a.dim, valid, a.dim, 1.f);
+    else if constexpr (KIND == DELTA_CHANNEL)
+      ld.fetch((const T*)a.dt + row0 * a.dt_stride + (long)h * a.dim, a.dt_stride, valid, a.dim, 0.f);
+    lq.stash(mine, LD);
+    wave_sync();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) q[kb] = *reinterpret_cast<const f32x4*>(fr + 16 * kb);
+    wave_sync();
+    lk.stash(mine, LD);
+    wave_sync();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) k[kb] = *reinterpret_cast<const f32x4*>(fr + 16 * kb);
+    if constexpr (CHAN) {
+      wave_sync();
+      ld.stash(mine, LD);
+      wave_sync();
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) dk[kb] = *reinterpret_cast<const f32x4*>(fr + 16 * kb);
+    }
+    wave_sync();
+  } else {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int j = 16 * kb + 4 * kh, left = ok ? a.dim - j : 0;
+      q[kb] = ld4(xr + a.q_off + (long)g * a.dim + j, left, 0.f);
+      k[kb] = ld4(xr + a.k_off + (long)g * a.dim + j, left, 0.f);
+      if constexpr (KIND == LINEAR_CHANNEL) dk[kb] = ld4(a.decay + (row * a.H + h) * (long)a.dim + j, left, 1.f);
+      if constexpr (KIND == DELTA_CHANNEL) dk[kb] = ld4((const T*)a.dt + row * a.dt_stride + (long)h * a.dim + j, left, 0.f);
+    }
+  }
+  if (a.silu) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { q[kb][e] *= sigmoid_f(q[kb][e]); k[kb][e] *= sigmoid_f(k[kb][e]); }
+  }
+  if constexpr (KIND == DELTA_CHANNEL) {
+    const float rate = expf(a.a_log[h]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = 16 * kb + 4 * kh + e;
+        dk[kb][e] = ok && j < a.dim ? expf(-rate * softplus_f(dk[kb][e] + a.dt_bias[h * a.dim + j])) : 1.f;
+      }
+  }
+  if constexpr (DELTA) {
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { sq += q[kb][e] * q[kb][e]; sk += k[kb][e] * k[kb][e]; }
+    sq += __shfl_xor(sq, 16, 64); sk += __shfl_xor(sk, 16, 64);
+    sq += __shfl_xor(sq, 32, 64); sk += __shfl_xor(sk, 32, 64);
+    const float iq = 1.0f / sqrtf(sq + a.eps) * (1.0f / sqrtf((float)a.dim)), ik = 1.0f / sqrtf(sk + a.eps);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { q[kb][e] *= iq; k[kb][e] *= ik; }
+    if (kh == 0) bl[r] = ok ? sigmoid_f(ldf((const T*)a.beta + row * a.beta_stride + h)) : 0.f;
+  }
+  float own = 1.f;                                 // per head: the row's decay,
+  double pd = 1.0;                                 // the product of the group's up to the row
+  if constexpr (CHAN) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { p[4 * kb + e] = prefix_product(dk[kb][e]); s[4 * kb + e] = suffix_product(dk[kb][e]); }
+    }
+  } else {
+    if (ok) {
+      if constexpr (KIND == LINEAR_HEAD) own = a.decay[h];
+      else {
+        const float step = softplus_f(ldf((const T*)a.dt + row * a.dt_stride + h) + a.dt_bias[h]);
+        own = expf(-expf(a.a_log[h]) * step);
+        if constexpr (KIND == STATE_SPACE) {
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb) k[kb] *= step;
+        }
+      }
+    }
+    // (a head's decay can be the same number in every row: rounded products of it would be off by the same amount in every
+    // chunk.  They are formed in 64 bits and rounded once)
+    double after = __shfl_down((double)own, 1, 16);
+    if (lr == 15) after = 1.0;
+    pd = own;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      const double before = __shfl_up(pd, o, 16), behind = __shfl_down(after, o, 16);
+      if (lr >= o) pd *= before;
+      if (lr + o < 16) after *= behind;
+    }
+    p[0] = (float)pd;
+    s[0] = (float)after;
+    if (lane == 15) td[wave] = pd;
+  }
+  bool far = false;                                // a product too small or too large to divide by
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    far = far || !(fabsf(p[i]) >= 0x1p-96f && fabsf(p[i]) <= 0x1p96f);
+  }
+  if (lr == 15) {
+    if constexpr (CHAN) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        *reinterpret_cast<f32x4*>(tl + wave * DP + 16 * kb + 4 * kh) = f32x4{p[4 * kb], p[4 * kb + 1], p[4 * kb + 2], p[4 * kb + 3]};
+    }
+  }
+  auto P = [&](int kb, int e) { return p[CHAN ? 4 * kb + e : 0]; };
+  auto Q = [&](int kb, int e) { return s[CHAN ? 4 * kb + e : 0]; };
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k[kb][e] * Q(kb, e);
+    *reinterpret_cast<f32x4*>(ks + r * LD + 16 * kb + 4 * kh) = v;
+  }
+  __syncthreads();
+  // G k up to the chunk's end, transposed: the wave's rows, a piece per 16 channels
+  {
+    double behind = 1.0;
+    if constexpr (!CHAN)
+      for (int b = wave + 1; b < 4; ++b) behind *= td[b];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      float after = 1.f;
+      if constexpr (CHAN)
+        for (int b = wave + 1; b < 4; ++b) after *= tl[b * DP + 16 * kb + lr];
+      else
+        after = (float)behind;
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = ks[(16 * wave + 4 * kh + e) * LD + 16 * kb + lr] * after;
+      *reinterpret_cast<f32x4*>(ws + L0.kt + piece(kb * 4 + wave, lane)) = v;
+    }
+    if ((int)threadIdx.x < DP) {
+      const int j = threadIdx.x;
+      ws[L0.bc + j] = CHAN ? tl[j] * tl[DP + j] * tl[2 * DP + j] * tl[3 * DP + j] : (float)(td[0] * td[1] * td[2] * td[3]);
+    }
+  }
+  // ---- A = q G k and (delta) L = k G k, lower triangles: the wave's rows against the column blocks 0 .. wave
+  const bool exact_diag = __any(far);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 da = zero, dl = zero;
+  if (!exact_diag) {
+    f32x4 sa[2] = {zero, zero}, sb[2] = {zero, zero};
+    const float over = (float)(1.0 / pd);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      f32x4 kd, qp, kp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kd[e] = CHAN ? k[kb][e] / P(kb, e) : k[kb][e] * over;
+        qp[e] = q[kb][e] * P(kb, e);
+        kp[e] = k[kb][e] * P(kb, e);
+      }
+      sa[kb & 1] += dot16(qp, kd);
+      if constexpr (DELTA) sb[kb & 1] += dot16(kp, kd);
+      if constexpr (CHAN) { q[kb] = qp; k[kb] = kp; }
+    }
+    da = sa[0] + sa[1];
+    dl = sb[0] + sb[1];
+  } else {
+    // diag_exact: pairs (i, i - m) of the wave's group; the product of the decays between them grows with m
+    float between[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) between[i] = 1.f;
+    for (int m = 0; m < 16; ++m) {
+      const int src = (lane & 48) | ((lr - m) & 15);
+      float sa = 0.f, sb = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        [[maybe_unused]] const f32x4 d = dk[CHAN ? kb : 0];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float kj = __shfl(k[kb][e], src, 64) * between[CHAN ? 4 * kb + e : 0];
+          sa += q[kb][e] * kj;
+          if constexpr (DELTA) sb += k[kb][e] * kj;
+          if constexpr (CHAN) between[4 * kb + e] *= __shfl(d[e], src, 64);
+        }
+      }
+      if constexpr (!CHAN) between[0] *= __shfl(own, src, 64);
+      sa += __shfl_xor(sa, 16, 64); sa += __shfl_xor(sa, 32, 64);
+      sb += __shfl_xor(sb, 16, 64); sb += __shfl_xor(sb, 32, 64);
+      // lane (.., i) has the sum of row i, column i - m; as an accumulator, lane (kh, j) has rows 4 kh + e of column j
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float va = __shfl(sa, 4 * kh + e, 64), vb = __shfl(sb, 4 * kh + e, 64);
+        if (4 * kh + e - m == lr) { da[e] = va; dl[e] = vb; }
+      }
+    }
+    if constexpr (CHAN)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { q[kb][e] *= P(kb, e); k[kb][e] *= P(kb, e); }
+  }
+  // (blocks to the left, nearest first: after each of them its whole product joins the left operands, which end as b q and b k)
+  for (int J = wave - 1; J >= 0; --J) {
+    f32x4 sa[2] = {zero, zero}, sb[2] = {zero, zero};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(ks + (16 * J + lr) * LD + 16 * kb + 4 * kh);
+      sa[kb & 1] += dot16(CHAN ? q[kb] : q[kb] * (float)pd, b);
+      if constexpr (DELTA) sb[kb & 1] += dot16(CHAN ? k[kb] : k[kb] * (float)pd, b);
+      if constexpr (CHAN) {
+        const f32x4 t = *reinterpret_cast<const f32x4*>(tl + J * DP + 16 * kb + 4 * kh);
+        q[kb] *= t;
+        k[kb] *= t;
+      }
+    }
+    if constexpr (!CHAN) pd *= td[J];
+    const f32x4 va = sa[0] + sa[1], vl = sb[0] + sb[1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * wave + 4 * kh + e;
+      ws[piece(wave * 4 + J, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = va[e];
+      if constexpr (DELTA) mn[i * LM + 16 * J + lr] = -bl[i] * vl[e];
+    }
+  }
+  if constexpr (!CHAN)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) { q[kb] *= (float)pd; k[kb] *= (float)pd; }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int i = 4 * kh + e;
+    ws[piece(wave * 5, (lr >> 2) * 16 + i) + (lr & 3)] = lr <= i ? da[e] : 0.f;
+    if constexpr (DELTA) mn[(16 * wave + i) * LM + 16 * wave + lr] = lr < i ? -bl[16 * wave + i] * dl[e] : 0.f;
+  }
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) *reinterpret_cast<f32x4*>(ws + L0.q + piece(wave * KB + kb, lane)) = q[kb];
+
+  const int vt = a.VP / 16;
+  const T* xv = (const T*)a.x + row0 * a.x_stride + a.v_off + (long)h * a.vdim;
+  // columns v0 .. v0 + DP - 1 of the wave's rows of v into its rows of ks
+  auto values = [&](int v0) {
+    if (a.vvec) {
+      RowLoad<T, DP> lv;
+      lv.fetch(xv + v0, a.x_stride, valid, a.vdim - v0, 0.f);
+      lv.stash(mine, LD);
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const int j = 16 * kb + 4 * kh;
+        *reinterpret_cast<f32x4*>(mine + lr * LD + j) = ld4(xv + (long)lr * a.x_stride + v0 + j, lr < valid ? a.vdim - v0 - j : 0, 0.f);
+      }
+    }
+  };
+  if constexpr (!DELTA) {
+    __syncthreads();                               // G k has been read
+    for (int t0 = 0; t0 < vt; t0 += KB) {
+      values(16 * t0);
+      wave_sync();
+#pragma unroll
+      for (int t = 0; t < KB; ++t)
+        if (t0 + t < vt) {
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = mine[(4 * kh + e) * LD + 16 * t + lr];
+            if (a.silu) v[e] *= sigmoid_f(v[e]);
+          }
+          *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 + t) * 4 + wave, lane)) = v;
+        }
+      wave_sync();
+    }
+  } else {
+    __syncthreads();                               // G k has been read, M is there
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) *reinterpret_cast<f32x4*>(ks + r * LD + 16 * kb + 4 * kh) = k[kb];
+    // (I - Mn)^-1 of the wave's diagonal block: lane lr a column, row by row
+    {
+      float t[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float* m = mn + (16 * wave + i) * LM + 16 * wave;
+        float v = i == lr ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < i; ++j) v += m[j] * t[j];
+        t[i] = v;
+      }
+      if (kh == 0)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ti[(16 * wave + i) * 20 + lr] = t[i];
+    }
+    __syncthreads();
+    // columns of [beta b k | beta v], 16 at a time; an accumulator's layout is the right operand's: solved blocks stay in registers
+    float* wp = ws + L0.u + a.VP * C;
+    for (int t0 = 0; t0 < KB + vt; t0 += KB) {
+      const bool keys = t0 == 0;
+      if (!keys) {
+        __syncthreads();                           // the other waves have read the previous columns
+        values(16 * (t0 - KB));
+        __syncthreads();
+      }
+      for (int t = wave; t < KB && t0 + t < KB + vt; t += 4) {
+        f32x4 X[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+          f32x4 acc;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 16 * I + 4 * kh + e;
+            acc[e] = ks[i * LD + 16 * t + lr] * bl[i];
+          }
+#pragma unroll
+          for (int J = 0; J < I; ++J)
+            acc += dot16(*reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh), X[J]);
+          X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
+          if (keys) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wp[piece(I * KB + t, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = -X[I][e];
+          } else {
+            *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 - KB + t) * 4 + I, lane)) = X[I];
+          }
+        }
+      }
+    }
+  }
+}
+
+// grid: (sequence, head) pairs x tiles of 32 value columns, the tiles of a pair on one die (workgroups go round the dies by
+// their index: they share what chunk_prep left in its L2), long sequences first.  Eight waves: 0 .. 3 keep rows
+// w * DP / 4 .. of the state tile as accumulators and carry it from chunk to chunk, 4 .. 7 form the output of 16 rows of the
+// chunk each, so that two waves per SIMD fill each other's waits.  Per chunk
+//   state waves    (delta rule) u = U - W S, S of the whole tile from LDS ;  S = b_64 S + (G k)^T u
+//   output waves   o = (b q) S + A u
+// with two barriers (S is there, u is there), linear kinds with one (u = v comes from memory).  Left operands come from
+// memory straight into registers, where the next chunk's take the place of those just used.
+// Bound by a chunk's matrix instructions (1.1 us of linear kinds, 1.5 of the delta rule, at 16 columns) and by its 90 - 115 KB
+// of operands, which come through the vector cache at 64 bytes a clock (0.6 - 0.8 us) whatever the tile's width; the two hardly
+// overlap, as all waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.5 us at 16 columns, 4.0 / 5.0 at
+// 32: narrow tiles where there are few workgroups (one prompt of 8000 rows, 16 heads, dim 128: 420 against 590 us), wide ones
+// where every compute unit has one anyway (five prompts, 8017 rows: 256 against 306 us).
+template <int DP, bool DELTA, int NC> struct Walk {
+  static constexpr int KB = DP / 16, NT = DP / 64, LD = DP + 4, LU = C + 4;
+  static constexpr Layout L0 = layout_of(DP, 0, false);
+  struct Shared {
+    __attribute__((aligned(16))) float sl[DELTA ? 1 : 2][16 * NC * LD];
+    __attribute__((aligned(16))) float ul[DELTA ? 16 * NC * LU : 4];
+  };
+  static __device__ __forceinline__ f32x4 at(const float* p, int offset) { return *reinterpret_cast<const f32x4*>(p + offset); }
+
+  const float* ws;                                 // the pair's first chunk
+  long step;
+  int nc, VP, tile, wave, lane, lr, kh;
+  Shared& sh;
+
+  // (chunks past the last are read as the last one: loads without a condition keep the waits for them exact)
+  __device__ __forceinline__ const float* chunk_at(int c) const { return ws + step * min(c, nc - 1); }
+  __device__ __forceinline__ f32x4 left(const float* p, int offset, int index) const { return at(p, offset + piece(index, lane)); }
+
+  struct StateOps { f32x4 w[DELTA ? KB : 1], k[NT][4], u[DELTA ? 1 : 4][NC], b[NT]; };
+  struct OutOps { f32x4 q[KB], a[4], u[DELTA ? 1 : 4][NC]; };
+
+  __device__ __forceinline__ void load_first(StateOps& r, int c) const {
+    const float* p = chunk_at(c);
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) r.w[kb] = left(p, L0.u + VP * C, wave * KB + kb);
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) r.u[0][ct] = left(p, L0.u, (NC * tile + ct) * 4 + wave);
+    }
+    __builtin_amdgcn_sched_barrier(0);             // (the loads stay where they are put)
+  }
+  template <typename Ops> __device__ __forceinline__ void load_values(Ops& r, const float* p) const {
+    if constexpr (!DELTA)
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) r.u[kb][ct] = left(p, L0.u, (NC * tile + ct) * 4 + kb);
+  }
+  __device__ __forceinline__ void load_second(StateOps& r, int c) const {
+    const float* p = chunk_at(c);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) r.k[t][kb] = left(p, L0.kt, (wave * NT + t) * 4 + kb);
+      r.b[t] = at(p, L0.bc + (wave * NT + t) * 16 + 4 * kh);
+    }
+    load_values(r, p);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void load_first(OutOps& r, int c) const {
+    const float* p = chunk_at(c);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) r.q[kb] = left(p, L0.q, wave * KB + kb);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void load_second(OutOps& r, int c) const {
+    const float* p = chunk_at(c);
+    // (the blocks right of the diagonal are never written: they are read, so that the loads carry no condition, and not used)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) r.a[kb] = left(p, 0, wave * 4 + kb);
+    load_values(r, p);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // o[ct][0 / 1] += the products of left operands l[0 .. 3] with right ones x[0 .. 3][ct], four chains of instructions side by side
+  static __device__ __forceinline__ void four(const f32x4* l, const f32x4 (&x)[4][NC], f32x4 (&o)[NC][2]) {
+    if constexpr (NC == 1) {
+      f32x4 d[4];
+      dots16<4>({&l[0], &l[1], &l[2], &l[3]}, {&x[0][0], &x[1][0], &x[2][0], &x[3][0]}, d);
+      o[0][0] += d[0] + d[1];
+      o[0][1] += d[2] + d[3];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        f32x4 d[4];
+        dots16<4>({&l[i], &l[i], &l[i + 1], &l[i + 1]}, {&x[i][0], &x[i][1], &x[i + 1][0], &x[i + 1][1]}, d);
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) o[ct][i >> 1] += d[ct] + d[2 + ct];
+      }
+    }
+  }
+  // reduction blocks kb .. kb + 3 of a right operand in LDS
+  template <int LDR> __device__ __forceinline__ void read_four(const float* right, int kb, f32x4 (&x)[4][NC]) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) x[i][ct] = at(right, (16 * ct + lr) * LDR + 16 * (kb + i) + 4 * kh);
+  }
+
+  __device__ __forceinline__ void chunk(StateOps& r, int c, f32x4 (&S)[NT][NC]) const {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    float* sl = sh.sl[DELTA ? 0 : c & 1];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct)
+        *reinterpret_cast<f32x4*>(sl + (16 * ct + lr) * LD + (wave * NT + t) * 16 + 4 * kh) = S[t][ct];
+    __syncthreads();
+    f32x4 x[4][NC];
+    if constexpr (DELTA) {
+      f32x4 us[NC][2];
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) { us[ct][0] = r.u[0][ct]; us[ct][1] = zero; }
+#pragma unroll
+      for (int kb = 0; kb < KB; kb += 4) {
+        read_four<LD>(sl, kb, x);
+        four(&r.w[kb], x, us);
+      }
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct)
+        *reinterpret_cast<f32x4*>(sh.ul + (16 * ct + lr) * LU + 16 * wave + 4 * kh) = us[ct][0] + us[ct][1];
+      load_first(r, c + 1);
+      __syncthreads();
+      read_four<LU>(sh.ul, 0, x);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) x[i][ct] = r.u[i][ct];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      f32x4 add[NC][2];
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) add[ct][0] = add[ct][1] = zero;
+      four(r.k[t], x, add);
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) S[t][ct] = S[t][ct] * r.b[t] + (add[ct][0] + add[ct][1]);
+    }
+    load_second(r, c + 1);
+  }
+  // o of the wave's 16 rows; u: those rows of u (linear kinds)
+  __device__ __forceinline__ void chunk(OutOps& r, int c, f32x4 (&o)[NC], f32x4 (&u)[NC]) const {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const float* sl = sh.sl[DELTA ? 0 : c & 1];
+    __syncthreads();
+    f32x4 os[NC][2], x[4][NC];
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) os[ct][0] = os[ct][1] = zero;
+#pragma unroll
+    for (int kb = 0; kb < KB; kb += 4) {
+      read_four<LD>(sl, kb, x);
+      four(&r.q[kb], x, os);
+    }
+    load_first(r, c + 1);
+    if constexpr (DELTA) {
+      __syncthreads();
+      read_four<LU>(sh.ul, 0, x);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) {
+          x[i][ct] = r.u[i][ct];
+          if (i == wave) u[ct] = r.u[i][ct];
+        }
+    }
+    // (the lower triangle's blocks; the wave's number is the same for all its lanes)
+    if (wave == 3) {
+      four(r.a, x, os);
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < 3; ++kb)
+        if (kb <= wave)
+#pragma unroll
+          for (int ct = 0; ct < NC; ++ct) os[ct][kb & 1] += dot16(r.a[kb], x[kb][ct]);
+    }
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) o[ct] = os[ct][0] + os[ct][1];
+    load_second(r, c + 1);
+  }
+};
+
+template <int DP, bool DELTA, int NC>
+__global__ __launch_bounds__(512, 2) void chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ wsp, long ws_stride,
+                                                            float* __restrict__ state, const int* __restrict__ slots,
+                                                            const int* __restrict__ qsl, const int* __restrict__ seq_lens,
+                                                            const float* __restrict__ d_skip, int B, int H, int dim, int vdim,
+                                                            int VP, int h0, int nh, int chunks, float scale) {
+  using W = Walk<DP, DELTA, NC>;
+  __shared__ typename W::Shared shared;
+  const int tiles = VP / (16 * NC);
+  const int id = blockIdx.x, die = id & 7, rest = id >> 3;
+  const int tile = rest % tiles, pair = (rest / tiles) * 8 + die;
+  if (pair >= B * nh) return;
+  const int hh = pair % nh, h = h0 + hh, seq = by_length(qsl, B, pair / nh);
+  const int q0 = qsl[seq], n = qsl[seq + 1] - q0;
+  if (n <= 0) return;
+  const int chunk0 = chunks_before(qsl, B, seq), nc = (n + C - 1) / C;
+  const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  const int lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;
+  const int col = 16 * NC * tile + lr;             // (and col + 16)
+  W w{wsp + ((long)hh * chunks + chunk0) * ws_stride, ws_stride, nc, VP, tile, wave, lane, lr, kh, shared};
+  if (role == 0) {
+    float* st = state + ((long)slots[seq] * H + h) * (long)dim * vdim;
+    const bool fresh = seq_lens[seq] - n <= 0;     // the rows start the sequence: whatever the slot holds is not ours
+    typename W::StateOps r;
+    w.load_first(r, 0);
+    w.load_second(r, 0);
+    f32x4 S[W::NT][NC];
+    auto place = [&](int t, int ct, int e) {        // of S[t][ct][e] in the state, -1: outside
+      const int d = (wave * W::NT + t) * 16 + 4 * kh + e, v = col + 16 * ct;
+      return d < dim && v < vdim ? d * vdim + v : -1;
+    };
+#pragma unroll
+    for (int t = 0; t < W::NT; ++t)
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[t][ct][e] = !fresh && place(t, ct, e) >= 0 ? st[place(t, ct, e)] : 0.f;
+    for (int c = 0; c < nc; ++c) w.chunk(r, c, S);
+#pragma unroll
+    for (int t = 0; t < W::NT; ++t)
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (place(t, ct, e) >= 0) st[place(t, ct, e)] = S[t][ct][e];
+  } else {
+    const float skip = d_skip != nullptr ? d_skip[h] : 0.f;
+    typename W::OutOps r;
+    w.load_first(r, 0);
+    w.load_second(r, 0);
+    for (int c = 0; c < nc; ++c) {
+      f32x4 o[NC], u[NC] = {};
+      w.chunk(r, c, o, u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = c * C + 16 * wave + 4 * kh + e;
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+          if (i < n && col + 16 * ct < vdim)
+            out[((long)(q0 + i) * H + h) * vdim + col + 16 * ct] = DELTA ? o[ct][e] * scale : o[ct][e] * scale + skip * u[ct][e];
+      }
+    }
+  }
+}
+
+template <typename T, int KIND>
+int launch(const ChunkArgs& a, int chunks, float* out, float* state, const int* slots, const int* seq_lens, const float* d_skip,
+           float scale, hipStream_t stream) {
+  constexpr bool DELTA = KIND >= DELTA_CHANNEL;
+  const dim3 prep(chunks, a.nh);
+  const long pairs = ((long)a.B * a.nh + 7) / 8 * 8;
+  // 32 columns per workgroup where that still leaves one for every compute unit
+  const int cols = pairs * (a.VP / 32) >= 256 ? 32 : 16;
+  const dim3 walk((unsigned)(pairs * (a.VP / cols)));
+#define WALK(DP_, NC_)                                                                                                       \
+  hipLaunchKernelGGL((chunk_walk_kernel<DP_, DELTA, NC_>), walk, dim3(512), 0, stream, out, a.ws, a.ws_stride, state, slots, \
+                     a.qsl, seq_lens, d_skip, a.B, a.H, a.dim, a.vdim, a.VP, a.h0, a.nh, chunks, scale)
+#define GO(DP_)                                                                                                            \
+  do {                                                                                                                     \
+    hipLaunchKernelGGL((chunk_prep_kernel<T, KIND, DP_>), prep, dim3(256), 0, stream, a);                                  \
+    if (cols == 32) WALK(DP_, 2);                                                                                          \
+    else WALK(DP_, 1);                                                                                                     \
+  } while (0)
+  if (a.dim <= 64) GO(64);
+  else GO(128);
+#undef GO
+#undef WALK
+  HIP_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace
+
+// floats of workspace per chunk and head
+VDAMD_API long vdamd_chunk_scan_floats(int kind, int dim, int vdim) {
+  return layout_of(dim <= 64 ? 64 : 128, (vdim + 31) / 32 * 32, kind >= DELTA_CHANNEL).total;
+}
+
+// Heads h0 .. h0 + nh - 1 of one call.  x [T, x_stride] of type dtype with q, k (of group 0) and v (of head 0) at the three
+// columns; dt / beta rows of the same type; out [T, H * vdim] fp32, state [slots, H, dim, vdim] fp32; `chunks`: a bound on the
+// batch's chunks of 64 rows; ws: chunks * nh * vdamd_chunk_scan_floats floats, 16-byte aligned; dim <= 128
+VDAMD_API int vdamd_chunk_scan(float* out, int kind, const void* x, long x_stride, int q_off, int k_off, int v_off,
+                               const void* beta, long beta_stride, const void* dt, long dt_stride, const float* dt_bias,
+                               const float* a_log, const float* decay, const float* d_skip, float* ws, int chunks, float* state,
+                               const int* slots, const int* qsl, const int* seq_lens, int B, int H, int G, int dim, int vdim,
+                               int h0, int nh, int silu, float eps, float scale, int dtype, hipStream_t stream) {
+  if (B <= 0 || chunks <= 0 || nh <= 0) return 0;
+  if (H <= 0 || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || h0 < 0 || h0 + nh > H || nh > 65535) return 1;
+  ChunkArgs a{};
+  a.x = x; a.x_stride = x_stride; a.q_off = q_off; a.k_off = k_off; a.v_off = v_off;
+  a.beta = beta; a.beta_stride = beta_stride; a.dt = dt; a.dt_stride = dt_stride; a.dt_bias = dt_bias; a.a_log = a_log;
+  a.decay = decay; a.ws = ws; a.ws_stride = vdamd_chunk_scan_floats(kind, dim, vdim); a.qsl = qsl;
+  a.B = B; a.H = H; a.G = G; a.dim = dim; a.vdim = vdim; a.VP = (vdim + 31) / 32 * 32; a.h0 = h0; a.nh = nh;
+  a.silu = silu; a.eps = eps;
+  const int per = dtype == DT_F32 ? 4 : 8;         // elements of 16 bytes
+  const bool rows16 = x_stride % per == 0 && (uintptr_t)x % 16 == 0;
+  a.vec = rows16 && dim % per == 0 && q_off % per == 0 && k_off % per == 0 &&
+          (kind != DELTA_CHANNEL || (dt_stride % per == 0 && (uintptr_t)dt % 16 == 0)) &&
+          (kind != LINEAR_CHANNEL || (uintptr_t)decay % 16 == 0);
+  a.vvec = rows16 && vdim % per == 0 && v_off % per == 0;
+#define KINDS(T)                                                                                                         \
+  switch (kind) {                                                                                                        \
+    case LINEAR_HEAD: return launch<T, LINEAR_HEAD>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);       \
+    case LINEAR_CHANNEL: return launch<T, LINEAR_CHANNEL>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream); \
+    case STATE_SPACE: return launch<T, STATE_SPACE>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);       \
+    case DELTA_CHANNEL: return launch<T, DELTA_CHANNEL>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);   \
+    case DELTA_HEAD: return launch<T, DELTA_HEAD>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);         \
+  }
+  switch (dtype) {
+    case DT_BF16: KINDS(bf16_t) break;
+    case DT_F16: KINDS(f16_t) break;
+    case DT_F32: KINDS(float) break;
+  }
+#undef KINDS
+  return 1;
+}

@@ -1,0 +1,151 @@
+"""The chunked kernels of the recurrent mixers (64 rows of a prompt at a time, fp32 matrix instructions) against the
+recurrences run row by row in 64 bits, and their error beside that of the row by row kernels."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from vllm_distributed_amd.ops import hip
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _lib():
+    hip.load()
+
+
+def _case(op, heads, groups, dim, vdim, new, lens, dtype, seed, strong=False, pad=0):
+    """Packed rows of ``new[i]`` rows per sequence; ``strong``: decays down to 1e-30 beside ones next to 1; ``pad``: columns
+    behind the projection (row strides that no vector load divides)."""
+    g = torch.Generator(DEV).manual_seed(seed)
+
+    def normal(*shape, std=1.0):
+        return torch.randn(*shape, generator=g, device=DEV) * std
+    t = sum(new)
+    cols = heads * vdim + 2 * groups * dim
+    c = {"op": op, "heads": heads, "groups": groups, "dim": dim, "vdim": vdim, "new": new, "lens": lens}
+    c["x"] = normal(t, cols + pad).to(dtype)[:, :cols]
+    c["state"] = normal(len(new) + 2, heads, dim, vdim, std=0.3)
+    c["slots"] = torch.randperm(len(new) + 2, generator=g, device=DEV)[:len(new)].to(torch.int32)
+    channels = heads * dim if op == "delta_channel" else heads
+    c["beta"] = normal(t, heads + pad).to(dtype)[:, :heads]
+    c["dt"] = normal(t, channels + pad, std=4.0 if strong else 0.5).to(dtype)[:, :channels]
+    c["dt_bias"] = normal(channels) - (0.0 if strong else 3.0)
+    c["a_log"] = normal(heads, std=0.5) + (1.5 if strong else 0.5)
+    c["skip"] = normal(heads)
+    if op == "linear_channel":
+        z = normal(t, heads * dim, std=3.0)
+        c["decay"] = torch.sigmoid(z) ** 8 if strong else torch.sigmoid(z + 2.0) ** (1.0 / 16.0)
+    else:
+        c["decay"] = torch.rand(heads, generator=g, device=DEV) * (0.9 if not strong else 1e-9) + (0.1 if not strong else 0.0)
+    return c
+
+
+def _run(c, chunked):
+    state = c["state"].clone()
+    qsl = torch.tensor([0] + c["new"]).cumsum(0).to(torch.int32).to(DEV)
+    at = (state, c["slots"], qsl, torch.tensor(c["lens"], dtype=torch.int32, device=DEV))
+    sizes = (c["heads"], c["groups"], c["dim"], c["vdim"])
+    most, op = max(c["new"]), c["op"]
+    if op.startswith("delta"):
+        out = hip.gated_delta_rule(c["x"], *sizes, c["beta"], c["dt"], c["dt_bias"], c["a_log"], *at, 1e-6, most, 0, chunked)
+    elif op == "state_space":
+        out = hip.selective_scan(c["x"], c["dt"], c["heads"], c["groups"], c["vdim"], c["dim"], c["a_log"], c["dt_bias"],
+                                 c["skip"], *at, most, chunked)
+    else:
+        out = hip.decay_linear_attention(c["x"], c["heads"], c["dim"], c["vdim"], c["decay"], *at, op == "linear_head", most,
+                                         0.25 if op == "linear_channel" else 1.0, chunked)
+    return out, state
+
+
+def _rows64(c):
+    h, gr, d, vd, op = c["heads"], c["groups"], c["dim"], c["vdim"], c["op"]
+    xd = c["x"].double()
+    t = xd.shape[0]
+    if op == "state_space":
+        v, k, q = xd.split([h * vd, gr * d, gr * d], -1)
+    else:
+        q, k, v = xd.split([gr * d, gr * d, h * vd], -1)
+    q, k, v = q.reshape(t, gr, d), k.reshape(t, gr, d), v.reshape(t, h, vd)
+    if op.startswith("delta"):
+        q = q * torch.rsqrt(q.pow(2).sum(-1, keepdim=True) + 1e-6) * d ** -0.5
+        k = k * torch.rsqrt(k.pow(2).sum(-1, keepdim=True) + 1e-6)
+    if op == "linear_head":
+        q, k, v = F.silu(q), F.silu(k), F.silu(v)
+    skip = 0.0
+    if op.startswith("delta") or op == "state_space":
+        step = F.softplus(c["dt"].double() + c["dt_bias"].double(), threshold=60.0).reshape(t, h, -1)
+        decay = torch.exp(-torch.exp(c["a_log"].double()).view(1, h, 1) * step)
+        if op == "state_space":
+            skip, v = c["skip"].double().view(1, h, 1) * v, v * step
+    elif op == "linear_channel":
+        decay = c["decay"].double().view(t, h, d)
+    else:
+        decay = c["decay"].double().view(1, h, 1).expand(t, h, 1)
+    q, k = q.repeat_interleave(h // gr, 1), k.repeat_interleave(h // gr, 1)
+    beta = torch.sigmoid(c["beta"].double())
+    out = torch.zeros(t, h, vd, dtype=torch.float64, device=DEV)
+    state = c["state"].double()
+    at = 0
+    for i, (n, ln) in enumerate(zip(c["new"], c["lens"])):
+        if n == 0:
+            continue
+        s = state[c["slots"][i].long()] * (0.0 if ln == n else 1.0)
+        for r in range(at, at + n):
+            s = s * decay[r].unsqueeze(-1)
+            u = v[r].unsqueeze(1)
+            if op.startswith("delta"):
+                u = beta[r].view(h, 1, 1) * (u - k[r].unsqueeze(1) @ s)
+            s = s + k[r].unsqueeze(2) * u
+            out[r] = (q[r].unsqueeze(1) @ s).squeeze(1)
+        state[c["slots"][i].long()] = s
+        at += n
+    return (out * (0.25 if op == "linear_channel" else 1.0) + skip).reshape(t, h * vd), state
+
+
+def _off(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+OPS = ["linear_head", "linear_channel", "state_space", "delta_channel", "delta_head"]
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("dim,vdim,new,extra,dtype,pad", [
+    (128, 128, [64], [0], torch.bfloat16, 0),                              # one whole chunk
+    (128, 128, [200, 1, 63, 0, 65, 17], [0, 9, 70, 3, 0, 1], torch.bfloat16, 8),   # remainders, an empty sequence, states read
+    (64, 64, [129, 16], [5, 0], torch.float16, 3),                         # rows no vector load divides
+    (96, 80, [70, 33], [0, 12], torch.bfloat16, 4),                        # padded keys
+    (20, 24, [67, 40], [2, 0], torch.float32, 0),
+    (33, 7, [66], [1], torch.bfloat16, 1)])                                # odd sizes
+def test_chunks_match_the_recurrence_in_64_bits(op, strong, dim, vdim, new, extra, dtype, pad):
+    """A row's result is a sum over at most a few hundred products of fp32 values, every one formed by at most 64 + 64
+    roundings: 3e-6 bounds its relative error in norm (measured: 1e-7 to 4e-7)."""
+    groups = 2 if op in ("state_space", "delta_head") else 4
+    c = _case(op, 4, groups, dim, vdim, new, [n + e for n, e in zip(new, extra)], dtype, 11, strong, pad)
+    want, want_state = _rows64(c)
+    out, state = _run(c, True)
+    off, off_state = _off(out, want), _off(state, want_state)
+    assert off < 3e-6 and off_state < 3e-6, (off, off_state)
+    untouched = [i for i in range(c["state"].shape[0]) if i not in c["slots"].tolist()]
+    assert torch.equal(state[untouched], c["state"][untouched])
+    again, state2 = _run(c, True)
+    assert torch.equal(out, again) and torch.equal(state, state2)
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_chunks_are_no_less_exact_than_the_walk(op):
+    c = _case(op, 4, 4, 128, 128, [700, 300], [700, 420], torch.bfloat16, 3, False, 0)
+    want, want_state = _rows64(c)
+    (a, sa), (b, sb) = _run(c, True), _run(c, False)
+    assert _off(a, want) <= 1.5 * _off(b, want) + 1e-7 and _off(sa, want_state) <= 1.5 * _off(sb, want_state) + 1e-7
+
+
+def test_many_heads_are_taken_in_turns(monkeypatch):
+    c = _case("delta_channel", 6, 3, 64, 64, [90, 70], [90, 71], torch.bfloat16, 5)
+    want = _run(c, True)
+    monkeypatch.setattr(hip, "CHUNK_SCRATCH_BYTES", 1)
+    got = _run(c, True)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])

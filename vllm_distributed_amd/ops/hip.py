@@ -95,6 +95,7 @@ def load() -> ctypes.CDLL:
         "vdamd_expert_epilogue": [P, P, P, L, P, P, I, I, P, P, L, I, I, I, P],
         "vdamd_decay_linear_attention": [P, P, L, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "vdamd_channel_decay_attention": [P, P, L, P, P, P, P, P, I, I, I, I, F, I, I, I, P],
+        "vdamd_chunk_scan": [P, I, P, L, I, I, I, P, L, P, L, P, P, P, P, P, I, P, P, P, P] + [I] * 8 + [F, F, I, P],
         "vdamd_low_rank_decay": [P, P, L, P, P, I, I, I, F, I, P],
         "vdamd_weighted_relu_squared": [P, P, L, P, P, I, I, I, P],
         "vdamd_latent_prep": [P, P, L, L, I, P, L, L, P, L, P, F, P, I, F, P, P, P, P, I, I, I, I, I, I, I, P],
@@ -104,6 +105,8 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = c_int
+    lib.vdamd_chunk_scan_floats.argtypes = [I, I, I]
+    lib.vdamd_chunk_scan_floats.restype = c_long
     lib.vdamd_decode_workspace_floats.argtypes = [I, I, I]
     lib.vdamd_decode_workspace_floats.restype = c_long
     lib.vdamd_max_splits.restype = c_int
@@ -1442,10 +1445,60 @@ def add_layer_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor
 DECAY_ATTENTION_MAX_DIM = 256
 
 
+# ------------------------------------------------ recurrent mixers over prompt portions, 64 rows at a time
+LINEAR_HEAD, LINEAR_CHANNEL, STATE_SPACE, DELTA_CHANNEL, DELTA_HEAD = range(5)
+CHUNK_MAX_DIM = 128
+CHUNK_MIN_ROWS = 48
+CHUNK_SCRATCH_BYTES = 1 << 30
+
+
+def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> bool:
+    """Whether ``seqs`` sequences with ``rows`` rows in all, at most ``max_rows`` in one (0: unknown), go through the chunked
+    kernels: modelled times in us, fitted on an MI355X over 1 - 24 sequences, 8 - 32 heads and sizes 64 and 128.  The walk
+    row by row is a chain of dependent steps per row of the longest sequence, or where many sequences run bound by
+    issue; a chunk of 64 rows costs a link of a shorter chain and its share of the chip, however few rows it holds (16 heads,
+    dim 128: one prompt of 8000 rows 640 against 3440 us under the delta rule, 24 of 250 rows 348 against 398, 21 of 27
+    rows 84 against 50)."""
+    longest = max_rows if max_rows > 0 else rows // max(seqs, 1)
+    if dim > CHUNK_MAX_DIM or longest < CHUNK_MIN_ROWS:
+        return False
+    delta = kind >= DELTA_CHANNEL
+    area = (64 if dim <= 64 else 128) * vdim / 16384
+    walk = (22.0 if delta else 8.0) + max(longest * (0.37 if delta or kind == STATE_SPACE else 0.27),
+                                          rows * heads * area * (0.0032 if delta else 0.0025))
+    chunks = rows / 64 + seqs
+    chunked = 26.0 + longest / 64 * (3.6 if delta else 2.6) + chunks * heads * area * (0.16 if delta else 0.095)
+    return chunked < walk
+
+
+def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_bias, a_log, decay, d_skip, num_heads: int,
+                groups: int, dim: int, vdim: int, state, slots, query_start_loc, seq_lens, silu: bool, eps: float,
+                scale: float) -> torch.Tensor:
+    """One of the five recurrences over all sequences of a step (shapes checked by the caller).  The workspace (about 120 KB
+    per chunk of 64 rows and head, the delta rule 150) is kept under ``CHUNK_SCRATCH_BYTES`` by taking the heads in turns."""
+    t, b = x.shape[0], seq_lens.shape[0]
+    out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
+    if t == 0 or b == 0:
+        return out
+    chunks = (t + 63 * min(b, t)) // 64
+    floats = int(_LIB.vdamd_chunk_scan_floats(kind, dim, vdim)) * chunks
+    heads = min(num_heads, max(1, CHUNK_SCRATCH_BYTES // (4 * floats)))
+    ws = torch.empty(heads * floats, dtype=torch.float32, device=x.device)
+    for h0 in range(0, num_heads, heads):
+        _check(_LIB.vdamd_chunk_scan(
+            out.data_ptr(), kind, x.data_ptr(), x.stride(0), q_off, k_off, v_off, _ptr(beta),
+            0 if beta is None else beta.stride(0), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(dt_bias), _ptr(a_log),
+            _ptr(decay), _ptr(d_skip), ws.data_ptr(), chunks, state.data_ptr(), slots.data_ptr(),
+            query_start_loc.data_ptr(), seq_lens.data_ptr(), b, num_heads, groups, dim, vdim, h0,
+            min(heads, num_heads - h0), int(silu), float(eps), float(scale), _dt(x), _stream()), "chunk_scan")
+    return out
+
+
 def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int, decay: torch.Tensor,
                            state: torch.Tensor, slots: torch.Tensor, query_start_loc: torch.Tensor,
                            seq_lens: torch.Tensor, silu: bool = True, max_query_len: int = 0,
-                           scale: float = 1.0) -> torch.Tensor:
+                           scale: float = 1.0, chunked: Optional[bool] = None) -> torch.Tensor:
+    """``chunked`` forces (or forbids) the chunked kernels (tests, benchmarks)."""
     t = x.shape[0]
     n = seq_lens.numel()
     if dim > DECAY_ATTENTION_MAX_DIM:
@@ -1454,16 +1507,23 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
     assert state.dtype == torch.float32 and state.is_contiguous() and tuple(state.shape[1:]) == (num_heads, dim, vdim)
     assert slots.dtype == seq_lens.dtype == query_start_loc.dtype == torch.int32
     assert slots.numel() >= n and query_start_loc.numel() >= n + 1
-    out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
     if decay.dim() == 2:                 # one per row, head and key channel
         assert decay.shape == (t, num_heads * dim) and decay.dtype == torch.float32 and decay.is_contiguous()
+    elif scale != 1.0:
+        raise NotImplementedError("a scale on the result needs decays per key channel")
+    kind = LINEAR_CHANNEL if decay.dim() == 2 else LINEAR_HEAD
+    if chunk_scan_profitable(kind, t, n, max_query_len, num_heads, dim, vdim) if chunked is None else chunked:
+        qs = num_heads * dim
+        return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None,
+                           decay if decay.dim() == 2 else _f32_vec(decay, num_heads, "decay"), None, num_heads, num_heads,
+                           dim, vdim, state, slots, query_start_loc, seq_lens, silu, 0.0, scale)
+    out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
+    if decay.dim() == 2:
         _check(_LIB.vdamd_channel_decay_attention(
             out.data_ptr(), x.data_ptr(), x.stride(0), decay.data_ptr(), state.data_ptr(), slots.data_ptr(),
             query_start_loc.data_ptr(), seq_lens.data_ptr(), n, num_heads, dim, vdim, float(scale), int(bool(silu)),
             int(max_query_len), _dt(x), _stream()), "channel_decay_attention")
         return out
-    if scale != 1.0:
-        raise NotImplementedError("a scale on the result needs decays per key channel")
     _check(_LIB.vdamd_decay_linear_attention(out.data_ptr(), x.data_ptr(), x.stride(0),
                                              _f32_vec(decay, num_heads, "decay").data_ptr(), state.data_ptr(),
                                              slots.data_ptr(), query_start_loc.data_ptr(), seq_lens.data_ptr(), n,
@@ -1720,8 +1780,9 @@ def short_conv_act(x, channels: int, conv_weight, state, slots, query_start_loc,
 
 def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, beta, dt, dt_bias, a_log, state, slots,
                      query_start_loc, seq_lens, norm_eps: float = 1e-6, max_query_len: int = 0,
-                     parts: int = 0) -> torch.Tensor:
-    """``max_query_len`` (0: unknown) only helps the kernel choose its tiling; ``parts`` forces one (benchmarks).
+                     parts: int = 0, chunked: Optional[bool] = None) -> torch.Tensor:
+    """``max_query_len`` (0: unknown) only helps the kernel choose its tiling; ``parts`` forces one of the row by row walk,
+    ``chunked`` the chunked kernels or the walk (tests, benchmarks).
     ``dt[T, H]``: one decay per head."""
     t = _rows2d(x, "x").shape[0]
     h, g = int(num_heads), int(num_qk_heads)
@@ -1733,6 +1794,12 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
     assert state is not None and state.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (h, dim, vdim), (tuple(state.shape), (h, dim, vdim))
     assert slots.shape[0] == b and query_start_loc.shape[0] >= b + 1
+    kind = DELTA_HEAD if per_head else DELTA_CHANNEL
+    if (not parts and chunk_scan_profitable(kind, t, b, max_query_len, h, dim, vdim)) if chunked is None else chunked:
+        return _chunk_scan(kind, x, 0, g * dim, 2 * g * dim, beta, dt,
+                           _f32_vec(dt_bias, dt.shape[1], "dt_bias"), _f32_vec(a_log, h, "a_log"), None, None, h, g, dim, vdim,
+                           state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"),
+                           False, norm_eps, 1.0)
     dev = x.device
     qn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
     kn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
@@ -1755,8 +1822,9 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
 # ------------------------------------------------ selective state-space scan, gate in front of a grouped norm,
 # ------------------------------------------------ q / k normed over all heads with values = keys, mixed head weights
 def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, a_log, dt_bias, d_skip, state, slots,
-                   query_start_loc, seq_lens, max_query_len: int = 0) -> torch.Tensor:
-    """``max_query_len`` (0: unknown) only helps the kernel choose its launch."""
+                   query_start_loc, seq_lens, max_query_len: int = 0, chunked: Optional[bool] = None) -> torch.Tensor:
+    """``max_query_len`` (0: unknown) only helps the kernel choose its launch; ``chunked`` forces (or forbids) the chunked
+    kernels (tests, benchmarks)."""
     t = _rows2d(x, "x").shape[0]
     h, g, n = int(num_heads), int(groups), int(n_state)
     b = seq_lens.shape[0]
@@ -1765,6 +1833,12 @@ def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, 
     assert state is not None and state.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (h, n, vdim), (tuple(state.shape), (h, n, vdim))
     assert slots.shape[0] == b and query_start_loc.shape[0] >= b + 1
+    if chunk_scan_profitable(STATE_SPACE, t, b, max_query_len, h, n, int(vdim)) if chunked is None else chunked:
+        inner = h * vdim
+        return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, _f32_vec(dt_bias, h, "dt_bias"),
+                           _f32_vec(a_log, h, "a_log"), None, _f32_vec(d_skip, h, "d_skip"), h, g, n, int(vdim), state,
+                           _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"), False,
+                           0.0, 1.0)
     out = torch.empty((t, h * vdim), dtype=torch.float32, device=x.device)
     _check(_LIB.vdamd_selective_scan(
         out.data_ptr(), x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), _f32_vec(a_log, h, "a_log").data_ptr(),
