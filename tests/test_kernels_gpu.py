@@ -480,6 +480,45 @@ def test_sample_respects_filters_statistically():
         assert probs[3, tok[3]] >= 0.2 * sp[3, 0] - 1e-7
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,k,E,H,I,local", [
+    (1, 1, 3, 128, 16, None), (100, 2, 8, 256, 144, None),      # a row per tile; tiles of a few rows, columns past the last
+    (513, 1, 2, 256, 128, None), (700, 3, 10, 512, 384, (2, 5)),   # tiles of 256, 1 and 0 rows; experts held elsewhere
+    (900, 2, 4, 384, 2176, None)])                              # 17 tile columns: two groups, the last one short
+def test_grouped_gemm_in_large_tiles(dtype, T, k, E, H, I, local):
+    """Against fp32 products of the same 16-bit operands: a 16-bit rounding of the result (2^-9 of it) and of nothing else."""
+    torch.manual_seed(T)
+    logits = _rand(T, E, dtype=torch.float32)
+    logits[: T // 2, 0] += 3.0                                  # an expert that is asked for more often, one hardly at all
+    logits[:, E - 1] -= 3.0
+    topi = logits.topk(k, -1).indices.to(torch.int32).contiguous()
+    start, count = local or (0, -1)
+    from vllm_distributed_amd.ops import hip
+    src, inv, tiles = hip.moe_align(topi, E, ops.GROUPED_BIG_ROWS, start, count)
+    x = _rand(T, H, dtype=dtype)
+    w13 = _rand(count if local else E, 2 * I, H, dtype=dtype, scale=H ** -0.5)
+    w2 = _rand(count if local else E, H, 128 * ((I + 127) // 128), dtype=dtype, scale=I ** -0.5)
+    xs = x.index_select(0, src)
+    act = hip.grouped_gemm(xs, w13, tiles, ops.GROUPED_BIG_ROWS, silu_mul=True)
+    wide = torch.nn.functional.pad(act, (0, w2.shape[2] - I))
+    filler = torch.full((T * k, H), 7.0, device=DEV, dtype=dtype)
+    y = hip.grouped_gemm(wide, w2, tiles, ops.GROUPED_BIG_ROWS, out=filler.clone())
+    seen = torch.zeros(T * k, dtype=torch.bool, device=DEV)
+    for e, r0, n in tiles.tolist():
+        if n == 0:
+            continue
+        assert 0 < n <= 256 and not seen[r0:r0 + n].any()
+        seen[r0:r0 + n] = True
+        h = xs[r0:r0 + n].float() @ w13[e].float().t()
+        ref = torch.nn.functional.silu(h[:, :I]) * h[:, I:]
+        assert (act[r0:r0 + n].float() - ref).norm() <= 3e-3 * ref.norm() + 1e-6
+        ref = wide[r0:r0 + n].float() @ w2[e].float().t()
+        assert (y[r0:r0 + n].float() - ref).norm() <= 3e-3 * ref.norm() + 1e-6
+    expert = topi.reshape(-1)[torch.argsort(inv.long())]
+    mine = (expert >= start) & (expert < start + count) if local else torch.ones_like(seen)
+    assert torch.equal(seen, mine) and torch.equal(y[~seen], filler[~seen])
+
+
 @pytest.mark.parametrize("V,dtype,spread,offset", [
     (1, torch.float32, 2.0, 0), (2, torch.bfloat16, 2.0, 1), (7, torch.float16, 2.0, 3),
     (1023, torch.float32, 2.0, 1), (4097, torch.bfloat16, 0.0, 0),           # more equal weights than the list holds

@@ -211,16 +211,20 @@ class FusedMoE(nn.Module):
         return F.linear(ops.silu_and_mul(F.linear(x, self.w13[e])), self.w2[e])
 
     def _grouped_tile_rows(self, x: torch.Tensor) -> int:
-        """Row-tile size for the grouped HIP GEMMs, or 0 to use the per-expert
-        library GEMMs (large prefill batches, where each expert has hundreds of
-        rows and hipBLASLt is compute-efficient; that path syncs with the host,
-        so it is never taken while a hipGraph is being captured)."""
+        """Row-tile size for the grouped HIP GEMMs - dense experts with more than 64 rows each go to the
+        large-batch kernel's grouped form, 256 rows a tile - or 0 to use the per-expert library GEMMs (4-bit
+        experts, and shapes that form does not take, with hundreds of rows each; that path syncs with the
+        host, so it is never taken while a hipGraph is being captured)."""
         if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and ops.hip_available()):
             return 0
         if self.quant is None and (self.w13.shape[2] % 128 or self.w2.shape[2] % 128 or self.w13.shape[1] % 16):
             return 0
         cap = 64 if self.qw13 is not None else 128
         avg = x.shape[0] * self.top_k / max(1, self.num_experts)
+        if self.quant is None and avg > 64 and ops.grouped_big_ok(x, self.top_k, self.w13, self.w2):
+            # (64 experts of 2048 x 1408 with 75 rows each: 268 us against 332 in tiles of 128; 8 of 4096 x 14336 with 50:
+            # 676 against 597 in tiles of 64, with 100: 673 against 803)
+            return ops.GROUPED_BIG_ROWS
         if avg > envs.VDAMD_MOE_GROUPED_MAX_ROWS * cap / 64 and not torch.cuda.is_current_stream_capturing():
             return 0
         for rows in (16, 32, 64, 128):
@@ -259,8 +263,8 @@ class FusedMoE(nn.Module):
             h = ops.grouped_linear(xs, tiles, tile_rows, qw=self.qw13, sz=self.sz13, alpha=self.alpha13)
             return ops.grouped_linear(h, tiles, tile_rows, qw=self.qw2, sz=self.sz2, alpha=self.alpha2,
                                       silu_mul=True)
-        h = ops.grouped_linear(xs, tiles, tile_rows, weight=self.w13)
-        return ops.grouped_linear(ops.silu_and_mul(h), tiles, tile_rows, weight=self.w2)
+        act = ops.grouped_gate_up_silu(xs, tiles, tile_rows, self.w13)
+        return ops.grouped_linear(act, tiles, tile_rows, weight=self.w2)
 
     def _forward_fused_routing(self, x: torch.Tensor, logits: torch.Tensor, tile_rows: int, deferred: bool = False):
         """Routing, expert GEMMs and the weighted sum in eight launches (router

@@ -577,6 +577,25 @@ def grouped_linear(x, tiles, tile_rows: int, weight=None, qw=None, sz=None, alph
     return _hip.grouped_gemm(x, weight, tiles, tile_rows)
 
 
+GROUPED_BIG_ROWS = 256      # the row-tile size of ``moe_align`` that stands for the large-batch kernel's grouped form
+
+
+def grouped_big_ok(x, top_k: int, w13, w2) -> bool:
+    """Whether dense experts ``w13 [E, 2I, H]`` / ``w2 [E, H, I]`` over the ``top_k`` slots of each row of ``x`` may run in
+    tiles of ``GROUPED_BIG_ROWS`` rows: shapes and types the kernel takes, every operand within 32-bit byte offsets."""
+    widest = max(w13.shape[1], w13.shape[2], w2.shape[1], w2.shape[2])
+    return (_use_hip(x) and envs.VDAMD_BIG_GEMM and x.shape[0] * top_k * widest * 2 < (1 << 32) - 64
+            and _hip.grouped_big_supported(x, w13, True) and _hip.grouped_big_supported(x, w2))
+
+
+def grouped_gate_up_silu(x, tiles, tile_rows: int, weight):
+    """``silu(x @ Wg^T) * (x @ Wu^T)`` per group for ``weight [G, 2I, K] = [Wg ; Wu]``: inside the GEMM in tiles of
+    ``GROUPED_BIG_ROWS`` rows, otherwise with the activation kernel behind it."""
+    if tile_rows == GROUPED_BIG_ROWS:
+        return _hip.grouped_gemm(x, weight, tiles, tile_rows, silu_mul=True)
+    return silu_and_mul(grouped_linear(x, tiles, tile_rows, weight=weight))
+
+
 def grouped_silu_fused(tile_rows: int, qw, sz) -> bool:
     """Whether the grouped GEMM of these weights forms ``silu(gate) * up`` itself at this tile size
     (integer 4-bit experts, few rows per expert: decode)."""

@@ -39,6 +39,7 @@ def load() -> ctypes.CDLL:
         "vdamd_mid_gemm": [P, L, P, L, P, L, P, I, I, I, I, I, I, I, I, P],
         "vdamd_stream_gemm": [P, L, P, L, P, L, P, P, L, I, I, I, I, I, I, I, I, I, P],
         "vdamd_big_gemm": [P, L, P, L, P, L, P, L, I, I, I, I, I, I, P],
+        "vdamd_big_gemm_grouped": [P, L, P, L, P, L, L, P, I, I, I, I, I, I, P],
         "vdamd_rope_cache": [P, P, P, P, L, L, L, P, P, P, P, I, I, I, I, I, I, P, P, F, I, I, P, P, P],
         "vdamd_rope_cache_slabs": [P, P, I, P, L, P, P, P, P, I, I, I, I, I, P, P, F, I, I, P, P, P],
         "vdamd_paged_attention_decode": [P, P, P, L, P, P, P, I, P, F, I, I, I, I, I, I, L, I, I, P, P, I, F, P, P, P],
@@ -911,18 +912,37 @@ def _check_tiles(tiles: torch.Tensor, x: torch.Tensor, tile_rows: int) -> int:
     return tiles.shape[0]
 
 
+GROUPED_BIG_ROWS = 256             # rows per tile of the grouped form of the large-batch GEMM
+
+
+def grouped_big_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = False) -> bool:
+    """Whether the large-batch kernel's grouped form takes rows like ``x`` and experts ``w [G, N, K]``."""
+    n, k = w.shape[1:]
+    return (w.is_contiguous() and w.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and k % 128 == 0
+            and n % (32 if silu_mul else 16) == 0 and w.data_ptr() % 16 == 0 and n * k * 2 < (1 << 32) - 64)
+
+
 def grouped_gemm(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, tile_rows: int,
-                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 out: Optional[torch.Tensor] = None, silu_mul: bool = False) -> torch.Tensor:
     """``out[r] = x[r] @ w[g(r)]^T`` for group-sorted rows: ``w [G, N, K]``,
     ``tiles [n, 3] int32`` = (group, first row, rows <= tile_rows; 0 = unused).
     Every row covered by a tile must lie inside ``x``; rows outside all tiles
-    are left untouched in ``out``."""
+    are left untouched in ``out``.  ``tile_rows`` 256: the large-batch kernel, with ``silu_mul`` for ``w = [gate ; up]`` and
+    ``silu(gate) * up`` as the result (``N / 2`` wide)."""
     nt = _check_tiles(tiles, x, tile_rows)
     g, n, k = w.shape
-    assert w.is_contiguous() and w.dtype == x.dtype and x.shape[1] == k and 16 <= tile_rows <= 128
+    assert w.is_contiguous() and w.dtype == x.dtype and x.shape[1] == k
     assert k % 128 == 0 and n % 16 == 0
+    n_out = n // 2 if silu_mul else n
     if out is None:
-        out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
+        out = torch.empty((x.shape[0], n_out), dtype=x.dtype, device=x.device)
+    if tile_rows == GROUPED_BIG_ROWS:
+        assert grouped_big_supported(x, w, silu_mul) and out.shape == (x.shape[0], n_out) and out.stride(1) == 1
+        _check(_LIB.vdamd_big_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k, n * k,
+                                           tiles.data_ptr(), nt, x.shape[0], n, k, EPI_SILU_MUL if silu_mul else EPI_NONE,
+                                           _dt(x), _stream()), "big_gemm_grouped")
+        return out
+    assert 16 <= tile_rows <= 128 and not silu_mul
     ntw = 1 if tile_rows > 64 or n <= 4096 else 2
     _check(_LIB.vdamd_skinny_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k,
                                           n * k, tiles.data_ptr(), nt, tile_rows, n, k, ntw, _dt(x), _stream()),
