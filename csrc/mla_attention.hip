@@ -264,6 +264,207 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// Decoded rows with up to 16 heads per workgroup, reading the key rows alone: a row's first DV values ARE its value, so the
+// V^T cache need not be read for them.  32 keys at a time go global -> LDS by DMA (one run of 32 * DK values: a group of
+// keys never crosses a block here), the next group's while the current one is multiplied, two workgroups per CU.
+//   * QK: as above, a wave per quarter of the reduction; K fragments are read from LDS by rows.
+//   * PV: a lane reads 4 neighbouring values of each of its 8 keys (8 bytes each) and turns them by byte permutes into V^T
+//     fragments of four tiles whose row i is value 4 i + tile of the wave's 64: a permutation of the output's columns that
+//     leaves a lane with 16 neighbouring ones of them.
+// The 16-byte pieces of a row are XOR-ed with bits 1, 3 and 4 of the key's number (the 16 rows of a K fragment then lie in
+// 16 different places of the LDS's 256 bytes).
+// Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 109 us against 211 through both
+// caches (441 and 833 MB; the chip's copy rate would take 91).
+// ---------------------------------------------------------------------------------------------------------------
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void mla_lds_void;
+typedef __attribute__((address_space(1))) void mla_glb_void;
+
+// 16 bytes per lane from global memory straight into LDS: the wave's 64 pieces land at lds_wave_base + 16 * lane
+__device__ __forceinline__ void mla_dma16(const void* g, void* lds_wave_base) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the builtin exists in the device pass only)
+  __builtin_amdgcn_global_load_lds((mla_glb_void*)const_cast<void*>(g), (mla_lds_void*)lds_wave_base, 16, 0, 0);
+#endif
+}
+
+template <typename T, int DK, int DV, bool P2>
+__global__ __launch_bounds__(256, 2) void mla_rows_kernel(
+    T* __restrict__ out, long out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const T* __restrict__ q, long q_stride, const T* __restrict__ k_cache, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ token_seq, const int* __restrict__ seq_lens, float scale_log2e, int Hq, int block_size,
+    int num_splits, MlaExtra ex) {
+  using V = typename Vec8<T>::type;
+  constexpr int KSTEPS = DK / 32, KS = (KSTEPS + 3) / 4;
+  constexpr int ROW = DK * 2, PIECES = DK / 8, NP = 32 * PIECES / 256;   // bytes, 16-byte pieces of a row; pieces per thread
+  constexpr int VI = DV / 256;                                          // runs of 64 values per wave
+  static_assert(DK % 64 == 0 && DV % 256 == 0 && 32 * PIECES % 256 == 0, "unsupported latent width");
+  // (one object for both uses: the compiler waits for DMA in flight at reads of an object that it knows to be its target)
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 32 * ROW + 4 * 2 * 64 * 16];
+  float (*s_part)[2][64][4] = reinterpret_cast<float (*)[2][64][4]>(smem + 2 * 32 * ROW);
+
+  const int split = blockIdx.x, qt = blockIdx.y, t = blockIdx.z;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int qh0 = qt * 16;
+  const int nq = min(16, Hq - qh0);
+  const int seq_len = seq_lens[t];
+  const int* bt_row = block_table + (long)(token_seq != nullptr ? token_seq[t] : t) * bt_stride;
+  const int win_lo = ex.window > 0 ? max(seq_len - ex.window, 0) : 0;
+  const int g_lo = win_lo >> 5;
+  const int n_groups = ((seq_len + 31) >> 5) - g_lo;
+  const int gps = (n_groups + num_splits - 1) / num_splits;
+  const int g_begin = g_lo + split * gps;
+  const int g_end = min(g_begin + gps, g_lo + n_groups);
+
+  V qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int sg = wid * KS + s;
+    V z;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) z[j] = (T)0.f;
+    qf[s] = (sg < KSTEPS && r16 < nq) ? ld8<T>(q + t * q_stride + (long)(qh0 + r16) * DK + 32 * sg + 8 * g4) : z;
+  }
+  f32x4 acc[VI][4];
+#pragma unroll
+  for (int i = 0; i < VI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = MLA_NEG_BIG, l = 0.f;
+
+  auto swz = [](int key) { return ((key >> 1) & 1) | (((key >> 3) & 3) << 1); };
+  // this thread's pieces of a group: (row, place in LDS) -> piece of the row in memory
+  int prow[NP], pbyte[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int c = i * 256 + (int)threadIdx.x;
+    prow[i] = c / PIECES;
+    pbyte[i] = ((c - prow[i] * PIECES) ^ swz(prow[i])) * 16;
+  }
+  auto stage = [&](int g, int buf) {
+    const int base = g * 32;
+    const long first = (long)bt_row[base / block_size] * block_size + (base % block_size);
+    const char* src = reinterpret_cast<const char*>(k_cache + first * DK);
+    // rows that hold no visible key repeat one that does: what a block holds behind the sequence's end is not looked at
+    const int lo = max(win_lo - base, 0), hi = min(seq_len - 1 - base, 31);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      mla_dma16(src + max(min(prow[i], hi), lo) * ROW + pbyte[i], smem + buf * 32 * ROW + (i * 256 + wid * 64) * 16);
+  };
+
+  const int key_a = 8 * (r16 >> 2) + (r16 & 3);    // K rows of the two interleaved S^T tiles: this one and 4 behind it
+  const int off_a = key_a * ROW, off_b = (key_a + 4) * ROW, swz_a = swz(key_a), swz_b = swz(key_a + 4);
+  if (g_begin < g_end) stage(g_begin, 0);
+  for (int g = g_begin; g < g_end; ++g) {
+    const int buf = (g - g_begin) & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                               // the group is in LDS, and nobody reads the other buffer any more
+    if (g + 1 < g_end) stage(g + 1, buf ^ 1);
+    const char* tile = smem + buf * 32 * ROW;
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int piece = min(wid * KS + s, KSTEPS - 1) * 4 + g4;
+      s0 = mfma16(*reinterpret_cast<const V*>(tile + off_a + ((piece ^ swz_a) << 4)), qf[s], s0);
+      s1 = mfma16(*reinterpret_cast<const V*>(tile + off_b + ((piece ^ swz_b) << 4)), qf[s], s1);
+    }
+    *reinterpret_cast<f32x4*>(s_part[wid][0][lane]) = s0;
+    *reinterpret_cast<f32x4*>(s_part[wid][1][lane]) = s1;
+    // (not __syncthreads(), which would also wait for the next group's rows)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    s0 = *reinterpret_cast<const f32x4*>(s_part[0][0][lane]);
+    s1 = *reinterpret_cast<const f32x4*>(s_part[0][1][lane]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      s0 += *reinterpret_cast<const f32x4*>(s_part[w][0][lane]);
+      s1 += *reinterpret_cast<const f32x4*>(s_part[w][1][lane]);
+    }
+    const int kidx0 = g * 32 + 8 * g4;
+    float p[8];
+    float tmax = MLA_NEG_BIG;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float sv = (j < 4 ? s0[j & 3] : s1[j & 3]) * scale_log2e;
+      p[j] = (kidx0 + j < seq_len && kidx0 + j >= win_lo) ? sv : MLA_NEG_BIG;
+      tmax = fmaxf(tmax, p[j]);
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m, tmax);
+    const float alpha = fast_exp2(m - m_new);
+    float psum = 0.f;
+    V pf;
+    [[maybe_unused]] V pl;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float e = p[j] <= 0.5f * MLA_NEG_BIG ? 0.f : fast_exp2(p[j] - m_new);
+      psum += e;
+      pf[j] = (T)e;
+      if constexpr (P2) pl[j] = (T)(e - (float)pf[j]);
+    }
+    l = l * alpha + psum;
+    m = m_new;
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      // the piece of a row this lane's four values lie in, and which half of it
+      const int piece = (wid * VI + i) * 8 + (r16 >> 1), half = (r16 & 1) * 8;
+      u32x2 w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = 8 * g4 + j;
+        w[j] = *reinterpret_cast<const u32x2*>(tile + key * ROW + ((piece ^ swz(key)) << 4) + half);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        union { uint32_t u[4]; V f; } fr;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t a = w[2 * j][v >> 1], b = w[2 * j + 1][v >> 1];
+          fr.u[j] = __builtin_amdgcn_perm(b, a, (v & 1) ? 0x07060302u : 0x05040100u);
+        }
+        acc[i][v] *= alpha;
+        acc[i][v] = mfma16(fr.f, pf, acc[i][v]);
+        if constexpr (P2) acc[i][v] = mfma16(fr.f, pl, acc[i][v]);
+      }
+    }
+  }
+
+  float lsum = l;
+  lsum += __shfl_xor(lsum, 16, 64);
+  lsum += __shfl_xor(lsum, 32, 64);
+  if (r16 >= nq) return;
+  const int qh = qh0 + r16;
+  // acc[i][v][r]: value 64 (wid * VI + i) + 16 g4 + 4 r + v
+  if (num_splits == 1) {
+    float factor = 1.f;
+    if (ex.sinks != nullptr) mla_add_sink(ex.sinks[qh] * 1.4426950408889634f, m, lsum, factor);
+    float inv = lsum > 0.f ? factor / lsum : 0.f;
+    if (ex.gate != nullptr) inv *= 1.f / (1.f + __expf(-(float)((const T*)ex.gate)[t * ex.gate_stride + qh]));
+    T* orow = out + t * out_stride + (long)qh * DV + 16 * g4;
+#pragma unroll
+    for (int i = 0; i < VI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        typename Vec4<T>::type o;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (T)(acc[i][v][r] * inv);
+        *reinterpret_cast<typename Vec4<T>::type*>(orow + 64 * (wid * VI + i) + 4 * r) = o;
+      }
+  } else {
+    const long pidx = ((long)t * Hq + qh) * num_splits + split;
+#pragma unroll
+    for (int i = 0; i < VI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(part_o + pidx * DV + 64 * (wid * VI + i) + 16 * g4 + 4 * r) =
+            f32x4{acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+    if (wid == 0 && g4 == 0) { part_ml[2 * pidx] = m; part_ml[2 * pidx + 1] = lsum; }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // Several query tiles per workgroup over ONE stream of cache fragments.  The kernel above requests every cached
 // row once per 16 query rows; wherever more rows share a sequence, that is the L2's bandwidth, not HBM's:
 //   * BY_TOKEN (prefill chunks, verification): the NQ tiles are NQ consecutive tokens of one sequence - the token
@@ -594,6 +795,15 @@ int launch_mla(void* out, long out_stride, void* part_o, void* part_ml, const vo
     mla_attention_multi_kernel<T, DK, DV, NQ, false, KV8, P2><<<dim3(num_splits, (q_tiles + NQ - 1) / NQ, T_), 256, 0, st>>>(
         (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, k_cache, v_cache, block_table,
         bt_stride, token_seq, seq_lens, sl2, T_, Hq, block_size, num_splits, ex);
+  } else if (mode == 3) {                           // a workgroup per 16 heads over the key rows alone
+    if constexpr (!KV8 && DV % 256 == 0 && DK % 64 == 0) {
+      if (block_size % 32) return -1;
+      mla_rows_kernel<T, DK, DV, P2><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(
+          (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, (const T*)k_cache, block_table, bt_stride,
+          token_seq, seq_lens, sl2, Hq, block_size, num_splits, ex);
+    } else {
+      return -4;
+    }
   } else {
     mla_attention_kernel<T, DK, DV, KV8, P2><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(
         (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, k_cache, v_cache, block_table,
@@ -640,6 +850,7 @@ int dispatch_mla(int DK, int DV, int kv_fp8, void* out, long out_stride, void* p
 // part_o / part_ml: num_splits * T * Hq * (DV | 2) floats when num_splits > 1.
 // mode 0: one workgroup per (token, 16 heads); 1: four consecutive tokens of a sequence per workgroup (needs
 // token_seq; positions inside a sequence must be consecutive); 2: four head tiles of a token per workgroup.
+// mode 3: as mode 0, the values taken from the key rows (16-bit caches, blocks of a multiple of 32 tokens, DV a multiple of 256).
 // Supported (DK, DV): (576, 512) DeepSeek-V2 / V3, (320, 256), (96, 64).
 VDAMD_API int vdamd_mla_attention(void* out, long out_stride, void* part_o, void* part_ml, const void* q,
                                   long q_stride, const void* k_cache, const void* v_cache, const int* block_table,

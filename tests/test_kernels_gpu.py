@@ -1193,6 +1193,14 @@ def test_latent_attention_decode_prefill_and_cache_write(dk, dv, hq, bs, dtype, 
     for mode in (None, 0, 2):             # by shape; a workgroup per 16 heads; four head tiles per workgroup
         got = _hip.mla_attention(q, kc, vc, table, None, sl, scale, max(lens), mode=mode)
         torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2)
+    if not kv8 and _hip.mla_rows_ok(kc, dv):      # values from the key rows; what lies behind a sequence's end is not looked at
+        behind = kc.clone()
+        for b, n in enumerate(lens):
+            behind[table[b, (n - 1) // bs].long(), 0, (n - 1) % bs + 1:] = float("nan")
+        for splits in (None, 1, 3):
+            got = _hip.mla_attention(q, behind, vc, table, None, sl, scale, max(lens), mode=3, splits=splits)
+            torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2)
+            assert _hip.mla_attention(q, behind, vc, table, None, 0 * sl, scale, max(lens), mode=3, splits=splits).eq(0).all()
     got = _hip.mla_attention(q, kc, vc, table, None, sl, scale, max(lens), mode=2, splits=1)
     torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2)
     assert _hip.mla_num_splits(len(lens), 1, max(lens)) > 1

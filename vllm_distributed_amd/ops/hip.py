@@ -1183,12 +1183,18 @@ def mla_cache_write(latent: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
            "mla_cache_write")
 
 
-def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int) -> int:
-    """KV splits: about one workgroup per CU in total and no split shorter than ~192 keys.  A workgroup
-    streams ~36 GB/s by itself (one group of 32 keys in flight ahead of the one being multiplied), so the
-    chip's bandwidth needs a few hundred of them; beyond that, more splits only add partial sums to write and
-    merge (scripts/dev/mla_split_sweep.py: the fastest count is within ~5 % of this rule from batch 1 to 256)."""
-    want = -(-256 // max(1, tokens * q_tiles))
+def mla_rows_ok(k_cache: torch.Tensor, dv: int) -> bool:
+    """Whether the kernel that takes the values from the key rows reads this cache (16-bit rows, whole groups of 32 keys in a
+    block, a value width that divides over its waves)."""
+    return k_cache.dtype != FP8_KV and k_cache.shape[2] % 32 == 0 and dv % 256 == 0
+
+
+def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int, workgroups: int = 256) -> int:
+    """KV splits: about one workgroup per CU in total (``workgroups``: two, of the kernel that lets two share a CU) and no
+    split shorter than ~192 keys.  A workgroup streams ~36 GB/s by itself (one group of 32 keys in flight ahead of the one
+    being multiplied), so the chip's bandwidth needs a few hundred of them; beyond that, more splits only add partial sums
+    to write and merge (scripts/dev/mla_split_sweep.py: the fastest count is within ~5 % of this rule from batch 1 to 256)."""
+    want = -(-workgroups // max(1, tokens * q_tiles))
     return int(max(1, min(want, max_seq_len // 192, 64)))
 
 
@@ -1201,7 +1207,10 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     ``token_seq[t]`` (``t`` itself when None) and sees keys ``0 .. seq_lens[t] - 1``.  ``mode`` (default: by
     shape): 0 = a workgroup per (token, 16 heads); 1 = four consecutive tokens of a sequence per workgroup
     (steps with ``token_seq``: prefill chunks, verification - the tokens of a sequence must be adjacent rows at
-    consecutive positions); 2 = four head tiles of a token per workgroup (64 heads per rank and more).
+    consecutive positions); 2 = four head tiles of a token per workgroup (64 heads per rank and more); 3 = as 0,
+    the values read from the key rows (their first ``DV`` values, which is what every writer puts into both caches):
+    half the bytes, 1.1 to 2.5 times as fast from one sequence of 100 keys to 256 of 1500, at every width and head
+    count measured, so 0 is left with what 3 does not read (``mla_rows_ok``).
     ``precise``: the softmax weights enter the PV product with fp32 precision (a high and a low 16-bit part).
     ``window`` > 0: only the last ``window`` of those keys; ``sinks[Hq]`` (fp32): ``exp(sinks[h])`` joins head ``h``'s
     softmax denominator; ``gate[T, Hq]`` (raw, rows may be strided): the output times its sigmoid."""
@@ -1220,13 +1229,16 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     if mode is None:
         # (four head tiles per workgroup need enough workgroups left to fill the chip)
         mode = 1 if token_seq is not None else (2 if q_tiles >= 4 and t * q_tiles >= 128 else 0)
+        if mode == 0 and mla_rows_ok(k_cache, dv):
+            mode = 3
     gate_stride = 0
     if gate is not None:
         assert gate.dim() == 2 and gate.shape[0] >= t and gate.shape[1] == hq and gate.stride(1) == 1 and gate.dtype == q.dtype
         gate_stride = gate.stride(0)
     if splits is None:
         keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
-        splits = mla_num_splits(-(-t // 4) if mode == 1 else t, -(-q_tiles // 4) if mode == 2 else q_tiles, keys)
+        splits = mla_num_splits(-(-t // 4) if mode == 1 else t, -(-q_tiles // 4) if mode == 2 else q_tiles, keys,
+                                512 if mode == 3 else 256)
     part_o = part_ml = None
     if splits > 1:
         part_o = torch.empty((t * hq * splits, dv), dtype=torch.float32, device=q.device)
