@@ -21,6 +21,7 @@
 // running max is shared by the four lanes that hold one query column (two
 // xor-shuffles per 32 keys); row sums stay lane-local until the end.
 #include "common.h"
+#include "split_merge.h"
 
 namespace {
 
@@ -340,21 +341,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
 }
 
 template <typename T, int D>
-__global__ void decode_reduce_kernel(T* __restrict__ out, const float* __restrict__ part_o,
-                                     const float* __restrict__ part_ml, int Hq, int num_splits, long out_stride,
-                                     const float* __restrict__ sinks) {
-  const int qh = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+__global__ __launch_bounds__(SPLIT_MERGE_MAX_THREADS) void decode_reduce_kernel(
+    T* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_ml, int Hq, int num_splits,
+    long out_stride, const float* __restrict__ sinks) {
+  const int qh = blockIdx.x, b = blockIdx.y;
   const long base = ((long)b * Hq + qh) * num_splits;
-  float mm = NEG_BIG;
-  for (int s = 0; s < num_splits; ++s) mm = fmaxf(mm, part_ml[2 * (base + s)]);
-  float o = 0.f, lt = 0.f;
-  for (int s = 0; s < num_splits; ++s) {
-    const float a = fast_exp2(part_ml[2 * (base + s)] - mm);
-    lt += part_ml[2 * (base + s) + 1] * a;
-    o += part_o[(base + s) * D + d] * a;
-  }
-  if (sinks != nullptr) lt += fast_exp2(sinks[qh] * LOG2E_F - mm);
-  out[b * out_stride + (long)qh * D + d] = (T)(lt > 0.f ? o / lt : 0.f);
+  f32x4 o;
+  float lt;
+  if (!split_merge<D>(part_o + base * D, part_ml + 2 * base, num_splits,
+                      sinks != nullptr ? sinks + qh : nullptr, NEG_BIG, o, lt)) return;
+  T* dst = out + b * out_stride + (long)qh * D + 4 * threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) dst[i] = (T)(lt > 0.f ? o[i] / lt : 0.f);
 }
 
 // ---------------------------------------------------------------------------
@@ -547,7 +545,7 @@ int launch_decode(void* out, float* ws, const void* q, long q_stride, const void
                      alibi);
   HIP_LAUNCH_CHECK();
   if (num_splits > 1) {
-    hipLaunchKernelGGL((decode_reduce_kernel<T, D>), dim3(Hq, B), dim3(D), 0, s, (T*)out, part_o, part_ml, Hq,
+    hipLaunchKernelGGL((decode_reduce_kernel<T, D>), dim3(Hq, B), dim3(split_merge_threads(D, num_splits)), 0, s, (T*)out, part_o, part_ml, Hq,
                        num_splits, out_stride, sinks);
     HIP_LAUNCH_CHECK();
   }

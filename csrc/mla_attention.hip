@@ -30,6 +30,7 @@
 // FlashMLA / vLLM's MLA backends are the CUDA counterparts; the reference framework reaches them through the
 // vLLM image it runs (/root/reference/Dockerfile:1).
 #include "common.h"
+#include "split_merge.h"
 
 namespace {
 
@@ -684,25 +685,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
-// Merge of the KV splits: out = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).
 template <typename T, int DV>
-__global__ void mla_reduce_kernel(T* __restrict__ out, long out_stride, const float* __restrict__ part_o,
-                                  const float* __restrict__ part_ml, int Hq, int num_splits, MlaExtra ex) {
+__global__ __launch_bounds__(SPLIT_MERGE_MAX_THREADS) void mla_reduce_kernel(
+    T* __restrict__ out, long out_stride, const float* __restrict__ part_o, const float* __restrict__ part_ml, int Hq,
+    int num_splits, MlaExtra ex) {
   const int t = blockIdx.y, qh = blockIdx.x;
   const long p0 = ((long)t * Hq + qh) * num_splits;
-  float mm = MLA_NEG_BIG;
-  for (int s = 0; s < num_splits; ++s) mm = fmaxf(mm, part_ml[2 * (p0 + s)]);
-  const float sink2 = ex.sinks != nullptr ? ex.sinks[qh] * 1.4426950408889634f : MLA_NEG_BIG;
-  mm = fmaxf(mm, sink2);
-  float lt = ex.sinks != nullptr ? fast_exp2(sink2 - mm) : 0.f;
-  for (int s = 0; s < num_splits; ++s) lt += part_ml[2 * (p0 + s) + 1] * fast_exp2(part_ml[2 * (p0 + s)] - mm);
+  f32x4 o;
+  float lt;
+  if (!split_merge<DV>(part_o + p0 * DV, part_ml + 2 * p0, num_splits, ex.sinks != nullptr ? ex.sinks + qh : nullptr,
+                       MLA_NEG_BIG, o, lt)) return;
   float inv = lt > 0.f ? 1.f / lt : 0.f;
   if (ex.gate != nullptr) inv *= 1.f / (1.f + __expf(-(float)((const T*)ex.gate)[t * ex.gate_stride + qh]));
-  for (int d = threadIdx.x; d < DV; d += blockDim.x) {
-    float o = 0.f;
-    for (int s = 0; s < num_splits; ++s) o += part_o[(p0 + s) * DV + d] * fast_exp2(part_ml[2 * (p0 + s)] - mm);
-    out[t * out_stride + (long)qh * DV + d] = (T)(o * inv);
-  }
+  T* dst = out + t * out_stride + (long)qh * DV + 4 * threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) dst[i] = (T)(o[i] * inv);
 }
 
 // One token's latent row into both cache forms.  x[T][DK] (row stride in elements); slot < 0: skipped.
@@ -811,8 +808,8 @@ int launch_mla(void* out, long out_stride, void* part_o, void* part_ml, const vo
   }
   HIP_LAUNCH_CHECK();
   if (num_splits > 1) {
-    mla_reduce_kernel<T, DV><<<dim3(Hq, T_), 128, 0, st>>>((T*)out, out_stride, (const float*)part_o,
-                                                          (const float*)part_ml, Hq, num_splits, ex);
+    mla_reduce_kernel<T, DV><<<dim3(Hq, T_), split_merge_threads(DV, num_splits), 0, st>>>(
+        (T*)out, out_stride, (const float*)part_o, (const float*)part_ml, Hq, num_splits, ex);
     HIP_LAUNCH_CHECK();
   }
   return 0;

@@ -1151,6 +1151,31 @@ def test_k_split_partial_sums_reduced_by_the_following_norm(m, n, k):
     assert (normed.float() - n2.float()).abs().max().item() < 0.13      # two bf16 roundings of values up to ~8
 
 
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+@pytest.mark.parametrize("with_sinks", [False, True])
+def test_decode_splits_merge_to_the_unsplit_result(d, with_sinks):
+    """Numbers of splits around what one round of the merge's groups holds, with splits that no key falls into."""
+    from vllm_distributed_amd.ops import hip as _hip
+    torch.manual_seed(d)
+    lens, hq, hkv, bs = [1, 33, 500, 2100], 6, 2, 64
+    nb = -(-max(lens) // bs)
+    kc = torch.randn(ops.k_cache_shape(len(lens) * nb, hkv, d, bs), device=DEV).bfloat16()
+    vc = torch.randn(ops.v_cache_shape(len(lens) * nb, hkv, d, bs), device=DEV).bfloat16()
+    table = torch.randperm(len(lens) * nb, device=DEV).int().view(len(lens), nb)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(len(lens), hq, d, device=DEV).bfloat16()
+    sinks = torch.tensor([0.5, -20.0, 3.0, 8.0, 0.0, float("-inf")], device=DEV) if with_sinks else None
+
+    def run(splits):
+        return _hip.paged_attention_decode(q, kc, vc, table, sl, d ** -0.5, max(lens), num_splits=splits, sinks=sinks).float()
+    whole = run(1)
+    # weights and the result are each rounded to 2^-9 of a value in both: 4 * 2^-9 of the largest value
+    for splits in (2, 3, 4, 7, 8, 9, 31, 33, 63, 64):
+        assert (run(splits) - whole).abs().max() <= 4 * 2.0 ** -9 * vc.float().abs().max(), splits
+    assert _hip.choose_num_splits(1, 8, 512) == 1 and _hip.choose_num_splits(1, 8, 800) == 12
+    assert _hip.choose_num_splits(64, 8, 4000) == 1 and _hip.choose_num_splits(32, 8, 9000) == 2
+
+
 @pytest.mark.parametrize("dk,dv,hq,bs", [(576, 512, 16, 64), (576, 512, 128, 16), (576, 512, 8, 64), (96, 64, 4, 16),
                                          (96, 64, 48, 32)])
 @pytest.mark.parametrize("dtype,kv8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True),

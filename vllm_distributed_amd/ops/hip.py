@@ -357,12 +357,16 @@ def decode_workspace_floats(max_bs: int, num_heads: int, head_dim: int, num_kv_h
 
 
 def choose_num_splits(batch: int, num_kv_heads: int, max_seq_len: int) -> int:
-    """Enough workgroups to fill 256 CUs twice over, each split >= 512 keys: up to 512 keys one
-    workgroup per (sequence, KV head) finishes in the time the merge kernel of a split takes to launch."""
+    """KV splits of a decode step: one up to 512 keys, else about 512 workgroups of at least 64 keys (512 where the
+    (sequence, KV head) pairs alone are a workgroup for every CU).  The four waves of a workgroup take the keys 32 at a time in turn, so a long context on few
+    workgroups is a serial chain: one sequence of 8 heads over 800 keys takes 12.5 us whole and 8.5 in 12 splits, over 2000
+    keys 14.2 in 3 and 8.9 in 31.  Below 512 keys a merge costs what it saves (400 keys: 9.1 whole, 8.4 in 6; 200: 6.8 and
+    8.2); with a workgroup for every CU a split adds the partial sums (32 x 8 heads over 1000 keys: 22.5 whole, 25.9 in 2)
+    and gives an even end where long contexts differ (32 x 8 heads over about 9000 keys: 354 whole, 311 in 2)."""
     wgs = max(1, batch * num_kv_heads)
-    want = (512 + wgs - 1) // wgs
-    by_len = max(1, max_seq_len // 512)
-    return max(1, min(MAX_SPLITS, want, by_len))
+    if max_seq_len <= 512:
+        return 1
+    return max(1, min(MAX_SPLITS, (512 + wgs - 1) // wgs, max_seq_len // (64 if wgs < 256 else 512)))
 
 
 def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
@@ -1191,11 +1195,12 @@ def mla_rows_ok(k_cache: torch.Tensor, dv: int) -> bool:
 
 def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int, workgroups: int = 256) -> int:
     """KV splits: about one workgroup per CU in total (``workgroups``: two, of the kernel that lets two share a CU) and no
-    split shorter than ~192 keys.  A workgroup streams ~36 GB/s by itself (one group of 32 keys in flight ahead of the one
+    split shorter than two groups of 32 keys.  A workgroup streams ~36 GB/s by itself (one group in flight ahead of the one
     being multiplied), so the chip's bandwidth needs a few hundred of them; beyond that, more splits only add partial sums
-    to write and merge (scripts/dev/mla_split_sweep.py: the fastest count is within ~5 % of this rule from batch 1 to 256)."""
+    to write and merge (scripts/dev/mla_split_sweep.py).  A merge costs ~2 us: 16 heads over 500 keys take 18 us in 2
+    splits, 12.6 in 4, 11.3 in 6; over 3000 keys 17 us in 15 splits, 11.7 in 46."""
     want = -(-workgroups // max(1, tokens * q_tiles))
-    return int(max(1, min(want, max_seq_len // 192, 64)))
+    return int(max(1, min(want, max_seq_len // 64, 64)))
 
 
 def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
