@@ -572,15 +572,16 @@ int launch_prefill(void* out, const void* q, long q_stride, const void* kc, cons
       }();
       const long total = (long)tiles * Hq * num_seqs;
       if (total > (1L << 30)) return -3;
-      const int grid = remap ? (int)((total + 7) / 8 * 8) : (int)total;
+      const int order = remap && num_seqs <= 65535 && tiles <= 65535;       // (see the kernel)
+      const dim3 grid = order ? dim3(Hq, num_seqs, tiles) : dim3(total);
 #define LDS_LAUNCH(PLAIN, BIAS)                                                                                  \
   if (sinks != nullptr || alibi != nullptr)                                                                      \
-    hipLaunchKernelGGL((BIAS<T, KV8>), dim3(grid), dim3(256), 0, s, (T*)out, (const T*)q, q_stride, kc, vc, bt,  \
-                       bt_stride, qsl, seq_lens, sl2, Hq, Hkv, block_size, out_stride, tiles, (int)total, remap, \
+    hipLaunchKernelGGL((BIAS<T, KV8>), grid, dim3(256), 0, s, (T*)out, (const T*)q, q_stride, kc, vc, bt,        \
+                       bt_stride, qsl, seq_lens, sl2, Hq, Hkv, block_size, out_stride, tiles, order, \
                        k_scales, v_scales, window, softcap, sinks, alibi);                                       \
   else                                                                                                           \
-    hipLaunchKernelGGL((PLAIN<T, KV8>), dim3(grid), dim3(256), 0, s, (T*)out, (const T*)q, q_stride, kc, vc, bt, \
-                       bt_stride, qsl, seq_lens, sl2, Hq, Hkv, block_size, out_stride, tiles, (int)total, remap, \
+    hipLaunchKernelGGL((PLAIN<T, KV8>), grid, dim3(256), 0, s, (T*)out, (const T*)q, q_stride, kc, vc, bt,       \
+                       bt_stride, qsl, seq_lens, sl2, Hq, Hkv, block_size, out_stride, tiles, order, \
                        k_scales, v_scales, window, softcap)
       if constexpr (D == 128) { LDS_LAUNCH(paged_prefill_lds_kernel, paged_prefill_lds_bias_kernel); }
       else if constexpr (D == 64) { LDS_LAUNCH(paged_prefill_lds64_kernel, paged_prefill_lds64_bias_kernel); }
