@@ -281,7 +281,7 @@ class DeepseekMoE(FusedMoE):
     def _forward_routed(self, x: torch.Tensor) -> torch.Tensor:
         """The routed experts' weighted sum (unreduced).  On the GPU: router GEMM, one routing kernel, slot sort +
         tile table, row gather, two grouped GEMMs with the activation between them, weighted combine."""
-        tile_rows = self._grouped_tile_rows(x) if x.dim() == 2 else 0
+        tile_rows = self._expert_tile_rows(x) if x.dim() == 2 else 0
         if not tile_rows or self.num_experts > 512 or self.top_k > 16 or self.n_group > 64:
             return super().forward(x, reduce=False)
         topw, topi = self._route_hip(self.router_logits(x))

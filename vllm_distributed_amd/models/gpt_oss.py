@@ -154,7 +154,7 @@ class GptOssMoE(FusedMoE):
 
     def forward(self, x: torch.Tensor, reduce: bool = True, staged: bool = False, deferred: bool = False):
         logits = self.gate(x)
-        tile_rows = self._grouped_tile_rows(x)
+        tile_rows = self._expert_tile_rows(x)
         if tile_rows and x.dim() == 2 and ops.moe_route_fused_ok(logits, self.num_experts, self.top_k):
             out = self._forward_fused_routing(x, logits, tile_rows)
         else:

@@ -211,26 +211,34 @@ class FusedMoE(nn.Module):
         return F.linear(ops.silu_and_mul(F.linear(x, self.w13[e])), self.w2[e])
 
     def _grouped_tile_rows(self, x: torch.Tensor) -> int:
-        """Row-tile size for the grouped HIP GEMMs - dense experts with more than 64 rows each go to the
-        large-batch kernel's grouped form, 256 rows a tile - or 0 to use the per-expert library GEMMs (4-bit
-        experts, and shapes that form does not take, with hundreds of rows each; that path syncs with the
-        host, so it is never taken while a hipGraph is being captured)."""
+        """Row-tile size for the grouped HIP GEMMs, or 0 to use the per-expert library GEMMs (4-bit experts, and
+        shapes that the large-batch kernel's grouped form does not take, with hundreds of rows each; that path
+        syncs with the host, so it is never taken while a hipGraph is being captured)."""
         if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and ops.hip_available()):
             return 0
         if self.quant is None and (self.w13.shape[2] % 128 or self.w2.shape[2] % 128 or self.w13.shape[1] % 16):
             return 0
         cap = 64 if self.qw13 is not None else 128
         avg = x.shape[0] * self.top_k / max(1, self.num_experts)
-        if self.quant is None and avg > 64 and ops.grouped_big_ok(x, self.top_k, self.w13, self.w2):
-            # (64 experts of 2048 x 1408 with 75 rows each: 268 us against 332 in tiles of 128; 8 of 4096 x 14336 with 50:
-            # 676 against 597 in tiles of 64, with 100: 673 against 803)
-            return ops.GROUPED_BIG_ROWS
-        if avg > envs.VDAMD_MOE_GROUPED_MAX_ROWS * cap / 64 and not torch.cuda.is_current_stream_capturing():
+        if (avg > envs.VDAMD_MOE_GROUPED_MAX_ROWS * cap / 64 and not torch.cuda.is_current_stream_capturing()
+                and not self._grouped_big(x)):
             return 0
         for rows in (16, 32, 64, 128):
             if avg <= rows or rows == cap:
                 return rows
         return cap
+
+    def _grouped_big(self, x: torch.Tensor) -> bool:
+        """Whether the experts go to the large-batch kernel's grouped form: dense ones with more than 64 rows each.
+        (64 experts of 2048 x 1408 with 75 rows each: 268 us against 332 in tiles of 128; 8 of 4096 x 14336 with 50:
+        676 against 597 in tiles of 64, with 100: 673 against 803.)"""
+        return (self.quant is None and x.shape[0] * self.top_k > 64 * self.num_experts
+                and ops.grouped_big_ok(x, self.top_k, self.w13, self.w2))
+
+    def _expert_tile_rows(self, x: torch.Tensor) -> int:
+        """``_grouped_tile_rows``, with the large-batch kernel's tiles in place of the largest ones where it takes them."""
+        rows = self._grouped_tile_rows(x)
+        return ops.GROUPED_BIG_ROWS if rows == 128 and self._grouped_big(x) else rows
 
     def _forward_grouped(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor, tile_rows: int,
                          ) -> torch.Tensor:
@@ -303,7 +311,7 @@ class FusedMoE(nn.Module):
     def forward(self, x: torch.Tensor, reduce: bool = True, staged: bool = False, deferred: bool = False):
         # `deferred`: the caller feeds the result to an add + RMSNorm and accepts ``ExpertRows``
         # `staged` (write the partial sums where the next direct all-reduce reads) is a hint only
-        tile_rows = self._grouped_tile_rows(x)
+        tile_rows = self._expert_tile_rows(x)
         logits = None
         if (tile_rows and not self.custom_routing and self.gate.bias is None
                 and getattr(self.gate, "lora", None) is None and self.num_experts <= 512 and self.top_k <= 16):
@@ -471,7 +479,7 @@ class GroupedIdentityMoE(FusedMoE):
 
     def forward(self, x: torch.Tensor, reduce: bool = True, staged: bool = False, deferred: bool = False):
         logits = self.router_logits(x)
-        tile_rows = self._grouped_tile_rows(x)
+        tile_rows = self._expert_tile_rows(x)
         if tile_rows:
             grouped = self.groups if self.keep_groups < self.groups else 1
             topw, topi = ops.moe_topk_grouped(logits, self.gate.e_score_correction_bias, self.top_k, grouped,
