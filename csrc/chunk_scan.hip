@@ -94,6 +94,28 @@ template <int N> __device__ __forceinline__ void dots16(const f32x4* const (&a)[
     for (int i = 0; i < N; ++i) c[i] = mfma4((*a[i])[e], (*b[i])[e], c[i]);
 }
 
+__device__ __forceinline__ bool all_finite(f32x4 v) {
+  return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
+}
+// A lower triangular block (left(i, j / 4, j % 4)) times a right operand with an infinity or a NaN in it.  In the matrix instruction the
+// zeros right of the diagonal would meet it and hand it to the rows in front of its own; here they are left out.
+template <typename F> __device__ __forceinline__ f32x4 lower16(F&& left, f32x4 x) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1                                   // (rare: few registers)
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const float xj = __shfl(x[f], g * 16 + lr, 64);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float l = left(4 * kh + e, g, f);
+        if (4 * g + f <= 4 * kh + e) o[e] += l * xj;
+      }
+    }
+  return o;
+}
+
 // p[0 .. 3], `fill` from `left` on
 template <typename T> __device__ __forceinline__ f32x4 ld4(const T* p, int left, float fill) {
   f32x4 o = {fill, fill, fill, fill};
@@ -555,7 +577,8 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
 #pragma unroll
           for (int J = 0; J < I; ++J)
             acc += dot16(*reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh), X[J]);
-          X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
+          if (__any(!all_finite(acc))) X[I] = lower16([&](int i, int g, int f) { return ti[(16 * I + i) * 20 + 4 * g + f]; }, acc);
+          else X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
           if (keys) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) wp[piece(I * KB + t, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = -X[I][e];
@@ -738,7 +761,29 @@ template <int DP, bool DELTA, int NC> struct Walk {
         }
     }
     // (the lower triangle's blocks; the wave's number is the same for all its lanes)
-    if (wave == 3) {
+    bool finite = true;                            // u of the wave's own rows, which the block on the diagonal meets
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i == wave)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) finite = finite && all_finite(x[i][ct]);
+    if (__any(!finite)) {
+      f32x4 own, u_own[NC];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i < wave)
+#pragma unroll
+          for (int ct = 0; ct < NC; ++ct) os[ct][i & 1] += dot16(r.a[i], x[i][ct]);
+        if (i == wave) {
+          own = r.a[i];
+#pragma unroll
+          for (int ct = 0; ct < NC; ++ct) u_own[ct] = x[i][ct];
+        }
+      }
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct)
+        os[ct][0] += lower16([&](int i, int g, int f) { return __shfl(own[f], g * 16 + i, 64); }, u_own[ct]);
+    } else if (wave == 3) {
       four(r.a, x, os);
     } else {
 #pragma unroll

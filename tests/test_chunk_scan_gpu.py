@@ -149,3 +149,29 @@ def test_many_heads_are_taken_in_turns(monkeypatch):
     monkeypatch.setattr(hip, "CHUNK_SCRATCH_BYTES", 1)
     got = _run(c, True)
     assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("what,value", [("v", float("nan")), ("v", float("inf")), ("k", float("nan")), ("q", float("nan")),
+                                        ("beta", float("nan")), ("dt", float("nan"))])
+@pytest.mark.parametrize("heads,dim,vdim", [(4, 128, 128), (64, 64, 64)])      # tiles of 16 and of 32 value columns
+def test_what_is_not_finite_stays_in_its_row_and_behind(op, what, value, heads, dim, vdim):
+    """A row's NaN or infinity changes nothing in the rows in front of it, nor in other sequences; its own row shows it."""
+    if (what == "beta" and not op.startswith("delta")) or (what == "dt" and op.startswith("linear")):
+        pytest.skip("the recurrence has no such input")
+    new, row, head = [150, 40, 70, 33], 21 + 64, 2                 # the first sequence's second chunk, inside a group of 16
+    c = _case(op, heads, heads, dim, vdim, new, [150, 47, 70, 35], torch.float32, 7)
+    clean, _ = _run(c, True)
+    if what in ("beta", "dt"):
+        c[what][row] = value
+    else:
+        at = {"q": 0, "k": heads * dim, "v": 2 * heads * dim}
+        if op == "state_space":
+            at = {"v": 0, "k": heads * vdim, "q": heads * vdim + heads * dim}
+        c["x"][row, at[what] + head * (vdim if what == "v" else dim) + 5] = value
+    got, _ = _run(c, True)
+    other = torch.ones(sum(new), dtype=torch.bool, device=DEV)
+    other[row:150] = False
+    # (a decay that is no number makes its group multiply out the products between two rows: other roundings)
+    assert _off(got[other], clean[other].double()) < 3e-6
+    assert not torch.isfinite(got[row].view(heads, vdim)[head]).all()
