@@ -94,8 +94,11 @@ template <int N> __device__ __forceinline__ void dots16(const f32x4* const (&a)[
     for (int i = 0; i < N; ++i) c[i] = mfma4((*a[i])[e], (*b[i])[e], c[i]);
 }
 
-__device__ __forceinline__ bool all_finite(f32x4 v) {
-  return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
+// 0, or NaN where v has an infinity or a NaN
+__device__ __forceinline__ float not_finite(f32x4 v, float so_far) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) so_far = fmaf(v[e], 0.f, so_far);
+  return so_far;
 }
 // A lower triangular block (left(i, j / 4, j % 4)) times a right operand with an infinity or a NaN in it.  In the matrix instruction the
 // zeros right of the diagonal would meet it and hand it to the rows in front of its own; here they are left out.
@@ -557,6 +560,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     __syncthreads();
     // columns of [beta b k | beta v], 16 at a time; an accumulator's layout is the right operand's: solved blocks stay in registers
     float* wp = ws + L0.u + a.VP * C;
+    float odd = 0.f;
     for (int t0 = 0; t0 < KB + vt; t0 += KB) {
       const bool keys = t0 == 0;
       if (!keys) {
@@ -564,29 +568,34 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
         values(16 * (t0 - KB));
         __syncthreads();
       }
-      for (int t = wave; t < KB && t0 + t < KB + vt; t += 4) {
-        f32x4 X[4];
+      auto solve = [&](auto apart) {
+        for (int t = wave; t < KB && t0 + t < KB + vt; t += 4) {
+          f32x4 X[4];
 #pragma unroll
-        for (int I = 0; I < 4; ++I) {
-          f32x4 acc;
+          for (int I = 0; I < 4; ++I) {
+            f32x4 acc;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int i = 16 * I + 4 * kh + e;
-            acc[e] = ks[i * LD + 16 * t + lr] * bl[i];
-          }
+            for (int e = 0; e < 4; ++e) {
+              const int i = 16 * I + 4 * kh + e;
+              acc[e] = ks[i * LD + 16 * t + lr] * bl[i];
+            }
 #pragma unroll
-          for (int J = 0; J < I; ++J)
-            acc += dot16(*reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh), X[J]);
-          if (__any(!all_finite(acc))) X[I] = lower16([&](int i, int g, int f) { return ti[(16 * I + i) * 20 + 4 * g + f]; }, acc);
-          else X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
-          if (keys) {
+            for (int J = 0; J < I; ++J)
+              acc += dot16(*reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh), X[J]);
+            if constexpr (apart) X[I] = lower16([&](int i, int g, int f) { return ti[(16 * I + i) * 20 + 4 * g + f]; }, acc);
+            else X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
+            if constexpr (!apart) odd = not_finite(X[I], odd);
+            if (keys) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) wp[piece(I * KB + t, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = -X[I][e];
-          } else {
-            *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 - KB + t) * 4 + I, lane)) = X[I];
+              for (int e = 0; e < 4; ++e) wp[piece(I * KB + t, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = -X[I][e];
+            } else {
+              *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 - KB + t) * 4 + I, lane)) = X[I];
+            }
           }
         }
-      }
+      };
+      solve(std::false_type{});
+      if (__builtin_expect(__any(odd != 0.f), 0)) solve(std::true_type{});
     }
   }
 }
@@ -761,13 +770,13 @@ template <int DP, bool DELTA, int NC> struct Walk {
         }
     }
     // (the lower triangle's blocks; the wave's number is the same for all its lanes)
-    bool finite = true;                            // u of the wave's own rows, which the block on the diagonal meets
+    float odd = 0.f;                               // u of the wave's own rows, which the block on the diagonal meets
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (i == wave)
 #pragma unroll
-        for (int ct = 0; ct < NC; ++ct) finite = finite && all_finite(x[i][ct]);
-    if (__any(!finite)) {
+        for (int ct = 0; ct < NC; ++ct) odd = not_finite(x[i][ct], odd);
+    if (__builtin_expect(__any(odd != 0.f), 0)) {
       f32x4 own, u_own[NC];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
