@@ -168,6 +168,9 @@ __device__ __forceinline__ void wave_sync() {
 template <int CTRL> __device__ __forceinline__ float dpp_mul(float v) {
   return v * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
+__device__ __forceinline__ float turn(float v) {                // of the lane in front, the first of 16 from the last
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
+}
 __device__ __forceinline__ float prefix_product(float v) {       // lanes up to and including this one
   v = dpp_mul<0x111>(v);
   v = dpp_mul<0x112>(v);
@@ -435,25 +438,35 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     da = sa[0] + sa[1];
     dl = sb[0] + sb[1];
   } else {
-    // diag_exact: pairs (i, i - m) of the wave's group; the product of the decays between them grows with m
-    float between[NP];
+    // diag_exact: pairs (i, i - m) of the wave's group; the product of the decays between them grows with m.  The rows i - m and
+    // their decays come by turning the 16 lanes on by one each time, in registers: wave shuffles, which go through LDS, made this
+    // a third of such a call's time (16 heads, dim 128, decays of 3e-4 a row: 8017 rows of the delta rule 545 us so, 445 turned,
+    // 421 where no group comes here; 60 rows of 8 heads 79, 54 and 46).
+    float pa[16], pb[16], between = 1.f, oj = own;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) between[i] = 1.f;
-    for (int m = 0; m < 16; ++m) {
-      const int src = (lane & 48) | ((lr - m) & 15);
-      float sa = 0.f, sb = 0.f;
+    for (int m = 0; m < 16; ++m) pa[m] = pb[m] = 0.f;
+    [[maybe_unused]] float by_row[CHAN ? 1 : 16];
+    if constexpr (!CHAN)
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        [[maybe_unused]] const f32x4 d = dk[CHAN ? kb : 0];
+      for (int m = 0; m < 16; ++m) { by_row[m] = between; between *= oj; oj = turn(oj); }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float kj = __shfl(k[kb][e], src, 64) * between[CHAN ? 4 * kb + e : 0];
-          sa += q[kb][e] * kj;
-          if constexpr (DELTA) sb += k[kb][e] * kj;
-          if constexpr (CHAN) between[4 * kb + e] *= __shfl(d[e], src, 64);
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float kj = k[kb][e], dj = dk[CHAN ? kb : 0][e];
+        between = 1.f;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+          const float kd = kj * (CHAN ? between : by_row[CHAN ? 0 : m]);
+          pa[m] += q[kb][e] * kd;
+          if constexpr (DELTA) pb[m] += k[kb][e] * kd;
+          kj = turn(kj);
+          if constexpr (CHAN) { between *= dj; dj = turn(dj); }
         }
       }
-      if constexpr (!CHAN) between[0] *= __shfl(own, src, 64);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      float sa = pa[m], sb = pb[m];
       sa += __shfl_xor(sa, 16, 64); sa += __shfl_xor(sa, 32, 64);
       sb += __shfl_xor(sb, 16, 64); sb += __shfl_xor(sb, 32, 64);
       // lane (.., i) has the sum of row i, column i - m; as an accumulator, lane (kh, j) has rows 4 kh + e of column j
