@@ -785,10 +785,8 @@ template <int DP, bool DELTA, int NC> struct Walk {
     // (the lower triangle's blocks; the wave's number is the same for all its lanes)
     float odd = 0.f;                               // u of the wave's own rows, which the block on the diagonal meets
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i == wave)
-#pragma unroll
-        for (int ct = 0; ct < NC; ++ct) odd = not_finite(x[i][ct], odd);
+    for (int ct = 0; ct < NC; ++ct)
+      odd = not_finite(DELTA ? at(sh.ul, (16 * ct + lr) * LU + 16 * wave + 4 * kh) : u[ct], odd);
     if (__builtin_expect(__any(odd != 0.f), 0)) {
       f32x4 own, u_own[NC];
 #pragma unroll
