@@ -1,0 +1,23 @@
+"""The rules that choose between kernels, at calls where both sides were measured (no GPU needed)."""
+import pytest
+
+from vllm_distributed_amd.ops import hip
+
+
+@pytest.mark.parametrize("kind,rows,seqs,longest,heads,dim,vdim,chunked", [
+    # decoded rows, whatever their number; prompts of unknown lengths; heads the kernels are not built for
+    (hip.DELTA_CHANNEL, 256, 256, 1, 16, 128, 128, False), (hip.LINEAR_HEAD, 1, 1, 1, 16, 128, 128, False),
+    (hip.DELTA_HEAD, 256, 256, 0, 16, 128, 128, False), (hip.DELTA_HEAD, 2000, 2, 0, 16, 128, 128, True),
+    (hip.LINEAR_CHANNEL, 8000, 1, 8000, 16, 129, 128, False), (hip.STATE_SPACE, 8000, 1, 8000, 16, 192, 64, False),
+    # long prompts (chunked, row by row in us): 423 / 974, 260 / 597, 263 / 705, 223 / 831, 79 / 297, 61 / 87
+    (hip.DELTA_CHANNEL, 8017, 5, 2000, 16, 128, 128, True), (hip.LINEAR_CHANNEL, 8017, 5, 2000, 16, 128, 128, True),
+    (hip.LINEAR_HEAD, 8017, 5, 2000, 16, 128, 128, True), (hip.STATE_SPACE, 8017, 5, 2000, 16, 128, 128, True),
+    (hip.DELTA_CHANNEL, 700, 1, 700, 16, 128, 128, True), (hip.DELTA_CHANNEL, 210, 2, 120, 32, 128, 128, True),
+    # one short prompt: 46 / 38; many prompts of a few chunks: 206 / 181, 370 / 303, 412 / 338
+    (hip.DELTA_CHANNEL, 60, 1, 60, 8, 128, 128, False), (hip.LINEAR_CHANNEL, 6000, 24, 250, 16, 128, 128, False),
+    (hip.LINEAR_HEAD, 8964, 54, 166, 16, 128, 128, False), (hip.DELTA_HEAD, 6720, 48, 140, 16, 128, 128, False),
+    # small heads, where a chunk costs more than its share of the products: 121 / 81, 113 / 69, 160 / 111, 180 / 126
+    (hip.LINEAR_HEAD, 960, 63, 300, 32, 16, 16, False), (hip.LINEAR_CHANNEL, 960, 63, 300, 32, 16, 16, False),
+    (hip.DELTA_CHANNEL, 8990, 58, 155, 16, 16, 16, False), (hip.STATE_SPACE, 960, 63, 300, 32, 64, 64, False)])
+def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest, heads, dim, vdim, chunked):
+    assert hip.chunk_scan_profitable(kind, rows, seqs, longest, heads, dim, vdim) is chunked

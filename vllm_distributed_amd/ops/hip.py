@@ -8,6 +8,7 @@ out-of-bounds access in a hand-written kernel can take the GPU down.
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 from ctypes import c_float, c_int, c_long, c_void_p
 from typing import Optional, Tuple
@@ -1489,23 +1490,39 @@ CHUNK_MIN_ROWS = 48
 CHUNK_SCRATCH_BYTES = 1 << 30
 
 
-def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> bool:
+# Per recurrence, in us.  The chunked kernels: a call, a link of 64 rows of the longest sequence (dim 128; three quarters of it
+# at 64), a chunk and head, the same per 128 x 128 of its keys and values.  The walk row by row: a call, a row of the longest
+# sequence, a row and head, the same per 128 x 128 of the state.
+CHUNK_COSTS = {LINEAR_HEAD: (24.5, 1.15, 0.020, 0.076, 3.1, 0.306, 0.00052, 0.00168),
+               LINEAR_CHANNEL: (24.0, 0.79, 0.036, 0.053, 5.3, 0.270, 0.00063, 0.00115),
+               STATE_SPACE: (21.3, 1.28, 0.027, 0.065, 4.9, 0.340, 0.00073, 0.00224),
+               DELTA_CHANNEL: (36.0, 2.04, 0.025, 0.122, 13.5, 0.396, 0.00068, 0.00239),
+               DELTA_HEAD: (24.0, 1.65, 0.015, 0.140, 15.9, 0.312, 0.00056, 0.00299)}
+
+
+def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int,
+                          aligned: bool = True) -> bool:
     """Whether ``seqs`` sequences with ``rows`` rows in all, at most ``max_rows`` in one (0: unknown), go through the chunked
-    kernels: modelled times in us, fitted on an MI355X over 1 - 24 sequences, 8 - 32 heads and sizes 64 and 128.  The walk
-    row by row is a chain of dependent steps per row of the longest sequence, or where many sequences run bound by
-    issue; a chunk of 64 rows costs a link of a shorter chain and its share of the chip, however few rows it holds (16 heads,
-    dim 128: one prompt of 8000 rows 640 against 3440 us under the delta rule, 24 of 250 rows 348 against 398, 21 of 27
-    rows 84 against 50)."""
+    kernels (``aligned``: their rows can be read 16 bytes at a time): modelled times in us, fitted on an MI355X over calls of
+    1 - 100 sequences, 2 - 64 heads and sizes 16 to 256 with mild and with strong decays.  Of 2680 such calls 18, most of them
+    short, come here although the walk is over 5 % faster, by 27 % at worst.  The walk row by row is a chain of dependent steps
+    per row of the longest sequence, and bound by issue where many sequences run; a chunk of 64 rows costs a link of a shorter
+    chain and its share of the chip, however few rows it holds and however small a head is (16 heads, dim 128: one prompt of 700
+    rows 79 against 297 us under the delta rule per channel, 60 rows of 8 heads 46 against 38; linear attention per channel of
+    24 x 250 rows 206 against 181; 63 sequences of 960 rows in all, 32 heads of 16 x 16: 121 against 81)."""
     longest = max_rows if max_rows > 0 else rows // max(seqs, 1)
     if dim > CHUNK_MAX_DIM or longest < CHUNK_MIN_ROWS:
         return False
-    delta = kind >= DELTA_CHANNEL
-    area = (64 if dim <= 64 else 128) * vdim / 16384
-    walk = (22.0 if delta else 8.0) + max(longest * (0.37 if delta or kind == STATE_SPACE else 0.27),
-                                          rows * heads * area * (0.0032 if delta else 0.0025))
-    chunks = rows / 64 + seqs
-    chunked = 26.0 + longest / 64 * (3.6 if delta else 2.6) + chunks * heads * area * (0.16 if delta else 0.095)
+    call, link, head, area, walk_call, row, row_head, row_area = CHUNK_COSTS[kind]
+    padded = 64 if dim <= 64 else 128
+    chunked = (call + longest / 64 * link * (0.5 + padded / 256)
+               + (rows / 64 + seqs) * heads * (head + area * padded * max(vdim, 32) / 16384)) * (1.0 if aligned else 1.2)
+    walk = walk_call + math.hypot(longest * row, rows * heads * (row_head + row_area * dim * vdim / 16384))
     return chunked < walk
+
+
+def _rows16(x: torch.Tensor) -> bool:
+    return x.stride(0) * x.element_size() % 16 == 0 and x.data_ptr() % 16 == 0
 
 
 def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_bias, a_log, decay, d_skip, num_heads: int,
@@ -1549,7 +1566,7 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
     elif scale != 1.0:
         raise NotImplementedError("a scale on the result needs decays per key channel")
     kind = LINEAR_CHANNEL if decay.dim() == 2 else LINEAR_HEAD
-    if chunk_scan_profitable(kind, t, n, max_query_len, num_heads, dim, vdim) if chunked is None else chunked:
+    if chunk_scan_profitable(kind, t, n, max_query_len, num_heads, dim, vdim, _rows16(x)) if chunked is None else chunked:
         qs = num_heads * dim
         return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None,
                            decay if decay.dim() == 2 else _f32_vec(decay, num_heads, "decay"), None, num_heads, num_heads,
@@ -1832,7 +1849,7 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
     assert tuple(state.shape[1:]) == (h, dim, vdim), (tuple(state.shape), (h, dim, vdim))
     assert slots.shape[0] == b and query_start_loc.shape[0] >= b + 1
     kind = DELTA_HEAD if per_head else DELTA_CHANNEL
-    if (not parts and chunk_scan_profitable(kind, t, b, max_query_len, h, dim, vdim)) if chunked is None else chunked:
+    if (not parts and chunk_scan_profitable(kind, t, b, max_query_len, h, dim, vdim, _rows16(x))) if chunked is None else chunked:
         return _chunk_scan(kind, x, 0, g * dim, 2 * g * dim, beta, dt,
                            _f32_vec(dt_bias, dt.shape[1], "dt_bias"), _f32_vec(a_log, h, "a_log"), None, None, h, g, dim, vdim,
                            state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"),
@@ -1870,7 +1887,7 @@ def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, 
     assert state is not None and state.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (h, n, vdim), (tuple(state.shape), (h, n, vdim))
     assert slots.shape[0] == b and query_start_loc.shape[0] >= b + 1
-    if chunk_scan_profitable(STATE_SPACE, t, b, max_query_len, h, n, int(vdim)) if chunked is None else chunked:
+    if chunk_scan_profitable(STATE_SPACE, t, b, max_query_len, h, n, int(vdim), _rows16(x)) if chunked is None else chunked:
         inner = h * vdim
         return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, _f32_vec(dt_bias, h, "dt_bias"),
                            _f32_vec(a_log, h, "a_log"), None, _f32_vec(d_skip, h, "d_skip"), h, g, n, int(vdim), state,
