@@ -21,3 +21,17 @@ from vllm_distributed_amd.ops import hip
     (hip.DELTA_CHANNEL, 8990, 58, 155, 16, 16, 16, False), (hip.STATE_SPACE, 960, 63, 300, 32, 64, 64, False)])
 def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest, heads, dim, vdim, chunked):
     assert hip.chunk_scan_profitable(kind, rows, seqs, longest, heads, dim, vdim) is chunked
+
+
+@pytest.mark.parametrize("batch,heads,keys,captured,splits", [
+    # (whole against split in us) 13.5 / 18 from Python; in a graph 12.5 / 8.5 and 9.3 / 9.0
+    (1, 8, 800, False, 1), (1, 8, 800, True, 12), (8, 8, 520, True, 1), (1, 8, 512, True, 1), (1, 8, 1, False, 1),
+    # a workgroup for most CUs: 18 / 20 and 20 / 22 in three; 22.5 / 25.9 in two; enough keys: 354 / 311
+    (24, 8, 800, True, 1), (31, 8, 800, True, 1), (24, 8, 1000, False, 1), (32, 8, 1000, True, 1), (32, 8, 9000, False, 2),
+    # 512 workgroups rather than more than that: 5 and 6 of 96 over 1000 keys 14.5 and 16
+    (12, 8, 1000, True, 5), (20, 8, 1400, True, 3), (20, 8, 4000, False, 4), (16, 8, 3000, False, 4), (64, 8, 4000, True, 1), (1, 1, 100000, True, 64)])
+def test_decode_splits(monkeypatch, batch, heads, keys, captured, splits):
+    monkeypatch.setattr(hip, "MAX_SPLITS", 64, raising=False)
+    assert hip.choose_num_splits(batch, heads, keys, captured) == splits
+    # the workspace of a captured step serves every call of its size
+    assert hip.decode_workspace_floats(batch, heads, 128, heads, keys) >= batch * splits * heads * 130

@@ -357,17 +357,24 @@ def decode_workspace_floats(max_bs: int, num_heads: int, head_dim: int, num_kv_h
     return worst * num_heads * (head_dim + 2)
 
 
-def choose_num_splits(batch: int, num_kv_heads: int, max_seq_len: int) -> int:
-    """KV splits of a decode step: one up to 512 keys, else about 512 workgroups of at least 64 keys (512 where the
-    (sequence, KV head) pairs alone are a workgroup for every CU).  The four waves of a workgroup take the keys 32 at a time in turn, so a long context on few
-    workgroups is a serial chain: one sequence of 8 heads over 800 keys takes 12.5 us whole and 8.5 in 12 splits, over 2000
-    keys 14.2 in 3 and 8.9 in 31.  Below 512 keys a merge costs what it saves (400 keys: 9.1 whole, 8.4 in 6; 200: 6.8 and
-    8.2); with a workgroup for every CU a split adds the partial sums (32 x 8 heads over 1000 keys: 22.5 whole, 25.9 in 2)
-    and gives an even end where long contexts differ (32 x 8 heads over about 9000 keys: 354 whole, 311 in 2)."""
+def choose_num_splits(batch: int, num_kv_heads: int, max_seq_len: int, captured: bool = True) -> int:
+    """KV splits of a decode step, ``captured`` in a graph or launched from Python.
+
+    The four waves of a workgroup take the keys 32 at a time in turn, so a long context on few workgroups is a serial chain:
+    where the (sequence, KV head) pairs leave room for three splits each, as many splits of at least 64 keys as make 512
+    workgroups.  One sequence of 8 heads over 800 keys takes 12.5 us whole and 8.5 in 12 splits, over 2000 keys 14.2 in 3 and 8.9
+    in 31.  A merge costs what that saves below about 512 keys, and later the more workgroups there are (64 of them over 520 keys:
+    9.3 whole, 9.0 in 8; 160 over 800 keys 17.5 and 18.5, over 1400 keys 26 in 2 and 24 in 4).  With a workgroup for most CUs a
+    split only adds the partial sums (192 over 800 keys: 18 whole, 20 in 3; 32 x 8 heads over 1000 keys: 22.5 whole, 25.9 in 2)
+    unless contexts are long enough to end unevenly (32 x 8 heads over about 9000 keys: 354 whole, 311 in 2): splits of at least
+    512 keys, and as many as make 512 workgroups or more (20 x 8 heads over 4000 keys: 62.8 in 3, 58.4 in 4).
+    Outside a graph a second launch costs the host 4.5 us (13.5 and 18.0 us a call), more than it saves below 1024 keys."""
     wgs = max(1, batch * num_kv_heads)
-    if max_seq_len <= 512:
-        return 1
-    return max(1, min(MAX_SPLITS, (512 + wgs - 1) // wgs, max_seq_len // (64 if wgs < 256 else 512)))
+    long = min((512 + wgs - 1) // wgs, max_seq_len // 512)
+    if 512 // wgs >= 3:
+        whole = 512 + 3 * wgs if captured else 1024
+        long = 1 if max_seq_len < whole else max(long, min(512 // wgs, max_seq_len // 64))
+    return max(1, min(MAX_SPLITS, long))
 
 
 def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
@@ -398,7 +405,8 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
         out = torch.empty((b, hq, d), dtype=q.dtype, device=q.device)
     assert out.is_contiguous() and out.shape == (b, hq, d)
     if num_splits is None:
-        num_splits = choose_num_splits(b, hkv, min(max_seq_len, window) if window > 0 else max_seq_len)
+        keys = min(max_seq_len, window) if window > 0 else max_seq_len
+        num_splits = choose_num_splits(b, hkv, keys, keys >= 1024 or torch.cuda.is_current_stream_capturing())
     ws_ptr = None
     assert 0 <= num_splits <= MAX_SPLITS       # 0 = the one-wave-per-sequence kernel
     if num_splits > 1:
