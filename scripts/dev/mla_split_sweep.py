@@ -31,4 +31,4 @@ for hq in (16, 32):
             res.append((sp, a.elapsed_time(b) / 20 * 1e3))
         best = min(res, key=lambda r: r[1])
         print(f"Hq={hq:3d} B={batch:4d} ctx={ctx:6d}: " + "  ".join(f"{sp}:{us:.1f}" for sp, us in res)
-              + f"   best {best[0]} chosen {_hip.mla_num_splits(batch, -(-hq // 16), ctx)}", flush=True)
+              + f"   best {best[0]} chosen {_hip.mla_plan(batch, hq, ctx, False, batch, _hip.mla_rows_ok(kc, DV), None, False)}", flush=True)

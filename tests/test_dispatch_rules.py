@@ -35,3 +35,22 @@ def test_decode_splits(monkeypatch, batch, heads, keys, captured, splits):
     assert hip.choose_num_splits(batch, heads, keys, captured) == splits
     # the workspace of a captured step serves every call of its size
     assert hip.decode_workspace_floats(batch, heads, 128, heads, keys) >= batch * splits * heads * 130
+
+
+@pytest.mark.parametrize("tokens,heads,keys,by_token,seqs,rows_ok,captured,plan", [
+    # decoded rows from Python: one launch up to 383 keys (13.6 / 20); in a graph split (12.7 / 10.6)
+    (1, 16, 200, False, 1, True, False, (3, 1)), (1, 16, 200, False, 1, True, True, (3, 3)),
+    (1, 16, 200, False, 1, False, False, (0, 1)), (1, 16, 4000, False, 1, True, False, (3, 62)),
+    # no more workgroups than run at once: 26.8 / 32.6, 93 / 117, 23.7 / 32.5, whole rows 14.5 / 19.7 and 24.7 / 32.8
+    (100, 16, 700, False, 100, True, True, (3, 5)), (160, 16, 3000, False, 160, True, True, (3, 3)),
+    (130, 16, 400, False, 130, True, True, (3, 3)), (15, 128, 200, False, 15, True, True, (3, 1)),
+    (256, 16, 400, False, 256, True, True, (3, 1)), (128, 16, 3100, False, 128, True, True, (3, 4)),
+    # four head tiles a workgroup: 54 / 72, 118 / 149
+    (40, 128, 500, False, 40, True, True, (2, 3)), (100, 128, 700, False, 100, True, True, (2, 1)),
+    # prompts: 47 / 66, 65 / 92, rows of different lengths in two 227 / 269 and 102 / 116; 3 tokens of 16 sequences 50 / 56
+    (200, 16, 700, True, 1, True, False, (1, 5)), (192, 32, 564, True, 3, True, False, (1, 2)),
+    (1000, 16, 1000, True, 2, True, False, (1, 2)), (600, 16, 300, True, 2, True, False, (1, 2)),
+    (700, 16, 700, True, 1, True, False, (1, 2)), (1500, 16, 1500, True, 1, True, False, (1, 1)),
+    (48, 16, 1500, True, 16, True, True, (1, 9)), (32, 16, 300, True, 1, True, False, (1, 4))])
+def test_latent_plan(tokens, heads, keys, by_token, seqs, rows_ok, captured, plan):
+    assert hip.mla_plan(tokens, heads, keys, by_token, seqs, rows_ok, None, captured) == plan

@@ -1203,13 +1203,47 @@ def mla_rows_ok(k_cache: torch.Tensor, dv: int) -> bool:
 
 
 def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int, workgroups: int = 256) -> int:
-    """KV splits: about one workgroup per CU in total (``workgroups``: two, of the kernel that lets two share a CU) and no
-    split shorter than two groups of 32 keys.  A workgroup streams ~36 GB/s by itself (one group in flight ahead of the one
-    being multiplied), so the chip's bandwidth needs a few hundred of them; beyond that, more splits only add partial sums
-    to write and merge (scripts/dev/mla_split_sweep.py).  A merge costs ~2 us: 16 heads over 500 keys take 18 us in 2
-    splits, 12.6 in 4, 11.3 in 6; over 3000 keys 17 us in 15 splits, 11.7 in 46."""
+    """KV splits of the kernel that reads both caches: about one workgroup per CU in total and no split shorter than two groups
+    of 32 keys.  A workgroup streams ~36 GB/s by itself (one group in flight ahead of the one being multiplied), so the chip's
+    bandwidth needs a few hundred of them; beyond that, more splits only add partial sums to write and merge
+    (scripts/dev/mla_split_sweep.py).  A merge costs ~2 us: 16 heads over 500 keys take 21 us in 2 splits, 12.5 in 7."""
     want = -(-workgroups // max(1, tokens * q_tiles))
     return int(max(1, min(want, max_seq_len // 64, 64)))
+
+
+def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows_ok: bool, mode: Optional[int] = None,
+             captured: bool = True) -> Tuple[int, int]:
+    """Kernel (``mla_attention``'s ``mode``, chosen here when None) and KV splits of a step of ``tokens`` rows of up to ``keys``
+    keys from ``seqs`` sequences (``by_token``: rows name theirs), ``captured`` in a graph or launched from Python.
+
+    Splits make as many workgroups as run at once - one per CU of the kernels that share keys between four tiles (1, 2), two of
+    the one over key rows (3) - and not more: what is left over waits for a second round.  Prompt of 200 tokens, 16 heads, 700 keys
+    (50 workgroups): 47 us in 5 splits, 66 in 6; three of 64, 32 heads, 564 keys (102): 65 in 2, 92 in 3; 100 decoded rows of
+    700 keys 26.8 in 5 and 32.6 in 6, 160 of 3000 keys 93 in 3 and 117 in 4.  Splits hold 64 keys, or 128 where more than 64
+    workgroups leave many partial sums (16 rows of 128 heads, 200 keys: 14.5 us whole, 19.7 in 3), 256 where there is a
+    workgroup for every CU (256 rows, 400 keys: 24.7 whole, 32.8 in 2).  Prompts that take most CUs whole still go in two, which
+    evens out their rows of different lengths (two of 500 rows on average behind 500 keys: 269 us whole, 227 in 2; one of 700: 116
+    and 102; though two of exactly 300: 58 and 62).
+    Outside a graph a second launch and its buffers cost the host 6.5 us: up to 383 keys of decoded rows are not split (200
+    keys: 13.6 us whole, 20 in 3; 500 keys 25 and 20)."""
+    q_tiles = -(-heads // 16)
+    if mode is None:
+        # (four head tiles per workgroup need enough workgroups left to fill the chip)
+        mode = 1 if by_token else 2 if q_tiles >= 4 and tokens * q_tiles >= 128 else 3 if rows_ok else 0
+    if mode in (0, 3) and keys < 384 and not captured:
+        return mode, 1
+    if mode == 0:
+        return mode, mla_num_splits(tokens, q_tiles, keys)
+    if mode == 1:
+        wgs = min(tokens, -(-tokens // 4) + seqs - 1) * q_tiles       # (a sequence's tokens start a group of four anywhere)
+    else:
+        wgs = tokens * (-(-q_tiles // 4) if mode == 2 else q_tiles)
+    per, shortest = (512 if mode == 3 else 256) // max(wgs, 1), 64
+    if mode == 1 and 128 < wgs < 256:
+        per = 2
+    if mode == 3 and wgs > 64:
+        shortest = 128 if wgs < 256 else 256
+    return mode, max(1, min(per, keys // shortest, 64))
 
 
 def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
@@ -1239,20 +1273,14 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     if out is None:
         out = torch.empty((t, hq, dv), dtype=q.dtype, device=q.device)
     assert out.stride(2) == 1 and out.stride(1) == dv
-    q_tiles = -(-hq // 16)
-    if mode is None:
-        # (four head tiles per workgroup need enough workgroups left to fill the chip)
-        mode = 1 if token_seq is not None else (2 if q_tiles >= 4 and t * q_tiles >= 128 else 0)
-        if mode == 0 and mla_rows_ok(k_cache, dv):
-            mode = 3
     gate_stride = 0
     if gate is not None:
         assert gate.dim() == 2 and gate.shape[0] >= t and gate.shape[1] == hq and gate.stride(1) == 1 and gate.dtype == q.dtype
         gate_stride = gate.stride(0)
-    if splits is None:
-        keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
-        splits = mla_num_splits(-(-t // 4) if mode == 1 else t, -(-q_tiles // 4) if mode == 2 else q_tiles, keys,
-                                512 if mode == 3 else 256)
+    keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
+    mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
+                          keys >= 384 or torch.cuda.is_current_stream_capturing())
+    splits = best if splits is None else splits
     part_o = part_ml = None
     if splits > 1:
         part_o = torch.empty((t * hq * splits, dv), dtype=torch.float32, device=q.device)
