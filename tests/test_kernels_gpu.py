@@ -1176,6 +1176,40 @@ def test_decode_splits_merge_to_the_unsplit_result(d, with_sinks):
     assert _hip.choose_num_splits(64, 8, 4000) == 1 and _hip.choose_num_splits(32, 8, 9000) == 2
 
 
+@pytest.mark.parametrize("dk,dv,hq,bs,dtype", [(576, 512, 5, 64, torch.bfloat16), (576, 512, 20, 32, torch.float16),
+                                              (320, 256, 16, 32, torch.bfloat16), (320, 256, 33, 64, torch.float16)])
+@pytest.mark.parametrize("window", [0, 19, 70])
+@pytest.mark.parametrize("precise", [False, True])
+@pytest.mark.parametrize("extras", [False, True])
+def test_latent_rows_take_windows_sinks_gates_and_precise_weights(dk, dv, hq, bs, dtype, window, precise, extras):
+    """Decoded rows whose values come from the key rows (the default over these caches) with every option of the op, whole and
+    in splits, some of which no key falls into.  Each weight is rounded to half a unit in its last place unless ``precise``, and
+    the result once: that much of the largest value, each, and half of it again for the scores and sums in 32 bits."""
+    from vllm_distributed_amd.ops import hip as _hip
+    torch.manual_seed(dk + hq + window)
+    lens = [1, 2, 18, 19, 20, 31, 32, 33, 64, 65, 97, 500]
+    per = -(-max(lens) // bs)
+    rows = torch.full(torch_ref.k_cache_shape(len(lens) * per, 1, dk, bs), float("nan"), device=DEV).to(dtype)
+    unread = torch.full(torch_ref.v_cache_shape(len(lens) * per, 1, dv, bs), float("nan"), device=DEV).to(dtype)
+    table = torch.randperm(len(lens) * per, device=DEV).int().view(len(lens), per)
+    for b, n in enumerate(lens):
+        at = torch.arange(n, device=DEV)
+        rows[table[b, at // bs].long(), 0, at % bs] = (torch.randn(n, dk, device=DEV) * 0.7).to(dtype)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = (2 * torch.randn(len(lens), hq, dk, device=DEV)).to(dtype)
+    sinks = torch.randn(hq, device=DEV) if extras else None
+    gate = torch.randn(len(lens), hq + 3, device=DEV).to(dtype)[:, 3:] if extras else None
+    clean = torch.nan_to_num(rows).float()
+    want = torch_ref.latent_row_attention(q.float(), clean, table, None, sl, 0.15, dv, window, sinks,
+                                          None if gate is None else gate.float())
+    half = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    bound = half * (1 if precise else 2) * 1.5 * clean[..., :dv].abs().max()
+    for splits in (None, 1, 2, 7):
+        got = _hip.mla_attention(q, rows, unread, table, None, sl, 0.15, max(lens), splits=splits, precise=precise, window=window,
+                                 sinks=sinks, gate=gate)
+        assert (got.float() - want).abs().max() <= bound, (splits, (got.float() - want).abs().max().item(), bound.item())
+
+
 @pytest.mark.parametrize("dk,dv,hq,bs", [(576, 512, 16, 64), (576, 512, 128, 16), (576, 512, 8, 64), (96, 64, 4, 16),
                                          (96, 64, 48, 32)])
 @pytest.mark.parametrize("dtype,kv8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True),

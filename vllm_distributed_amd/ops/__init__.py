@@ -622,7 +622,11 @@ def mla_cache_write(latent, k_cache, v_cache, slot_mapping):
 
 def mla_attention(q, k_cache, v_cache, block_table, token_seq, seq_lens, scale, max_seq_len, out=None,
                   precise: bool = False, window: int = 0, sinks=None, gate=None):
-    """``precise``: softmax weights with fp32 precision in the weighted sum (models that define them in 32-bit).
+    """``k_cache`` and ``v_cache`` are two forms of ONE latent cache: the value of a position is the first ``DV`` values of its
+    key row, which ``mla_cache_write``, ``mla_prep`` and ``latent_prep`` leave in both.  A kernel reads the values from whichever
+    form suits it (decoded rows over a 16-bit cache from the key rows alone), so other values in ``v_cache`` than those have no
+    defined effect.
+    ``precise``: softmax weights with fp32 precision in the weighted sum (models that define them in 32-bit).
     ``window`` / ``sinks`` / ``gate``: a sliding window, a sink per head in the denominator, a sigmoid gate per
     (token, head) on the output (the matrix-core kernels only)."""
     on_hip = _use_hip(q) and _hip.mla_supported(q.shape[2], v_cache.shape[2] * v_cache.shape[4], q.dtype)

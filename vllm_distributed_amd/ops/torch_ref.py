@@ -404,7 +404,7 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                   token_seq: Optional[torch.Tensor], seq_lens: torch.Tensor, scale: float, max_seq_len: int = 0,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``q[T, Hq, DK]`` against the latent cache -> ``[T, Hq, DV]`` in fp32 arithmetic.  Keys come from the
-    key-row cache, values from the V^T fragment cache (so a test of a kernel against this checks both)."""
+    key-row cache, values from the V^T fragment cache, its other form (so a test of a kernel against this checks both)."""
     t, hq, dk = q.shape
     bs = k_cache.shape[2]
     dv = v_cache.shape[2] * V_ROWS
