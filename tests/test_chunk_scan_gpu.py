@@ -175,3 +175,22 @@ def test_what_is_not_finite_stays_in_its_row_and_behind(op, what, value, heads, 
     # (a decay that is no number makes its group multiply out the products between two rows: other roundings)
     assert _off(got[other], clean[other].double()) < 3e-6
     assert not torch.isfinite(got[row].view(heads, vdim)[head]).all()
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("new", [[700, 300, 1, 1], [900] + [1] * 40])
+def test_the_memory_profile_holds_what_a_step_allocates(op, new):
+    """``chunk_scan_bytes`` (the runner keeps as much aside) covers the peak of a call, also for a step of fewer rows."""
+    from vllm_distributed_amd import ops
+    heads, groups, dim, vdim = 16, 16, 64, 128
+    c = _case(op, heads, groups, dim, vdim, new, new, torch.bfloat16, 9)
+    _run(c, True)
+    state = c["state"].nbytes                                       # (``_run`` works on a copy)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    _run(c, True)
+    torch.cuda.synchronize()
+    used = torch.cuda.max_memory_allocated() - before - state
+    bound = ops.recurrence_bytes(2000, len(new), heads, dim, vdim, op.startswith("delta"))
+    assert 0 < used <= bound + 65536, (used, bound)                 # (offsets and lengths, rounded up to 512 bytes each)

@@ -54,3 +54,27 @@ def test_decode_splits(monkeypatch, batch, heads, keys, captured, splits):
     (48, 16, 1500, True, 16, True, True, (1, 9)), (32, 16, 300, True, 1, True, False, (1, 4))])
 def test_latent_plan(tokens, heads, keys, by_token, seqs, rows_ok, captured, plan):
     assert hip.mla_plan(tokens, heads, keys, by_token, seqs, rows_ok, None, captured) == plan
+
+
+def test_recurrent_layers_report_their_prompt_memory():
+    """What a prompt through a recurrent layer allocates counts in the memory profile, which does not run its kernels."""
+    import torch
+
+    from vllm_distributed_amd import ops
+    from vllm_distributed_amd.models.layers import linear_attention as la
+    from vllm_distributed_amd.worker.model_runner import ModelRunner
+    if not ops.hip_available():
+        pytest.skip("the kernel library is not built")
+    layers = [la.DecayLinearAttention(8, 64, 64, [0.9] * 8, 0), la.GatedDeltaRule(16, 8, 128, 128, 1),
+              la.SelectiveStateSpace(8, 2, 64, 64, 2),
+              la.GatedLinearHeads(256, 4, 64, 64, 16, 16.0, 1e-6, 3, torch.bfloat16)]
+    # (rows + 63 for each sequence) / 64 chunks of 128 KB and more per head, and the fp32 result
+    for layer, heads, vdim in zip(layers, (8, 16, 8, 4), (64, 128, 64, 64)):
+        assert layer.prompt_bytes(16, 16) == 4 * 16 * heads * vdim                       # never chunked
+        assert layer.prompt_bytes(2048, 32) > layer.prompt_bytes(2048, 1) > 32 * heads * 48 * 1024
+        assert layer.prompt_bytes(1 << 17, 64) <= hip.CHUNK_SCRATCH_BYTES + 4 * (1 << 17) * heads * vdim
+    runner = ModelRunner.__new__(ModelRunner)
+    runner.model, runner.max_num_reqs, runner.is_gpu = torch.nn.ModuleList(layers + [torch.nn.Linear(2, 2)]), 32, True
+    assert runner._prompt_bytes(2048) == layers[1].prompt_bytes(2048, 32) == max(m.prompt_bytes(2048, 32) for m in layers)
+    runner.is_gpu = False
+    assert runner._prompt_bytes(2048) == 0

@@ -46,6 +46,10 @@ class DecayLinearAttention(nn.Module):
     def bind_state(self, state: Optional[torch.Tensor]) -> None:
         self.state = state
 
+    def prompt_bytes(self, rows: int, seqs: int) -> int:
+        """What a step's kernels allocate at most, for the memory profile (no pass through here sees it)."""
+        return ops.recurrence_bytes(rows, seqs, self.num_heads, self.dim, self.vdim)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         md = get_forward_context().attn_metadata
         if md is None:                    # memory-profiling pass: no state bound
@@ -72,6 +76,9 @@ class GatedLinearHeads(nn.Module):
         self.a2_bias = nn.Parameter(torch.zeros(heads * dim, dtype=torch.float32), requires_grad=False)
         self.norm = nn.Parameter(torch.zeros(vdim, dtype=torch.float32), requires_grad=False)
         self.slot_state = SlotState((heads, dim, vdim), torch.float32)
+
+    def prompt_bytes(self, rows: int, seqs: int) -> int:
+        return ops.recurrence_bytes(rows, seqs, self.heads, self.dim, self.vdim)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """``x[T, sum(sizes)]`` (rows may be strided) -> the gated heads ``[T, heads * vdim]``."""
@@ -108,6 +115,9 @@ class GatedDeltaRule(nn.Module):
     def per_slot_shape(self) -> Tuple[int, int, int]:
         return (self.heads, self.dim, self.vdim)
 
+    def prompt_bytes(self, rows: int, seqs: int) -> int:
+        return ops.recurrence_bytes(rows, seqs, self.heads, self.dim, self.vdim, True)
+
     def forward(self, x: torch.Tensor, beta: torch.Tensor, dt: torch.Tensor, state: Optional[torch.Tensor]) -> torch.Tensor:
         md = get_forward_context().attn_metadata
         if md is None or state is None:   # memory-profiling pass: no state bound
@@ -143,6 +153,9 @@ class SelectiveStateSpace(nn.Module):
 
     def per_slot_shape(self) -> Tuple[int, int, int]:
         return (self.heads, self.n_state, self.vdim)
+
+    def prompt_bytes(self, rows: int, seqs: int) -> int:
+        return ops.recurrence_bytes(rows, seqs, self.heads, self.n_state, self.vdim)
 
     def forward(self, x: torch.Tensor, dt: torch.Tensor, state: Optional[torch.Tensor]) -> torch.Tensor:
         md = get_forward_context().attn_metadata

@@ -736,6 +736,13 @@ def add_layer_norm(y, residual, weight, bias, eps: float, out_dtype):
     return torch_ref.add_layer_norm(y, residual, weight, bias, eps, out_dtype)
 
 
+def recurrence_bytes(rows: int, seqs: int, heads: int, dim: int, vdim: int, delta: bool = False) -> int:
+    """Bound on what a recurrent mixer's kernels allocate for a step of ``rows`` rows of up to ``seqs`` sequences (0 on the CPU)."""
+    if not hip_available():
+        return 0
+    return _hip.chunk_scan_bytes(_hip.DELTA_CHANNEL if delta else _hip.LINEAR_CHANNEL, rows, seqs, heads, dim, vdim)
+
+
 def decay_linear_attention(x, num_heads: int, dim: int, vdim: int, decay, state, slots, query_start_loc, seq_lens,
                            silu: bool = True, max_query_len: int = 0, scale: float = 1.0):
     """Linear attention with a decay per head, or per row, head and key channel (``decay`` 2-D), and a per-request fp32

@@ -1561,6 +1561,23 @@ def _rows16(x: torch.Tensor) -> bool:
     return x.stride(0) * x.element_size() % 16 == 0 and x.data_ptr() % 16 == 0
 
 
+def _chunk_workspace(kind: int, rows: int, seqs: int, heads: int, dim: int, vdim: int) -> Tuple[int, int, int]:
+    """A bound on a step's chunks, the floats of workspace per head, and the heads taken at a time under
+    ``CHUNK_SCRATCH_BYTES``."""
+    chunks = (rows + 63 * min(seqs, rows)) // 64
+    floats = int(_LIB.vdamd_chunk_scan_floats(kind, dim, vdim)) * chunks
+    return chunks, floats, min(heads, max(1, CHUNK_SCRATCH_BYTES // (4 * floats)))
+
+
+def chunk_scan_bytes(kind: int, rows: int, seqs: int, heads: int, dim: int, vdim: int) -> int:
+    """What a recurrence over up to ``rows`` rows of up to ``seqs`` sequences allocates at most: workspace and result."""
+    out = 4 * rows * heads * vdim
+    if dim > CHUNK_MAX_DIM or rows < CHUNK_MIN_ROWS:
+        return out
+    _, floats, at_a_time = _chunk_workspace(kind, rows, max(seqs, 1), heads, dim, vdim)
+    return out + 4 * floats * at_a_time
+
+
 def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_bias, a_log, decay, d_skip, num_heads: int,
                 groups: int, dim: int, vdim: int, state, slots, query_start_loc, seq_lens, silu: bool, eps: float,
                 scale: float) -> torch.Tensor:
@@ -1570,9 +1587,7 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
     out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
     if t == 0 or b == 0:
         return out
-    chunks = (t + 63 * min(b, t)) // 64
-    floats = int(_LIB.vdamd_chunk_scan_floats(kind, dim, vdim)) * chunks
-    heads = min(num_heads, max(1, CHUNK_SCRATCH_BYTES // (4 * floats)))
+    chunks, floats, heads = _chunk_workspace(kind, t, b, num_heads, dim, vdim)
     ws = torch.empty(heads * floats, dtype=torch.float32, device=x.device)
     for h0 in range(0, num_heads, heads):
         _check(_LIB.vdamd_chunk_scan(

@@ -372,6 +372,7 @@ class ModelRunner:
         ids = torch.zeros(t, dtype=torch.int32, device=self.device)
         pos = torch.arange(t, dtype=torch.int32, device=self.device) % self.max_model_len
         set_forward_context(None, pos)
+        held = torch.empty(self._prompt_bytes(t), dtype=torch.uint8, device=self.device)    # next to everything of the pass
         inter = None
         if not self.pp.is_first_rank:
             h = self.model_config.hidden_size
@@ -382,8 +383,14 @@ class ModelRunner:
             n = min(self.max_num_reqs, t)
             self.model.compute_logits(out[:n])
         self.tp.end_step()
+        del held
         if self.is_gpu:
             torch.cuda.synchronize()
+
+    def _prompt_bytes(self, tokens: int) -> int:
+        """The most a layer whose kernels the profiling pass does not reach allocates in a step (one layer at a time)."""
+        return max((m.prompt_bytes(tokens, self.max_num_reqs) for m in self.model.modules() if hasattr(m, "prompt_bytes")),
+                   default=0) if self.is_gpu else 0
 
     def initialize_kv_cache(self, num_blocks: int) -> None:
         spec = self.get_kv_cache_spec()
