@@ -135,6 +135,33 @@ def test_chunks_match_the_recurrence_in_64_bits(op, strong, dim, vdim, new, extr
     assert torch.equal(out, again) and torch.equal(state, state2)
 
 
+def _many(n):
+    """Lengths of ``n`` sequences around the chunk's 64 rows, some empty, and rows before them."""
+    new = [(0, 1, 17, 64, 65, 5, 0, 33)[i % 8] for i in range(n)]
+    return new, [(0, 3, 70)[i % 3] if m else 0 for i, m in enumerate(new)]
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("heads,dim,vdim,new,extra,dtype,pad", [
+    (16, 128, 128, [70, 64, 130, 65], [0, 9, 0, 3], torch.bfloat16, 8),        # 64 pairs and more: tiles of 32 columns
+    (16, 128, 112, [33, 200, 1, 64], [0, 2, 5, 0], torch.float16, 0),          # the last tile half empty
+    (32, 64, 200, [66, 90], [4, 0], torch.float32, 0),                         # values wider than a pass over them
+    (4, 64, 128, [129, 20], [0, 7], torch.bfloat16, 0),
+    (4, 64, 128, [80, 65], [1, 0], torch.float32, 3),                          # the same without vector loads
+    (2, 128, 256, [65, 100], [0, 6], torch.bfloat16, 1),
+    (4, 64, 64, *_many(70), torch.bfloat16, 8),                                # more sequences than a wave has lanes
+    (8, 128, 128, *_many(131), torch.bfloat16, 0)])
+def test_wide_tiles_wide_values_and_many_sequences(op, heads, dim, vdim, new, extra, dtype, pad):
+    """The bound of ``test_chunks_match_the_recurrence_in_64_bits``."""
+    groups = heads // 2 if op in ("state_space", "delta_head") else heads
+    c = _case(op, heads, groups, dim, vdim, new, [n + e for n, e in zip(new, extra)], dtype, 17, False, pad)
+    want, want_state = _rows64(c)
+    out, state = _run(c, True)
+    assert _off(out, want) < 3e-6 and _off(state, want_state) < 3e-6, (_off(out, want), _off(state, want_state))
+    untouched = [i for i in range(c["state"].shape[0]) if i not in [int(x) for x, n in zip(c["slots"], new) if n]]
+    assert torch.equal(state[untouched], c["state"][untouched])
+
+
 @pytest.mark.parametrize("op", OPS)
 def test_chunks_are_no_less_exact_than_the_walk(op):
     c = _case(op, 4, 4, 128, 128, [700, 300], [700, 420], torch.bfloat16, 3, False, 0)

@@ -523,12 +523,14 @@ def test_grouped_gemm_in_large_tiles(dtype, T, k, E, H, I, local):
     (1, torch.float32, 2.0, 0), (2, torch.bfloat16, 2.0, 1), (7, torch.float16, 2.0, 3),
     (1023, torch.float32, 2.0, 1), (4097, torch.bfloat16, 0.0, 0),           # more equal weights than the list holds
     (50257, torch.bfloat16, 2.5, 1), (50257, torch.float32, 0.02, 2),        # misaligned rows; bins cut twice and three times
-    (128256, torch.bfloat16, 0.3, 0), (151936, torch.float32, 30.0, 0)])
+    (128256, torch.bfloat16, 0.3, 0), (151936, torch.float32, 30.0, 0),
+    ((1 << 22) + 77, torch.bfloat16, 1.0, 1)])                               # counts and sums in words of their own
 def test_sample_draws_inside_the_interval_of_the_kept_distribution(V, dtype, spread, offset):
-    """The drawn entry's stretch of the descending cumulative distribution (64-bit) holds ``u`` times the kept mass.
-    A weight's relative error is under 1e-5 (an fp32 exponent of at most a hundred, rounded) and the filter's border
-    may move by one entry."""
-    B = 40
+    """The drawn entry's stretch of the descending cumulative distribution (64-bit) holds ``u`` times the kept mass, and the entry
+    is kept.  A weight's relative error is under 1e-5 (an fp32 exponent of at most a hundred, rounded): so much of the kept mass
+    is the slack, the filters' borders are taken once 1e-5 lower and once higher, and entries of other logits whose weights are
+    that close may change places."""
+    B = 40 if V < 1 << 20 else 8
     logits = (_rand(B, V + offset, dtype=torch.float32, scale=spread) + 0.0).to(dtype)[:, offset:]
     masked = torch.rand(B, V, device=DEV) < 0.3
     masked[:, V // 2] = False
@@ -546,19 +548,49 @@ def test_sample_draws_inside_the_interval_of_the_kept_distribution(V, dtype, spr
     p = torch.softmax(logits.double() / torch.where(greedy, 1.0, temperature).double().unsqueeze(1), -1)
     sp, si = p.sort(dim=-1, descending=True, stable=True)
     cum = sp.cumsum(-1)
-    keep = torch.arange(V, device=DEV).unsqueeze(0) < torch.where(top_k <= 0, V, top_k).unsqueeze(1)
-    keep &= ((cum - sp) < top_p.double().unsqueeze(1)) | (top_p >= 1).unsqueeze(1)
-    keep &= sp >= min_p.double().unsqueeze(1) * sp[:, :1]
-    keep[:, 0] = True
-    kept = keep.sum(-1)
-    total = cum.gather(1, (kept - 1).unsqueeze(1)).squeeze(1)
-    border = torch.where(kept < V, sp.gather(1, (kept - 1).unsqueeze(1)).squeeze(1), 0.0)
+
+    def kept(off):
+        keep = torch.arange(V, device=DEV).unsqueeze(0) < torch.where(top_k <= 0, V, top_k).unsqueeze(1)
+        keep &= ((cum - sp) < (top_p.double() + off).unsqueeze(1)) | (top_p >= 1).unsqueeze(1)
+        keep &= sp >= (min_p.double() * (1 - off)).unsqueeze(1) * sp[:, :1]
+        keep[:, 0] = True
+        n = keep.sum(-1)
+        return n, cum.gather(1, (n - 1).unsqueeze(1)).squeeze(1)
+    (_, low), (most, high) = kept(-1e-5), kept(1e-5)
     rank = (si == got.unsqueeze(1)).to(torch.int8).argmax(-1)
+    mine = sp.gather(1, rank.unsqueeze(1)).squeeze(1)
+    border = sp.gather(1, (most - 1).unsqueeze(1)).squeeze(1)
     hi = cum.gather(1, rank.unsqueeze(1)).squeeze(1)
-    lo = hi - sp.gather(1, rank.unsqueeze(1)).squeeze(1)
-    slack, target = 1e-5 + border, u.double() * total
-    ok = (target >= lo - slack) & (target <= hi + slack) & (rank <= kept)
-    assert (ok | greedy).all(), (got[~ok].tolist(), rank[~ok].tolist(), kept[~ok].tolist())
+    near = ((sp - mine.unsqueeze(1)).abs() <= 1e-5 * mine.unsqueeze(1)) & (sp != mine.unsqueeze(1))
+    slack = 1e-5 * high + torch.where(near, sp, 0.0).sum(-1)
+    ok = (u.double() * high >= hi - mine - slack) & (u.double() * low <= hi + slack)
+    ok &= (rank < most) | ((mine != border) & (mine >= border * (1 - 1e-5)))
+    assert (ok | greedy).all(), (got[~ok].tolist(), rank[~ok].tolist(), most[~ok].tolist())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sample_cuts_bins_of_many_entries_where_the_filter_does(dtype):
+    """Borders inside more entries of one histogram bin than the list holds (4096), drawn with ``u`` at both ends of the kept
+    mass and in the middle: equal weights, kept and drawn in the order of their indices, and (fp32) weights that differ by
+    5e-6 each, drawn in descending order; the masses are multiples of one weight, or far from any border by comparison."""
+    V, few = 8192, torch.tensor([1e-6, 0.5, 1 - 1e-6], device=DEV)
+
+    def draw(row, k, top_p=1.0):
+        full = lambda v, t=torch.float32: torch.full((3,), v, device=DEV, dtype=t)
+        return ops.sample(row.expand(3, -1).contiguous(), full(1.0), full(k, torch.int32), full(top_p), full(0.0), few).tolist()
+    row = torch.full((V,), 1.25, device=DEV, dtype=dtype)
+    assert draw(row, 50) == [0, 24, 49] and draw(row, 5000) == [0, 2499, 4999] and draw(row, 0) == [0, 4095, V - 1]
+    assert draw(row, 0, 0.25) == [0, 1023, 2047] and draw(row, 1024, 0.25) == [0, 511, 1023]
+    row[7000], row[:100] = 3.0, -1.0                                # a likelier one, and some behind the cut
+    assert draw(row, 4500)[0::2] == [7000, 100 + 4498]
+    if dtype == torch.float32:
+        order = torch.randperm(6000, device=DEV)
+        row = torch.full((V,), -9.0, device=DEV)
+        row[order] = torch.log(torch.linspace(0.62, 0.60, 6000, device=DEV, dtype=torch.float64)).float()     # one bin: 19/32 .. 20/32
+        row[V - 1] = 0.0
+        first, _, last = draw(row, 5001)
+        assert first == V - 1 and last == order[4999].item()
+        assert draw(row, 5001, 0.5)[0] == V - 1
 
 
 def test_sample_of_rows_without_a_distribution_is_entry_zero():
