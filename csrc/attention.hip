@@ -545,8 +545,8 @@ int launch_decode(void* out, float* ws, const void* q, long q_stride, const void
                      alibi);
   HIP_LAUNCH_CHECK();
   if (num_splits > 1) {
-    hipLaunchKernelGGL((decode_reduce_kernel<T, D>), dim3(Hq, B), dim3(split_merge_threads(D, num_splits)), 0, s, (T*)out, part_o, part_ml, Hq,
-                       num_splits, out_stride, sinks);
+    hipLaunchKernelGGL((decode_reduce_kernel<T, D>), dim3(Hq, B), dim3(split_merge_threads(D, num_splits)), 0, s, (T*)out,
+                       part_o, part_ml, Hq, num_splits, out_stride, sinks);
     HIP_LAUNCH_CHECK();
   }
   return 0;

@@ -41,7 +41,8 @@ struct ChunkArgs {
   const float* dt_bias;
   const float* a_log;
   const float* decay;                              // [H] (LINEAR_HEAD) or [T, H * dim] (LINEAR_CHANNEL)
-  float* ws;                                       // per (chunk, head of the launch): A | b q | G k, transposed | b_64 | U, transposed | -W
+  float* ws;                                       // per (chunk, head of the launch): A | b q | G k, transposed | b_64 | U,
+                                                   // transposed | -W
   long ws_stride;
   const int* qsl;
   int B, H, G, dim, vdim, VP;                      // VP: vdim up to a multiple of 32
@@ -100,8 +101,8 @@ __device__ __forceinline__ float not_finite(f32x4 v, float so_far) {
   for (int e = 0; e < 4; ++e) so_far = fmaf(v[e], 0.f, so_far);
   return so_far;
 }
-// A lower triangular block (left(i, j / 4, j % 4)) times a right operand with an infinity or a NaN in it.  In the matrix instruction the
-// zeros right of the diagonal would meet it and hand it to the rows in front of its own; here they are left out.
+// A lower triangular block (left(i, j / 4, j % 4)) times a right operand with an infinity or a NaN in it.  In the matrix
+// instruction the zeros right of the diagonal would meet it and hand it to the rows in front of its own; here they are left out.
 template <typename F> __device__ __forceinline__ f32x4 lower16(F&& left, f32x4 x) {
   const int lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -127,7 +128,6 @@ template <typename T> __device__ __forceinline__ f32x4 ld4(const T* p, int left,
   return o;
 }
 
-// one step of a running product over the 16 lanes of a row; lanes without a source multiply by one
 // Sixteen rows of a wave, `cols` values each, on their way into LDS: a row is read by neighbouring lanes, 16 bytes each, whole
 // lines at a time (read as operands, four lanes to a row, every line is asked for again while it is on its way: the kernel then
 // spends 65 % of its time in such stalls of the vector cache).
@@ -165,6 +165,7 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// one step of a running product over the 16 lanes of a row; lanes without a source multiply by one
 template <int CTRL> __device__ __forceinline__ float dpp_mul(float v) {
   return v * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }

@@ -274,8 +274,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //     leaves a lane with 16 neighbouring ones of them.
 // The 16-byte pieces of a row are XOR-ed with bits 1, 3 and 4 of the key's number (the 16 rows of a K fragment then lie in
 // 16 different places of the LDS's 256 bytes).
-// Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 109 us against 211 through both
-// caches (441 and 833 MB; the chip's copy rate would take 91).
+// Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 109 us against 211
+// through both caches (441 and 833 MB; the chip's copy rate would take 91).
 // ---------------------------------------------------------------------------------------------------------------
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void mla_lds_void;

@@ -74,18 +74,7 @@ __global__ __launch_bounds__(ST) void argmax_kernel(int* __restrict__ out, const
   }
 }
 
-// block-wide (sum, count) reduction; result broadcast to all threads
-__device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  a = wave_sum(a); b = wave_sum(b);
-  if (lane == 0) { red[wid] = a; red[16 + wid] = b; }
-  __syncthreads();
-  float ta = lane < 16 ? red[lane] : 0.f, tb = lane < 16 ? red[16 + lane] : 0.f;
-  ta = wave_sum(ta); tb = wave_sum(tb);
-  __syncthreads();
-  a = ta; b = tb;
-}
-
+// block-wide maximum, broadcast to all threads
 __device__ __forceinline__ float block_max(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   v = wave_max(v);
@@ -237,7 +226,7 @@ __global__ __launch_bounds__(ST) void sample_kernel(int* __restrict__ out, const
   __shared__ Hist<WIDE> h1, h2;
   __shared__ unsigned long long list[CAP];
   __shared__ SampleShared s;
-  __shared__ float red[32];
+  __shared__ float red[16];
   __shared__ int s_idx;
   const int b = blockIdx.x;
   const T* row = logits + b * stride;
