@@ -19,7 +19,7 @@
 // logarithms: a product between two rows of different groups of 16 is (from the start of i's group up to i) * (whole groups
 // between) * (behind j to the end of its group), each at most 1 where decays are, so nothing overflows; inside a group it
 // is the quotient of two products from the group's start, unless one of those is smaller than 2^-96 or larger than 2^96,
-// where the group's 120 pairs are multiplied out (diag_exact).
+// where the group's 120 pairs are multiplied out (diag_exact).  A head's products are formed so in 64 bits (2^-960, 2^960).
 #include "common.h"
 #include <math.h>
 #include <type_traits>
@@ -77,22 +77,30 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 
 // The product over 16 reduction indices.  Every product here is summed up in such pieces, each from zero, that are then
 // added in turns to two sums: one accumulator running through 192 terms loses twice the digits that the row by row kernels
-// lose (relative error in norm of the delta rule's output against 64 bits 4.1e-7; so 2.2e-7, row by row 2.2e-7).
+// lose (relative error in norm of the delta rule's output against 64 bits 4.1e-7; so 2.2e-7, row by row 2.2e-7).  What the
+// outputs are sums of (A, and o itself) comes in halves of eight: ten prompts of 450 to 4265 rows under the delta rule per head
+// are then 1.00 times as far off as row by row on average (1.05 without, 1.07 with the decays in A's factors as well), for
+// 1 to 2 % of the time (55.0 -> 56.2 us on average, 8017 rows per channel 403 -> 409); in u and the state it would cost 5 %.
 __device__ __forceinline__ f32x4 dot16(f32x4 a, f32x4 b) {
-  f32x4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) c = mfma4(a[e], b[e], c);
-  return c;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  return mfma4(a[1], b[1], mfma4(a[0], b[0], zero)) + mfma4(a[3], b[3], mfma4(a[2], b[2], zero));
 }
 
 // N such products side by side: a matrix instruction of these takes 32 cycles and its result another few, which the others fill
-template <int N> __device__ __forceinline__ void dots16(const f32x4* const (&a)[N], const f32x4* const (&b)[N], f32x4 (&c)[N]) {
+template <int N, bool HALVES = false> __device__ __forceinline__ void dots16(const f32x4* const (&a)[N], const f32x4* const (&b)[N], f32x4 (&c)[N]) {
+  f32x4 d[N];
 #pragma unroll
-  for (int i = 0; i < N; ++i) c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < N; ++i) c[i] = d[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int i = 0; i < N; ++i) c[i] = mfma4((*a[i])[e], (*b[i])[e], c[i]);
+    for (int i = 0; i < N; ++i) {
+      f32x4& to = HALVES && e >= 2 ? d[i] : c[i];
+      to = mfma4((*a[i])[e], (*b[i])[e], to);
+    }
+  if constexpr (HALVES)
+#pragma unroll
+    for (int i = 0; i < N; ++i) c[i] += d[i];
 }
 
 // 0, or NaN where v has an infinity or a NaN
@@ -250,7 +258,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   __shared__ __attribute__((aligned(16))) float mn[DELTA ? C * LM : 4];      // -beta L
   __shared__ __attribute__((aligned(16))) float ti[DELTA ? 4 * 16 * 20 : 4]; // inverses of the diagonal blocks
   __shared__ float bl[C];
-  __shared__ double td[4];
+  __shared__ double td[4], sd[CHAN ? 1 : C];       // per head: products of whole groups, and of the group's decays behind a row
   int seq, c;
   if (!locate(a.qsl, a.B, blockIdx.x, seq, c)) return;           // (the same for every wave)
   const int hh = blockIdx.y, h = a.h0 + hh, g = h / (a.H / a.G);
@@ -338,7 +346,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     if (kh == 0) bl[r] = ok ? sigmoid_f(ldf((const T*)a.beta + row * a.beta_stride + h)) : 0.f;
   }
   float own = 1.f;                                 // per head: the row's decay,
-  double pd = 1.0;                                 // the product of the group's up to the row
+  double pd = 1.0, after = 1.0;                    // the products of the group's up to the row, and behind it
   if constexpr (CHAN) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
@@ -358,8 +366,9 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
       }
     }
     // (a head's decay can be the same number in every row: rounded products of it would be off by the same amount in every
-    // chunk.  They are formed in 64 bits and rounded once)
-    double after = __shfl_down((double)own, 1, 16);
+    // chunk.  They are formed in 64 bits, and A and L take the one between their rows, rounded once, behind their sums; with
+    // decays in the factors, which rounds each term twice, the error against 64 bits was up to 1.25 times the walk's)
+    after = __shfl_down((double)own, 1, 16);
     if (lr == 15) after = 1.0;
     pd = own;
 #pragma unroll
@@ -368,14 +377,15 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
       if (lr >= o) pd *= before;
       if (lr + o < 16) after *= behind;
     }
-    p[0] = (float)pd;
-    s[0] = (float)after;
     if (lane == 15) td[wave] = pd;
+    if (kh == 0) sd[r] = after;
   }
   bool far = false;                                // a product too small or too large to divide by
+  if constexpr (CHAN) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    far = far || !(fabsf(p[i]) >= 0x1p-96f && fabsf(p[i]) <= 0x1p96f);
+    for (int i = 0; i < NP; ++i) far = far || !(fabsf(p[i]) >= 0x1p-96f && fabsf(p[i]) <= 0x1p96f);
+  } else {
+    far = !(fabs(pd) >= 0x1p-960 && fabs(pd) <= 0x1p960);
   }
   if (lr == 15) {
     if constexpr (CHAN) {
@@ -384,31 +394,38 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
         *reinterpret_cast<f32x4*>(tl + wave * DP + 16 * kb + 4 * kh) = f32x4{p[4 * kb], p[4 * kb + 1], p[4 * kb + 2], p[4 * kb + 3]};
     }
   }
-  auto P = [&](int kb, int e) { return p[CHAN ? 4 * kb + e : 0]; };
-  auto Q = [&](int kb, int e) { return s[CHAN ? 4 * kb + e : 0]; };
+  [[maybe_unused]] auto P = [&](int kb, int e) { return p[CHAN ? 4 * kb + e : 0]; };
+  // per head: the products of the group's decays up to the rows of a lane's accumulator
+  [[maybe_unused]] double pr[4];
+  if constexpr (!CHAN)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pr[e] = __shfl(pd, 4 * kh + e, 16);
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
-    f32x4 v;
+    f32x4 v = k[kb];
+    if constexpr (CHAN)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = k[kb][e] * Q(kb, e);
+      for (int e = 0; e < 4; ++e) v[e] *= s[4 * kb + e];
     *reinterpret_cast<f32x4*>(ks + r * LD + 16 * kb + 4 * kh) = v;
   }
   __syncthreads();
   // G k up to the chunk's end, transposed: the wave's rows, a piece per 16 channels
   {
-    double behind = 1.0;
-    if constexpr (!CHAN)
+    [[maybe_unused]] float end[4];                 // per head: the products of the decays behind those rows
+    if constexpr (!CHAN) {
+      double behind = 1.0;
       for (int b = wave + 1; b < 4; ++b) behind *= td[b];
 #pragma unroll
+      for (int e = 0; e < 4; ++e) end[e] = (float)(sd[16 * wave + 4 * kh + e] * behind);
+    }
+#pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      float after = 1.f;
+      float groups = 1.f;
       if constexpr (CHAN)
-        for (int b = wave + 1; b < 4; ++b) after *= tl[b * DP + 16 * kb + lr];
-      else
-        after = (float)behind;
+        for (int b = wave + 1; b < 4; ++b) groups *= tl[b * DP + 16 * kb + lr];
       f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = ks[(16 * wave + 4 * kh + e) * LD + 16 * kb + lr] * after;
+      for (int e = 0; e < 4; ++e) v[e] = ks[(16 * wave + 4 * kh + e) * LD + 16 * kb + lr] * (CHAN ? groups : end[e]);
       *reinterpret_cast<f32x4*>(ws + L0.kt + piece(kb * 4 + wave, lane)) = v;
     }
     if ((int)threadIdx.x < DP) {
@@ -422,22 +439,26 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   f32x4 da = zero, dl = zero;
   if (!exact_diag) {
     f32x4 sa[2] = {zero, zero}, sb[2] = {zero, zero};
-    const float over = (float)(1.0 / pd);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      f32x4 kd, qp, kp;
+      f32x4 kd = k[kb];
+      if constexpr (CHAN)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        kd[e] = CHAN ? k[kb][e] / P(kb, e) : k[kb][e] * over;
-        qp[e] = q[kb][e] * P(kb, e);
-        kp[e] = k[kb][e] * P(kb, e);
-      }
-      sa[kb & 1] += dot16(qp, kd);
-      if constexpr (DELTA) sb[kb & 1] += dot16(kp, kd);
-      if constexpr (CHAN) { q[kb] = qp; k[kb] = kp; }
+        for (int e = 0; e < 4; ++e) {
+          kd[e] /= P(kb, e);
+          q[kb][e] *= P(kb, e);
+          k[kb][e] *= P(kb, e);
+        }
+      sa[kb & 1] += dot16(q[kb], kd);
+      if constexpr (DELTA) sb[kb & 1] += dot16(k[kb], kd);
     }
     da = sa[0] + sa[1];
     dl = sb[0] + sb[1];
+    if constexpr (!CHAN) {
+      const double over = 1.0 / pd;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { da[e] *= (float)(pr[e] * over); dl[e] *= (float)(pr[e] * over); }
+    }
   } else {
     // diag_exact: pairs (i, i - m) of the wave's group; the product of the decays between them grows with m.  The rows i - m and
     // their decays come by turning the 16 lanes on by one each time, in registers: wave shuffles, which go through LDS, made this
@@ -484,21 +505,27 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
         for (int e = 0; e < 4; ++e) { q[kb][e] *= P(kb, e); k[kb][e] *= P(kb, e); }
   }
   // (blocks to the left, nearest first: after each of them its whole product joins the left operands, which end as b q and b k)
+  double whole = 1.0;                              // per head: of the groups between
   for (int J = wave - 1; J >= 0; --J) {
     f32x4 sa[2] = {zero, zero}, sb[2] = {zero, zero};
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const f32x4 b = *reinterpret_cast<const f32x4*>(ks + (16 * J + lr) * LD + 16 * kb + 4 * kh);
-      sa[kb & 1] += dot16(CHAN ? q[kb] : q[kb] * (float)pd, b);
-      if constexpr (DELTA) sb[kb & 1] += dot16(CHAN ? k[kb] : k[kb] * (float)pd, b);
+      sa[kb & 1] += dot16(q[kb], b);
+      if constexpr (DELTA) sb[kb & 1] += dot16(k[kb], b);
       if constexpr (CHAN) {
         const f32x4 t = *reinterpret_cast<const f32x4*>(tl + J * DP + 16 * kb + 4 * kh);
         q[kb] *= t;
         k[kb] *= t;
       }
     }
-    if constexpr (!CHAN) pd *= td[J];
-    const f32x4 va = sa[0] + sa[1], vl = sb[0] + sb[1];
+    f32x4 va = sa[0] + sa[1], vl = sb[0] + sb[1];
+    if constexpr (!CHAN) {
+      const double left = whole * sd[16 * J + lr];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { va[e] *= (float)(pr[e] * left); vl[e] *= (float)(pr[e] * left); }
+      whole *= td[J];
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = 16 * wave + 4 * kh + e;
@@ -508,7 +535,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   }
   if constexpr (!CHAN)
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) { q[kb] *= (float)pd; k[kb] *= (float)pd; }
+    for (int kb = 0; kb < KB; ++kb) { q[kb] *= (float)(pd * whole); k[kb] *= (float)(pd * whole); }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int i = 4 * kh + e;
@@ -691,17 +718,17 @@ template <int DP, bool DELTA, int NC> struct Walk {
     __builtin_amdgcn_sched_barrier(0);
   }
   // o[ct][0 / 1] += the products of left operands l[0 .. 3] with right ones x[0 .. 3][ct], four chains of instructions side by side
-  static __device__ __forceinline__ void four(const f32x4* l, const f32x4 (&x)[4][NC], f32x4 (&o)[NC][2]) {
+  template <bool HALVES> static __device__ __forceinline__ void four(const f32x4* l, const f32x4 (&x)[4][NC], f32x4 (&o)[NC][2]) {
     if constexpr (NC == 1) {
       f32x4 d[4];
-      dots16<4>({&l[0], &l[1], &l[2], &l[3]}, {&x[0][0], &x[1][0], &x[2][0], &x[3][0]}, d);
+      dots16<4, HALVES>({&l[0], &l[1], &l[2], &l[3]}, {&x[0][0], &x[1][0], &x[2][0], &x[3][0]}, d);
       o[0][0] += d[0] + d[1];
       o[0][1] += d[2] + d[3];
     } else {
 #pragma unroll
       for (int i = 0; i < 4; i += 2) {
         f32x4 d[4];
-        dots16<4>({&l[i], &l[i], &l[i + 1], &l[i + 1]}, {&x[i][0], &x[i][1], &x[i + 1][0], &x[i + 1][1]}, d);
+        dots16<4, HALVES>({&l[i], &l[i], &l[i + 1], &l[i + 1]}, {&x[i][0], &x[i][1], &x[i + 1][0], &x[i + 1][1]}, d);
 #pragma unroll
         for (int ct = 0; ct < NC; ++ct) o[ct][i >> 1] += d[ct] + d[2 + ct];
       }
@@ -732,7 +759,7 @@ template <int DP, bool DELTA, int NC> struct Walk {
 #pragma unroll
       for (int kb = 0; kb < KB; kb += 4) {
         read_four<LD>(sl, kb, x);
-        four(&r.w[kb], x, us);
+        four<false>(&r.w[kb], x, us);
       }
 #pragma unroll
       for (int ct = 0; ct < NC; ++ct)
@@ -751,7 +778,7 @@ template <int DP, bool DELTA, int NC> struct Walk {
       f32x4 add[NC][2];
 #pragma unroll
       for (int ct = 0; ct < NC; ++ct) add[ct][0] = add[ct][1] = zero;
-      four(r.k[t], x, add);
+      four<false>(r.k[t], x, add);
 #pragma unroll
       for (int ct = 0; ct < NC; ++ct) S[t][ct] = S[t][ct] * r.b[t] + (add[ct][0] + add[ct][1]);
     }
@@ -768,7 +795,7 @@ template <int DP, bool DELTA, int NC> struct Walk {
 #pragma unroll
     for (int kb = 0; kb < KB; kb += 4) {
       read_four<LD>(sl, kb, x);
-      four(&r.q[kb], x, os);
+      four<true>(&r.q[kb], x, os);
     }
     load_first(r, c + 1);
     if constexpr (DELTA) {
@@ -805,7 +832,7 @@ template <int DP, bool DELTA, int NC> struct Walk {
       for (int ct = 0; ct < NC; ++ct)
         os[ct][0] += lower16([&](int i, int g, int f) { return __shfl(own[f], g * 16 + i, 64); }, u_own[ct]);
     } else if (wave == 3) {
-      four(r.a, x, os);
+      four<true>(r.a, x, os);
     } else {
 #pragma unroll
       for (int kb = 0; kb < 3; ++kb)
