@@ -406,7 +406,8 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
     assert out.is_contiguous() and out.shape == (b, hq, d)
     if num_splits is None:
         keys = min(max_seq_len, window) if window > 0 else max_seq_len
-        num_splits = choose_num_splits(b, hkv, keys, keys >= 1024 or torch.cuda.is_current_stream_capturing())
+        # (whole up to 512 keys and the same from 1024 on: asking costs 0.4 us)
+        num_splits = choose_num_splits(b, hkv, keys, keys >= 1024 or keys > 512 and torch.cuda.is_current_stream_capturing())
     ws_ptr = None
     assert 0 <= num_splits <= MAX_SPLITS       # 0 = the one-wave-per-sequence kernel
     if num_splits > 1:
@@ -1279,7 +1280,7 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         gate_stride = gate.stride(0)
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
-                          keys >= 384 or torch.cuda.is_current_stream_capturing())
+                          keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
     splits = best if splits is None else splits
     part_o = part_ml = None
     if splits > 1:
