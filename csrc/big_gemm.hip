@@ -30,10 +30,11 @@
 //  * Grouped form (sparse experts, rows sorted by expert): a table names each row tile's weight matrix, first row and
 //    rows; W's buffer descriptor moves on with the tile being staged.  Units of two row tiles and about eight columns go
 //    round the XCDs: the 11 or 8 tile columns of a narrow expert would not divide over the XCDs, nor the four pairs of row
-//    tiles of a few wide ones; neighbouring row tiles are mostly one expert's.  Table entries without rows (experts held elsewhere, the table's end) are skipped.
-//    36006 rows over 64 experts of 2048 x 1408 (gate and up with SiLU*mul, then down): 434 and 229 us against 979 + 50
-//    (activation) and 517 us of 128-row tiles with W straight from memory (skinny_gemm.hip), 530 us of matrix
-//    instructions at the rate of a large product.
+//    tiles of a few wide ones; neighbouring row tiles are mostly one expert's.  Table entries without rows (experts held
+//    elsewhere, the table's end) are skipped.
+//    36006 rows over 64 experts of 2048 x 1408 (gate and up with SiLU*mul, then down), traced: 416 - 464 and 234 - 267 us against
+//    979 + 50 (activation) and 517 us of 128-row tiles with W straight from memory (skinny_gemm.hip); 530 us of matrix
+//    instructions at the rate of the library's 8192^3 product.  Partial tiles are multiplied whole: 768 rows for 563.
 //  * Workgroup -> tiles: bands of 8 row tiles; inside a band each XCD owns a range of tile columns and
 //    its 32 workgroups hold an 8 x 4 block of tiles at a time, sharing x and W panels in that XCD's L2
 //    (81 % L2 hit rate measured).

@@ -214,7 +214,7 @@ __device__ void sort_list(unsigned long long* list, int n) {
 // Masses are whole multiples of a bin's last bit, added up in 64-bit integers and doubles: no result depends on the
 // order of additions.
 // A row is read three or four times; a bisection over the bits of both thresholds reads it up to 70 times (256 rows of
-// 128256 bf16 logits, every kind of filter among them: 117 us here, 5456 us so; one pass over these logits at the rate
+// 128256 bf16 logits, every kind of filter among them: 112 - 117 us here, 5.2 - 6.1 ms so; one pass over them at the rate
 // of a large copy: 14 us).  What is left is the LDS atomics of the counting pass (25 us), two sorts of about a thousand entries
 // (10 us each) and the scans.  One row takes 46 - 80 us: it is one compute unit's work.
 template <typename T, bool WIDE>
