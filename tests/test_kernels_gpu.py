@@ -593,6 +593,41 @@ def test_sample_cuts_bins_of_many_entries_where_the_filter_does(dtype):
         assert draw(row, 5001, 0.5)[0] == V - 1
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,offset", [(1, 0), (7, 3), (511, 1), (519, 0), (8192, 0), (50257, 1), (128256, 0), (151936, 5), ((1 << 23) + 9, 0)])
+def test_sample_of_counted_patterns_is_the_one_of_the_same_values_in_32_bits(V, offset, dtype):
+    """16-bit rows go by how often each pattern occurs, 32-bit ones by their weights: the same weights, so the same tokens.
+    Rows: ordinary, of few distinct values, masked with the lowest value and with minus infinity, of more equal values than a
+    16-bit count holds, of subnormal values, with a NaN, under a temperature that makes all weights alike and a negative one."""
+    B = 33
+    g = torch.Generator(DEV).manual_seed(V)
+    x = (torch.randn(B, V + offset, generator=g, device=DEV) * 2.5).to(dtype)[:, offset:]
+    masked = torch.rand(V, generator=g, device=DEV) < 0.97
+    masked[V // 2] = False
+    x[1] = (x[1] * 2).round() / 2
+    x[2][masked] = torch.finfo(dtype).min
+    x[3][masked] = float("-inf")
+    x[4][masked] = 0.25                                             # 124 thousand of the longer rows
+    x[5] = 1.0
+    x[6] = x[6] * torch.finfo(dtype).tiny * 0.1
+    x[7][V // 3] = float("nan")
+    x[8][V // 3] = float("inf")
+    x[9] = float("-inf")
+    x[10] = torch.finfo(dtype).min
+    i = torch.arange(B, device=DEV)
+    temperature = 0.4 + 1.5 * torch.rand(B, generator=g, device=DEV)
+    temperature[11:14], temperature[14:17], temperature[17] = 1e7, -0.7, 0.0
+    x[15][V // 3], x[16][masked] = float("nan"), torch.finfo(dtype).max
+    top_k = torch.where(i % 3 == 0, 50, torch.where(i % 3 == 1, 0, int(0.7 * V) + 1)).to(torch.int32)
+    top_p = torch.where(i % 4 == 0, 1.0, torch.where(i % 4 == 1, 0.3, 0.95)).float()
+    min_p = torch.where(i % 5 == 0, 0.05, 0.0).float()
+    for _ in range(3):
+        u = torch.rand(B, generator=g, device=DEV).clamp(1e-6, 1 - 1e-6)
+        got = ops.sample(x, temperature, top_k, top_p, min_p, u)
+        want = ops.sample(x.float(), temperature, top_k, top_p, min_p, u)
+        assert torch.equal(got, want), (got.tolist(), want.tolist())
+
+
 def test_sample_of_rows_without_a_distribution_is_entry_zero():
     """Rows of nothing but minus infinity, with a NaN or with an infinity: token 0, no hang, neighbours unharmed."""
     logits = _rand(4, 5000, dtype=torch.float32, scale=2.0)
