@@ -34,7 +34,11 @@
 //    elsewhere, the table's end) are skipped.
 //    36006 rows over 64 experts of 2048 x 1408 (gate and up with SiLU*mul, then down), traced: 416 - 464 and 234 - 267 us against
 //    979 + 50 (activation) and 517 us of 128-row tiles with W straight from memory (skinny_gemm.hip); 530 us of matrix
-//    instructions at the rate of the library's 8192^3 product.  Partial tiles are multiplied whole: 768 rows for 563.
+//    instructions at the rate of the library's 8192^3 product.  Partial tiles are multiplied whole: 768 rows for 563.  Neither that
+//    nor the first read of an expert's weights alone is the bound: without the multiplications of empty sub-tiles the time stays
+//    the same (and the plain form loses 3.5 %), and so it does with every unit's K loop begun at another place.
+//    The first product reads the rows it multiplies where they are, through the sorted list: a gather in front of it wrote
+//    147 MB of them (42 us), the product itself is as fast.
 //  * Workgroup -> tiles: bands of 8 row tiles; inside a band each XCD owns a range of tile columns and
 //    its 32 workgroups hold an 8 x 4 block of tiles at a time, sharing x and W panels in that XCD's L2
 //    (81 % L2 hit rate measured).
@@ -63,10 +67,11 @@ __host__ __device__ __forceinline__ int bg_column_groups(int ntn) { return ntn >
 
 // VAR bit 0: 8-byte stores (one per fragment) instead of the paired 16-byte ones.
 // GROUPED: tiles [ntm, 3] = (weight matrix, first row, rows <= 256; 0 = nothing), matrices w_group elements apart.
-template <typename T, int EPI, int VAR, bool GROUPED = false>
+// GATHER (grouped form): row r of the product is row src[r] of x; src holds at least eight rows.
+template <typename T, int EPI, int VAR, bool GROUPED = false, bool GATHER = false>
 __global__ __launch_bounds__(BG_THREADS) void big_gemm_kernel(
     const T* x, long xs, const T* w, long ws, T* out, long os, const T* res, long rs, int M, int N, int K,
-    int ntm, int ntn, int up_row, const int* __restrict__ tiles, long w_group) {
+    int ntm, int ntn, int up_row, const int* __restrict__ tiles, long w_group, const int* __restrict__ src, int x_rows) {
 #if defined(__HIP_DEVICE_COMPILE__)      // the buffer-descriptor builtins exist in the device pass only
   using V8 = typename Vec8<T>::type;
   using V4 = typename Vec4<T>::type;
@@ -125,7 +130,7 @@ __global__ __launch_bounds__(BG_THREADS) void big_gemm_kernel(
 
   // ---- staging: this wave moves pieces 2 wid and 2 wid + 1 (8 rows x 128 B each) of every half-tile
   unsigned offA[2][2], offB[2][2];          // [half][piece] byte offsets of this lane's 16 bytes
-  const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x), 0, (int)((long)M * xs * 2), 0x00020000);
+  const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x), 0, (int)((long)(GATHER ? x_rows : M) * xs * 2), 0x00020000);
   auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w), 0, (int)((long)N * ws * 2), 0x00020000);
   auto set_stage_tile = [&](int tl) {
     if constexpr (GROUPED)
@@ -142,13 +147,29 @@ __global__ __launch_bounds__(BG_THREADS) void big_gemm_kernel(
     const int nb0 = EPI == BG_EPI_SILU_MUL ? tn * 128 : tn * 256;
     const int nb1 = EPI == BG_EPI_SILU_MUL ? up_row + tn * 128 : tn * 256 + 128;
     const int nl0 = EPI == BG_EPI_SILU_MUL ? up_row : N;
+    // the row of x behind each row of the product.  A piece's eight come by a scalar load (a vector load would have to be waited
+    // for together with all of the half-tiles in flight) from a place where eight exist, and each lane picks its own.
+    auto x_row = [&](int first, int r8) {
+      const int row = min(first + r8, mend - 1);
+      if constexpr (!GATHER) return row;
+      const int base = min(min(first, mend - 1), M - 8), at = row - base;
+      int rows8[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) rows8[e] = src[base + e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) asm("" : "+s"(rows8[e]));      // (or the choice becomes the address of a vector load)
+      int v = rows8[0];
+#pragma unroll
+      for (int e = 1; e < 8; ++e) v = at == e ? rows8[e] : v;
+      return v;
+    };
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = 8 * (2 * wid + i) + (ln >> 3);
       const int c = (ln & 7) ^ ((r >> 1) & 7);
       // (all byte offsets fit 32 bits: checked on the host)
-      offA[0][i] = ((unsigned)min(m0 + r, mend - 1) * (unsigned)xs + 8 * c) * 2;
-      offA[1][i] = ((unsigned)min(m0 + 128 + r, mend - 1) * (unsigned)xs + 8 * c) * 2;
+      offA[0][i] = ((unsigned)x_row(m0 + 8 * (2 * wid + i), ln >> 3) * (unsigned)xs + 8 * c) * 2;
+      offA[1][i] = ((unsigned)x_row(m0 + 128 + 8 * (2 * wid + i), ln >> 3) * (unsigned)xs + 8 * c) * 2;
       offB[0][i] = ((unsigned)min(nb0 + r, nl0 - 1) * (unsigned)ws + 8 * c) * 2;
       offB[1][i] = ((unsigned)min(nb1 + r, N - 1) * (unsigned)ws + 8 * c) * 2;
     }
@@ -364,20 +385,20 @@ int launch(void* out, long os, const void* x, long xs, const void* w, long ws, c
   const int per = ntm * ((ntn + 7) / 8);                     // most tiles any XCD gets
   const int grid = 8 * (per < bg_num_cus() / 8 ? per : bg_num_cus() / 8);
   big_gemm_kernel<T, EPI, VAR><<<grid, BG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os,
-                                                            (const T*)res, rs, M, N, K, ntm, ntn, up_row, nullptr, 0);
+                                                            (const T*)res, rs, M, N, K, ntm, ntn, up_row, nullptr, 0, nullptr, 0);
   HIP_LAUNCH_CHECK();
   return 0;
 }
 
-template <typename T, int EPI>
+template <typename T, int EPI, bool GATHER>
 int launch_grouped(void* out, long os, const void* x, long xs, const void* w, long ws, long w_group, const int* tiles, int ntm,
-                   int M, int N, int K, int up_row, hipStream_t st) {
+                   int M, int N, int K, int up_row, const int* src, int x_rows, hipStream_t st) {
   const int ntn = EPI == BG_EPI_SILU_MUL ? (up_row + 127) / 128 : (N + 255) / 256;
   const int groups = bg_column_groups(ntn);
   const int per = ((ntm + 1) / 2 * groups + 7) / 8 * 2 * ((ntn + groups - 1) / groups);    // most entries of any XCD's list
   const int grid = 8 * (per < bg_num_cus() / 8 ? per : bg_num_cus() / 8);
-  big_gemm_kernel<T, EPI, 0, true><<<grid, BG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os, nullptr, 0, M,
-                                                                N, K, ntm, ntn, up_row, tiles, w_group);
+  big_gemm_kernel<T, EPI, 0, true, GATHER><<<grid, BG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os, nullptr, 0,
+                                                                        M, N, K, ntm, ntn, up_row, tiles, w_group, src, x_rows);
   HIP_LAUNCH_CHECK();
   return 0;
 }
@@ -420,25 +441,29 @@ VDAMD_API int vdamd_big_gemm(void* out, long out_stride, const void* x, long x_s
 }
 
 // Row-grouped form: out rows [tiles[i][1], + tiles[i][2]) = epilogue(x rows . w[tiles[i][0]]^T), tiles [num_tiles, 3] on the
-// device, at most 256 rows each (0: skipped), every row inside the M of x and out; w [groups, N, K] with matrices w_group
+// device, at most 256 rows each (0: skipped), every row inside the M of x and out (src != null, epi 2: of src, whose entries are
+// the rows of x [x_rows], M >= 8); w [groups, N, K] with matrices w_group
 // elements apart.  epi 0 or 2 as above; rows of no tile stay as they are.
 VDAMD_API int vdamd_big_gemm_grouped(void* out, long out_stride, const void* x, long x_stride, const void* w, long w_stride,
-                                     long w_group, const int* tiles, int num_tiles, int M, int N, int K, int epi, int dtype,
-                                     void* stream) {
+                                     long w_group, const int* tiles, int num_tiles, const int* src, int x_rows, int M, int N,
+                                     int K, int epi, int dtype, void* stream) {
   if (M <= 0 || num_tiles <= 0) return 0;
   if (K % 128 || N % 16 || (epi == BG_EPI_SILU_MUL && N % 32) || (epi != BG_EPI_NONE && epi != BG_EPI_SILU_MUL)) return -1;
   if ((x_stride | w_stride | out_stride | w_group) % 8) return -5;
+  if (src != nullptr && (epi != BG_EPI_SILU_MUL || M < 8 || x_rows <= 0)) return -4;
   const long lim = (1L << 32) - 64;
-  if ((long)M * x_stride * 2 >= lim || (long)N * w_stride * 2 >= lim || (long)M * out_stride * 2 >= lim) return -7;
+  if ((long)(src != nullptr ? x_rows : M) * x_stride * 2 >= lim || (long)N * w_stride * 2 >= lim || (long)M * out_stride * 2 >= lim) return -7;
   if (((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) % 16) return -8;
   hipStream_t st = (hipStream_t)stream;
-#define BG_GO(T)                                                                                                        \
-  return epi == BG_EPI_NONE ? launch_grouped<T, BG_EPI_NONE>(out, out_stride, x, x_stride, w, w_stride, w_group, tiles,  \
-                                                             num_tiles, M, N, K, 0, st)                                  \
-                            : launch_grouped<T, BG_EPI_SILU_MUL>(out, out_stride, x, x_stride, w, w_stride, w_group,     \
-                                                                 tiles, num_tiles, M, N, K, N / 2, st)
+#define BG_FORM(T, EPI, GATHER) \
+  launch_grouped<T, EPI, GATHER>(out, out_stride, x, x_stride, w, w_stride, w_group, tiles, num_tiles, M, N, K, N / 2, src, x_rows, st)
+#define BG_GO(T)                                                 \
+  return epi == BG_EPI_NONE ? BG_FORM(T, BG_EPI_NONE, false)     \
+         : src == nullptr   ? BG_FORM(T, BG_EPI_SILU_MUL, false) \
+                            : BG_FORM(T, BG_EPI_SILU_MUL, true)
   if (dtype == DT_BF16) BG_GO(bf16_t);
   if (dtype == DT_F16) BG_GO(f16_t);
 #undef BG_GO
+#undef BG_FORM
   return -3;
 }

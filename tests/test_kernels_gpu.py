@@ -519,6 +519,49 @@ def test_grouped_gemm_in_large_tiles(dtype, T, k, E, H, I, local):
     assert torch.equal(seen, mine) and torch.equal(y[~seen], filler[~seen])
 
 
+@pytest.mark.parametrize("T,k,E,H,I,local,pad", [
+    (8, 1, 3, 128, 16, None, 0), (3, 3, 3, 128, 16, None, 8), (700, 3, 10, 512, 384, (2, 5), 0), (513, 1, 2, 256, 128, None, 24),
+    (900, 2, 4, 384, 2176, None, 0)])
+def test_grouped_gemm_reads_rows_where_they_are(T, k, E, H, I, local, pad):
+    """``x[src_row]`` read by the kernel against the same rows gathered first: the same bits; rows of no tile stay."""
+    from vllm_distributed_amd.ops import hip
+    torch.manual_seed(T)
+    topi = _rand(T, E, dtype=torch.float32).topk(k, -1).indices.to(torch.int32).contiguous()
+    start, count = local or (0, -1)
+    src, inv, tiles = hip.moe_align(topi, E, ops.GROUPED_BIG_ROWS, start, count)
+    x = _rand(T, H + pad)[:, :H]                                    # (rows further apart than they are long)
+    w13 = _rand(count if local else E, 2 * I, H, scale=H ** -0.5)
+    filler = torch.full((T * k, I), 7.0, device=DEV, dtype=x.dtype)
+    want = hip.grouped_gemm(x.index_select(0, src), w13, tiles, ops.GROUPED_BIG_ROWS, out=filler.clone(), silu_mul=True)
+    got = hip.grouped_gemm(x, w13, tiles, ops.GROUPED_BIG_ROWS, out=filler.clone(), silu_mul=True, src_row=src)
+    assert torch.equal(got, want)
+    odd = _rand(T, H + 1)[:, :H]                                    # rows that the kernel cannot read: gathered
+    assert not hip.grouped_gather_ok(odd, src) and not hip.grouped_gather_ok(x[:1].expand(T, H), src)
+    want = hip.grouped_gemm(odd.index_select(0, src), w13, tiles, ops.GROUPED_BIG_ROWS, silu_mul=True)
+    got = ops.grouped_gate_up_silu(odd, tiles, ops.GROUPED_BIG_ROWS, w13, src)
+    for _, r0, n in tiles.tolist():
+        assert torch.equal(got[r0:r0 + n], want[r0:r0 + n])
+
+
+@pytest.mark.parametrize("T,k,E,tile_rows,local", [(1, 1, 1, 16, None), (300, 6, 64, 64, None), (2047, 1, 3, 256, None),
+                                                   (1024, 2, 1000, 16, (3, 500)), (2049, 3, 8, 256, (4, 4)), (9000, 6, 64, 256, None)])
+def test_moe_align_sorts_the_slots_of_any_number_of_workgroups(T, k, E, tile_rows, local):
+    from vllm_distributed_amd.ops import hip
+    g = torch.Generator(DEV).manual_seed(T)
+    topi = torch.randint(0, E, (T, k), generator=g, device=DEV, dtype=torch.int32)
+    topi[:T // 3, 0] = E // 2
+    start, count = local or (0, -1)
+    src, inv, tiles = hip.moe_align(topi, E, tile_rows, start, count)
+    assert torch.equal(inv.long().sort().values, torch.arange(T * k, device=DEV))
+    sorted_e = torch.empty(T * k, dtype=torch.int32, device=DEV)
+    sorted_e[inv.long()] = topi.reshape(-1)
+    assert torch.equal(sorted_e, topi.reshape(-1).sort().values)
+    assert torch.equal(src[inv.long()].long(), torch.arange(T * k, device=DEV) // k)
+    _, want = ops.moe_align(topi.long(), E, tile_rows, start, count)
+    used = want[:, 2] > 0
+    assert torch.equal(tiles[used], want[used]) and int(tiles[:, 2].sum()) == int(want[:, 2].sum())
+
+
 @pytest.mark.parametrize("V,dtype,spread,offset", [
     (1, torch.float32, 2.0, 0), (2, torch.bfloat16, 2.0, 1), (7, torch.float16, 2.0, 3),
     (1023, torch.float32, 2.0, 1), (4097, torch.bfloat16, 0.0, 0),           # more equal weights than the list holds

@@ -287,7 +287,7 @@ class DeepseekMoE(FusedMoE):
         topw, topi = self._route_hip(self.router_logits(x))
         local = self.local_experts if self.expert_parallel else -1
         src_row, inv, tiles = ops.moe_align_fused(topi, self.num_experts, tile_rows, self.expert_start, local)
-        y = self._experts_grouped(x.index_select(0, src_row), tiles, tile_rows)
+        y = self._experts_grouped(x, src_row, tiles, tile_rows)
         return ops.moe_combine(y, topw, topi, inv, self.expert_start, local)
 
     def forward(self, x: torch.Tensor, reduce: bool = True, staged: bool = False) -> torch.Tensor:

@@ -266,12 +266,14 @@ class FusedMoE(nn.Module):
         inv[order] = torch.arange(order.numel(), device=order.device)
         return y.index_select(0, inv).view(t, k, -1).sum(dim=1)      # fixed order: deterministic
 
-    def _experts_grouped(self, xs: torch.Tensor, tiles: torch.Tensor, tile_rows: int) -> torch.Tensor:
+    def _experts_grouped(self, x: torch.Tensor, src_row: Optional[torch.Tensor], tiles: torch.Tensor, tile_rows: int) -> torch.Tensor:
+        """Experts over rows sorted by expert: ``x[src_row]``, or ``x`` itself."""
         if self.qw13 is not None:
+            xs = x if src_row is None else x.index_select(0, src_row)
             h = ops.grouped_linear(xs, tiles, tile_rows, qw=self.qw13, sz=self.sz13, alpha=self.alpha13)
             return ops.grouped_linear(h, tiles, tile_rows, qw=self.qw2, sz=self.sz2, alpha=self.alpha2,
                                       silu_mul=True)
-        act = ops.grouped_gate_up_silu(xs, tiles, tile_rows, self.w13)
+        act = ops.grouped_gate_up_silu(x, tiles, tile_rows, self.w13, src_row)
         return ops.grouped_linear(act, tiles, tile_rows, weight=self.w2)
 
     def _forward_fused_routing(self, x: torch.Tensor, logits: torch.Tensor, tile_rows: int, deferred: bool = False):
@@ -284,13 +286,13 @@ class FusedMoE(nn.Module):
             # decode-sized batch: top-k, slot sort, tile table and the row gather are one launch
             topw, topi, inv, tiles, xs = ops.moe_route_small(logits, x, self.top_k, self.renormalize, tile_rows,
                                                              self.expert_start, local)
-            y = self._experts_grouped(xs, tiles, tile_rows)
+            y = self._experts_grouped(xs, None, tiles, tile_rows)
             if deferred:
                 return ExpertRows(y, topw, topi, inv, self.expert_start, local)
             return ops.moe_combine(y, topw, topi, inv, self.expert_start, local)
         topw, topi = ops.moe_topk(logits, self.top_k, self.renormalize)
         src_row, inv, tiles = ops.moe_align_fused(topi, self.num_experts, tile_rows, self.expert_start, local)
-        y = self._experts_grouped(x.index_select(0, src_row), tiles, tile_rows)
+        y = self._experts_grouped(x, src_row, tiles, tile_rows)
         return ops.moe_combine(y, topw, topi, inv, self.expert_start, local)
 
     # True in subclasses that override ``route``: the fused top-k kernel (softmax routing) is skipped

@@ -40,7 +40,7 @@ def load() -> ctypes.CDLL:
         "vdamd_mid_gemm": [P, L, P, L, P, L, P, I, I, I, I, I, I, I, I, P],
         "vdamd_stream_gemm": [P, L, P, L, P, L, P, P, L, I, I, I, I, I, I, I, I, I, P],
         "vdamd_big_gemm": [P, L, P, L, P, L, P, L, I, I, I, I, I, I, P],
-        "vdamd_big_gemm_grouped": [P, L, P, L, P, L, L, P, I, I, I, I, I, I, P],
+        "vdamd_big_gemm_grouped": [P, L, P, L, P, L, L, P, I, P, I, I, I, I, I, I, P],
         "vdamd_rope_cache": [P, P, P, P, L, L, L, P, P, P, P, I, I, I, I, I, I, P, P, F, I, I, P, P, P],
         "vdamd_rope_cache_slabs": [P, P, I, P, L, P, P, P, P, I, I, I, I, I, P, P, F, I, I, P, P, P],
         "vdamd_paged_attention_decode": [P, P, P, L, P, P, P, I, P, F, I, I, I, I, I, I, L, I, I, P, P, I, F, P, P, P],
@@ -936,27 +936,39 @@ def grouped_big_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = Fal
             and n % (32 if silu_mul else 16) == 0 and w.data_ptr() % 16 == 0 and n * k * 2 < (1 << 32) - 64)
 
 
-def grouped_gemm(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, tile_rows: int,
-                 out: Optional[torch.Tensor] = None, silu_mul: bool = False) -> torch.Tensor:
+def grouped_gather_ok(x: torch.Tensor, src_row: torch.Tensor) -> bool:
+    """Whether the large-batch kernel's grouped form can read the rows ``x[src_row]`` where they are: whole, aligned rows of x
+    within 32-bit byte offsets, and eight entries at least (it fetches that many at a time)."""
+    return (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1] and x.data_ptr() % 16 == 0
+            and x.shape[0] * x.stride(0) * 2 < (1 << 32) - 64 and src_row.numel() >= 8)
+
+
+def grouped_gemm(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, tile_rows: int, out: Optional[torch.Tensor] = None,
+                 silu_mul: bool = False, src_row: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out[r] = x[r] @ w[g(r)]^T`` for group-sorted rows: ``w [G, N, K]``,
     ``tiles [n, 3] int32`` = (group, first row, rows <= tile_rows; 0 = unused).
     Every row covered by a tile must lie inside ``x``; rows outside all tiles
     are left untouched in ``out``.  ``tile_rows`` 256: the large-batch kernel, with ``silu_mul`` for ``w = [gate ; up]`` and
-    ``silu(gate) * up`` as the result (``N / 2`` wide)."""
+    ``silu(gate) * up`` as the result (``N / 2`` wide); ``src_row`` (with ``silu_mul``, at least eight): the tiles' rows are
+    ``x[src_row]``, read where they are."""
     nt = _check_tiles(tiles, x, tile_rows)
     g, n, k = w.shape
     assert w.is_contiguous() and w.dtype == x.dtype and x.shape[1] == k
     assert k % 128 == 0 and n % 16 == 0
     n_out = n // 2 if silu_mul else n
+    rows = x.shape[0] if src_row is None else src_row.numel()
     if out is None:
-        out = torch.empty((x.shape[0], n_out), dtype=x.dtype, device=x.device)
+        out = torch.empty((rows, n_out), dtype=x.dtype, device=x.device)
     if tile_rows == GROUPED_BIG_ROWS:
-        assert grouped_big_supported(x, w, silu_mul) and out.shape == (x.shape[0], n_out) and out.stride(1) == 1
+        assert grouped_big_supported(x, w, silu_mul) and out.shape == (rows, n_out) and out.stride(1) == 1
+        assert src_row is None or (silu_mul and src_row.dtype == torch.int32 and src_row.is_contiguous() and src_row.is_cuda
+                                   and grouped_gather_ok(x, src_row))
         _check(_LIB.vdamd_big_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k, n * k,
-                                           tiles.data_ptr(), nt, x.shape[0], n, k, EPI_SILU_MUL if silu_mul else EPI_NONE,
-                                           _dt(x), _stream()), "big_gemm_grouped")
+                                           tiles.data_ptr(), nt, None if src_row is None else src_row.data_ptr(), x.shape[0],
+                                           rows, n, k, EPI_SILU_MUL if silu_mul else EPI_NONE, _dt(x), _stream()),
+               "big_gemm_grouped")
         return out
-    assert 16 <= tile_rows <= 128 and not silu_mul
+    assert 16 <= tile_rows <= 128 and not silu_mul and src_row is None
     ntw = 1 if tile_rows > 64 or n <= 4096 else 2
     _check(_LIB.vdamd_skinny_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k,
                                           n * k, tiles.data_ptr(), nt, tile_rows, n, k, ntw, _dt(x), _stream()),
