@@ -1,325 +1,229 @@
-// GEMM for decode batches of 17..512 rows:  y[M][N] = x[M][K] . W[N][K]^T  (bf16 / f16, fp32 accumulate).
+// GEMM for decode batches of 1..512 rows:  y[M][N] = x[M][K] . W[N][K]^T  (bf16 / f16, fp32 accumulate), plain or with
+// SiLU(gate) * up over a [gate ; up] weight.
 //
-// In this range a step is bound by reading W once from HBM while the MFMA work per weight byte is
-// already substantial (M flops per byte), and the output has too few large tiles to fill 256 CUs
-// (N = 8192 gives 32 tiles of 256 columns).  Hence:
+// In this range a step is bound by reading W once from HBM while the MFMA work per weight byte is already substantial
+// (M flops per byte), and the output has too few large tiles to fill 256 CUs (N = 8192: 64 tiles of 128 columns).  Hence:
 //
-//  * one workgroup tile spans BM rows - all of M when M <= 256 - so every W byte is fetched from
-//    HBM exactly once, and K is split across workgroups (SPLITK slices; fp32 partial slabs and a
-//    small reduce kernel) until the grid covers the chip;
-//  * W never touches LDS.  The 8 waves of a workgroup sit side by side along N; a wave owns 16*FN
-//    output columns for ALL rows of the tile, so its W fragments (the MFMA A operand: lane (r, q)
-//    holds W[n + r][k + 8q .. +8], 16 rows x 64 bytes per instruction) are private to it and go from
-//    global memory straight into a three-deep register ring: two K tiles of W (8 KiB per wave,
-//    64 KiB per CU) are in flight while the third is multiplied, with no barrier in their way;
-//  * x is shared by all waves and comes from L2: 128-byte lines into registers two tiles ahead,
-//    into a double-buffered LDS image one tile ahead (16-byte slots XOR-ed with (row >> 1) & 7, so
-//    the 16-lane groups of a `ds_read_b128` fragment read hit 16 distinct slots of the 256-byte
-//    bank row), one barrier per 64-deep K tile;
-//  * every load is an ordinary one, issued in the fixed order x(t+2), W(t+2): the compiler's own
-//    counted `s_waitcnt vmcnt(N)` then leaves exactly the younger tiles in flight at each use;
-//  * workgroup id -> (tile, slice) puts equal slices on the same XCD (ids are dealt round-robin to
-//    the 8 XCDs), so an XCD's L2 only has to hold its slice of x.
+//  * a workgroup tile spans BM rows - all of M when M <= 256 - so every W byte is fetched from HBM once, and K is split
+//    across workgroups (fp32 partial slabs, summed by a small kernel or by the next one) until the grid covers the chip;
+//  * both operands go global -> LDS by LDS-DMA (`buffer_load_dwordx4 ... lds`, 8 rows x 128 bytes per wave instruction,
+//    never through registers) into rings of XS and WS images of one 64-deep K tile.  What is in flight is what the rate hangs
+//    on: at 5.7 TB/s a CU takes 16 KB of W in 0.73 us, an HBM round trip under load takes about 2.  Per tile the pieces of x
+//    are issued before those of W, and loads retire in order: the one counted wait of a K tile leaves two (XS - 1) tiles of W
+//    and one of x behind it in flight, and the tile issued right after it makes three;
+//  * the 16-byte slots of a row are XOR-ed with (row >> 1) & 7 - on the per-lane SOURCE address, the LDS-DMA destination
+//    being lane-linear - so the 16-lane groups of a `ds_read_b128` fragment read hit 16 distinct slots of the 256-byte bank
+//    row: no bank conflicts;
+//  * the fragments of the next 32-deep K step are read between the MFMAs of this one, column by column, and so are the DMA
+//    issues: read in one go in front of them, they held the MFMAs up (70B gate_up at 256 rows 217 -> 187 us);
+//  * one barrier per K tile, between its two K steps: behind it every wave has read all of the tile (its place in both rings
+//    is free) and every wave's pieces of the next one have landed;
+//  * W is read past the caches (nontemporal): it is not used again before it would be evicted, and x stays in the L2
+//    (8B gate_up at 48 rows 45.7 -> 41.5 us, 70B gate_up at 256 rows 209 -> 187);
+//  * ids are dealt to the XCDs in turn, and an XCD takes one run of the (slice, column tile, row tile) list: its L2 holds
+//    one or two slices of x, and the row tiles of a column tile share their W.
+//
+// Measured in captured graphs over copies of W larger than the caches, us, against the kernels before (W in registers,
+// x through LDS; a barrier-free stream at up to 8 rows) or the library; the fp32 slabs of a split K left unreduced:
+//   rows          1            16           100           256
+//   70B qkv       34 -> 29     36 -> 29     55 -> 37      61 -> 49       (10240 x 8192)
+//   70B o         27 -> 24     28 -> 24     34 -> 30      49 -> 40       (8192 x 8192)
+//   70B gate_up   162 -> 150   165 -> 154   180 -> 158    215 -> 190     (57344 x 8192, with SiLU * up)
+//   70B down      87 -> 77     89 -> 77     (no) -> 87    133 -> 105     (8192 x 28672)
+//   8B qkv        16 -> 11     16 -> 12     24 -> 16      28 -> 22       (6144 x 4096)
+//   8B gate_up    47 -> 41     68 -> 41     58 -> 51      77 -> 62       (28672 x 4096, with SiLU * up)
+// 5.7 to 6.2 TB/s of W up to 48 rows.  At 256 rows the power limit sets the pace: back to back for milliseconds, gate_up takes
+// 211 us and not 187.  The LDS traffic of a K tile (x and W written once, each wave's fragments read) and its MFMAs take 2048
+// clocks each of about 3000.  Matrix instructions of 32x32x16 (fewer, the same LDS reads: gate_up 227 us), four waves of twice
+// the columns (77 / 66 us for 8B's at 256 x 128), each workgroup's K loop begun elsewhere and an early touch of x for the XCD's
+// L2 (both within 1 %) were tried and left out.
 #include "common.h"
 
 namespace {
 
 constexpr int MG_BK = 64;            // K elements per tile = 128 bytes per row
-constexpr int MG_THREADS = 512;
-constexpr int MG_WAVES = 8;
+enum { MG_EPI_NONE = 0, MG_EPI_SILU_MUL = 2 };     // as in stream_gemm.hip
+typedef __attribute__((address_space(3))) void mg_lds_void;
 
-template <typename T, int BM, int FN>
-__global__ __launch_bounds__(MG_THREADS) void mid_gemm_kernel(
-    const T* x, long x_stride, const T* w, long w_stride, T* out, long out_stride, float* partial, int M, int N,
-    int K, int ksplit) {
-  // x and w are deliberately not __restrict__: loads from provably unaliased read-only memory may be
-  // moved across the barriers, and the pipeline below depends on WHEN each load is issued.
+// WM waves along the rows, WN along the columns; XS <= WS: images of x and W kept
+template <typename T, int BM, int BN, int WM, int WN, int XS, int WS, int EPI>
+__global__ __launch_bounds__(WM * WN * 64) void mid_gemm_kernel(const T* x, long x_stride, const T* w, long w_stride, T* out,
+                                                          long out_stride, float* partial, int M, int N, int K, int ksplit,
+                                                          int ntn, int up_row) {
+#if defined(__HIP_DEVICE_COMPILE__)
   using V8 = typename Vec8<T>::type;
-  constexpr int BN = MG_WAVES * 16 * FN;
-  constexpr int FM = BM / 16;
-  constexpr int XL = BM * 8 / MG_THREADS;       // 16-byte chunks of the x tile per thread
-  constexpr int STAGE = BM * 128;               // bytes of one x image
-  static_assert(XL >= 1 && FM % 2 == 0, "unsupported tile");
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * STAGE];
-
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int r16 = lane & 15, q = lane >> 4;
-
-  const int ntn = (N + BN - 1) / BN;
-  const int id = blockIdx.x;
-  const int ks = id % ksplit, tn = id / ksplit;
-  if (tn >= ntn) return;
-  const int m0 = blockIdx.y * BM, n0 = tn * BN + wid * 16 * FN;
-  const int KT = K / MG_BK;
-  const int kt_lo = KT * ks / ksplit, kt_hi = KT * (ks + 1) / ksplit;
-  const int nt = kt_hi - kt_lo;
-
-  // W fragment rows of this lane (clamped: columns past N are computed and dropped)
-  const T* wsrc[FN];
-#pragma unroll
-  for (int j = 0; j < FN; ++j)
-    wsrc[j] = w + (long)min(n0 + 16 * j + r16, N - 1) * w_stride + 8 * q + (long)kt_lo * MG_BK;
-  // x staging: chunk c = threadIdx.x + 512 i -> row c >> 3, 16-byte slot c & 7 (8 threads = one 128-byte line)
-  const T* xsrc[XL];
-  int xdst[XL];
-#pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int c = threadIdx.x + MG_THREADS * i;
-    const int row = c >> 3, slot = c & 7;
-    xsrc[i] = x + (long)min(m0 + row, M - 1) * x_stride + 8 * slot + (long)kt_lo * MG_BK;
-    xdst[i] = row * 128 + ((slot ^ ((row >> 1) & 7)) << 4);
-  }
-  // x fragment reads: lane (r16, q) of fragment i reads row 16 i + r16, slot (4 s + q) ^ swz(row)
-  int xoff = r16 * 128;                       // + 16 i * 128
-  const int xswz = (r16 >> 1) & 7;            // (16 i + r16) >> 1 & 7 == r16 >> 1 & 7
-
-  f32x4 acc[FN][FM];
-#pragma unroll
-  for (int j = 0; j < FN; ++j)
-#pragma unroll
-    for (int i = 0; i < FM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  V8 wreg[3][FN][2], xreg[2][XL];
-  auto load_w = [&](int slot, int t) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) wreg[slot][j][s] = ld8(wsrc[j] + (long)t * MG_BK + 32 * s);
-  };
-  auto load_x = [&](int slot, int t) {
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xreg[slot][i] = ld8(xsrc[i] + (long)t * MG_BK);
-  };
-  auto write_x = [&](int slot, int stage) {
-#pragma unroll
-    for (int i = 0; i < XL; ++i) *reinterpret_cast<V8*>(smem + stage * STAGE + xdst[i]) = xreg[slot][i];
-  };
-  // One K tile: 2 k-steps x FM row fragments, taken two fragments at a time.  The reads of pair p + 1
-  // are issued before the MFMAs of pair p, so an LDS round trip is covered by 2 * FN MFMAs of this
-  // wave plus whatever the SIMD's other wave issues.
-  auto compute = [&](int wslot, int stage) {
-    const unsigned char* base = smem + stage * STAGE + xoff;
-    constexpr int PAIRS = FM;                      // 2 k-steps * FM / 2
-    const int so0 = ((q) ^ xswz) << 4, so1 = ((4 + q) ^ xswz) << 4;
-    V8 b[2][2];
-    auto rd = [&](int p, V8 (&dst)[2]) {
-      const int s = p / (FM / 2), i = (p % (FM / 2)) * 2;
-      const int so = s ? so1 : so0;
-      dst[0] = *reinterpret_cast<const V8*>(base + i * 2048 + so);
-      dst[1] = *reinterpret_cast<const V8*>(base + (i + 1) * 2048 + so);
-    };
-    rd(0, b[0]);
-#pragma unroll
-    for (int p = 0; p < PAIRS; ++p) {
-      if (p + 1 < PAIRS) rd(p + 1, b[(p + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);           // or the reads sink down to their first use
-      const int s = p / (FM / 2), i = (p % (FM / 2)) * 2;
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[j][i + e] = mfma16(wreg[wslot][j][s], b[p & 1][e], acc[j][i + e]);
-    }
-  };
-
-  // Loads and LDS writes are unconditional (past the end they repeat the last tile and are never
-  // used): a branch around a load would make the compiler's wait for it a full drain.
-  if (nt <= 0) return;                     // block-uniform; cannot happen for ksplit <= K / 64
-  const int last = nt - 1;
-  load_x(0, 0); load_w(0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  load_x(1, min(1, last)); load_w(1, min(1, last));
-  __builtin_amdgcn_sched_barrier(0);
-  write_x(0, 0);
-  __syncthreads();
-  for (int t = 0; t < nt; t += 6) {
-#pragma unroll
-    for (int u = 0; u < 6; ++u) {
-      const int tt = t + u;
-      if (tt >= nt) break;
-      load_x(u & 1, min(tt + 2, last));
-      load_w((u + 2) % 3, min(tt + 2, last));
-      __builtin_amdgcn_sched_barrier(0);     // keep the issue order the in-flight accounting relies on
-      compute(u % 3, u & 1);
-      __builtin_amdgcn_sched_barrier(0);
-      write_x((u + 1) & 1, (u + 1) & 1);
-      __syncthreads();
-    }
-  }
-
-  // ---- epilogue: lane (r16, q) of fragment (j, i) holds y[m0 + 16 i + r16][n0 + 16 j + 4 q .. +4]
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int m = m0 + 16 * i + r16;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int n = n0 + 16 * j + 4 * q;
-      if (n >= N) continue;                  // N % 16 == 0: a fragment column group is all in or all out
-      if (ksplit == 1) {
-        typename Vec4<T>::type o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (T)acc[j][i][r];
-        *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
-      } else {
-        *reinterpret_cast<f32x4*>(partial + ((size_t)ks * M + m) * N + n) = acc[j][i];
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Deep-prefetch variant.  The loop above can keep two K tiles of W in flight and no more: loads
-// retire in order, and the wait for the x registers of tile t+1 also waits for every W load issued
-// before them.  Here x never enters a register: it goes global -> LDS by LDS-DMA
-// (`global_load_lds_dwordx4`, 8 rows x 128 bytes per wave instruction, the XOR swizzle applied to
-// the per-lane SOURCE address because the destination of an LDS-DMA is lane-linear) into a
-// three-stage image, two tiles ahead; W goes into a four-slot register ring, four tiles ahead.
-// Issue order per iteration is [x(t+2) | ... compute(t) ... | W(t+4)], so the one wait of an
-// iteration, `vmcnt(12)`, retires x(t) - and with it W(t), W(t+1), which are older - while W(t+2),
-// x(t+1), W(t+3) stay in flight: an HBM round trip has three to four tile times to complete.
-// The W loads are inline asm: next to an LDS-DMA in flight the compiler would wait `vmcnt(0)` for
-// any ordinary load it can see; their destinations are only read after the counted wait, which
-// names them as read-write operands so that nothing can be scheduled across it.
-// ---------------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-typedef const __attribute__((address_space(1))) void glb_void;
-
-template <typename V8>
-__device__ __forceinline__ void asm_load2(V8& a, V8& b, const void* p) {
-  asm volatile("global_load_dwordx4 %0, %2, off\n\tglobal_load_dwordx4 %1, %2, off offset:64"
-               : "=&v"(a), "=&v"(b) : "v"(p) : "memory");
-}
-
-template <typename T, int BM, int FN>
-__global__ __launch_bounds__(MG_THREADS) void mid_gemm_deep_kernel(
-    const T* x, long x_stride, const T* w, long w_stride, T* out, long out_stride, float* partial, int M, int N,
-    int K, int ksplit) {
-  using V8 = typename Vec8<T>::type;
-  constexpr int BN = MG_WAVES * 16 * FN;
-  constexpr int FM = BM / 16;
-  constexpr int STAGE = BM * 128;               // bytes of one x image
-  constexpr int XS = 3;                         // x stages
-  constexpr int WS = 4;                         // W ring slots
-  constexpr int PPW = BM / 8 / MG_WAVES;        // 1 KiB DMA pieces per wave per tile
-  static_assert(PPW >= 1 && FM % 2 == 0, "unsupported tile");
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[XS * STAGE];
+  constexpr int WAVES = WM * WN, FM = BM / WM / 16, FN = BN / WN / 16;
+  constexpr int PX = BM / 8 / WAVES, PW = BN / 8 / WAVES;      // 1 KiB pieces per wave and K tile
+  constexpr int XB = BM * 128, WB = BN * 128;
+  constexpr int MG_NT = 2;           // cache policy of W's loads: nontemporal
+  static_assert(XS >= 2 && WS >= XS && WS <= XS + 1 && XS * XB + WS * WB <= 160 * 1024, "unsupported tile");
+  static_assert(EPI != MG_EPI_SILU_MUL || FN % 2 == 0, "unsupported tile");
+  // loads of a wave behind x and W of the tile that a wait is for: with WS > XS that W is older than that x
+  constexpr int AHEAD = WS > XS ? (XS - 1) * PW + (XS - 2) * PX : (XS - 2) * (PX + PW);
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[XS * XB + WS * WB];
+  unsigned char* const smw = smem + XS * XB;
 
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid % WM, wn = wid / WM;
   const int r16 = lane & 15, q = lane >> 4;
-  const int ntn = (N + BN - 1) / BN;
-  const int id = blockIdx.x;
-  const int ks = id % ksplit, tn = id / ksplit;
-  if (tn >= ntn) return;
-  const int m0 = blockIdx.y * BM, n0 = tn * BN + wid * 16 * FN;
+  const int per = gridDim.x >> 3, work = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  const int ntm = (M + BM - 1) / BM;
+  if (work >= ntn * ksplit * ntm) return;
+  const int mt = work % ntm, wide = work / ntm;
+  const int ks = wide / ntn, tn = wide - ks * ntn;
+  const int m0 = mt * BM;
   const int KT = K / MG_BK;
-  const int kt_lo = KT * ks / ksplit, kt_hi = KT * (ks + 1) / ksplit;
+  const int kt_lo = (int)((long)KT * ks / ksplit), kt_hi = (int)((long)KT * (ks + 1) / ksplit);
   const int nt = kt_hi - kt_lo;
-  if (nt <= 0) return;
+  if (nt <= 0) return;                     // block-uniform; cannot happen for ksplit <= K / 64
   const int last = nt - 1;
 
-  const T* wsrc[FN];
+  // row of W behind row r of the tile, from the tile's first one: plain, tn * BN ..; with SiLU, BN / 2 gate rows and as many up
+  // rows in turns of half a wave's columns, so that a lane holds gate and up of the same column.  Columns past N repeat the last.
+  const int first = EPI == MG_EPI_SILU_MUL ? tn * (BN / 2) : tn * BN;
+  auto w_row = [&](int r) {
+    if constexpr (EPI == MG_EPI_SILU_MUL) {
+      constexpr int H = BN / WN / 2;
+      const int col = min(r / (2 * H) * H + r % H, up_row - 1 - first);
+      return r % (2 * H) < H ? col : up_row + col;
+    }
+    return min(r, N - 1 - first);
+  };
+  const int mrows = min(BM, M - m0), wrows = EPI == MG_EPI_SILU_MUL ? N - first : min(BN, N - first);
+  // (the spans fit 32 bits: checked on the host)
+  const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x + (long)m0 * x_stride), 0,
+                                                       (int)(((mrows - 1) * x_stride + K) * 2), 0x00020000);
+  const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w + (long)first * w_stride), 0,
+                                                       (int)(((wrows - 1) * w_stride + K) * 2), 0x00020000);
+  unsigned offx[PX], offw[PW];
 #pragma unroll
-  for (int j = 0; j < FN; ++j)
-    wsrc[j] = w + (long)min(n0 + 16 * j + r16, N - 1) * w_stride + 8 * q + (long)kt_lo * MG_BK;
-  // DMA piece p (8 rows x 128 B) of this wave: lane -> row 8p + (lane >> 3), source chunk (lane & 7) ^ swz(row)
-  const T* xsrc[PPW];
-#pragma unroll
-  for (int i = 0; i < PPW; ++i) {
-    const int row = 8 * (wid * PPW + i) + (lane >> 3);
-    xsrc[i] = x + (long)min(m0 + row, M - 1) * x_stride + 8 * ((lane & 7) ^ ((row >> 1) & 7)) + (long)kt_lo * MG_BK;
+  for (int i = 0; i < PX; ++i) {
+    const int r = 8 * (wid * PX + i) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    offx[i] = ((unsigned)min(r, mrows - 1) * (unsigned)x_stride + kt_lo * MG_BK + 8 * c) * 2;
   }
-  const int xoff = r16 * 128;
-  const int xswz = (r16 >> 1) & 7;
-  const int so0 = (q ^ xswz) << 4, so1 = ((4 + q) ^ xswz) << 4;
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int r = 8 * (wid * PW + i) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    offw[i] = ((unsigned)w_row(r) * (unsigned)w_stride + kt_lo * MG_BK + 8 * c) * 2;
+  }
+  const int swz = (r16 >> 1) & 7;
+  const int so[2] = {(q ^ swz) << 4, ((4 + q) ^ swz) << 4};
+  const int xro = (wm * FM * 16 + r16) * 128, wro = (wn * FN * 16 + r16) * 128;
 
   f32x4 acc[FN][FM];
 #pragma unroll
   for (int j = 0; j < FN; ++j)
 #pragma unroll
     for (int i = 0; i < FM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  V8 wreg[WS][FN][2];
-
-  auto dma_x = [&](int stage, int t) {
+  V8 xf[2][FM], wf[2][FN];
+  constexpr int XR = (FM + FN - 1) / FN, LR = (PX + PW + FN - 1) / FN;
+  // the j-th of FN parts of a K step's fragment reads, and of a K tile's DMA
+  auto read = [&](int s, int sx, int sw, int j) {
+    const unsigned char* bx = smem + sx * XB + xro + so[s];
+    const unsigned char* bw = smw + sw * WB + wro + so[s];
 #pragma unroll
-    for (int i = 0; i < PPW; ++i)
-      __builtin_amdgcn_global_load_lds((glb_void*)(xsrc[i] + (long)t * MG_BK),
-                                       (lds_void*)(smem + stage * STAGE + (wid * PPW + i) * 1024), 16, 0, 0);
+    for (int i = j * XR; i < (j + 1) * XR && i < FM; ++i) xf[s][i] = *reinterpret_cast<const V8*>(bx + i * 2048);
+    wf[s][j] = *reinterpret_cast<const V8*>(bw + j * 2048);
   };
-  auto load_w = [&](int slot, int t) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j) asm_load2(wreg[slot][j][0], wreg[slot][j][1], wsrc[j] + (long)t * MG_BK);
+  // (past the last tile it is fetched again and never used: the counted waits need the same loads in every iteration)
+  auto load_x = [&](int stage, int t, int p) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (mg_lds_void*)(smem + stage * XB + (wid * PX + p) * 1024), 16, offx[p],
+                                             min(t, last) * 128, 0, 0);
   };
-
-  // prologue, in the order the steady-state accounting expects: W(0) W(1) x(0) W(2) x(1) W(3)
-  load_w(0, 0);
-  load_w(1, min(1, last));
-  dma_x(0, 0);
-  load_w(2, min(2, last));
-  dma_x(1, min(1, last));
-  load_w(3, min(3, last));
-
-  for (int t = 0; t < nt; t += 12) {
+  auto load_w = [&](int stage, int t, int p) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, (mg_lds_void*)(smw + stage * WB + (wid * PW + p) * 1024), 16, offw[p],
+                                             min(t, last) * 128, 0, MG_NT);
+  };
+  auto load = [&](int sx, int sw, int t, int j) {
 #pragma unroll
-    for (int u = 0; u < 12; ++u) {
-      const int tt = t + u;
-      if (tt >= nt) break;
-      const int stage = u % XS, slot = u % WS;
-      // x(tt) and W(tt) have landed once only W(tt+2), x(tt+1), W(tt+3) are outstanding
-      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * 2 * FN + PPW) : "memory");
-      // the W fragments of this slot are valid from here on: make every later use depend on this point
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        asm volatile("" : "+v"(wreg[slot][j][0]), "+v"(wreg[slot][j][1]));
-      __builtin_amdgcn_s_barrier();               // every wave's pieces of x(tt) are in LDS; stage of x(tt-1) is free
-      __builtin_amdgcn_sched_barrier(0);
-      dma_x((u + 2) % XS, min(tt + 2, last));
-      __builtin_amdgcn_sched_barrier(0);
-      {
-        const unsigned char* base = smem + stage * STAGE + xoff;
-        V8 b[2][2];
-        auto rd = [&](int p, V8 (&dst)[2]) {
-          const int s = p / (FM / 2), i = (p % (FM / 2)) * 2;
-          const int so = s ? so1 : so0;
-          dst[0] = *reinterpret_cast<const V8*>(base + i * 2048 + so);
-          dst[1] = *reinterpret_cast<const V8*>(base + (i + 1) * 2048 + so);
-        };
-        rd(0, b[0]);
-#pragma unroll
-        for (int p = 0; p < FM; ++p) {
-          if (p + 1 < FM) rd(p + 1, b[(p + 1) & 1]);
-          __builtin_amdgcn_sched_barrier(0);
-          const int s = p / (FM / 2), i = (p % (FM / 2)) * 2;
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acc[j][i + e] = mfma16(wreg[slot][j][s], b[p & 1][e], acc[j][i + e]);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      load_w(slot, min(tt + WS, last));           // into the slot just consumed
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = j * LR; i < (j + 1) * LR && i < PX + PW; ++i) {
+      if (i < PX) load_x(sx, t + XS, i);
+      else load_w(sw, t + WS, i - PX);
     }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stray tail prefetches must not outlive the registers / LDS
-
+  };
+  auto mma = [&](int s, int j) {
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int m = m0 + 16 * i + r16;
-    if (m >= M) continue;
+    for (int i = 0; i < FM; ++i) acc[j][i] = mfma16(wf[s][j], xf[s][i], acc[j][i]);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  // as iterations -WS .. -2 of the loop would have issued them
+#pragma unroll
+  for (int i = -WS; i < -1; ++i) {
+    if (i + XS >= 0)
+#pragma unroll
+      for (int p = 0; p < PX; ++p) load_x(i + XS, i + XS, p);
+#pragma unroll
+    for (int p = 0; p < PW; ++p) load_w(i + WS, i + WS, p);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < FN; ++j) load(XS - 1, WS - 1, -1, j);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < FN; ++j) read(0, 0, 0, j);
+  int sx = 0, sw = 0;
+  for (int t = 0; t < nt; ++t) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      const int n = n0 + 16 * j + 4 * q;
-      if (n >= N) continue;
-      if (ksplit == 1) {
+      read(1, sx, sw, j);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(0, j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AHEAD) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const int nx = sx + 1 == XS ? 0 : sx + 1, nw = sw + 1 == WS ? 0 : sw + 1;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      load(sx, sw, t, j);
+      read(0, nx, nw, j);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(1, j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    sx = nx;
+    sw = nw;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // the tail prefetches must not outlive the LDS
+
+  // ---- lane (r16, q) of fragment (j, i) holds y[row 16 i + r16][column 16 j + 4 q .. + 4] of the wave's part
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + (wm * FM + i) * 16 + r16;
+    if (m >= M) continue;
+    if constexpr (EPI == MG_EPI_SILU_MUL) {
+#pragma unroll
+      for (int j = 0; j < FN / 2; ++j) {
+        const int n = tn * (BN / 2) + (wn * (FN / 2) + j) * 16 + 4 * q;
+        if (n >= up_row) continue;
         typename Vec4<T>::type o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (T)acc[j][i][r];
+        for (int r = 0; r < 4; ++r) o[r] = (T)(fast_silu(acc[j][i][r]) * acc[FN / 2 + j][i][r]);
         *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
-      } else {
-        *reinterpret_cast<f32x4*>(partial + ((size_t)ks * M + m) * N + n) = acc[j][i];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int n = tn * BN + (wn * FN + j) * 16 + 4 * q;
+        if (n >= N) continue;                // N % 16 == 0: a fragment column group is all in or all out
+        if (ksplit == 1) {
+          typename Vec4<T>::type o;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = (T)acc[j][i][r];
+          *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
+        } else {
+          *reinterpret_cast<f32x4*>(partial + ((size_t)ks * M + m) * N + n) = acc[j][i];
+        }
       }
     }
   }
+#endif
 }
 
 template <typename T>
@@ -338,24 +242,18 @@ __global__ void mid_reduce_kernel(T* __restrict__ out, long out_stride, const fl
   *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
 }
 
-template <typename T, int BM, int FN>
-int launch(const void* x, long xs, const void* w, long ws, void* out, long os, void* partial, int M, int N, int K,
-           int ksplit, int variant, hipStream_t st) {
-  constexpr int BN = MG_WAVES * 16 * FN;
-  const int ntn = (N + BN - 1) / BN;
-  dim3 grid(ntn * ksplit, (M + BM - 1) / BM);
-  if constexpr (BM >= 64 && FN <= 2) {
-    if (variant == 1) {
-      mid_gemm_deep_kernel<T, BM, FN><<<grid, MG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os,
-                                                                   (float*)partial, M, N, K, ksplit);
-    } else {
-      mid_gemm_kernel<T, BM, FN><<<grid, MG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os,
-                                                              (float*)partial, M, N, K, ksplit);
-    }
-  } else {
-    mid_gemm_kernel<T, BM, FN><<<grid, MG_THREADS, 0, st>>>((const T*)x, xs, (const T*)w, ws, (T*)out, os,
-                                                            (float*)partial, M, N, K, ksplit);
-  }
+template <typename T, int BM, int BN, int WM, int WN, int XS, int WS>
+int launch(const void* x, long xs, const void* w, long ws, void* out, long os, void* partial, int M, int N, int K, int ksplit,
+           int epi, hipStream_t st) {
+  const bool silu = epi == MG_EPI_SILU_MUL;
+  const int ntn = silu ? (N / 2 + BN / 2 - 1) / (BN / 2) : (N + BN - 1) / BN;
+  const int grid = (ntn * ksplit * ((M + BM - 1) / BM) + 7) / 8 * 8;
+#define MG_GO(EPI)                                                                                                             \
+  mid_gemm_kernel<T, BM, BN, WM, WN, XS, WS, EPI><<<grid, WM * WN * 64, 0, st>>>(                                              \
+      (const T*)x, xs, (const T*)w, ws, (T*)out, os, (float*)partial, M, N, K, ksplit, ntn, N / 2)
+  if (silu) MG_GO(MG_EPI_SILU_MUL);
+  else MG_GO(MG_EPI_NONE);
+#undef MG_GO
   HIP_LAUNCH_CHECK();
   if (ksplit > 1 && out != nullptr) {            // out == nullptr: the caller consumes the K-split slabs itself
     const long n = (long)M * (N / 4);
@@ -366,35 +264,43 @@ int launch(const void* x, long xs, const void* w, long ws, void* out, long os, v
   return 0;
 }
 
+// 64 rows: two workgroups of four waves to a CU (72 KB), which level out what is left of a round (eight waves, each with half
+// the columns, read more of LDS: 70B down at 48 rows 81 us, so 77); larger tiles take a CU each
 template <typename T>
 int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os, void* partial, int M, int N, int K,
-             int ksplit, int bm, int bn, int variant, hipStream_t st) {
-#define MG_CASE(BM_, FN_)                                                                       \
-  if (bm == BM_ && bn == MG_WAVES * 16 * FN_)                                                   \
-    return launch<T, BM_, FN_>(x, xs, w, ws, out, os, partial, M, N, K, ksplit, variant, st);
-  MG_CASE(256, 2) MG_CASE(256, 1) MG_CASE(128, 2) MG_CASE(128, 1) MG_CASE(64, 2) MG_CASE(64, 4)
+             int ksplit, int bm, int bn, int epi, hipStream_t st) {
+#define MG_CASE(BM, BN, WM, WN, XS, WS) \
+  if (bm == BM && bn == BN) return launch<T, BM, BN, WM, WN, XS, WS>(x, xs, w, ws, out, os, partial, M, N, K, ksplit, epi, st);
+  MG_CASE(256, 256, 4, 2, 2, 3)
+  MG_CASE(256, 128, 2, 4, 3, 4)
+  MG_CASE(128, 256, 2, 4, 2, 3)
+  MG_CASE(128, 128, 4, 2, 4, 5)
+  MG_CASE(64, 128, 2, 2, 3, 3)
 #undef MG_CASE
   return -4;
 }
 
 }  // namespace
 
-// out[M][N] = x[M][K] . w[N][K]^T.  K % 64 == 0, N % 16 == 0; strides in elements, multiples of 8;
-// pointers 16-byte aligned.  (bm, bn) is the workgroup tile: (256, 128|256), (128, 128|256), (64, 256|512).
-// partial holds ksplit * M * N floats when ksplit > 1.  variant 0: x staged through registers, W two tiles
-// ahead; variant 1: x by LDS-DMA, W four tiles ahead (tiles with bn <= 256).
+// out = epilogue(x[M][K] . w[N][K]^T).  K % 64 == 0, N % 16 == 0; strides in elements, multiples of 8; pointers 16-byte
+// aligned.  (bm, bn) is the workgroup tile: (256, 128|256), (128, 128|256), (64, 128).
+// epi 0: out[M][N]; partial holds ksplit * M * N floats when ksplit > 1, and out may be null then: the slabs are the result.
+// epi 2: w = [gate ; up], N % 32 == 0, ksplit 1, out[M][N/2] = silu(gate) * up.
 VDAMD_API int vdamd_mid_gemm(void* out, long out_stride, const void* x, long x_stride, const void* w, long w_stride,
-                             void* partial, int M, int N, int K, int ksplit, int bm, int bn, int variant, int dtype,
+                             void* partial, int M, int N, int K, int ksplit, int bm, int bn, int epi, int dtype,
                              void* stream) {
   if (M <= 0) return 0;
   if (K % MG_BK || N % 16 || ksplit < 1 || ksplit > K / MG_BK) return -1;
+  if (epi != MG_EPI_NONE && (epi != MG_EPI_SILU_MUL || N % 32 || ksplit != 1)) return -1;
   if (ksplit > 1 && partial == nullptr) return -2;
   if (out == nullptr && ksplit == 1) return -2;
   if ((x_stride | w_stride) % 8 || out_stride % 4) return -5;
+  const long lim = (1L << 32) - 64;                // bytes that a tile's buffer descriptor spans
+  if ((long)(M < bm ? M : bm) * x_stride * 2 >= lim || (long)(epi == MG_EPI_SILU_MUL ? N : bn) * w_stride * 2 >= lim) return -7;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == DT_BF16)
-    return dispatch<bf16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, variant, st);
+    return dispatch<bf16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, epi, st);
   if (dtype == DT_F16)
-    return dispatch<f16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, variant, st);
+    return dispatch<f16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, epi, st);
   return -3;
 }

@@ -56,6 +56,33 @@ def test_latent_plan(tokens, heads, keys, by_token, seqs, rows_ok, captured, pla
     assert hip.mla_plan(tokens, heads, keys, by_token, seqs, rows_ok, None, captured) == plan
 
 
+@pytest.mark.parametrize("m,n,k,reduced,takes", [
+    # the next kernel sums the slabs (library / this, us): 8.5 / 5.5, 16.2 / 11.2; a small W at many rows 8.9 / 9.9, 10.2 / 13.3,
+    # 17.7 / 16.5; 32 / 18; a router
+    (1, 2048, 2048, False, True), (1, 6144, 4096, False, True), (128, 2048, 2048, False, False), (256, 2048, 2048, False, False),
+    (256, 3072, 3072, False, False), (256, 4608, 3072, False, True), (16, 160, 6144, False, False),
+    # with a reduction of its own: 26.7 / 28, 18.1 / 20; 41 / 33; 81 / 50; 11 / 21
+    (1, 8192, 8192, True, False), (8, 6144, 6144, True, False), (48, 4096, 14336, True, True), (256, 8192, 8192, True, True),
+    (256, 3072, 2048, True, False),
+    # wide enough unsplit: 190 / 164, 309 / 252, 57 / 44
+    (1, 128256, 4096, True, True), (256, 128256, 4096, True, True), (8, 32000, 4096, True, True),
+    # above 256 rows: 316 / 186, 76 / 73, 94 / 97
+    (512, 8192, 28672, True, True), (512, 8192, 8192, True, False), (512, 28672, 4096, True, False), (513, 8192, 28672, True, False)])
+def test_short_batch_products(m, n, k, reduced, takes):
+    assert hip.mid_profitable(m, n, k, reduced) is takes
+    if takes:
+        bm, bn, ksplit = hip.mid_choose(m, n, k, reduced)
+        assert (bm, bn) in hip._MID_TILES and bm >= min(m, 256) and 1 <= ksplit <= k // 64
+
+
+def test_gate_up_at_short_batches():
+    assert hip.mid_silu_profitable(1, 28672, 4096) and hip.mid_silu_profitable(256, 57344, 8192)
+    assert not hip.mid_silu_profitable(257, 57344, 8192) and not hip.mid_silu_profitable(9, 28672, 2048)
+    assert not hip.mid_silu_profitable(1, 7168, 8192)
+    # 8 rows and a reduction below 4096: the barrier-free stream
+    assert hip.stream_profitable(8, 28672, 2048) and not hip.stream_profitable(8, 28672, 4096)
+
+
 def test_recurrent_layers_report_their_prompt_memory():
     """What a prompt through a recurrent layer allocates counts in the memory profile, which does not run its kernels."""
     import torch

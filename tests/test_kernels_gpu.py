@@ -1117,6 +1117,41 @@ def test_mid_gemm_matches_fp32(dtype, m, n, k, pad):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (64, 1040, 128), (65, 160, 192), (129, 992, 256), (256, 416, 320), (257, 272, 4096)])
+def test_mid_gemm_rings_of_few_tiles_and_silu(dtype, m, n, k):
+    """Fewer K tiles than the rings hold, last columns and rows inside a tile, every tile of the kernel; plain and with
+    SiLU(gate) * up.  Bound: the rounding of the result, and K roundings of the sums."""
+    from vllm_distributed_amd.ops import hip
+    x, w = _rand(m, k, dtype=dtype), _padded_weight(n, k, 8, dtype)
+    ref = x.double() @ w.double().t()
+    eps = torch.finfo(dtype).eps
+    acc = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    h = n // 2
+    g, u = ref[:, :h], ref[:, h:]
+    act = torch.nn.functional.silu(g) * u
+    act_bound = eps * act.abs() + 1.1 * (acc[:, :h] * u.abs() + acc[:, h:] * g.abs()) + 1e-6
+    for bm, bn in hip._MID_TILES:
+        for ks in {1, 2, k // 64} & set(range(1, k // 64 + 1)):
+            got = hip.mid_gemm(x, w, bm=bm, bn=bn, ksplit=ks)
+            assert ((got.double() - ref).abs() <= eps * ref.abs() + acc + 1e-6).all(), (bm, bn, ks)
+            if ks > 1:
+                slabs = hip.mid_gemm(x, w, bm=bm, bn=bn, ksplit=ks, partials=True)
+                assert slabs.shape == (ks, m, n) and ((slabs.double().sum(0) - ref).abs() <= acc + 1e-6).all()
+        if n % 32 == 0:
+            got = hip.mid_gemm(x, w, bm=bm, bn=bn, silu_mul=True)
+            assert got.shape == (m, h) and ((got.double() - act).abs() <= act_bound).all(), (bm, bn)
+
+
+def test_mid_gemm_of_one_row_with_any_row_stride():
+    """One row may carry any stride (an expanded or sliced tensor): its span is K columns all the same."""
+    from vllm_distributed_amd.ops import hip
+    x, w = _rand(1, 512), _padded_weight(256, 512, 128)
+    want = hip.mid_gemm(x, w)
+    for stride in (0, 8, 4096):
+        assert torch.equal(hip.mid_gemm(torch.as_strided(x, (1, 512), (stride, 1)), w), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k,pad", [(256, 256, 128, 0), (512, 512, 256, 128), (300, 336, 384, 8),
                                        (1000, 2048, 2048, 128), (2048, 1024, 8192, 128),
                                        # more tiles than CUs (9 x 30): workgroups walk several tiles, with a

@@ -117,15 +117,15 @@ environment_variables: Dict[str, Callable[[], Any]] = {
     # mapped round-robin onto the visible devices and torch.distributed runs on
     # gloo with host staging (RCCL refuses two ranks on one device).
     "VDAMD_SHARE_DEVICE": _bool("VDAMD_SHARE_DEVICE", False),
-    # Short-batch weight-streaming GEMM for long-reduction shapes (0 = library GEMM only).
+    # Hand-written GEMMs of short batches (up to 256 rows, 512 into long reductions; 0 = library GEMM only).
     "VDAMD_SKINNY_GEMM": _bool("VDAMD_SKINNY_GEMM", True),
     # Large-batch (M >= 512) 256 x 256-tile LDS-DMA GEMM with fused SiLU*mul / residual epilogues
     # (0 = library GEMM + separate activation kernel).
     "VDAMD_BIG_GEMM": _bool("VDAMD_BIG_GEMM", True),
     # The K-split slabs of a row-parallel projection (TP = 1) are summed by the add + RMSNorm that follows it
     # instead of by a reduction kernel of their own (one launch and a 16-bit round trip fewer per projection).
-    # Up to 8 rows into a very wide output (gate_up with the SiLU epilogue, LM head): the barrier-free
-    # weight-streaming GEMM instead of the library.
+    # Up to 8 rows into a very wide output over a reduction below 4096 (gate_up with the SiLU epilogue, LM head):
+    # the barrier-free weight-streaming GEMM instead of the library.
     "VDAMD_STREAM_GEMM": _bool("VDAMD_STREAM_GEMM", True),
     # DeepSeek's multi-head latent attention keeps the latent (kv_lora_rank + rope values per token) in the
     # cache and attends with the up-projections absorbed into q and the output; 0 = expand to per-head

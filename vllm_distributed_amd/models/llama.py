@@ -118,13 +118,13 @@ class LlamaMLP(nn.Module):
         if act is not None:
             if residual is not None and self.down_proj.forward_add(act, residual):
                 return None
-            if partials and act.shape[0] <= 256:
+            if partials and act.shape[0] <= ops.SHORT_BATCH:
                 part = self.down_proj.forward_partials(act)
                 if part is not None:
                     return part
             return self.down_proj(act, reduce, staged)
         gate_up = self.gate_up_proj(x)
-        if partials and gate_up.dim() == 2 and gate_up.shape[0] <= 256:
+        if partials and gate_up.dim() == 2 and gate_up.shape[0] <= ops.SHORT_BATCH:
             # short batches: the K-split slabs go to the next add + RMSNorm unreduced
             act = ops.silu_and_mul(gate_up)
             part = self.down_proj.forward_partials(act)

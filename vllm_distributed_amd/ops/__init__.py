@@ -15,6 +15,9 @@ from .. import envs
 from . import torch_ref
 from .torch_ref import k_cache_shape, v_cache_shape  # noqa: F401  (the paged-cache layouts every backend shares)
 
+# rows up to which a projection may leave fp32 partial sums of a split K to the kernel that follows
+SHORT_BATCH = 512
+
 _hip = None
 _hip_error: Optional[BaseException] = None
 
@@ -101,11 +104,11 @@ def linear_partials(x, weight):
     """``x @ weight^T`` left as the fp32 K-split slabs ``[ks, M, N]`` of the short-batch kernels, for a
     consumer that reduces them itself (the add + RMSNorm that follows a row-parallel projection); None
     where the shape runs unsplit or on another kernel."""
-    if not (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= 256 and envs.VDAMD_SKINNY_GEMM
+    if not (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= SHORT_BATCH and envs.VDAMD_SKINNY_GEMM
             and envs.VDAMD_FUSED_REDUCE_NORM and _use_hip(x)):
         return None
     m, n, k = x.shape[0], weight.shape[0], weight.shape[1]
-    if _hip.mid_profitable(m, n, k) and _hip.mid_supported(x, weight):
+    if _hip.mid_profitable(m, n, k, reduced=False) and _hip.mid_supported(x, weight):
         return _hip.mid_gemm(x, weight, partials=True)
     if m <= 128 and _hip.skinny_profitable(m, n, k) and _hip.skinny_supported(x, weight):
         return _hip.skinny_gemm_partials(x, weight)
@@ -237,7 +240,7 @@ def linear(x, weight, bias=None, out=None):
     long-reduction shapes where the weight-streaming HIP kernel is faster.
     ``out`` (2-D ``x`` only): write the result there (e.g. straight into the
     buffer the following all-reduce reads)."""
-    if x.is_cuda and x.dim() == 2 and x.shape[0] <= 256 and envs.VDAMD_SKINNY_GEMM and _use_hip(x):
+    if x.is_cuda and x.dim() == 2 and x.shape[0] <= SHORT_BATCH and envs.VDAMD_SKINNY_GEMM and _use_hip(x):
         m, n, k = x.shape[0], weight.shape[0], weight.shape[1]
         if (envs.VDAMD_STREAM_GEMM and _hip.stream_profitable(m, n, k) and _hip.stream_supported(x, weight)
                 and (out is None or out.stride(0) == n)):
@@ -334,12 +337,16 @@ def linear_add(x, weight, residual) -> bool:
 def gate_up_silu(x, weight):
     """``silu(x @ Wg^T) * (x @ Wu^T)`` for ``weight = [Wg ; Wu]`` in one kernel (the large-batch GEMM
     forms the activation in its epilogue: the ``[M, 2F]`` intermediate is never written), or ``None``
-    when that kernel does not take the shape - the caller then runs the two-step path.  A handful of rows
-    take the barrier-free weight-streaming kernel, which has the same epilogue."""
+    when that kernel does not take the shape - the caller then runs the two-step path.  Up to 256 rows
+    take the short-batch kernels, which have the same epilogue."""
     if (x.is_cuda and x.dim() == 2 and envs.VDAMD_STREAM_GEMM and envs.VDAMD_SKINNY_GEMM and _use_hip(x)
             and _hip.stream_profitable(x.shape[0], weight.shape[0], weight.shape[1])
             and _hip.stream_supported(x, weight) and weight.shape[0] % 64 == 0):
         return _hip.stream_gemm(x, weight, silu_mul=True)
+    if (x.is_cuda and x.dim() == 2 and envs.VDAMD_SKINNY_GEMM and _use_hip(x)
+            and _hip.mid_silu_profitable(x.shape[0], weight.shape[0], weight.shape[1])
+            and _hip.mid_supported(x, weight, True)):
+        return _hip.mid_gemm(x, weight, silu_mul=True)
     if (x.is_cuda and x.dim() == 2 and envs.VDAMD_BIG_GEMM and _use_hip(x) and x.shape[0] >= _hip.BIG_MIN_M_SILU
             and _hip.big_profitable(x.shape[0], weight.shape[0], weight.shape[1], True)
             and _hip.big_supported(x, weight, True)):

@@ -709,11 +709,9 @@ STREAM_WIRED_MAX_M = 8
 
 
 def stream_profitable(m: int, n: int, k: int) -> bool:
-    """Where this kernel beats the library GEMM on MI355X (benchmarks/stream_silu_probe.py and
-    stream_gemm_sweep.py, padded weight rows, inside graphs): up to 8 rows into a very wide output - a gate_up
-    projection (8B-class: 48 us with the activation in the epilogue against 67 us for library + activation
-    kernel; 70B: 164 against 166 us) or an LM head (356 against 369 us).  Narrow outputs (a TP=8 shard) lose."""
-    return 0 < m <= STREAM_WIRED_MAX_M and n >= 24576 and k >= 2048
+    """Up to 8 rows into a very wide output over a reduction of 2048 to 4095 (library and activation kernel 67 us, this 48 in
+    an 8B-class gate_up); longer ones are ``mid_gemm``'s (41 us), narrow outputs (a TP=8 shard) the library's."""
+    return 0 < m <= STREAM_WIRED_MAX_M and n >= MID_SILU_MIN_N and 2048 <= k < MID_SILU_MIN_K
 
 
 def stream_choose(n: int, k: int, silu: bool = False) -> Tuple[int, int, int]:
@@ -757,110 +755,139 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     return out
 
 
-# ---------------------------------------- split-K LDS-DMA GEMM, 16 < M <= 512
+# ---------------------------------------- split-K LDS-DMA GEMM, 1 <= M <= 512
 MID_MAX_M = 512
-# -1: the LDS-DMA / four-tile-prefetch kernel for 256-row tiles (2-7 % faster there), the register-staged
-# one for smaller tiles (where the deep variant is 2-5 % slower); 0 / 1 force one of them
-MID_VARIANT = int(os.environ.get("VDAMD_MID_GEMM_VARIANT", "-1"))
 
 
-def mid_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+def mid_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = False) -> bool:
     return (x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= MID_MAX_M and x.dtype == w.dtype
             and x.dtype in (torch.bfloat16, torch.float16) and x.shape[1] == w.shape[1]
-            and w.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and x.stride(1) == 1 and w.stride(1) == 1
+            and w.shape[1] % 64 == 0 and w.shape[0] % (32 if silu_mul else 16) == 0 and x.stride(1) == 1 and w.stride(1) == 1
             and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and w.data_ptr() % 16 == 0)
+            and w.data_ptr() % 16 == 0 and max(x.stride(0), w.stride(0)) < (1 << 22)
+            and (not silu_mul or w.shape[0] * w.stride(0) * 2 < (1 << 32) - 64))
 
 
-# measured time of one 64-deep K tile of one workgroup, us (70B o-projection, unsplit): the part of it
-# that does not shrink with the tile is the HBM latency the two-tile prefetch cannot cover
-_MID_TILE_US = {(256, 256): 1.6, (256, 128): 1.05, (128, 256): 1.2, (128, 128): 0.75, (64, 256): 1.0}
+# workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
+# TB/s of W that those reach.  Least squares over 930 timings of 20 weight shapes (1.3 to 940 MB) at 1 to 512 rows and every
+# split: 6 to 8 % off in the mean
+_MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (128, 256): (6.5, 0.89, 256, 5.9),
+              (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
+_MID_KSPLITS = (1, 2, 3, 4, 5, 6, 7, 8, 12, 16)
 
 
-# K-split counts the choice is made from (VDAMD_MID_KSPLITS=1,2,4,8,16 restricts it, for A/B measurements)
-_MID_KSPLITS = tuple(int(v) for v in os.environ.get("VDAMD_MID_KSPLITS", "1,2,3,4,5,6,7,8,12,16").split(","))
+def _mid_blocks(m: int, n: int, bm: int, bn: int, ksplit: int) -> int:
+    return -(-n // bn) * ksplit * -(-m // bm)
 
 
-def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int) -> float:
-    """Modelled run time in us: rounds of workgroups x K tiles x time per tile (at least the HBM time
-    of W), plus the fp32 slab round trip and the reduce launch when K is split."""
-    blocks = -(-n // bn) * ksplit * -(-m // bm)
-    rounds = -(-blocks // 256)
-    main = max(rounds * (k / 64 / ksplit) * _MID_TILE_US[(bm, bn)], n * k * 2 / 5.0e6)
-    slabs = (3.0 + 2 * ksplit * m * n * 4 / 3.5e6) if ksplit > 1 else 0.0
-    return 6.0 + main + slabs
+def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int, reduced: bool) -> float:
+    """Modelled run time in us: rounds of workgroups x K tiles x time per tile, at least that of reading its part of W, plus
+    the fp32 slabs, written and read again, and the launch that sums them up."""
+    fixed, tile_us, slots, tbs = _MID_TILES[(bm, bn)]
+    blocks = _mid_blocks(m, n, bm, bn, ksplit)
+    left = blocks % slots
+    again = 1.25 if bn == 128 and slots == 256 else 1.1     # a CU's one workgroup fills and drains its ring in every round
+
+    def round_us(count):                   # per K tile of `count` workgroups side by side: the full rate once most CUs read
+        return max(tile_us, bn * 128 * count / (tbs * 1e6) / min(1.0, 0.5 + count / 440)) * (again if blocks > slots else 1.0)
+    main = (k / 64 / ksplit) * (blocks // slots * round_us(slots) + (round_us(left) if left else 0.0))
+    slabs = ((3.0 if reduced else 0.0) + ksplit * m * n * 4 * 0.4e-6) if ksplit > 1 else 0.0
+    return fixed + main + slabs
 
 
-def mid_choose(m: int, n: int, k: int) -> Tuple[int, int, int]:
+def mid_choose(m: int, n: int, k: int, reduced: bool = True) -> Tuple[int, int, int]:
     """``(bm, bn, ksplit)`` with the smallest modelled time.  The row tile covers all of M up to 256
     (W is then read from HBM once); splitting K buys parallelism and costs slab traffic."""
     best = None
-    for (bm, bn) in _MID_TILE_US:
-        if bm < min(m, 256) or (bm == 64 and m > 48 and k < 2 * n):
+    for (bm, bn) in _MID_TILES:
+        if bm < min(m, 256) or (bm > 64 and bm >= 4 * m):
             continue
-        # (counts that are not powers of two as well: a 70B qkv projection's 40 column tiles fill 240 of the
-        # 256 CUs at 6, 160 at 4)
+        # (counts that are not powers of two as well: a 70B qkv projection's 80 column tiles fill 240 of the
+        # 256 CUs at 3, 160 at 2)
         for ksplit in _MID_KSPLITS:
-            if k // 64 // ksplit < 4:
+            if ksplit > 1 and k // 64 // ksplit < (4 if ksplit <= 8 else 8):
                 break
-            e = _mid_estimate(m, n, k, bm, bn, ksplit)
+            e = _mid_estimate(m, n, k, bm, bn, ksplit, reduced)
             if best is None or e < best[0]:
                 best = (e, bm, bn, ksplit)
     return best[1], best[2], best[3]
 
 
-def mid_profitable(m: int, n: int, k: int) -> bool:
-    """Where this kernel beats the library GEMM on MI355X (benchmarks/stream_gemm_sweep.py, padded weight
-    rows): outputs too narrow to fill the chip with the library's tiles.  Down-projection shapes
-    (K >= 2 N) from 48 rows, square-ish ones from 128 rows (from 48 when K >= 8192 and N <= 8192);
-    very wide outputs (a 70B gate_up) stay with the library, which already has enough tiles there."""
-    if m <= 16 or m > 256 or n > 12288 or k < 2048:
+def mid_profitable(m: int, n: int, k: int, reduced: bool = True) -> bool:
+    """Where this kernel beats the library GEMM on MI355X (padded weight rows, in graphs).  Where the next kernel sums the
+    K-split slabs (not ``reduced``): one row through an 8B qkv projection 11.2 against 16.2 us, 2048 x 2048 5.5 / 8.5, but
+    not once the slabs outweigh a small W (2048 x 2048 at 128 and 256 rows 9.9 / 8.9 and 13.3 / 10.2, 3072 x 3072 at 256
+    16.5 / 17.7; 4608 x 3072 18.3 / 32).  With a reduction of its own (4 to 9 us): 48 rows into K >= 2 N, 128 into squarer
+    shapes (from 48 when K >= 8192 and N <= 8192); small W stay with the library (3072 x 2048 at 256 rows 21 / 11).
+    Outputs wide enough to fill the chip unsplit: always (an LM head of 128256 x 4096 at 1 / 64 / 256 rows 164 / 200 / 252 us,
+    the library 190 / 222 / 309).  Above 256 rows W is read twice: only where the library's tiles leave the chip idle as well
+    (8192 x 28672 at 384 and 512 rows 183 and 186 us / 203 and 316; 4096 x 14336 52 and 57 / 78 and 88)."""
+    if m <= 0 or m > MID_MAX_M or n < 512 or k < 1024:
         return False
-    if k >= 2 * n:
-        return m >= 48
-    if m >= 128:
-        return True
-    return m >= 48 and n <= 8192 and k >= 8192
+    if m > 256:
+        return k >= 2 * n and n * k >= 12 << 20
+    bm, bn, ksplit = mid_choose(m, n, k, reduced)
+    if ksplit == 1:
+        return _mid_blocks(m, n, bm, bn, 1) >= 192 and k >= 2048
+    if not reduced:
+        return n * k >= (2 << 20 if m <= 64 else 8 << 20 if m <= 128 else 12 << 20)
+    if n > 12288 or k < 2048 or n * k < 12 << 20:
+        return False
+    return m >= 128 or (m >= 48 and (k >= 2 * n or (n <= 8192 and k >= 8192)))
+
+
+MID_SILU_MIN_N, MID_SILU_MIN_K = 24576, 4096
+
+
+def mid_silu_profitable(m: int, n: int, k: int) -> bool:
+    """``[gate ; up]`` with the activation in the epilogue: outputs whose unsplit tiles fill the chip (14336 + 14336 columns:
+    224 of 128), over K long enough that filling and draining the ring is little of it.  8B at 1, 48 and 256 rows 41, 42 and
+    62 us (``stream_gemm`` 47, library and activation 69 and 77), 70B 151, 157 and 190 (162, 166, 215)."""
+    return 0 < m <= 256 and n >= MID_SILU_MIN_N and k >= MID_SILU_MIN_K
 
 
 def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, ksplit: Optional[int] = None,
              bm: Optional[int] = None, bn: Optional[int] = None, variant: Optional[int] = None,
-             partials: bool = False) -> Optional[torch.Tensor]:
+             partials: bool = False, silu_mul: bool = False) -> Optional[torch.Tensor]:
     """``x [M<=512, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
-    fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit)."""
-    assert mid_supported(x, w), (x.shape, x.stride(), w.shape, w.stride(), x.dtype)
+    fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit).  ``silu_mul``:
+    ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  A tile wider than the kernel is built for
+    runs as its widest; ``variant`` names what is one kernel now and is accepted as before."""
+    assert mid_supported(x, w, silu_mul), (x.shape, x.stride(), w.shape, w.stride(), x.dtype)
+    assert not (silu_mul and (partials or (ksplit or 1) != 1))
     m, k = x.shape
     n = w.shape[0]
-    a, b, c = mid_choose(m, n, k)
+    if silu_mul:
+        a, b = min(((t for t in _MID_TILES if t[0] >= m or t[0] == 256)), key=lambda t: _mid_estimate(m, n, k, *t, 1, False))
+        c = 1
+    else:
+        a, b, c = mid_choose(m, n, k, not partials)
     bm = a if bm is None else bm
-    bn = b if bn is None else bn
+    bn = min(b if bn is None else bn, max(v for u, v in _MID_TILES if u == bm))
     ksplit = c if ksplit is None else ksplit
     assert 1 <= ksplit <= k // 64
-    if variant is None:
-        variant = MID_VARIANT
-    if variant < 0:
-        variant = 1 if bm == 256 and bn <= 256 else 0
     if partials:
         if ksplit <= 1:
             return None
         partial = torch.empty((ksplit, m, n), dtype=torch.float32, device=x.device)
         _check(_LIB.vdamd_mid_gemm(None, n, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), partial.data_ptr(),
-                                   m, n, k, ksplit, bm, bn, variant, _dt(x), _stream()), "mid_gemm (partial sums)")
+                                   m, n, k, ksplit, bm, bn, EPI_NONE, _dt(x), _stream()), "mid_gemm (partial sums)")
         return partial
+    n_out = n // 2 if silu_mul else n
     if out is None:
-        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    assert out.shape == (m, n) and out.dtype == x.dtype and out.stride(1) == 1 and out.data_ptr() % 8 == 0
+        out = torch.empty((m, n_out), dtype=x.dtype, device=x.device)
+    assert out.shape == (m, n_out) and out.dtype == x.dtype and out.stride(1) == 1 and out.data_ptr() % 8 == 0
     partial = torch.empty(ksplit * m * n, dtype=torch.float32, device=x.device) if ksplit > 1 else None
     _check(_LIB.vdamd_mid_gemm(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                                None if partial is None else partial.data_ptr(), m, n, k, ksplit, bm, bn,
-                               variant, _dt(x), _stream()), "mid_gemm")
+                               EPI_SILU_MUL if silu_mul else EPI_NONE, _dt(x), _stream()), "mid_gemm")
     return out
 
 
 # ------------------------------------- 256 x 256 tile LDS-DMA GEMM, M >= 512
 BIG_MIN_M = 512
-# with the SiLU*mul epilogue a single full row of tiles already beats library GEMM + activation kernel
-# (70B gate_up at 256 rows: 216 us against 229 + 9; profiles/r2_big_gemm_vs_library.txt)
+# with the SiLU*mul epilogue a single full row of tiles already beats library GEMM + activation kernel (70B gate_up at 256
+# rows: 216 us against 229 + 9; profiles/r2_big_gemm_vs_library.txt); where mid_gemm takes the shape it is ahead of both (190)
 BIG_MIN_M_SILU = 240
 BIG_VARIANT = int(os.environ.get("VDAMD_BIG_GEMM_VARIANT", "0"))
 
