@@ -2,7 +2,7 @@
 // inverse-CDF sampling, one 1024-thread workgroup per logits row.
 //
 // Semantics match ops/torch_ref.py::sample (descending order, ties by index);
-// the thresholds and the draw are found without sorting the row, see sample_by_bins and sample_by_counts.
+// the thresholds and the draw are found without sorting the row, see sampling_row.inc and sample_by_counts.
 #include "common.h"
 
 namespace {
@@ -113,13 +113,14 @@ __device__ __forceinline__ unsigned sig_of(unsigned bits) {
 }
 __device__ __forceinline__ int lsb_of(unsigned bits) { return (int)max(bits >> 23, 1u) - 150; }
 
+// what sample_by_counts keeps beside the counts
+struct CountShared { unsigned low, inf, lo, hi, counted, of_stretch[128]; };
 struct SampleShared {
   double wmass[16];
   unsigned wcnt[16];
   double mass, above_mass;
   unsigned above_cnt, cnt, n_list;
   int best, n, token, bad;
-  unsigned low, inf, lo, hi, counted, of_stretch[128];
 };
 
 // exclusive scan of (count, mass) over the block in thread order; totals to every thread
@@ -210,165 +211,6 @@ template <bool WIDE> struct ListShared {
   unsigned long long list[CAP];
 };
 
-// One workgroup per row.  With weights e = exp((logit - max) / T) in descending order (ties by index) an entry is kept
-// while fewer than K lie in front of it, less than M of mass lies in front of it, and it is at least min_p; the sampled
-// entry is the last one in front of which less than `u * kept mass` lies: the same question, asked twice.
-// It is answered without sorting the row: one pass for the maximum, one that counts the weights into 2048 bins by
-// their leading bits (exponent and four bits more), a scan over the bins that finds the bin the answer lies in, and a
-// pass that lists that bin's entries (a thousand of a Gaussian row of 128k) in LDS, where they are sorted and summed up.
-// A bin of more than 4096 entries is cut by the next bits first, and one of equal weights is walked by index.
-// Masses are whole multiples of a bin's last bit, added up in 64-bit integers and doubles: no result depends on the
-// order of additions.
-// For 32-bit logits, and the 16-bit rows that sample_by_counts leaves.  A row is read three or four times: 256 rows of 128256
-// fp32 logits 123 us, one row 62 (a pass over them at the rate of a large copy: 27); the LDS atomics of the counting pass take
-// 25 us, the two sorts of about a thousand entries 10 us each.
-template <typename T, bool WIDE>
-__device__ int sample_by_bins(const T* row, int V, float inv_t, unsigned k, float tp, float mp, float u, ListShared<WIDE>& ls,
-                              SampleShared& s, float* red) {
-  Hist<WIDE>&h1 = ls.h1, &h2 = ls.h2;
-  unsigned long long* list = ls.list;
-  h1.clear();
-  if (threadIdx.x == 0) s.bad = 0;
-  const float sign = inv_t < 0.f ? -1.f : 1.f, to_exp2 = inv_t * 1.4426950408889634f;
-  float mx = -INFINITY;
-  for_row(row, V, [&](float v, int) { mx = fmaxf(mx, v * sign); });
-  const float top = sign * block_max(mx, red);
-  // (the difference first: the largest entry weighs exactly 1, and every pass sees the same bits)
-  auto weight = [&](float v) { return __float_as_uint(fast_exp2((v - top) * to_exp2)); };
-  int bad = 0;
-  for_row(row, V, [&](float v, int) {
-    const unsigned w = weight(v);
-    if (w >= NORMAL_END) bad = 1;                  // (NaN, or a row of infinities)
-    else if (w) h1.add(w >> 19, w & 0x7ffffu);     // (a weight of zero is never sampled and adds nothing)
-  });
-  if (bad) s.bad = 1;
-  __syncthreads();
-  if (s.bad) return 0;
-
-  unsigned kept = (unsigned)V;
-  double mass = 0;
-  int listed = -1;                                 // the bin whose entries the list holds
-  int token = 0;
-  // step 0: how much is kept; step 1: the entry drawn from it
-  for (int step = 0; step < 2; ++step) {
-    const unsigned minb = step == 0 && mp > 0.f ? __float_as_uint(fminf(mp, 1.f)) : 0u;
-    double M;
-    if (step == 0) {
-      scan_bins<WIDE>(h1, 0u, 19, 0, 0u, 0.0, 1u, 1.0, s);           // (its total is the mass of the row)
-      const double z = s.mass;
-      mass = z;
-      if (k >= (unsigned)V && tp >= 1.f && minb == 0u) continue;     // everything is kept
-      M = tp >= 1.f ? 1e300 : fmax((double)tp * z, 1e-300);          // (the first entry always is)
-    } else {
-      M = fmax((double)u * mass, 1e-300);
-    }
-    const unsigned K = step == 0 ? k : kept;
-    unsigned prefix = 0u;
-    int shift = 19;
-    scan_bins<WIDE>(h1, 0u, 19, (int)(minb >> 19), 0u, 0.0, K, M, s);
-    if (s.best < 0) break;                         // (no weights at all)
-    const int bin1 = s.best;
-    prefix = (unsigned)bin1 << 19;
-    bool some = true;
-    while (some && s.cnt > CAP && shift > 0) {
-      const int next = shift == 19 ? 8 : 0;
-      const unsigned above_cnt = s.above_cnt;
-      const double above_mass = s.above_mass;
-      h2.clear();
-      __syncthreads();
-      for_row(row, V, [&](float v, int) {
-        const unsigned w = weight(v);
-        if (w < NORMAL_END && w >> shift == prefix >> shift && w && w >= minb)
-          h2.add((w >> next) & ((1u << (shift - next)) - 1u), w & ((1u << next) - 1u));
-      });
-      __syncthreads();
-      scan_bins<WIDE>(h2, prefix, next, 0, above_cnt, above_mass, K, M, s);
-      some = s.best >= 0;
-      if (some) prefix |= (unsigned)s.best << next;
-      else if (threadIdx.x == 0) { s.above_cnt = above_cnt; s.above_mass = above_mass; }
-      shift = next;
-      __syncthreads();
-    }
-    const unsigned above_cnt = s.above_cnt;
-    const double above_mass = s.above_mass;
-    const int cnt = some ? (int)s.cnt : 0;
-    if (cnt > CAP) {
-      // entries of one and the same weight, in index order
-      const double v = sig_of(prefix) * pow2(lsb_of(prefix));
-      const double fit = ceil((M - above_mass) / v);
-      int n = (int)fmin(fmin((double)cnt, (double)(K - above_cnt)), fmax(fit, 1.0));
-      if (step == 0) { kept = above_cnt + n; mass = above_mass + n * v; continue; }
-      int seen = 0;                                // in front of this stretch of the row
-      for (int base = 0; base < V; base += ST) {
-        const int i = base + threadIdx.x;
-        const bool hit = i < V && weight(to_f(row[i])) == prefix;
-        unsigned ec;
-        double em, total;
-        block_scan(hit ? 1u : 0u, hit ? 1.0 : 0.0, ec, em, total, s);
-        if (hit && seen + (int)ec == n - 1) s.token = i;
-        seen += (int)total;
-        if (seen >= n) break;
-      }
-      __syncthreads();
-      token = s.token;
-      break;
-    }
-    if (listed != bin1) {
-      listed = shift == 19 ? bin1 : -1;
-      if (threadIdx.x == 0) s.n_list = 0;
-      __syncthreads();
-      if (cnt > 0)
-        for_row(row, V, [&](float v, int i) {
-          const unsigned w = weight(v);
-          if (w < NORMAL_END && w >> shift == prefix >> shift && w && w >= minb) {
-            const unsigned pos = atomicAdd(&s.n_list, 1u);
-            if (pos < CAP) list[pos] = ((unsigned long long)w << 32) | (0xffffffffu - (unsigned)i);
-          }
-        });
-      __syncthreads();
-      sort_list(list, min((int)s.n_list, CAP));
-    }
-    const int n_list = min((int)s.n_list, CAP);
-    // four entries per thread, summed up in order: how many are in front of the border
-    unsigned w4[4];
-    double m4 = 0;
-    const int at = 4 * (int)threadIdx.x;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      w4[e] = at + e < n_list ? (unsigned)(list[at + e] >> 32) : 0u;
-      m4 += sig_of(w4[e]) * pow2(lsb_of(w4[e]));
-    }
-    unsigned ec;
-    double em, total;
-    block_scan(0u, m4, ec, em, total, s);
-    if (threadIdx.x == 0) { s.n = 0; s.mass = above_mass; }
-    __syncthreads();
-    double front = above_mass + em, upto = front;
-    int n = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (at + e < n_list && above_cnt + at + e < K && front < M) {
-        n = at + e + 1;
-        front += sig_of(w4[e]) * pow2(lsb_of(w4[e]));
-        upto = front;
-      } else {
-        front = 1e301;
-      }
-    }
-    if (n) atomicMax(&s.n, n);
-    __syncthreads();
-    if (n && s.n == n) {
-      s.mass = upto;
-      s.token = (int)(0xffffffffu - (unsigned)list[n - 1]);
-    }
-    __syncthreads();
-    if (step == 0) { kept = above_cnt + s.n; mass = s.mass; }
-    else if (s.n) token = s.token;
-    __syncthreads();
-  }
-  return token;
-}
-
 constexpr int PATTERNS = 65536;
 
 // The 16-bit patterns of T in the order of their weights: place d = 0 .. 65535 falls with the value (`flip`: rises)
@@ -426,7 +268,7 @@ template <typename T, typename F, typename G> __device__ __forceinline__ void fo
   if (rest < V) g((unsigned)raw[rest], rest);
 }
 
-// Rows of 16-bit logits: the same two questions (see sample_by_bins), answered from how often each of the 65536 patterns
+// Rows of 16-bit logits: the same two questions (see sampling_row.inc), answered from how often each of the 65536 patterns
 // occurs.  One pass over the row counts them (16 bits each, 128 KB of LDS); the ones that occur - a few thousand - are packed
 // into a list in order, weighed once each, and summed up; what is kept and the pattern that the draw falls on follow from the
 // list, with no further look at the row and no sort.  A second pass finds the element: the drawn pattern's elements come in
@@ -442,7 +284,7 @@ template <typename T, typename F, typename G> __device__ __forceinline__ void fo
 // masks fill rows with, are counted apart, in registers.
 template <typename T>
 __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, float tp, float mp, float u, unsigned* tab,
-                                SampleShared& s) {
+                                SampleShared& s, CountShared& cs) {
   using O = Order16<T>;
   typedef unsigned Vec __attribute__((ext_vector_type(4)));
   if (V > 1 << 23) return -1;
@@ -451,7 +293,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
 #pragma unroll
   for (int j = 0; j < PATTERNS / 2 / (4 * ST); ++j) *reinterpret_cast<Vec*>(tab + 4 * (j * ST + tid)) = Vec{0u, 0u, 0u, 0u};
-  if (tid == 0) { s.bad = 0; s.low = 0; s.inf = 0; s.counted = 0; }
+  if (tid == 0) { s.bad = 0; cs.low = 0; cs.inf = 0; cs.counted = 0; }
   __syncthreads();
   // ---- how often each pattern occurs
   unsigned low = 0, inf = 0, nan = 0;
@@ -479,8 +321,8 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         }
       },
       [&](unsigned x, int) { one(x); });
-  if (low) atomicAdd(&s.low, low);
-  if (inf) atomicAdd(&s.inf, inf);
+  if (low) atomicAdd(&cs.low, low);
+  if (inf) atomicAdd(&cs.inf, inf);
   if (nan) s.bad = 1;
   __syncthreads();
   // ---- those that occur, in order, as (place, count) words in the counts' stead: 128 stretches of 512 places, eight a lane,
@@ -512,7 +354,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
           c += (lo != 0) + (hi != 0);
           sum += lo + hi;
         }
-        if (sum) atomicAdd(&s.counted, sum);
+        if (sum) atomicAdd(&cs.counted, sum);
         unsigned before = 0;
 #pragma unroll
         for (int bit = 0; bit < 4; ++bit) {
@@ -522,15 +364,15 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         }
         pos[j] = before;
       }
-      if (lane == 0) s.of_stretch[j * (ST / 64) + wid] = total;
+      if (lane == 0) cs.of_stretch[j * (ST / 64) + wid] = total;
     }
     __syncthreads();
-    const unsigned even = s.of_stretch[2 * lane], odd = s.of_stretch[2 * lane + 1];
+    const unsigned even = cs.of_stretch[2 * lane], odd = cs.of_stretch[2 * lane + 1];
     unsigned upto = even + odd;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { const unsigned x = __shfl_up(upto, o, 64); if (lane >= o) upto += x; }
     n = __shfl(upto, 63, 64);
-    if (s.counted != (unsigned)V - s.low - s.inf && !s.bad) return -1;
+    if (cs.counted != (unsigned)V - cs.low - cs.inf && !s.bad) return -1;
     if (n > PATTERNS / 2) return -1;
 #pragma unroll
     for (int j = 0; j < ROUNDS; ++j) {
@@ -546,12 +388,12 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
     }
     __syncthreads();
   }
-  const unsigned lows = s.low;
+  const unsigned lows = cs.low;
   // the row's largest entry (its place: the one in front of all); NaN, and an infinity there, are no distribution
   const unsigned first = n ? tab[0] >> 16 : (lows ? O::LOWEST : O::LOWEST + 1);
   const float top = O::value(first, flip);
   auto weight = [&](unsigned d) { return __float_as_uint(fast_exp2((O::value(d, flip) - top) * to_exp2)); };
-  if (s.bad || first <= O::FIRST || (s.inf && weight(O::LOWEST + 1) >= NORMAL_END)) return 0;
+  if (s.bad || first <= O::FIRST || (cs.inf && weight(O::LOWEST + 1) >= NORMAL_END)) return 0;
   // ---- entry n is the type's lowest value; a thread has `per` of them in a row
   const unsigned per = (n + 1 + ST - 1) / ST, e0 = min(per * tid, n + 1), e1 = min(e0 + per, n + 1);
   auto entry = [&](unsigned e, unsigned& d, unsigned& c) {
@@ -620,19 +462,19 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
   // ---- the rank-th element (from 1) of the patterns that weigh as much: those beside the found one count in front of it
   const int found = s.best;
   const unsigned wanted = s.cnt;
-  if (tid == 0) { s.n_list = rank; s.lo = 0xffffu; s.hi = 0u; }
+  if (tid == 0) { s.n_list = rank; cs.lo = 0xffffu; cs.hi = 0u; }
   __syncthreads();
   for (unsigned e = e0; e < e1; ++e) {
     unsigned d, c;
     entry(e, d, c);
     if (!c || weight(d) != wanted) continue;
-    atomicMin(&s.lo, d);
-    atomicMax(&s.hi, d);
+    atomicMin(&cs.lo, d);
+    atomicMax(&cs.hi, d);
     if ((int)e < found) atomicAdd(&s.n_list, c);
   }
   __syncthreads();
   rank = s.n_list;
-  const unsigned lo = s.lo, span = s.hi - lo;
+  const unsigned lo = cs.lo, span = cs.hi - lo;
   // ---- how many of them each 512 elements hold: counter 0 for what lies in front of the first 16-byte border
   const int head = min(V, (int)(((16u - ((unsigned)(uintptr_t)row & 15u)) & 15u) / sizeof(T)));
   const int nvec = (V - head) / 8, parts = (nvec + 63) / 64;
@@ -721,48 +563,44 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
   return s.token;
 }
 
+// 32-bit logits
 template <typename T, bool WIDE>
 __global__ __launch_bounds__(ST) void sample_kernel(int* __restrict__ out, const T* __restrict__ logits, int V,
                                                     long stride, const float* __restrict__ temperature,
                                                     const int* __restrict__ top_k, const float* __restrict__ top_p,
                                                     const float* __restrict__ min_p,
                                                     const float* __restrict__ uniform) {
-  constexpr bool COUNTED = sizeof(T) == 2;
-  __shared__ union {
-    ListShared<WIDE> bins;
-    unsigned counts[COUNTED ? PATTERNS / 2 : 1];
-  } sh;
+  __shared__ Hist<WIDE> h1, h2;
+  __shared__ unsigned long long list[CAP];
   __shared__ SampleShared s;
   __shared__ float red[16];
   __shared__ int s_idx;
-  const int b = blockIdx.x;
-  const T* row = logits + b * stride;
-  const float temp = temperature[b];
-  // ---- greedy row: plain argmax (lowest index on ties)
-  if (temp == 0.f) {
-    ArgMax best{-INFINITY, 0x7fffffff};
-    for_row(row, V, [&](float v, int i) {
-      if (v > best.v || (v == best.v && i < best.i)) best = ArgMax{v, i};
-    });
-    const float mx = block_max(best.v, red);
-    const int cand = (best.v == mx) ? best.i : 0x7fffffff;
-    if (threadIdx.x == 0) s_idx = 0x7fffffff;
-    __syncthreads();
-    atomicMin(&s_idx, cand);
-    __syncthreads();
-    if (threadIdx.x == 0) out[b] = s_idx == 0x7fffffff ? 0 : s_idx;
-    return;
-  }
-  const float inv_t = 1.f / temp;
-  const unsigned k = top_k[b] <= 0 || top_k[b] > V ? (unsigned)V : (unsigned)top_k[b];
-  const float tp = top_p[b], mp = min_p[b], u = uniform[b];
-  int token = -1;
-  if constexpr (COUNTED) token = sample_by_counts(row, V, inv_t, k, tp, mp, u, sh.counts, s);
-  if (token < 0) {
-    __syncthreads();
-    token = sample_by_bins<T, WIDE>(row, V, inv_t, k, tp, mp, u, sh.bins, s, red);
-  }
-  if (threadIdx.x == 0) out[b] = token;
+  static_assert(sizeof(T) == 4, "");
+  unsigned* const tab = nullptr;
+  CountShared cs;
+#include "sampling_row.inc"
+}
+
+// 16-bit logits: the counts take the place of the histograms
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(ST) void sample16_kernel(int* __restrict__ out, const T* __restrict__ logits, int V,
+                                                    long stride, const float* __restrict__ temperature,
+                                                    const int* __restrict__ top_k, const float* __restrict__ top_p,
+                                                    const float* __restrict__ min_p,
+                                                    const float* __restrict__ uniform) {
+  __shared__ union {
+    ListShared<WIDE> bins;
+    unsigned counts[PATTERNS / 2];
+  } sh;
+  __shared__ SampleShared s;
+  __shared__ CountShared cs;
+  __shared__ float red[16];
+  __shared__ int s_idx;
+  static_assert(sizeof(T) == 2, "");
+  Hist<WIDE>&h1 = sh.bins.h1, &h2 = sh.bins.h2;
+  unsigned long long* const list = sh.bins.list;
+  unsigned* const tab = sh.counts;
+#include "sampling_row.inc"
 }
 
 }  // namespace
@@ -784,18 +622,18 @@ VDAMD_API int vdamd_sample(int* out, const void* logits, int B, int V, long stri
                            const int* top_k, const float* top_p, const float* min_p, const float* uniform,
                            int dtype, hipStream_t s) {
   if (B == 0) return 0;
-#define L(TY)                                                                                                       \
+#define L(KERNEL, TY)                                                                                                       \
   do {                                                                                                              \
     if (V <= (1 << 22))                                                                                             \
-      hipLaunchKernelGGL((sample_kernel<TY, false>), dim3(B), dim3(ST), 0, s, out, (const TY*)logits, V, stride,    \
+      hipLaunchKernelGGL((KERNEL<TY, false>), dim3(B), dim3(ST), 0, s, out, (const TY*)logits, V, stride,    \
                          temperature, top_k, top_p, min_p, uniform);                                                \
     else                                                                                                            \
-      hipLaunchKernelGGL((sample_kernel<TY, true>), dim3(B), dim3(ST), 0, s, out, (const TY*)logits, V, stride,     \
+      hipLaunchKernelGGL((KERNEL<TY, true>), dim3(B), dim3(ST), 0, s, out, (const TY*)logits, V, stride,     \
                          temperature, top_k, top_p, min_p, uniform);                                                \
   } while (0)
-  if (dtype == DT_BF16) L(bf16_t);
-  else if (dtype == DT_F16) L(f16_t);
-  else if (dtype == DT_F32) L(float);
+  if (dtype == DT_BF16) L(sample16_kernel, bf16_t);
+  else if (dtype == DT_F16) L(sample16_kernel, f16_t);
+  else if (dtype == DT_F32) L(sample_kernel, float);
   else return -2;
 #undef L
   HIP_LAUNCH_CHECK();
