@@ -68,7 +68,11 @@ __host__ __device__ constexpr Layout layout_of(int DP, int VP, bool delta) {
 }
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p) { return (float)(*p); }
-__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+// (both sides are formed: a branch around the library functions would keep their latencies from filling each other)
+__device__ __forceinline__ float softplus_f(float x) {
+  const float l = log1pf(expf(x > 20.f ? 20.f : x));
+  return x > 20.f ? x : l;
+}
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
@@ -173,26 +177,32 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// one step of a running product over the 16 lanes of a row; lanes without a source multiply by one
-template <int CTRL> __device__ __forceinline__ float dpp_mul(float v) {
-  return v * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
 __device__ __forceinline__ float turn(float v) {                // of the lane in front, the first of 16 from the last
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
 }
-__device__ __forceinline__ float prefix_product(float v) {       // lanes up to and including this one
-  v = dpp_mul<0x111>(v);
-  v = dpp_mul<0x112>(v);
-  v = dpp_mul<0x114>(v);
-  return dpp_mul<0x118>(v);
+// Products over the 16 lanes of a row, four values side by side: the lanes up to and including this one, and those behind it.  One
+// instruction a step (a lane without a source keeps its value); from the builtin the compiler makes three, and waits between
+// them.  (A step reads what was written four instructions before; it has to be two at least, and the s_nop sees to the first.)
+#define MUL4(STEP)                                               \
+  "v_mul_f32_dpp %0, %0, %0 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_mul_f32_dpp %1, %1, %1 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_mul_f32_dpp %2, %2, %2 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_mul_f32_dpp %3, %3, %3 " STEP " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void prefix_products(float& a, float& b, float& c, float& d) {
+  asm("s_nop 1\n\t" MUL4("row_shr:1") MUL4("row_shr:2") MUL4("row_shr:4") MUL4("row_shr:8")
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
-__device__ __forceinline__ float suffix_product(float v) {       // lanes behind this one
-  v = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, v), 0x101, 0xf, 0xf, false));
-  v = dpp_mul<0x101>(v);
-  v = dpp_mul<0x102>(v);
-  v = dpp_mul<0x104>(v);
-  return dpp_mul<0x108>(v);
+__device__ __forceinline__ void suffix_products(const f32x4& v, float& a, float& b, float& c, float& d) {
+  a = b = c = d = 1.f;
+  asm("s_nop 1\n\t"
+      "v_mov_b32_dpp %0, %4 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %1, %5 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %2, %6 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %3, %7 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+      MUL4("row_shl:1") MUL4("row_shl:2") MUL4("row_shl:4") MUL4("row_shl:8")
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
 }
+#undef MUL4
 
 __device__ __forceinline__ int chunks_of(const int* qsl, int B, int s) {
   const int n = s < B ? qsl[s + 1] - qsl[s] : 0;
@@ -247,7 +257,9 @@ __device__ __forceinline__ int by_length(const int* qsl, int B, int rank) {
 // (row, reduction index 4 kh + e) and the right one of the matrix instruction and the lane layout of the products
 // over rows (DPP).  Only G k and, in the solve, M and beta b k cross waves, through LDS.
 // Bound by what it writes (112 KB per chunk and head, the delta rule 144: linear attention's 6007 rows x 16 heads, 170 MB,
-// in 74 us) and, with a decay per channel under the delta rule, by their exponentials (200 us for 8017 rows x 16 heads).
+// in 67 us) and, with a decay per channel under the delta rule, by vector instructions (half of the time: 8017 rows x 16 heads
+// 189 us; 215 with a branch around each element's exponentials and their bias loaded inside it, and running products of three
+// instructions a step).
 template <typename T, int KIND, int DP>
 __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   constexpr bool DELTA = KIND >= DELTA_CHANNEL, CHAN = KIND == LINEAR_CHANNEL || KIND == DELTA_CHANNEL;
@@ -273,6 +285,11 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   // ---- the wave's rows: q, k, the decays
   f32x4 q[KB], k[KB], dk[CHAN ? KB : 1];           // dk: the row's decays (raw dt for the delta rule, until below)
   float p[NP], s[NP];
+  // (all on their way at once: loaded where they are used, under the condition there, each was waited for by itself)
+  [[maybe_unused]] float bias[KIND == DELTA_CHANNEL ? 4 * KB : 1];
+  if constexpr (KIND == DELTA_CHANNEL)
+#pragma unroll
+    for (int i = 0; i < 4 * KB; ++i) bias[i] = a.dt_bias[h * a.dim + min(16 * (i / 4) + 4 * kh + i % 4, a.dim - 1)];
   const int valid = min(16, n - (c * C + 16 * wave));            // rows of the wave that exist (none: <= 0)
   const long row0 = q0 + c * C + 16 * wave;
   float* mine = ks + 16 * wave * LD;               // the wave's rows of ks, free until it writes G k there
@@ -326,8 +343,8 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int j = 16 * kb + 4 * kh + e;
-        dk[kb][e] = ok && j < a.dim ? expf(-rate * softplus_f(dk[kb][e] + a.dt_bias[h * a.dim + j])) : 1.f;
+        const float decay = expf(-rate * softplus_f(dk[kb][e] + bias[4 * kb + e]));
+        dk[kb][e] = ok && 16 * kb + 4 * kh + e < a.dim ? decay : 1.f;
       }
   }
   if constexpr (DELTA) {
@@ -351,7 +368,9 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { p[4 * kb + e] = prefix_product(dk[kb][e]); s[4 * kb + e] = suffix_product(dk[kb][e]); }
+      for (int e = 0; e < 4; ++e) p[4 * kb + e] = dk[kb][e];
+      prefix_products(p[4 * kb], p[4 * kb + 1], p[4 * kb + 2], p[4 * kb + 3]);
+      suffix_products(dk[kb], s[4 * kb], s[4 * kb + 1], s[4 * kb + 2], s[4 * kb + 3]);
     }
   } else {
     if (ok) {
