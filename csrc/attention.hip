@@ -64,15 +64,19 @@ __device__ __forceinline__ typename Vec8<T>::type fp8x8_to(uint2 w, float scale)
   return r.v;
 }
 
-// 8 consecutive cache elements starting at element offset `off`: 16 bytes of T, or 8 bytes
-// of e4m3 widened to T (KV8: the cache holds one byte per element, same layouts).
+// 8 consecutive cache elements starting at element offset `off`, as the cache holds them: 16 bytes of T, or 8 bytes of e4m3
+// (KV8: same layouts), which are widened to T where they are multiplied.  (Widened where they are loaded, each load is
+// waited for before the next: the decode kernels were 1.2 to 2.6 times as slow over e4m3 as over 16 bits.)
+template <typename T, bool KV8> struct Raw8 { using type = typename Vec8<T>::type; };
+template <typename T> struct Raw8<T, true> { using type = uint2; };
 template <typename T, bool KV8>
-__device__ __forceinline__ typename Vec8<T>::type ld_kv(const void* cache, long off, float scale) {
-  if constexpr (KV8) {
-    return fp8x8_to<T>(*reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(cache) + off), scale);
-  } else {
-    return ld8<T>(reinterpret_cast<const T*>(cache) + off);
-  }
+__device__ __forceinline__ typename Raw8<T, KV8>::type ld_kv(const void* cache, long off) {
+  if constexpr (KV8) return *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(cache) + off);
+  else return ld8<T>(reinterpret_cast<const T*>(cache) + off);
+}
+template <typename T, typename R> __device__ __forceinline__ typename Vec8<T>::type widen(const R& r) {
+  if constexpr (__is_same(R, uint2)) return fp8x8_to<T>(r, 1.f);
+  else return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -82,16 +86,15 @@ __device__ __forceinline__ typename Vec8<T>::type ld_kv(const void* cache, long 
 //   qpos_hi[n] : largest key index the lane's query row may attend to
 // ---------------------------------------------------------------------------
 // K / V^T fragments of one 32-key group, as loaded from the paged cache.
-template <typename T, int D>
+template <typename T, int D, bool KV8>
 struct KVFrag {
-  typename Vec8<T>::type kfa[D / 32], kfb[D / 32], vf[D / 16];
+  typename Raw8<T, KV8>::type kfa[D / 32], kfb[D / 32], vf[D / 16];
 };
 
 template <typename T, int D, bool KV8>
-__device__ __forceinline__ void load_kv_group(KVFrag<T, D>& f, const void* __restrict__ k_cache,
+__device__ __forceinline__ void load_kv_group(KVFrag<T, D, KV8>& f, const void* __restrict__ k_cache,
                                               const void* __restrict__ v_cache, const int* __restrict__ bt_row,
-                                              int kvh, int Hkv, int block_size, int base, int seq_len,
-                                              float k_scale, float v_scale) {
+                                              int kvh, int Hkv, int block_size, int base, int seq_len) {
   const int lane = threadIdx.x & 63;
   const int r16 = lane & 15, g4 = lane >> 4;
   // ---- K rows for the two interleaved tiles
@@ -103,8 +106,8 @@ __device__ __forceinline__ void load_kv_group(KVFrag<T, D>& f, const void* __res
   const long kb_off = ((blk_b * Hkv + kvh) * block_size + (kb % block_size)) * (long)D + 8 * g4;
 #pragma unroll
   for (int s = 0; s < D / 32; ++s) {
-    f.kfa[s] = ld_kv<T, KV8>(k_cache, ka_off + 32 * s, k_scale);
-    f.kfb[s] = ld_kv<T, KV8>(k_cache, kb_off + 32 * s, k_scale);
+    f.kfa[s] = ld_kv<T, KV8>(k_cache, ka_off + 32 * s);
+    f.kfb[s] = ld_kv<T, KV8>(k_cache, kb_off + 32 * s);
   }
   // ---- V^T rows: this lane's 8 keys are base + 8*g4 .. +7 (one block: block_size % 8 == 0)
   const int vkey = min(base + 8 * g4, seq_len - 1) & ~7;
@@ -112,7 +115,7 @@ __device__ __forceinline__ void load_kv_group(KVFrag<T, D>& f, const void* __res
   const int slab = block_size * 16;                           // elements of one 16-row slab of a block
   const long v_off = (blk_v * Hkv + kvh) * (long)(D / 16) * slab + ((vkey % block_size) >> 3) * 128 + 8 * r16;
 #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) f.vf[dt] = ld_kv<T, KV8>(v_cache, v_off + (long)dt * slab, v_scale);
+  for (int dt = 0; dt < D / 16; ++dt) f.vf[dt] = ld_kv<T, KV8>(v_cache, v_off + (long)dt * slab);
 }
 
 // Score capping (Gemma-2): cap * tanh(score / cap) on the natural-log scale; `s2` and the result are
@@ -126,9 +129,9 @@ __device__ __forceinline__ float soft_cap_log2(float s2, float cap) {
   return t * (cap * 1.4426950408889634f);
 }
 
-template <typename T, int D, int NQ>
+template <typename T, int D, int NQ, bool KV8>
 __device__ __forceinline__ void attend_loaded(
-    const KVFrag<T, D>& f, int base, int seq_len, float scale_log2e, float softcap,
+    const KVFrag<T, D, KV8>& f, int base, int seq_len, float scale_log2e, float softcap,
     const typename Vec8<T>::type (&qf)[NQ][D / 32], f32x4 (&acc)[NQ][D / 16], float (&m)[NQ], float (&l)[NQ],
     const int (&qpos_hi)[NQ], const int (&qpos_lo)[NQ], float alibi_l2 = 0.f) {
   // alibi_l2: this lane's query head's ALiBi slope times log2(e) (0: none); the bias of key k for the
@@ -141,8 +144,8 @@ __device__ __forceinline__ void attend_loaded(
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < D / 32; ++s) {
-      s0 = mfma16(f.kfa[s], qf[n][s], s0);
-      s1 = mfma16(f.kfb[s], qf[n][s], s1);
+      s0 = mfma16(widen<T>(f.kfa[s]), qf[n][s], s0);
+      s1 = mfma16(widen<T>(f.kfb[s]), qf[n][s], s1);
     }
     const int hi = min(qpos_hi[n], seq_len - 1);
     const int lo = qpos_lo[n];           // first key inside the sliding window (0 without one)
@@ -175,7 +178,7 @@ __device__ __forceinline__ void attend_loaded(
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) {
       acc[n][dt] *= alpha;
-      acc[n][dt] = mfma16(f.vf[dt], pf, acc[n][dt]);
+      acc[n][dt] = mfma16(widen<T>(f.vf[dt]), pf, acc[n][dt]);
     }
   }
 }
@@ -185,10 +188,11 @@ __device__ __forceinline__ void attend_group(
     const void* __restrict__ k_cache, const void* __restrict__ v_cache, const int* __restrict__ bt_row, int kvh,
     int Hkv, int block_size, int base, int seq_len, float scale_log2e, float softcap,
     const typename Vec8<T>::type (&qf)[NQ][D / 32], f32x4 (&acc)[NQ][D / 16], float (&m)[NQ], float (&l)[NQ],
-    const int (&qpos_hi)[NQ], const int (&qpos_lo)[NQ], float k_scale, float v_scale, float alibi_l2 = 0.f) {
-  KVFrag<T, D> f;
-  load_kv_group<T, D, KV8>(f, k_cache, v_cache, bt_row, kvh, Hkv, block_size, base, seq_len, k_scale, v_scale);
-  attend_loaded<T, D, NQ>(f, base, seq_len, scale_log2e, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+    const int (&qpos_hi)[NQ], const int (&qpos_lo)[NQ], float alibi_l2 = 0.f) {
+  KVFrag<T, D, KV8> f;
+  load_kv_group<T, D, KV8>(f, k_cache, v_cache, bt_row, kvh, Hkv, block_size, base, seq_len);
+  if constexpr (KV8) __builtin_amdgcn_sched_barrier(0);        // (all loads are on their way before anything is widened)
+  attend_loaded<T, D, NQ, KV8>(f, base, seq_len, scale_log2e, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
 }
 
 // ---------------------------------------------------------------------------
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   // measured 3-8% slower than letting 4 resident workgroups per CU hide the latency
   for (int g = g_begin + wid; g < g_end; g += 4)
     attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                               scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, 1.f, 1.f, alibi_l2);
+                               scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
 
   float lsum = l[0];
   lsum += __shfl_xor(lsum, 16, 64);
@@ -323,7 +327,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
   const float alibi_l2 = (alibi != nullptr && r16 < nq) ? alibi[qh0 + r16] * LOG2E_F : 0.f;
   for (int g = qpos_lo[0] >> 5; g < n_groups; ++g)
     attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                               scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, 1.f, 1.f, alibi_l2);
+                               scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
   float lsum = l[0];
   lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
@@ -411,7 +415,7 @@ __global__ __launch_bounds__(256) void paged_prefill_kernel(
   const float alibi_l2 = alibi != nullptr ? alibi[h] * LOG2E_F : 0.f;
   for (int g = g_first; g < n_groups; ++g)
     attend_group<T, D, NQ, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                                scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, 1.f, 1.f, alibi_l2);
+                                scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
     float lsum = l[n];
