@@ -252,9 +252,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 
   // no register double-buffering here: it halves the occupancy (202 VGPRs) and
   // measured 3-8% slower than letting 4 resident workgroups per CU hide the latency
-  for (int g = g_begin + wid; g < g_end; g += 4)
-    attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                               scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+  if constexpr (KV8 && D <= 64) {
+    // bytes take half the registers: two groups at a time (40 rows of 9000 keys, 8 heads of 64: 112 -> 92 us; of 128 they do not
+    // fit the four waves' registers, 175 -> 290, and with three waves nothing is gained, 170)
+    int g = g_begin + wid;
+    for (; g + 4 < g_end; g += 8) {
+      KVFrag<T, D, KV8> f[2];
+      load_kv_group<T, D, KV8>(f[0], k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len);
+      load_kv_group<T, D, KV8>(f[1], k_cache, v_cache, bt_row, kvh, Hkv, block_size, (g + 4) * 32, seq_len);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        attend_loaded<T, D, 1, KV8>(f[i], (g + 4 * i) * 32, seq_len, scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo,
+                                    alibi_l2);
+    }
+    if (g < g_end)
+      attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
+                                 scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+  } else {
+    for (int g = g_begin + wid; g < g_end; g += 4)
+      attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
+                                 scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+  }
 
   float lsum = l[0];
   lsum += __shfl_xor(lsum, 16, 64);
