@@ -33,7 +33,7 @@
 //    tiles of a few wide ones; neighbouring row tiles are mostly one expert's.  Table entries without rows (experts held
 //    elsewhere, the table's end) are skipped.
 //    36006 rows over 64 experts of 2048 x 1408 (gate and up with SiLU*mul, then down), traced: 416 - 464 and 234 - 267 us against
-//    979 + 50 (activation) and 517 us of 128-row tiles with W straight from memory (skinny_gemm.hip); 530 us of matrix
+//    979 + 50 (activation) and 517 us of 128-row tiles with W straight from memory; 530 us of matrix
 //    instructions at the rate of the library's 8192^3 product.  Partial tiles are multiplied whole: 768 rows for 563.  Neither that
 //    nor the first read of an expert's weights alone is the bound: without the multiplications of empty sub-tiles the time stays
 //    the same (and the plain form loses 3.5 %), and so it does with every unit's K loop begun at another place.

@@ -1142,6 +1142,41 @@ def test_mid_gemm_rings_of_few_tiles_and_silu(dtype, m, n, k):
             assert got.shape == (m, h) and ((got.double() - act).abs() <= act_bound).all(), (bm, bn)
 
 
+@pytest.mark.parametrize("tile_rows", [16, 64, 128])
+@pytest.mark.parametrize("n,k,pad,rows", [(96, 128, 0, [1, 0, 16, 3]), (1056, 256, 8, [64, 65, 0, 2, 127]), (416, 384, 0, [256, 1, 0, 130])])
+def test_grouped_products_on_the_rings(n, k, pad, rows, tile_rows):
+    """Every tile of the grouped form against fp32: experts without rows, one row, whole and one more than whole tiles; rows read
+    through a list; SiLU * up; rows of no tile stay as they are.  Bounds as above."""
+    from vllm_distributed_amd.ops import hip
+    g, total = len(rows), sum(rows)
+    w = (_rand(g, n, k) * 0.05).contiguous()
+    x = _rand(total + 9, k + pad)[:, :k]
+    src = torch.randperm(total + 9, device=DEV)[:total].to(torch.int32)
+    table, at = [], 0
+    for e, r in enumerate(rows):
+        for lo in range(0, r, tile_rows):
+            table.append([e, at + lo, min(tile_rows, r - lo)])
+        at += r
+    tiles = torch.tensor(table + [[0, 0, 0]] * 3, dtype=torch.int32, device=DEV)
+    group = torch.repeat_interleave(torch.arange(g, device=DEV), torch.tensor(rows, device=DEV))
+    for gather in (False, True):
+        xs = x[src.long()] if gather else x[:total]
+        ref = torch.bmm(xs.double().unsqueeze(1), w.double()[group].transpose(1, 2).contiguous()).squeeze(1)
+        acc = k * 2.0 ** -24 * torch.bmm(xs.double().abs().unsqueeze(1), w.double().abs()[group].transpose(1, 2).contiguous()).squeeze(1)
+        if not gather:
+            out = torch.full((total + 9, n), 7.0, device=DEV, dtype=torch.bfloat16)
+            got = hip.grouped_gemm(x, w, tiles, tile_rows, out=out)
+            assert ((got[:total].double() - ref).abs() <= 2.0 ** -7 * ref.abs() + acc + 1e-6).all()
+            assert (got[total:] == 7.0).all()
+        h = n // 2
+        u, v = ref[:, :h], ref[:, h:]
+        act = torch.nn.functional.silu(u) * v
+        got = (hip.grouped_gemm(x, w, tiles, tile_rows, silu_mul=True, src_row=src) if gather
+               else hip.grouped_gemm(xs.contiguous(), w, tiles, tile_rows, silu_mul=True))
+        bound = 2.0 ** -7 * act.abs() + 1.1 * (acc[:, :h] * v.abs() + acc[:, h:] * u.abs()) + 1e-6
+        assert got.shape == (total, h) and ((got.double() - act).abs() <= bound).all()
+
+
 def test_mid_gemm_of_one_row_with_any_row_stride():
     """One row may carry any stride (an expanded or sliced tensor): its span is K columns all the same."""
     from vllm_distributed_amd.ops import hip

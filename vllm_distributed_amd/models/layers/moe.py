@@ -223,16 +223,18 @@ class FusedMoE(nn.Module):
         if (avg > envs.VDAMD_MOE_GROUPED_MAX_ROWS * cap / 64 and not torch.cuda.is_current_stream_capturing()
                 and not self._grouped_big(x)):
             return 0
-        for rows in (16, 32, 64, 128):
-            if avg <= rows or rows == cap:
+        if self.quant is None:          # (64 / 128, in us: 8 experts of 4096 x 14336 with 38 rows each 516 / 538, with 41 609 / 524)
+            return 64 if avg <= 40 else 128
+        for rows in (16, 32):
+            if avg <= rows:
                 return rows
         return cap
 
     def _grouped_big(self, x: torch.Tensor) -> bool:
-        """Whether the experts go to the large-batch kernel's grouped form: dense ones with more than 64 rows each.
-        (64 experts of 2048 x 1408 with 75 rows each: 268 us against 332 in tiles of 128; 8 of 4096 x 14336 with 50:
-        676 against 597 in tiles of 64, with 100: 673 against 803.)"""
-        return (self.quant is None and x.shape[0] * self.top_k > 64 * self.num_experts
+        """Whether the experts go to the large-batch kernel's grouped form: dense ones with more than 72 rows each (in tiles of
+        128 / of 256, in us: 64 experts of 2048 x 1408 with 56 rows 263 / 267, with 70 274 / 274, with 94 305 / 275; 8 of 4096 x
+        14336 with 68 554 / 695, with 82 672 / 698, with 100 745 / 703)."""
+        return (self.quant is None and x.shape[0] * self.top_k > 72 * self.num_experts
                 and ops.grouped_big_ok(x, self.top_k, self.w13, self.w2))
 
     def _expert_tile_rows(self, x: torch.Tensor) -> int:

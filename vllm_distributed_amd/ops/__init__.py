@@ -596,13 +596,13 @@ def grouped_big_ok(x, top_k: int, w13, w2) -> bool:
 
 
 def grouped_gate_up_silu(x, tiles, tile_rows: int, weight, src_row=None):
-    """``silu(x @ Wg^T) * (x @ Wu^T)`` per group for ``weight [G, 2I, K] = [Wg ; Wu]``: inside the GEMM in tiles of
-    ``GROUPED_BIG_ROWS`` rows, otherwise with the activation kernel behind it.  ``src_row``: the rows are ``x[src_row]``, which
-    those tiles read where they are."""
+    """``silu(x @ Wg^T) * (x @ Wu^T)`` per group for ``weight [G, 2I, K] = [Wg ; Wu]``, inside the GEMM where its columns come in
+    whole tiles of 16.  ``src_row``: the rows are ``x[src_row]``, which that GEMM reads where they are."""
     assert _use_hip(x)
-    if src_row is not None and not (tile_rows == GROUPED_BIG_ROWS and _hip.grouped_gather_ok(x, src_row)):
+    fused = _hip.grouped_silu_supported(x, weight)
+    if src_row is not None and not (fused and _hip.grouped_gather_ok(x, src_row)):
         x, src_row = x.index_select(0, src_row), None
-    if tile_rows == GROUPED_BIG_ROWS:
+    if fused:
         return _hip.grouped_gemm(x, weight, tiles, tile_rows, silu_mul=True, src_row=src_row)
     return silu_and_mul(grouped_linear(x, tiles, tile_rows, weight=weight))
 

@@ -38,6 +38,7 @@ def load() -> ctypes.CDLL:
         "vdamd_silu_and_mul": [P, P, L, I, I, P],
         "vdamd_embedding": [P, P, P, I, I, I, I, I, P],
         "vdamd_mid_gemm": [P, L, P, L, P, L, P, I, I, I, I, I, I, I, I, P],
+        "vdamd_mid_gemm_grouped": [P, L, P, L, P, L, L, P, I, P, I, I, I, I, I, I, I, I, P],
         "vdamd_stream_gemm": [P, L, P, L, P, L, P, P, L, I, I, I, I, I, I, I, I, I, P],
         "vdamd_big_gemm": [P, L, P, L, P, L, P, L, I, I, I, I, I, I, P],
         "vdamd_big_gemm_grouped": [P, L, P, L, P, L, L, P, I, P, I, I, I, I, I, I, P],
@@ -51,7 +52,6 @@ def load() -> ctypes.CDLL:
         "vdamd_w4_dequant": [P, P, P, I, I, I, I, P],
         "vdamd_skinny_gemm": [P, L, P, L, P, L, P, I, I, I, I, I, I, L, P],
         "vdamd_dynamic_fp8_quant": [P, P, P, I, I, L, I, P],
-        "vdamd_skinny_gemm_grouped": [P, L, P, L, P, L, L, P, I, I, I, I, I, I, P],
         "vdamd_w4a16_gemm_grouped": [P, L, P, L, P, P, L, L, P, I, I, I, I, I, I, I, P],
         "vdamd_moe_topk": [P, L, P, P, I, I, I, I, I, P],
         "vdamd_moe_align": [P, I, I, I, I, I, I, P, P, P, I, P],
@@ -963,9 +963,15 @@ def grouped_big_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = Fal
             and n % (32 if silu_mul else 16) == 0 and w.data_ptr() % 16 == 0 and n * k * 2 < (1 << 32) - 64)
 
 
+def grouped_silu_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the grouped GEMMs form ``silu(gate) * up`` of ``w = [gate ; up]`` themselves: halves of whole 16 columns, an expert's
+    matrix within 32-bit byte offsets."""
+    return w.shape[1] % 32 == 0 and w.shape[1] * w.shape[2] * 2 < (1 << 32) - 64
+
+
 def grouped_gather_ok(x: torch.Tensor, src_row: torch.Tensor) -> bool:
-    """Whether the large-batch kernel's grouped form can read the rows ``x[src_row]`` where they are: whole, aligned rows of x
-    within 32-bit byte offsets, and eight entries at least (it fetches that many at a time)."""
+    """Whether the grouped GEMMs can read the rows ``x[src_row]`` where they are: whole, aligned rows of x within 32-bit byte
+    offsets, and eight entries at least (the large-batch kernel fetches that many at a time)."""
     return (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1] and x.data_ptr() % 16 == 0
             and x.shape[0] * x.stride(0) * 2 < (1 << 32) - 64 and src_row.numel() >= 8)
 
@@ -975,31 +981,32 @@ def grouped_gemm(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, tile_row
     """``out[r] = x[r] @ w[g(r)]^T`` for group-sorted rows: ``w [G, N, K]``,
     ``tiles [n, 3] int32`` = (group, first row, rows <= tile_rows; 0 = unused).
     Every row covered by a tile must lie inside ``x``; rows outside all tiles
-    are left untouched in ``out``.  ``tile_rows`` 256: the large-batch kernel, with ``silu_mul`` for ``w = [gate ; up]`` and
-    ``silu(gate) * up`` as the result (``N / 2`` wide); ``src_row`` (with ``silu_mul``, at least eight): the tiles' rows are
-    ``x[src_row]``, read where they are."""
+    are left untouched in ``out``.  ``tile_rows`` 256: the large-batch kernel, otherwise the short-batch one in tiles of 64 or 128
+    rows.  ``silu_mul``: ``w = [gate ; up]`` and ``silu(gate) * up`` the result (``N / 2`` wide);
+    ``src_row`` (with ``silu_mul``, at least eight): the tiles' rows are ``x[src_row]``, read where they are."""
     nt = _check_tiles(tiles, x, tile_rows)
     g, n, k = w.shape
     assert w.is_contiguous() and w.dtype == x.dtype and x.shape[1] == k
-    assert k % 128 == 0 and n % 16 == 0
+    assert k % 128 == 0 and n % (32 if silu_mul else 16) == 0 and (16 <= tile_rows <= 128 or tile_rows == GROUPED_BIG_ROWS)
     n_out = n // 2 if silu_mul else n
     rows = x.shape[0] if src_row is None else src_row.numel()
     if out is None:
         out = torch.empty((rows, n_out), dtype=x.dtype, device=x.device)
+    assert src_row is None or (silu_mul and src_row.dtype == torch.int32 and src_row.is_contiguous() and src_row.is_cuda
+                               and grouped_gather_ok(x, src_row))
+    src = None if src_row is None else src_row.data_ptr()
+    epi = EPI_SILU_MUL if silu_mul else EPI_NONE
     if tile_rows == GROUPED_BIG_ROWS:
         assert grouped_big_supported(x, w, silu_mul) and out.shape == (rows, n_out) and out.stride(1) == 1
-        assert src_row is None or (silu_mul and src_row.dtype == torch.int32 and src_row.is_contiguous() and src_row.is_cuda
-                                   and grouped_gather_ok(x, src_row))
         _check(_LIB.vdamd_big_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k, n * k,
-                                           tiles.data_ptr(), nt, None if src_row is None else src_row.data_ptr(), x.shape[0],
-                                           rows, n, k, EPI_SILU_MUL if silu_mul else EPI_NONE, _dt(x), _stream()),
+                                           tiles.data_ptr(), nt, src, x.shape[0], rows, n, k, epi, _dt(x), _stream()),
                "big_gemm_grouped")
         return out
-    assert 16 <= tile_rows <= 128 and not silu_mul and src_row is None
-    ntw = 1 if tile_rows > 64 or n <= 4096 else 2
-    _check(_LIB.vdamd_skinny_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k,
-                                          n * k, tiles.data_ptr(), nt, tile_rows, n, k, ntw, _dt(x), _stream()),
-           "skinny_gemm_grouped")
+    assert out.shape == (rows, n_out) and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
+    _check(_LIB.vdamd_mid_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k, n * k,
+                                       tiles.data_ptr(), nt, src, x.shape[0], rows, n, k, 64 if tile_rows <= 64 else 128, 128, epi, _dt(x),
+                                       _stream()),
+           "mid_gemm_grouped")
     return out
 
 
