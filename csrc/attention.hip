@@ -69,10 +69,16 @@ __device__ __forceinline__ typename Vec8<T>::type fp8x8_to(uint2 w, float scale)
 // waited for before the next: the decode kernels were 1.2 to 2.6 times as slow over e4m3 as over 16 bits.)
 template <typename T, bool KV8> struct Raw8 { using type = typename Vec8<T>::type; };
 template <typename T> struct Raw8<T, true> { using type = uint2; };
-template <typename T, bool KV8>
+// ONCE: past the caches (nontemporal), for more than the memory-side cache holds (48 rows of 9000 keys, 8 heads of 128: 310 -> 303
+// us; a smaller cache may still be there from the step before, 16 rows of 4000 keys, 2 heads: 22.1 / 24.0; bytes come a quarter of a
+// line at a time, and are fetched again: 175 / 214)
+template <typename T, bool KV8, bool ONCE = false>
 __device__ __forceinline__ typename Raw8<T, KV8>::type ld_kv(const void* cache, long off) {
-  if constexpr (KV8) return *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(cache) + off);
-  else return ld8<T>(reinterpret_cast<const T*>(cache) + off);
+  using R = typename Raw8<T, KV8>::type;
+  typedef unsigned Words __attribute__((ext_vector_type(sizeof(R) / 4)));
+  const char* p = reinterpret_cast<const char*>(cache) + off * (long)(sizeof(R) / 8);
+  if constexpr (ONCE) return __builtin_bit_cast(R, __builtin_nontemporal_load(reinterpret_cast<const Words*>(p)));
+  else return __builtin_bit_cast(R, *reinterpret_cast<const Words*>(p));
 }
 template <typename T, typename R> __device__ __forceinline__ typename Vec8<T>::type widen(const R& r) {
   if constexpr (__is_same(R, uint2)) return fp8x8_to<T>(r, 1.f);
@@ -91,7 +97,7 @@ struct KVFrag {
   typename Raw8<T, KV8>::type kfa[D / 32], kfb[D / 32], vf[D / 16];
 };
 
-template <typename T, int D, bool KV8>
+template <typename T, int D, bool KV8, bool ONCE = false>
 __device__ __forceinline__ void load_kv_group(KVFrag<T, D, KV8>& f, const void* __restrict__ k_cache,
                                               const void* __restrict__ v_cache, const int* __restrict__ bt_row,
                                               int kvh, int Hkv, int block_size, int base, int seq_len) {
@@ -106,8 +112,8 @@ __device__ __forceinline__ void load_kv_group(KVFrag<T, D, KV8>& f, const void* 
   const long kb_off = ((blk_b * Hkv + kvh) * block_size + (kb % block_size)) * (long)D + 8 * g4;
 #pragma unroll
   for (int s = 0; s < D / 32; ++s) {
-    f.kfa[s] = ld_kv<T, KV8>(k_cache, ka_off + 32 * s);
-    f.kfb[s] = ld_kv<T, KV8>(k_cache, kb_off + 32 * s);
+    f.kfa[s] = ld_kv<T, KV8, ONCE>(k_cache, ka_off + 32 * s);
+    f.kfb[s] = ld_kv<T, KV8, ONCE>(k_cache, kb_off + 32 * s);
   }
   // ---- V^T rows: this lane's 8 keys are base + 8*g4 .. +7 (one block: block_size % 8 == 0)
   const int vkey = min(base + 8 * g4, seq_len - 1) & ~7;
@@ -115,7 +121,7 @@ __device__ __forceinline__ void load_kv_group(KVFrag<T, D, KV8>& f, const void* 
   const int slab = block_size * 16;                           // elements of one 16-row slab of a block
   const long v_off = (blk_v * Hkv + kvh) * (long)(D / 16) * slab + ((vkey % block_size) >> 3) * 128 + 8 * r16;
 #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) f.vf[dt] = ld_kv<T, KV8>(v_cache, v_off + (long)dt * slab);
+  for (int dt = 0; dt < D / 16; ++dt) f.vf[dt] = ld_kv<T, KV8, ONCE>(v_cache, v_off + (long)dt * slab);
 }
 
 // Score capping (Gemma-2): cap * tanh(score / cap) on the natural-log scale; `s2` and the result are
@@ -183,14 +189,14 @@ __device__ __forceinline__ void attend_loaded(
   }
 }
 
-template <typename T, int D, int NQ, bool KV8>
+template <typename T, int D, int NQ, bool KV8, bool ONCE = false>
 __device__ __forceinline__ void attend_group(
     const void* __restrict__ k_cache, const void* __restrict__ v_cache, const int* __restrict__ bt_row, int kvh,
     int Hkv, int block_size, int base, int seq_len, float scale_log2e, float softcap,
     const typename Vec8<T>::type (&qf)[NQ][D / 32], f32x4 (&acc)[NQ][D / 16], float (&m)[NQ], float (&l)[NQ],
     const int (&qpos_hi)[NQ], const int (&qpos_lo)[NQ], float alibi_l2 = 0.f) {
   KVFrag<T, D, KV8> f;
-  load_kv_group<T, D, KV8>(f, k_cache, v_cache, bt_row, kvh, Hkv, block_size, base, seq_len);
+  load_kv_group<T, D, KV8, ONCE>(f, k_cache, v_cache, bt_row, kvh, Hkv, block_size, base, seq_len);
   if constexpr (KV8) __builtin_amdgcn_sched_barrier(0);        // (all loads are on their way before anything is widened)
   attend_loaded<T, D, NQ, KV8>(f, base, seq_len, scale_log2e, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
 }
@@ -200,7 +206,7 @@ __device__ __forceinline__ void attend_group(
 // q-tile, sequence); its 4 waves stride over the split's 32-key groups and are
 // merged through LDS.  The 16 MFMA columns carry the GQA group's query heads.
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool KV8>
+template <typename T, int D, bool KV8, bool ONCE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void paged_decode_kernel(
     T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, const T* __restrict__ q,
     long q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
@@ -258,8 +264,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     int g = g_begin + wid;
     for (; g + 4 < g_end; g += 8) {
       KVFrag<T, D, KV8> f[2];
-      load_kv_group<T, D, KV8>(f[0], k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len);
-      load_kv_group<T, D, KV8>(f[1], k_cache, v_cache, bt_row, kvh, Hkv, block_size, (g + 4) * 32, seq_len);
+      load_kv_group<T, D, KV8, ONCE>(f[0], k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len);
+      load_kv_group<T, D, KV8, ONCE>(f[1], k_cache, v_cache, bt_row, kvh, Hkv, block_size, (g + 4) * 32, seq_len);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
@@ -267,11 +273,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                                     alibi_l2);
     }
     if (g < g_end)
-      attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
+      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
                                  scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
   } else {
     for (int g = g_begin + wid; g < g_end; g += 4)
-      attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
+      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
                                  scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
   }
 
@@ -545,7 +551,7 @@ __device__ __forceinline__ void prefill_dma16(const void* g, void* lds_wave_base
 #undef PREFILL_LDS_D
 #undef PREFILL_LDS_OCC
 
-template <typename T, int D, bool KV8>
+template <typename T, int D, bool KV8, bool ONCE = false>
 int launch_decode(void* out, float* ws, const void* q, long q_stride, const void* kc, const void* vc, const int* bt,
                   int bt_stride, const int* seq_lens, float scale, int B, int Hq, int Hkv, int block_size,
                   int num_splits, long out_stride, const float* k_scales, const float* v_scales, int window,
@@ -562,7 +568,7 @@ int launch_decode(void* out, float* ws, const void* q, long q_stride, const void
     HIP_LAUNCH_CHECK();
     return 0;
   }
-  hipLaunchKernelGGL((paged_decode_kernel<T, D, KV8>), dim3(num_splits, Hkv * q_tiles, B), dim3(256), 0, s, (T*)out,
+  hipLaunchKernelGGL((paged_decode_kernel<T, D, KV8, ONCE>), dim3(num_splits, Hkv * q_tiles, B), dim3(256), 0, s, (T*)out,
                      part_o, part_ml, (const T*)q, q_stride, kc, vc, bt, bt_stride, seq_lens,
                      sl2, Hq, Hkv, block_size, num_splits, out_stride, k_scales, v_scales, window, softcap, sinks,
                      alibi);
@@ -630,8 +636,9 @@ VDAMD_API long vdamd_decode_workspace_floats(int B, int Hq, int D) {
   return (long)B * Hq * MAX_SPLITS * (D + 2);
 }
 
-// kv_fp8 != 0: k_cache / v_cache hold OCP e4m3 bytes in the same layouts; k_scales / v_scales
-// (one float per KV head, or null for 1.0) multiply the stored values back to their range.
+// kv_fp8 1: k_cache / v_cache hold OCP e4m3 bytes in the same layouts; k_scales / v_scales
+// (one float per KV head, or null for 1.0) multiply the stored values back to their range.  2 (decode, heads of up to 128): a
+// cache of T, read past the chip's caches.
 VDAMD_API int vdamd_paged_attention_decode(void* out, float* workspace, const void* q, long q_stride,
                                            const void* k_cache, const void* v_cache, const int* block_table,
                                            int bt_stride, const int* seq_lens, float scale, int B, int Hq, int Hkv,
@@ -644,10 +651,15 @@ VDAMD_API int vdamd_paged_attention_decode(void* out, float* workspace, const vo
   if (num_splits > 1 && workspace == nullptr) return -3;
 #define CASE(TY, DD)                                                                                             \
   do {                                                                                                           \
-    if (kv_fp8)                                                                                                  \
+    if (kv_fp8 == 1)                                                                                             \
       return launch_decode<TY, DD, true>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride,   \
                                          seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride,         \
                                          k_scales, v_scales, window, softcap, sinks, alibi, s);                            \
+    if constexpr (DD <= 128)                                                                                     \
+      if (kv_fp8 == 2)                                                                                           \
+        return launch_decode<TY, DD, false, true>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride, \
+                                                  seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride, \
+                                                  nullptr, nullptr, window, softcap, sinks, alibi, s);           \
     return launch_decode<TY, DD, false>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride,    \
                                         seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride, nullptr, \
                                         nullptr, window, softcap, sinks, alibi, s);                                      \

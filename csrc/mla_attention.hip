@@ -274,21 +274,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //     leaves a lane with 16 neighbouring ones of them.
 // The 16-byte pieces of a row are XOR-ed with bits 1, 3 and 4 of the key's number (the 16 rows of a K fragment then lie in
 // 16 different places of the LDS's 256 bytes).
-// Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 109 us against 211
-// through both caches (441 and 833 MB; the chip's copy rate would take 91).
+// Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 99 us against 211
+// through both caches (441 and 833 MB).  ONCE: nontemporal, for more rows than the memory-side cache holds (108 us without; 16
+// sequences of 3000 keys, which it holds, 27.5 / 29).
 // ---------------------------------------------------------------------------------------------------------------
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void mla_lds_void;
 typedef __attribute__((address_space(1))) void mla_glb_void;
 
 // 16 bytes per lane from global memory straight into LDS: the wave's 64 pieces land at lds_wave_base + 16 * lane
-__device__ __forceinline__ void mla_dma16(const void* g, void* lds_wave_base) {
+// (NT: cache policy, 2 = nontemporal)
+template <int NT> __device__ __forceinline__ void mla_dma16(const void* g, void* lds_wave_base) {
 #if defined(__HIP_DEVICE_COMPILE__)      // (the builtin exists in the device pass only)
-  __builtin_amdgcn_global_load_lds((mla_glb_void*)const_cast<void*>(g), (mla_lds_void*)lds_wave_base, 16, 0, 0);
+  __builtin_amdgcn_global_load_lds((mla_glb_void*)const_cast<void*>(g), (mla_lds_void*)lds_wave_base, 16, 0, NT);
 #endif
 }
 
-template <typename T, int DK, int DV, bool P2>
+template <typename T, int DK, int DV, bool P2, bool ONCE>
 __global__ __launch_bounds__(256, 2) void mla_rows_kernel(
     T* __restrict__ out, long out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
     const T* __restrict__ q, long q_stride, const T* __restrict__ k_cache, const int* __restrict__ block_table, int bt_stride,
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(256, 2) void mla_rows_kernel(
     const int lo = max(win_lo - base, 0), hi = min(seq_len - 1 - base, 31);
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      mla_dma16(src + max(min(prow[i], hi), lo) * ROW + pbyte[i], smem + buf * 32 * ROW + (i * 256 + wid * 64) * 16);
+      mla_dma16<ONCE ? 2 : 0>(src + max(min(prow[i], hi), lo) * ROW + pbyte[i], smem + buf * 32 * ROW + (i * 256 + wid * 64) * 16);
   };
 
   const int key_a = 8 * (r16 >> 2) + (r16 & 3);    // K rows of the two interleaved S^T tiles: this one and 4 behind it
@@ -792,12 +794,16 @@ int launch_mla(void* out, long out_stride, void* part_o, void* part_ml, const vo
     mla_attention_multi_kernel<T, DK, DV, NQ, false, KV8, P2><<<dim3(num_splits, (q_tiles + NQ - 1) / NQ, T_), 256, 0, st>>>(
         (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, k_cache, v_cache, block_table,
         bt_stride, token_seq, seq_lens, sl2, T_, Hq, block_size, num_splits, ex);
-  } else if (mode == 3) {                           // a workgroup per 16 heads over the key rows alone
+  } else if (mode == 3 || mode == 4) {              // a workgroup per 16 heads over the key rows alone (4: past the caches)
     if constexpr (!KV8 && DV % 256 == 0 && DK % 64 == 0) {
       if (block_size % 32) return -1;
-      mla_rows_kernel<T, DK, DV, P2><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(
-          (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, (const T*)k_cache, block_table, bt_stride,
-          token_seq, seq_lens, sl2, Hq, block_size, num_splits, ex);
+#define MLA_ROWS(ONCE)                                                                                                     \
+  mla_rows_kernel<T, DK, DV, P2, ONCE><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(                                      \
+      (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, (const T*)k_cache, block_table, bt_stride, \
+      token_seq, seq_lens, sl2, Hq, block_size, num_splits, ex)
+      if (mode == 4) MLA_ROWS(true);
+      else MLA_ROWS(false);
+#undef MLA_ROWS
     } else {
       return -4;
     }

@@ -133,7 +133,8 @@ __global__ __launch_bounds__(256) void w4a16_gemm_kernel(
   auto load_w = [&](int kb, u32x4 (&w)[W4_NTW], V8 (&s)[W4_NTW], uint32_t (&f)[W4_NTW]) {
 #pragma unroll
     for (int t = 0; t < W4_NTW; ++t) {
-      w[t] = *reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4);
+      // (past the caches: 16 rows through 160 experts of 6144 x 2560 475 -> 465 us, one row 85 -> 80)
+      w[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4));
       if (FMT == W4_INT)
         s[t] = ld8(sz + ((((size_t)ntc[t] * NG + kb / kb_per_group) * 16 + 4 * g) << 1));
       else
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(256) void w4a16_gemm_lds_kernel(
   auto load_w = [&](int kb, u32x4 (&w)[NTW], V8 (&s)[NTW], uint32_t (&f)[NTW]) {
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      w[t] = *reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4);
+      w[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4));
       if (FMT == W4_INT)
         s[t] = ld8(sz + ((((size_t)ntc[t] * NG + kb / kb_per_group) * 16 + 4 * g) << 1));
       else

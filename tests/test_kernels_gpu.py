@@ -1532,3 +1532,37 @@ def test_latent_attention_prep_kernel_matches_its_parts(h, nope, rank, rope, kv8
     torch.testing.assert_close(vc.float(), vc_ref.float(), **tol)
     only_q = _hip.mla_prep(q, nope, q_lat, latent, w, 1e-6, cos_sin, positions, None, None, None)
     assert torch.equal(only_q, got)
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_decode_attention_past_the_caches_reads_the_same(d, splits, monkeypatch):
+    from vllm_distributed_amd.ops import hip
+    lens = [1, 33, 200, 517]
+    blocks = sum(-(-n // 64) for n in lens)
+    kc = (_rand(blocks, 2, 64, d) * 0.5).contiguous()
+    vc = _rand(blocks, 2, d // 16, 8, 16, 8).contiguous()
+    table = torch.zeros(4, 9, dtype=torch.int32, device=DEV)
+    order, at = torch.randperm(blocks, device=DEV).to(torch.int32), 0
+    for i, n in enumerate(lens):
+        table[i, :-(-n // 64)] = order[at:at + -(-n // 64)]
+        at += -(-n // 64)
+    args = (_rand(4, 8, d), kc, vc, table, torch.tensor(lens, dtype=torch.int32, device=DEV), d ** -0.5, 517)
+    want = hip.paged_attention_decode(*args, num_splits=splits)
+    monkeypatch.setattr(hip, "DECODE_ONCE_BYTES", 0)
+    assert torch.equal(hip.paged_attention_decode(*args, num_splits=splits), want)
+
+
+def test_latent_rows_past_the_caches_read_the_same(monkeypatch):
+    from vllm_distributed_amd.ops import hip
+    lens = [5, 64, 300]
+    kc, vc = (torch.zeros(shape, dtype=torch.bfloat16, device=DEV)
+              for shape in (ops.k_cache_shape(8, 1, 576, 64), ops.v_cache_shape(8, 1, 512, 64)))
+    ops.mla_cache_write(_rand(512, 576), kc, vc, torch.arange(512, device=DEV, dtype=torch.int32))
+    table = torch.tensor([[3, 0, 0, 0, 0], [5, 0, 0, 0, 0], [7, 1, 0, 2, 4]], dtype=torch.int32, device=DEV)
+    args = (_rand(3, 16, 576), kc, vc, table, None, torch.tensor(lens, dtype=torch.int32, device=DEV), 0.07, 300)
+    for splits in (1, 2):
+        want = hip.mla_attention(*args, splits=splits, mode=3)
+        with monkeypatch.context() as m:
+            m.setattr(hip, "LATENT_ONCE_BYTES", 0)
+            assert torch.equal(hip.mla_attention(*args, splits=splits, mode=3), want)

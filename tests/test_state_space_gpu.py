@@ -189,3 +189,26 @@ def test_crossed_decode_with_a_workgroup_per_cu_or_more(h, g, d):
                                     crossed=True)
     want = torch_ref.crossed_bias_attention(q, k, v, table, qsl, sls, 0.2, r1, r2)
     _close(got, want, dtype, 4)
+
+
+def test_decoded_rows_of_large_states_read_past_the_caches():
+    """64 rows x 16 heads x 128 x 128 are 64 MB of state, half the rows less: the same values either way."""
+    hip = _hip()
+    gen = torch.Generator("cuda").manual_seed(5)
+    b, h, g, n, v = 64, 16, 2, 128, 128
+
+    def rand(*shape, dtype=torch.float32):
+        return torch.randn(*shape, generator=gen, device="cuda").to(dtype)
+    x, dt = rand(b, h * v + 2 * g * n, dtype=torch.bfloat16), rand(b, h, dtype=torch.bfloat16)
+    a_log, bias, skip, state = rand(h), rand(h), rand(h), rand(b, h, n, v)
+    lens = torch.full((b,), 9, dtype=torch.int32, device="cuda")
+
+    def scan(rows):
+        k = len(rows)
+        st, at = state.clone(), torch.tensor(rows, device="cuda")
+        out = hip.selective_scan(x[at], dt[at], h, g, v, n, a_log, bias, skip, st, at.to(torch.int32), _i32(*range(k + 1)),
+                                 lens[:k], 1)
+        return out, st[at]
+    whole, halves = scan(list(range(b))), [scan(list(range(i, b, 2))) for i in (0, 1)]
+    for got, parts in zip(whole, zip(*halves)):
+        assert torch.equal(got[0::2], parts[0]) and torch.equal(got[1::2], parts[1])

@@ -385,6 +385,10 @@ def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
     return t.data_ptr()
 
 
+# decode attention reads more than this past the chip's caches (256 MB of them on the memory's side)
+DECODE_ONCE_BYTES = 320 << 20
+
+
 def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, max_seq_len=0, out=None,
                            workspace=None, num_splits: Optional[int] = None, kv_scales=None,
                            window: int = 0, softcap: float = 0.0, sinks=None, alibi_slopes=None) -> torch.Tensor:
@@ -415,10 +419,14 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
         if workspace is None or workspace.numel() < need:
             workspace = torch.empty(need, dtype=torch.float32, device=q.device)
         ws_ptr = workspace.data_ptr()
+    kv = _kv_args(k_cache, kv_scales, hkv)
+    # (keys and values of the longest row for all of them: about 200 MB for rows of mixed lengths)
+    if kv[0] == 0 and d <= 128 and num_splits and b * max_seq_len * hkv * d * 4 >= DECODE_ONCE_BYTES:
+        kv = (2,) + tuple(kv[1:])
     _check(_LIB.vdamd_paged_attention_decode(
         out.data_ptr(), ws_ptr, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
         block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), float(scale), b, hq, hkv, d, bs,
-        num_splits, hq * d, _dt(q), *_kv_args(k_cache, kv_scales, hkv), int(window), float(softcap),
+        num_splits, hq * d, _dt(q), *kv, int(window), float(softcap),
         _per_head(sinks, hq, q), _per_head(alibi_slopes, hq, q), _stream()), "paged_attention_decode")
     return out
 
@@ -1293,6 +1301,10 @@ def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows
     return mode, max(1, min(per, keys // shortest, 64))
 
 
+# rows of the longest sequence for all of them (57 and 86 MB of rows are slower past the caches, 210 MB faster: 63 -> 57 us)
+LATENT_ONCE_BYTES = 192 << 20
+
+
 def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
                   token_seq: Optional[torch.Tensor], seq_lens: torch.Tensor, scale: float, max_seq_len: int,
                   out: Optional[torch.Tensor] = None, splits: Optional[int] = None,
@@ -1327,6 +1339,8 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
+    if mode == 3 and hq <= 16 and t * keys * dk * 2 >= LATENT_ONCE_BYTES:
+        mode = 4                          # the same kernel, its rows read past the caches
     splits = best if splits is None else splits
     part_o = part_ml = None
     if splits > 1:
