@@ -83,6 +83,27 @@ def test_gate_up_at_short_batches():
     assert hip.stream_profitable(8, 28672, 2048) and not hip.stream_profitable(8, 28672, 4096)
 
 
+def test_short_batch_products_are_planned_once_a_shape(monkeypatch):
+    """A step outside a graph asks for the plan of every product several times over: only a shape's first answer is worked out."""
+    asked = []
+    real = hip._mid_estimate
+    monkeypatch.setattr(hip, "_mid_estimate", lambda *a: (asked.append(a), real(*a))[1])
+
+    def layer(m):                            # rows that no other test asks for
+        plans = []
+        for n, k in ((10224, 8128), (8176, 8128), (8176, 28608)):
+            for reduced in (False, True):
+                plans.append((hip.mid_profitable(m, n, k, reduced), hip.mid_choose(m, n, k, reduced)))
+        return plans
+    for m in (1, 101, 129, 250, 401):
+        first = layer(m)
+        assert asked, "the rule no longer asks the model of a product's time"
+        asked.clear()
+        assert layer(m) == first and not asked
+    for rule in (hip.mid_choose, hip.mid_profitable, hip.mid_silu_tile):
+        assert rule.cache_info().maxsize is not None          # (bounded)
+
+
 def test_recurrent_layers_report_their_prompt_memory():
     """What a prompt through a recurrent layer allocates counts in the memory profile, which does not run its kernels."""
     import torch

@@ -8,6 +8,7 @@ out-of-bounds access in a hand-written kernel can take the GPU down.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 from ctypes import c_float, c_int, c_long, c_void_p
@@ -792,17 +793,20 @@ def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int, reduced
     """Modelled run time in us: rounds of workgroups x K tiles x time per tile, at least that of reading its part of W, plus
     the fp32 slabs, written and read again, and the launch that sums them up."""
     fixed, tile_us, slots, tbs = _MID_TILES[(bm, bn)]
-    blocks = _mid_blocks(m, n, bm, bn, ksplit)
-    left = blocks % slots
-    again = 1.25 if bn == 128 and slots == 256 else 1.1     # a CU's one workgroup fills and drains its ring in every round
-
-    def round_us(count):                   # per K tile of `count` workgroups side by side: the full rate once most CUs read
-        return max(tile_us, bn * 128 * count / (tbs * 1e6) / min(1.0, 0.5 + count / 440)) * (again if blocks > slots else 1.0)
-    main = (k / 64 / ksplit) * (blocks // slots * round_us(slots) + (round_us(left) if left else 0.0))
+    rounds, left = divmod(_mid_blocks(m, n, bm, bn, ksplit), slots)
+    read_us = bn * 128 / (tbs * 1e6)       # per K tile and workgroup, at the full rate once most CUs read
+    tile = rounds * max(tile_us, read_us * slots / min(1.0, 0.5 + slots / 440))
+    if left:
+        tile += max(tile_us, read_us * left / min(1.0, 0.5 + left / 440))
+    if rounds + (left > 0) > 1:            # a CU's one workgroup fills and drains its ring in every round
+        tile *= 1.25 if bn == 128 and slots == 256 else 1.1
     slabs = ((3.0 if reduced else 0.0) + ksplit * m * n * 4 * 0.4e-6) if ksplit > 1 else 0.0
-    return fixed + main + slabs
+    return fixed + k / 64 / ksplit * tile + slabs
 
 
+# The rules below are functions of whole numbers alone, asked several times for every product of a step that runs outside a
+# graph: their answers are kept (by shape, the last 4096 of them; 50 to 150 us a question, as much as a product takes, against 0.1)
+@functools.lru_cache(maxsize=4096)
 def mid_choose(m: int, n: int, k: int, reduced: bool = True) -> Tuple[int, int, int]:
     """``(bm, bn, ksplit)`` with the smallest modelled time.  The row tile covers all of M up to 256
     (W is then read from HBM once); splitting K buys parallelism and costs slab traffic."""
@@ -821,6 +825,13 @@ def mid_choose(m: int, n: int, k: int, reduced: bool = True) -> Tuple[int, int, 
     return best[1], best[2], best[3]
 
 
+@functools.lru_cache(maxsize=4096)
+def mid_silu_tile(m: int, n: int, k: int) -> Tuple[int, int]:
+    """The tile of the unsplit form with the activation in its epilogue."""
+    return min((t for t in _MID_TILES if t[0] >= m or t[0] == 256), key=lambda t: _mid_estimate(m, n, k, *t, 1, False))
+
+
+@functools.lru_cache(maxsize=4096)
 def mid_profitable(m: int, n: int, k: int, reduced: bool = True) -> bool:
     """Where this kernel beats the library GEMM on MI355X (padded weight rows, in graphs).  Where the next kernel sums the
     K-split slabs (not ``reduced``): one row through an 8B qkv projection 11.2 against 16.2 us, 2048 x 2048 5.5 / 8.5, but
@@ -866,7 +877,7 @@ def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
     m, k = x.shape
     n = w.shape[0]
     if silu_mul:
-        a, b = min(((t for t in _MID_TILES if t[0] >= m or t[0] == 256)), key=lambda t: _mid_estimate(m, n, k, *t, 1, False))
+        a, b = mid_silu_tile(m, n, k)
         c = 1
     else:
         a, b, c = mid_choose(m, n, k, not partials)
