@@ -104,6 +104,14 @@ def test_short_batch_products_are_planned_once_a_shape(monkeypatch):
         assert rule.cache_info().maxsize is not None          # (bounded)
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,dim,keys,once", [
+    (48, 32, 8, 128, 13500, True), (48, 128, 8, 128, 13500, True), (4, 32, 8, 128, 13500, False), (48, 32, 8, 256, 13500, False),
+    # the same keys in several workgroups, one for every 16 query heads of a key head (cached / past the caches: 141 / 174, 153 / 236)
+    (48, 64, 2, 128, 13500, False), (200, 64, 2, 128, 4500, False), (100, 71, 1, 64, 13500, False), (48, 34, 2, 128, 13500, False)])
+def test_decode_attention_reads_past_the_caches_what_one_workgroup_reads(batch, heads, kv_heads, dim, keys, once):
+    assert hip.decode_reads_once(batch, heads, kv_heads, dim, keys) is once
+
+
 def test_recurrent_layers_report_their_prompt_memory():
     """What a prompt through a recurrent layer allocates counts in the memory profile, which does not run its kernels."""
     import torch

@@ -390,6 +390,16 @@ def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
 DECODE_ONCE_BYTES = 320 << 20
 
 
+def decode_reads_once(batch: int, heads: int, num_kv_heads: int, head_dim: int, max_seq_len: int) -> bool:
+    """Whether a decode step over a 16-bit cache reads keys and values past the caches: more of them than those hold (the longest
+    row's for every row: about 200 MB for rows of mixed lengths), and each read by one workgroup only.  In turn over several
+    caches, cached / past them, us: 48 rows of about 9000 keys, 8 heads of 128, 32 query heads 319 / 293; but with two tiles of
+    query heads to a key head, 64 over 2, 141 / 174, and with five, 71 over 1 of 64 (100 rows), 153 / 236."""
+    if -(-heads // num_kv_heads) > 16 or head_dim > 128:
+        return False
+    return batch * max_seq_len * num_kv_heads * head_dim * 4 >= DECODE_ONCE_BYTES
+
+
 def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, max_seq_len=0, out=None,
                            workspace=None, num_splits: Optional[int] = None, kv_scales=None,
                            window: int = 0, softcap: float = 0.0, sinks=None, alibi_slopes=None) -> torch.Tensor:
@@ -421,8 +431,7 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
             workspace = torch.empty(need, dtype=torch.float32, device=q.device)
         ws_ptr = workspace.data_ptr()
     kv = _kv_args(k_cache, kv_scales, hkv)
-    # (keys and values of the longest row for all of them: about 200 MB for rows of mixed lengths)
-    if kv[0] == 0 and d <= 128 and num_splits and b * max_seq_len * hkv * d * 4 >= DECODE_ONCE_BYTES:
+    if kv[0] == 0 and num_splits and decode_reads_once(b, hq, hkv, d, max_seq_len):
         kv = (2,) + tuple(kv[1:])
     _check(_LIB.vdamd_paged_attention_decode(
         out.data_ptr(), ws_ptr, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
