@@ -112,6 +112,26 @@ def test_decode_attention_reads_past_the_caches_what_one_workgroup_reads(batch, 
     assert hip.decode_reads_once(batch, heads, kv_heads, dim, keys) is once
 
 
+@pytest.mark.parametrize("window,once", [(0, True), (257, True), (256, True), (255, False), (32, False)])
+def test_decode_attention_past_the_caches_counts_the_keys_of_the_window(window, once, monkeypatch):
+    import torch
+    from vllm_distributed_amd import ops
+    handed = []
+
+    class Lib:
+        @staticmethod
+        def vdamd_paged_attention_decode(*args):
+            handed.append(args[18])
+            return 0
+    monkeypatch.setattr(hip, "_LIB", Lib)
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "DECODE_ONCE_BYTES", 2 * 256 * 64 * 4)
+    kc, vc = (torch.zeros(shape, dtype=torch.bfloat16) for shape in (ops.k_cache_shape(8, 1, 64, 64), ops.v_cache_shape(8, 1, 64, 64)))
+    hip.paged_attention_decode(torch.zeros(2, 4, 64, dtype=torch.bfloat16), kc, vc, torch.zeros(2, 8, dtype=torch.int32),
+                               torch.tensor([512, 3], dtype=torch.int32), 0.1, 512, num_splits=1, window=window)
+    assert handed == [2 if once else 0]
+
+
 def test_recurrent_layers_report_their_prompt_memory():
     """What a prompt through a recurrent layer allocates counts in the memory profile, which does not run its kernels."""
     import torch

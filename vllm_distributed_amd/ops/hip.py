@@ -390,14 +390,14 @@ def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
 DECODE_ONCE_BYTES = 320 << 20
 
 
-def decode_reads_once(batch: int, heads: int, num_kv_heads: int, head_dim: int, max_seq_len: int) -> bool:
-    """Whether a decode step over a 16-bit cache reads keys and values past the caches: more of them than those hold (the longest
-    row's for every row: about 200 MB for rows of mixed lengths), and each read by one workgroup only.  In turn over several
-    caches, cached / past them, us: 48 rows of about 9000 keys, 8 heads of 128, 32 query heads 319 / 293; but with two tiles of
-    query heads to a key head, 64 over 2, 141 / 174, and with five, 71 over 1 of 64 (100 rows), 153 / 236."""
+def decode_reads_once(batch: int, heads: int, num_kv_heads: int, head_dim: int, keys: int) -> bool:
+    """Whether a decode step over a 16-bit cache reads keys and values past the caches: more of them than those hold (the ``keys``
+    that the longest row sees for every row: about 200 MB for rows of mixed lengths), and each read by one workgroup only.  In
+    turn over several caches, cached / past them, us: 48 rows of about 9000 keys, 8 heads of 128, 32 query heads 319 / 293; but
+    with two tiles of query heads to a key head, 64 over 2, 141 / 174, and with five, 71 over 1 of 64 (100 rows), 153 / 236."""
     if -(-heads // num_kv_heads) > 16 or head_dim > 128:
         return False
-    return batch * max_seq_len * num_kv_heads * head_dim * 4 >= DECODE_ONCE_BYTES
+    return batch * keys * num_kv_heads * head_dim * 4 >= DECODE_ONCE_BYTES
 
 
 def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, max_seq_len=0, out=None,
@@ -419,8 +419,8 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
     if out is None:
         out = torch.empty((b, hq, d), dtype=q.dtype, device=q.device)
     assert out.is_contiguous() and out.shape == (b, hq, d)
+    keys = min(max_seq_len, window) if window > 0 else max_seq_len
     if num_splits is None:
-        keys = min(max_seq_len, window) if window > 0 else max_seq_len
         # (whole up to 512 keys and the same from 1024 on: asking costs 0.4 us)
         num_splits = choose_num_splits(b, hkv, keys, keys >= 1024 or keys > 512 and torch.cuda.is_current_stream_capturing())
     ws_ptr = None
@@ -431,7 +431,7 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
             workspace = torch.empty(need, dtype=torch.float32, device=q.device)
         ws_ptr = workspace.data_ptr()
     kv = _kv_args(k_cache, kv_scales, hkv)
-    if kv[0] == 0 and num_splits and decode_reads_once(b, hq, hkv, d, max_seq_len):
+    if kv[0] == 0 and num_splits and decode_reads_once(b, hq, hkv, d, keys):
         kv = (2,) + tuple(kv[1:])
     _check(_LIB.vdamd_paged_attention_decode(
         out.data_ptr(), ws_ptr, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
