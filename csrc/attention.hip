@@ -69,9 +69,8 @@ __device__ __forceinline__ typename Vec8<T>::type fp8x8_to(uint2 w, float scale)
 // waited for before the next: the decode kernels were 1.2 to 2.6 times as slow over e4m3 as over 16 bits.)
 template <typename T, bool KV8> struct Raw8 { using type = typename Vec8<T>::type; };
 template <typename T> struct Raw8<T, true> { using type = uint2; };
-// ONCE: past the caches (nontemporal), for more than the memory-side cache holds (48 rows of 9000 keys, 8 heads of 128: 310 -> 303
-// us; a smaller cache may still be there from the step before, 16 rows of 4000 keys, 2 heads: 22.1 / 24.0; bytes come a quarter of a
-// line at a time, and are fetched again: 175 / 214)
+// ONCE: past the caches (nontemporal), for more than the memory-side cache holds (a smaller cache may still be there from the step
+// before, 16 rows of 4000 keys, 2 heads: 22.1 / 24.0; bytes come a quarter of a line at a time, and are fetched again: 175 / 214)
 template <typename T, bool KV8, bool ONCE = false>
 __device__ __forceinline__ typename Raw8<T, KV8>::type ld_kv(const void* cache, long off) {
   using R = typename Raw8<T, KV8>::type;
@@ -213,7 +212,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ seq_lens, float scale_log2e,
     int Hq, int Hkv, int block_size, int num_splits, long out_stride, const float* __restrict__ k_scales,
     const float* __restrict__ v_scales, int window, float softcap, const float* __restrict__ sinks,
-    const float* __restrict__ alibi) {
+    const float* __restrict__ alibi, float past_bytes) {
   // sinks[Hq] (natural-log units): an extra score per query head that takes part in the softmax's
   // denominator only (attention sinks); alibi[Hq]: slopes of a linear position bias.  Either may be null.
   using V = typename Vec8<T>::type;
@@ -241,6 +240,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const int gps = (n_groups + num_splits - 1) / num_splits;
   const int g_begin = g_first + split * gps;
   const int g_end = min(g_begin + gps, g_first + n_groups);
+
+  bool past = false;
+  if constexpr (ONCE) {
+    // What the step reads, and whether other rows read the same: pages that several rows share (the front of a context: cached
+    // prefixes, samples of one prompt) are fetched once for all of them only through the caches.  A row that shares any page of
+    // the split shares its first.  Thread t asks the t-th row from here on: all of them up to 256 rows, else 256 as a sample.
+    // A microsecond or two: splits of less than eight groups do not ask (2048 rows of 150 keys: 253 -> 268 us).
+    if (g_end - g_begin >= 8) {
+      const int B = gridDim.z, asked = min(B, 256), page = g_begin * 32 / block_size;
+      const int* bt = block_table + page;
+      int keys = 0;
+      bool same = false;
+      if ((int)threadIdx.x < asked) {
+        const int r = b + (int)threadIdx.x < B ? b + (int)threadIdx.x : b + (int)threadIdx.x - B;
+        keys = seq_lens[r];
+        same = r != b && keys > page * block_size && bt[(long)r * bt_stride] == bt[(long)b * bt_stride];
+        if (window > 0) keys = min(keys, window);
+      }
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) keys += __shfl_xor(keys, o, 64);
+      if (lane == 0) s_m[wid][0] = (float)keys;
+      const bool shared = __syncthreads_or(same);
+      const float read = (s_m[0][0] + s_m[1][0] + s_m[2][0] + s_m[3][0]) * B / asked;
+      past = __builtin_amdgcn_readfirstlane(!shared && read * (4.f * D * Hkv) >= past_bytes);
+      __syncthreads();                     // (s_m is written again below)
+    }
+  }
 
   V qf[1][D / 32];
 #pragma unroll
@@ -276,9 +302,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
                                  scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
   } else {
-    for (int g = g_begin + wid; g < g_end; g += 4)
-      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                                 scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+    if (ONCE && past) {
+      for (int g = g_begin + wid; g < g_end; g += 4)
+        attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale_log2e * k_scale,
+                                         softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+    } else {
+      for (int g = g_begin + wid; g < g_end; g += 4)
+        attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale_log2e * k_scale, softcap,
+                                   qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+    }
   }
 
   float lsum = l[0];
@@ -555,7 +587,7 @@ template <typename T, int D, bool KV8, bool ONCE = false>
 int launch_decode(void* out, float* ws, const void* q, long q_stride, const void* kc, const void* vc, const int* bt,
                   int bt_stride, const int* seq_lens, float scale, int B, int Hq, int Hkv, int block_size,
                   int num_splits, long out_stride, const float* k_scales, const float* v_scales, int window,
-                  float softcap, const float* sinks, const float* alibi, hipStream_t s) {
+                  float softcap, const float* sinks, const float* alibi, float past_bytes, hipStream_t s) {
   const int G = Hq / Hkv;
   const int q_tiles = (G + 15) / 16;
   float* part_o = ws;
@@ -571,7 +603,7 @@ int launch_decode(void* out, float* ws, const void* q, long q_stride, const void
   hipLaunchKernelGGL((paged_decode_kernel<T, D, KV8, ONCE>), dim3(num_splits, Hkv * q_tiles, B), dim3(256), 0, s, (T*)out,
                      part_o, part_ml, (const T*)q, q_stride, kc, vc, bt, bt_stride, seq_lens,
                      sl2, Hq, Hkv, block_size, num_splits, out_stride, k_scales, v_scales, window, softcap, sinks,
-                     alibi);
+                     alibi, past_bytes);
   HIP_LAUNCH_CHECK();
   if (num_splits > 1) {
     hipLaunchKernelGGL((decode_reduce_kernel<T, D>), dim3(Hq, B), dim3(split_merge_threads(D, num_splits)), 0, s, (T*)out,
@@ -637,32 +669,34 @@ VDAMD_API long vdamd_decode_workspace_floats(int B, int Hq, int D) {
 }
 
 // kv_fp8 1: k_cache / v_cache hold OCP e4m3 bytes in the same layouts; k_scales / v_scales
-// (one float per KV head, or null for 1.0) multiply the stored values back to their range.  2 (decode, heads of up to 128): a
-// cache of T, read past the chip's caches.
+// (one float per KV head, or null for 1.0) multiply the stored values back to their range.  past_bytes > 0 (a 16-bit cache of
+// heads of up to 128): where the rows' keys and values are that many bytes, those that one row alone reads are read past the
+// chip's caches.
 VDAMD_API int vdamd_paged_attention_decode(void* out, float* workspace, const void* q, long q_stride,
                                            const void* k_cache, const void* v_cache, const int* block_table,
                                            int bt_stride, const int* seq_lens, float scale, int B, int Hq, int Hkv,
                                            int D, int block_size, int num_splits, long out_stride, int dtype,
                                            int kv_fp8, const float* k_scales, const float* v_scales, int window,
-                                           float softcap, const float* sinks, const float* alibi, hipStream_t s) {
+                                           float softcap, const float* sinks, const float* alibi, long past_bytes,
+                                           hipStream_t s) {
   if (B == 0) return 0;
   // num_splits == 0 selects the one-wave-per-sequence kernel (short contexts, large batches)
   if (Hq % Hkv != 0 || block_size % 8 != 0 || num_splits < 0 || num_splits > MAX_SPLITS) return -1;
   if (num_splits > 1 && workspace == nullptr) return -3;
 #define CASE(TY, DD)                                                                                             \
   do {                                                                                                           \
-    if (kv_fp8 == 1)                                                                                             \
+    if (kv_fp8)                                                                                                  \
       return launch_decode<TY, DD, true>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride,   \
                                          seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride,         \
-                                         k_scales, v_scales, window, softcap, sinks, alibi, s);                            \
+                                         k_scales, v_scales, window, softcap, sinks, alibi, 0.f, s);              \
     if constexpr (DD <= 128)                                                                                     \
-      if (kv_fp8 == 2)                                                                                           \
+      if (past_bytes > 0)                                                                                        \
         return launch_decode<TY, DD, false, true>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride, \
                                                   seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride, \
-                                                  nullptr, nullptr, window, softcap, sinks, alibi, s);           \
+                                                  nullptr, nullptr, window, softcap, sinks, alibi, (float)past_bytes, s); \
     return launch_decode<TY, DD, false>(out, workspace, q, q_stride, k_cache, v_cache, block_table, bt_stride,    \
                                         seq_lens, scale, B, Hq, Hkv, block_size, num_splits, out_stride, nullptr, \
-                                        nullptr, window, softcap, sinks, alibi, s);                                      \
+                                        nullptr, window, softcap, sinks, alibi, 0.f, s);                          \
   } while (0)
   if (dtype == DT_BF16) {
     if (D == 128) CASE(bf16_t, 128);

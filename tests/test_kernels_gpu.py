@@ -1553,6 +1553,23 @@ def test_decode_attention_past_the_caches_reads_the_same(d, splits, monkeypatch)
     assert torch.equal(hip.paged_attention_decode(*args, num_splits=splits), want)
 
 
+@pytest.mark.parametrize("rows,window,splits", [(3, 0, 1), (257, 0, 2), (300, 290, 1)])
+def test_decode_attention_past_the_caches_of_rows_that_share_pages(rows, window, splits, monkeypatch):
+    """Rows with a common front, rows with none and empty ones; more rows than a workgroup asks; every split long enough to ask."""
+    from vllm_distributed_amd.ops import hip
+    g = torch.Generator().manual_seed(rows)
+    lens = torch.randint(1, 900, (rows,), generator=g)
+    lens[0], lens[1], lens[2] = 899, 0, 1
+    table = torch.randint(0, 64, (rows, 15), generator=g).to(torch.int32)
+    table[::2, :7] = table[0, :7]
+    kc, vc = (_rand(64, 2, 64, 128) * 0.5).contiguous(), _rand(64, 2, 8, 8, 16, 8).contiguous()
+    args = (_rand(rows, 8, 128), kc, vc, table.to(DEV), lens.to(DEV).int(), 128 ** -0.5, 900)
+    want = hip.paged_attention_decode(*args, num_splits=splits, window=window)
+    for limit in (0, 1 << 14, 1 << 19):          # past the caches wherever nothing is shared; by what the rows hold
+        monkeypatch.setattr(hip, "DECODE_ONCE_BYTES", limit)
+        assert torch.equal(hip.paged_attention_decode(*args, num_splits=splits, window=window), want)
+
+
 def test_latent_rows_past_the_caches_read_the_same(monkeypatch):
     from vllm_distributed_amd.ops import hip
     lens = [5, 64, 300]

@@ -45,7 +45,7 @@ def load() -> ctypes.CDLL:
         "vdamd_big_gemm_grouped": [P, L, P, L, P, L, L, P, I, P, I, I, I, I, I, I, P],
         "vdamd_rope_cache": [P, P, P, P, L, L, L, P, P, P, P, I, I, I, I, I, I, P, P, F, I, I, P, P, P],
         "vdamd_rope_cache_slabs": [P, P, I, P, L, P, P, P, P, I, I, I, I, I, P, P, F, I, I, P, P, P],
-        "vdamd_paged_attention_decode": [P, P, P, L, P, P, P, I, P, F, I, I, I, I, I, I, L, I, I, P, P, I, F, P, P, P],
+        "vdamd_paged_attention_decode": [P, P, P, L, P, P, P, I, P, F, I, I, I, I, I, I, L, I, I, P, P, I, F, P, P, L, P],
         "vdamd_paged_attention_prefill": [P, P, L, P, P, P, I, P, P, F, I, I, I, I, I, I, L, I, I, P, P, I, F, P, P, P],
         "vdamd_argmax": [P, P, I, I, L, I, P],
         "vdamd_sample": [P, P, I, I, L, P, P, P, P, P, I, P],
@@ -387,14 +387,17 @@ def _per_head(t: Optional[torch.Tensor], hq: int, q: torch.Tensor):
 
 
 # decode attention reads more than this past the chip's caches (256 MB of them on the memory's side)
-DECODE_ONCE_BYTES = 320 << 20
+DECODE_ONCE_BYTES = 208 << 20
 
 
 def decode_reads_once(batch: int, heads: int, num_kv_heads: int, head_dim: int, keys: int) -> bool:
-    """Whether a decode step over a 16-bit cache reads keys and values past the caches: more of them than those hold (the ``keys``
-    that the longest row sees for every row: about 200 MB for rows of mixed lengths), and each read by one workgroup only.  In
-    turn over several caches, cached / past them, us: 48 rows of about 9000 keys, 8 heads of 128, 32 query heads 319 / 293; but
-    with two tiles of query heads to a key head, 64 over 2, 141 / 174, and with five, 71 over 1 of 64 (100 rows), 153 / 236."""
+    """Whether a decode step over a 16-bit cache may read keys and values past the caches: if every row saw ``keys`` of them they
+    would be too many to be kept, and each is read by one workgroup only (with two tiles of query heads to a key head, 64 over
+    2 of 128, 48 rows of about 9000 keys, 141 us through the caches and 174 past them; with five, 71 over 1 of 64, 153 and 236).
+    What the rows do see, and which pages several of them share, the kernel asks where it runs: ``keys`` is a bound, in a graph
+    a loose one.  Several caches in turn, us (cached / past them / asking first): 48 rows of about 9000 keys, 32 heads over 8 of
+    128, 318 / 302 / 304, 256 of 400 86 / 79 / 78, with three quarters of the pages shared 210 / 241 / 219 and, 128 rows of
+    3000, 186 / 210 / 186; 16 rows of 1000, which four caches hold, under a bound of 32768 18.2 / 20.6 / 18.5."""
     if -(-heads // num_kv_heads) > 16 or head_dim > 128:
         return False
     return batch * keys * num_kv_heads * head_dim * 4 >= DECODE_ONCE_BYTES
@@ -431,13 +434,12 @@ def paged_attention_decode(q, k_cache, v_cache, block_table, seq_lens, scale, ma
             workspace = torch.empty(need, dtype=torch.float32, device=q.device)
         ws_ptr = workspace.data_ptr()
     kv = _kv_args(k_cache, kv_scales, hkv)
-    if kv[0] == 0 and num_splits and decode_reads_once(b, hq, hkv, d, keys):
-        kv = (2,) + tuple(kv[1:])
+    past = max(1, DECODE_ONCE_BYTES) if kv[0] == 0 and num_splits and decode_reads_once(b, hq, hkv, d, keys) else 0
     _check(_LIB.vdamd_paged_attention_decode(
         out.data_ptr(), ws_ptr, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
         block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), float(scale), b, hq, hkv, d, bs,
         num_splits, hq * d, _dt(q), *kv, int(window), float(softcap),
-        _per_head(sinks, hq, q), _per_head(alibi_slopes, hq, q), _stream()), "paged_attention_decode")
+        _per_head(sinks, hq, q), _per_head(alibi_slopes, hq, q), past, _stream()), "paged_attention_decode")
     return out
 
 
