@@ -40,8 +40,10 @@ __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf
 // R - 1 of column c of the head's state, in registers (G * R >= N).  Per chunk of C rows: d * B and C vectors of the
 // head's group, the tile's u columns and the row's decay go to LDS, the next chunk's loads are in flight while the
 // current one is computed, and the G row groups' partial outputs are summed after one barrier: two barriers per chunk.
-// ONCE: states read past the caches (nontemporal), which then keep what is written: for 64 MB of states and more (128 rows x 16 heads
-// x 128 x 128, 268 MB in and out: 66 -> 56 us; 34 MB 19.6 / 20.2)
+// ONCE: states read past the caches (nontemporal), which are then left to what is written: from 64 to 320 MB of states.  Over 1.6 GB of
+// states in turn, so that none is left from the pass before, cached / past them: 33 MB 22.8 / 22.9 us, 67 MB 38.2 / 34.9, 100 MB
+// 55.0 / 50.3, 134 MB (128 rows x 16 heads x 128 x 128) 67.5 / 63.0, 201 MB 94.1 / 90.9, 268 MB (32 heads) 118.9 / 116.2, 537 MB
+// 221.5 / 225.4.
 template <typename T, int R, int G, int C, bool ONCE>
 __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(G >= 16 ? 8 : 1, 8))) void selective_scan_kernel(
     float* __restrict__ out, const T* __restrict__ x, long x_stride, const T* __restrict__ dt, long dt_stride,
@@ -362,7 +364,8 @@ VDAMD_API int vdamd_selective_scan(float* out, const void* x, long x_stride, con
                      groups, N, vdim)
     if (max_rows > 0 && max_rows <= 2) {
       // decoded rows only: bound by reading and writing the states, so small workgroups that overlap each other
-      const bool once = (long)num_seqs * H * N * vdim >= 16 << 20;
+      const long floats = (long)num_seqs * H * N * vdim;
+      const bool once = floats >= 16 << 20 && floats < 80 << 20;
 #define SSM_DECODE(R_, G_, C_) \
   if (once) SSM(R_, G_, C_, true); \
   else SSM(R_, G_, C_, false)

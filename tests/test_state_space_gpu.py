@@ -191,11 +191,13 @@ def test_crossed_decode_with_a_workgroup_per_cu_or_more(h, g, d):
     _close(got, want, dtype, 4)
 
 
-def test_decoded_rows_of_large_states_read_past_the_caches():
-    """64 rows x 16 heads x 128 x 128 are 64 MB of state, half the rows less: the same values either way."""
+@pytest.mark.parametrize("b", [64, 320])
+def test_decoded_rows_of_large_states_read_past_the_caches(b):
+    """64 rows x 16 heads x 128 x 128 are 64 MB of state, half the rows less; 320 rows are 320 MB, which are read through the
+    caches again, half of them not: the same values either way."""
     hip = _hip()
     gen = torch.Generator("cuda").manual_seed(5)
-    b, h, g, n, v = 64, 16, 2, 128, 128
+    h, g, n, v = 16, 2, 128, 128
 
     def rand(*shape, dtype=torch.float32):
         return torch.randn(*shape, generator=gen, device="cuda").to(dtype)
