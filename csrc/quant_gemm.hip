@@ -133,8 +133,12 @@ __global__ __launch_bounds__(256) void w4a16_gemm_kernel(
   auto load_w = [&](int kb, u32x4 (&w)[W4_NTW], V8 (&s)[W4_NTW], uint32_t (&f)[W4_NTW]) {
 #pragma unroll
     for (int t = 0; t < W4_NTW; ++t) {
-      // (past the caches: 16 rows through 160 experts of 6144 x 2560 475 -> 465 us, one row 85 -> 80)
-      w[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4));
+      const u32x4* const src = reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4);
+      // One row tile, which alone reads these weights: past the caches (copies in turn: 160 experts of 6144 x 2560 by 1, 4 and 16 rows
+      // 84.5 -> 78.4, 199 -> 193, 496 -> 485 us, 28672 x 4096 by one row 23.2 -> 22.4).  More rows than 16 fetch them again for each
+      // tile or wave (10240 x 8192 by 33 rows 38.9 -> 40.3, by 160 95 -> 102).
+      if constexpr (MT == 1) w[t] = __builtin_nontemporal_load(src);
+      else w[t] = *src;
       if (FMT == W4_INT)
         s[t] = ld8(sz + ((((size_t)ntc[t] * NG + kb / kb_per_group) * 16 + 4 * g) << 1));
       else
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(256) void w4a16_gemm_lds_kernel(
   auto load_w = [&](int kb, u32x4 (&w)[NTW], V8 (&s)[NTW], uint32_t (&f)[NTW]) {
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      w[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4));
+      w[t] = *reinterpret_cast<const u32x4*>(qw + (((size_t)ntc[t] * KB + kb) << 8) + lane * 4);
       if (FMT == W4_INT)
         s[t] = ld8(sz + ((((size_t)ntc[t] * NG + kb / kb_per_group) * 16 + 4 * g) << 1));
       else
@@ -686,7 +690,7 @@ static int launch_w4_grouped(void* out, long os, const void* x, long xs, const v
   return 0;
 }
 
-// Grouped form for mixture-of-experts (see vdamd_skinny_gemm_grouped): group g's
+// Grouped form for mixture-of-experts (see vdamd_mid_gemm_grouped): group g's
 // packed weights start at qw + g * qw_group_stride words, sz + g * sz_group_stride
 // elements; tile_rows is 16, 32, 48 or 64.
 // up_off > 0 (tile_rows <= 32 only): x rows are [gate | up] with the up half up_off elements after the
