@@ -1177,6 +1177,24 @@ def test_grouped_products_on_the_rings(n, k, pad, rows, tile_rows):
         assert got.shape == (total, h) and ((got.double() - act).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192)])
+def test_linear_writes_any_output_of_a_short_batch(m, n, k):
+    """Rows that the short-batch kernels cannot write in place (odd strides and places, columns apart) are the library's.
+    Bound: the rounding of the result, and K roundings of the sums."""
+    from vllm_distributed_amd.ops import hip
+    assert hip.mid_profitable(m, n, k)
+    x, w = _rand(m, k), _padded_weight(n, k, 128)
+    ref = x.double() @ w.double().t()
+    bound = 2.0 ** -8 * ref.abs() + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-6
+    flat = torch.zeros(m * 2 * (n + 9) + 8, dtype=torch.bfloat16, device=DEV)
+    for size, strides, at, ok in (((m, n), (n, 1), 0, True), ((m, n), (n + 4, 1), 4, True), ((m, n), (n + 1, 1), 0, False),
+                                  ((m, n), (n, 1), 2, False), ((m, n), (2 * n, 2), 0, False), ((m, n), (1, m), 0, False)):
+        out = flat.as_strided(size, strides, at)
+        assert hip.mid_out_ok(out, x, n) is ok
+        got = ops.linear(x, w, out=out)
+        assert got.data_ptr() == out.data_ptr() and ((out.double() - ref).abs() <= bound).all()
+
+
 def test_mid_gemm_of_one_row_with_any_row_stride():
     """One row may carry any stride (an expanded or sliced tensor): its span is K columns all the same."""
     from vllm_distributed_amd.ops import hip

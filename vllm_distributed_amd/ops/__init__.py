@@ -243,13 +243,14 @@ def linear(x, weight, bias=None, out=None):
     if x.is_cuda and x.dim() == 2 and x.shape[0] <= SHORT_BATCH and envs.VDAMD_SKINNY_GEMM and _use_hip(x):
         m, n, k = x.shape[0], weight.shape[0], weight.shape[1]
         if (envs.VDAMD_STREAM_GEMM and _hip.stream_profitable(m, n, k) and _hip.stream_supported(x, weight)
-                and (out is None or out.stride(0) == n)):
+                and _hip.mid_out_ok(out, x, n) and (out is None or out.stride(0) == n)):
             y = _hip.stream_gemm(x, weight, out=out)
             return y if bias is None else y.add_(bias)
-        if _hip.mid_profitable(m, n, k) and _hip.mid_supported(x, weight):
+        if _hip.mid_profitable(m, n, k) and _hip.mid_supported(x, weight) and _hip.mid_out_ok(out, x, n):
             y = _hip.mid_gemm(x, weight, out=out)
             return y if bias is None else y.add_(bias)
-        if m <= 128 and _hip.skinny_profitable(m, n, k) and _hip.skinny_supported(x, weight):
+        if (m <= 128 and _hip.skinny_profitable(m, n, k) and _hip.skinny_supported(x, weight)
+                and _hip.mid_out_ok(out, x, n) and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0)):
             y = _hip.skinny_gemm(x, weight, out=out)
             return y if bias is None else y.add_(bias)
     if (x.is_cuda and x.dim() == 2 and envs.VDAMD_BIG_GEMM and _use_hip(x) and x.shape[0] >= _hip.BIG_MIN_M

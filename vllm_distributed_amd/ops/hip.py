@@ -788,6 +788,12 @@ def mid_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = False) -> b
             and (not silu_mul or w.shape[0] * w.stride(0) * 2 < (1 << 32) - 64))
 
 
+def mid_out_ok(out: Optional[torch.Tensor], x: torch.Tensor, n: int) -> bool:
+    """Whether the kernel can write its rows into ``out`` (the library takes any other strides and places)."""
+    return out is None or (out.shape == (x.shape[0], n) and out.dtype == x.dtype and out.stride(1) == 1
+                           and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)
+
+
 # workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
 # TB/s of W that those reach.  Least squares over 930 timings of 20 weight shapes (1.3 to 940 MB) at 1 to 512 rows and every
 # split: 6 to 8 % off in the mean
@@ -906,7 +912,7 @@ def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
     n_out = n // 2 if silu_mul else n
     if out is None:
         out = torch.empty((m, n_out), dtype=x.dtype, device=x.device)
-    assert out.shape == (m, n_out) and out.dtype == x.dtype and out.stride(1) == 1 and out.data_ptr() % 8 == 0
+    assert mid_out_ok(out, x, n_out)
     partial = torch.empty(ksplit * m * n, dtype=torch.float32, device=x.device) if ksplit > 1 else None
     _check(_LIB.vdamd_mid_gemm(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                                None if partial is None else partial.data_ptr(), m, n, k, ksplit, bm, bn,
