@@ -59,7 +59,7 @@ template <typename T, int BM, int BN, int WM, int WN, int XS, int WS, int EPI, b
 __global__ __launch_bounds__(WM * WN * 64) void mid_gemm_kernel(const T* x, long x_stride, const T* w, long w_stride, T* out,
                                                           long out_stride, float* partial, int M, int N, int K, int ksplit,
                                                           int ntn, int up_row, const int* __restrict__ tiles, long w_group,
-                                                              const int* __restrict__ src, int x_rows) {
+                                                              const int* __restrict__ src, int x_rows, const T* bias) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using V8 = typename Vec8<T>::type;
   constexpr int WAVES = WM * WN, FM = BM / WM / 16, FN = BN / WN / 16;
@@ -239,6 +239,11 @@ __global__ __launch_bounds__(WM * WN * 64) void mid_gemm_kernel(const T* x, long
         if (n >= N) continue;                // N % 16 == 0: a fragment column group is all in or all out
         if (ksplit == 1) {
           typename Vec4<T>::type o;
+          if (!GROUPED && bias != nullptr) {
+            const typename Vec4<T>::type add = *reinterpret_cast<const typename Vec4<T>::type*>(bias + n);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[j][i][r] += (float)add[r];
+          }
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[r] = (T)acc[j][i][r];
           *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(WM * WN * 64) void mid_gemm_kernel(const T* x, long
 
 template <typename T>
 __global__ void mid_reduce_kernel(T* __restrict__ out, long out_stride, const float* __restrict__ partial, int M,
-                                  int N, int ksplit) {
+                                  int N, int ksplit, const T* __restrict__ bias) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const int n4 = N >> 2;
   if (idx >= (long)M * n4) return;
@@ -261,21 +266,22 @@ __global__ void mid_reduce_kernel(T* __restrict__ out, long out_stride, const fl
   const int m = (int)mu, n = (int)((unsigned)idx - mu * (unsigned)n4) * 4;
   f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int k = 0; k < ksplit; ++k) s += *reinterpret_cast<const f32x4*>(partial + ((size_t)k * M + m) * N + n);
-  typename Vec4<T>::type o;
+  typename Vec4<T>::type o, add = {};
+  if (bias != nullptr) add = *reinterpret_cast<const typename Vec4<T>::type*>(bias + n);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) o[r] = (T)s[r];
+  for (int r = 0; r < 4; ++r) o[r] = (T)(s[r] + (float)add[r]);
   *reinterpret_cast<typename Vec4<T>::type*>(out + (long)m * out_stride + n) = o;
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int XS, int WS>
-int launch(const void* x, long xs, const void* w, long ws, void* out, long os, void* partial, int M, int N, int K, int ksplit,
-           int epi, hipStream_t st) {
+int launch(const void* x, long xs, const void* w, long ws, void* out, long os, const void* bias, void* partial, int M, int N, int K,
+           int ksplit, int epi, hipStream_t st) {
   const bool silu = epi == MG_EPI_SILU_MUL;
   const int ntn = silu ? (N / 2 + BN / 2 - 1) / (BN / 2) : (N + BN - 1) / BN;
   const int grid = (ntn * ksplit * ((M + BM - 1) / BM) + 7) / 8 * 8;
 #define MG_GO(EPI)                                                                                                             \
   mid_gemm_kernel<T, BM, BN, WM, WN, XS, WS, EPI, false><<<grid, WM * WN * 64, 0, st>>>(                                       \
-      (const T*)x, xs, (const T*)w, ws, (T*)out, os, (float*)partial, M, N, K, ksplit, ntn, N / 2, nullptr, 0, nullptr, 0)
+      (const T*)x, xs, (const T*)w, ws, (T*)out, os, (float*)partial, M, N, K, ksplit, ntn, N / 2, nullptr, 0, nullptr, 0, (const T*)bias)
   if (silu) MG_GO(MG_EPI_SILU_MUL);
   else MG_GO(MG_EPI_NONE);
 #undef MG_GO
@@ -283,7 +289,7 @@ int launch(const void* x, long xs, const void* w, long ws, void* out, long os, v
   if (ksplit > 1 && out != nullptr) {            // out == nullptr: the caller consumes the K-split slabs itself
     const long n = (long)M * (N / 4);
     mid_reduce_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, st>>>((T*)out, os, (const float*)partial, M, N,
-                                                                     ksplit);
+                                                                     ksplit, (const T*)bias);
     HIP_LAUNCH_CHECK();
   }
   return 0;
@@ -296,7 +302,7 @@ int launch_grouped(const void* x, long xs, const void* w, long ws, long w_group,
   const int ntn = silu ? (N / 2 + BN / 2 - 1) / (BN / 2) : (N + BN - 1) / BN;
 #define MG_GO(EPI)                                                                                                             \
   mid_gemm_kernel<T, BM, BN, WM, WN, XS, WS, EPI, true><<<ntn * num_tiles, WM * WN * 64, 0, st>>>(                             \
-      (const T*)x, xs, (const T*)w, ws, (T*)out, os, nullptr, M, N, K, 1, ntn, N / 2, tiles, w_group, src, x_rows)
+      (const T*)x, xs, (const T*)w, ws, (T*)out, os, nullptr, M, N, K, 1, ntn, N / 2, tiles, w_group, src, x_rows, nullptr)
   if (silu) MG_GO(MG_EPI_SILU_MUL);
   else MG_GO(MG_EPI_NONE);
 #undef MG_GO
@@ -307,10 +313,10 @@ int launch_grouped(const void* x, long xs, const void* w, long ws, long w_group,
 // 64 rows: two workgroups of four waves to a CU (72 KB), which level out what is left of a round (eight waves, each with half
 // the columns, read more of LDS: 70B down at 48 rows 81 us, so 77); larger tiles take a CU each
 template <typename T>
-int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os, void* partial, int M, int N, int K,
-             int ksplit, int bm, int bn, int epi, hipStream_t st) {
+int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os, const void* bias, void* partial, int M, int N,
+             int K, int ksplit, int bm, int bn, int epi, hipStream_t st) {
 #define MG_CASE(BM, BN, WM, WN, XS, WS) \
-  if (bm == BM && bn == BN) return launch<T, BM, BN, WM, WN, XS, WS>(x, xs, w, ws, out, os, partial, M, N, K, ksplit, epi, st);
+  if (bm == BM && bn == BN) return launch<T, BM, BN, WM, WN, XS, WS>(x, xs, w, ws, out, os, bias, partial, M, N, K, ksplit, epi, st);
   MG_CASE(256, 256, 4, 2, 2, 3)
   MG_CASE(256, 128, 2, 4, 3, 4)
   MG_CASE(128, 256, 2, 4, 2, 3)
@@ -324,24 +330,25 @@ int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os,
 
 // out = epilogue(x[M][K] . w[N][K]^T).  K % 64 == 0, N % 16 == 0; strides in elements, multiples of 8; pointers 16-byte
 // aligned.  (bm, bn) is the workgroup tile: (256, 128|256), (128, 128|256), (64, 128).
-// epi 0: out[M][N]; partial holds ksplit * M * N floats when ksplit > 1, and out may be null then: the slabs are the result.
+// epi 0: out[M][N], with bias[N] (or null, 8-byte aligned) added before the one rounding; partial holds ksplit * M * N floats when ksplit > 1, and out may be null then: the slabs are the result.
 // epi 2: w = [gate ; up], N % 32 == 0, ksplit 1, out[M][N/2] = silu(gate) * up.
 VDAMD_API int vdamd_mid_gemm(void* out, long out_stride, const void* x, long x_stride, const void* w, long w_stride,
-                             void* partial, int M, int N, int K, int ksplit, int bm, int bn, int epi, int dtype,
-                             void* stream) {
+                             const void* bias, void* partial, int M, int N, int K, int ksplit, int bm, int bn, int epi,
+                             int dtype, void* stream) {
   if (M <= 0) return 0;
   if (K % MG_BK || N % 16 || ksplit < 1 || ksplit > K / MG_BK) return -1;
   if (epi != MG_EPI_NONE && (epi != MG_EPI_SILU_MUL || N % 32 || ksplit != 1)) return -1;
   if (ksplit > 1 && partial == nullptr) return -2;
   if (out == nullptr && ksplit == 1) return -2;
+  if (bias != nullptr && (epi != MG_EPI_NONE || out == nullptr || (uintptr_t)bias % 8)) return -2;
   if ((x_stride | w_stride) % 8 || out_stride % 4) return -5;
   const long lim = (1L << 32) - 64;                // bytes that a tile's buffer descriptor spans
   if ((long)(M < bm ? M : bm) * x_stride * 2 >= lim || (long)(epi == MG_EPI_SILU_MUL ? N : bn) * w_stride * 2 >= lim) return -7;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == DT_BF16)
-    return dispatch<bf16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, epi, st);
+    return dispatch<bf16_t>(x, x_stride, w, w_stride, out, out_stride, bias, partial, M, N, K, ksplit, bm, bn, epi, st);
   if (dtype == DT_F16)
-    return dispatch<f16_t>(x, x_stride, w, w_stride, out, out_stride, partial, M, N, K, ksplit, bm, bn, epi, st);
+    return dispatch<f16_t>(x, x_stride, w, w_stride, out, out_stride, bias, partial, M, N, K, ksplit, bm, bn, epi, st);
   return -3;
 }
 

@@ -1195,6 +1195,27 @@ def test_linear_writes_any_output_of_a_short_batch(m, n, k):
         assert got.data_ptr() == out.data_ptr() and ((out.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(16, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192), (100, 2048, 8192)])
+def test_linear_adds_a_bias_before_the_one_rounding(m, n, k, dtype):
+    """A bias near the negative of a row's products leaves what a rounding in between would swamp.  Bound: one rounding of the
+    result, and K roundings of the sums."""
+    from vllm_distributed_amd.ops import hip
+    assert hip.mid_profitable(m, n, k)
+    x, w = _rand(m, k, dtype=dtype), _padded_weight(n, k, 128, dtype)
+    y = x.double() @ w.double().t()
+    bias = (-y[m // 2]).to(dtype)
+    ref = y + bias.double()
+    acc = (k + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + bias.double().abs())
+    bound = torch.finfo(dtype).eps / 2 * ref.abs() + acc + 1e-7
+    for b in (bias, torch.cat([bias[:1], bias])[1:]):             # (an odd place: added afterwards, not in the kernel)
+        got = ops.linear(x, w, bias=b)
+        if hip.mid_bias_ok(b, x, w):
+            assert ((got.double() - ref).abs() <= bound).all()
+        else:
+            assert ((got.double() - ref).abs() <= bound + torch.finfo(dtype).eps / 2 * 1.01 * y.abs()).all()
+
+
 def test_mid_gemm_of_one_row_with_any_row_stride():
     """One row may carry any stride (an expanded or sliced tensor): its span is K columns all the same."""
     from vllm_distributed_amd.ops import hip

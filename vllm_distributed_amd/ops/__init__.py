@@ -247,8 +247,9 @@ def linear(x, weight, bias=None, out=None):
             y = _hip.stream_gemm(x, weight, out=out)
             return y if bias is None else y.add_(bias)
         if _hip.mid_profitable(m, n, k) and _hip.mid_supported(x, weight) and _hip.mid_out_ok(out, x, n):
-            y = _hip.mid_gemm(x, weight, out=out)
-            return y if bias is None else y.add_(bias)
+            if bias is None or _hip.mid_bias_ok(bias, x, weight):
+                return _hip.mid_gemm(x, weight, out=out, bias=bias)
+            return _hip.mid_gemm(x, weight, out=out).add_(bias)
         if (m <= 128 and _hip.skinny_profitable(m, n, k) and _hip.skinny_supported(x, weight)
                 and _hip.mid_out_ok(out, x, n) and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0)):
             y = _hip.skinny_gemm(x, weight, out=out)

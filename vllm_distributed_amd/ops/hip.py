@@ -38,7 +38,7 @@ def load() -> ctypes.CDLL:
         "vdamd_reduce_add_rms_norm": [P, P, I, P, P, F, I, I, L, I, P],
         "vdamd_silu_and_mul": [P, P, L, I, I, P],
         "vdamd_embedding": [P, P, P, I, I, I, I, I, P],
-        "vdamd_mid_gemm": [P, L, P, L, P, L, P, I, I, I, I, I, I, I, I, P],
+        "vdamd_mid_gemm": [P, L, P, L, P, L, P, P, I, I, I, I, I, I, I, I, P],
         "vdamd_mid_gemm_grouped": [P, L, P, L, P, L, L, P, I, P, I, I, I, I, I, I, I, I, P],
         "vdamd_stream_gemm": [P, L, P, L, P, L, P, P, L, I, I, I, I, I, I, I, I, I, P],
         "vdamd_big_gemm": [P, L, P, L, P, L, P, L, I, I, I, I, I, I, P],
@@ -794,6 +794,11 @@ def mid_out_ok(out: Optional[torch.Tensor], x: torch.Tensor, n: int) -> bool:
                            and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)
 
 
+def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (bias.shape == w.shape[:1] and bias.dtype == x.dtype and bias.is_cuda and bias.is_contiguous()
+            and bias.data_ptr() % 8 == 0)
+
+
 # workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
 # TB/s of W that those reach.  Least squares over 930 timings of 20 weight shapes (1.3 to 940 MB) at 1 to 512 rows and every
 # split: 6 to 8 % off in the mean
@@ -884,13 +889,14 @@ def mid_silu_profitable(m: int, n: int, k: int) -> bool:
 
 def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, ksplit: Optional[int] = None,
              bm: Optional[int] = None, bn: Optional[int] = None, variant: Optional[int] = None,
-             partials: bool = False, silu_mul: bool = False) -> Optional[torch.Tensor]:
+             partials: bool = False, silu_mul: bool = False, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``x [M<=512, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
     fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit).  ``silu_mul``:
-    ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  A tile wider than the kernel is built for
+    ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  ``bias [N]`` is added to the fp32 sums.  A tile wider than the kernel is built for
     runs as its widest; ``variant`` names what is one kernel now and is accepted as before."""
     assert mid_supported(x, w, silu_mul), (x.shape, x.stride(), w.shape, w.stride(), x.dtype)
     assert not (silu_mul and (partials or (ksplit or 1) != 1))
+    assert bias is None or (mid_bias_ok(bias, x, w) and not partials and not silu_mul)
     m, k = x.shape
     n = w.shape[0]
     if silu_mul:
@@ -906,8 +912,8 @@ def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
         if ksplit <= 1:
             return None
         partial = torch.empty((ksplit, m, n), dtype=torch.float32, device=x.device)
-        _check(_LIB.vdamd_mid_gemm(None, n, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), partial.data_ptr(),
-                                   m, n, k, ksplit, bm, bn, EPI_NONE, _dt(x), _stream()), "mid_gemm (partial sums)")
+        _check(_LIB.vdamd_mid_gemm(None, n, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), None,
+                                   partial.data_ptr(), m, n, k, ksplit, bm, bn, EPI_NONE, _dt(x), _stream()), "mid_gemm (partial sums)")
         return partial
     n_out = n // 2 if silu_mul else n
     if out is None:
@@ -915,7 +921,7 @@ def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
     assert mid_out_ok(out, x, n_out)
     partial = torch.empty(ksplit * m * n, dtype=torch.float32, device=x.device) if ksplit > 1 else None
     _check(_LIB.vdamd_mid_gemm(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
-                               None if partial is None else partial.data_ptr(), m, n, k, ksplit, bm, bn,
+                               _ptr(bias), None if partial is None else partial.data_ptr(), m, n, k, ksplit, bm, bn,
                                EPI_SILU_MUL if silu_mul else EPI_NONE, _dt(x), _stream()), "mid_gemm")
     return out
 
