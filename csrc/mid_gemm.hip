@@ -342,6 +342,7 @@ VDAMD_API int vdamd_mid_gemm(void* out, long out_stride, const void* x, long x_s
   if (out == nullptr && ksplit == 1) return -2;
   if (bias != nullptr && (epi != MG_EPI_NONE || out == nullptr || (uintptr_t)bias % 8)) return -2;
   if ((x_stride | w_stride) % 8 || out_stride % 4) return -5;
+  if (((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)out % 8) return -8;
   const long lim = (1L << 32) - 64;                // bytes that a tile's buffer descriptor spans
   if ((long)(M < bm ? M : bm) * x_stride * 2 >= lim || (long)(epi == MG_EPI_SILU_MUL ? N : bn) * w_stride * 2 >= lim) return -7;
   hipStream_t st = (hipStream_t)stream;
@@ -362,6 +363,7 @@ VDAMD_API int vdamd_mid_gemm_grouped(void* out, long out_stride, const void* x, 
   if (K % MG_BK || N % 16 || (epi != MG_EPI_NONE && (epi != MG_EPI_SILU_MUL || N % 32))) return -1;
   if ((x_stride | w_stride | w_group) % 8 || out_stride % 4) return -5;
   if (src != nullptr && x_rows <= 0) return -4;
+  if (((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)out % 8) return -8;
   const long lim = (1L << 32) - 64;
   if ((long)(src != nullptr ? x_rows : bm) * x_stride * 2 >= lim || (long)(epi == MG_EPI_SILU_MUL ? N : bn) * w_stride * 2 >= lim) return -7;
   hipStream_t st = (hipStream_t)stream;

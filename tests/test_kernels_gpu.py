@@ -1177,6 +1177,19 @@ def test_grouped_products_on_the_rings(n, k, pad, rows, tile_rows):
         assert got.shape == (total, h) and ((got.double() - act).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("tile_rows", [16, 128])
+def test_grouped_products_of_experts_at_an_odd_place(tile_rows):
+    """Contiguous experts that begin two bytes into a buffer: the same bits as the same experts at its front."""
+    from vllm_distributed_amd.ops import hip
+    w = (_rand(3, 96, 128) * 0.1).contiguous()
+    odd = torch.cat([w.reshape(-1)[:1], w.reshape(-1)])[1:].view(3, 96, 128)
+    assert odd.data_ptr() % 16 and odd.is_contiguous()
+    x = _rand(24, 128)
+    tiles = torch.tensor([[0, 0, 7], [2, 7, 16], [1, 23, 1]], dtype=torch.int32, device=DEV)
+    for kw in ({}, {"silu_mul": True}):
+        assert torch.equal(hip.grouped_gemm(x, odd, tiles, tile_rows, **kw), hip.grouped_gemm(x, w, tiles, tile_rows, **kw))
+
+
 @pytest.mark.parametrize("m,n,k", [(3, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192)])
 def test_linear_writes_any_output_of_a_short_batch(m, n, k):
     """Rows that the short-batch kernels cannot write in place (odd strides and places, columns apart) are the library's.

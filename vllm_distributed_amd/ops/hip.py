@@ -1045,6 +1045,8 @@ def grouped_gemm(x: torch.Tensor, w: torch.Tensor, tiles: torch.Tensor, tile_row
                "big_gemm_grouped")
         return out
     assert out.shape == (rows, n_out) and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
+    if w.data_ptr() % 16:                  # (experts at an odd place of a larger buffer: their rows are fetched 16 bytes at a time)
+        w = w.clone()
     _check(_LIB.vdamd_mid_gemm_grouped(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), k, n * k,
                                        tiles.data_ptr(), nt, src, x.shape[0], rows, n, k, 64 if tile_rows <= 64 else 128, 128, epi, _dt(x),
                                        _stream()),
