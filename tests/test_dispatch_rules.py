@@ -104,6 +104,20 @@ def test_short_batch_products_are_planned_once_a_shape(monkeypatch):
         assert rule.cache_info().maxsize is not None          # (bounded)
 
 
+def test_the_k_splits_to_choose_from_can_be_restricted():
+    """VDAMD_MID_KSPLITS is read when the module is loaded; a switch that lost its meaning says so."""
+    import os
+    import subprocess
+    import sys
+    code = ("from vllm_distributed_amd.ops import hip\n"
+            "print(sorted({hip.mid_choose(m, n, k)[2] for m in (1, 64, 256) for n, k in ((8192, 8192), (10240, 8192), (8192, 28672))}))")
+    env = dict(os.environ, VDAMD_MID_KSPLITS="1,5", VDAMD_MID_GEMM_VARIANT="0",
+               PYTHONPATH=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    got = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True)
+    assert got.stdout.strip().splitlines()[-1] in ("[5]", "[1, 5]")
+    assert "VDAMD_MID_GEMM_VARIANT has no effect" in got.stdout + got.stderr
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,dim,keys,once", [
     (48, 32, 8, 128, 13500, True), (48, 128, 8, 128, 13500, True), (3, 32, 8, 128, 13500, False), (48, 32, 8, 256, 13500, False),
     # the same keys in several workgroups, one for every 16 query heads of a key head (cached / past the caches: 141 / 174, 153 / 236)

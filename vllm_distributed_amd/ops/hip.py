@@ -16,6 +16,9 @@ from typing import Optional, Tuple
 
 import torch
 
+from ..logger import init_logger
+
+logger = init_logger(__name__)
 _LIB: Optional[ctypes.CDLL] = None
 # VDAMD_OPS_LIB selects another build of the library (the host-sanitizer preset of build.py)
 _LIB_PATH = os.environ.get("VDAMD_OPS_LIB") or os.path.join(
@@ -804,7 +807,10 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 # split: 6 to 8 % off in the mean
 _MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
-_MID_KSPLITS = (1, 2, 3, 4, 5, 6, 7, 8, 12, 16)
+# K-split counts the choice is made from (VDAMD_MID_KSPLITS=1,2,4,8,16 restricts it, for A/B measurements)
+_MID_KSPLITS = tuple(int(v) for v in os.environ.get("VDAMD_MID_KSPLITS", "1,2,3,4,5,6,7,8,12,16").split(","))
+if os.environ.get("VDAMD_MID_GEMM_VARIANT", "-1") != "-1":
+    logger.warning("VDAMD_MID_GEMM_VARIANT has no effect: what it chose between is one kernel now")
 
 
 def _mid_blocks(m: int, n: int, bm: int, bn: int, ksplit: int) -> int:
