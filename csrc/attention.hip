@@ -243,29 +243,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 
   bool past = false;
   if constexpr (ONCE) {
-    // What the step reads, and whether other rows read the same: pages that several rows share (the front of a context: cached
-    // prefixes, samples of one prompt) are fetched once for all of them only through the caches.  A row that shares any page of
-    // the split shares its first.  Thread t asks the t-th row from here on: all of them up to 256 rows, else 256 as a sample.
-    // A microsecond or two: splits of less than eight groups do not ask (2048 rows of 150 keys: 253 -> 268 us).
-    if (g_end - g_begin >= 8) {
-      const int B = gridDim.z, asked = min(B, 256), page = g_begin * 32 / block_size;
-      const int* bt = block_table + page;
-      int keys = 0;
-      bool same = false;
-      if ((int)threadIdx.x < asked) {
-        const int r = b + (int)threadIdx.x < B ? b + (int)threadIdx.x : b + (int)threadIdx.x - B;
-        keys = seq_lens[r];
-        same = r != b && keys > page * block_size && bt[(long)r * bt_stride] == bt[(long)b * bt_stride];
-        if (window > 0) keys = min(keys, window);
-      }
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) keys += __shfl_xor(keys, o, 64);
-      if (lane == 0) s_m[wid][0] = (float)keys;
-      const bool shared = __syncthreads_or(same);
-      const float read = (s_m[0][0] + s_m[1][0] + s_m[2][0] + s_m[3][0]) * B / asked;
-      past = __builtin_amdgcn_readfirstlane(!shared && read * (4.f * D * Hkv) >= past_bytes);
-      __syncthreads();                     // (s_m is written again below)
-    }
+    // (a microsecond or two: splits of less than eight groups do not ask; 2048 rows of 150 keys: 253 -> 268 us if they did)
+    if (g_end - g_begin >= 8)
+      past = reads_alone(&s_m[0][0], b, gridDim.z, seq_lens, block_table, bt_stride, g_begin * 32 / block_size, block_size, window,
+                         4.f * D * Hkv, past_bytes);
   }
 
   V qf[1][D / 32];

@@ -114,6 +114,34 @@ template <int P, bool NEAR> __device__ __forceinline__ float parts_sum(float v) 
   return v;
 }
 
+// Decode steps that may read a paged cache past the chip's caches (256 threads, all of them here): whether the step reads
+// past_bytes or more, bytes_per_key for each key that its rows see, and no other row has this one's page `page`.  Pages that
+// several rows share (the front of a context: cached prefixes, samples of one prompt) are fetched once for all of them only
+// through the caches, and a row that shares any page of a split shares its first.  Thread t asks the t-th row from b on: all B
+// rows up to 256, else 256 as a sample.  red: four floats of LDS, free again when this returns.
+__device__ __forceinline__ bool reads_alone(float* red, int b, int B, const int* __restrict__ seq_lens,
+                                            const int* __restrict__ block_table, long bt_stride, int page, int block_size,
+                                            int window, float bytes_per_key, float past_bytes) {
+  const int asked = min(B, 256);
+  const int* bt = block_table + page;
+  int keys = 0;
+  bool same = false;
+  if ((int)threadIdx.x < asked) {
+    const int r = b + (int)threadIdx.x < B ? b + (int)threadIdx.x : b + (int)threadIdx.x - B;
+    keys = seq_lens[r];
+    same = r != b && keys > page * block_size && bt[(long)r * bt_stride] == bt[(long)b * bt_stride];
+    if (window > 0) keys = min(keys, window);
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) keys += __shfl_xor(keys, o, 64);
+  const bool any = __any(same);                    // (not __syncthreads_or(), which brings an LDS object of its own)
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = any ? -1e30f : (float)keys;
+  __syncthreads();
+  const float read = (red[0] + red[1] + red[2] + red[3]) * B / asked * bytes_per_key;
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(read >= past_bytes);
+}
+
 #define HIP_LAUNCH_CHECK()                                  \
   do {                                                      \
     hipError_t e_ = hipGetLastError();                      \

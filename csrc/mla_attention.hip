@@ -99,6 +99,7 @@ struct MlaExtra {
   int window;
   const float* sinks;                // [Hq] or null
   const void* gate; long gate_stride;  // [T, gate_stride] raw values of the element type, or null
+  float past_bytes;                  // mla_rows_kernel: read past the caches what is this much and one row's alone (0: nothing)
 };
 
 // l (relative to the running maximum m, log2 scale) and the factor the accumulators take when the sink joins
@@ -275,8 +276,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // The 16-byte pieces of a row are XOR-ed with bits 1, 3 and 4 of the key's number (the 16 rows of a K fragment then lie in
 // 16 different places of the LDS's 256 bytes).
 // Bound by reading the rows: 128 sequences of about 3100 keys, 16 heads, write of the new rows included: 99 us against 211
-// through both caches (441 and 833 MB).  ONCE: nontemporal, for more rows than the memory-side cache holds (108 us without; 16
-// sequences of 3000 keys, which it holds, 27.5 / 29).
+// through both caches (441 and 833 MB).  ONCE: what one sequence alone reads comes past the caches (nontemporal) where the
+// sequences' rows are more than the memory-side cache holds.  Several caches in turn, us, cached / past them / asking first: 128
+// sequences of 3100 keys 112 / 104 / 103, 16 of 12000 68 / 61 / 62; with 90 % of the pages shared 60 of 3000 44.9 / 46.2 / 45.5,
+// 16 of 3000 (which the cache holds) 21.9 / 24.0 / 22.3.
 // ---------------------------------------------------------------------------------------------------------------
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void mla_lds_void;
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void mla_rows_kernel(
     prow[i] = c / PIECES;
     pbyte[i] = ((c - prow[i] * PIECES) ^ swz(prow[i])) * 16;
   }
-  auto stage = [&](int g, int buf) {
+  auto stage = [&](int g, int buf, auto nt) {
     const int base = g * 32;
     const long first = (long)bt_row[base / block_size] * block_size + (base % block_size);
     const char* src = reinterpret_cast<const char*>(k_cache + first * DK);
@@ -352,86 +355,102 @@ __global__ __launch_bounds__(256, 2) void mla_rows_kernel(
     const int lo = max(win_lo - base, 0), hi = min(seq_len - 1 - base, 31);
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      mla_dma16<ONCE ? 2 : 0>(src + max(min(prow[i], hi), lo) * ROW + pbyte[i], smem + buf * 32 * ROW + (i * 256 + wid * 64) * 16);
+      mla_dma16<decltype(nt)::value>(src + max(min(prow[i], hi), lo) * ROW + pbyte[i],
+                                     smem + buf * 32 * ROW + (i * 256 + wid * 64) * 16);
   };
 
   const int key_a = 8 * (r16 >> 2) + (r16 & 3);    // K rows of the two interleaved S^T tiles: this one and 4 behind it
   const int off_a = key_a * ROW, off_b = (key_a + 4) * ROW, swz_a = swz(key_a), swz_b = swz(key_a + 4);
-  if (g_begin < g_end) stage(g_begin, 0);
-  for (int g = g_begin; g < g_end; ++g) {
-    const int buf = (g - g_begin) & 1;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();                               // the group is in LDS, and nobody reads the other buffer any more
-    if (g + 1 < g_end) stage(g + 1, buf ^ 1);
-    const char* tile = smem + buf * 32 * ROW;
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+  using Cached = std::integral_constant<int, 0>;
+  using Past = std::integral_constant<int, 2>;
+  if (g_begin < g_end) stage(g_begin, 0, Cached{});
+  auto walk = [&](auto nt) {
+    for (int g = g_begin; g < g_end; ++g) {
+      const int buf = (g - g_begin) & 1;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();                               // the group is in LDS, and nobody reads the other buffer any more
+      if (g + 1 < g_end) stage(g + 1, buf ^ 1, nt);
+      const char* tile = smem + buf * 32 * ROW;
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int piece = min(wid * KS + s, KSTEPS - 1) * 4 + g4;
-      s0 = mfma16(*reinterpret_cast<const V*>(tile + off_a + ((piece ^ swz_a) << 4)), qf[s], s0);
-      s1 = mfma16(*reinterpret_cast<const V*>(tile + off_b + ((piece ^ swz_b) << 4)), qf[s], s1);
-    }
-    *reinterpret_cast<f32x4*>(s_part[wid][0][lane]) = s0;
-    *reinterpret_cast<f32x4*>(s_part[wid][1][lane]) = s1;
-    // (not __syncthreads(), which would also wait for the next group's rows)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    s0 = *reinterpret_cast<const f32x4*>(s_part[0][0][lane]);
-    s1 = *reinterpret_cast<const f32x4*>(s_part[0][1][lane]);
+      for (int s = 0; s < KS; ++s) {
+        const int piece = min(wid * KS + s, KSTEPS - 1) * 4 + g4;
+        s0 = mfma16(*reinterpret_cast<const V*>(tile + off_a + ((piece ^ swz_a) << 4)), qf[s], s0);
+        s1 = mfma16(*reinterpret_cast<const V*>(tile + off_b + ((piece ^ swz_b) << 4)), qf[s], s1);
+      }
+      *reinterpret_cast<f32x4*>(s_part[wid][0][lane]) = s0;
+      *reinterpret_cast<f32x4*>(s_part[wid][1][lane]) = s1;
+      // (not __syncthreads(), which would also wait for the next group's rows)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      s0 = *reinterpret_cast<const f32x4*>(s_part[0][0][lane]);
+      s1 = *reinterpret_cast<const f32x4*>(s_part[0][1][lane]);
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      s0 += *reinterpret_cast<const f32x4*>(s_part[w][0][lane]);
-      s1 += *reinterpret_cast<const f32x4*>(s_part[w][1][lane]);
-    }
-    const int kidx0 = g * 32 + 8 * g4;
-    float p[8];
-    float tmax = MLA_NEG_BIG;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float sv = (j < 4 ? s0[j & 3] : s1[j & 3]) * scale_log2e;
-      p[j] = (kidx0 + j < seq_len && kidx0 + j >= win_lo) ? sv : MLA_NEG_BIG;
-      tmax = fmaxf(tmax, p[j]);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m, tmax);
-    const float alpha = fast_exp2(m - m_new);
-    float psum = 0.f;
-    V pf;
-    [[maybe_unused]] V pl;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float e = p[j] <= 0.5f * MLA_NEG_BIG ? 0.f : fast_exp2(p[j] - m_new);
-      psum += e;
-      pf[j] = (T)e;
-      if constexpr (P2) pl[j] = (T)(e - (float)pf[j]);
-    }
-    l = l * alpha + psum;
-    m = m_new;
-#pragma unroll
-    for (int i = 0; i < VI; ++i) {
-      // the piece of a row this lane's four values lie in, and which half of it
-      const int piece = (wid * VI + i) * 8 + (r16 >> 1), half = (r16 & 1) * 8;
-      u32x2 w[8];
+      for (int w = 1; w < 4; ++w) {
+        s0 += *reinterpret_cast<const f32x4*>(s_part[w][0][lane]);
+        s1 += *reinterpret_cast<const f32x4*>(s_part[w][1][lane]);
+      }
+      const int kidx0 = g * 32 + 8 * g4;
+      float p[8];
+      float tmax = MLA_NEG_BIG;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int key = 8 * g4 + j;
-        w[j] = *reinterpret_cast<const u32x2*>(tile + key * ROW + ((piece ^ swz(key)) << 4) + half);
+        const float sv = (j < 4 ? s0[j & 3] : s1[j & 3]) * scale_log2e;
+        p[j] = (kidx0 + j < seq_len && kidx0 + j >= win_lo) ? sv : MLA_NEG_BIG;
+        tmax = fmaxf(tmax, p[j]);
       }
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      const float m_new = fmaxf(m, tmax);
+      const float alpha = fast_exp2(m - m_new);
+      float psum = 0.f;
+      V pf;
+      [[maybe_unused]] V pl;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        union { uint32_t u[4]; V f; } fr;
+      for (int j = 0; j < 8; ++j) {
+        const float e = p[j] <= 0.5f * MLA_NEG_BIG ? 0.f : fast_exp2(p[j] - m_new);
+        psum += e;
+        pf[j] = (T)e;
+        if constexpr (P2) pl[j] = (T)(e - (float)pf[j]);
+      }
+      l = l * alpha + psum;
+      m = m_new;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t a = w[2 * j][v >> 1], b = w[2 * j + 1][v >> 1];
-          fr.u[j] = __builtin_amdgcn_perm(b, a, (v & 1) ? 0x07060302u : 0x05040100u);
+      for (int i = 0; i < VI; ++i) {
+        // the piece of a row this lane's four values lie in, and which half of it
+        const int piece = (wid * VI + i) * 8 + (r16 >> 1), half = (r16 & 1) * 8;
+        u32x2 w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = 8 * g4 + j;
+          w[j] = *reinterpret_cast<const u32x2*>(tile + key * ROW + ((piece ^ swz(key)) << 4) + half);
         }
-        acc[i][v] *= alpha;
-        acc[i][v] = mfma16(fr.f, pf, acc[i][v]);
-        if constexpr (P2) acc[i][v] = mfma16(fr.f, pl, acc[i][v]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          union { uint32_t u[4]; V f; } fr;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t a = w[2 * j][v >> 1], b = w[2 * j + 1][v >> 1];
+            fr.u[j] = __builtin_amdgcn_perm(b, a, (v & 1) ? 0x07060302u : 0x05040100u);
+          }
+          acc[i][v] *= alpha;
+          acc[i][v] = mfma16(fr.f, pf, acc[i][v]);
+          if constexpr (P2) acc[i][v] = mfma16(fr.f, pl, acc[i][v]);
+        }
       }
     }
+  };
+  bool past = false;
+  if constexpr (ONCE)                              // (while the first group is on its way)
+    if (g_end - g_begin >= 4)
+      past = reads_alone(&s_part[0][0][0][0], t, gridDim.z, seq_lens, block_table, bt_stride, g_begin * 32 / block_size, block_size,
+                         ex.window, ROW, ex.past_bytes);
+  if constexpr (ONCE) {
+    if (past) walk(Past{});
+    else walk(Cached{});
+  } else {
+    walk(Cached{});
   }
 
   float lsum = l;
@@ -794,14 +813,14 @@ int launch_mla(void* out, long out_stride, void* part_o, void* part_ml, const vo
     mla_attention_multi_kernel<T, DK, DV, NQ, false, KV8, P2><<<dim3(num_splits, (q_tiles + NQ - 1) / NQ, T_), 256, 0, st>>>(
         (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, k_cache, v_cache, block_table,
         bt_stride, token_seq, seq_lens, sl2, T_, Hq, block_size, num_splits, ex);
-  } else if (mode == 3 || mode == 4) {              // a workgroup per 16 heads over the key rows alone (4: past the caches)
+  } else if (mode == 3) {                           // a workgroup per 16 heads over the key rows alone
     if constexpr (!KV8 && DV % 256 == 0 && DK % 64 == 0) {
       if (block_size % 32) return -1;
 #define MLA_ROWS(ONCE)                                                                                                     \
   mla_rows_kernel<T, DK, DV, P2, ONCE><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(                                      \
       (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, (const T*)k_cache, block_table, bt_stride, \
       token_seq, seq_lens, sl2, Hq, block_size, num_splits, ex)
-      if (mode == 4) MLA_ROWS(true);
+      if (ex.past_bytes > 0) MLA_ROWS(true);
       else MLA_ROWS(false);
 #undef MLA_ROWS
     } else {
@@ -853,17 +872,18 @@ int dispatch_mla(int DK, int DV, int kv_fp8, void* out, long out_stride, void* p
 // part_o / part_ml: num_splits * T * Hq * (DV | 2) floats when num_splits > 1.
 // mode 0: one workgroup per (token, 16 heads); 1: four consecutive tokens of a sequence per workgroup (needs
 // token_seq; positions inside a sequence must be consecutive); 2: four head tiles of a token per workgroup.
-// mode 3: as mode 0, the values taken from the key rows (16-bit caches, blocks of a multiple of 32 tokens, DV a multiple of 256).
+// mode 3: as mode 0, the values taken from the key rows (16-bit caches, blocks of a multiple of 32 tokens, DV a multiple of 256);
+// past_bytes > 0 (token_seq null): where the rows seen are that many bytes, those of one token alone are read past the caches.
 // Supported (DK, DV): (576, 512) DeepSeek-V2 / V3, (320, 256), (96, 64).
 VDAMD_API int vdamd_mla_attention(void* out, long out_stride, void* part_o, void* part_ml, const void* q,
                                   long q_stride, const void* k_cache, const void* v_cache, const int* block_table,
                                   int bt_stride, const int* token_seq, const int* seq_lens, float scale, int T_,
                                   int Hq, int DK, int DV, int block_size, int num_splits, int mode, int dtype,
                                   int kv_fp8, int precise, int window, const float* sinks, const void* gate,
-                                  long gate_stride, void* stream) {
+                                  long gate_stride, long past_bytes, void* stream) {
   if (T_ <= 0) return 0;
-  if (window < 0) return -1;
-  const MlaExtra ex{window, sinks, gate, gate_stride};
+  if (window < 0 || (past_bytes > 0 && token_seq != nullptr)) return -1;
+  const MlaExtra ex{window, sinks, gate, gate_stride, (float)past_bytes};
   if (block_size % 8 || num_splits < 1 || num_splits > MLA_MAX_SPLITS) return -1;
   if (num_splits > 1 && (part_o == nullptr || part_ml == nullptr)) return -2;
   if (q_stride % 8 || out_stride % 4) return -5;

@@ -1635,3 +1635,22 @@ def test_latent_rows_past_the_caches_read_the_same(monkeypatch):
         with monkeypatch.context() as m:
             m.setattr(hip, "LATENT_ONCE_BYTES", 0)
             assert torch.equal(hip.mla_attention(*args, splits=splits, mode=3), want)
+
+
+@pytest.mark.parametrize("rows,window,splits", [(3, 0, 1), (257, 0, 2), (300, 290, 1)])
+def test_latent_rows_past_the_caches_that_share_pages(rows, window, splits, monkeypatch):
+    """Rows with a common front, rows with none and short ones; more rows than a workgroup asks; every split long enough to ask."""
+    from vllm_distributed_amd.ops import hip
+    g = torch.Generator().manual_seed(rows)
+    kc, vc = (torch.zeros(shape, dtype=torch.bfloat16, device=DEV)
+              for shape in (ops.k_cache_shape(64, 1, 576, 64), ops.v_cache_shape(64, 1, 512, 64)))
+    ops.mla_cache_write(_rand(4096, 576), kc, vc, torch.arange(4096, device=DEV, dtype=torch.int32))
+    lens = torch.randint(1, 900, (rows,), generator=g)
+    lens[0], lens[1] = 899, 1
+    table = torch.randint(0, 64, (rows, 15), generator=g).to(torch.int32)
+    table[::2, :7] = table[0, :7]
+    args = (_rand(rows, 16, 576), kc, vc, table.to(DEV), None, lens.to(DEV).int(), 0.07, 900)
+    want = hip.mla_attention(*args, splits=splits, mode=3, window=window)
+    for limit in (0, 1 << 14, 1 << 19):          # past the caches wherever nothing is shared; by what the rows hold
+        monkeypatch.setattr(hip, "LATENT_ONCE_BYTES", limit)
+        assert torch.equal(hip.mla_attention(*args, splits=splits, mode=3, window=window), want)

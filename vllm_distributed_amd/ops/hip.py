@@ -63,7 +63,7 @@ def load() -> ctypes.CDLL:
         "vdamd_moe_combine": [P, L, P, L, P, P, P, I, I, I, I, I, P, I, P],
         "vdamd_bias_clamped_glu": [P, L, P, L, P, P, P, I, I, I, I, F, F, I, P],
         "vdamd_moe_topk_grouped": [P, L, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
-        "vdamd_mla_attention": [P, L, P, P, P, L, P, P, P, I, P, P, F, I, I, I, I, I, I, I, I, I, I, I, P, P, L, P],
+        "vdamd_mla_attention": [P, L, P, P, P, L, P, P, P, I, P, P, F, I, I, I, I, I, I, I, I, I, I, I, P, P, L, L, P],
         "vdamd_mla_cache_write": [P, L, P, P, P, I, I, I, I, I, I, P],
         "vdamd_mla_prep": [P, P, L, I, I, P, L, L, P, L, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "vdamd_moe_combine_add_rms_norm": [P, L, P, L, P, P, P, I, I, I, I, I, P, P, F, I, P],
@@ -1343,8 +1343,8 @@ def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows
     return mode, max(1, min(per, keys // shortest, 64))
 
 
-# rows of the longest sequence for all of them (57 and 86 MB of rows are slower past the caches, 210 MB faster: 63 -> 57 us)
-LATENT_ONCE_BYTES = 192 << 20
+# latent rows of a decode step that are read past the caches (again and again 57 and 86 MB are slower so, 210 MB 63 -> 57 us)
+LATENT_ONCE_BYTES = 128 << 20
 
 
 def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
@@ -1381,8 +1381,9 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
-    if mode == 3 and hq <= 16 and t * keys * dk * 2 >= LATENT_ONCE_BYTES:
-        mode = 4                          # the same kernel, its rows read past the caches
+    # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
+    past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
+                                         and t * keys * dk * 2 >= LATENT_ONCE_BYTES) else 0
     splits = best if splits is None else splits
     part_o = part_ml = None
     if splits > 1:
@@ -1394,7 +1395,7 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         v_cache.data_ptr(), block_table.data_ptr(), block_table.stride(0),
         None if token_seq is None else token_seq.data_ptr(), seq_lens.data_ptr(), float(scale), t, hq, dk, dv, bs,
         splits, int(mode), _dt(q), _mla_fp8(k_cache, v_cache, q.dtype), int(bool(precise)), int(window),
-        _ptr(_f32_vec(sinks, hq, "sinks")), _ptr(gate), gate_stride, _stream()), "mla_attention")
+        _ptr(_f32_vec(sinks, hq, "sinks")), _ptr(gate), gate_stride, past, _stream()), "mla_attention")
     return out
 
 
