@@ -1,5 +1,5 @@
 """Probe: the 70B gate_up shape (N = 57344, K = 8192; 940 MB of weights) at 16 < M <= 512 through the
-library, the split-K register-ring kernel (mid_gemm, K unsplit) and the 256 x 256 LDS-DMA kernel with its
+library, the tiles of the short-batch kernel (mid_gemm, K unsplit) and the 256 x 256 LDS-DMA kernel with its
 SiLU epilogue.  Random operands, 10 launches per graph replay."""
 import os
 import sys
@@ -45,7 +45,7 @@ for m in (32, 64, 128, 192, 256, 384, 512):
     t2 = timeit(lambda: ops.silu_and_mul(torch.nn.functional.linear(x, w)))
     row.append(f"lib {t:7.1f} us ({n * k * 2 / t / 1e6:.2f} TB/s, {2 * m * n * k / t / 1e6:.0f} TF) +silu {t2:7.1f}")
     if m <= 256:
-        for bm, bn in ((256, 256), (256, 128), (128, 256), (128, 128), (64, 256)):
+        for bm, bn in hip._MID_TILES:
             if bm < min(m, 256):
                 continue
             try:

@@ -40,7 +40,7 @@
 // In tiles of 256 rows it is within 7 % of the large-batch kernel both ways between 70 and 160 rows an expert, and not built.
 //
 // 5.7 to 6.2 TB/s of W up to 48 rows.  At 256 rows the power limit sets the pace: back to back for milliseconds, gate_up takes
-// 211 us and not 187.  The LDS traffic of a K tile (x and W written once, each wave's fragments read) and its MFMAs take 2048
+// 207 - 211 us and not 187, qkv 56, o 45, down 127 (profiles/mid_gemm_tiles_mi355x.txt).  The LDS traffic of a K tile (x and W written once, each wave's fragments read) and its MFMAs take 2048
 // clocks each of about 3000.  Matrix instructions of 32x32x16 (fewer, the same LDS reads: gate_up 227 us), four waves of twice
 // the columns (77 / 66 us for 8B's at 256 x 128), each workgroup's K loop begun elsewhere and an early touch of x for the XCD's
 // L2 (both within 1 %) were tried and left out.

@@ -1102,11 +1102,13 @@ def test_mid_gemm_matches_fp32(dtype, m, n, k, pad):
     tol = dict(rtol=2e-2, atol=2e-2 * max(1.0, ref.abs().max().item()) / 4)
     got = hip.mid_gemm(x, w)
     torch.testing.assert_close(got.float(), ref, **tol)
+    # (tiles and variants as callers of the kernels before this one name them: (64, 256) and (64, 512) run as (64, 128), and every
+    # variant is the one kernel.  Each tile under its own name: test_mid_gemm_rings_of_few_tiles_and_silu)
     for bm, bn in [(256, 256), (256, 128), (128, 256), (128, 128), (64, 256), (64, 512)]:
         for ks in (1, 3, 4):
             if ks > k // 64:
                 continue
-            for variant in ((0, 1) if bn <= 256 else (0,)):      # register-staged x / LDS-DMA x with deep W prefetch
+            for variant in ((0, 1) if bn <= 256 else (0,)):
                 got = hip.mid_gemm(x, w, bm=bm, bn=bn, ksplit=ks, variant=variant)
                 torch.testing.assert_close(got.float(), ref, **tol)
     # strided output (a slice of a wider buffer), as the fused-collective path uses

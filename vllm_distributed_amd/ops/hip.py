@@ -732,8 +732,11 @@ STREAM_WIRED_MAX_M = 8
 
 
 def stream_profitable(m: int, n: int, k: int) -> bool:
-    """Up to 8 rows into a very wide output over a reduction of 2048 to 4095 (library and activation kernel 67 us, this 48 in
-    an 8B-class gate_up); longer ones are ``mid_gemm``'s (41 us), narrow outputs (a TP=8 shard) the library's."""
+    """Up to 8 rows into a very wide output over a reduction of 2048 to 4095; longer ones are ``mid_gemm``'s (28672 x 4096 by one
+    row 47 us here, 41 there), narrow outputs (a TP=8 shard) the library's.  With SiLU * up, us at 1 / 8 rows, here, by
+    ``mid_gemm`` and by library and activation kernel: 28672 x 2048 28 / 31, 23 / 23, 42 / 41; 49152 x 3072 55 / 57, 60 / 60,
+    74 / 74; 37888 x 3584 51 / 54, 58 / 60, 65 / 69; 30720 x 3840 48 / 53, 41 / 42, 60 / 60: ahead of ``mid_gemm`` only where
+    that one's last round is nearly empty."""
     return 0 < m <= STREAM_WIRED_MAX_M and n >= MID_SILU_MIN_N and 2048 <= k < MID_SILU_MIN_K
 
 
@@ -803,8 +806,9 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
-# TB/s of W that those reach.  Least squares over 930 timings of 20 weight shapes (1.3 to 940 MB) at 1 to 512 rows and every
-# split: 6 to 8 % off in the mean
+# TB/s of W that those reach.  Fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
+# and every split 8.4 % off in the mean, the chosen tile and split 3.3 % above the fastest in the mean, 40 % at most (8192 x
+# 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model)
 _MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
 # K-split counts the choice is made from (VDAMD_MID_KSPLITS=1,2,4,8,16 restricts it, for A/B measurements)
@@ -888,8 +892,10 @@ MID_SILU_MIN_N, MID_SILU_MIN_K = 24576, 4096
 
 def mid_silu_profitable(m: int, n: int, k: int) -> bool:
     """``[gate ; up]`` with the activation in the epilogue: outputs whose unsplit tiles fill the chip (14336 + 14336 columns:
-    224 of 128), over K long enough that filling and draining the ring is little of it.  8B at 1, 48 and 256 rows 41, 42 and
-    62 us (``stream_gemm`` 47, library and activation 69 and 77), 70B 151, 157 and 190 (162, 166, 215)."""
+    224 of 128).  8B at 1, 48 and 256 rows 41, 44 and 66 us (``stream_gemm`` 47, library and activation 75 and 82), 70B 152, 157
+    and 190 (162, 166, 215).  Reductions below 4096 stay where they were: up to 8 rows ``stream_gemm``'s, above that the
+    library's, though this kernel is ahead there too (37888 x 3584 at 16, 128 and 256 rows 61, 73 and 88 against 68, 85 and 93
+    outside a graph; 28672 x 2048 22, 30 and 39 against 40, 39 and 48)."""
     return 0 < m <= 256 and n >= MID_SILU_MIN_N and k >= MID_SILU_MIN_K
 
 
@@ -898,8 +904,9 @@ def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
              partials: bool = False, silu_mul: bool = False, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``x [M<=512, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
     fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit).  ``silu_mul``:
-    ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  ``bias [N]`` is added to the fp32 sums.  A tile wider than the kernel is built for
-    runs as its widest; ``variant`` names what is one kernel now and is accepted as before."""
+    ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  ``bias [N]`` is added to the fp32 sums.  Calls written for
+    the kernels before this one keep working: a tile wider than those in ``_MID_TILES`` runs as the widest of its rows, and
+    ``variant``, which named one of two kernels that are one now, has no effect."""
     assert mid_supported(x, w, silu_mul), (x.shape, x.stride(), w.shape, w.stride(), x.dtype)
     assert not (silu_mul and (partials or (ksplit or 1) != 1))
     assert bias is None or (mid_bias_ok(bias, x, w) and not partials and not silu_mul)
