@@ -1656,3 +1656,45 @@ def test_latent_rows_past_the_caches_that_share_pages(rows, window, splits, monk
     for limit in (0, 1 << 14, 1 << 19):          # past the caches wherever nothing is shared; by what the rows hold
         monkeypatch.setattr(hip, "LATENT_ONCE_BYTES", limit)
         assert torch.equal(hip.mla_attention(*args, splits=splits, mode=3, window=window), want)
+
+
+@pytest.mark.parametrize("latent", [False, True])
+def test_reads_past_the_caches_of_a_replayed_graph_go_by_the_lengths_of_the_replay(latent, monkeypatch):
+    """Captured under a bound of 960 keys; replayed over long rows, short ones, rows that share pages and rows that do not."""
+    from vllm_distributed_amd.ops import hip
+    g = torch.Generator().manual_seed(11)
+    rows, d = 20, 576 if latent else 128
+    monkeypatch.setattr(hip, "LATENT_ONCE_BYTES" if latent else "DECODE_ONCE_BYTES", 8 << 20)
+    if latent:
+        kc, vc = (torch.zeros(shape, dtype=torch.bfloat16, device=DEV)
+                  for shape in (ops.k_cache_shape(64, 1, 576, 64), ops.v_cache_shape(64, 1, 512, 64)))
+        ops.mla_cache_write(_rand(4096, 576), kc, vc, torch.arange(4096, device=DEV, dtype=torch.int32))
+    else:
+        kc, vc = (_rand(64, 2, 64, 128) * 0.5).contiguous(), _rand(64, 2, 8, 8, 16, 8).contiguous()
+    q, table, lens = _rand(rows, 16, d), torch.zeros(rows, 15, dtype=torch.int32, device=DEV), torch.ones(rows, dtype=torch.int32, device=DEV)
+
+    def attend():
+        if latent:
+            return hip.mla_attention(q, kc, vc, table, None, lens, 0.07, 960, splits=2, mode=3)
+        return hip.paged_attention_decode(q, kc, vc, table, lens, d ** -0.5, 960, num_splits=2)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        attend()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = attend()
+    for longest, shared in ((960, 0), (960, 9), (90, 0), (700, 3), (960, 15), (33, 1), (960, 0)):
+        pages = torch.randint(0, 64, (rows, 15), generator=g).to(torch.int32)
+        pages[:, :shared] = pages[0, :shared]
+        table.copy_(pages)
+        lens.copy_(torch.randint(max(1, longest // 2), longest + 1, (rows,), generator=g).to(torch.int32))
+        q.copy_(_rand(rows, 16, d))
+        graph.replay()
+        got = out.clone()
+        with monkeypatch.context() as m:
+            m.setattr(hip, "LATENT_ONCE_BYTES", 1 << 60)
+            m.setattr(hip, "DECODE_ONCE_BYTES", 1 << 60)
+            assert torch.equal(got, attend())
