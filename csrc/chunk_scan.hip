@@ -668,12 +668,12 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
 //   output waves   o = (b q) S + A u
 // with two barriers (S is there, u is there), linear kinds with one (u = v comes from memory).  Left operands come from
 // memory straight into registers, where the next chunk's take the place of those just used.
-// Bound by the chain of a chunk: its matrix instructions (1.1 us of linear kinds, 1.5 of the delta rule, at 16 columns) and its 90 -
-// 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes from the L2 through its vector cache,
-// about 64 bytes a clock; 45 - 61 KB per us of what comes from the memory-side cache) hardly overlap, as all waves wait at the same
-// barriers.  Measured per chunk and workgroup 2.5 / 3.5 us at 16 columns, 4.0 / 5.0 at
-// 32: narrow tiles where there are few workgroups (one prompt of 8000 rows, 16 heads, dim 128: 420 against 590 us), wide ones
-// where every compute unit has one anyway (five prompts, 8017 rows: 256 against 306 us).
+// Bound by the chain of a chunk: its matrix instructions (1.1 us of linear kinds, 1.5 of the delta rule, at 16 columns) and
+// its 90 - 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes from the L2 through its
+// vector cache, about 64 bytes a clock; 45 - 61 KB per us of what comes from the memory-side cache) hardly overlap, as all
+// waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.5 us at 16 columns, 4.0 / 5.0 at 32: narrow
+// tiles where there are few workgroups (one prompt of 8000 rows, 16 heads, dim 128: 420 against 590 us), wide ones where
+// every compute unit has one anyway (five prompts, 8017 rows: 256 against 306 us).
 template <int DP, bool DELTA, int NC> struct Walk {
   static constexpr int KB = DP / 16, NT = DP / 64, LD = DP + 4, LU = C + 4;
   static constexpr Layout L0 = layout_of(DP, 0, false);

@@ -40,10 +40,10 @@
 // In tiles of 256 rows it is within 7 % of the large-batch kernel both ways between 70 and 160 rows an expert, and not built.
 //
 // 5.7 to 6.2 TB/s of W up to 48 rows.  At 256 rows the power limit sets the pace: back to back for milliseconds, gate_up takes
-// 207 - 211 us and not 187, qkv 56, o 45, down 127 (profiles/mid_gemm_tiles_mi355x.txt).  The LDS traffic of a K tile (x and W written once, each wave's fragments read) and its MFMAs take 2048
-// clocks each of about 3000.  Matrix instructions of 32x32x16 (fewer, the same LDS reads: gate_up 227 us), four waves of twice
-// the columns (77 / 66 us for 8B's at 256 x 128), each workgroup's K loop begun elsewhere and an early touch of x for the XCD's
-// L2 (both within 1 %) were tried and left out.
+// 207 - 211 us and not 187, qkv 56, o 45, down 127 (profiles/mid_gemm_tiles_mi355x.txt).  The LDS traffic of a K tile (x and W
+// written once, each wave's fragments read) and its MFMAs take 2048 clocks each of about 3000.  Matrix instructions of 32x32x16
+// (fewer, the same LDS reads: gate_up 227 us), four waves of twice the columns (77 / 66 us for 8B's at 256 x 128), each
+// workgroup's K loop begun elsewhere and an early touch of x for the XCD's L2 (both within 1 %) were tried and left out.
 #include "common.h"
 
 namespace {
@@ -330,7 +330,8 @@ int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os,
 
 // out = epilogue(x[M][K] . w[N][K]^T).  K % 64 == 0, N % 16 == 0; strides in elements, multiples of 8; pointers 16-byte
 // aligned.  (bm, bn) is the workgroup tile: (256, 128|256), (128, 128|256), (64, 128).
-// epi 0: out[M][N], with bias[N] (or null, 8-byte aligned) added before the one rounding; partial holds ksplit * M * N floats when ksplit > 1, and out may be null then: the slabs are the result.
+// epi 0: out[M][N], with bias[N] (or null, 8-byte aligned) added before the one rounding; partial holds ksplit * M * N floats
+// when ksplit > 1, and out may be null then: the slabs are the result.
 // epi 2: w = [gate ; up], N % 32 == 0, ksplit 1, out[M][N/2] = silu(gate) * up.
 VDAMD_API int vdamd_mid_gemm(void* out, long out_stride, const void* x, long x_stride, const void* w, long w_stride,
                              const void* bias, void* partial, int M, int N, int K, int ksplit, int bm, int bn, int epi,
