@@ -13,22 +13,19 @@
 //   chunk_prep  a workgroup per (chunk, head), all chunks at once: A, b q, G k, U and W (everything without S)
 //   chunk_walk  a workgroup per (sequence, head, 32 value columns): the chunks one after the other, three products each
 //
-// The walk row by row (delta_rule.hip, linear_latent.hip, state_space.hip) is bound by a chain of dependent steps per
+// The linear kinds come here where segment_scan.hip, which cuts sequences into segments that run side by side, is not ahead
+// (segment_rows in ops/hip.py has the rule).  The walk row by row (delta_rule.hip, linear_latent.hip, state_space.hip) is bound by a chain of dependent steps per
 // row; here the chain has a link per 64 rows and the sums are 16x16x4 fp32 matrix instructions (a fused multiply-add per
 // term like the vector unit's: no input is narrowed).  Products of decays are formed directly, never as differences of
 // logarithms: a product between two rows of different groups of 16 is (from the start of i's group up to i) * (whole groups
 // between) * (behind j to the end of its group), each at most 1 where decays are, so nothing overflows; inside a group it
 // is the quotient of two products from the group's start, unless one of those is smaller than 2^-96 or larger than 2^96,
 // where the group's 120 pairs are multiplied out (diag_exact).  A head's products are formed so in 64 bits (2^-960, 2^960).
-#include "common.h"
-#include <math.h>
-#include <type_traits>
+#include "chunk_parts.h"
 
 namespace {
 
 constexpr int C = 64;                              // rows of a chunk
-
-enum { LINEAR_HEAD = 0, LINEAR_CHANNEL = 1, STATE_SPACE = 2, DELTA_CHANNEL = 3, DELTA_HEAD = 4 };
 
 struct ChunkArgs {
   const void* x;                                   // [T, x_stride]: q, k, v of head 0 (group 0) at the three columns
@@ -66,14 +63,6 @@ __host__ __device__ constexpr Layout layout_of(int DP, int VP, bool delta) {
   l.total = l.w + (delta ? C * DP : 0);
   return l;
 }
-
-template <typename T> __device__ __forceinline__ float ldf(const T* p) { return (float)(*p); }
-// (both sides are formed: a branch around the library functions would keep their latencies from filling each other)
-__device__ __forceinline__ float softplus_f(float x) {
-  const float l = log1pf(expf(x > 20.f ? 20.f : x));
-  return x > 20.f ? x : l;
-}
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -177,57 +166,9 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ float turn(float v) {                // of the lane in front, the first of 16 from the last
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
-}
-// Products over the 16 lanes of a row, four values side by side: the lanes up to and including this one, and those behind it.  One
-// instruction a step (a lane without a source keeps its value); from the builtin the compiler makes three, and waits between
-// them.  (A step reads what was written four instructions before; it has to be two at least, and the s_nop sees to the first.)
-#define MUL4(STEP)                                               \
-  "v_mul_f32_dpp %0, %0, %0 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_mul_f32_dpp %1, %1, %1 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_mul_f32_dpp %2, %2, %2 " STEP " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_mul_f32_dpp %3, %3, %3 " STEP " row_mask:0xf bank_mask:0xf\n\t"
-__device__ __forceinline__ void prefix_products(float& a, float& b, float& c, float& d) {
-  asm("s_nop 1\n\t" MUL4("row_shr:1") MUL4("row_shr:2") MUL4("row_shr:4") MUL4("row_shr:8")
-      : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-}
-__device__ __forceinline__ void suffix_products(const f32x4& v, float& a, float& b, float& c, float& d) {
-  a = b = c = d = 1.f;
-  asm("s_nop 1\n\t"
-      "v_mov_b32_dpp %0, %4 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-      "v_mov_b32_dpp %1, %5 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-      "v_mov_b32_dpp %2, %6 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-      "v_mov_b32_dpp %3, %7 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-      MUL4("row_shl:1") MUL4("row_shl:2") MUL4("row_shl:4") MUL4("row_shl:8")
-      : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
-}
-#undef MUL4
-
 __device__ __forceinline__ int chunks_of(const int* qsl, int B, int s) {
   const int n = s < B ? qsl[s + 1] - qsl[s] : 0;
   return n > 0 ? (n + C - 1) / C : 0;
-}
-
-// the sequence and its chunk that the batch's chunk `want` is (false: there are fewer); a wave's work
-__device__ __forceinline__ bool locate(const int* qsl, int B, int want, int& seq, int& c) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int s0 = 0; s0 < B; s0 += 64) {
-    const int cnt = chunks_of(qsl, B, s0 + lane);
-    int incl = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
-    const unsigned long long past = __ballot(base + incl > want);
-    if (past) {
-      const int l = __ffsll(past) - 1;
-      seq = s0 + l;
-      c = want - base - (__shfl(incl, l, 64) - __shfl(cnt, l, 64));
-      return true;
-    }
-    base += __shfl(incl, 63, 64);
-  }
-  return false;
 }
 
 __device__ __forceinline__ int chunks_before(const int* qsl, int B, int seq) {
@@ -237,19 +178,6 @@ __device__ __forceinline__ int chunks_before(const int* qsl, int B, int seq) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
   return sum;
-}
-
-// the sequence that is place `rank` of the batch by length, longest first (up to 64 sequences; beyond, in their order): what is
-// started first is what takes longest
-__device__ __forceinline__ int by_length(const int* qsl, int B, int rank) {
-  if (B > 64) return rank;
-  const int lane = threadIdx.x & 63, n = lane < B ? qsl[lane + 1] - qsl[lane] : -1;
-  int place = 0;
-  for (int o = 0; o < B; ++o) {
-    const int other = __shfl(n, o, 64);
-    place += other > n || (other == n && o < lane);
-  }
-  return __ffsll(__ballot(lane < B && place == rank)) - 1;
 }
 
 // grid (bound on the batch's chunks, heads of the launch), 4 waves; wave w has rows 16 w .. 16 w + 15 of the chunk: lane (kh =
@@ -272,7 +200,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   __shared__ float bl[C];
   __shared__ double td[4], sd[CHAN ? 1 : C];       // per head: products of whole groups, and of the group's decays behind a row
   int seq, c;
-  if (!locate(a.qsl, a.B, blockIdx.x, seq, c)) return;           // (the same for every wave)
+  if (!locate(a.B, blockIdx.x, seq, c, [&](int i) { return chunks_of(a.qsl, a.B, i); })) return;           // (the same for every wave)
   const int hh = blockIdx.y, h = a.h0 + hh, g = h / (a.H / a.G);
   const int q0 = a.qsl[seq], n = a.qsl[seq + 1] - q0;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;

@@ -235,3 +235,74 @@ def test_the_memory_profile_holds_what_a_step_allocates(op, new):
     used = torch.cuda.max_memory_allocated() - before - state
     bound = ops.recurrence_bytes(2000, len(new), heads, dim, vdim, op.startswith("delta"))
     assert 0 < used <= bound + 65536, (used, bound)                 # (offsets and lengths, rounded up to 512 bytes each)
+
+
+@pytest.mark.parametrize("op", OPS[:3])
+@pytest.mark.parametrize("rows", [0, 32, 96])
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("heads,dim,vdim,new,extra,dtype", [
+    (4, 128, 128, [200, 1, 63, 0, 65, 17, 96, 97], [0, 9, 70, 3, 0, 1, 0, 5], torch.bfloat16),     # remainders, states read
+    (2, 64, 64, [129, 16, 192], [5, 0, 0], torch.float16),
+    (4, 96, 80, [70, 33], [0, 12], torch.bfloat16),                        # keys and columns that end inside a tile
+    (2, 24, 40, [67, 40], [2, 0], torch.float32),
+    (2, 128, 256, [65, 100], [0, 6], torch.bfloat16),                      # two tiles of columns
+    (2, 72, 64, [161], [3], torch.bfloat16),
+    (2, 64, 136, [31, 160], [0, 0], torch.float32),
+    (3, 64, 64, *_many(70), torch.bfloat16)])                              # more sequences than a wave has lanes
+def test_segments_match_the_recurrence_in_64_bits(monkeypatch, op, rows, strong, heads, dim, vdim, new, extra, dtype):
+    """The bound of ``test_chunks_match_the_recurrence_in_64_bits``, whatever sequences are cut at (0: nowhere)."""
+    asked = []
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: asked.append(sizes) or rows)
+    c = _case(op, heads, 1 if op == "state_space" else heads, dim, vdim, new, [n + e for n, e in zip(new, extra)], dtype, 23,
+              strong, 8)
+    want, want_state = _rows64(c)
+    out, state = _run(c, True)
+    assert asked and _off(out, want) < 3e-6 and _off(state, want_state) < 3e-6, (_off(out, want), _off(state, want_state))
+    untouched = [i for i in range(c["state"].shape[0]) if i not in [int(x) for x, n in zip(c["slots"], new) if n]]
+    assert torch.equal(state[untouched], c["state"][untouched])
+    again, state2 = _run(c, True)
+    assert torch.equal(out, again) and torch.equal(state, state2)
+
+
+@pytest.mark.parametrize("op", OPS[:3])
+@pytest.mark.parametrize("rows", [0, 96])
+def test_segments_are_no_less_exact_than_chunks(monkeypatch, op, rows):
+    """Products in thirds of 24 digits, whose left-out parts are below 2^-21 of them with either sign."""
+    c = _case(op, 4, 4, 128, 128, [700, 300], [700, 420], torch.bfloat16, 3)
+    want, want_state = _rows64(c)
+    off = []
+    for cut in (rows, -1):
+        monkeypatch.setattr(hip, "segment_rows", lambda *sizes: cut)
+        out, state = _run(c, True)
+        off.append((_off(out, want), _off(state, want_state)))
+    assert off[0][0] <= 1.05 * off[1][0] and off[0][1] <= 1.05 * off[1][1], off
+
+
+@pytest.mark.parametrize("op", OPS[:3])
+@pytest.mark.parametrize("what,value", [("v", float("nan")), ("v", float("inf")), ("k", float("nan")), ("q", float("nan")),
+                                        ("dt", float("nan"))])
+@pytest.mark.parametrize("rows", [0, 64])
+def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch, op, what, value, rows):
+    if what == "dt" and op.startswith("linear"):
+        pytest.skip("the recurrence has no such input")
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    heads, dim, vdim, new, row, head = 4, 128, 128, [150, 40, 70, 33], 21 + 64, 2
+    c = _case(op, heads, heads, dim, vdim, new, [150, 47, 70, 35], torch.float32, 7)
+    clean, _ = _run(c, True)
+    if what == "dt":
+        c[what][row] = value
+    else:
+        at = {"q": 0, "k": heads * dim, "v": 2 * heads * dim}
+        if op == "state_space":
+            at = {"v": 0, "k": heads * vdim, "q": heads * vdim + heads * dim}
+        c["x"][row, at[what] + head * (vdim if what == "v" else dim) + 5] = value
+    got, _ = _run(c, True)
+    other = torch.ones(sum(new), dtype=torch.bool, device=DEV)
+    other[row:150] = False
+    assert _off(got[other], clean[other].double()) < 3e-6
+    assert not torch.isfinite(got[row].view(heads, vdim)[head]).all()
+    if what == "v":                                                 # the columns beside it are as they were
+        beside = torch.ones(vdim, dtype=torch.bool, device=DEV)
+        beside[5] = False
+        there = slice(row, 150)
+        assert _off(got[there].view(-1, heads, vdim)[:, :, beside], clean[there].view(-1, heads, vdim)[:, :, beside].double()) < 3e-6

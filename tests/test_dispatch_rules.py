@@ -23,6 +23,24 @@ def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest
     assert hip.chunk_scan_profitable(kind, rows, seqs, longest, heads, dim, vdim) is chunked
 
 
+@pytest.mark.parametrize("kind,rows,seqs,longest,heads,dim,vdim,least,most", [
+    # decoded rows, heads and states the kernels are not built for
+    (hip.LINEAR_CHANNEL, 256, 256, 1, 16, 128, 128, -1, -1), (hip.STATE_SPACE, 8000, 1, 8000, 16, 192, 128, -1, -1),
+    (hip.LINEAR_HEAD, 8000, 1, 8000, 16, 128, 512, -1, -1),
+    # long prompts, cut (chunked, segments in us): 205 / 149, 237 / 87, 113 / 56
+    (hip.LINEAR_CHANNEL, 6007, 3, 2464, 16, 128, 128, 384, 512), (hip.STATE_SPACE, 7000, 1, 7000, 8, 128, 128, 128, 320),
+    (hip.LINEAR_CHANNEL, 3000, 1, 3000, 8, 128, 128, 96, 160),
+    # many short ones, whole: 108 / 75, 64 / 50, 85 / 53
+    (hip.STATE_SPACE, 4000, 20, 400, 32, 64, 64, 0, 0), (hip.LINEAR_CHANNEL, 2512, 22, 195, 8, 128, 128, 0, 0),
+    (hip.LINEAR_HEAD, 1017, 22, 94, 16, 128, 128, 0, 0),
+    # few short ones, whose chains of 32 rows would be longer: 23 / 36, 32 / 44, 26 / 34
+    (hip.LINEAR_HEAD, 215, 1, 215, 16, 64, 128, -1, -1), (hip.LINEAR_CHANNEL, 230, 1, 230, 32, 128, 128, -1, -1),
+    (hip.STATE_SPACE, 668, 2, 374, 16, 64, 64, -1, -1)])
+def test_segments_run_where_they_are_faster(kind, rows, seqs, longest, heads, dim, vdim, least, most):
+    cut = hip.segment_rows(kind, rows, seqs, longest, heads, dim, vdim)
+    assert least <= cut <= most and (cut <= 0 or cut % 32 == 0)
+
+
 @pytest.mark.parametrize("batch,heads,keys,captured,splits", [
     # (whole against split in us) 13.5 / 18 from Python; in a graph 12.5 / 8.5 and 9.3 / 9.0
     (1, 8, 800, False, 1), (1, 8, 800, True, 12), (8, 8, 520, True, 1), (1, 8, 512, True, 1), (1, 8, 1, False, 1),

@@ -102,6 +102,7 @@ def load() -> ctypes.CDLL:
         "vdamd_decay_linear_attention": [P, P, L, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "vdamd_channel_decay_attention": [P, P, L, P, P, P, P, P, I, I, I, I, F, I, I, I, P],
         "vdamd_chunk_scan": [P, I, P, L, I, I, I, P, L, P, L, P, P, P, P, P, I, P, P, P, P] + [I] * 8 + [F, F, I, P],
+        "vdamd_segment_scan": [P, I, P, L, I, I, I, P, L, P, P, P, P, P, I, I, P, P, P, P] + [I] * 6 + [F, I, P],
         "vdamd_low_rank_decay": [P, P, L, P, P, I, I, I, F, I, P],
         "vdamd_weighted_relu_squared": [P, P, L, P, P, I, I, I, P],
         "vdamd_latent_prep": [P, P, L, L, I, P, L, L, P, L, P, F, P, I, F, P, P, P, P, I, I, I, I, I, I, I, P],
@@ -113,6 +114,8 @@ def load() -> ctypes.CDLL:
         fn.restype = c_int
     lib.vdamd_chunk_scan_floats.argtypes = [I, I, I]
     lib.vdamd_chunk_scan_floats.restype = c_long
+    lib.vdamd_segment_scan_floats.argtypes = [I, I, I]
+    lib.vdamd_segment_scan_floats.restype = c_long
     lib.vdamd_decode_workspace_floats.argtypes = [I, I, I]
     lib.vdamd_decode_workspace_floats.restype = c_long
     lib.vdamd_max_splits.restype = c_int
@@ -1647,6 +1650,7 @@ CHUNK_COSTS = {LINEAR_HEAD: (24.5, 1.15, 0.020, 0.076, 3.1, 0.306, 0.00052, 0.00
                DELTA_HEAD: (24.0, 1.65, 0.015, 0.140, 15.9, 0.312, 0.00056, 0.00299)}
 
 
+@functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
 def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int,
                           aligned: bool = True) -> bool:
     """Whether ``seqs`` sequences with ``rows`` rows in all, at most ``max_rows`` in one (0: unknown), go through the chunked
@@ -1713,6 +1717,76 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
     return out
 
 
+# The recurrences without a delta rule over segments, in us: a call, a chunk of 32 rows (fixed, and per 128 x 128 of the state),
+# what a workgroup begins with, a chunk of the pass over the states alone; beside them the chunked kernels as in CHUNK_COSTS,
+# fitted over the calls that segments were measured on.
+SEGMENT_COSTS = {LINEAR_HEAD: (6.9, 2.42, 5.1, 7.1, 0.0, 1.18), LINEAR_CHANNEL: (8.3, 2.03, 3.9, 5.0, 0.62, 0.0),
+                 STATE_SPACE: (9.4, 2.20, 2.8, 5.4, 0.0, 0.91)}
+CHUNK_COSTS_BESIDE = {LINEAR_HEAD: (18.6, 0.89, 0.015, 0.078), LINEAR_CHANNEL: (16.3, 1.30, 0.007, 0.081),
+                      STATE_SPACE: (18.0, 1.18, 0.015, 0.060)}
+
+
+@functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
+def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> int:
+    """Rows at which sequences are cut into segments that run side by side (0: none is cut), or -1: the chunked kernels, whose
+    preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all segments run at a time,
+    by an estimate of how many there are, or 96 rows.  Modelled times on an MI355X, fitted over 980 timings of 220 calls (8 to 32
+    heads, 1 to 24 sequences, 30 to 7500 rows); as the model is off by 13 % (root mean square), segments where they are 15 to 20 %
+    ahead: 1.2 times as fast on average as the chunked kernels alone (one prompt of 7000 rows, 8 heads of 128 x 128, state space 237 against
+    87 us; five of 500 rows, 32 heads of 64 x 128, 111 against 137: not chosen)."""
+    longest = max_rows if max_rows > 0 else -(-rows // max(seqs, 1))
+    if longest < CHUNK_MIN_ROWS or dim > CHUNK_MAX_DIM or vdim > 256:     # (wider: more scratch than the chunks' operands)
+        return -1
+    dp, vp = 64 if dim <= 64 else 128, 64 if vdim <= 64 else -(-vdim // 128) * 128
+    call, link, head, per = CHUNK_COSTS_BESIDE[kind]
+    limit = call + longest / 64 * link * (0.5 + dp / 256) + (rows / 64 + seqs) * heads * (head + per * dp * vdim / 16384)
+    walk_call, row, row_head, row_area = CHUNK_COSTS[kind][4:]
+    limit = min(limit, walk_call + math.hypot(longest * row, rows * heads * (row_head + row_area * dim * vdim / 16384)))
+    limit *= 0.8 if kind == LINEAR_HEAD else 0.85
+    begin, fixed, area, over, state_fixed, state_area = SEGMENT_COSTS[kind]
+    share = min(vp, 128) * dp / 16384              # of a workgroup in the largest state tile
+    work = heads * max(vp // 128, 1) / (512 if share <= 0.25 else 256)           # of the workgroups that run at a time, a segment's
+    chunk, state = fixed + area * share, state_fixed + state_area * share
+    best, choice = begin + max(longest / 32 * chunk + over, ((rows / 32 + 0.5 * seqs) * chunk + seqs * over) * work), 0
+    others, unsure = (rows - longest) / max(seqs - 1, 1), 0.6 * math.sqrt(seqs - 1)
+    room = 1.0 / work - unsure - 0.5 * seqs        # segments of whole length that run at a time
+    for cut in (96, max(96, int(rows / room / 32 + 1) * 32) if room > 0 else 96):
+        if cut >= longest:
+            continue
+        segments = -(-longest // cut) + (seqs - 1) * (others / cut + 0.5)
+        turns = (segments + unsure) * work
+        turns = max(1, math.ceil(turns)) if turns < 4 else turns + 0.5
+        time = (begin + turns * (cut / 32 * chunk + over) + 0.5 * over
+                + max(1.0, (segments - seqs) * work) * (cut / 32 * state + over) + segments * heads * dp * vp / 16384 * 0.03)
+        if time < best:
+            best, choice = time, cut
+    return choice if best < limit else -1
+
+
+def _segment_scan(kind: int, x, q_off: int, k_off: int, v_off: int, dt, dt_bias, a_log, decay, d_skip, num_heads: int,
+                  groups: int, dim: int, vdim: int, state, slots, query_start_loc, seq_lens, silu: bool, scale: float,
+                  max_rows: int) -> Optional[torch.Tensor]:
+    """A recurrence without a delta rule over all sequences of a step (shapes checked by the caller) in segments; None where other
+    kernels are to do it."""
+    t, b, per = x.shape[0], seq_lens.shape[0], 16 // x.element_size()
+    rows = segment_rows(kind, t, b, max_rows, num_heads, dim, vdim) if t and b else -1
+    if rows < 0 or (x.stride(0) % per or x.data_ptr() % 16 or q_off % per or k_off % per or v_off % per or dim % 8 or vdim % 8
+                    or (kind == LINEAR_CHANNEL and decay.data_ptr() % 16) or num_heads * vdim > 1 << 20):
+        return None
+    segments = b if rows == 0 else (t + (rows - 1) * min(b, t)) // rows
+    floats = int(_LIB.vdamd_segment_scan_floats(num_heads, dim, vdim)) * segments if rows else 0
+    if 8 * floats > CHUNK_SCRATCH_BYTES:           # (no more than chunk_scan_bytes, however many heads at a time that counts)
+        return None
+    out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
+    ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
+    _check(_LIB.vdamd_segment_scan(
+        out.data_ptr(), kind, x.data_ptr(), x.stride(0), q_off, k_off, v_off, _ptr(dt), 0 if dt is None else dt.stride(0),
+        _ptr(dt_bias), _ptr(a_log), _ptr(decay), _ptr(d_skip), _ptr(ws), rows, segments, state.data_ptr(), slots.data_ptr(),
+        query_start_loc.data_ptr(), seq_lens.data_ptr(), b, num_heads, groups, dim, vdim, int(silu), float(scale), _dt(x),
+        _stream()), "segment_scan")
+    return out
+
+
 def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int, decay: torch.Tensor,
                            state: torch.Tensor, slots: torch.Tensor, query_start_loc: torch.Tensor,
                            seq_lens: torch.Tensor, silu: bool = True, max_query_len: int = 0,
@@ -1731,11 +1805,16 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
     elif scale != 1.0:
         raise NotImplementedError("a scale on the result needs decays per key channel")
     kind = LINEAR_CHANNEL if decay.dim() == 2 else LINEAR_HEAD
-    if _chunked(kind, x, t, n, max_query_len, num_heads, dim, vdim) if chunked is None else chunked:
+    if chunked or (chunked is None and not 0 < max_query_len < CHUNK_MIN_ROWS):
         qs = num_heads * dim
-        return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None,
-                           decay if decay.dim() == 2 else _f32_vec(decay, num_heads, "decay"), None, num_heads, num_heads,
-                           dim, vdim, state, slots, query_start_loc, seq_lens, silu, 0.0, scale)
+        rates = decay if decay.dim() == 2 else _f32_vec(decay, num_heads, "decay")
+        out = _segment_scan(kind, x, 0, qs, 2 * qs, None, None, None, rates, None, num_heads, num_heads, dim, vdim, state, slots,
+                            query_start_loc, seq_lens, silu, scale, max_query_len)
+        if out is not None:
+            return out
+        if chunked or _chunked(kind, x, t, n, max_query_len, num_heads, dim, vdim):
+            return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None, rates, None, num_heads, num_heads, dim, vdim,
+                               state, slots, query_start_loc, seq_lens, silu, 0.0, scale)
     out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
     if decay.dim() == 2:
         _check(_LIB.vdamd_channel_decay_attention(
@@ -2052,12 +2131,15 @@ def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, 
     assert state is not None and state.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (h, n, vdim), (tuple(state.shape), (h, n, vdim))
     assert slots.shape[0] == b and query_start_loc.shape[0] >= b + 1
-    if _chunked(STATE_SPACE, x, t, b, max_query_len, h, n, int(vdim)) if chunked is None else chunked:
+    if chunked or (chunked is None and not 0 < max_query_len < CHUNK_MIN_ROWS):
         inner = h * vdim
-        return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, _f32_vec(dt_bias, h, "dt_bias"),
-                           _f32_vec(a_log, h, "a_log"), None, _f32_vec(d_skip, h, "d_skip"), h, g, n, int(vdim), state,
-                           _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"), False,
-                           0.0, 1.0)
+        mine = (_f32_vec(dt_bias, h, "dt_bias"), _f32_vec(a_log, h, "a_log"), None, _f32_vec(d_skip, h, "d_skip"), h, g, n, int(vdim),
+                state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"), False)
+        out = _segment_scan(STATE_SPACE, x, inner + g * n, inner, 0, dt, *mine, 1.0, max_query_len)
+        if out is not None:
+            return out
+        if chunked or _chunked(STATE_SPACE, x, t, b, max_query_len, h, n, int(vdim)):
+            return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, *mine, 0.0, 1.0)
     out = torch.empty((t, h * vdim), dtype=torch.float32, device=x.device)
     _check(_LIB.vdamd_selective_scan(
         out.data_ptr(), x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), _f32_vec(a_log, h, "a_log").data_ptr(),
