@@ -16,6 +16,25 @@ __device__ __forceinline__ float softplus_f(float x) {
   return x > 20.f ? x : l;
 }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+// e^x for x above -200 (below: as there, zero).  The library's function less its compares and selects
+__device__ __forceinline__ float exp_f(float x) {
+  x = x < -200.f ? -200.f : x;
+  const float n = rintf(x * 1.44269502f);
+  return ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -n))), (int)n);
+}
+// e^(-rate softplus(x)).  softplus(x) is softplus(-|x|) more than x where x > 0, and ln(1 + t) = 2 atanh(t / (2 + t)), whose series
+// converges for t <= 1 (arguments up to 1 / 3; the coefficients are those of a fit by Chebyshev polynomials, off by 1e-9).  A fifth
+// of the instructions of the library's exponentials and logarithm; error against 64 bits, root mean square, library and here:
+// rate 4, x in -6 .. -2 2.2e-8 and 2.2e-8, x in -2 .. 2 1.20e-7 and 1.25e-7, x in 2 .. 8 4.9e-7 and 4.8e-7
+__device__ __forceinline__ float decay_f(float x, float rate) {
+  const float t = exp_f(-fabsf(x)), w = 2.f + t, wl = t - (w - 2.f), r = __builtin_amdgcn_rcpf(w);
+  float s = t * r;
+  s = fmaf(fmaf(-wl, s, fmaf(-w, s, t)), r, s);
+  const float z = s * s;
+  const float p = fmaf(fmaf(fmaf(fmaf(0.122047015f, z, 0.106971338f), z, 0.143103123f), z, 0.199993476f), z, 0.333333403f);
+  const float l = fmaf(2.f * s, z * p, 2.f * s);
+  return exp_f(-rate * ((x > 0.f ? x : 0.f) + l));
+}
 // x sigmoid(x), within two units of the last place: the exponent's product with what it was rounded by, and the reciprocal with a
 // step of Newton's, are a third of the library's instructions (whose scaling and fix-up have nothing to do here)
 __device__ __forceinline__ float silu_f(float x) {
@@ -138,6 +157,29 @@ template <bool UP, int P, int N> __device__ __forceinline__ void store4(bf16_t (
   if constexpr (!UP) {
     *reinterpret_cast<bf16x4*>(planes[1] + at) = four(t.m);
     *reinterpret_cast<bf16x4*>(planes[2] + at) = four(t.l);
+  }
+}
+// a lane's N values of row r, columns c0 .. (c1 given: four there and four from c1 on), into planes by column, LD to a column: two
+// rows' values of a column are one word, the even row's lane writes the even columns and the odd row's, its neighbour, the odd ones
+template <int LD, bool UP, int N, int P, int M>
+__device__ __forceinline__ void store_columns(bf16_t (&planes)[P][M], int c0, int r, const Thirds& t, int c1 = -1) {
+  const bool odd = r & 1;
+  const unsigned pick = odd ? 0x03020706u : 0x05040100u;
+  if (c1 < 0) c1 = c0 + 4;
+  auto plane = [&](bf16_t* p, bf16x8 v) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const i32x4 w = __builtin_bit_cast(i32x4, v);
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const int near = __builtin_amdgcn_update_dpp(0, w[i], 0xB1, 0xf, 0xf, false);        // of the row r ^ 1
+      const int column = (i < 2 ? c0 + 2 * i : c1 + 2 * i - 4) + odd;
+      *reinterpret_cast<unsigned*>(p + column * LD + (r & ~1)) = __builtin_amdgcn_perm(near, w[i], pick);
+    }
+  };
+  plane(planes[0], t.h);
+  if constexpr (!UP) {
+    plane(planes[1], t.m);
+    plane(planes[2], t.l);
   }
 }
 template <int M, bool UP, int P, int N> __device__ __forceinline__ Thirds load_third(const bf16_t (&planes)[P][N], int at) {

@@ -8,20 +8,22 @@
 // row i, a chunk is
 //   linear      o_i = (b_i q_i)^T S_0 + sum_(j <= i) A_ij v_j,  A_ij = q_i^T G_ij k_j ;  S = b_64 S_0 + sum_j (G_64,j k_j) v_j^T
 //   delta rule  the same with u for v, where (I + diag(beta) L) u = diag(beta) (v - (b k)^T S_0), L_ij = k_i^T G_ij k_j (j < i):
-//               u = U - W S_0 with U and W, the solutions for beta v and for beta (b k), known without the state
+//               u = U - W S_0 with U = T v and W = T (b k), T = (I + diag(beta) L)^-1 diag(beta), known without the state
 //
 //   chunk_prep  a workgroup per (chunk, head), all chunks at once: A, b q, G k, U and W (everything without S)
 //   chunk_walk  a workgroup per (sequence, head, 32 value columns): the chunks one after the other, three products each
 //
 // The linear kinds come here where segment_scan.hip, which cuts sequences into segments that run side by side, is not ahead
-// (segment_rows in ops/hip.py has the rule).  The walk row by row (delta_rule.hip, linear_latent.hip, state_space.hip) is bound by a chain of dependent steps per
-// row; here the chain has a link per 64 rows and the sums are 16x16x4 fp32 matrix instructions (a fused multiply-add per
-// term like the vector unit's: no input is narrowed).  Products of decays are formed directly, never as differences of
-// logarithms: a product between two rows of different groups of 16 is (from the start of i's group up to i) * (whole groups
+// (segment_rows in ops/hip.py has the rule).  The walk row by row (delta_rule.hip, linear_latent.hip, state_space.hip) is bound by a
+// chain of dependent steps per row; here the chain has a link per 64 rows and the sums are matrix instructions: A, L and the linear
+// kinds' walk 16x16x4 fp32 ones (a fused multiply-add per term like the vector unit's: no input is narrowed), the delta rule's U, W
+// and walk 16-bit ones on operands in three pieces (Thirds in chunk_parts.h).  Products of decays are formed directly, never as
+// differences of logarithms: a product between two rows of different groups of 16 is (from the start of i's group up to i) * (whole groups
 // between) * (behind j to the end of its group), each at most 1 where decays are, so nothing overflows; inside a group it
 // is the quotient of two products from the group's start, unless one of those is smaller than 2^-96 or larger than 2^96,
 // where the group's 120 pairs are multiplied out (diag_exact).  A head's products are formed so in 64 bits (2^-960, 2^960).
 #include "chunk_parts.h"
+#include <utility>
 
 namespace {
 
@@ -183,19 +185,22 @@ __device__ __forceinline__ int chunks_before(const int* qsl, int B, int seq) {
 // grid (bound on the batch's chunks, heads of the launch), 4 waves; wave w has rows 16 w .. 16 w + 15 of the chunk: lane (kh =
 // lane / 16, lane % 16) holds channels 16 kb + 4 kh + e of row lane % 16 in registers, which is at once the left operand
 // (row, reduction index 4 kh + e) and the right one of the matrix instruction and the lane layout of the products
-// over rows (DPP).  Only G k and, in the solve, M and beta b k cross waves, through LDS.
+// over rows (DPP).  Only G k and, for U and W, M, its inverse and b k cross waves, through LDS.
 // Bound by what it writes (112 KB per chunk and head, the delta rule 144: linear attention's 6007 rows x 16 heads, 170 MB,
-// in 67 us) and, with a decay per channel under the delta rule, by vector instructions (half of the time: 8017 rows x 16 heads
-// 189 us; 215 with a branch around each element's exponentials and their bias loaded inside it, and running products of three
-// instructions a step).
+// in 67 us) and, under the delta rule, by instructions: of 65 000 cycles of a workgroup, two to a compute unit, 14 000 wait for its
+// rows, 16 000 go into A and L of the last 16 rows, 17 000 into U, W and the inverse, 8 000 into norms and running products (16 heads,
+// 8017 rows, a decay per channel).  There 150 us; 195 with the library's exponentials and logarithm (a third of its instructions)
+// and with U and W by substitution in fp32, W stored as it left the accumulators, four bytes a lane.
 template <typename T, int KIND, int DP>
 __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   constexpr bool DELTA = KIND >= DELTA_CHANNEL, CHAN = KIND == LINEAR_CHANNEL || KIND == DELTA_CHANNEL;
-  constexpr int KB = DP / 16, NP = CHAN ? KB * 4 : 1, LD = DP + 4, LM = C + 4;
+  constexpr int KB = DP / 16, NP = CHAN ? KB * 4 : 1, LD = DP + 4, LM = C + 4, LT = C + 8;
   constexpr Layout L0 = layout_of(DP, 0, false);
   __shared__ __attribute__((aligned(16))) float ks[C * LD];
   __shared__ __attribute__((aligned(16))) float tl[CHAN ? 4 * DP : 4];
-  __shared__ __attribute__((aligned(16))) float mn[DELTA ? C * LM : 4];      // -beta L
+  // -beta L, and in its place the thirds of (I + beta L)^-1 beta
+  __shared__ __attribute__((aligned(16))) union { float l[DELTA ? C * LM : 4]; bf16_t t[3][DELTA ? C * LT : 8]; } m;
+  float* const mn = m.l;
   __shared__ __attribute__((aligned(16))) float ti[DELTA ? 4 * 16 * 20 : 4]; // inverses of the diagonal blocks
   __shared__ float bl[C];
   __shared__ double td[4], sd[CHAN ? 1 : C];       // per head: products of whole groups, and of the group's decays behind a row
@@ -218,6 +223,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   if constexpr (KIND == DELTA_CHANNEL)
 #pragma unroll
     for (int i = 0; i < 4 * KB; ++i) bias[i] = a.dt_bias[h * a.dim + min(16 * (i / 4) + 4 * kh + i % 4, a.dim - 1)];
+  [[maybe_unused]] const float raw_beta = DELTA ? ldf((const T*)a.beta + row * a.beta_stride + h) : 0.f;
   const int valid = min(16, n - (c * C + 16 * wave));            // rows of the wave that exist (none: <= 0)
   const long row0 = q0 + c * C + 16 * wave;
   float* mine = ks + 16 * wave * LD;               // the wave's rows of ks, free until it writes G k there
@@ -271,7 +277,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float decay = expf(-rate * softplus_f(dk[kb][e] + bias[4 * kb + e]));
+        const float decay = decay_f(dk[kb][e] + bias[4 * kb + e], rate);
         dk[kb][e] = ok && 16 * kb + 4 * kh + e < a.dim ? decay : 1.f;
       }
   }
@@ -288,7 +294,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) { q[kb][e] *= iq; k[kb][e] *= ik; }
-    if (kh == 0) bl[r] = ok ? sigmoid_f(ldf((const T*)a.beta + row * a.beta_stride + h)) : 0.f;
+    if (kh == 0) bl[r] = ok ? sigmoid_f(raw_beta) : 0.f;
   }
   float own = 1.f;                                 // per head: the row's decay,
   double pd = 1.0, after = 1.0;                    // the products of the group's up to the row, and behind it
@@ -329,8 +335,10 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
   }
   bool far = false;                                // a product too small or too large to divide by
   if constexpr (CHAN) {
+    unsigned beyond = 0;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) far = far || !(fabsf(p[i]) >= 0x1p-96f && fabsf(p[i]) <= 0x1p96f);
+    for (int i = 0; i < NP; ++i) beyond = max(beyond, (bits(p[i]) << 1) - 0x1f000000u);
+    far = beyond > 0xc0000000u;                    // (an exponent outside -96 .. 96, infinities and NaN among them)
   } else {
     far = !(fabs(pd) >= 0x1p-960 && fabs(pd) <= 0x1p960);
   }
@@ -392,7 +400,9 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
       if constexpr (CHAN)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          kd[e] /= P(kb, e);
+          float r = __builtin_amdgcn_rcpf(P(kb, e));           // (within an ulp of the quotient: its scale and fix-up have
+          r = fmaf(fmaf(-P(kb, e), r, 1.f), r, r);             // nothing to do here)
+          kd[e] *= r;
           q[kb][e] *= P(kb, e);
           k[kb][e] *= P(kb, e);
         }
@@ -545,45 +555,134 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) ti[(16 * wave + i) * 20 + lr] = t[i];
     }
+    RowLoad<T, DP> lv;                             // the first columns of v, on their way
+    if (a.vvec) lv.fetch(xv, a.x_stride, valid, a.vdim, 0.f);
     __syncthreads();
-    // columns of [beta b k | beta v], 16 at a time; an accumulator's layout is the right operand's: solved blocks stay in registers
-    float* wp = ws + L0.u + a.VP * C;
-    float odd = 0.f;
-    for (int t0 = 0; t0 < KB + vt; t0 += KB) {
-      const bool keys = t0 == 0;
-      if (!keys) {
-        __syncthreads();                           // the other waves have read the previous columns
-        values(16 * (t0 - KB));
-        __syncthreads();
-      }
-      auto solve = [&](auto apart) {
-        for (int t = wave; t < KB && t0 + t < KB + vt; t += 4) {
-          f32x4 X[4];
+    // the rest of the inverse: a wave 16 columns, block by block; an accumulator's layout is the right operand's
+    f32x4 X[4], below[4][3], own_block[4];          // (all read at once: one by one, each is waited for in the chain)
 #pragma unroll
-          for (int I = 0; I < 4; ++I) {
-            f32x4 acc;
+    for (int I = 0; I < 4; ++I) {
+      own_block[I] = *reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int i = 16 * I + 4 * kh + e;
-              acc[e] = ks[i * LD + 16 * t + lr] * bl[i];
-            }
+      for (int J = 0; J < I; ++J) below[I][J] = *reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh);
+    }
+    auto rest = [&](auto apart) {
 #pragma unroll
-            for (int J = 0; J < I; ++J)
-              acc += dot16(*reinterpret_cast<const f32x4*>(mn + (16 * I + lr) * LM + 16 * J + 4 * kh), X[J]);
-            if constexpr (apart) X[I] = lower16([&](int i, int g, int f) { return ti[(16 * I + i) * 20 + 4 * g + f]; }, acc);
-            else X[I] = dot16(*reinterpret_cast<const f32x4*>(ti + (16 * I + lr) * 20 + 4 * kh), acc);
-            if constexpr (!apart) odd = not_finite(X[I], odd);
-            if (keys) {
+      for (int I = 0; I < 4; ++I) {
+        X[I] = zero;
+        if (I == wave)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) wp[piece(I * KB + t, (lr >> 2) * 16 + 4 * kh + e) + (lr & 3)] = -X[I][e];
-            } else {
-              *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 - KB + t) * 4 + I, lane)) = X[I];
-            }
-          }
+          for (int e = 0; e < 4; ++e) X[I][e] = ti[(16 * I + 4 * kh + e) * 20 + lr];
+        if (I > wave) {
+          f32x4 acc = zero;
+#pragma unroll
+          for (int J = 0; J < I; ++J)
+            if (J >= wave) acc += dot16(below[I][J], X[J]);
+          if constexpr (apart) X[I] = lower16([&](int i, int g, int f) { return ti[(16 * I + i) * 20 + 4 * g + f]; }, acc);
+          else X[I] = dot16(own_block[I], acc);
         }
-      };
-      solve(std::false_type{});
-      if (__builtin_expect(__any(odd != 0.f), 0)) solve(std::true_type{});
+      }
+    };
+    rest(std::false_type{});
+    if (__builtin_expect(__any(not_finite(X[3], not_finite(X[2], not_finite(X[1], 0.f))) != 0.f), 0)) rest(std::true_type{});
+    const float beta = bl[16 * wave + lr];
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) X[I][e] = I > wave || (I == wave && 4 * kh + e >= lr) ? X[I][e] * beta : 0.f;
+    __syncthreads();                               // M has been read
+#pragma unroll
+    for (int I = 0; I < 4; I += 2)
+      store_columns<LT, false, 8>(m.t, 16 * I + 4 * kh, 16 * wave + lr, thirds<false>(X[I], X[I + 1]), 16 * (I + 1) + 4 * kh);
+    __syncthreads();
+    // rows 32 s .. of the columns 16 t .. in ks
+    auto column = [&](int t, int s) {
+      f32x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = ks[(32 * s + 8 * kh + e) * LD + 16 * t + lr];
+        hi[e] = ks[(32 * s + 8 * kh + 4 + e) * LD + 16 * t + lr];
+      }
+      return std::pair<f32x4, f32x4>(lo, hi);
+    };
+    auto inverse = [&](int I, int s) { return load_third<8, false>(m.t, (16 * I + lr) * LT + 32 * s + 8 * kh); };
+    // term by term, where something is not finite: a zero of the inverse would hand it to the rows in front
+    auto apart = [&](int i, int col) {
+      float o = 0.f;
+#pragma unroll 1
+      for (int j = 0; j <= i; ++j) {
+        const float h = (float)m.t[0][i * LT + j], sum = h + ((float)m.t[1][i * LT + j] + (float)m.t[2][i * LT + j]);
+        o += (sum != sum ? h : sum) * ks[j * LD + col];
+      }
+      return o;
+    };
+    // W, transposed (keys by rows: the layout of a left operand as it leaves the accumulator), of 16 keys at a time
+    float* wp = ws + L0.u + a.VP * C;
+    for (int t = wave; t < KB; t += 4) {
+      Thirds keys[2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const auto k2 = column(t, s);
+        keys[s] = thirds<false>(k2.first, k2.second);
+      }
+      Sum sum[4] = {};
+#pragma unroll
+      for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int s = 0; s <= I / 2; ++s) {
+          const Thirds rows[1] = {inverse(I, s)};
+          products<false, false>(keys[s], rows, *reinterpret_cast<Sum(*)[1]>(&sum[I]));
+        }
+      f32x4 w[4];
+      float odd = 0.f;
+#pragma unroll
+      for (int I = 0; I < 4; ++I) {
+        w[I] = sum[I].h + sum[I].s;
+        odd = not_finite(w[I], odd);
+      }
+      if (__builtin_expect(__any(odd != 0.f), 0))
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[I][e] = apart(16 * I + lr, 16 * t + 4 * kh + e);
+#pragma unroll
+      for (int I = 0; I < 4; ++I) *reinterpret_cast<f32x4*>(wp + piece(I * KB + t, lane)) = -w[I];
+    }
+    // U, of 16 columns at a time
+    for (int t0 = 0; t0 < vt; t0 += KB) {
+      __syncthreads();                             // the other waves have read what is there
+      if (a.vvec && t0 == 0) lv.stash(mine, LD);
+      else values(16 * t0);
+      __syncthreads();
+      for (int t = wave; t < KB && t0 + t < vt; t += 4) {
+        constexpr bool V16 = std::is_same_v<T, bf16_t>;
+        Thirds v[2][1];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const auto v2 = column(t, s);
+          if constexpr (V16) v[s][0].h = upper(v2.first, v2.second);
+          else v[s][0] = thirds<false>(v2.first, v2.second);
+        }
+        Sum sum[4] = {};
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+#pragma unroll
+          for (int s = 0; s <= I / 2; ++s) products<false, V16>(inverse(I, s), v[s], *reinterpret_cast<Sum(*)[1]>(&sum[I]));
+        f32x4 u[4];
+        float odd = 0.f;
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+          u[I] = sum[I].h + sum[I].s;
+          odd = not_finite(u[I], odd);
+        }
+        if (__builtin_expect(__any(odd != 0.f), 0))
+#pragma unroll
+          for (int I = 0; I < 4; ++I)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[I][e] = apart(16 * I + 4 * kh + e, 16 * t + lr);
+#pragma unroll
+        for (int I = 0; I < 4; ++I) *reinterpret_cast<f32x4*>(ws + L0.u + piece((t0 + t) * 4 + I, lane)) = u[I];
+      }
     }
   }
 }
@@ -596,18 +695,16 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
 //   output waves   o = (b q) S + A u
 // with two barriers (S is there, u is there), linear kinds with one (u = v comes from memory).  Left operands come from
 // memory straight into registers, where the next chunk's take the place of those just used.
-// Bound by the chain of a chunk: its matrix instructions (1.1 us of linear kinds, 1.5 of the delta rule, at 16 columns) and
-// its 90 - 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes from the L2 through its
+// Bound by the chain of a chunk: its matrix instructions (1.1 us of linear kinds at 16 columns, the delta rule 0.6 and as much
+// again to split its operands) and its 90 - 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes from the L2 through its
 // vector cache, about 64 bytes a clock; 45 - 61 KB per us of what comes from the memory-side cache) hardly overlap, as all
-// waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.5 us at 16 columns, 4.0 / 5.0 at 32: narrow
-// tiles where there are few workgroups (one prompt of 8000 rows, 16 heads, dim 128: 420 against 590 us), wide ones where
-// every compute unit has one anyway (five prompts, 8017 rows: 256 against 306 us).
-template <int DP, bool DELTA, int NC> struct Walk {
-  static constexpr int KB = DP / 16, NT = DP / 64, LD = DP + 4, LU = C + 4;
+// waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.0 us at 16 columns, 4.0 / 3.8 at 32 (the delta
+// rule in fp32: 3.5 and 5.0; five prompts of 8017 rows, 16 heads: 221 against 177 us).
+template <int DP, int NC> struct LinearWalk {
+  static constexpr int KB = DP / 16, NT = DP / 64, LD = DP + 4;
   static constexpr Layout L0 = layout_of(DP, 0, false);
   struct Shared {
-    __attribute__((aligned(16))) float sl[DELTA ? 1 : 2][16 * NC * LD];
-    __attribute__((aligned(16))) float ul[DELTA ? 16 * NC * LU : 4];
+    __attribute__((aligned(16))) float sl[2][16 * NC * LD];
   };
   static __device__ __forceinline__ f32x4 at(const float* p, int offset) { return *reinterpret_cast<const f32x4*>(p + offset); }
 
@@ -620,25 +717,15 @@ template <int DP, bool DELTA, int NC> struct Walk {
   __device__ __forceinline__ const float* chunk_at(int c) const { return ws + step * min(c, nc - 1); }
   __device__ __forceinline__ f32x4 left(const float* p, int offset, int index) const { return at(p, offset + piece(index, lane)); }
 
-  struct StateOps { f32x4 w[DELTA ? KB : 1], k[NT][4], u[DELTA ? 1 : 4][NC], b[NT]; };
-  struct OutOps { f32x4 q[KB], a[4], u[DELTA ? 1 : 4][NC]; };
+  struct StateOps { f32x4 k[NT][4], u[4][NC], b[NT]; };
+  struct OutOps { f32x4 q[KB], a[4], u[4][NC]; };
 
-  __device__ __forceinline__ void load_first(StateOps& r, int c) const {
-    const float* p = chunk_at(c);
-    if constexpr (DELTA) {
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) r.w[kb] = left(p, L0.u + VP * C, wave * KB + kb);
-#pragma unroll
-      for (int ct = 0; ct < NC; ++ct) r.u[0][ct] = left(p, L0.u, (NC * tile + ct) * 4 + wave);
-    }
-    __builtin_amdgcn_sched_barrier(0);             // (the loads stay where they are put)
-  }
+  __device__ __forceinline__ void load_first(StateOps&, int) const {}
   template <typename Ops> __device__ __forceinline__ void load_values(Ops& r, const float* p) const {
-    if constexpr (!DELTA)
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+    for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int ct = 0; ct < NC; ++ct) r.u[kb][ct] = left(p, L0.u, (NC * tile + ct) * 4 + kb);
+      for (int ct = 0; ct < NC; ++ct) r.u[kb][ct] = left(p, L0.u, (NC * tile + ct) * 4 + kb);
   }
   __device__ __forceinline__ void load_second(StateOps& r, int c) const {
     const float* p = chunk_at(c);
@@ -692,7 +779,7 @@ template <int DP, bool DELTA, int NC> struct Walk {
 
   __device__ __forceinline__ void chunk(StateOps& r, int c, f32x4 (&S)[NT][NC]) const {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    float* sl = sh.sl[DELTA ? 0 : c & 1];
+    float* sl = sh.sl[c & 1];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -700,27 +787,10 @@ template <int DP, bool DELTA, int NC> struct Walk {
         *reinterpret_cast<f32x4*>(sl + (16 * ct + lr) * LD + (wave * NT + t) * 16 + 4 * kh) = S[t][ct];
     __syncthreads();
     f32x4 x[4][NC];
-    if constexpr (DELTA) {
-      f32x4 us[NC][2];
 #pragma unroll
-      for (int ct = 0; ct < NC; ++ct) { us[ct][0] = r.u[0][ct]; us[ct][1] = zero; }
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int kb = 0; kb < KB; kb += 4) {
-        read_four<LD>(sl, kb, x);
-        four<false>(&r.w[kb], x, us);
-      }
-#pragma unroll
-      for (int ct = 0; ct < NC; ++ct)
-        *reinterpret_cast<f32x4*>(sh.ul + (16 * ct + lr) * LU + 16 * wave + 4 * kh) = us[ct][0] + us[ct][1];
-      load_first(r, c + 1);
-      __syncthreads();
-      read_four<LU>(sh.ul, 0, x);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int ct = 0; ct < NC; ++ct) x[i][ct] = r.u[i][ct];
-    }
+      for (int ct = 0; ct < NC; ++ct) x[i][ct] = r.u[i][ct];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       f32x4 add[NC][2];
@@ -732,10 +802,10 @@ template <int DP, bool DELTA, int NC> struct Walk {
     }
     load_second(r, c + 1);
   }
-  // o of the wave's 16 rows; u: those rows of u (linear kinds)
+  // o of the wave's 16 rows; u: those rows of v
   __device__ __forceinline__ void chunk(OutOps& r, int c, f32x4 (&o)[NC], f32x4 (&u)[NC]) const {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const float* sl = sh.sl[DELTA ? 0 : c & 1];
+    const float* sl = sh.sl[c & 1];
     __syncthreads();
     f32x4 os[NC][2], x[4][NC];
 #pragma unroll
@@ -746,23 +816,17 @@ template <int DP, bool DELTA, int NC> struct Walk {
       four<true>(&r.q[kb], x, os);
     }
     load_first(r, c + 1);
-    if constexpr (DELTA) {
-      __syncthreads();
-      read_four<LU>(sh.ul, 0, x);
-    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int ct = 0; ct < NC; ++ct) {
-          x[i][ct] = r.u[i][ct];
-          if (i == wave) u[ct] = r.u[i][ct];
-        }
-    }
+      for (int ct = 0; ct < NC; ++ct) {
+        x[i][ct] = r.u[i][ct];
+        if (i == wave) u[ct] = r.u[i][ct];
+      }
     // (the lower triangle's blocks; the wave's number is the same for all its lanes)
     float odd = 0.f;                               // u of the wave's own rows, which the block on the diagonal meets
 #pragma unroll
-    for (int ct = 0; ct < NC; ++ct)
-      odd = not_finite(DELTA ? at(sh.ul, (16 * ct + lr) * LU + 16 * wave + 4 * kh) : u[ct], odd);
+    for (int ct = 0; ct < NC; ++ct) odd = not_finite(u[ct], odd);
     if (__builtin_expect(__any(odd != 0.f), 0)) {
       f32x4 own, u_own[NC];
 #pragma unroll
@@ -794,13 +858,187 @@ template <int DP, bool DELTA, int NC> struct Walk {
   }
 };
 
+// The delta rule's, its fp32 products as thirds on the 16-bit instructions.  S and u cross through LDS as thirds, split once by
+// the wave that has them; what comes from memory is split where it is used.
+template <int DP, int NC> struct DeltaWalk {
+  static constexpr int KB = DP / 16, KS = DP / 32, NT = DP / 64, LD = DP + 8, LU = C + 8;
+  static constexpr Layout L0 = layout_of(DP, 0, false);
+  struct Shared {
+    __attribute__((aligned(16))) bf16_t sl[3][16 * NC * LD];
+    __attribute__((aligned(16))) bf16_t ul[3][16 * NC * LU];
+  };
+  static __device__ __forceinline__ f32x4 at(const float* p, int offset) { return *reinterpret_cast<const f32x4*>(p + offset); }
+
+  const float* ws;                                 // the pair's first chunk
+  long step;
+  int nc, VP, tile, wave, lane, lr, kh;
+  Shared& sh;
+
+  // (chunks past the last are read as the last one: loads without a condition keep the waits for them exact)
+  __device__ __forceinline__ const float* chunk_at(int c) const { return ws + step * min(c, nc - 1); }
+  __device__ __forceinline__ f32x4 left(const float* p, int offset, int index) const { return at(p, offset + piece(index, lane)); }
+
+  struct StateOps { f32x4 w[KB], k[NT][4], u[NC], b[NT]; };
+  struct OutOps { f32x4 q[KB], a[4]; };
+
+  __device__ __forceinline__ void load_first(StateOps& r, int c) const {
+    const float* p = chunk_at(c);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) r.w[kb] = left(p, L0.u + VP * C, wave * KB + kb);
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) r.u[ct] = left(p, L0.u, (NC * tile + ct) * 4 + wave);
+    __builtin_amdgcn_sched_barrier(0);             // (the loads stay where they are put)
+  }
+  __device__ __forceinline__ void load_second(StateOps& r, int c) const {
+    const float* p = chunk_at(c);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) r.k[t][kb] = left(p, L0.kt, (wave * NT + t) * 4 + kb);
+      r.b[t] = at(p, L0.bc + (wave * NT + t) * 16 + 4 * kh);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void load_first(OutOps& r, int c) const {
+    const float* p = chunk_at(c);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) r.q[kb] = left(p, L0.q, wave * KB + kb);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void load_second(OutOps& r, int c) const {
+    const float* p = chunk_at(c);
+    // (the blocks right of the diagonal are never written: they are read, so that the loads carry no condition, and not used)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) r.a[kb] = left(p, 0, wave * 4 + kb);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // S and u in LDS: a column's rows 32 j + 16 half + 4 kh + e at 32 j + 8 kh + 4 half + e, what a lane takes as one right operand
+  template <int LDR, int N> __device__ __forceinline__ Thirds read_right(const bf16_t (&planes)[3][N], int j, int ct) const {
+    const int o = (16 * ct + lr) * LDR + 32 * j + 8 * kh;
+    return {*reinterpret_cast<const bf16x8*>(planes[0] + o), *reinterpret_cast<const bf16x8*>(planes[1] + o),
+            *reinterpret_cast<const bf16x8*>(planes[2] + o)};
+  }
+  template <int LDR, int N> __device__ __forceinline__ void write_half(bf16_t (&planes)[3][N], int block, int ct, f32x4 v) const {
+    const Thirds t = thirds<false>(v, f32x4{0.f, 0.f, 0.f, 0.f});
+    const int o = (16 * ct + lr) * LDR + 32 * (block >> 1) + 8 * kh + 4 * (block & 1);
+    *reinterpret_cast<bf16x4*>(planes[0] + o) = __builtin_shufflevector(t.h, t.h, 0, 1, 2, 3);
+    *reinterpret_cast<bf16x4*>(planes[1] + o) = __builtin_shufflevector(t.m, t.m, 0, 1, 2, 3);
+    *reinterpret_cast<bf16x4*>(planes[2] + o) = __builtin_shufflevector(t.l, t.l, 0, 1, 2, 3);
+  }
+  // reduction blocks 2 j, 2 j + 1 of a right operand in LDS
+  template <int LDR, int N> __device__ __forceinline__ void read_columns(const bf16_t (&planes)[3][N], int j, Thirds (&x)[NC]) const {
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) x[ct] = read_right<LDR>(planes, j, ct);
+  }
+
+  __device__ __forceinline__ void chunk(StateOps& r, int c, f32x4 (&S)[NT][NC]) const {
+    auto& sl = sh.sl;
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) {
+      if constexpr (NT == 2) {
+        const Thirds t = thirds(S[0][ct], S[1][ct]);
+        const int o = (16 * ct + lr) * LD + 32 * wave + 8 * kh;
+        *reinterpret_cast<bf16x8*>(sl[0] + o) = t.h;
+        *reinterpret_cast<bf16x8*>(sl[1] + o) = t.m;
+        *reinterpret_cast<bf16x8*>(sl[2] + o) = t.l;
+      } else {
+        write_half<LD>(sl, wave, ct, S[0][ct]);
+      }
+    }
+    __syncthreads();
+    Thirds x[NC];
+    Sum us[NC] = {};
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+      read_columns<LD>(sl, j, x);
+      products<false, false>(thirds(r.w[2 * j], r.w[2 * j + 1]), x, us);
+    }
+    f32x4 add_u[NC];
+    values(us, add_u);
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) write_half<LU>(sh.ul, wave, ct, r.u[ct] + add_u[ct]);
+    load_first(r, c + 1);
+    __syncthreads();
+    Sum add[NT * NC] = {};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      read_columns<LU>(sh.ul, j, x);
+      Thirds keys[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) keys[t] = thirds(r.k[t][2 * j], r.k[t][2 * j + 1]);
+      products<false, false>(keys, x, add);
+    }
+    f32x4 by[NT * NC];
+    values(add, by);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) S[t][ct] = S[t][ct] * r.b[t] + by[t * NC + ct];
+    load_second(r, c + 1);
+  }
+  // o of the wave's 16 rows
+  __device__ __forceinline__ void chunk(OutOps& r, int c, f32x4 (&o)[NC], f32x4 (&)[NC]) const {
+    __syncthreads();
+    Sum os[NC] = {};
+    Thirds x[NC];
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+      read_columns<LD>(sh.sl, j, x);
+      products<false, false>(thirds(r.q[2 * j], r.q[2 * j + 1]), x, os);
+    }
+    load_first(r, c + 1);
+    __syncthreads();
+    // (the lower triangle's blocks; the wave's number is the same for all its lanes)
+    float odd = 0.f;                               // u of the wave's own rows, which the block on the diagonal meets
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) {
+      const bf16x4 v = *reinterpret_cast<const bf16x4*>(sh.ul[0] + (16 * ct + lr) * LU + 32 * (wave >> 1) + 8 * kh + 4 * (wave & 1));
+      odd = not_finite(f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}, odd);
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const bool apart = __builtin_expect(__any(odd != 0.f), 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const bool last = j == wave >> 1;
+      if (j > wave >> 1 || (last && apart && !(wave & 1))) continue;
+      const bool both = !last || ((wave & 1) && !apart);
+      read_columns<LU>(sh.ul, j, x);
+      // (a block that is left out is zeros on both sides: a later row's infinity would come through a zero)
+      if (!both)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+          for (int e = 4; e < 8; ++e) x[ct].h[e] = x[ct].m[e] = x[ct].l[e] = (bf16_t)0.f;
+      products<false, false>(thirds(r.a[2 * j], both ? r.a[2 * j + 1] : zero), x, os);
+    }
+    if (apart) {
+      f32x4 own = zero;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) if (i == wave) own = r.a[i];
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int at = (16 * ct + lr) * LU + 32 * (wave >> 1) + 8 * kh + 4 * (wave & 1) + e;
+          const float h = (float)sh.ul[0][at], sum = h + ((float)sh.ul[1][at] + (float)sh.ul[2][at]);
+          v[e] = sum != sum ? h : sum;
+        }
+        os[ct].h += lower16([&](int i, int g, int f) { return __shfl(own[f], g * 16 + i, 64); }, v);
+      }
+    }
+    values(os, o);
+    load_second(r, c + 1);
+  }
+};
+
 template <int DP, bool DELTA, int NC>
 __global__ __launch_bounds__(512, 2) void chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ wsp, long ws_stride,
                                                             float* __restrict__ state, const int* __restrict__ slots,
                                                             const int* __restrict__ qsl, const int* __restrict__ seq_lens,
                                                             const float* __restrict__ d_skip, int B, int H, int dim, int vdim,
                                                             int VP, int h0, int nh, int chunks, float scale) {
-  using W = Walk<DP, DELTA, NC>;
+  using W = std::conditional_t<DELTA, DeltaWalk<DP, NC>, LinearWalk<DP, NC>>;
   __shared__ typename W::Shared shared;
   const int tiles = VP / (16 * NC);
   const int id = blockIdx.x, die = id & 7, rest = id >> 3;
@@ -865,8 +1103,11 @@ int launch(const ChunkArgs& a, int chunks, float* out, float* state, const int* 
   constexpr bool DELTA = KIND >= DELTA_CHANNEL;
   const dim3 prep(chunks, a.nh);
   const long pairs = ((long)a.B * a.nh + 7) / 8 * 8;
-  // 32 columns per workgroup where that still leaves one for every compute unit
-  const int cols = pairs * (a.VP / 32) >= 256 ? 32 : 16;
+  // 32 columns per workgroup where that still leaves one for every compute unit; delta rule, us at 32 and 16 columns: 16 heads of
+  // 128 x 128, 8000 rows of two prompts (128 workgroups of 32) 350 / 284, of three (192) 219 / 242, of five 173 / 223; 64 keys, where two
+  // workgroups of 16 columns fit a compute unit, 32 heads of 128 columns, 4000 rows of two (256) 132 / 113, of four (512) 97 / 99
+  const int enough = !DELTA ? 256 : a.dim > 64 ? 160 : 512;
+  const int cols = pairs * (a.VP / 32) >= enough ? 32 : 16;
   const dim3 walk((unsigned)(pairs * (a.VP / cols)));
 #define WALK(DP_, NC_)                                                                                                       \
   hipLaunchKernelGGL((chunk_walk_kernel<DP_, DELTA, NC_>), walk, dim3(512), 0, stream, out, a.ws, a.ws_stride, state, slots, \

@@ -66,28 +66,6 @@ __device__ __forceinline__ int segments_of(const int* qsl, int s, int rows) {
 // a state in the workspace: [tile of 16 keys][tile of 16 values][lane][4] as the matrix instruction's accumulator, then the decays
 __host__ __device__ constexpr long state_floats(int DP, int VP) { return (long)DP * VP + DP; }
 
-// N values of row r, columns c0 .., into planes by column: two rows' values of a column are one word, the even row's lane writes
-// the even columns and the odd row's, its neighbour, the odd ones
-template <bool UP, int N, int P, int M>
-__device__ __forceinline__ void store_columns(bf16_t (&planes)[P][M], int c0, int r, const Thirds& t) {
-  const bool odd = r & 1;
-  const unsigned pick = odd ? 0x03020706u : 0x05040100u;
-  auto plane = [&](bf16_t* p, bf16x8 v) {
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    const i32x4 w = __builtin_bit_cast(i32x4, v);
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-      const int near = __builtin_amdgcn_update_dpp(0, w[i], 0xB1, 0xf, 0xf, false);        // of the row r ^ 1
-      *reinterpret_cast<unsigned*>(p + (c0 + 2 * i + odd) * LR + (r & ~1)) = __builtin_amdgcn_perm(near, w[i], pick);
-    }
-  };
-  plane(planes[0], t.h);
-  if constexpr (!UP) {
-    plane(planes[1], t.m);
-    plane(planes[2], t.l);
-  }
-}
-
 // Eight waves.  In front of a chunk's products a wave prepares a group of 16 rows and a quarter of the channels and of the value
 // columns, lane (lr, kh) has NV channels of row lr; in the products it has half of the keys and a quarter of the columns, S of them as
 // accumulators, which is at once the right operand of q S.  Three barriers a chunk: the groups' products of decays are there; the
@@ -178,7 +156,8 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
     return v < a.vdim ? (d * a.vdim + v) * 4 : 0x40000000;
   };
   auto kept = [&](float* p, int db, int ct) {      // the same in the workspace
-    return reinterpret_cast<f32x4*>(p + (((long)(dh * DB + db) * (gridDim.z * VW / 16) + blockIdx.z * (VW / 16) + cg * CT + ct) * 64 + lane) * 4);
+    const int tile = blockIdx.z * (VW / 16) + cg * CT + ct;
+    return reinterpret_cast<f32x4*>(p + (((long)(dh * DB + db) * (gridDim.z * VW / 16) + tile) * 64 + lane) * 4);
   };
   fetch(0);
 #pragma unroll
@@ -378,8 +357,8 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
         for (int i = 0; i < NV / 4; ++i) end[i] = k[i] * f;
       }
     }
-    store_columns<false, NV>(kt, ch0, G16 * g + lr, thirds_of<NV / 4, false, false>(end));
-    store_columns<X, NVV>(vv, col0, G16 * g + lr, thirds_of<NVV / 4, X, false>(v));
+    store_columns<LR, false, NV>(kt, ch0, G16 * g + lr, thirds_of<NV / 4, false, false>(end));
+    store_columns<LR, X, NVV>(vv, col0, G16 * g + lr, thirds_of<NVV / 4, X, false>(v));
     __syncthreads();                               // the operands are there
     // ---- A between the groups, over the wave's channels
     if constexpr (OUT)
@@ -629,7 +608,8 @@ VDAMD_API int vdamd_segment_scan(float* out, int kind, const void* x, long x_str
                                  const int* seq_lens, int B, int H, int G, int dim, int vdim, int silu, float scale, int dtype,
                                  hipStream_t stream) {
   if (B <= 0 || segments <= 0) return 0;
-  if (H <= 0 || H > 65535 || (long)H * vdim > (1 << 20) || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || rows < 0 || rows % R || (rows && !ws) ||
+  if (H <= 0 || H > 65535 || (long)H * vdim > (1 << 20) || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || rows < 0 ||
+      rows % R || (rows && !ws) ||
       (!rows && segments != B) || (kind == STATE_SPACE && (!dt || !dt_bias || !a_log)) ||
       (kind != STATE_SPACE && !decay))
     return 1;
