@@ -68,14 +68,43 @@ __device__ __forceinline__ float fast_softplus(float x) {
   return x > 20.f ? x : (dw == 0.f ? t : l);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// v of lane i and of lane i ^ 32, of lane i ^ 16 (in either order), and over a row of 16: halves of it that hold the same numbers.
+// Vector instructions all the way: a shuffle goes through LDS, 60 to 100 cycles where one of these takes 8
+template <typename F> __device__ __forceinline__ float wave_reduce(float v, F&& join) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const unsigned a = __builtin_bit_cast(unsigned, v);
+  const auto far = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  v = join(__builtin_bit_cast(float, (unsigned)far[0]), __builtin_bit_cast(float, (unsigned)far[1]));
+  const unsigned b = __builtin_bit_cast(unsigned, v);
+  const auto near = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  v = join(__builtin_bit_cast(float, (unsigned)near[0]), __builtin_bit_cast(float, (unsigned)near[1]));
+#define ACROSS(CTRL) v = join(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)))
+  ACROSS(0x128);                                  // row_ror:8
+  ACROSS(0x124);                                  // row_ror:4: lane i ^ 4 where lanes i and i ^ 8 hold the same
+  ACROSS(0x4E);                                   // quad_perm [2, 3, 0, 1]
+  ACROSS(0xB1);                                   // quad_perm [1, 0, 3, 2]
+#undef ACROSS
+#endif
   return v;
 }
+// (all 64 lanes run; every lane gets the result, the same bits as from a butterfly of shuffles over 32, 16, 8, 4, 2, 1 lanes)
+__device__ __forceinline__ float wave_sum(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
+// the sum over lanes 0 .. lane (all 64 run), in vector instructions too
+__device__ __forceinline__ int wave_scan(int v) {
+#define FROM(CTRL, ROWS) v += __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false)
+  FROM(0x111, 0xf);                               // row_shr:1, 2, 4, 8
+  FROM(0x112, 0xf);
+  FROM(0x114, 0xf);
+  FROM(0x118, 0xf);
+  FROM(0x142, 0xa);                               // row_bcast:15 into rows 1 and 3
+  FROM(0x143, 0xc);                               // row_bcast:31 into rows 2 and 3
+#undef FROM
   return v;
 }
 
