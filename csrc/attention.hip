@@ -72,10 +72,10 @@ template <typename T> struct Raw8<T, true> { using type = uint2; };
 // ONCE: past the caches (nontemporal), for more than the memory-side cache holds (a smaller cache may still be there from the step
 // before, 16 rows of 4000 keys, 2 heads: 22.1 / 24.0; bytes come a quarter of a line at a time, and are fetched again: 175 / 214)
 template <typename T, bool KV8, bool ONCE = false>
-__device__ __forceinline__ typename Raw8<T, KV8>::type ld_kv(const void* cache, long off) {
+__device__ __forceinline__ typename Raw8<T, KV8>::type ld_kv(const void* cache, long off, unsigned lane = 0) {
   using R = typename Raw8<T, KV8>::type;
   typedef unsigned Words __attribute__((ext_vector_type(sizeof(R) / 4)));
-  const char* p = reinterpret_cast<const char*>(cache) + off * (long)(sizeof(R) / 8);
+  const char* p = reinterpret_cast<const char*>(cache) + off * (long)(sizeof(R) / 8) + lane * (unsigned)(sizeof(R) / 8);
   if constexpr (ONCE) return __builtin_bit_cast(R, __builtin_nontemporal_load(reinterpret_cast<const Words*>(p)));
   else return __builtin_bit_cast(R, *reinterpret_cast<const Words*>(p));
 }
@@ -96,31 +96,65 @@ struct KVFrag {
   typename Raw8<T, KV8>::type kfa[D / 32], kfb[D / 32], vf[D / 16];
 };
 
-template <typename T, int D, bool KV8, bool ONCE = false>
+// K rows and V^T rows of a group.  WHOLE: the group lies in one block (blocks of a power of two of 32 keys or more; a group begins at a
+// multiple of 32): one entry of the table for all lanes, and addresses of a scalar base and 32 bits a lane.  Otherwise each lane
+// looks its rows up.
+template <bool WHOLE, typename T, int D, bool KV8, bool ONCE = false>
+__device__ __forceinline__ void load_k_group(typename Raw8<T, KV8>::type (&kfa)[D / 32], typename Raw8<T, KV8>::type (&kfb)[D / 32],
+                                             const void* __restrict__ k_cache, const int* __restrict__ bt_row, int kvh, int Hkv,
+                                             int block_size, int base, int seq_len) {
+  const int lane = threadIdx.x & 63;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int row = 8 * (r16 >> 2) + (r16 & 3);                 // the two interleaved tiles: row and row + 4
+  if constexpr (WHOLE) {
+    const int at = __builtin_amdgcn_readfirstlane(base), last = seq_len - 1 - at;
+    const long first = ((long)bt_row[at >> (31 - __builtin_clz(block_size))] * Hkv + kvh) * block_size + (at & (block_size - 1));
+    const unsigned ka = min(row, last) * D + 8 * g4, kb = min(row + 4, last) * D + 8 * g4;
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+      kfa[s] = ld_kv<T, KV8, ONCE>(k_cache, first * D + 32 * s, ka);
+      kfb[s] = ld_kv<T, KV8, ONCE>(k_cache, first * D + 32 * s, kb);
+    }
+  } else {
+    const int ka = min(base + row, seq_len - 1), kb = min(base + row + 4, seq_len - 1);
+    const long blk_a = bt_row[ka / block_size], blk_b = bt_row[kb / block_size];
+    const long ka_off = ((blk_a * Hkv + kvh) * block_size + (ka % block_size)) * (long)D + 8 * g4;
+    const long kb_off = ((blk_b * Hkv + kvh) * block_size + (kb % block_size)) * (long)D + 8 * g4;
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+      kfa[s] = ld_kv<T, KV8, ONCE>(k_cache, ka_off + 32 * s);
+      kfb[s] = ld_kv<T, KV8, ONCE>(k_cache, kb_off + 32 * s);
+    }
+  }
+}
+template <bool WHOLE, typename T, int D, bool KV8, bool ONCE = false>
+__device__ __forceinline__ void load_v_group(typename Raw8<T, KV8>::type (&vf)[D / 16], const void* __restrict__ v_cache,
+                                             const int* __restrict__ bt_row, int kvh, int Hkv, int block_size, int base, int seq_len) {
+  const int lane = threadIdx.x & 63;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int slab = block_size * 16;                           // elements of one 16-row slab of a block
+  // this lane's 8 keys are base + 8*g4 .. +7 (one block: block_size % 8 == 0)
+  if constexpr (WHOLE) {
+    const int at = __builtin_amdgcn_readfirstlane(base), last = seq_len - 1 - at;
+    const long first = ((long)bt_row[at >> (31 - __builtin_clz(block_size))] * Hkv + kvh) * block_size * D +
+                       (at & (block_size - 1)) * 16;
+    const unsigned va = (min(8 * g4, last) >> 3) * 128 + 8 * r16;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) vf[dt] = ld_kv<T, KV8, ONCE>(v_cache, first + (long)dt * slab, va);
+  } else {
+    const int vkey = min(base + 8 * g4, seq_len - 1) & ~7;
+    const long blk_v = bt_row[vkey / block_size];
+    const long v_off = (blk_v * Hkv + kvh) * (long)(D / 16) * slab + ((vkey % block_size) >> 3) * 128 + 8 * r16;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) vf[dt] = ld_kv<T, KV8, ONCE>(v_cache, v_off + (long)dt * slab);
+  }
+}
+template <typename T, int D, bool KV8, bool ONCE = false, bool WHOLE = false>
 __device__ __forceinline__ void load_kv_group(KVFrag<T, D, KV8>& f, const void* __restrict__ k_cache,
                                               const void* __restrict__ v_cache, const int* __restrict__ bt_row,
                                               int kvh, int Hkv, int block_size, int base, int seq_len) {
-  const int lane = threadIdx.x & 63;
-  const int r16 = lane & 15, g4 = lane >> 4;
-  // ---- K rows for the two interleaved tiles
-  const int key0 = base + 8 * (r16 >> 2) + (r16 & 3);        // tile 0 row; tile 1 row = key0 + 4
-  const int ka = min(key0, seq_len - 1);
-  const int kb = min(key0 + 4, seq_len - 1);
-  const long blk_a = bt_row[ka / block_size], blk_b = bt_row[kb / block_size];
-  const long ka_off = ((blk_a * Hkv + kvh) * block_size + (ka % block_size)) * (long)D + 8 * g4;
-  const long kb_off = ((blk_b * Hkv + kvh) * block_size + (kb % block_size)) * (long)D + 8 * g4;
-#pragma unroll
-  for (int s = 0; s < D / 32; ++s) {
-    f.kfa[s] = ld_kv<T, KV8, ONCE>(k_cache, ka_off + 32 * s);
-    f.kfb[s] = ld_kv<T, KV8, ONCE>(k_cache, kb_off + 32 * s);
-  }
-  // ---- V^T rows: this lane's 8 keys are base + 8*g4 .. +7 (one block: block_size % 8 == 0)
-  const int vkey = min(base + 8 * g4, seq_len - 1) & ~7;
-  const long blk_v = bt_row[vkey / block_size];
-  const int slab = block_size * 16;                           // elements of one 16-row slab of a block
-  const long v_off = (blk_v * Hkv + kvh) * (long)(D / 16) * slab + ((vkey % block_size) >> 3) * 128 + 8 * r16;
-#pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) f.vf[dt] = ld_kv<T, KV8, ONCE>(v_cache, v_off + (long)dt * slab);
+  load_k_group<WHOLE, T, D, KV8, ONCE>(f.kfa, f.kfb, k_cache, bt_row, kvh, Hkv, block_size, base, seq_len);
+  load_v_group<WHOLE, T, D, KV8, ONCE>(f.vf, v_cache, bt_row, kvh, Hkv, block_size, base, seq_len);
 }
 
 // Score capping (Gemma-2): cap * tanh(score / cap) on the natural-log scale; `s2` and the result are
@@ -134,58 +168,113 @@ __device__ __forceinline__ float soft_cap_log2(float s2, float cap) {
   return t * (cap * 1.4426950408889634f);
 }
 
+// scores of one sub-tile over a group, as this lane's 8 of them ...
+template <typename T, int D, bool KV8>
+__device__ __forceinline__ void group_scores(const typename Raw8<T, KV8>::type (&kfa)[D / 32],
+                                             const typename Raw8<T, KV8>::type (&kfb)[D / 32],
+                                             const typename Vec8<T>::type (&qf)[D / 32], f32x4& s0, f32x4& s1) {
+  s0 = s1 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < D / 32; ++s) {
+    s0 = mfma16(widen<T>(kfa[s]), qf[s], s0);
+    s1 = mfma16(widen<T>(kfb[s]), qf[s], s1);
+  }
+}
+// ... and into its softmax: the probabilities, and the factor of what was summed before.
+// alibi_l2: this lane's query head's ALiBi slope times log2(e) (0: none); the bias of key k for the query at position p is
+// slope * (k - p).  lo: first key inside the sliding window (0 without one)
+template <typename T>
+__device__ __forceinline__ typename Vec8<T>::type group_softmax(f32x4 s0, f32x4 s1, int base, int seq_len, float scale_log2e,
+                                                                float softcap, float& m, float& l, float& alpha, int qpos, int lo,
+                                                                float alibi_l2) {
+  const int g4 = (threadIdx.x & 63) >> 4;
+  const int kidx0 = base + 8 * g4;     // key index of P element j is kidx0 + j
+  const int hi = min(qpos, seq_len - 1);
+  float p[8];
+  float tmax = NEG_BIG;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float sv = (j < 4 ? s0[j & 3] : s1[j & 3]) * scale_log2e;
+    if (softcap > 0.f) sv = soft_cap_log2(sv, softcap);
+    sv = fmaf(alibi_l2, (float)(kidx0 + j - qpos), sv);
+    p[j] = (kidx0 + j <= hi && kidx0 + j >= lo) ? sv : NEG_BIG;
+    tmax = fmaxf(tmax, p[j]);
+  }
+  tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+  tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+  const float m_new = fmaxf(m, tmax);
+  alpha = fast_exp2(m - m_new);
+  float psum = 0.f;
+  typename Vec8<T>::type pf;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    // (a row may have no visible key in a group below its window: its running max is still the
+    // sentinel then, and the masked scores must not turn into exp2(0))
+    const float e = p[j] <= 0.5f * NEG_BIG ? 0.f : fast_exp2(p[j] - m_new);
+    psum += e;
+    pf[j] = (T)e;
+  }
+  l = l * alpha + psum;
+  m = m_new;
+  return pf;
+}
+template <typename T, int D, bool KV8>
+__device__ __forceinline__ void group_values(const typename Raw8<T, KV8>::type (&vf)[D / 16], const typename Vec8<T>::type& pf,
+                                             float alpha, f32x4 (&acc)[D / 16]) {
+#pragma unroll
+  for (int dt = 0; dt < D / 16; ++dt) {
+    acc[dt] *= alpha;
+    acc[dt] = mfma16(widen<T>(vf[dt]), pf, acc[dt]);
+  }
+}
+
 template <typename T, int D, int NQ, bool KV8>
 __device__ __forceinline__ void attend_loaded(
     const KVFrag<T, D, KV8>& f, int base, int seq_len, float scale_log2e, float softcap,
     const typename Vec8<T>::type (&qf)[NQ][D / 32], f32x4 (&acc)[NQ][D / 16], float (&m)[NQ], float (&l)[NQ],
     const int (&qpos_hi)[NQ], const int (&qpos_lo)[NQ], float alibi_l2 = 0.f) {
-  // alibi_l2: this lane's query head's ALiBi slope times log2(e) (0: none); the bias of key k for the
-  // query at position p is slope * (k - p)
-  using V = typename Vec8<T>::type;
-  const int g4 = (threadIdx.x & 63) >> 4;
-  const int kidx0 = base + 8 * g4;     // key index of P element j is kidx0 + j
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s) {
-      s0 = mfma16(widen<T>(f.kfa[s]), qf[n][s], s0);
-      s1 = mfma16(widen<T>(f.kfb[s]), qf[n][s], s1);
-    }
-    const int hi = min(qpos_hi[n], seq_len - 1);
-    const int lo = qpos_lo[n];           // first key inside the sliding window (0 without one)
-    float p[8];
-    float tmax = NEG_BIG;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float sv = (j < 4 ? s0[j & 3] : s1[j & 3]) * scale_log2e;
-      if (softcap > 0.f) sv = soft_cap_log2(sv, softcap);
-      sv = fmaf(alibi_l2, (float)(kidx0 + j - qpos_hi[n]), sv);
-      p[j] = (kidx0 + j <= hi && kidx0 + j >= lo) ? sv : NEG_BIG;
-      tmax = fmaxf(tmax, p[j]);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m[n], tmax);
-    const float alpha = fast_exp2(m[n] - m_new);
-    float psum = 0.f;
-    V pf;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      // (a row may have no visible key in a group below its window: its running max is still the
-      // sentinel then, and the masked scores must not turn into exp2(0))
-      const float e = p[j] <= 0.5f * NEG_BIG ? 0.f : fast_exp2(p[j] - m_new);
-      psum += e;
-      pf[j] = (T)e;
-    }
-    l[n] = l[n] * alpha + psum;
-    m[n] = m_new;
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) {
-      acc[n][dt] *= alpha;
-      acc[n][dt] = mfma16(widen<T>(f.vf[dt]), pf, acc[n][dt]);
-    }
+    f32x4 s0, s1;
+    float alpha;
+    group_scores<T, D, KV8>(f.kfa, f.kfb, qf[n], s0, s1);
+    const auto pf = group_softmax<T>(s0, s1, base, seq_len, scale_log2e, softcap, m[n], l[n], alpha, qpos_hi[n], qpos_lo[n], alibi_l2);
+    group_values<T, D, KV8>(f.vf, pf, alpha, acc[n]);
   }
+}
+
+// Groups g, g + step, .. < g_end of one sub-tile, of blocks that hold whole groups: the next group's keys are on their way while this
+// one's values are multiplied, and its values while its keys are, in the registers that the products have just left.  A whole second
+// group would not fit three waves on a SIMD (202 registers, 3 to 8 % slower than four waves that wait for each group); this takes 152.
+// What bounds it is the memory; before, a wave waited for a group without one of its own under way, after about 130 vector
+// instructions for addresses.  us, before and after: e4m3, 64 rows of about 2000 keys, 8 heads of 128, 67 and 58.8, 200 of 1500 136
+// and 126, 7 of 700 14.9 and 11.5; 16 bits, 250 rows of 800 146 and 140, 2048 of 150 260 and 257, heads of 256, 100 of 500, 83 and 78.
+// With lanes that look up their own rows the loop gains nothing (64 rows of 700 keys in blocks of 16 26.0 and 26.6, e4m3 of 2000 51
+// and 57): those take a group at a time.
+template <typename T, int D, bool KV8, bool ONCE>
+__device__ __forceinline__ void attend_groups(
+    const void* __restrict__ k_cache, const void* __restrict__ v_cache, const int* __restrict__ bt_row, int kvh, int Hkv,
+    int block_size, int g, int step, int g_end, int seq_len, float scale_log2e, float softcap,
+    const typename Vec8<T>::type (&qf)[D / 32], f32x4 (&acc)[D / 16], float& m, float& l, int qpos, int lo, float alibi_l2) {
+  if (g >= g_end) return;
+  KVFrag<T, D, KV8> f;
+  load_kv_group<T, D, KV8, ONCE, true>(f, k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len);
+  f32x4 s0, s1;
+  float alpha;
+  for (; g + step < g_end; g += step) {
+    group_scores<T, D, KV8>(f.kfa, f.kfb, qf, s0, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k_group<true, T, D, KV8, ONCE>(f.kfa, f.kfb, k_cache, bt_row, kvh, Hkv, block_size, (g + step) * 32, seq_len);
+    __builtin_amdgcn_sched_barrier(0);
+    const auto pf = group_softmax<T>(s0, s1, g * 32, seq_len, scale_log2e, softcap, m, l, alpha, qpos, lo, alibi_l2);
+    group_values<T, D, KV8>(f.vf, pf, alpha, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v_group<true, T, D, KV8, ONCE>(f.vf, v_cache, bt_row, kvh, Hkv, block_size, (g + step) * 32, seq_len);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  group_scores<T, D, KV8>(f.kfa, f.kfb, qf, s0, s1);
+  const auto pf = group_softmax<T>(s0, s1, g * 32, seq_len, scale_log2e, softcap, m, l, alpha, qpos, lo, alibi_l2);
+  group_values<T, D, KV8>(f.vf, pf, alpha, acc);
 }
 
 template <typename T, int D, int NQ, bool KV8, bool ONCE = false>
@@ -205,8 +294,8 @@ __device__ __forceinline__ void attend_group(
 // q-tile, sequence); its 4 waves stride over the split's 32-key groups and are
 // merged through LDS.  The 16 MFMA columns carry the GQA group's query heads.
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool KV8, bool ONCE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void paged_decode_kernel(
+template <typename T, int D, bool KV8, bool ONCE, bool WHOLE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WHOLE ? 3 : 4, 4))) void paged_decode_kernel(
     T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, const T* __restrict__ q,
     long q_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ seq_lens, float scale_log2e,
@@ -263,11 +352,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const int* bt_row = block_table + (long)b * bt_stride;
   const float alibi_l2 = (alibi != nullptr && r16 < nq) ? alibi[qh0 + r16] * LOG2E_F : 0.f;
 
-  // no register double-buffering here: it halves the occupancy (202 VGPRs) and
-  // measured 3-8% slower than letting 4 resident workgroups per CU hide the latency
-  if constexpr (KV8 && D <= 64) {
-    // bytes take half the registers: two groups at a time (40 rows of 9000 keys, 8 heads of 64: 112 -> 92 us; of 128 they do not
-    // fit the four waves' registers, 175 -> 290, and with three waves nothing is gained, 170)
+  const float scale = scale_log2e * k_scale;
+  if constexpr (WHOLE) {
+    if (ONCE && past)
+      attend_groups<T, D, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g_begin + wid, 4, g_end, seq_len, scale, softcap,
+                                     qf[0], acc[0], m[0], l[0], qpos_hi[0], qpos_lo[0], alibi_l2);
+    else
+      attend_groups<T, D, KV8, false>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g_begin + wid, 4, g_end, seq_len, scale, softcap,
+                                      qf[0], acc[0], m[0], l[0], qpos_hi[0], qpos_lo[0], alibi_l2);
+  } else if constexpr (KV8 && D <= 64) {
+    // bytes take half the registers: two groups at a time (40 rows of 9000 keys, 8 heads of 64: 112 -> 92 us)
     int g = g_begin + wid;
     for (; g + 4 < g_end; g += 8) {
       KVFrag<T, D, KV8> f[2];
@@ -276,48 +370,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        attend_loaded<T, D, 1, KV8>(f[i], (g + 4 * i) * 32, seq_len, scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo,
-                                    alibi_l2);
+        attend_loaded<T, D, 1, KV8>(f[i], (g + 4 * i) * 32, seq_len, scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
     }
     if (g < g_end)
-      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len,
-                                 scale_log2e * k_scale, softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
+      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale, softcap, qf, acc, m, l,
+                                       qpos_hi, qpos_lo, alibi_l2);
+  } else if (ONCE && past) {
+    for (int g = g_begin + wid; g < g_end; g += 4)
+      attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale, softcap, qf, acc, m, l,
+                                       qpos_hi, qpos_lo, alibi_l2);
   } else {
-    if (ONCE && past) {
-      for (int g = g_begin + wid; g < g_end; g += 4)
-        attend_group<T, D, 1, KV8, ONCE>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale_log2e * k_scale,
-                                         softcap, qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
-    } else {
-      for (int g = g_begin + wid; g < g_end; g += 4)
-        attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale_log2e * k_scale, softcap,
-                                   qf, acc, m, l, qpos_hi, qpos_lo, alibi_l2);
-    }
+    for (int g = g_begin + wid; g < g_end; g += 4)
+      attend_group<T, D, 1, KV8>(k_cache, v_cache, bt_row, kvh, Hkv, block_size, g * 32, seq_len, scale, softcap, qf, acc, m, l,
+                                 qpos_hi, qpos_lo, alibi_l2);
   }
 
   float lsum = l[0];
   lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
   if (g4 == 0) { s_m[wid][r16] = m[0]; s_l[wid][r16] = lsum; }
+  if (r16 < nq) {
 #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt)
-    *reinterpret_cast<f32x4*>(&s_o[wid][r16][16 * dt + 4 * g4]) = acc[0][dt];
+    for (int dt = 0; dt < D / 16; ++dt)
+      *reinterpret_cast<f32x4*>(&s_o[wid][r16][16 * dt + 4 * g4]) = acc[0][dt];
+  }
   __syncthreads();
 
-  for (int e = threadIdx.x; e < 16 * D; e += 256) {
-    const int qi = e / D, d = e - qi * D;
-    if (qi >= nq) continue;
+  for (int e = threadIdx.x; e < nq * (D / 4); e += 256) {
+    const int qi = e / (D / 4), d = 4 * (e - qi * (D / 4));
     const float m0 = s_m[0][qi], m1 = s_m[1][qi], m2 = s_m[2][qi], m3 = s_m[3][qi];
     const float mm = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));
     const float a0 = fast_exp2(m0 - mm), a1 = fast_exp2(m1 - mm), a2 = fast_exp2(m2 - mm), a3 = fast_exp2(m3 - mm);
-    const float o = (s_o[0][qi][d] * a0 + s_o[1][qi][d] * a1 + s_o[2][qi][d] * a2 + s_o[3][qi][d] * a3) * v_scale;
+    const auto part = [&](int w) { return *reinterpret_cast<const f32x4*>(&s_o[w][qi][d]); };
+    const f32x4 o = (part(0) * a0 + part(1) * a1 + part(2) * a2 + part(3) * a3) * v_scale;
     float lt = s_l[0][qi] * a0 + s_l[1][qi] * a1 + s_l[2][qi] * a2 + s_l[3][qi] * a3;
     const int qh = qh0 + qi;
     if (num_splits == 1) {
       if (sinks != nullptr) lt += fast_exp2(sinks[qh] * LOG2E_F - mm);       // (with splits: added by the merge kernel)
-      out[b * out_stride + (long)qh * D + d] = (T)(lt > 0.f ? o / lt : 0.f);
+      typename Vec4<T>::type o4;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o4[r] = (T)(lt > 0.f ? o[r] / lt : 0.f);
+      __builtin_memcpy(out + b * out_stride + (long)qh * D + d, &o4, sizeof(o4));       // (`out` is aligned to its elements only)
     } else {
       const long pidx = ((long)b * Hq + qh) * num_splits + split;
-      part_o[pidx * D + d] = o;
+      __builtin_memcpy(part_o + pidx * D + d, &o, sizeof(o));
       if (d == 0) { part_ml[2 * pidx] = mm; part_ml[2 * pidx + 1] = lt; }
     }
   }
@@ -581,7 +677,9 @@ int launch_decode(void* out, float* ws, const void* q, long q_stride, const void
     HIP_LAUNCH_CHECK();
     return 0;
   }
-  hipLaunchKernelGGL((paged_decode_kernel<T, D, KV8, ONCE>), dim3(num_splits, Hkv * q_tiles, B), dim3(256), 0, s, (T*)out,
+  const bool whole = block_size >= 32 && (block_size & (block_size - 1)) == 0;         // no group of 32 keys spans two blocks
+  hipLaunchKernelGGL((whole ? paged_decode_kernel<T, D, KV8, ONCE, true> : paged_decode_kernel<T, D, KV8, ONCE, false>),
+                      dim3(num_splits, Hkv * q_tiles, B), dim3(256), 0, s, (T*)out,
                      part_o, part_ml, (const T*)q, q_stride, kc, vc, bt, bt_stride, seq_lens,
                      sl2, Hq, Hkv, block_size, num_splits, out_stride, k_scales, v_scales, window, softcap, sinks,
                      alibi, past_bytes);

@@ -201,6 +201,34 @@ def test_paged_attention_decode(hq, hkv, d, bs, splits):
     torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("hq,hkv,d", [(8, 1, 128), (34, 2, 64), (4, 4, 96), (6, 2, 256)])
+@pytest.mark.parametrize("splits,window", [(1, 0), (3, 0), (1, 40), (2, 129)])
+def test_paged_attention_decode_is_the_same_for_every_block_size(hq, hkv, d, splits, window, kv8):
+    """Blocks of 16, 24 and 48 keys are looked up lane by lane, of 32, 64 and 256 once for a group of 32: the same sums in the same
+    order, so equal to the bit.  Contexts end at both sides of groups and blocks, in a wave's first, last and missing group."""
+    from vllm_distributed_amd.ops import hip
+    lens = [1, 7, 8, 31, 32, 33, 64, 65, 127, 128, 129, 255, 257, 300]
+    dtype = torch.float8_e4m3fn if kv8 else torch.bfloat16
+    k, v = _rand(len(lens), max(lens), hkv, d), _rand(len(lens), max(lens), hkv, d)
+    sl = torch.tensor(lens, device=DEV, dtype=torch.int32)
+    q = _rand(len(lens), hq, d)
+    got = {}
+    for bs in (16, 24, 48, 32, 64, 256):
+        per = -(-max(lens) // bs)
+        bt = torch.randperm(len(lens) * per, device=DEV).to(torch.int32).view(len(lens), per)
+        kc = torch.zeros(len(lens) * per, hkv, bs, d, device=DEV, dtype=dtype)
+        vc = torch.zeros(len(lens) * per, hkv, d // 16, bs // 8, 16, 8, device=DEV, dtype=dtype)
+        for i, n in enumerate(lens):
+            pos = torch.arange(n, device=DEV)
+            ops.reshape_and_cache(k[i, :n], v[i, :n], kc, vc, (bt[i].long()[pos // bs] * bs + pos % bs).to(torch.int32))
+        got[bs] = hip.paged_attention_decode(q, kc, vc, bt, sl, d ** -0.5, max_seq_len=max(lens), num_splits=splits, window=window)
+    ref = torch_ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl, d ** -0.5, window=window)
+    torch.testing.assert_close(got[16].float(), ref, rtol=2e-2, atol=2e-2)
+    for bs in got:
+        assert torch.equal(got[bs], got[16]), bs
+
+
 def test_paged_attention_decode_strided_q_and_padding_rows():
     from vllm_distributed_amd.ops import hip
     hq, hkv, d, bs = 32, 8, 128, 64
