@@ -108,6 +108,22 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
+// (doubles: both halves of a number move, and lanes without a source add zero)
+__device__ __forceinline__ double wave_scan(double v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#define FROM(CTRL, ROWS)                                                                                                  \
+  {                                                                                                                       \
+    const unsigned long long bits = __builtin_bit_cast(unsigned long long, v);                                            \
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)bits, CTRL, ROWS, 0xf, false);                      \
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(bits >> 32), CTRL, ROWS, 0xf, false);              \
+    v += __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);                                                   \
+  }
+  FROM(0x111, 0xf) FROM(0x112, 0xf) FROM(0x114, 0xf) FROM(0x118, 0xf) FROM(0x142, 0xa) FROM(0x143, 0xc)
+#undef FROM
+#endif
+  return v;
+}
+
 // block-wide sum over up to 16 waves; every thread gets the result.
 // `red` must hold >= 17 floats of LDS.
 __device__ __forceinline__ float block_sum(float v, float* red) {

@@ -123,17 +123,12 @@ struct SampleShared {
   int best, n, token, bad;
 };
 
-// exclusive scan of (count, mass) over the block in thread order; totals to every thread
+// exclusive scan of (count, mass) over the block in thread order; totals to every thread (by shuffles, which go through LDS, a row's
+// two scans of sample_by_counts took 2.5 us more)
 __device__ __forceinline__ void block_scan(unsigned c, double m, unsigned& ec, double& em, double& total, SampleShared& s) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  unsigned ic = c;
-  double im = m;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned oc = __shfl_up(ic, o, 64);
-    const double om = __shfl_up(im, o, 64);
-    if (lane >= o) { ic += oc; im += om; }
-  }
+  const unsigned ic = (unsigned)wave_scan((int)c);
+  const double im = wave_scan(m);
   if (lane == 63) { s.wcnt[wid] = ic; s.wmass[wid] = im; }
   __syncthreads();
   unsigned bc = 0;
@@ -148,44 +143,51 @@ __device__ __forceinline__ void block_scan(unsigned c, double m, unsigned& ec, d
   __syncthreads();
 }
 
-// The lowest non-empty bin (at or above `first`) in front of which fewer than K elements and less than M of mass lie:
-// its index, count and what lies above it go to `s` (best = -1: none).  Bins hold the bits `prefix | bin << shift ..`.
-template <bool WIDE>
-__device__ void scan_bins(const Hist<WIDE>& h, unsigned prefix, int shift, int first, unsigned above_cnt, double above_mass,
-                          unsigned K, double M, SampleShared& s) {
-  unsigned c[2];
-  double m[2];
+// A histogram's two bins of each thread, the heaviest of all first: counts, masses, and what lies in front of them.  Bins hold the
+// bits `prefix | bin << shift ..`.
+struct Bins {
+  unsigned c[2], ec;
+  double m[2], em, total;
+};
+template <bool WIDE> __device__ __forceinline__ Bins sum_bins(const Hist<WIDE>& h, unsigned prefix, int shift, SampleShared& s) {
+  Bins t;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int bin = BINS - 1 - (2 * (int)threadIdx.x + e);
     const unsigned bits = prefix | ((unsigned)bin << shift);
-    c[e] = h.count(bin);
-    m[e] = c[e] ? ((double)c[e] * sig_of(bits) + (double)h.lows(bin)) * pow2(lsb_of(bits)) : 0.0;
+    t.c[e] = h.count(bin);
+    t.m[e] = t.c[e] ? ((double)t.c[e] * sig_of(bits) + (double)h.lows(bin)) * pow2(lsb_of(bits)) : 0.0;
   }
-  unsigned ec;
-  double em, total;
+  block_scan(t.c[0] + t.c[1], t.m[0] + t.m[1], t.ec, t.em, t.total, s);
+  return t;
+}
+// The lowest non-empty bin (at or above `first`) in front of which, `above` included, fewer than K elements and less than M of mass
+// lie: its index, count and what lies above it go to `s` (best = -1: none).
+__device__ __forceinline__ void find_bin(const Bins& t, int first, unsigned above_cnt, double above_mass, unsigned K, double M,
+                                         SampleShared& s) {
   if (threadIdx.x == 0) s.best = -1;
-  block_scan(c[0] + c[1], m[0] + m[1], ec, em, total, s);
-  ec += above_cnt;
-  em += above_mass;
+  __syncthreads();
+  const unsigned ec = t.ec + above_cnt;
+  const double em = t.em + above_mass;
   int mine = -1;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int order = 2 * (int)threadIdx.x + e;
-    if (c[e] && BINS - 1 - order >= first && ec + (e ? c[0] : 0) < K && em + (e ? m[0] : 0.0) < M) mine = order;
+    if (t.c[e] && BINS - 1 - order >= first && ec + (e ? t.c[0] : 0) < K && em + (e ? t.m[0] : 0.0) < M) mine = order;
   }
-  if (mine >= 0) atomicMax(&s.best, mine);
+  // (orders rise with the lanes: a wave's last one speaks for it)
+  const unsigned long long those = __ballot(mine >= 0);
+  if (mine >= 0 && (those >> (threadIdx.x & 63)) == 1ull) atomicMax(&s.best, mine);
   __syncthreads();
   const int best = s.best;
   __syncthreads();
   if (best >= 0 && best >> 1 == (int)threadIdx.x) {
     const bool second = best & 1;
-    s.above_cnt = ec + (second ? c[0] : 0);
-    s.above_mass = em + (second ? m[0] : 0.0);
-    s.cnt = second ? c[1] : c[0];
+    s.above_cnt = ec + (second ? t.c[0] : 0);
+    s.above_mass = em + (second ? t.m[0] : 0.0);
+    s.cnt = second ? t.c[1] : t.c[0];
     s.best = BINS - 1 - best;
   }
-  if (threadIdx.x == 0) s.mass = total;
   __syncthreads();
 }
 
@@ -276,9 +278,9 @@ template <typename T, typename F, typename G> __device__ __forceinline__ void fo
 // lies in is looked at again.  Masses are counts times weights, in doubles: no result depends on the order of additions.
 // Bound by the LDS atomics and the vector instructions of the counting pass (10 us of a row of 128256 alone, 16 of 256 rows at
 // once, whose logits take 14 from memory), by the second pass (6 and 9) and by a dozen steps of a microsecond or two between
-// them.  256 rows of 128256 bf16 logits, every kind of filter among them: 41 us, by bins 118; one row 30 (62), one of 32000 19
-// (37).  The patterns are packed by stretches of 512 places a wave: with 64 places a thread the few threads that have any
-// were 7 us on their own (3.2 so).
+// them.  256 rows of 128256 bf16 logits, every kind of filter among them: 38 us, by bins 118 when this was chosen (93 now); one row
+// 29 (62, 53), one of 32000 18 (37, 25).  The patterns are packed by stretches of 512 places a wave: with 64 places a thread the few
+// threads that have any were 7 us on their own (3.2 so).
 // -1: a pattern occurs 65536 times or more (a count ran over: the counts' sum is then too small), more than 32768 patterns
 // occur, or the row is longer than the second pass has counters for.  The type's lowest value and the infinity next to it, which
 // masks fill rows with, are counted apart, in registers.
@@ -368,9 +370,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
     }
     __syncthreads();
     const unsigned even = cs.of_stretch[2 * lane], odd = cs.of_stretch[2 * lane + 1];
-    unsigned upto = even + odd;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { const unsigned x = __shfl_up(upto, o, 64); if (lane >= o) upto += x; }
+    const unsigned upto = (unsigned)wave_scan((int)(even + odd));
     n = __shfl(upto, 63, 64);
     if (cs.counted != (unsigned)V - cs.low - cs.inf && !s.bad) return -1;
     if (n > PATTERNS / 2) return -1;
@@ -441,7 +441,8 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         in_front += c;
         above += c * mass_of(w);
       }
-    if (best >= 0) atomicMax(&s.best, best);
+    // (entries rise with the lanes: a wave's last one speaks for it)
+    if (best >= 0 && (__ballot(best >= 0) >> lane) == 1ull) atomicMax(&s.best, best);
     __syncthreads();
     if (best >= 0 && s.best == best) {
       const double v = mass_of(best_w);
@@ -549,9 +550,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         hits |= (unsigned)hit(v[w] & 0xffffu) << (2 * w) | (unsigned)hit(v[w] >> 16) << (2 * w + 1);
       if (!live) hits = 0;
       const unsigned c = __popc(hits);
-      unsigned upto = c;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) { const unsigned x = __shfl_up(upto, o, 64); if (lane >= o) upto += x; }
+      const unsigned upto = (unsigned)wave_scan((int)c);
       if (upto - c < want && want <= upto) {
         want -= upto - c;
         for (int e = 0; e < 8; ++e)

@@ -664,6 +664,29 @@ def test_sample_cuts_bins_of_many_entries_where_the_filter_does(dtype):
         assert draw(row, 5001, 0.5)[0] == V - 1
 
 
+@pytest.mark.parametrize("equal", [False, True])
+@pytest.mark.parametrize("n", [63, 64, 65, 300, 2048, 2049, 4096])
+def test_sample_finds_the_border_inside_one_bin(n, equal):
+    """``n`` entries of one histogram bin, all alike or 1e-2 / n apart: sorted as they are up to 64 and where more than 2048 agree in
+    the next bits too, cut by those bits between.  Kept by count, drawn at the middle of an entry's stretch of the mass: half an
+    entry is 1e-4 of it or more, a weight is off by 1e-5 of itself at most."""
+    V = 9000
+    order = torch.randperm(V - 2, device=DEV)[:n]
+    if equal:
+        order = order.sort().values
+    w = torch.linspace(0.61, 0.61 if equal else 0.60, n, device=DEV, dtype=torch.float64)         # (19/32 .. 20/32: one bin)
+    row = torch.full((V,), -40.0, device=DEV)
+    row[order], row[V - 1] = torch.log(w).float(), 0.0
+    cum = torch.cat([torch.ones(1, device=DEV, dtype=torch.float64), w]).cumsum(0)
+    ranks = sorted({1, 2, n // 2, n - 1, n})
+    for kept in (n, n // 2, 2):
+        at = [r for r in ranks if r <= kept]
+        u = torch.stack([(cum[r] - 0.5 * w[r - 1]) / cum[kept] for r in at]).float()
+        full = lambda v, t=torch.float32: torch.full((len(at),), v, device=DEV, dtype=t)
+        got = ops.sample(row.expand(len(at), -1).contiguous(), full(1.0), full(kept + 1, torch.int32), full(1.0), full(0.0), u)
+        assert got.tolist() == [order[r - 1].item() for r in at], kept
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("V,offset", [(1, 0), (7, 3), (511, 1), (519, 0), (8192, 0), (50257, 1), (128256, 0), (151936, 5), ((1 << 23) + 9, 0)])
 def test_sample_of_counted_patterns_is_the_one_of_the_same_values_in_32_bits(V, offset, dtype):
