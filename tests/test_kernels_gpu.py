@@ -1566,6 +1566,48 @@ def test_latent_attention_decode_prefill_and_cache_write(dk, dv, hq, bs, dtype, 
         torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("dk,dv,hq", [(576, 512, 16), (576, 512, 128), (320, 256, 70)])
+@pytest.mark.parametrize("what", ["plain", "window", "precise"])
+def test_latent_attention_of_prompts_and_many_heads_reads_key_rows(dk, dv, hq, what):
+    """Steps whose rows name their sequence, and decoded rows of enough heads for four tiles, go over the key rows alone where they can
+    be read so: against 64-bit sums, no further from them than the kernel that shares keys between four tiles is (which rounds
+    the same weights to 16 bits; 1.2 for the different order of the sums), sinks and gates as well."""
+    from vllm_distributed_amd.ops import hip as _hip
+    torch.manual_seed(hq)
+    bs, lens = 64, [1, 33, 64, 95, 130, 700]
+    per = -(-max(lens) // bs)
+    table = (torch.randperm(len(lens) * per, device=DEV) + 1).to(torch.int32).view(len(lens), per)
+    nblk = len(lens) * per + 1
+    kc = torch.zeros(torch_ref.k_cache_shape(nblk, 1, dk, bs), dtype=torch.bfloat16, device=DEV)
+    vc = torch.zeros(torch_ref.v_cache_shape(nblk, 1, dv, bs), dtype=torch.bfloat16, device=DEV)
+    _hip.mla_cache_write(_rand(nblk * bs, dk), kc, vc, torch.arange(nblk * bs, dtype=torch.int32, device=DEV))
+    sinks = torch.randn(hq, device=DEV)
+    extra = {"window": 40 if what == "window" else 0, "precise": what == "precise", "sinks": sinks}
+    # every token of the last 37 of a sequence, in steps that begin at any position; then one row a sequence
+    seq = [b for b, n in enumerate(lens) for _ in range(min(n, 37))]
+    seen = [n - min(n, 37) + 1 + i for n in lens for i in range(min(n, 37))]
+    for rows, keys in ((torch.tensor(seq, dtype=torch.int32, device=DEV), seen), (None, lens * 5)):
+        bt = table if rows is not None else table.repeat(5, 1)
+        sl = torch.tensor(keys, dtype=torch.int32, device=DEV)
+        q = _rand(len(keys), hq, dk)
+        gate = _rand(len(keys), hq)
+        want = torch.zeros(len(keys), hq, dv, dtype=torch.float64, device=DEV)
+        for t, n in enumerate(keys):
+            b = seq[t] if rows is not None else t % len(lens)
+            lo = max(n - 40, 0) if what == "window" else 0
+            k = kc[table[b].long(), 0].reshape(-1, dk)[lo:n].double()
+            s = torch.cat([q[t].double() @ k.T * 0.08, sinks.double().unsqueeze(1)], 1).softmax(-1)[:, :-1]
+            want[t] = s @ k[:, :dv] * gate[t].double().sigmoid().unsqueeze(1)
+        run = lambda mode, splits=None: _hip.mla_attention(q, kc, vc, bt, rows, sl, 0.08, max(lens), mode=mode, splits=splits,
+                                                           gate=gate, **extra)
+        got = run(None)
+        assert torch.equal(got, run(3))
+        err = lambda o: ((o.double() - want).norm() / want.norm()).item()
+        bound = 1.2 * err(run(1 if rows is not None else 2))
+        for splits in (None, 1, 3):
+            assert err(run(None, splits)) <= bound < 2 ** -7
+
+
 @pytest.mark.parametrize("e,k,n_group,topk_group,v3,renorm", [
     (256, 8, 8, 4, True, True), (256, 8, 1, 1, True, True), (160, 6, 8, 3, False, False), (64, 6, 1, 1, False, False),
     (64, 6, 1, 1, False, True), (8, 2, 4, 2, True, True), (128, 1, 1, 1, True, True), (72, 4, 8, 8, False, True)])

@@ -1320,8 +1320,9 @@ def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int, workgroups: int 
 
 def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows_ok: bool, mode: Optional[int] = None,
              captured: bool = True) -> Tuple[int, int]:
-    """Kernel (``mla_attention``'s ``mode``, chosen here when None) and KV splits of a step of ``tokens`` rows of up to ``keys``
-    keys from ``seqs`` sequences (``by_token``: rows name theirs), ``captured`` in a graph or launched from Python.
+    """Kernel (``mla_attention``'s ``mode``, chosen here when None; who can always read key rows passes 3) and KV splits of a step of
+    ``tokens`` rows of up to ``keys`` keys from ``seqs`` sequences (``by_token``: rows name theirs), ``captured`` in a graph or
+    launched from Python.
 
     Splits make as many workgroups as run at once - one per CU of the kernels that share keys between four tiles (1, 2), two of
     the one over key rows (3) - and not more: what is left over waits for a second round.  Prompt of 200 tokens, 16 heads, 700 keys
@@ -1368,8 +1369,8 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     (steps with ``token_seq``: prefill chunks, verification - the tokens of a sequence must be adjacent rows at
     consecutive positions); 2 = four head tiles of a token per workgroup (64 heads per rank and more); 3 = as 0,
     the values read from the key rows (their first ``DV`` values, which is what every writer puts into both caches):
-    half the bytes, 1.1 to 2.5 times as fast from one sequence of 100 keys to 256 of 1500, at every width and head
-    count measured, so 0 is left with what 3 does not read (``mla_rows_ok``).
+    half the bytes, 1.1 to 4.6 times as fast from one sequence of 32 keys to 256 of 1500 and prompts of 5000, at every width and
+    head count measured, so the others are left with what 3 does not read (``mla_rows_ok``).
     ``precise``: the softmax weights enter the PV product with fp32 precision (a high and a low 16-bit part).
     ``window`` > 0: only the last ``window`` of those keys; ``sinks[Hq]`` (fp32): ``exp(sinks[h])`` joins head ``h``'s
     softmax denominator; ``gate[T, Hq]`` (raw, rows may be strided): the output times its sigmoid."""
@@ -1389,7 +1390,16 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         assert gate.dim() == 2 and gate.shape[0] >= t and gate.shape[1] == hq and gate.stride(1) == 1 and gate.dtype == q.dtype
         gate_stride = gate.stride(0)
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
-    mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
+    rows_ok = mla_rows_ok(k_cache, dv)
+    if mode is None and rows_ok:
+        # It reads a row once per token and 16 heads, but out of the caches and by DMA; the two that share keys between four tiles
+        # read both caches into registers, 70 KB per 5 us a workgroup.  us, shared / rows: prompt tokens of 16 heads, 2611 of three
+        # sequences 377 / 232, 1834 of one 419 / 236, 85 behind 330 34 / 21, four each of 64 sequences of 4000 keys 664 / 182, of 16
+        # of 1000 57 / 23; of 128 heads, 880 of three 902 / 584, 76 77 / 31, 565 of 5000 keys 3647 / 2255; decoded rows of 128
+        # heads, 69 of 780 keys 167 / 101, 20 of 3000 124 / 101, 128 of 600 139 / 112; of 64, 100 of 800 104 / 68, 256 of 1500
+        # 346 / 288.
+        mode = 3
+    mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], rows_ok, mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
     # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
     past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
