@@ -16,11 +16,20 @@ __device__ __forceinline__ float softplus_f(float x) {
   return x > 20.f ? x : l;
 }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-// e^x for x above -200 (below: as there, zero).  The library's function less its compares and selects
+// e^x for x up to zero (below -200 as there: zero).  Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980):
+// x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact, and for |r| <= ln 2 / 2 a polynomial whose
+// coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits, root mean square / largest, x in -10 .. 0:
+// 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
 __device__ __forceinline__ float exp_f(float x) {
   x = x < -200.f ? -200.f : x;
-  const float n = rintf(x * 1.44269502f);
-  return ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -n))), (int)n);
+  const float n = rintf(x * 1.44269504f);
+  const float r = fmaf(-n, 1.42860677e-6f, fmaf(-n, 0.693145752f, x));
+  float p = fmaf(r, 0.0013814529f, 0.008368751f);
+  p = fmaf(r, p, 0.041668393f);
+  p = fmaf(r, p, 0.1666652f);
+  p = fmaf(r, p, 0.49999994f);
+  p = fmaf(r, p, 1.f);
+  return ldexpf(fmaf(r, p, 1.f), (int)n);
 }
 // e^(-rate softplus(x)).  softplus(x) is softplus(-|x|) more than x where x > 0, and ln(1 + t) = 2 atanh(t / (2 + t)), whose series
 // converges for t <= 1 (arguments up to 1 / 3; the coefficients are those of a fit by Chebyshev polynomials, off by 1e-9).  A fifth
