@@ -44,16 +44,20 @@ __device__ __forceinline__ float decay_f(float x, float rate) {
   const float l = fmaf(2.f * s, z * p, 2.f * s);
   return exp_f(-rate * ((x > 0.f ? x : 0.f) + l));
 }
-// x sigmoid(x), within two units of the last place: the exponent's product with what it was rounded by, and the reciprocal with a
-// step of Newton's, are a third of the library's instructions (whose scaling and fix-up have nothing to do here)
+// a / d, as the correctly rounded quotient for d between 2^-96 and 2^96 and results that are no denormals: the product with the
+// reciprocal, and what is left over once more.  (The maximum drops a remainder that is no number: infinities stay what they are.)
+// Three quarters of the instructions of the library's division, which scales its operands first
+__device__ __forceinline__ float quotient(float a, float d, float left_out = 0.f) {
+  const float r = __builtin_amdgcn_rcpf(d), q = a * r;
+  return fmaf(fmaxf(fmaf(-left_out, q, fmaf(-d, q, a)), -3.40282347e38f), r, q);
+}
+// x sigmoid(x) = x / (1 + t), t = e^-|x|, or x t / (1 + t) below zero, with what 1 + t lost to rounding in the remainder.  No clamp of
+// the exponent: below -88, where 1 + e^-x is beyond 32 bits, it goes to zero as the function does.  Error against 64 bits, root mean
+// square, and of the product with the library's sigmoid: x in -8 .. 8 3.5e-8 and 4.5e-8, -60 .. -20 3.7e-8 and 4.4e-8, 8 .. 60 1.2e-8
+// and 1.8e-8
 __device__ __forceinline__ float silu_f(float x) {
-  const float t = fmaxf(x * -1.44269502f, -126.f), u = fminf(t, 126.f);
-  const float lo = fmaf(x, -1.44269502f, -u) + x * -1.92596303e-8f;            // (u is the product's rounded value where it counts)
-  float e = __builtin_amdgcn_exp2f(u);
-  e = fmaf(e, fabsf(t) < 126.f ? lo * 0.693147182f : 0.f, e) + 1.f;
-  float r = __builtin_amdgcn_rcpf(e);
-  r = fmaf(fmaf(-e, r, 1.f), r, r);
-  return x * r;
+  const float t = exp_f(-fabsf(x)), d = 1.f + t;
+  return quotient(x < 0.f ? x * t : x, d, t - (d - 1.f));
 }
 
 // A 32-bit value as the exact sum of three of 16 bits, 8 digits each.  Of the nine products of two such sums the six largest are

@@ -306,3 +306,24 @@ def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch,
         beside[5] = False
         there = slice(row, 150)
         assert _off(got[there].view(-1, heads, vdim)[:, :, beside], clean[there].view(-1, heads, vdim)[:, :, beside].double()) < 3e-6
+
+
+@pytest.mark.parametrize("rows", [-1, 0, 32])                                  # the chunked kernels; segments, whole and cut
+def test_activated_inputs_far_below_zero_go_to_zero(monkeypatch, rows):
+    """SiLU of what its exponential overflows for.  One row's key and query have one entry, and its value is read out again: a
+    product of three activations, each within 2e-7 of 64 bits, and zero (to denormals) where they are."""
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    heads, dim, new = 1, 64, [48, 48]
+    x = torch.zeros(96, 3 * dim, device=DEV)
+    entries = torch.tensor([-0.5, -20.0, -80.0, -87.0, -88.0, -90.0, -100.0, -200.0, -1e4, -1e30, -3e38, 3e37], device=DEV)
+    x[5, 0], x[5, dim] = 1.5, 2.5
+    x[5, 2 * dim:2 * dim + len(entries)] = entries
+    c = {"op": "linear_head", "heads": heads, "groups": heads, "dim": dim, "vdim": dim, "new": new, "lens": new, "x": x,
+         "state": torch.zeros(2, heads, dim, dim, device=DEV), "slots": torch.tensor([1, 0], dtype=torch.int32, device=DEV),
+         "decay": torch.full((heads,), 0.5, device=DEV), "beta": torch.zeros(96, heads, device=DEV)}
+    want, want_state = _rows64(c)
+    out, state = _run(c, True)
+    got, ref = out[5].double(), want[5]
+    assert torch.isfinite(out).all() and torch.isfinite(state).all()
+    assert ((got - ref).abs() <= 8e-7 * ref.abs() + 1e-36).all(), (got[:len(entries)].tolist(), ref[:len(entries)].tolist())
+    assert float((state.double() - want_state).abs().max()) <= 8e-7 * float(want_state.abs().max())
