@@ -16,7 +16,7 @@ __device__ __forceinline__ float softplus_f(float x) {
   return x > 20.f ? x : l;
 }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-// e^x for x up to zero (below -200 as there: zero).  Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980):
+// e^x for x from -200, where it is zero, up to zero.  Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980):
 // x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact, and for |r| <= ln 2 / 2 a polynomial whose
 // coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits, root mean square / largest, x in -10 .. 0:
 // 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
@@ -44,20 +44,16 @@ __device__ __forceinline__ float decay_f(float x, float rate) {
   const float l = fmaf(2.f * s, z * p, 2.f * s);
   return exp_f(-rate * ((x > 0.f ? x : 0.f) + l));
 }
-// a / d, as the correctly rounded quotient for d between 2^-96 and 2^96 and results that are no denormals: the product with the
-// reciprocal, and what is left over once more.  (The maximum drops a remainder that is no number: infinities stay what they are.)
-// Three quarters of the instructions of the library's division, which scales its operands first
-__device__ __forceinline__ float quotient(float a, float d, float left_out = 0.f) {
-  const float r = __builtin_amdgcn_rcpf(d), q = a * r;
-  return fmaf(fmaxf(fmaf(-left_out, q, fmaf(-d, q, a)), -3.40282347e38f), r, q);
-}
-// x sigmoid(x) = x / (1 + t), t = e^-|x|, or x t / (1 + t) below zero, with what 1 + t lost to rounding in the remainder.  No clamp of
-// the exponent: below -88, where 1 + e^-x is beyond 32 bits, it goes to zero as the function does.  Error against 64 bits, root mean
-// square, and of the product with the library's sigmoid: x in -8 .. 8 3.5e-8 and 4.5e-8, -60 .. -20 3.7e-8 and 4.4e-8, 8 .. 60 1.2e-8
-// and 1.8e-8
+// x sigmoid(x), where sigmoid(x) = 1 / (1 + t), or t / (1 + t) below zero, with t = e^-|x|: that reduction in base two, -|x| log2(e) =
+// n + f with log2(e) in two pieces, and the instruction's 2^f.  No exponent is cut off but where t is zero, so that far below zero the
+// result goes to zero as the function does.  The quotient is the product with the reciprocal and what that leaves over, with what
+// 1 + t lost to rounding.  Error against 64 bits, root mean square, and of the product with the library's sigmoid: x in -8 .. 8 3.8e-8
+// and 4.5e-8, -20 .. -8 4.4e-8 and 4.6e-8, -60 .. -20 3.7e-8 and 4.4e-8, 8 .. 60 1.5e-8 and 1.8e-8
 __device__ __forceinline__ float silu_f(float x) {
-  const float t = exp_f(-fabsf(x)), d = 1.f + t;
-  return quotient(x < 0.f ? x * t : x, d, t - (d - 1.f));
+  const float y = __builtin_amdgcn_fmed3f(-fabsf(x), -200.f, 0.f), n = rintf(y * 1.44269502f);
+  const float t = ldexpf(__builtin_amdgcn_exp2f(fmaf(y, 1.92596303e-8f, fmaf(y, 1.44269502f, -n))), (int)n);
+  const float d = 1.f + t, left_out = t - (d - 1.f), a = x < 0.f ? t : 1.f, r = __builtin_amdgcn_rcpf(d), s = a * r;
+  return x * fmaf(fmaf(-left_out, s, fmaf(-d, s, a)), r, s);
 }
 
 // A 32-bit value as the exact sum of three of 16 bits, 8 digits each.  Of the nine products of two such sums the six largest are
