@@ -16,14 +16,15 @@ __device__ __forceinline__ float softplus_f(float x) {
   return x > 20.f ? x : l;
 }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-// e^x for x from -200, where it is zero, up to zero.  Cody and Waite's reduction (Software Manual for the Elementary Functions, 1980):
-// x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact, and for |r| <= ln 2 / 2 a polynomial whose
-// coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits, root mean square / largest, x in -10 .. 0:
-// 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
-__device__ __forceinline__ float exp_f(float x) {
-  x = x < -200.f ? -200.f : x;
+// e^(x + rest) for x from -200, where it is zero, up to zero, and a `rest` that x had no place for.  Cody and Waite's reduction (Software
+// Manual for the Elementary Functions, 1980): x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact,
+// and for |r| <= ln 2 / 2 a polynomial whose coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits,
+// root mean square / largest, x in -10 .. 0: 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
+__device__ __forceinline__ float exp_f(float x, float rest = 0.f) {
+  const bool gone = x < -200.f;                    // (a rest that is no number then, too)
+  x = gone ? -200.f : x;
   const float n = rintf(x * 1.44269504f);
-  const float r = fmaf(-n, 1.42860677e-6f, fmaf(-n, 0.693145752f, x));
+  const float r = fmaf(-n, 1.42860677e-6f, fmaf(-n, 0.693145752f, x)) + (gone ? 0.f : rest);
   float p = fmaf(r, 0.0013814529f, 0.008368751f);
   p = fmaf(r, p, 0.041668393f);
   p = fmaf(r, p, 0.1666652f);
@@ -32,17 +33,18 @@ __device__ __forceinline__ float exp_f(float x) {
   return ldexpf(fmaf(r, p, 1.f), (int)n);
 }
 // e^(-rate softplus(x)).  softplus(x) is softplus(-|x|) more than x where x > 0, and ln(1 + t) = 2 atanh(t / (2 + t)), whose series
-// converges for t <= 1 (arguments up to 1 / 3; the coefficients are those of a fit by Chebyshev polynomials, off by 1e-9).  A fifth
-// of the instructions of the library's exponentials and logarithm; error against 64 bits, root mean square, library and here:
-// rate 4, x in -6 .. -2 2.2e-8 and 2.2e-8, x in -2 .. 2 1.20e-7 and 1.25e-7, x in 2 .. 8 4.9e-7 and 4.8e-7
+// converges for t <= 1 (arguments up to 1 / 3; the coefficients are those of a fit by Chebyshev polynomials, off by 1e-9).  What the
+// quotient and the last product lose to rounding goes on as a piece of its own.  Error against 64 bits, root mean square, with the
+// library's exponentials and logarithm (several times the instructions) and here: rate 4, x in -6 .. -2 2.20e-8 and 2.17e-8, -2 .. 2
+// 1.58e-7 and 1.14e-7, 2 .. 8 7.1e-7 and 4.8e-7; rate 16, -6 .. -2 3.9e-8 and 3.5e-8
 __device__ __forceinline__ float decay_f(float x, float rate) {
   const float t = exp_f(-fabsf(x)), w = 2.f + t, wl = t - (w - 2.f), r = __builtin_amdgcn_rcpf(w);
-  float s = t * r;
-  s = fmaf(fmaf(-wl, s, fmaf(-w, s, t)), r, s);
+  const float s0 = t * r, more = fmaf(-wl, s0, fmaf(-w, s0, t)) * r, s = s0 + more;
   const float z = s * s;
   const float p = fmaf(fmaf(fmaf(fmaf(0.122047015f, z, 0.106971338f), z, 0.143103123f), z, 0.199993476f), z, 0.333333403f);
-  const float l = fmaf(2.f * s, z * p, 2.f * s);
-  return exp_f(-rate * ((x > 0.f ? x : 0.f) + l));
+  const float l = fmaf(2.f, s0, fmaf(2.f * s, z * p, 2.f * more)), plus = (x > 0.f ? x : 0.f) + l;
+  const float y = -rate * plus;
+  return exp_f(y, fmaf(-rate, plus, -y));
 }
 // x sigmoid(x), where sigmoid(x) = 1 / (1 + t), or t / (1 + t) below zero, with t = e^-|x|: that reduction in base two, -|x| log2(e) =
 // n + f with log2(e) in two pieces, and the instruction's 2^f.  No exponent is cut off but where t is zero, so that far below zero the
