@@ -46,6 +46,12 @@ __device__ __forceinline__ float decay_f(float x, float rate) {
   const float y = -rate * plus;
   return exp_f(y, fmaf(-rate, plus, -y));
 }
+// a / d rounded as the division rounds it, d between 2^-96 and 2^96 and the quotient no denormal: the product with the reciprocal, and
+// what that leaves over once more (with the maximum, which drops a remainder that is no number: infinities stay what they are)
+__device__ __forceinline__ float quotient(float a, float d) {
+  const float r = __builtin_amdgcn_rcpf(d), q = a * r;
+  return fmaf(fmaxf(fmaf(-d, q, a), -3.40282347e38f), r, q);
+}
 // x sigmoid(x), where sigmoid(x) = 1 / (1 + t), or t / (1 + t) below zero, with t = e^-|x|: that reduction in base two, -|x| log2(e) =
 // n + f with log2(e) in two pieces, and the instruction's 2^f.  No exponent is cut off but where t is zero, so that far below zero the
 // result goes to zero as the function does.  The quotient is the product with the reciprocal and what that leaves over, with what

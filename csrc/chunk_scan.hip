@@ -400,9 +400,7 @@ __global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
       if constexpr (CHAN)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float r = __builtin_amdgcn_rcpf(P(kb, e));           // (within an ulp of the quotient: its scale and fix-up have
-          r = fmaf(fmaf(-P(kb, e), r, 1.f), r, r);             // nothing to do here)
-          kd[e] *= r;
+          kd[e] = quotient(kd[e], P(kb, e));
           q[kb][e] *= P(kb, e);
           k[kb][e] *= P(kb, e);
         }

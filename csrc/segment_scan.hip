@@ -274,11 +274,7 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
 #pragma unroll
         for (int i = 0; i < NV / 4; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {            // (within an ulp of the quotient; its scale and fix-up have nothing to do here)
-            float r = __builtin_amdgcn_rcpf(p[i][e]);
-            r = fmaf(fmaf(-p[i][e], r, 1.f), r, r);
-            kd[i][e] = k[i][e] * r;
-          }
+          for (int e = 0; e < 4; ++e) kd[i][e] = quotient(k[i][e], p[i][e]);
       }
     }
     if constexpr (OUT) {

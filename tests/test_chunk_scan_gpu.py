@@ -353,3 +353,28 @@ def test_decays_per_channel_are_as_exact_as_row_by_row(rate):
                                  state, slots, qsl, lens, 1e-6, 1, 0, chunked)
             off.append(float(((state.double() - want.unsqueeze(-1)) / want.unsqueeze(-1))[..., 0].pow(2).mean().sqrt()))
         assert 0.0 < off[0] <= 1.01 * off[1], (lo, hi, off)
+
+
+@pytest.mark.parametrize("rows", [-1, 0])                                      # the chunked kernels, segments
+def test_a_key_over_its_decays_is_rounded_once(monkeypatch, rows):
+    """Sequences of one group of 16 rows, whose first brings a key and whose queries read it again: the decays behind it, divided by and
+    multiplied with, leave the key.  Rounded to nearest, a number is off by 2.5e-8 (root mean square): the quotient, the product,
+    and with operands in thirds the 1.9e-8 of what is left out."""
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    heads, dim, seqs, at = 16, 64, 512, 37
+    g = torch.Generator(DEV).manual_seed(29)
+    key = torch.randn(seqs, heads, generator=g, device=DEV)
+    x = torch.zeros(seqs, 16, 3, heads, dim, device=DEV)
+    x[:, :, 0, :, at] = 1.0
+    x[:, 0, 1, :, at] = key
+    x[:, 0, 2, :, 5] = 1.0
+    decay = torch.ones(seqs, 16, heads, dim, device=DEV)
+    decay[:, 0, :, at] = torch.rand(seqs, heads, generator=g, device=DEV) * 0.9 + 0.1
+    qsl = torch.arange(seqs + 1, dtype=torch.int32, device=DEV) * 16
+    lens = torch.full((seqs,), 16, dtype=torch.int32, device=DEV)
+    out = hip.decay_linear_attention(x.view(seqs * 16, -1), heads, dim, dim, decay.view(seqs * 16, -1),
+                                     torch.zeros(seqs, heads, dim, dim, device=DEV), torch.arange(seqs, dtype=torch.int32, device=DEV),
+                                     qsl, lens, False, 16, 1.0, True).view(seqs, 16, heads, dim)
+    off = float(((out[:, 15, :, 5].double() - key.double()) / key.double()).pow(2).mean().sqrt())
+    parts = [2.53e-8, 2.53e-8] + ([1.9e-8] if rows == 0 else [])
+    assert 0.0 < off <= 1.06 * sum(p * p for p in parts) ** 0.5, off
