@@ -51,8 +51,11 @@ __device__ __forceinline__ void wave_topk(const T* __restrict__ row, int E, int 
 #pragma unroll
   for (int i = 0; i < TOPK_MAX_VPL; ++i)
     if (i < nv) {
-      // probabilities are >= 0: -1 marks "taken / absent"; a logit that is no number counts as zero
-      v[i] = (lane + 64 * i) < E ? fmaxf(__expf(v[i] - mx), 0.f) : -1.f;
+      // probabilities are >= 0: -1 marks "taken / absent"; a logit that is no number counts as zero, or no place would hold the maximum
+      // (by its bits, out of the compiler's sight: this file's float arithmetic is compiled as if there were no such numbers)
+      float p = __expf(v[i] - mx);
+      asm("" : "+v"(p));
+      v[i] = (lane + 64 * i) < E ? (__float_as_uint(p) < 0x7f800000u ? p : 0.f) : -1.f;
       sum += fmaxf(v[i], 0.f);
     }
   sum = wave_sum(sum);

@@ -846,6 +846,41 @@ def test_moe_topk_matches_softmax_topk(dtype, tokens, experts, k, renorm):
     assert (topw[:, :-1] >= topw[:, 1:]).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("experts,k", [(8, 8), (60, 4), (64, 6), (65, 16), (160, 8), (512, 16)])
+def test_moe_topk_ties_go_to_the_lowest_expert_and_what_is_no_number_is_never_weighed(dtype, experts, k):
+    """Equal logits on both sides of the 64 experts that a ballot covers, whole rows of them, and rows with NaN and infinities: every
+    pick is an expert, none twice, in the order of (logit, id)."""
+    from vllm_distributed_amd.ops import hip
+    ops.hip_available()
+    g = torch.Generator(DEV).manual_seed(experts)
+    logits = (torch.randint(-8, 8, (64, experts), generator=g, device=DEV) * 0.25).to(dtype)      # (many ties, distinct probabilities)
+    borders = [e for e in (63, 64, 127, 128, 191, 256, 511) if e < experts]
+    logits[0], logits[1, borders], logits[2, [e for e in (0, 59, 63, 64, 127) if e < experts]] = 1.0, 3.0, 3.0
+    nan, inf = float("nan"), float("inf")
+    odd = logits[:8].clone()
+    odd[0, experts // 2], odd[1, :experts - 1], odd[2], odd[3] = nan, nan, nan, -inf
+    odd[4, experts - 1], odd[5, 1:3], odd[6, 2], odd[7, ::2] = inf, inf, -inf, -inf
+    for rows in (logits, odd):
+        w, picked = hip.moe_topk(rows, k, True)
+        assert ((picked >= 0) & (picked < experts)).all()
+        assert (picked.sort(-1).values.diff(dim=-1) > 0).all()
+        x = torch.zeros(rows.shape[0], 64, dtype=torch.bfloat16, device=DEV)
+        if rows is odd:
+            _, small, inv, _, _ = hip.moe_route_small(rows, x, k, True, 16)
+            assert torch.equal(small, picked) and torch.equal(inv.long().sort().values, torch.arange(8 * k, device=DEV))
+            finite = [0, 1, 6, 7]                                             # (rows whose maximum is a number)
+            x32 = odd[finite].float().nan_to_num(nan=-inf, neginf=-inf)
+            w, picked = w[finite], picked[finite]
+        else:
+            x32 = rows.float()
+        probs = torch.softmax(x32, -1)
+        want = torch.sort(probs, dim=-1, descending=True, stable=True).indices[:, :k]
+        assert torch.equal(picked.long(), want)
+        ref = probs.gather(1, want)
+        assert torch.allclose(w, ref / ref.sum(-1, keepdim=True), atol=1e-6, rtol=1e-5)
+
+
 @pytest.mark.parametrize("tokens,experts,k,tile_rows,ep", [(1, 160, 8, 16, None), (64, 16, 4, 16, None),
                                                            (1000, 160, 8, 64, None), (300, 16, 4, 32, (4, 8)),
                                                            (9000, 64, 8, 128, None)])
