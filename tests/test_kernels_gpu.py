@@ -687,6 +687,34 @@ def test_sample_finds_the_border_inside_one_bin(n, equal):
         assert got.tolist() == [order[r - 1].item() for r in at], kept
 
 
+@pytest.mark.parametrize("n", [65, 1500, 4096])
+@pytest.mark.parametrize("values,share", [(2, 0.9), (2, 0.5), (3, 0.34), (4096, 0.8), (4096, 0.3)])
+def test_sample_finds_the_border_among_weights_that_many_entries_have(n, values, share):
+    """``n`` entries of one histogram bin, a ``share`` of them alike and the others of ``values`` weights, in no order of their indices:
+    kept by count and by mass, drawn in the order of (weight, index) as in ``test_sample_finds_the_border_inside_one_bin``."""
+    V = 9000
+    g = torch.Generator(DEV).manual_seed(n + values)
+    order = torch.randperm(V - 2, generator=g, device=DEV)[:n].sort().values
+    step = torch.randint(0, min(values, n), (n,), generator=g, device=DEV)
+    step[torch.rand(n, generator=g, device=DEV) < share] = min(values, n) // 2
+    w = 0.61 - 0.01 * step.double() / max(min(values, n) - 1, 1)
+    rank = torch.argsort(w, descending=True, stable=True)
+    order, w = order[rank], w[rank]
+    row = torch.full((V,), -40.0, device=DEV)
+    row[order], row[V - 1] = torch.log(w).float(), 0.0
+    cum = torch.cat([torch.ones(1, device=DEV, dtype=torch.float64), w]).cumsum(0)
+    ranks = sorted({1, 2, n // 3, n // 2, n - 1, n})
+    for kept, by_mass in ((n, False), (n // 2, False), (2, False), (n // 2, True)):
+        at = [r for r in ranks if r <= kept]
+        u = torch.stack([(cum[r] - 0.5 * w[r - 1]) / cum[kept] for r in at]).float()
+        full = lambda v, t=torch.float32: torch.full((len(at),), v, device=DEV, dtype=t)
+        all_of_it = cum[-1] + (V - 1 - n) * torch.exp(torch.tensor(-40.0, dtype=torch.float64, device=DEV))
+        top_p = float((cum[kept] - 0.5 * w[kept - 1]) / all_of_it) if by_mass else 1.0
+        got = ops.sample(row.expand(len(at), -1).contiguous(), full(1.0), full(0 if by_mass else kept + 1, torch.int32), full(top_p),
+                         full(0.0), u)
+        assert got.tolist() == [order[r - 1].item() for r in at], (kept, by_mass)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("V,offset", [(1, 0), (7, 3), (511, 1), (519, 0), (8192, 0), (50257, 1), (128256, 0), (151936, 5), ((1 << 23) + 9, 0)])
 def test_sample_of_counted_patterns_is_the_one_of_the_same_values_in_32_bits(V, offset, dtype):
