@@ -5,7 +5,7 @@ from vllm_distributed_amd.ops import hip as _hip, torch_ref
 assert ops.hip_available()
 DK, DV, BS = 576, 512, 64
 dev = "cuda"
-for hq in (16, 32):
+for hq in (16, 32, 128):
     for batch, ctx in ((1, 1024), (1, 4096), (1, 32768), (4, 4096), (8, 4096), (16, 4096), (32, 4096), (64, 4096), (128, 4096), (64, 512), (256, 1024), (32, 32768)):
         nblk = batch * (-(-ctx // BS)) + 1
         kc = (torch.randn(torch_ref.k_cache_shape(nblk, 1, DK, BS), device=dev) * 0.3).bfloat16()

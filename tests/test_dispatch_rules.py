@@ -63,15 +63,52 @@ def test_decode_splits(monkeypatch, batch, heads, keys, captured, splits):
     (100, 16, 700, False, 100, True, True, (3, 5)), (160, 16, 3000, False, 160, True, True, (3, 3)),
     (130, 16, 400, False, 130, True, True, (3, 3)), (15, 128, 200, False, 15, True, True, (3, 1)),
     (256, 16, 400, False, 256, True, True, (3, 1)), (128, 16, 3100, False, 128, True, True, (3, 4)),
-    # four head tiles a workgroup: 54 / 72, 118 / 149
-    (40, 128, 500, False, 40, True, True, (2, 3)), (100, 128, 700, False, 100, True, True, (2, 1)),
+    # many heads by one, whatever the number of rows (four head tiles a workgroup, one): 167 / 101, 139 / 112, 346 / 288
+    (69, 128, 780, False, 69, True, True, (3, 1)), (128, 128, 600, False, 128, True, True, (3, 1)),
+    (256, 64, 1500, False, 256, True, True, (3, 1)), (20, 128, 3000, False, 20, True, True, (3, 3)),
+    # prompts and verified rows over key rows (both caches, key rows): 47 / 31, 62 / 26, 231 / 133, 31 / 21, 56 / 24, 58 / 22, 50 / 32,
+    # 42 / 30; from Python whole up to 383 keys (whole, split): 17.0 / 21.2; in a graph split: 17.4 / 12.8
+    (200, 16, 700, True, 1, True, False, (3, 2)), (600, 16, 300, True, 2, True, False, (3, 1)),
+    (1000, 16, 1500, True, 1, True, False, (3, 1)), (8, 16, 2000, True, 1, True, False, (3, 31)),
+    (4, 16, 16000, True, 1, True, False, (3, 64)), (64, 16, 1000, True, 16, True, True, (3, 8)),
+    (32, 128, 600, True, 1, True, False, (3, 2)), (8, 128, 2000, True, 1, True, False, (3, 8)),
+    (32, 16, 300, True, 1, True, False, (3, 1)), (32, 16, 300, True, 1, True, True, (3, 4)),
+    # caches whose key rows cannot be read.  Four head tiles a workgroup: 54 / 72, 118 / 149
+    (40, 128, 500, False, 40, False, True, (2, 3)), (100, 128, 700, False, 100, False, True, (2, 1)),
     # prompts: 47 / 66, 65 / 92, rows of different lengths in two 227 / 269 and 102 / 116; 3 tokens of 16 sequences 50 / 56
-    (200, 16, 700, True, 1, True, False, (1, 5)), (192, 32, 564, True, 3, True, False, (1, 2)),
-    (1000, 16, 1000, True, 2, True, False, (1, 2)), (600, 16, 300, True, 2, True, False, (1, 2)),
-    (700, 16, 700, True, 1, True, False, (1, 2)), (1500, 16, 1500, True, 1, True, False, (1, 1)),
-    (48, 16, 1500, True, 16, True, True, (1, 9)), (32, 16, 300, True, 1, True, False, (1, 4))])
+    (200, 16, 700, True, 1, False, False, (1, 5)), (192, 32, 564, True, 3, False, False, (1, 2)),
+    (1000, 16, 1000, True, 2, False, False, (1, 2)), (600, 16, 300, True, 2, False, False, (1, 2)),
+    (700, 16, 700, True, 1, False, False, (1, 2)), (1500, 16, 1500, True, 1, False, False, (1, 1)),
+    (48, 16, 1500, True, 16, False, True, (1, 9)), (32, 16, 300, True, 1, False, False, (1, 4))])
 def test_latent_plan(tokens, heads, keys, by_token, seqs, rows_ok, captured, plan):
     assert hip.mla_plan(tokens, heads, keys, by_token, seqs, rows_ok, None, captured) == plan
+
+
+@pytest.mark.parametrize("rows_ok", [True, False])
+def test_latent_attention_takes_the_plan(rows_ok, monkeypatch):
+    """What ``mla_plan`` answers is what the kernels are handed; there is no rule beside it."""
+    import torch
+    handed = []
+
+    class Lib:
+        @staticmethod
+        def vdamd_mla_attention(*args):
+            handed.append(args[18:20])                 # splits, mode
+            return 0
+    monkeypatch.setattr(hip, "_LIB", Lib)
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "mla_supported", lambda *shape: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    block = 32 if rows_ok else 16
+    kc = torch.zeros(128 // block, 1, block, 320, dtype=torch.bfloat16)
+    vc = torch.zeros(128 // block, 1, 16, block // 8, 16, 8, dtype=torch.bfloat16)
+    for tokens, heads, by_token in ((9, 16, True), (40, 64, False), (2, 16, False)):
+        table = torch.zeros(1 if by_token else tokens, 128 // block, dtype=torch.int32)
+        hip.mla_attention(torch.zeros(tokens, heads, 320, dtype=torch.bfloat16), kc, vc, table,
+                          torch.zeros(tokens, dtype=torch.int32) if by_token else None,
+                          torch.full((tokens,), 100, dtype=torch.int32), 0.1, 100)
+        mode, splits = hip.mla_plan(tokens, heads, 100, by_token, table.shape[0], rows_ok, None, False)
+        assert handed[-1] == (splits, mode) and (mode == 3) is rows_ok
 
 
 @pytest.mark.parametrize("m,n,k,reduced,takes", [

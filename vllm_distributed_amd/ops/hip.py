@@ -1320,24 +1320,30 @@ def mla_num_splits(tokens: int, q_tiles: int, max_seq_len: int, workgroups: int 
 
 def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows_ok: bool, mode: Optional[int] = None,
              captured: bool = True) -> Tuple[int, int]:
-    """Kernel (``mla_attention``'s ``mode``, chosen here when None; who can always read key rows passes 3) and KV splits of a step of
-    ``tokens`` rows of up to ``keys`` keys from ``seqs`` sequences (``by_token``: rows name theirs), ``captured`` in a graph or
-    launched from Python.
+    """Kernel (``mla_attention``'s ``mode``, chosen here when None) and KV splits of a step of ``tokens`` rows of up to ``keys`` keys
+    from ``seqs`` sequences (``by_token``: rows name theirs), ``captured`` in a graph or launched from Python.
 
-    Splits make as many workgroups as run at once - one per CU of the kernels that share keys between four tiles (1, 2), two of
-    the one over key rows (3) - and not more: what is left over waits for a second round.  Prompt of 200 tokens, 16 heads, 700 keys
-    (50 workgroups): 47 us in 5 splits, 66 in 6; three of 64, 32 heads, 564 keys (102): 65 in 2, 92 in 3; 100 decoded rows of
-    700 keys 26.8 in 5 and 32.6 in 6, 160 of 3000 keys 93 in 3 and 117 in 4.  Splits hold 64 keys, or 128 where more than 64
-    workgroups leave many partial sums (16 rows of 128 heads, 200 keys: 14.5 us whole, 19.7 in 3), 256 where there is a
-    workgroup for every CU (256 rows, 400 keys: 24.7 whole, 32.8 in 2).  Prompts that take most CUs whole still go in two, which
-    evens out their rows of different lengths (two of 500 rows on average behind 500 keys: 269 us whole, 227 in 2; one of 700: 116
-    and 102; though two of exactly 300: 58 and 62).
-    Outside a graph a second launch and its buffers cost the host 6.5 us: up to 383 keys of decoded rows are not split (200
-    keys: 13.6 us whole, 20 in 3; 500 keys 25 and 20)."""
+    The kernel over the key rows (3) wherever it reads the cache (``rows_ok``): it reads a row once per token and 16 heads, but out of
+    the caches and by DMA; the two that share keys between four tiles (1, 2) read both caches into registers, 70 KB per 5 us a
+    workgroup.  us, shared / rows: prompt tokens of 16 heads, 2611 of three sequences 377 / 232, 1834 of one 419 / 236, 85 behind 330
+    34 / 21, four each of 64 sequences of 4000 keys 664 / 182, of 16 of 1000 58 / 24; of 128 heads, 880 of three 902 / 584, 76 77 / 31,
+    565 of 5000 keys 3647 / 2255; decoded rows of 128 heads, 69 of 780 keys 167 / 101, 20 of 3000 124 / 101, 128 of 600 139 / 112; of
+    64, 100 of 800 104 / 68, 256 of 1500 346 / 288.
+
+    Splits make as many workgroups as run at once - one per CU of the kernels that share keys, two of the one over key rows - and not
+    more: what is left over waits for a second round.  Over key rows 100 decoded rows of 700 keys 26.8 in 5 and 32.6 in 6, 160 of 3000
+    keys 93 in 3 and 117 in 4.  Over both caches a prompt of 200 tokens, 16 heads, 700 keys (50 workgroups) 47 us in 5 splits, 66 in 6;
+    three of 64, 32 heads, 564 keys (102) 65 in 2, 92 in 3; prompts that take most CUs whole still go in two, which evens out their
+    rows of different lengths (two of 500 rows on average behind 500 keys: 269 us whole, 227 in 2; one of 700: 116 and 102; though two
+    of exactly 300: 58 and 62).  Splits hold 64 keys, or 128 where more than 64 workgroups leave many partial sums (16 rows of 128
+    heads, 200 keys: 14.5 us whole, 19.7 in 3), 256 where there is a workgroup for every CU (256 rows, 400 keys: 24.7 whole, 32.8
+    in 2).
+    Outside a graph a second launch and its buffers cost the host 6.5 us: up to 383 keys rows are not split (a decoded row of 200 keys
+    13.6 us whole, 20 in 3; 32 prompt tokens of 300 keys 17.0 and 21.2, 8 of 380 19.7 and 21.0; 500 keys 25 and 20)."""
     q_tiles = -(-heads // 16)
     if mode is None:
         # (four head tiles per workgroup need enough workgroups left to fill the chip)
-        mode = 1 if by_token else 2 if q_tiles >= 4 and tokens * q_tiles >= 128 else 3 if rows_ok else 0
+        mode = 3 if rows_ok else 1 if by_token else 2 if q_tiles >= 4 and tokens * q_tiles >= 128 else 0
     if mode in (0, 3) and keys < 384 and not captured:
         return mode, 1
     if mode == 0:
@@ -1390,16 +1396,7 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         assert gate.dim() == 2 and gate.shape[0] >= t and gate.shape[1] == hq and gate.stride(1) == 1 and gate.dtype == q.dtype
         gate_stride = gate.stride(0)
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
-    rows_ok = mla_rows_ok(k_cache, dv)
-    if mode is None and rows_ok:
-        # It reads a row once per token and 16 heads, but out of the caches and by DMA; the two that share keys between four tiles
-        # read both caches into registers, 70 KB per 5 us a workgroup.  us, shared / rows: prompt tokens of 16 heads, 2611 of three
-        # sequences 377 / 232, 1834 of one 419 / 236, 85 behind 330 34 / 21, four each of 64 sequences of 4000 keys 664 / 182, of 16
-        # of 1000 57 / 23; of 128 heads, 880 of three 902 / 584, 76 77 / 31, 565 of 5000 keys 3647 / 2255; decoded rows of 128
-        # heads, 69 of 780 keys 167 / 101, 20 of 3000 124 / 101, 128 of 600 139 / 112; of 64, 100 of 800 104 / 68, 256 of 1500
-        # 346 / 288.
-        mode = 3
-    mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], rows_ok, mode,
+    mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
     # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
     past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
