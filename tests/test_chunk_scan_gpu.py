@@ -1,5 +1,7 @@
-"""The chunked kernels of the recurrent mixers (64 rows of a prompt at a time, fp32 matrix instructions) against the
-recurrences run row by row in 64 bits, and their error beside that of the row by row kernels."""
+"""The chunked kernels of the recurrent mixers (64 rows of a prompt at a time) and those over segments (32 rows at a time, prompts cut
+into pieces that run side by side) against the recurrences run row by row in 64 bits, and their error beside that of the row by row
+kernels.  Both form products of 32-bit values; the delta rule's walk and all of the segments' on 16-bit matrix instructions, the
+operands in three pieces."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -57,6 +59,15 @@ def _run(c, chunked):
         out = hip.decay_linear_attention(c["x"], c["heads"], c["dim"], c["vdim"], c["decay"], *at, op == "linear_head", most,
                                          0.25 if op == "linear_channel" else 1.0, chunked)
     return out, state
+
+
+def _segments(monkeypatch, rows):
+    """Calls that choose by size (``chunked`` None) go over segments of ``rows`` rows (0: whole sequences), or fail."""
+    def refuse(*args):
+        raise AssertionError("the call did not go over segments")
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    monkeypatch.setattr(hip, "_chunked", refuse)
+    monkeypatch.setattr(hip, "_chunk_scan", refuse)
 
 
 def _rows64(c):
@@ -220,17 +231,23 @@ def test_what_is_not_finite_stays_in_its_row_and_behind(op, what, value, heads, 
 
 @pytest.mark.parametrize("op", OPS)
 @pytest.mark.parametrize("new", [[700, 300, 1, 1], [900] + [1] * 40])
-def test_the_memory_profile_holds_what_a_step_allocates(op, new):
-    """``chunk_scan_bytes`` (the runner keeps as much aside) covers the peak of a call, also for a step of fewer rows."""
+@pytest.mark.parametrize("chunked", [True, None])
+def test_the_memory_profile_holds_what_a_step_allocates(monkeypatch, op, new, chunked):
+    """``chunk_scan_bytes`` (the runner keeps as much aside) covers the peak of a call, also for a step of fewer rows, and with the
+    shortest segments that are made (``chunked`` None)."""
+    if chunked is None:
+        if op.startswith("delta"):
+            pytest.skip("the delta rule has no segments")
+        _segments(monkeypatch, 96)
     from vllm_distributed_amd import ops
     heads, groups, dim, vdim = 16, 16, 64, 128
     c = _case(op, heads, groups, dim, vdim, new, new, torch.bfloat16, 9)
-    _run(c, True)
+    _run(c, chunked)
     state = c["state"].nbytes                                       # (``_run`` works on a copy)
     torch.cuda.synchronize()
     torch.cuda.reset_peak_memory_stats()
     before = torch.cuda.memory_allocated()
-    _run(c, True)
+    _run(c, chunked)
     torch.cuda.synchronize()
     used = torch.cuda.max_memory_allocated() - before - state
     bound = ops.recurrence_bytes(2000, len(new), heads, dim, vdim, op.startswith("delta"))
@@ -251,16 +268,15 @@ def test_the_memory_profile_holds_what_a_step_allocates(op, new):
     (3, 64, 64, *_many(70), torch.bfloat16)])                              # more sequences than a wave has lanes
 def test_segments_match_the_recurrence_in_64_bits(monkeypatch, op, rows, strong, heads, dim, vdim, new, extra, dtype):
     """The bound of ``test_chunks_match_the_recurrence_in_64_bits``, whatever sequences are cut at (0: nowhere)."""
-    asked = []
-    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: asked.append(sizes) or rows)
+    _segments(monkeypatch, rows)
     c = _case(op, heads, 1 if op == "state_space" else heads, dim, vdim, new, [n + e for n, e in zip(new, extra)], dtype, 23,
               strong, 8)
     want, want_state = _rows64(c)
-    out, state = _run(c, True)
-    assert asked and _off(out, want) < 3e-6 and _off(state, want_state) < 3e-6, (_off(out, want), _off(state, want_state))
+    out, state = _run(c, None)
+    assert _off(out, want) < 3e-6 and _off(state, want_state) < 3e-6, (_off(out, want), _off(state, want_state))
     untouched = [i for i in range(c["state"].shape[0]) if i not in [int(x) for x, n in zip(c["slots"], new) if n]]
     assert torch.equal(state[untouched], c["state"][untouched])
-    again, state2 = _run(c, True)
+    again, state2 = _run(c, None)
     assert torch.equal(out, again) and torch.equal(state, state2)
 
 
@@ -271,10 +287,11 @@ def test_segments_are_no_less_exact_than_chunks(monkeypatch, op, rows):
     c = _case(op, 4, 4, 128, 128, [700, 300], [700, 420], torch.bfloat16, 3)
     want, want_state = _rows64(c)
     off = []
-    for cut in (rows, -1):
-        monkeypatch.setattr(hip, "segment_rows", lambda *sizes: cut)
-        out, state = _run(c, True)
-        off.append((_off(out, want), _off(state, want_state)))
+    for chunked in (True, None):
+        if chunked is None:
+            _segments(monkeypatch, rows)
+        out, state = _run(c, chunked)
+        off.insert(0, (_off(out, want), _off(state, want_state)))
     assert off[0][0] <= 1.05 * off[1][0] and off[0][1] <= 1.05 * off[1][1], off
 
 
@@ -282,13 +299,14 @@ def test_segments_are_no_less_exact_than_chunks(monkeypatch, op, rows):
 @pytest.mark.parametrize("what,value", [("v", float("nan")), ("v", float("inf")), ("k", float("nan")), ("q", float("nan")),
                                         ("dt", float("nan"))])
 @pytest.mark.parametrize("rows", [0, 64])
-def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch, op, what, value, rows):
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])      # (of 16 bits, operands may be one piece)
+def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch, op, what, value, rows, dtype):
     if what == "dt" and op.startswith("linear"):
         pytest.skip("the recurrence has no such input")
-    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    _segments(monkeypatch, rows)
     heads, dim, vdim, new, row, head = 4, 128, 128, [150, 40, 70, 33], 21 + 64, 2
-    c = _case(op, heads, heads, dim, vdim, new, [150, 47, 70, 35], torch.float32, 7)
-    clean, _ = _run(c, True)
+    c = _case(op, heads, heads, dim, vdim, new, [150, 47, 70, 35], dtype, 7)
+    clean, _ = _run(c, None)
     if what == "dt":
         c[what][row] = value
     else:
@@ -296,7 +314,7 @@ def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch,
         if op == "state_space":
             at = {"v": 0, "k": heads * vdim, "q": heads * vdim + heads * dim}
         c["x"][row, at[what] + head * (vdim if what == "v" else dim) + 5] = value
-    got, _ = _run(c, True)
+    got, _ = _run(c, None)
     other = torch.ones(sum(new), dtype=torch.bool, device=DEV)
     other[row:150] = False
     assert _off(got[other], clean[other].double()) < 3e-6
@@ -312,7 +330,8 @@ def test_what_is_not_finite_stays_in_its_row_and_behind_in_segments(monkeypatch,
 def test_activated_inputs_far_below_zero_go_to_zero(monkeypatch, rows):
     """SiLU of what its exponential overflows for.  One row's key and query have one entry, and its value is read out again: a
     product of three activations, each within 2e-7 of 64 bits, and zero (to denormals) where they are."""
-    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    if rows >= 0:
+        _segments(monkeypatch, rows)
     heads, dim, new = 1, 64, [48, 48]
     x = torch.zeros(96, 3 * dim, device=DEV)
     entries = torch.tensor([-0.5, -20.0, -80.0, -87.0, -88.0, -90.0, -100.0, -200.0, -1e4, -1e30, -3e38, 3e37], device=DEV)
@@ -322,7 +341,7 @@ def test_activated_inputs_far_below_zero_go_to_zero(monkeypatch, rows):
          "state": torch.zeros(2, heads, dim, dim, device=DEV), "slots": torch.tensor([1, 0], dtype=torch.int32, device=DEV),
          "decay": torch.full((heads,), 0.5, device=DEV), "beta": torch.zeros(96, heads, device=DEV)}
     want, want_state = _rows64(c)
-    out, state = _run(c, True)
+    out, state = _run(c, True if rows < 0 else None)
     got, ref = out[5].double(), want[5]
     assert torch.isfinite(out).all() and torch.isfinite(state).all()
     assert ((got - ref).abs() <= 8e-7 * ref.abs() + 1e-36).all(), (got[:len(entries)].tolist(), ref[:len(entries)].tolist())
@@ -360,7 +379,8 @@ def test_a_key_over_its_decays_is_rounded_once(monkeypatch, rows):
     """Sequences of one group of 16 rows, whose first brings a key and whose queries read it again: the decays behind it, divided by and
     multiplied with, leave the key.  Rounded to nearest, a number is off by 2.5e-8 (root mean square): the quotient, the product,
     and with operands in thirds the 1.9e-8 of what is left out."""
-    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: rows)
+    if rows >= 0:
+        _segments(monkeypatch, rows)
     heads, dim, seqs, at = 16, 64, 512, 37
     g = torch.Generator(DEV).manual_seed(29)
     key = torch.randn(seqs, heads, generator=g, device=DEV)
@@ -374,7 +394,7 @@ def test_a_key_over_its_decays_is_rounded_once(monkeypatch, rows):
     lens = torch.full((seqs,), 16, dtype=torch.int32, device=DEV)
     out = hip.decay_linear_attention(x.view(seqs * 16, -1), heads, dim, dim, decay.view(seqs * 16, -1),
                                      torch.zeros(seqs, heads, dim, dim, device=DEV), torch.arange(seqs, dtype=torch.int32, device=DEV),
-                                     qsl, lens, False, 16, 1.0, True).view(seqs, 16, heads, dim)
+                                     qsl, lens, False, 0, 1.0, True if rows < 0 else None).view(seqs, 16, heads, dim)
     off = float(((out[:, 15, :, 5].double() - key.double()) / key.double()).pow(2).mean().sqrt())
     parts = [2.53e-8, 2.53e-8] + ([1.9e-8] if rows == 0 else [])
     assert 0.0 < off <= 1.06 * sum(p * p for p in parts) ** 0.5, off

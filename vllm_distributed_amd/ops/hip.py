@@ -1798,7 +1798,7 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
                            state: torch.Tensor, slots: torch.Tensor, query_start_loc: torch.Tensor,
                            seq_lens: torch.Tensor, silu: bool = True, max_query_len: int = 0,
                            scale: float = 1.0, chunked: Optional[bool] = None) -> torch.Tensor:
-    """``chunked`` forces (or forbids) the chunked kernels (tests, benchmarks)."""
+    """``chunked`` forces the chunked kernels, or the walk row by row (tests, benchmarks); None: by size, segments among them."""
     t = x.shape[0]
     n = seq_lens.numel()
     if dim > DECAY_ATTENTION_MAX_DIM:
@@ -1815,10 +1815,11 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
     if chunked or (chunked is None and not 0 < max_query_len < CHUNK_MIN_ROWS):
         qs = num_heads * dim
         rates = decay if decay.dim() == 2 else _f32_vec(decay, num_heads, "decay")
-        out = _segment_scan(kind, x, 0, qs, 2 * qs, None, None, None, rates, None, num_heads, num_heads, dim, vdim, state, slots,
-                            query_start_loc, seq_lens, silu, scale, max_query_len)
-        if out is not None:
-            return out
+        if chunked is None:
+            out = _segment_scan(kind, x, 0, qs, 2 * qs, None, None, None, rates, None, num_heads, num_heads, dim, vdim, state, slots,
+                                query_start_loc, seq_lens, silu, scale, max_query_len)
+            if out is not None:
+                return out
         if chunked or _chunked(kind, x, t, n, max_query_len, num_heads, dim, vdim):
             return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None, rates, None, num_heads, num_heads, dim, vdim,
                                state, slots, query_start_loc, seq_lens, silu, 0.0, scale)
@@ -2128,8 +2129,8 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
 # ------------------------------------------------ q / k normed over all heads with values = keys, mixed head weights
 def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, a_log, dt_bias, d_skip, state, slots,
                    query_start_loc, seq_lens, max_query_len: int = 0, chunked: Optional[bool] = None) -> torch.Tensor:
-    """``max_query_len`` (0: unknown) only helps the kernel choose its launch; ``chunked`` forces (or forbids) the chunked
-    kernels (tests, benchmarks)."""
+    """``max_query_len`` (0: unknown) only helps choose the kernel; ``chunked`` forces the chunked kernels, or the walk row by row
+    (tests, benchmarks); None: by size, segments among them."""
     t = _rows2d(x, "x").shape[0]
     h, g, n = int(num_heads), int(groups), int(n_state)
     b = seq_lens.shape[0]
@@ -2142,9 +2143,10 @@ def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, 
         inner = h * vdim
         mine = (_f32_vec(dt_bias, h, "dt_bias"), _f32_vec(a_log, h, "a_log"), None, _f32_vec(d_skip, h, "d_skip"), h, g, n, int(vdim),
                 state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"), False)
-        out = _segment_scan(STATE_SPACE, x, inner + g * n, inner, 0, dt, *mine, 1.0, max_query_len)
-        if out is not None:
-            return out
+        if chunked is None:
+            out = _segment_scan(STATE_SPACE, x, inner + g * n, inner, 0, dt, *mine, 1.0, max_query_len)
+            if out is not None:
+                return out
         if chunked or _chunked(STATE_SPACE, x, t, b, max_query_len, h, n, int(vdim)):
             return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, *mine, 0.0, 1.0)
     out = torch.empty((t, h * vdim), dtype=torch.float32, device=x.device)
