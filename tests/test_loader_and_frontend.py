@@ -745,8 +745,9 @@ def test_hot_attention_kernels_fit_the_register_file(tmp_path):
         pytest.skip("no hipcc")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     asm = tmp_path / "attention.s"
-    subprocess.run([hipcc, "-S", "--offload-arch=gfx950", "--cuda-device-only", "-O3", "-std=c++17",
-                    "-I" + os.path.join(root, "csrc"), os.path.join(root, "csrc", "attention.hip"), "-o", str(asm)],
+    from vllm_distributed_amd import build                     # (as the library is built: other flags, other registers)
+    assert "attention.hip" not in build.EXACT_MATH_SOURCES
+    subprocess.run([hipcc, "-S", "--cuda-device-only", *build.HIP_FLAGS, os.path.join(root, "csrc", "attention.hip"), "-o", str(asm)],
                    check=True, capture_output=True, timeout=600)
     spilled = {}
     for m in re.finditer(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", asm.read_text(), re.S):
