@@ -45,7 +45,7 @@ struct SegArgs {
   const int* slots;
   const int* qsl;
   const int* seq_lens;
-  int B, H, G, dim, vdim;
+  int B, H, G, dim, vdim, tiles;                   // tiles of columns
   int rows;                                        // of a segment (a multiple of 32); 0: a sequence is one
   int silu;
   float scale;
@@ -95,26 +95,30 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
   __shared__ double td[2][2], sd[CHAN ? 1 : G16];
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, kh = lane >> 4;
-  // ---- which segment
+  // ---- which segment: neighbours in the grid, which go to the eight dies in turn, are a segment's heads.  (With the segments side by
+  // side, 8 sequences or a multiple of it put all heads of one on one die: 32 heads of 128 x 64, 589 rows of 32, one of 376, 274 us,
+  // now 76; 2048 rows of 8 in segments of 480 115 and 67)
+  const int heads = a.H * a.tiles, want = blockIdx.x / heads, h = (blockIdx.x - want * heads) % a.H;
+  const int tile = (blockIdx.x - want * heads) / a.H;
   int seq, s, ns;
   if (a.rows) {
-    if (!locate(a.B, blockIdx.x, seq, s, [&](int i) { return segments_of(a.qsl, i, a.rows); })) return;
+    if (!locate(a.B, want, seq, s, [&](int i) { return segments_of(a.qsl, i, a.rows); })) return;
     seq = __builtin_amdgcn_readfirstlane(seq);     // (the same in all lanes, which the compiler does not see)
     s = __builtin_amdgcn_readfirstlane(s);
     ns = segments_of(a.qsl, seq, a.rows);
   } else {
-    seq = __builtin_amdgcn_readfirstlane(by_length(a.qsl, a.B, blockIdx.x));
+    seq = __builtin_amdgcn_readfirstlane(by_length(a.qsl, a.B, want));
     s = 0;
     ns = 1;
   }
   const int n_all = a.qsl[seq + 1] - a.qsl[seq];
   if (n_all <= 0 || (!OUT && s == ns - 1)) return;
-  const int h = blockIdx.y, grp = h / (a.H / a.G), v0 = blockIdx.z * VW;
+  const int grp = h / (a.H / a.G), v0 = tile * VW;
   const int each = a.rows ? segment_rows(n_all, a.rows) : n_all;
   const long q0 = a.qsl[seq] + (long)s * each;
   const int n = min(each, n_all - s * each), nc = (n + R - 1) / R;
-  const long unit = state_floats(DP, gridDim.z * VW);
-  float* const wst = a.ws + ((long)blockIdx.x * a.H + h) * unit;
+  const long unit = state_floats(DP, a.tiles * VW);
+  float* const wst = a.ws + ((long)want * a.H + h) * unit;
 
   // ---- the preparation: wave (group of 16 rows, quarter of the channels), lane (row lr, channels kh NV ..)
   const int g = wave >> 2, qt = wave & 3;
@@ -156,8 +160,8 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
     return v < a.vdim ? (d * a.vdim + v) * 4 : 0x40000000;
   };
   auto kept = [&](float* p, int db, int ct) {      // the same in the workspace
-    const int tile = blockIdx.z * (VW / 16) + cg * CT + ct;
-    return reinterpret_cast<f32x4*>(p + (((long)(dh * DB + db) * (gridDim.z * VW / 16) + tile) * 64 + lane) * 4);
+    const int at = tile * (VW / 16) + cg * CT + ct;
+    return reinterpret_cast<f32x4*>(p + (((long)(dh * DB + db) * (a.tiles * VW / 16) + at) * 64 + lane) * 4);
   };
   fetch(0);
 #pragma unroll
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) *kept(next, db, ct) = S[db][ct];
-    if (blockIdx.z == 0 && threadIdx.x < DP) next[unit - DP + threadIdx.x] = CHAN ? all : (float)all_d;
+    if (tile == 0 && threadIdx.x < DP) next[unit - DP + threadIdx.x] = CHAN ? all : (float)all_d;
   }
 #endif
 }
@@ -563,9 +567,10 @@ __global__ __launch_bounds__(256) void segment_starts(SegArgs a, int DP, int VP)
   }
 }
 
-template <typename T, int KIND, bool X, int DP, int VW> int launch(const SegArgs& a, int segments, hipStream_t st) {
-  const int tiles = (a.vdim + VW - 1) / VW;
-  const dim3 grid(segments, a.H, tiles);
+template <typename T, int KIND, bool X, int DP, int VW> int launch(SegArgs a, int segments, hipStream_t st) {
+  const int tiles = a.tiles = (a.vdim + VW - 1) / VW;
+  if ((long)segments * a.H * tiles * 512 > 0xffffffffl) return 1;                  // (of threads, a launch's limit)
+  const dim3 grid(segments * a.H * tiles);
   if (a.rows) {
     hipLaunchKernelGGL((segment_kernel<T, KIND, X, DP, VW, false>), grid, dim3(512), 0, st, a);
     hipLaunchKernelGGL(segment_starts, dim3(a.B * a.H, (DP * tiles * VW + 1023) / 1024), dim3(256), 0, st, a, DP, tiles * VW);
