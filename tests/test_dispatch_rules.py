@@ -13,12 +13,11 @@ from vllm_distributed_amd.ops import hip
     (hip.DELTA_CHANNEL, 8017, 5, 2000, 16, 128, 128, True), (hip.LINEAR_CHANNEL, 8017, 5, 2000, 16, 128, 128, True),
     (hip.LINEAR_HEAD, 8017, 5, 2000, 16, 128, 128, True), (hip.STATE_SPACE, 8017, 5, 2000, 16, 128, 128, True),
     (hip.DELTA_CHANNEL, 700, 1, 700, 16, 128, 128, True), (hip.DELTA_CHANNEL, 210, 2, 120, 32, 128, 128, True),
-    # one short prompt: 46 / 38; many prompts of a few chunks: 206 / 181, 370 / 303, 412 / 338
-    (hip.DELTA_CHANNEL, 60, 1, 60, 8, 128, 128, False), (hip.LINEAR_CHANNEL, 6000, 24, 250, 16, 128, 128, False),
-    (hip.LINEAR_HEAD, 8964, 54, 166, 16, 128, 128, False), (hip.DELTA_HEAD, 6720, 48, 140, 16, 128, 128, False),
-    # small heads, where a chunk costs more than its share of the products: 121 / 81, 113 / 69, 160 / 111, 180 / 126
+    # one short prompt: 34 / 38, of many heads 46 / 93
+    (hip.DELTA_CHANNEL, 60, 1, 60, 8, 128, 128, True), (hip.DELTA_CHANNEL, 97, 1, 97, 64, 128, 128, True),
+    # small heads, where a chunk costs more than its share of the products: 109 / 91, 101 / 72, 151 / 110
     (hip.LINEAR_HEAD, 960, 63, 300, 32, 16, 16, False), (hip.LINEAR_CHANNEL, 960, 63, 300, 32, 16, 16, False),
-    (hip.DELTA_CHANNEL, 8990, 58, 155, 16, 16, 16, False), (hip.STATE_SPACE, 960, 63, 300, 32, 64, 64, False)])
+    (hip.DELTA_CHANNEL, 8990, 58, 155, 16, 16, 16, False)])
 def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest, heads, dim, vdim, chunked):
     assert hip.chunk_scan_profitable(kind, rows, seqs, longest, heads, dim, vdim) is chunked
 
@@ -33,6 +32,11 @@ def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest
     # many short ones, whole: 108 / 75, 64 / 50, 85 / 53
     (hip.STATE_SPACE, 4000, 20, 400, 32, 64, 64, 0, 0), (hip.LINEAR_CHANNEL, 2512, 22, 195, 8, 128, 128, 0, 0),
     (hip.LINEAR_HEAD, 1017, 22, 94, 16, 128, 128, 0, 0),
+    # the same against the walk, where chunks are further behind: 194 / 119, 298 / 214, 131 / 80, 97 / 45
+    (hip.LINEAR_CHANNEL, 6000, 24, 250, 16, 128, 128, 0, 0), (hip.LINEAR_HEAD, 8964, 54, 166, 16, 128, 128, 0, 0),
+    (hip.STATE_SPACE, 960, 63, 300, 32, 64, 64, 0, 0), (hip.LINEAR_CHANNEL, 1196, 11, 173, 16, 96, 96, 0, 0),
+    # many heads beside short rows: walk / segments 26 / 34
+    (hip.LINEAR_CHANNEL, 710, 23, 50, 64, 32, 64, -1, -1),
     # few short ones, whose chains of 32 rows would be longer: 23 / 36, 32 / 44, 26 / 34
     (hip.LINEAR_HEAD, 215, 1, 215, 16, 64, 128, -1, -1), (hip.LINEAR_CHANNEL, 230, 1, 230, 32, 128, 128, -1, -1),
     (hip.STATE_SPACE, 668, 2, 374, 16, 64, 64, -1, -1)])

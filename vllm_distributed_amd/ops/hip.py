@@ -1647,36 +1647,48 @@ CHUNK_MIN_ROWS = 48
 CHUNK_SCRATCH_BYTES = 1 << 30
 
 
-# Per recurrence, in us.  The chunked kernels: a call, a link of 64 rows of the longest sequence (dim 128; three quarters of it
-# at 64), a chunk and head, the same per 128 x 128 of its keys and values.  The walk row by row: a call, a row of the longest
-# sequence, a row and head, the same per 128 x 128 of the state.
-CHUNK_COSTS = {LINEAR_HEAD: (24.5, 1.15, 0.020, 0.076, 3.1, 0.306, 0.00052, 0.00168),
-               LINEAR_CHANNEL: (24.0, 0.79, 0.036, 0.053, 5.3, 0.270, 0.00063, 0.00115),
-               STATE_SPACE: (21.3, 1.28, 0.027, 0.065, 4.9, 0.340, 0.00073, 0.00224),
-               DELTA_CHANNEL: (36.0, 2.04, 0.025, 0.122, 13.5, 0.396, 0.00068, 0.00239),
-               DELTA_HEAD: (24.0, 1.65, 0.015, 0.140, 15.9, 0.312, 0.00056, 0.00299)}
+# Per recurrence, in us.  The chunked kernels: a call; a link of 64 rows of the longest sequence, and of 128 keys; per chunk and head
+# the preparation of 128 keys, and the walk over them of 128 values, and of 128 values and 128 keys; the chunks that a sequence adds
+# to its rows'.  The walk row by row: a call, a row of the longest sequence, a row and head, the same per 128 x 128 of the state, the
+# rows that a sequence adds, and the power of (longest / average sequence) by which unequal ones leave the chip idle.  Fitted over
+# 8000 to 12000 calls of each kind, one after the other from Python: 1 - 100 sequences, alike, unequal, prompts beside decoded rows, the
+# longest of 48 rows and more, 2 - 64 heads, sizes 16 to 256, mild and strong decays.  Off by 9 to 18 % (root mean square), chunks of
+# many sequences that fill their last one badly by up to 25.
+CHUNK_COSTS = {LINEAR_HEAD: (18.8, 0.55, 1.74, 0.0201, 0.0230, 0.0423, 1.55, 3.9, 0.273, 0.00020, 0.00218, 3.1, 0.47),
+               LINEAR_CHANNEL: (17.2, 0.59, 1.61, 0.0220, 0.0163, 0.0491, 1.47, 6.1, 0.234, 0.00004, 0.00203, 1.0, 0.64),
+               STATE_SPACE: (18.2, 0.74, 1.28, 0.0162, 0.0236, 0.0367, 1.50, 4.5, 0.345, 0.00023, 0.00264, 3.9, 0.42),
+               DELTA_CHANNEL: (25.1, 0.17, 2.85, 0.0481, 0.0127, 0.0542, 1.30, 15.8, 0.374, 0.00061, 0.00294, 7.0, 0.18),
+               DELTA_HEAD: (21.3, 0.49, 2.36, 0.0383, 0.0317, 0.0291, 1.34, 14.1, 0.341, 0.00045, 0.00255, 6.8, 0.14)}
+
+
+def _chunk_and_walk(kind: int, rows: int, seqs: int, longest: int, heads: int, dim: int, vdim: int) -> Tuple[float, float]:
+    """Modelled times of the chunked kernels and of the walk row by row."""
+    call, link, link_keys, prep, share, share_keys, seq, walk_call, row, row_head, row_area, walk_seq, unequal = CHUNK_COSTS[kind]
+    keys, values = (0.5 if dim <= 64 else 1.0), max(vdim, 32) / 128
+    chunks = (rows / 64 + seq * seqs) * heads
+    chunked = call + chunks * prep * keys + math.hypot(longest / 64 * (link + link_keys * keys),
+                                                       chunks * values * (share + share_keys * keys))
+    lanes = 1 << max(dim - 1, 1).bit_length()                  # (the walk's keys: the next power of two)
+    idle = min(max(longest * seqs / max(rows, 1), 1.0), 8.0) ** unequal
+    return chunked, walk_call + math.hypot(longest * row, (rows + walk_seq * seqs) * heads * idle
+                                           * (row_head + row_area * lanes * vdim / 16384))
 
 
 @functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
 def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int,
                           aligned: bool = True) -> bool:
     """Whether ``seqs`` sequences with ``rows`` rows in all, at most ``max_rows`` in one (0: unknown), go through the chunked
-    kernels (``aligned``: their rows can be read 16 bytes at a time): modelled times in us, fitted on an MI355X over calls of
-    1 - 100 sequences, 2 - 64 heads and sizes 16 to 256 with mild and with strong decays.  Of 2680 such calls 18, most of them
-    short, come here although the walk is over 5 % faster, by 27 % at worst.  The walk row by row is a chain of dependent steps
-    per row of the longest sequence, and bound by issue where many sequences run; a chunk of 64 rows costs a link of a shorter
-    chain and its share of the chip, however few rows it holds and however small a head is (16 heads, dim 128: one prompt of 700
-    rows 79 against 297 us under the delta rule per channel, 60 rows of 8 heads 46 against 38; linear attention per channel of
-    24 x 250 rows 206 against 181; 63 sequences of 960 rows in all, 32 heads of 16 x 16: 121 against 81)."""
+    kernels (``aligned``: their rows can be read 16 bytes at a time), by the times of ``CHUNK_COSTS``.  Over the calls that those were
+    fitted on, and 7300 others in graphs, the delta rule's choice is 0.4 to 0.7 % above the faster of the two on average, over 5 %
+    above it in one call of 30 (58 prompts of 150 rows in chunks of 64, 16 heads: 343 / 323).  The walk row by row is a chain of dependent steps per row of the longest sequence, and bound by issue
+    where many sequences run; a chunk of 64 rows costs a link of a shorter chain and its share of the chip, however few rows it holds
+    and however small a head is (walk / chunks: 16 heads, dim 128, one prompt of 700 rows 298 / 63 us under the delta rule per channel,
+    64 heads, 97 rows 93 / 46; 16 heads of 16 x 16, 58 prompts of 155 rows 110 / 151)."""
     longest = max_rows if max_rows > 0 else rows // max(seqs, 1)
     if dim > CHUNK_MAX_DIM or longest < CHUNK_MIN_ROWS:
         return False
-    call, link, head, area, walk_call, row, row_head, row_area = CHUNK_COSTS[kind]
-    padded = 64 if dim <= 64 else 128
-    chunked = (call + longest / 64 * link * (0.5 + padded / 256)
-               + (rows / 64 + seqs) * heads * (head + area * padded * max(vdim, 32) / 16384)) * (1.0 if aligned else 1.2)
-    walk = walk_call + math.hypot(longest * row, rows * heads * (row_head + row_area * dim * vdim / 16384))
-    return chunked < walk
+    chunked, walk = _chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim)
+    return chunked * (1.0 if aligned else 1.2) < walk
 
 
 def _chunked(kind: int, x: torch.Tensor, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> bool:
@@ -1725,48 +1737,47 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
 
 
 # The recurrences without a delta rule over segments, in us: a call, a chunk of 32 rows (fixed, and per 128 x 128 of the state),
-# what a workgroup begins with, a chunk of the pass over the states alone; beside them the chunked kernels as in CHUNK_COSTS,
-# fitted over the calls that segments were measured on.
-SEGMENT_COSTS = {LINEAR_HEAD: (6.9, 2.42, 5.1, 7.1, 0.0, 1.18), LINEAR_CHANNEL: (8.3, 2.03, 3.9, 5.0, 0.62, 0.0),
-                 STATE_SPACE: (9.4, 2.20, 2.8, 5.4, 0.0, 0.91)}
-CHUNK_COSTS_BESIDE = {LINEAR_HEAD: (18.6, 0.89, 0.015, 0.078), LINEAR_CHANNEL: (16.3, 1.30, 0.007, 0.081),
-                      STATE_SPACE: (18.0, 1.18, 0.015, 0.060)}
+# what a workgroup begins with.  Fitted over 16000 timings of 4500 calls of each kind like those of CHUNK_COSTS, whole and with cuts of 96
+# to 480 rows: off by 13 % (under a decay per channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the
+# time, which only the kernel sees).
+SEGMENT_COSTS = {LINEAR_HEAD: (2.1, 3.26, 4.10, 5.5), LINEAR_CHANNEL: (4.0, 2.40, 3.11, 3.9), STATE_SPACE: (4.3, 2.55, 2.18, 4.2)}
 
 
 @functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
 def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> int:
     """Rows at which sequences are cut into segments that run side by side (0: none is cut), or -1: the chunked kernels, whose
-    preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all segments run at a time,
-    by an estimate of how many there are, or 96 rows.  Modelled times on an MI355X, fitted over 980 timings of 220 calls (8 to 32
-    heads, 1 to 24 sequences, 30 to 7500 rows); as the model is off by 13 % (root mean square), segments where they are 15 to 20 %
-    ahead: 1.2 times as fast on average as the chunked kernels alone (one prompt of 7000 rows, 8 heads of 128 x 128, state space 237 against
-    87 us; five of 500 rows, 32 heads of 64 x 128, 111 against 137: not chosen)."""
+    preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all
+    segments run at a time, by an estimate of how many there are, or 96 rows.  A time is between the chain of the longest segment and
+    the share of the chip that all of them take.  Segments where their modelled time is 7 % ahead of the others':
+    over the calls of SEGMENT_COSTS the choice is 2.1 to 2.6 % above the fastest kernel on average (without segments 19 to 37), over 5 %
+    slower than without segments in one call of 60 with mild decays, of 5 with strong ones per channel (us without / with: one prompt
+    of 7000 rows, 8 heads of 128 x 128, state space 237 / 79; 16 sequences of 473 rows in all, 64 heads of 96 x 96, 114 / 59; 54 of
+    8964, 16 heads of 128 x 128, linear attention 298 / 214; 23 of 710, 64 heads of 32 x 64, per channel 26 / 34: not chosen)."""
     longest = max_rows if max_rows > 0 else -(-rows // max(seqs, 1))
     if longest < CHUNK_MIN_ROWS or dim > CHUNK_MAX_DIM or vdim > 256:     # (wider: more scratch than the chunks' operands)
         return -1
+    limit = 0.93 * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
+    begin, fixed, area, over = SEGMENT_COSTS[kind]
     dp, vp = 64 if dim <= 64 else 128, 64 if vdim <= 64 else -(-vdim // 128) * 128
-    call, link, head, per = CHUNK_COSTS_BESIDE[kind]
-    limit = call + longest / 64 * link * (0.5 + dp / 256) + (rows / 64 + seqs) * heads * (head + per * dp * vdim / 16384)
-    walk_call, row, row_head, row_area = CHUNK_COSTS[kind][4:]
-    limit = min(limit, walk_call + math.hypot(longest * row, rows * heads * (row_head + row_area * dim * vdim / 16384)))
-    limit *= 0.8 if kind == LINEAR_HEAD else 0.85
-    begin, fixed, area, over, state_fixed, state_area = SEGMENT_COSTS[kind]
     share = min(vp, 128) * dp / 16384              # of a workgroup in the largest state tile
     work = heads * max(vp // 128, 1) / (512 if share <= 0.25 else 256)           # of the workgroups that run at a time, a segment's
-    chunk, state = fixed + area * share, state_fixed + state_area * share
-    best, choice = begin + max(longest / 32 * chunk + over, ((rows / 32 + 0.5 * seqs) * chunk + seqs * over) * work), 0
-    others, unsure = (rows - longest) / max(seqs - 1, 1), 0.6 * math.sqrt(seqs - 1)
-    room = 1.0 / work - unsure - 0.5 * seqs        # segments of whole length that run at a time
+    chunk = fixed + area * share
+
+    def time(cut: int, segments: float) -> float:
+        return begin + ((cut / 32 * chunk + over) ** 1.5
+                        + (((rows / 32 + 0.8 * seqs) * chunk + segments * over) * work) ** 1.5) ** (2 / 3)
+    best, choice = time(longest, seqs), 0
+    others = (rows - longest) / max(seqs - 1, 1)
+    room = 1.0 / work - 0.6 * math.sqrt(seqs - 1) - 0.5 * seqs                   # segments of whole length that run at a time
     for cut in (96, max(96, int(rows / room / 32 + 1) * 32) if room > 0 else 96):
         if cut >= longest:
             continue
         segments = -(-longest // cut) + (seqs - 1) * (others / cut + 0.5)
-        turns = (segments + unsure) * work
-        turns = max(1, math.ceil(turns)) if turns < 4 else turns + 0.5
-        time = (begin + turns * (cut / 32 * chunk + over) + 0.5 * over
-                + max(1.0, (segments - seqs) * work) * (cut / 32 * state + over) + segments * heads * dp * vp / 16384 * 0.03)
-        if time < best:
-            best, choice = time, cut
+        more = max(segments - seqs, 1.0)           # (of the pass over the states alone; their sums go through memory)
+        cut_time = (time(cut, segments) + 5.0 + over * (1.0 + (more * work) ** 1.5) ** (2 / 3)
+                    + segments * heads * dp * vp / 16384 * 0.055)
+        if cut_time < best:
+            best, choice = cut_time, cut
     return choice if best < limit else -1
 
 
