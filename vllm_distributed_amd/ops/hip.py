@@ -1652,13 +1652,13 @@ CHUNK_SCRATCH_BYTES = 1 << 30
 # to its rows'.  The walk row by row: a call, a row of the longest sequence, a row and head, the same per 128 x 128 of the state, the
 # rows that a sequence adds, and the power of (longest / average sequence) by which unequal ones leave the chip idle.  Fitted over
 # 8000 to 12000 calls of each kind, one after the other from Python: 1 - 100 sequences, alike, unequal, prompts beside decoded rows, the
-# longest of 48 rows and more, 2 - 64 heads, sizes 16 to 256, mild and strong decays.  Off by 9 to 18 % (root mean square), chunks of
-# many sequences that fill their last one badly by up to 25.
-CHUNK_COSTS = {LINEAR_HEAD: (18.8, 0.55, 1.74, 0.0201, 0.0230, 0.0423, 1.55, 3.9, 0.273, 0.00020, 0.00218, 3.1, 0.47),
-               LINEAR_CHANNEL: (17.2, 0.59, 1.61, 0.0220, 0.0163, 0.0491, 1.47, 6.1, 0.234, 0.00004, 0.00203, 1.0, 0.64),
-               STATE_SPACE: (18.2, 0.74, 1.28, 0.0162, 0.0236, 0.0367, 1.50, 4.5, 0.345, 0.00023, 0.00264, 3.9, 0.42),
-               DELTA_CHANNEL: (25.1, 0.17, 2.85, 0.0481, 0.0127, 0.0542, 1.30, 15.8, 0.374, 0.00061, 0.00294, 7.0, 0.18),
-               DELTA_HEAD: (21.3, 0.49, 2.36, 0.0383, 0.0317, 0.0291, 1.34, 14.1, 0.341, 0.00045, 0.00255, 6.8, 0.14)}
+# longest of 48 rows and more, 2 - 64 heads, sizes 16 to 256, mild and strong decays (8 to 32 heads of 64 and 128 counting fivefold).
+# Off by 9 to 18 % (root mean square), chunks of many sequences that fill their last one badly by up to 25.
+CHUNK_COSTS = {LINEAR_HEAD: (18.6, 0.58, 1.71, 0.0204, 0.0236, 0.0419, 1.55, 3.7, 0.271, 0.00017, 0.00222, 3.7, 0.46),
+               LINEAR_CHANNEL: (16.8, 0.58, 1.63, 0.0223, 0.0167, 0.0480, 1.47, 6.3, 0.230, 0.00002, 0.00208, 1.0, 0.65),
+               STATE_SPACE: (17.8, 0.76, 1.26, 0.0166, 0.0241, 0.0357, 1.50, 4.3, 0.343, 0.00021, 0.00269, 4.2, 0.41),
+               DELTA_CHANNEL: (24.3, 0.22, 2.80, 0.0480, 0.0130, 0.0533, 1.32, 16.2, 0.377, 0.00059, 0.00294, 7.1, 0.18),
+               DELTA_HEAD: (20.9, 0.53, 2.34, 0.0392, 0.0314, 0.0287, 1.35, 14.3, 0.342, 0.00042, 0.00257, 7.0, 0.16)}
 
 
 def _chunk_and_walk(kind: int, rows: int, seqs: int, longest: int, heads: int, dim: int, vdim: int) -> Tuple[float, float]:
@@ -1738,9 +1738,9 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
 
 # The recurrences without a delta rule over segments, in us: a call, a chunk of 32 rows (fixed, and per 128 x 128 of the state),
 # what a workgroup begins with.  Fitted over 16000 timings of 4500 calls of each kind like those of CHUNK_COSTS, whole and with cuts of 96
-# to 480 rows: off by 13 % (under a decay per channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the
-# time, which only the kernel sees).
-SEGMENT_COSTS = {LINEAR_HEAD: (2.1, 3.26, 4.10, 5.5), LINEAR_CHANNEL: (4.0, 2.40, 3.11, 3.9), STATE_SPACE: (4.3, 2.55, 2.18, 4.2)}
+# to 480 rows, those of 8 to 32 heads of 64 and 128 counting fivefold: off by 10 to 11 % where the cut is the rule's (under a decay per
+# channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the time, which only the kernel sees).
+SEGMENT_COSTS = {LINEAR_HEAD: (1.6, 3.27, 4.12, 7.1), LINEAR_CHANNEL: (3.4, 2.37, 3.14, 5.4), STATE_SPACE: (4.0, 2.59, 2.15, 5.5)}
 
 
 @functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
@@ -1748,15 +1748,15 @@ def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim
     """Rows at which sequences are cut into segments that run side by side (0: none is cut), or -1: the chunked kernels, whose
     preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all
     segments run at a time, by an estimate of how many there are, or 96 rows.  A time is between the chain of the longest segment and
-    the share of the chip that all of them take.  Segments where their modelled time is 7 % ahead of the others':
-    over the calls of SEGMENT_COSTS the choice is 2.1 to 2.6 % above the fastest kernel on average (without segments 19 to 37), over 5 %
-    slower than without segments in one call of 60 with mild decays, of 5 with strong ones per channel (us without / with: one prompt
+    the share of the chip that all of them take.  Segments where their modelled time is 4 % ahead of the others':
+    over the calls of SEGMENT_COSTS the choice is 1.8 to 2.4 % above the fastest kernel on average (without segments 19 to 37), over 5 %
+    slower than without segments in one call of 45 with mild decays, of 5 with strong ones per channel (us without / with: one prompt
     of 7000 rows, 8 heads of 128 x 128, state space 237 / 79; 16 sequences of 473 rows in all, 64 heads of 96 x 96, 114 / 59; 54 of
     8964, 16 heads of 128 x 128, linear attention 298 / 214; 23 of 710, 64 heads of 32 x 64, per channel 26 / 34: not chosen)."""
     longest = max_rows if max_rows > 0 else -(-rows // max(seqs, 1))
     if longest < CHUNK_MIN_ROWS or dim > CHUNK_MAX_DIM or vdim > 256:     # (wider: more scratch than the chunks' operands)
         return -1
-    limit = 0.93 * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
+    limit = 0.96 * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
     begin, fixed, area, over = SEGMENT_COSTS[kind]
     dp, vp = 64 if dim <= 64 else 128, 64 if vdim <= 64 else -(-vdim // 128) * 128
     share = min(vp, 128) * dp / 16384              # of a workgroup in the largest state tile
@@ -1764,8 +1764,7 @@ def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim
     chunk = fixed + area * share
 
     def time(cut: int, segments: float) -> float:
-        return begin + ((cut / 32 * chunk + over) ** 1.5
-                        + (((rows / 32 + 0.8 * seqs) * chunk + segments * over) * work) ** 1.5) ** (2 / 3)
+        return begin + math.hypot(cut / 32 * chunk + over, ((rows / 32 + 0.8 * seqs) * chunk + segments * over) * work)
     best, choice = time(longest, seqs), 0
     others = (rows - longest) / max(seqs - 1, 1)
     room = 1.0 / work - 0.6 * math.sqrt(seqs - 1) - 0.5 * seqs                   # segments of whole length that run at a time
@@ -1774,8 +1773,8 @@ def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim
             continue
         segments = -(-longest // cut) + (seqs - 1) * (others / cut + 0.5)
         more = max(segments - seqs, 1.0)           # (of the pass over the states alone; their sums go through memory)
-        cut_time = (time(cut, segments) + 5.0 + over * (1.0 + (more * work) ** 1.5) ** (2 / 3)
-                    + segments * heads * dp * vp / 16384 * 0.055)
+        cut_time = (time(cut, segments) + 3.3 + (cut / 32 * chunk * 0.07 + over) * math.hypot(1.0, more * work)
+                    + segments * heads * dp * vp / 16384 * 0.052)
         if cut_time < best:
             best, choice = cut_time, cut
     return choice if best < limit else -1
