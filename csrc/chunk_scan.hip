@@ -1,4 +1,4 @@
-// Prompt portions of the recurrent mixers in chunks of 64 rows on the matrix cores, all in 32-bit floats, gfx950:
+// Prompt portions of the recurrent mixers in chunks of 64 rows on the matrix cores, values, products and sums of 32 bits, gfx950:
 //
 //   linear      S <- g S + k v^T ; o = S^T q                            (decayed linear attention, the state-space scan)
 //   delta rule  S <- g S ; u = b (v - S^T k) ; S <- S + k u^T ; o = S^T q
