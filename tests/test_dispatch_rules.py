@@ -45,6 +45,30 @@ def test_segments_run_where_they_are_faster(kind, rows, seqs, longest, heads, di
     assert least <= cut <= most and (cut <= 0 or cut % 32 == 0)
 
 
+@pytest.mark.parametrize("cut,seqs,heads,vdim,goes", [(0, 1 << 20, 7, 8, True), (0, 1 << 20, 8, 8, False), (0, 1 << 19, 8, 136, False),
+                                                      (96, 1, 65535, 16, True), (96, 1, 65536, 16, False)])
+def test_segments_leave_what_a_launch_cannot_hold_to_other_kernels(monkeypatch, cut, seqs, heads, vdim, goes):
+    import torch
+    handed = []
+
+    class Lib:
+        @staticmethod
+        def vdamd_segment_scan_floats(*sizes):
+            return 1
+
+        @staticmethod
+        def vdamd_segment_scan(*args):
+            handed.append(args)
+            return 0
+    monkeypatch.setattr(hip, "_LIB", Lib)
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "segment_rows", lambda *sizes: cut)
+    x, lens = torch.empty(1, heads * (16 + vdim)), torch.empty(seqs, dtype=torch.int32)
+    out = hip._segment_scan(hip.LINEAR_HEAD, x, 0, heads * 8, heads * 16, None, None, None, x, None, heads, heads, 8, vdim, x, lens, lens,
+                            lens, False, 1.0, 100)
+    assert (out is not None) is goes is bool(handed)
+
+
 @pytest.mark.parametrize("batch,heads,keys,captured,splits", [
     # (whole against split in us) 13.5 / 18 from Python; in a graph 12.5 / 8.5 and 9.3 / 9.0
     (1, 8, 800, False, 1), (1, 8, 800, True, 12), (8, 8, 520, True, 1), (1, 8, 512, True, 1), (1, 8, 1, False, 1),

@@ -1792,7 +1792,8 @@ def _segment_scan(kind: int, x, q_off: int, k_off: int, v_off: int, dt, dt_bias,
         return None
     segments = b if rows == 0 else (t + (rows - 1) * min(b, t)) // rows
     floats = int(_LIB.vdamd_segment_scan_floats(num_heads, dim, vdim)) * segments if rows else 0
-    if 8 * floats > CHUNK_SCRATCH_BYTES:           # (no more than chunk_scan_bytes, however many heads at a time that counts)
+    # (no more than chunk_scan_bytes, however many heads at a time that counts; workgroups that a launch can have)
+    if 8 * floats > CHUNK_SCRATCH_BYTES or num_heads > 65535 or segments * num_heads * -(-vdim // 128) >= 1 << 23:
         return None
     out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
     ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
