@@ -16,21 +16,25 @@ __device__ __forceinline__ float softplus_f(float x) {
   return x > 20.f ? x : l;
 }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-// e^(x + rest) for x from -200, where it is zero, up to zero, and a `rest` that x had no place for.  Cody and Waite's reduction (Software
-// Manual for the Elementary Functions, 1980): x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact,
-// and for |r| <= ln 2 / 2 a polynomial whose coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits,
-// root mean square / largest, x in -10 .. 0: 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
-__device__ __forceinline__ float exp_f(float x, float rest = 0.f) {
-  const bool gone = x < -200.f;                    // (a rest that is no number then, too)
-  x = gone ? -200.f : x;
+// e^x for x from -200 to zero, or of x and a `rest` that it had no place for.  Cody and Waite's reduction (Software Manual for the
+// Elementary Functions, 1980): x = n ln 2 + r with ln 2 in two pieces, the first short enough that n times it is exact, and for
+// |r| <= ln 2 / 2 a polynomial whose coefficients are a fit by weighted least squares (off by 5e-9).  Error against 64 bits, root
+// mean square / largest, x in -10 .. 0: 2.6e-8 / 7.4e-8 (the library's: 2.6e-8 / 8.3e-8)
+template <typename... Rest> __device__ __forceinline__ float exp_inside(float x, Rest... rest) {
   const float n = rintf(x * 1.44269504f);
-  const float r = fmaf(-n, 1.42860677e-6f, fmaf(-n, 0.693145752f, x)) + (gone ? 0.f : rest);
+  float r = fmaf(-n, 1.42860677e-6f, fmaf(-n, 0.693145752f, x));
+  ((r += rest), ...);
   float p = fmaf(r, 0.0013814529f, 0.008368751f);
   p = fmaf(r, p, 0.041668393f);
   p = fmaf(r, p, 0.1666652f);
   p = fmaf(r, p, 0.49999994f);
   p = fmaf(r, p, 1.f);
   return ldexpf(fmaf(r, p, 1.f), (int)n);
+}
+// the same for x below -200 too, where it is zero
+__device__ __forceinline__ float exp_f(float x, float rest = 0.f) {
+  const bool gone = x < -200.f;                    // (a rest that is no number then, too)
+  return exp_inside(gone ? -200.f : x, gone ? 0.f : rest);
 }
 // e^(-rate softplus(x)).  softplus(x) is softplus(-|x|) more than x where x > 0, and ln(1 + t) = 2 atanh(t / (2 + t)), whose series
 // converges for t <= 1 (arguments up to 1 / 3; the coefficients are those of a fit by Chebyshev polynomials, off by 1e-9).  What the
@@ -52,14 +56,12 @@ __device__ __forceinline__ float quotient(float a, float d) {
   const float r = __builtin_amdgcn_rcpf(d), q = a * r;
   return fmaf(fmaxf(fmaf(-d, q, a), -3.40282347e38f), r, q);
 }
-// x sigmoid(x), where sigmoid(x) = 1 / (1 + t), or t / (1 + t) below zero, with t = e^-|x|: that reduction in base two, -|x| log2(e) =
-// n + f with log2(e) in two pieces, and the instruction's 2^f.  No exponent is cut off but where t is zero, so that far below zero the
-// result goes to zero as the function does.  The quotient is the product with the reciprocal and what that leaves over, with what
-// 1 + t lost to rounding.  Error against 64 bits, root mean square, and of the product with the library's sigmoid: x in -8 .. 8 3.8e-8
-// and 4.5e-8, -20 .. -8 4.4e-8 and 4.6e-8, -60 .. -20 3.7e-8 and 4.4e-8, 8 .. 60 1.5e-8 and 1.8e-8
+// x sigmoid(x), where sigmoid(x) = 1 / (1 + t), or t / (1 + t) below zero, with t = e^-|x|.  No exponent is cut off but where t is zero,
+// so that far below zero the result goes to zero as the function does.  The quotient is the product with the reciprocal and what that
+// leaves over, with what 1 + t lost to rounding.  Error against 64 bits, root mean square, and of the product with the library's
+// sigmoid: x in -8 .. 8 3.8e-8 and 4.5e-8, -20 .. -8 4.4e-8 and 4.6e-8, -60 .. -20 3.7e-8 and 4.4e-8, 8 .. 60 1.5e-8 and 1.8e-8
 __device__ __forceinline__ float silu_f(float x) {
-  const float y = __builtin_amdgcn_fmed3f(-fabsf(x), -200.f, 0.f), n = rintf(y * 1.44269502f);
-  const float t = ldexpf(__builtin_amdgcn_exp2f(fmaf(y, 1.92596303e-8f, fmaf(y, 1.44269502f, -n))), (int)n);
+  const float t = exp_inside(__builtin_amdgcn_fmed3f(-fabsf(x), -200.f, 0.f));
   const float d = 1.f + t, left_out = t - (d - 1.f), a = x < 0.f ? t : 1.f, r = __builtin_amdgcn_rcpf(d), s = a * r;
   return x * fmaf(fmaf(-left_out, s, fmaf(-d, s, a)), r, s);
 }
@@ -68,7 +70,8 @@ __device__ __forceinline__ float silu_f(float x) {
 // formed, each exact, with 32-bit sums; the three left out are below 2^-21 of the product (1.9e-8 root mean square, where a rounding
 // of the product is 2.5e-8), with either sign (the first third is about rounded, so that the second is as often below zero as above:
 // cut off without that, every product would be 2^-24 too small).  From 3.389e38 on, 0.4 % below the largest number, the first third
-// rounds to infinity, and so does the value.  Words of two values all the way: v_cvt_pk_bf16_f32 takes 12 cycles of a SIMD, what is here 2 to 3 each.
+// rounds to infinity, and so does the value.  Words of two values all the way: v_cvt_pk_bf16_f32 takes 12 cycles of a SIMD, what is
+// here 2 to 3 each.
 struct Thirds { bf16x8 h, m, l; };
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned bits(float v) { return __builtin_bit_cast(unsigned, v); }
