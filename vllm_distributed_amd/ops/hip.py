@@ -1680,9 +1680,9 @@ def chunk_scan_profitable(kind: int, rows: int, seqs: int, max_rows: int, heads:
     """Whether ``seqs`` sequences with ``rows`` rows in all, at most ``max_rows`` in one (0: unknown), go through the chunked
     kernels (``aligned``: their rows can be read 16 bytes at a time), by the times of ``CHUNK_COSTS``.  Over the calls that those were
     fitted on, and 7300 others in graphs, the delta rule's choice is 0.4 to 0.7 % above the faster of the two on average, over 5 %
-    above it in one call of 30 (58 prompts of 150 rows in chunks of 64, 16 heads: 343 / 323).  The walk row by row is a chain of dependent steps per row of the longest sequence, and bound by issue
-    where many sequences run; a chunk of 64 rows costs a link of a shorter chain and its share of the chip, however few rows it holds
-    and however small a head is (walk / chunks: 16 heads, dim 128, one prompt of 700 rows 298 / 63 us under the delta rule per channel,
+    above it in one call of 30 (58 prompts of 150 rows in chunks of 64, 16 heads: 343 / 323).  The walk row by row is a chain of dependent
+    steps per row of the longest sequence, and bound by issue where many sequences run; a chunk of 64 rows costs a link of a shorter
+    chain and its share of the chip, however few rows it holds and however small a head is (walk / chunks: 16 heads, dim 128, one prompt of 700 rows 298 / 63 us under the delta rule per channel,
     64 heads, 97 rows 93 / 46; 16 heads of 16 x 16, 58 prompts of 155 rows 110 / 151)."""
     longest = max_rows if max_rows > 0 else rows // max(seqs, 1)
     if dim > CHUNK_MAX_DIM or longest < CHUNK_MIN_ROWS:
@@ -1739,8 +1739,12 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
 # The recurrences without a delta rule over segments, in us: a call, a chunk of 32 rows (fixed, and per 128 x 128 of the state),
 # what a workgroup begins with.  Fitted over 16000 timings of 4500 calls of each kind like those of CHUNK_COSTS, whole and with cuts of 96
 # to 480 rows, those of 8 to 32 heads of 64 and 128 counting fivefold: off by 10 to 11 % where the cut is the rule's (under a decay per
-# channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the time, which only the kernel sees).
-SEGMENT_COSTS = {LINEAR_HEAD: (1.6, 3.27, 4.12, 7.1), LINEAR_CHANNEL: (3.4, 2.37, 3.14, 5.4), STATE_SPACE: (4.0, 2.59, 2.15, 5.5)}
+# channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the time, which only the kernel sees).  Last, the
+# part of the others' modelled time below which segments are taken: of 393 calls of linear attention, 8 to 32 heads, prompts of 1 to 24
+# sequences, 17 were over 2 % slower than without segments with 0.96 (at worst 107 us / 79) and 3 with 0.88 (at worst 1.08 times), with
+# the same sum of times; per channel and in the state space 12 of 450 and 6 of 417 are, and less would lose more than it saves.
+SEGMENT_COSTS = {LINEAR_HEAD: (1.6, 3.27, 4.12, 7.1, 0.88), LINEAR_CHANNEL: (3.4, 2.37, 3.14, 5.4, 0.96),
+                 STATE_SPACE: (4.0, 2.59, 2.15, 5.5, 0.96)}
 
 
 @functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
@@ -1748,16 +1752,16 @@ def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim
     """Rows at which sequences are cut into segments that run side by side (0: none is cut), or -1: the chunked kernels, whose
     preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all
     segments run at a time, by an estimate of how many there are, or 96 rows.  A time is between the chain of the longest segment and
-    the share of the chip that all of them take.  Segments where their modelled time is 4 % ahead of the others':
-    over the calls of SEGMENT_COSTS the choice is 1.8 to 2.4 % above the fastest kernel on average (without segments 19 to 37), over 5 %
+    the share of the chip that all of them take.  Segments where their modelled time is 4 to 12 % ahead of the others':
+    over the calls of SEGMENT_COSTS the choice is about 2 % above the fastest kernel on average (without segments 19 to 37), over 5 %
     slower than without segments in one call of 45 with mild decays, of 5 with strong ones per channel (us without / with: one prompt
     of 7000 rows, 8 heads of 128 x 128, state space 237 / 79; 16 sequences of 473 rows in all, 64 heads of 96 x 96, 114 / 59; 54 of
     8964, 16 heads of 128 x 128, linear attention 298 / 214; 23 of 710, 64 heads of 32 x 64, per channel 26 / 34: not chosen)."""
     longest = max_rows if max_rows > 0 else -(-rows // max(seqs, 1))
     if longest < CHUNK_MIN_ROWS or dim > CHUNK_MAX_DIM or vdim > 256:     # (wider: more scratch than the chunks' operands)
         return -1
-    limit = 0.96 * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
-    begin, fixed, area, over = SEGMENT_COSTS[kind]
+    begin, fixed, area, over, ahead = SEGMENT_COSTS[kind]
+    limit = ahead * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
     dp, vp = 64 if dim <= 64 else 128, 64 if vdim <= 64 else -(-vdim // 128) * 128
     share = min(vp, 128) * dp / 16384              # of a workgroup in the largest state tile
     work = heads * max(vp // 128, 1) / (512 if share <= 0.25 else 256)           # of the workgroups that run at a time, a segment's
