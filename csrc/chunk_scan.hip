@@ -191,8 +191,10 @@ __device__ __forceinline__ int chunks_before(const int* qsl, int B, int seq) {
 // rows, 16 000 go into A and L of the last 16 rows, 17 000 into U, W and the inverse, 8 000 into norms and running products (16 heads,
 // 8017 rows, a decay per channel).  There 150 us; 195 with the library's exponentials and logarithm (a third of its instructions)
 // and with U and W by substitution in fp32, W stored as it left the accumulators, four bytes a lane.
+// 64 keys: three workgroups to a compute unit, which takes 168 registers; with the 172 that the compiler likes best a decay per head
+// has two, 3736 rows of 32 heads 82 us, now 71 (fp32 rows would not fit, and keep two).
 template <typename T, int KIND, int DP>
-__global__ __launch_bounds__(256, 2) void chunk_prep_kernel(ChunkArgs a) {
+__global__ __launch_bounds__(256, DP > 64 || sizeof(T) == 4 ? 2 : 3) void chunk_prep_kernel(ChunkArgs a) {
   constexpr bool DELTA = KIND >= DELTA_CHANNEL, CHAN = KIND == LINEAR_CHANNEL || KIND == DELTA_CHANNEL;
   constexpr int KB = DP / 16, NP = CHAN ? KB * 4 : 1, LD = DP + 4, LM = C + 4, LT = C + 8;
   constexpr Layout L0 = layout_of(DP, 0, false);

@@ -765,6 +765,31 @@ def test_hot_attention_kernels_fit_the_register_file(tmp_path):
     assert all(v <= 160 for k, v in spilled.items() if "prefill_lds" in k), spilled
 
 
+def test_the_preparation_of_64_keys_runs_three_workgroups_to_a_compute_unit(tmp_path):
+    """Of four waves each, one to a SIMD: 168 of its 512 registers, a third of the LDS, and nothing in scratch memory.  (Where it had
+    four registers more, two ran, and prompts through the delta rule took up to 17 % longer.)"""
+    import re
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    from vllm_distributed_amd import build
+    assert "chunk_scan.hip" in build.EXACT_MATH_SOURCES
+    asm = tmp_path / "chunk_scan.s"
+    flags = [f for f in build.HIP_FLAGS if f != "-ffast-math"]
+    subprocess.run([hipcc, "-S", "--cuda-device-only", *flags, os.path.join(build.CSRC, "chunk_scan.hip"), "-o", str(asm)],
+                   check=True, capture_output=True, timeout=600)
+    seen = 0
+    for m in re.finditer(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", asm.read_text(), re.S):
+        size = lambda what: int(re.search(what + r" (\d+)", m.group(2)).group(1))
+        if re.search(r"chunk_prep_kernelIDF16b?_?Li[34]ELi64E", m.group(1)):
+            seen += 1
+            assert size("amdhsa_next_free_vgpr") <= 168 and size("group_segment_fixed_size") <= 160 * 1024 // 3, m.group(1)
+        assert size("private_segment_fixed_size") == 0, m.group(1)
+    assert seen == 4                                           # bf16 and fp16, a decay per channel and per head
+
+
 def test_eagle_head_checkpoint_in_the_authors_layout(tmp_path):
     """EAGLE's published head checkpoints name their tensors without a ``model.`` prefix, carry a copy of the
     embedding, ``fc`` with a bias, one decoder layer without an input norm, and no LM head: the file loads, the
