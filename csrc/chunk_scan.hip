@@ -1098,16 +1098,11 @@ __global__ __launch_bounds__(512, 2) void chunk_walk_kernel(float* __restrict__ 
 }
 
 template <typename T, int KIND>
-int launch(const ChunkArgs& a, int chunks, float* out, float* state, const int* slots, const int* seq_lens, const float* d_skip,
-           float scale, hipStream_t stream) {
+int launch(const ChunkArgs& a, int chunks, int cols, float* out, float* state, const int* slots, const int* seq_lens,
+           const float* d_skip, float scale, hipStream_t stream) {
   constexpr bool DELTA = KIND >= DELTA_CHANNEL;
   const dim3 prep(chunks, a.nh);
   const long pairs = ((long)a.B * a.nh + 7) / 8 * 8;
-  // 32 columns per workgroup where that still leaves one for every compute unit; delta rule, us at 32 and 16 columns: 16 heads of
-  // 128 x 128, 8000 rows of two prompts (128 workgroups of 32) 350 / 284, of three (192) 219 / 242, of five 173 / 223; 64 keys, where two
-  // workgroups of 16 columns fit a compute unit, 32 heads of 128 columns, 4000 rows of two (256) 132 / 113, of four (512) 97 / 99
-  const int enough = !DELTA ? 256 : a.dim > 64 ? 160 : 512;
-  const int cols = pairs * (a.VP / 32) >= enough ? 32 : 16;
   const dim3 walk((unsigned)(pairs * (a.VP / cols)));
 #define WALK(DP_, NC_)                                                                                                       \
   hipLaunchKernelGGL((chunk_walk_kernel<DP_, DELTA, NC_>), walk, dim3(512), 0, stream, out, a.ws, a.ws_stride, state, slots, \
@@ -1135,14 +1130,17 @@ VDAMD_API long vdamd_chunk_scan_floats(int kind, int dim, int vdim) {
 
 // Heads h0 .. h0 + nh - 1 of one call.  x [T, x_stride] of type dtype with q, k (of group 0) and v (of head 0) at the three
 // columns; dt / beta rows of the same type; out [T, H * vdim] fp32, state [slots, H, dim, vdim] fp32; `chunks`: a bound on the
-// batch's chunks of 64 rows; ws: chunks * nh * vdamd_chunk_scan_floats floats, 16-byte aligned; dim <= 128
+// batch's chunks of 64 rows; ws: chunks * nh * vdamd_chunk_scan_floats floats, 16-byte aligned; dim <= 128; cols: columns of a
+// workgroup of the walk, 16 or 32
 VDAMD_API int vdamd_chunk_scan(float* out, int kind, const void* x, long x_stride, int q_off, int k_off, int v_off,
                                const void* beta, long beta_stride, const void* dt, long dt_stride, const float* dt_bias,
                                const float* a_log, const float* decay, const float* d_skip, float* ws, int chunks, float* state,
                                const int* slots, const int* qsl, const int* seq_lens, int B, int H, int G, int dim, int vdim,
-                               int h0, int nh, int silu, float eps, float scale, int dtype, hipStream_t stream) {
+                               int h0, int nh, int cols, int silu, float eps, float scale, int dtype, hipStream_t stream) {
   if (B <= 0 || chunks <= 0 || nh <= 0) return 0;
-  if (H <= 0 || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || h0 < 0 || h0 + nh > H || nh > 65535) return 1;
+  if (H <= 0 || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || h0 < 0 || h0 + nh > H || nh > 65535 ||
+      (cols != 16 && cols != 32))
+    return 1;
   ChunkArgs a{};
   a.x = x; a.x_stride = x_stride; a.q_off = q_off; a.k_off = k_off; a.v_off = v_off;
   a.beta = beta; a.beta_stride = beta_stride; a.dt = dt; a.dt_stride = dt_stride; a.dt_bias = dt_bias; a.a_log = a_log;
@@ -1155,13 +1153,13 @@ VDAMD_API int vdamd_chunk_scan(float* out, int kind, const void* x, long x_strid
           (kind != DELTA_CHANNEL || (dt_stride % per == 0 && (uintptr_t)dt % 16 == 0)) &&
           (kind != LINEAR_CHANNEL || (uintptr_t)decay % 16 == 0);
   a.vvec = rows16 && vdim % per == 0 && v_off % per == 0;
-#define KINDS(T)                                                                                                         \
-  switch (kind) {                                                                                                        \
-    case LINEAR_HEAD: return launch<T, LINEAR_HEAD>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);       \
-    case LINEAR_CHANNEL: return launch<T, LINEAR_CHANNEL>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream); \
-    case STATE_SPACE: return launch<T, STATE_SPACE>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);       \
-    case DELTA_CHANNEL: return launch<T, DELTA_CHANNEL>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);   \
-    case DELTA_HEAD: return launch<T, DELTA_HEAD>(a, chunks, out, state, slots, seq_lens, d_skip, scale, stream);         \
+#define KINDS(T)                                                                                                               \
+  switch (kind) {                                                                                                              \
+    case LINEAR_HEAD: return launch<T, LINEAR_HEAD>(a, chunks, cols, out, state, slots, seq_lens, d_skip, scale, stream);       \
+    case LINEAR_CHANNEL: return launch<T, LINEAR_CHANNEL>(a, chunks, cols, out, state, slots, seq_lens, d_skip, scale, stream); \
+    case STATE_SPACE: return launch<T, STATE_SPACE>(a, chunks, cols, out, state, slots, seq_lens, d_skip, scale, stream);       \
+    case DELTA_CHANNEL: return launch<T, DELTA_CHANNEL>(a, chunks, cols, out, state, slots, seq_lens, d_skip, scale, stream);   \
+    case DELTA_HEAD: return launch<T, DELTA_HEAD>(a, chunks, cols, out, state, slots, seq_lens, d_skip, scale, stream);         \
   }
   switch (dtype) {
     case DT_BF16: KINDS(bf16_t) break;

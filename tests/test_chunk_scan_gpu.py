@@ -230,6 +230,19 @@ def test_what_is_not_finite_stays_in_its_row_and_behind(op, what, value, heads, 
 
 
 @pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 64, 32), (2, 128, 136), (1, 128, 16)])
+def test_columns_of_the_walk_are_the_same_numbers_by_16_and_by_32(monkeypatch, op, heads, dim, vdim):
+    c = _case(op, heads, 1 if op == "state_space" else heads, dim, vdim, [130, 64, 1, 200], [130, 80, 9, 200], torch.bfloat16, 31)
+    got = []
+    for columns in (16, 32):
+        monkeypatch.setattr(hip, "chunk_columns", lambda *sizes: columns)
+        got.append(_run(c, True))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    want, want_state = _rows64(c)
+    assert _off(got[1][0], want) < 3e-6 and _off(got[1][1], want_state) < 3e-6
+
+
+@pytest.mark.parametrize("op", OPS)
 @pytest.mark.parametrize("new", [[700, 300, 1, 1], [900] + [1] * 40])
 @pytest.mark.parametrize("chunked", [True, None])
 def test_the_memory_profile_holds_what_a_step_allocates(monkeypatch, op, new, chunked):

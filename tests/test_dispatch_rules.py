@@ -22,6 +22,24 @@ def test_chunked_recurrences_run_where_they_are_faster(kind, rows, seqs, longest
     assert hip.chunk_scan_profitable(kind, rows, seqs, longest, heads, dim, vdim) is chunked
 
 
+@pytest.mark.parametrize("kind,rows,seqs,longest,heads,dim,vdim,columns", [
+    # prompts alike, and one longer than the others (32 / 16 columns, us): 128 / 160, 119 / 147; 176 / 145, 65 / 56, 161 / 134, 75 / 74
+    (hip.DELTA_HEAD, 7000, 5, 1400, 8, 128, 128, 32), (hip.DELTA_HEAD, 7000, 6, 1167, 8, 128, 128, 32),
+    (hip.DELTA_HEAD, 7000, 5, 2420, 8, 128, 128, 16), (hip.DELTA_HEAD, 1785, 5, 668, 8, 128, 128, 16),
+    (hip.DELTA_HEAD, 7000, 6, 2065, 8, 128, 128, 16), (hip.DELTA_HEAD, 6038, 3, 2884, 16, 128, 128, 16),
+    # 118 / 136, 292 / 340, 220 / 242; one prompt 284 / 350; a prompt beside decoded rows is by itself
+    (hip.DELTA_HEAD, 7000, 7, 1200, 8, 128, 128, 32), (hip.DELTA_CHANNEL, 7000, 3, 2515, 16, 128, 128, 32),
+    (hip.DELTA_CHANNEL, 8017, 5, 2000, 16, 128, 128, 32), (hip.DELTA_CHANNEL, 8000, 1, 8000, 32, 128, 128, 16),
+    (hip.DELTA_CHANNEL, 2100, 101, 2000, 16, 128, 128, 16),
+    # the longest is not known: as if all were alike
+    (hip.DELTA_HEAD, 7000, 5, 0, 8, 128, 128, 32), (hip.DELTA_HEAD, 7000, 4, 0, 8, 128, 128, 16),
+    # 64 keys; kinds without a delta rule
+    (hip.DELTA_HEAD, 4000, 2, 2000, 32, 64, 128, 16), (hip.DELTA_HEAD, 4000, 4, 1000, 32, 64, 128, 32),
+    (hip.LINEAR_HEAD, 4000, 4, 3000, 16, 128, 128, 32), (hip.STATE_SPACE, 4000, 3, 3000, 16, 128, 128, 16)])
+def test_columns_of_the_chunked_walk(kind, rows, seqs, longest, heads, dim, vdim, columns):
+    assert hip.chunk_columns(kind, rows, seqs, longest, heads, dim, vdim) == columns
+
+
 @pytest.mark.parametrize("kind,rows,seqs,longest,heads,dim,vdim,least,most", [
     # decoded rows, heads and states the kernels are not built for
     (hip.LINEAR_CHANNEL, 256, 256, 1, 16, 128, 128, -1, -1), (hip.STATE_SPACE, 8000, 1, 8000, 16, 192, 128, -1, -1),

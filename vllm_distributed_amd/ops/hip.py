@@ -101,7 +101,7 @@ def load() -> ctypes.CDLL:
         "vdamd_expert_epilogue": [P, P, P, L, P, P, I, I, P, P, L, I, I, I, P],
         "vdamd_decay_linear_attention": [P, P, L, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "vdamd_channel_decay_attention": [P, P, L, P, P, P, P, P, I, I, I, I, F, I, I, I, P],
-        "vdamd_chunk_scan": [P, I, P, L, I, I, I, P, L, P, L, P, P, P, P, P, I, P, P, P, P] + [I] * 8 + [F, F, I, P],
+        "vdamd_chunk_scan": [P, I, P, L, I, I, I, P, L, P, L, P, P, P, P, P, I, P, P, P, P] + [I] * 9 + [F, F, I, P],
         "vdamd_segment_scan": [P, I, P, L, I, I, I, P, L, P, P, P, P, P, I, I, P, P, P, P] + [I] * 6 + [F, I, P],
         "vdamd_low_rank_decay": [P, P, L, P, P, I, I, I, F, I, P],
         "vdamd_weighted_relu_squared": [P, P, L, P, P, I, I, I, P],
@@ -1715,9 +1715,25 @@ def chunk_scan_bytes(kind: int, rows: int, seqs: int, heads: int, dim: int, vdim
     return out + 4 * floats * at_a_time
 
 
+def chunk_columns(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> int:
+    """Columns of the state that a workgroup of the chunked kernels' walk has, 16 or 32.  With 32 a chunk takes longer, 3.8 against 3.0
+    us under the delta rule, but the work in all is less: where the workgroups of 32 still give every compute unit one.  Delta rule
+    over more than 64 keys: where 136 of them are busy on average until the longest sequence's end.  us at 32 / 16 columns, 8 heads of
+    128 x 128, a decay per head: 7000 rows of five prompts alike (160 busy) 128 / 160, of five with one of 2420 (92) 176 / 145, of
+    seven with one of 1200 (187) 118 / 136, 3000 rows of seven with one of 686 (140) 70 / 69; 260 calls of 8 to 32 heads agree to 2 %.
+    64 keys, where two workgroups of 16 fit a compute unit, 32 heads of 128 columns, 4000 rows of two prompts (256) 132 / 113, of four
+    (512) 97 / 99."""
+    wide = -(-seqs * heads // 8) * 8 * -(-vdim // 32)
+    if kind in (DELTA_CHANNEL, DELTA_HEAD):
+        if dim <= 64:
+            return 32 if wide >= 512 else 16
+        return 32 if wide * rows >= 136 * seqs * max_rows and wide >= 136 else 16
+    return 32 if wide >= 256 else 16
+
+
 def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_bias, a_log, decay, d_skip, num_heads: int,
                 groups: int, dim: int, vdim: int, state, slots, query_start_loc, seq_lens, silu: bool, eps: float,
-                scale: float) -> torch.Tensor:
+                scale: float, max_rows: int) -> torch.Tensor:
     """One of the five recurrences over all sequences of a step (shapes checked by the caller).  The workspace (about 120 KB
     per chunk of 64 rows and head, the delta rule 150) is kept under ``CHUNK_SCRATCH_BYTES`` by taking the heads in turns."""
     t, b = x.shape[0], seq_lens.shape[0]
@@ -1732,7 +1748,8 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
             0 if beta is None else beta.stride(0), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(dt_bias), _ptr(a_log),
             _ptr(decay), _ptr(d_skip), ws.data_ptr(), chunks, state.data_ptr(), slots.data_ptr(),
             query_start_loc.data_ptr(), seq_lens.data_ptr(), b, num_heads, groups, dim, vdim, h0,
-            min(heads, num_heads - h0), int(silu), float(eps), float(scale), _dt(x), _stream()), "chunk_scan")
+            min(heads, num_heads - h0), chunk_columns(kind, t, b, max_rows, min(heads, num_heads - h0), dim, vdim), int(silu),
+            float(eps), float(scale), _dt(x), _stream()), "chunk_scan")
     return out
 
 
@@ -1837,7 +1854,7 @@ def decay_linear_attention(x: torch.Tensor, num_heads: int, dim: int, vdim: int,
                 return out
         if chunked or _chunked(kind, x, t, n, max_query_len, num_heads, dim, vdim):
             return _chunk_scan(kind, x, 0, qs, 2 * qs, None, None, None, None, rates, None, num_heads, num_heads, dim, vdim,
-                               state, slots, query_start_loc, seq_lens, silu, 0.0, scale)
+                               state, slots, query_start_loc, seq_lens, silu, 0.0, scale, max_query_len)
     out = torch.empty((t, num_heads * vdim), dtype=torch.float32, device=x.device)
     if decay.dim() == 2:
         _check(_LIB.vdamd_channel_decay_attention(
@@ -2120,7 +2137,7 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
         return _chunk_scan(kind, x, 0, g * dim, 2 * g * dim, beta, dt,
                            _f32_vec(dt_bias, dt.shape[1], "dt_bias"), _f32_vec(a_log, h, "a_log"), None, None, h, g, dim, vdim,
                            state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"),
-                           False, norm_eps, 1.0)
+                           False, norm_eps, 1.0, max_query_len)
     dev = x.device
     qn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
     kn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
@@ -2163,7 +2180,7 @@ def selective_scan(x, dt, num_heads: int, groups: int, vdim: int, n_state: int, 
             if out is not None:
                 return out
         if chunked or _chunked(STATE_SPACE, x, t, b, max_query_len, h, n, int(vdim)):
-            return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, *mine, 0.0, 1.0)
+            return _chunk_scan(STATE_SPACE, x, inner + g * n, inner, 0, None, dt, *mine, 0.0, 1.0, max_query_len)
     out = torch.empty((t, h * vdim), dtype=torch.float32, device=x.device)
     _check(_LIB.vdamd_selective_scan(
         out.data_ptr(), x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), _f32_vec(a_log, h, "a_log").data_ptr(),
