@@ -696,9 +696,9 @@ __global__ __launch_bounds__(256, DP > 64 || sizeof(T) == 4 ? 2 : 3) void chunk_
 // with two barriers (S is there, u is there), linear kinds with one (u = v comes from memory).  Left operands come from
 // memory straight into registers, where the next chunk's take the place of those just used.
 // Bound by the chain of a chunk: its matrix instructions (1.1 us of linear kinds at 16 columns, the delta rule 0.6 and as much
-// again to split its operands) and its 90 - 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes from the L2 through its
-// vector cache, about 64 bytes a clock; 45 - 61 KB per us of what comes from the memory-side cache) hardly overlap, as all
-// waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.0 us at 16 columns, 4.0 / 3.8 at 32 (the delta
+// again to split its operands) and its 90 - 115 KB of operands (0.6 - 0.95 us at the 119 - 143 KB per us that a compute unit takes
+// from the L2 through its vector cache, about 64 bytes a clock; 45 - 61 KB per us of what comes from the memory-side cache) hardly
+// overlap, as all waves wait at the same barriers.  Measured per chunk and workgroup 2.5 / 3.0 us at 16 columns, 4.0 / 3.8 at 32 (the delta
 // rule in fp32: 3.5 and 5.0; five prompts of 8017 rows, 16 heads: 221 against 177 us).
 template <int DP, int NC> struct LinearWalk {
   static constexpr int KB = DP / 16, NT = DP / 64, LD = DP + 4;
@@ -859,7 +859,10 @@ template <int DP, int NC> struct LinearWalk {
 };
 
 // The delta rule's, its fp32 products as thirds on the 16-bit instructions.  S and u cross through LDS as thirds, split once by
-// the wave that has them; what comes from memory is split where it is used.
+// the wave that has them; what comes from memory is split where it is used (in front of the barriers instead: half a percent of
+// calls' times; in the shadow of the products' chain, with loads a chunk ahead: 5 % slower).  A chain of few workgroups over 64 keys
+// is bound by its operands, 68 KB a chunk at 45 - 61 KB per us from the memory-side cache, and by what splits them: there the fp32
+// instructions were up to 10 % faster (5908 rows of 8 heads of 64 x 64 140 us and 154), and less exact.
 template <int DP, int NC> struct DeltaWalk {
   static constexpr int KB = DP / 16, KS = DP / 32, NT = DP / 64, LD = DP + 8, LU = C + 8;
   static constexpr Layout L0 = layout_of(DP, 0, false);
