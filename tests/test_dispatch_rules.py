@@ -53,7 +53,8 @@ def test_columns_of_the_chunked_walk(kind, rows, seqs, longest, heads, dim, vdim
     # the same against the walk, where chunks are further behind: 194 / 119, 298 / 214, 131 / 80, 97 / 45
     (hip.LINEAR_CHANNEL, 6000, 24, 250, 16, 128, 128, 0, 0), (hip.LINEAR_HEAD, 8964, 54, 166, 16, 128, 128, 0, 0),
     (hip.STATE_SPACE, 960, 63, 300, 32, 64, 64, 0, 0), (hip.LINEAR_CHANNEL, 1196, 11, 173, 16, 96, 96, 0, 0),
-    # a second round of segments, which the model does not see: chunked / segments 80 / 107, 72 / 88, 104 / 121
+    # one round of segments; where a second one would be nearly empty chunked / segments 80 / 107, 72 / 88, 104 / 121
+    (hip.LINEAR_HEAD, 6007, 3, 2434, 16, 128, 128, 384, 416), (hip.LINEAR_CHANNEL, 6007, 3, 2434, 16, 128, 128, 384, 416),
     (hip.LINEAR_HEAD, 6524, 13, 899, 16, 64, 64, -1, -1), (hip.LINEAR_HEAD, 5247, 10, 909, 16, 64, 64, -1, -1),
     (hip.LINEAR_HEAD, 1931, 1, 1931, 32, 128, 128, -1, -1),
     # many heads beside short rows: walk / segments 26 / 34

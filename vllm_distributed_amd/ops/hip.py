@@ -1756,39 +1756,41 @@ def _chunk_scan(kind: int, x, q_off: int, k_off: int, v_off: int, beta, dt, dt_b
 # The recurrences without a delta rule over segments, in us: a call, a chunk of 32 rows (fixed, and per 128 x 128 of the state),
 # what a workgroup begins with.  Fitted over 16000 timings of 4500 calls of each kind like those of CHUNK_COSTS, whole and with cuts of 96
 # to 480 rows, those of 8 to 32 heads of 64 and 128 counting fivefold: off by 10 to 11 % where the cut is the rule's (under a decay per
-# channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the time, which only the kernel sees).  Last, the
-# part of the others' modelled time below which segments are taken: of 393 calls of linear attention, 8 to 32 heads, prompts of 1 to 24
-# sequences, 17 were over 2 % slower than without segments with 0.96 (at worst 107 us / 79) and 3 with 0.88 (at worst 1.08 times), with
-# the same sum of times; per channel and in the state space 12 of 450 and 6 of 417 are, and less would lose more than it saves.
-SEGMENT_COSTS = {LINEAR_HEAD: (1.6, 3.27, 4.12, 7.1, 0.88), LINEAR_CHANNEL: (3.4, 2.37, 3.14, 5.4, 0.96),
-                 STATE_SPACE: (4.0, 2.59, 2.15, 5.5, 0.96)}
+# channel where decays are mild: 32 strong ones in a row are multiplied out, at twice the time, which only the kernel sees).  Then what a
+# chunk of 64 x 64 takes more where two workgroups share a compute unit, and the part of the others' modelled time below which segments
+# are taken.
+SEGMENT_COSTS = {LINEAR_HEAD: (1.6, 3.07, 3.87, 7.1, 1.1, 0.90), LINEAR_CHANNEL: (3.4, 2.37, 3.14, 5.4, 1.0, 0.98),
+                 STATE_SPACE: (4.0, 2.59, 2.15, 5.5, 1.0, 0.96)}
 
 
 @functools.lru_cache(maxsize=1024)              # (a step's layers ask with the same sizes)
 def segment_rows(kind: int, rows: int, seqs: int, max_rows: int, heads: int, dim: int, vdim: int) -> int:
     """Rows at which sequences are cut into segments that run side by side (0: none is cut), or -1: the chunked kernels, whose
     preparation of all chunks at once leaves a sequence the shorter chain, or the walk row by row.  A cut is the one with which all
-    segments run at a time, by an estimate of how many there are, or 96 rows.  A time is between the chain of the longest segment and
-    the share of the chip that all of them take.  Segments where their modelled time is 4 to 12 % ahead of the others':
-    over the calls of SEGMENT_COSTS the choice is about 2 % above the fastest kernel on average (without segments 19 to 37), over 5 %
-    slower than without segments in one call of 45 with mild decays, of 5 with strong ones per channel (us without / with: one prompt
-    of 7000 rows, 8 heads of 128 x 128, state space 237 / 79; 16 sequences of 473 rows in all, 64 heads of 96 x 96, 114 / 59; 54 of
-    8964, 16 heads of 128 x 128, linear attention 298 / 214; 23 of 710, 64 heads of 32 x 64, per channel 26 / 34: not chosen)."""
+    segments run at a time, by an estimate of how many there are (half a segment more for each sequence), or 96 rows.  A time is between
+    the chain of the longest segment and the share of the chip that all of them take.
+
+    Over 1050 calls of 8 to 32 heads of 64 and 128, prompts of 1 to 24 sequences, the choice is above the fastest kernel and cut by
+    1.5 % (linear attention), 1.0 (per channel) and 1.9 (state space) on average; 8, 1 and 2 of 350 calls each are over 5 % slower than
+    without segments, at worst 1.14 times.  us without / with: 6007 rows of three prompts, 16 heads of 128 x 128, linear attention
+    192 / 167; one prompt of 7000, 8 heads of 128 x 128, state space 237 / 74; 16 sequences of 473 rows in all, 64 heads of 96 x 96,
+    114 / 59; 54 of 8964, 16 heads of 128 x 128, linear attention 298 / 214; 23 of 710, 64 heads of 32 x 64, per channel 26 / 34: not
+    chosen."""
     longest = max_rows if max_rows > 0 else -(-rows // max(seqs, 1))
     if longest < CHUNK_MIN_ROWS or dim > CHUNK_MAX_DIM or vdim > 256:     # (wider: more scratch than the chunks' operands)
         return -1
-    begin, fixed, area, over, ahead = SEGMENT_COSTS[kind]
+    begin, fixed, area, over, shared, ahead = SEGMENT_COSTS[kind]
     limit = ahead * min(_chunk_and_walk(kind, rows, seqs, longest, heads, dim, vdim))
     dp, vp = 64 if dim <= 64 else 128, 64 if vdim <= 64 else -(-vdim // 128) * 128
     share = min(vp, 128) * dp / 16384              # of a workgroup in the largest state tile
     work = heads * max(vp // 128, 1) / (512 if share <= 0.25 else 256)           # of the workgroups that run at a time, a segment's
-    chunk = fixed + area * share
+    chunk = (fixed + area * share) * (shared if share <= 0.25 else 1.0)
 
     def time(cut: int, segments: float) -> float:
         return begin + math.hypot(cut / 32 * chunk + over, ((rows / 32 + 0.8 * seqs) * chunk + segments * over) * work)
     best, choice = time(longest, seqs), 0
     others = (rows - longest) / max(seqs - 1, 1)
-    room = 1.0 / work - 0.6 * math.sqrt(seqs - 1) - 0.5 * seqs                   # segments of whole length that run at a time
+    room = 1.0 / work - 0.5 * seqs                 # segments of whole length that run at a time
     for cut in (96, max(96, int(rows / room / 32 + 1) * 32) if room > 0 else 96):
         if cut >= longest:
             continue
