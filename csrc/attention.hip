@@ -247,8 +247,8 @@ __device__ __forceinline__ void attend_loaded(
 // one's values are multiplied, and its values while its keys are, in the registers that the products have just left.  A whole second
 // group would not fit three waves on a SIMD (202 registers, 3 to 8 % slower than four waves that wait for each group); this takes 152.
 // What bounds it is the memory; before, a wave waited for a group without one of its own under way, after about 130 vector
-// instructions for addresses.  us, before and after: e4m3, 64 rows of about 2000 keys, 8 heads of 128, 67 and 58.8, 200 of 1500 136
-// and 126, 7 of 700 14.9 and 11.5; 16 bits, 250 rows of 800 146 and 140, 2048 of 150 260 and 257, heads of 256, 100 of 500, 83 and 78.
+// instructions for addresses.  us with the write of the step's keys, before and after: e4m3, 64 rows of about 2000 keys, 8 heads of 128,
+// 71 and 63, 7 of 700, replayed, 11.4 and 10.7; 16 bits, 250 rows of 800 158 and 152, heads of 256, 100 of 500, 89 and 85.
 // With lanes that look up their own rows the loop gains nothing (64 rows of 700 keys in blocks of 16 26.0 and 26.6, e4m3 of 2000 51
 // and 57): those take a group at a time.
 template <typename T, int D, bool KV8, bool ONCE>

@@ -74,8 +74,8 @@ __host__ __device__ constexpr long state_floats(int DP, int VP) { return (long)D
 // and 90 matrix instructions of 16, two waves to a SIMD, and neither fills the other's time: 13 000 - 14 000 cycles a chunk, 5.5 us,
 // of which 3 300 are the barriers' waits.  16 waves of half the columns each spilled and were slower (104 -> 164 us, 6007 rows x 16 heads).
 // v_cvt_pk_bf16_f32, products of decays through LDS and a branch for each four values that look for what is not finite cost
-// 40 % more.  6007 rows of three prompts, 16 heads of 128 x 128, a decay per channel: states 37, starts 7.5, outputs 104 us, against
-// 67 (preparation) and 143 of the chunked kernels; one prompt of 7000 rows, 8 heads, state space: 87 against 237.
+// 40 % more.  6007 rows of three prompts, 16 heads of 128 x 128, a decay per channel: states 35, starts 8, outputs 97 us, against
+// 67 (preparation) and 143 of the chunked kernels; one prompt of 7000 rows, 8 heads, state space: 74 against 234.
 // LDS: 117 KB (137 where v has thirds): one workgroup to a compute unit; 64 x 64 two (54 - 79 KB, 128 registers).
 template <typename T, int KIND, bool X, int DP, int VW, bool OUT>
 __global__ __launch_bounds__(512, DP * VW > 64 * 64 ? 2 : 4) void segment_kernel(SegArgs a) {
