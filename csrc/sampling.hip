@@ -86,17 +86,19 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return t;
 }
 
-constexpr int BINS = 2048, CAP = 4096;
+// A row's histogram goes by a weight's exponent and its SHIFT1 = 17 lowest bits' neighbours above (six): a bin of a Gaussian row of 128k
+// has some 250 entries.  What is cut further goes by the next eleven bits, and by the last six
+constexpr int BINS1 = 8192, SHIFT1 = 17, BINS = 2048, SHIFT2 = 6, CAP = 4096;
 constexpr unsigned NORMAL_END = 0x40000000u;     // bits of 2.0: weights are at most 1; NaN and infinity lie above
 
 // Weights (positive floats) by the leading bits of their representation: how many, and the sum of the bits below -
 // whole numbers, so any order of additions gives the same.  Up to 2^22 elements both share one 64-bit word (19 low bits
 // times 2^22 stays under 2^41), a single LDS atomic per element; WIDE keeps them apart.
-template <bool WIDE> struct Hist {
-  unsigned long long sum[BINS];
-  unsigned cnt[WIDE ? BINS : 1];
+template <bool WIDE, int N> struct Hist {
+  unsigned long long sum[N];
+  unsigned cnt[WIDE ? N : 1];
   __device__ void clear() {
-    for (int i = threadIdx.x; i < BINS; i += ST) { sum[i] = 0; if (WIDE) cnt[i] = 0; }
+    for (int i = threadIdx.x; i < N; i += ST) { sum[i] = 0; if (WIDE) cnt[i] = 0; }
   }
   __device__ void add(int bin, unsigned low) {
     if (WIDE) { atomicAdd(&sum[bin], (unsigned long long)low); atomicAdd(&cnt[bin], 1u); }
@@ -116,77 +118,115 @@ __device__ __forceinline__ int lsb_of(unsigned bits) { return (int)max(bits >> 2
 // what sample_by_counts keeps beside the counts
 struct CountShared { unsigned low, inf, lo, hi, counted, of_stretch[128]; };
 struct SampleShared {
-  double wmass[16];
-  unsigned wcnt[16];
+  double wmass[2][16];
+  unsigned wcnt[2][16];
+  int wbest[2][16];
   double mass, above_mass;
   unsigned above_cnt, cnt, n_list;
   int best, n, token, bad;
 };
 
+// The waves' words take turns in two places, so that a step needs no barrier to have its words read before the next one's are written:
+// between two uses of a place lies the barrier of the step between.
+typedef unsigned Turn;
+
 // exclusive scan of (count, mass) over the block in thread order; totals to every thread (by shuffles, which go through LDS, a row's
-// two scans of sample_by_counts took 2.5 us more)
-__device__ __forceinline__ void block_scan(unsigned c, double m, unsigned& ec, double& em, double& total, SampleShared& s) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+// two scans of sample_by_counts took 2.5 us more).  The waves' totals, one a lane, are scanned by every wave: sixteen conditional
+// additions of doubles in each of sixteen waves took 0.8 us
+__device__ __forceinline__ void block_scan(unsigned c, double m, unsigned& ec, double& em, double& total, SampleShared& s, Turn& turn) {
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned ic = (unsigned)wave_scan((int)c);
   const double im = wave_scan(m);
-  if (lane == 63) { s.wcnt[wid] = ic; s.wmass[wid] = im; }
+  unsigned* const wcnt = s.wcnt[turn & 1];
+  double* const wmass = s.wmass[turn & 1];
+  ++turn;
+  if (lane == 63) { wcnt[wid] = ic; wmass[wid] = im; }
   __syncthreads();
-  unsigned bc = 0;
-  double bm = 0, all = 0;
-  for (int w = 0; w < 16; ++w) {
-    if (w < wid) { bc += s.wcnt[w]; bm += s.wmass[w]; }
-    all += s.wmass[w];
-  }
+  const bool one = lane < 16;
+  const unsigned tc = (unsigned)wave_scan(one ? (int)wcnt[lane & 15] : 0);
+  const double tm = wave_scan(one ? wmass[lane & 15] : 0.0);
+  auto of = [&](double v, int l) {
+    const unsigned long long w = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)w, l), hi = __builtin_amdgcn_readlane((unsigned)(w >> 32), l);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  };
+  const unsigned bc = wid ? (unsigned)__builtin_amdgcn_readlane((int)tc, wid - 1) : 0u;
+  const double bm = wid ? of(tm, wid - 1) : 0.0;
   ec = bc + ic - c;
   em = bm + im - m;
-  total = all;
+  total = of(tm, 15);
+}
+// the largest of the threads' numbers, which rise with the threads of a wave (-1: none)
+__device__ __forceinline__ int block_last(int mine, SampleShared& s, Turn& turn) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long those = __ballot(mine >= 0);
+  int* const wbest = s.wbest[turn & 1];
+  ++turn;
+  if (those ? (those >> lane) == 1ull : lane == 0) wbest[threadIdx.x >> 6] = mine;
   __syncthreads();
+  int best = wbest[lane & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    const int other = o == 8 ? __builtin_amdgcn_update_dpp(0, best, 0x128, 0xf, 0xf, true)
+                    : o == 4 ? __builtin_amdgcn_update_dpp(0, best, 0x124, 0xf, 0xf, true)
+                    : o == 2 ? __builtin_amdgcn_update_dpp(0, best, 0x4E, 0xf, 0xf, true)
+                             : __builtin_amdgcn_update_dpp(0, best, 0xB1, 0xf, 0xf, true);
+    best = max(best, other);
+  }
+  return __builtin_amdgcn_readfirstlane(best);
 }
 
-// A histogram's two bins of each thread, the heaviest of all first: counts, masses, and what lies in front of them.  Bins hold the
+// A histogram's bins of each thread, the heaviest of all first: counts, masses, and what lies in front of them.  Bins hold the
 // bits `prefix | bin << shift ..`.
-struct Bins {
-  unsigned c[2], ec;
-  double m[2], em, total;
+template <int PER> struct Bins {
+  unsigned c[PER], ec;
+  double m[PER], em, total;
 };
-template <bool WIDE> __device__ __forceinline__ Bins sum_bins(const Hist<WIDE>& h, unsigned prefix, int shift, SampleShared& s) {
-  Bins t;
+template <bool WIDE, int N>
+__device__ __forceinline__ Bins<N / ST> sum_bins(const Hist<WIDE, N>& h, unsigned prefix, int shift, SampleShared& s, Turn& turn) {
+  Bins<N / ST> t;
+  unsigned c = 0;
+  double m = 0;
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int bin = BINS - 1 - (2 * (int)threadIdx.x + e);
+  for (int e = 0; e < N / ST; ++e) {
+    const int bin = N - 1 - (N / ST * (int)threadIdx.x + e);
     const unsigned bits = prefix | ((unsigned)bin << shift);
     t.c[e] = h.count(bin);
     t.m[e] = t.c[e] ? ((double)t.c[e] * sig_of(bits) + (double)h.lows(bin)) * pow2(lsb_of(bits)) : 0.0;
+    c += t.c[e];
+    m += t.m[e];
   }
-  block_scan(t.c[0] + t.c[1], t.m[0] + t.m[1], t.ec, t.em, t.total, s);
+  block_scan(c, m, t.ec, t.em, t.total, s, turn);
   return t;
 }
 // The lowest non-empty bin (at or above `first`) in front of which, `above` included, fewer than K elements and less than M of mass
 // lie: its index, count and what lies above it go to `s` (best = -1: none).
-__device__ __forceinline__ void find_bin(const Bins& t, int first, unsigned above_cnt, double above_mass, unsigned K, double M,
-                                         SampleShared& s) {
-  if (threadIdx.x == 0) s.best = -1;
-  __syncthreads();
-  const unsigned ec = t.ec + above_cnt;
-  const double em = t.em + above_mass;
+template <int PER>
+__device__ __forceinline__ void find_bin(const Bins<PER>& t, int first, unsigned above_cnt, double above_mass, unsigned K, double M,
+                                         SampleShared& s, Turn& turn) {
+  unsigned ec = t.ec + above_cnt, best_c = 0, best_ec = 0;
+  double em = t.em + above_mass, best_em = 0;
   int mine = -1;
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int order = 2 * (int)threadIdx.x + e;
-    if (t.c[e] && BINS - 1 - order >= first && ec + (e ? t.c[0] : 0) < K && em + (e ? t.m[0] : 0.0) < M) mine = order;
+  for (int e = 0; e < PER; ++e) {
+    const int order = PER * (int)threadIdx.x + e;
+    if (t.c[e] && PER * ST - 1 - order >= first && ec < K && em < M) {
+      mine = order;
+      best_c = t.c[e];
+      best_ec = ec;
+      best_em = em;
+    }
+    ec += t.c[e];
+    em += t.m[e];
   }
-  // (orders rise with the lanes: a wave's last one speaks for it)
-  const unsigned long long those = __ballot(mine >= 0);
-  if (mine >= 0 && (those >> (threadIdx.x & 63)) == 1ull) atomicMax(&s.best, mine);
-  __syncthreads();
-  const int best = s.best;
-  __syncthreads();
-  if (best >= 0 && best >> 1 == (int)threadIdx.x) {
-    const bool second = best & 1;
-    s.above_cnt = ec + (second ? t.c[0] : 0);
-    s.above_mass = em + (second ? t.m[0] : 0.0);
-    s.cnt = second ? t.c[1] : t.c[0];
-    s.best = BINS - 1 - best;
+  const int best = block_last(mine, s, turn);
+  if (best < 0) {
+    if (threadIdx.x == 0) s.best = -1;
+  } else if (best == mine) {
+    s.above_cnt = best_ec;
+    s.above_mass = best_em;
+    s.cnt = best_c;
+    s.best = PER * ST - 1 - best;
   }
   __syncthreads();
 }
@@ -209,7 +249,8 @@ __device__ void sort_list(unsigned long long* list, int n) {
 }
 
 template <bool WIDE> struct ListShared {
-  Hist<WIDE> h1, h2;
+  Hist<WIDE, BINS1> h1;
+  Hist<WIDE, BINS> h2;
   unsigned long long list[CAP];
 };
 
@@ -235,40 +276,57 @@ typedef unsigned short Pair16 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ Pair16 pair16(unsigned x) { return __builtin_bit_cast(Pair16, x); }
 __device__ __forceinline__ unsigned both16(unsigned x) { return x | x << 16; }
 
-// f(the 16 bytes of eight elements, their place among the row's) for the row's part between its first and last 16-byte borders,
-// g(element, its index) for the others; every thread of the block takes part in every round (`live`: it has a piece)
-template <typename T, typename F, typename G> __device__ __forceinline__ void for_row16(const T* row, int V, F&& f, G&& g) {
+// A row of 16-bit elements between its first and last 16-byte borders, eight elements at a time: a thread's first HELD pieces stay in
+// registers from the first pass to the second (64 of the 128 that a thread of 1024 has: rows of up to 131072 entries as a whole), what
+// is longer is read again.
+template <typename T> struct HeldRow {
   typedef unsigned Vec __attribute__((ext_vector_type(4)));
-  const int head = min(V, (int)(((16u - ((unsigned)(uintptr_t)row & 15u)) & 15u) / sizeof(T)));
-  const int nvec = (V - head) / 8;
-  const Vec* body = reinterpret_cast<const Vec*>(row + head);
-  const unsigned short* raw = reinterpret_cast<const unsigned short*>(row);
-  if ((int)threadIdx.x < head) g((unsigned)raw[threadIdx.x], (int)threadIdx.x);
-  int i = threadIdx.x;
-  if (nvec >= 4 * ST) {
-    Vec v[4], next[4];
+  static constexpr int HELD = 16;
+  const T* row;
+  int V, head, nvec;
+  Vec held[HELD];
+  __device__ __forceinline__ HeldRow(const T* row_, int V_) : row(row_), V(V_) {
+    head = min(V, (int)(((16u - ((unsigned)(uintptr_t)row & 15u)) & 15u) / sizeof(T)));
+    nvec = (V - head) / 8;
+  }
+  __device__ __forceinline__ const Vec* body() const { return reinterpret_cast<const Vec*>(row + head); }
+  __device__ __forceinline__ void fetch() {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = body[i + e * ST];
-    for (;;) {
-      const bool more = i - (int)threadIdx.x + 8 * ST <= nvec;   // (the next four are on their way while these are looked at)
-      if (more)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) next[e] = body[i + (4 + e) * ST];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f(v[e], i + e * ST, true);
-      i += 4 * ST;
-      if (!more) break;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = next[e];
+    for (int e = 0; e < HELD; ++e) {
+      held[e] = Vec{0u, 0u, 0u, 0u};
+      if (e * ST < nvec) {                         // (the same for all threads)
+        const int i = e * ST + (int)threadIdx.x;
+        if (i < nvec) held[e] = body()[i];
+      }
     }
   }
-  for (; i - (int)threadIdx.x < nvec; i += ST) {
-    const bool live = i < nvec;
-    f(live ? body[i] : Vec{0u, 0u, 0u, 0u}, i, live);
+  // f(the 16 bytes, their place, whether the thread has a piece at all) for every round, all threads of the block taking part; f comes
+  // once a held round: a few instructions, or the code is larger than the instruction cache
+  template <typename F> __device__ __forceinline__ void each(F&& f) const {
+#pragma unroll
+    for (int e = 0; e < HELD; ++e)
+      if (e * ST < nvec) f(held[e], e * ST + (int)threadIdx.x, e * ST + (int)threadIdx.x < nvec);
+    again(HELD * ST, f);
   }
-  const int rest = head + nvec * 8 + (int)threadIdx.x;
-  if (rest < V) g((unsigned)raw[rest], rest);
-}
+  // the same, from memory, from the piece `from` on (a multiple of ST)
+  template <typename F> __device__ __forceinline__ void again(int from, F&& f) const {
+#pragma unroll 1
+    for (int i0 = from; i0 < nvec; i0 += ST) {
+      const int i = i0 + (int)threadIdx.x;
+      Vec v{0u, 0u, 0u, 0u};
+      if (i < nvec) v = body()[i];
+      f(v, i, i < nvec);
+    }
+  }
+  // g(element, its index) for those in front of the first border and behind the last
+  template <typename G> __device__ __forceinline__ void ends(G&& g) const {
+    const unsigned short* raw = reinterpret_cast<const unsigned short*>(row);
+    const int rest = head + nvec * 8 + (int)threadIdx.x;
+    const bool front = (int)threadIdx.x < head, back = rest < V;
+    if (front) g((unsigned)raw[threadIdx.x], (int)threadIdx.x);
+    if (back) g((unsigned)raw[rest], rest);
+  }
+};
 
 // Rows of 16-bit logits: the same two questions (see sampling_row.inc), answered from how often each of the 65536 patterns
 // occurs.  One pass over the row counts them (16 bits each, 128 KB of LDS); the ones that occur - a few thousand - are packed
@@ -276,17 +334,17 @@ template <typename T, typename F, typename G> __device__ __forceinline__ void fo
 // list, with no further look at the row and no sort.  A second pass finds the element: the drawn pattern's elements come in
 // the order of their indices, so each wave counts them in its 512 elements at a time, and the one stretch that the wanted one
 // lies in is looked at again.  Masses are counts times weights, in doubles: no result depends on the order of additions.
-// Bound by the LDS atomics and the vector instructions of the counting pass (10 us of a row of 128256 alone, 16 of 256 rows at
-// once, whose logits take 14 from memory), by the second pass (6 and 9) and by a dozen steps of a microsecond or two between
-// them.  256 rows of 128256 bf16 logits, every kind of filter among them: 38 us, by bins 118 when this was chosen (93 now); one row
-// 29 (62, 53), one of 32000 18 (37, 25).  The patterns are packed by stretches of 512 places a wave: with 64 places a thread the few
-// threads that have any were 7 us on their own (3.2 so).
+// Bound by the first pass (15 us of 256 rows of 128256 at once, whose logits take 14 from memory; 10 of one row, LDS atomics) and by a
+// dozen steps of a microsecond or two behind it.  256 rows of 128256 bf16 logits, every kind of filter among them: 31 us, one row
+// 24, 32000 entries 17; with the row read again for the second pass (10 us for 2.5 from registers), the counts' sum as an atomic a
+// lane (2 us) and the waves' totals added up by every wave 39, 29 and 18; by bins, as 32-bit rows are, 79, 36 and 18.  The patterns are
+// packed by stretches of 512 places a wave: with 64 places a thread the few threads that have any were 7 us on their own.
 // -1: a pattern occurs 65536 times or more (a count ran over: the counts' sum is then too small), more than 32768 patterns
-// occur, or the row is longer than the second pass has counters for.  The type's lowest value and the infinity next to it, which
+// occur or more than 16384 of the likelier sign, or the row is longer than the second pass has counters for.  The type's lowest value and the infinity next to it, which
 // masks fill rows with, are counted apart, in registers.
 template <typename T>
-__device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, float tp, float mp, float u, unsigned* tab,
-                                SampleShared& s, CountShared& cs) {
+__device__ __forceinline__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, float tp, float mp, float u, unsigned* tab,
+                                SampleShared& s, CountShared& cs, Turn& turn) {
   using O = Order16<T>;
   typedef unsigned Vec __attribute__((ext_vector_type(4)));
   if (V > 1 << 23) return -1;
@@ -296,7 +354,9 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
 #pragma unroll
   for (int j = 0; j < PATTERNS / 2 / (4 * ST); ++j) *reinterpret_cast<Vec*>(tab + 4 * (j * ST + tid)) = Vec{0u, 0u, 0u, 0u};
   if (tid == 0) { s.bad = 0; cs.low = 0; cs.inf = 0; cs.counted = 0; }
-  __syncthreads();
+  __syncthreads();                                 // (in front of the loads: a barrier waits for what is under way)
+  HeldRow<T> data(row, V);
+  data.fetch();
   // ---- how often each pattern occurs
   unsigned low = 0, inf = 0, nan = 0;
   const unsigned lowest = O::bits(O::LOWEST, flip), magnitude = lowest & 0x7fffu;
@@ -307,37 +367,51 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
     else if ((x & 0x7fffu) > magnitude + 1) nan = 1;
     else count(x);
   };
-  for_row16(
-      row, V,
-      [&](Vec v, int, bool live) {
-        if (!live) return;
-        const Pair16 most = __builtin_elementwise_max(
-            __builtin_elementwise_max(pair16(v[0] & 0x7fff7fffu), pair16(v[1] & 0x7fff7fffu)),
-            __builtin_elementwise_max(pair16(v[2] & 0x7fff7fffu), pair16(v[3] & 0x7fff7fffu)));
-        if (__builtin_expect(max((unsigned)most[0], (unsigned)most[1]) < magnitude, 1)) {
+  bool some_odd = false;
+  auto ordinary = [&](Vec v) {
+    const Pair16 most = __builtin_elementwise_max(
+        __builtin_elementwise_max(pair16(v[0] & 0x7fff7fffu), pair16(v[1] & 0x7fff7fffu)),
+        __builtin_elementwise_max(pair16(v[2] & 0x7fff7fffu), pair16(v[3] & 0x7fff7fffu)));
+    return max((unsigned)most[0], (unsigned)most[1]) < magnitude;
+  };
+  data.each([&](Vec v, int, bool live) {
+    const bool plain = ordinary(v);
+    if (live && plain) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w) { count(v[w] & 0xffffu); count(v[w] >> 16); }
-        } else {
-#pragma unroll
-          for (int w = 0; w < 4; ++w) { one(v[w] & 0xffffu); one(v[w] >> 16); }
-        }
-      },
-      [&](unsigned x, int) { one(x); });
+      for (int w = 0; w < 4; ++w) { count(v[w] & 0xffffu); count(v[w] >> 16); }
+    }
+    some_odd = some_odd || !plain;
+  });
+  if (__builtin_expect(__any(some_odd), 0))        // (from memory, once more)
+    data.again(0, [&](Vec v, int, bool live) {
+      if (!live || ordinary(v)) return;
+#pragma unroll 1
+      for (int j = 0; j < 8; ++j) {
+        one(v[0] & 0xffffu);
+        v = Vec{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+      }
+    });
+  data.ends([&](unsigned x, int) { one(x); });
   if (low) atomicAdd(&cs.low, low);
   if (inf) atomicAdd(&cs.inf, inf);
   if (nan) s.bad = 1;
   __syncthreads();
   // ---- those that occur, in order, as (place, count) words in the counts' stead: 128 stretches of 512 places, eight a lane,
-  // dealt to the waves in turn (values lie in a few octaves: most stretches are empty, and neighbours go to different waves)
-  unsigned n;
-  {
-    constexpr int ROUNDS = PATTERNS / 8 / ST;
+  // dealt to the waves in turn (values lie in a few octaves: most stretches are empty, and neighbours go to different waves).  In two
+  // halves, whose counts lie in halves of the table: the first half's words take the place of its own counts
+  unsigned n = 0, all_counts = 0;
+  const unsigned list0 = flip ? PATTERNS / 4 : 0u;               // where the list begins
+  auto word = [&](unsigned e) -> unsigned& { return tab[(list0 + e) & (PATTERNS / 2 - 1)]; };
+#pragma unroll 1
+  for (unsigned half = 0; half < 2; ++half) {
+    constexpr int ROUNDS = PATTERNS / 16 / ST;
+    const unsigned piece0 = half * (PATTERNS / 16) + tid;        // of the lane's first round
+    const bool back = half == 0;                                 // (positive patterns lie backwards; flipped, the negative ones do)
     Vec v[ROUNDS];
     unsigned pos[ROUNDS], used = 0;
 #pragma unroll
     for (int j = 0; j < ROUNDS; ++j) {
-      const unsigned piece = j * ST + tid, there = flip ? PATTERNS / 8 - 1 - piece : piece;     // (positive patterns lie backwards)
-      const bool back = (there < PATTERNS / 16) != (flip != 0u);
+      const unsigned piece = j * ST + piece0, there = flip ? PATTERNS / 8 - 1 - piece : piece;
       v[j] = *reinterpret_cast<const Vec*>(tab + 4 * (there < PATTERNS / 16 ? PATTERNS / 16 - 1 - there : there));
       if (back) v[j] = Vec{v[j][3], v[j][2], v[j][1], v[j][0]};
     }
@@ -346,8 +420,6 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
       unsigned total = 0;
       if (__any((v[j][0] | v[j][1] | v[j][2] | v[j][3]) != 0)) {
         used |= 1u << j;
-        const unsigned there = flip ? PATTERNS / 8 - 1 - (j * ST + tid) : j * ST + tid;
-        const bool back = (there < PATTERNS / 16) != (flip != 0u);
         unsigned c = 0, sum = 0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -356,7 +428,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
           c += (lo != 0) + (hi != 0);
           sum += lo + hi;
         }
-        if (sum) atomicAdd(&cs.counted, sum);
+        all_counts += sum;
         unsigned before = 0;
 #pragma unroll
         for (int bit = 0; bit < 4; ++bit) {
@@ -366,38 +438,43 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         }
         pos[j] = before;
       }
-      if (lane == 0) cs.of_stretch[j * (ST / 64) + wid] = total;
+      if (lane == 0) cs.of_stretch[half * 64 + j * (ST / 64) + wid] = total;
+    }
+    if (half == 1) {                               // (one atomic a wave: 64 lanes' on one word are a loop of their own)
+      const unsigned wave_counts = (unsigned)wave_scan((int)all_counts);
+      if (lane == 63) atomicAdd(&cs.counted, wave_counts);
     }
     __syncthreads();
-    const unsigned even = cs.of_stretch[2 * lane], odd = cs.of_stretch[2 * lane + 1];
-    const unsigned upto = (unsigned)wave_scan((int)(even + odd));
-    n = __shfl(upto, 63, 64);
-    if (cs.counted != (unsigned)V - cs.low - cs.inf && !s.bad) return -1;
-    if (n > PATTERNS / 2) return -1;
+    const unsigned mine = cs.of_stretch[half * 64 + lane];
+    const unsigned upto = (unsigned)wave_scan((int)mine);
+    const unsigned before = n;
+    n += __shfl(upto, 63, 64);
+    if (half == 0 && n > PATTERNS / 4) return -1;
+    if (half == 1 && ((cs.counted != (unsigned)V - cs.low - cs.inf && !s.bad) || n > PATTERNS / 2)) return -1;
 #pragma unroll
     for (int j = 0; j < ROUNDS; ++j) {
       if (!(used >> j & 1u)) continue;
       const int stretch = j * (ST / 64) + wid;
-      unsigned at = pos[j] + __shfl(upto - even - odd, stretch >> 1, 64) + (stretch & 1 ? __shfl(even, stretch >> 1, 64) : 0u);
+      unsigned at = before + pos[j] + __shfl(upto - mine, stretch, 64);
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        const unsigned d = 8u * (j * ST + tid) + 2u * w;
-        if (v[j][w] & 0xffffu) tab[at++] = d << 16 | (v[j][w] & 0xffffu);
-        if (v[j][w] >> 16) tab[at++] = (d + 1u) << 16 | v[j][w] >> 16;
+        const unsigned d = 8u * (j * ST + piece0) + 2u * w;
+        if (v[j][w] & 0xffffu) word(at++) = d << 16 | (v[j][w] & 0xffffu);
+        if (v[j][w] >> 16) word(at++) = (d + 1u) << 16 | v[j][w] >> 16;
       }
     }
     __syncthreads();
   }
   const unsigned lows = cs.low;
   // the row's largest entry (its place: the one in front of all); NaN, and an infinity there, are no distribution
-  const unsigned first = n ? tab[0] >> 16 : (lows ? O::LOWEST : O::LOWEST + 1);
+  const unsigned first = n ? word(0) >> 16 : (lows ? O::LOWEST : O::LOWEST + 1);
   const float top = O::value(first, flip);
   auto weight = [&](unsigned d) { return __float_as_uint(fast_exp2((O::value(d, flip) - top) * to_exp2)); };
   if (s.bad || first <= O::FIRST || (cs.inf && weight(O::LOWEST + 1) >= NORMAL_END)) return 0;
   // ---- entry n is the type's lowest value; a thread has `per` of them in a row
   const unsigned per = (n + 1 + ST - 1) / ST, e0 = min(per * tid, n + 1), e1 = min(e0 + per, n + 1);
   auto entry = [&](unsigned e, unsigned& d, unsigned& c) {
-    const unsigned x = e < n ? tab[e] : 0u;
+    const unsigned x = e < n ? word(e) : 0u;
     d = e < n ? x >> 16 : O::LOWEST;
     c = e < n ? x & 0xffffu : lows;
   };
@@ -415,17 +492,16 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
     m += c * mass_of(w);
   }
   if (odd) s.bad = 1;
-  block_scan(cnt, m, ec, em, z, s);
+  block_scan(cnt, m, ec, em, z, s, turn);
   if (s.bad) return 0;
   unsigned kept = (unsigned)V, rank = 0;
+  int found = -1;
   double mass = z;
   for (int step = 0; step < 2; ++step) {
     const unsigned minb = step == 0 && mp > 0.f ? __float_as_uint(fminf(mp, 1.f)) : 0u;
     if (step == 0 && k >= (unsigned)V && tp >= 1.f && minb == 0u) continue;      // everything is kept
     const double M = step == 0 ? (tp >= 1.f ? 1e300 : fmax((double)tp * z, 1e-300)) : fmax((double)u * mass, 1e-300);
     const unsigned K = step == 0 ? k : kept;
-    if (tid == 0) s.best = -1;
-    __syncthreads();
     int best = -1;
     unsigned in_front = ec, best_c = 0, best_front = 0, best_w = 0;
     double above = em, best_above = 0;
@@ -441,10 +517,9 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
         in_front += c;
         above += c * mass_of(w);
       }
-    // (entries rise with the lanes: a wave's last one speaks for it)
-    if (best >= 0 && (__ballot(best >= 0) >> lane) == 1ull) atomicMax(&s.best, best);
-    __syncthreads();
-    if (best >= 0 && s.best == best) {
+    found = block_last(best, s, turn);
+    if (found < 0) return 0;                       // (no weights at all)
+    if (found == best) {
       const double v = mass_of(best_w);
       const double fit = fmin(fmax(ceil((M - best_above) / v), 1.0), (double)best_c);
       const unsigned take = min((unsigned)fit, K - best_front);
@@ -454,14 +529,11 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
       s.n = (int)take;
     }
     __syncthreads();
-    if (s.best < 0) return 0;                      // (no weights at all)
     kept = s.above_cnt;
     mass = s.mass;
     rank = (unsigned)s.n;
-    __syncthreads();
   }
   // ---- the rank-th element (from 1) of the patterns that weigh as much: those beside the found one count in front of it
-  const int found = s.best;
   const unsigned wanted = s.cnt;
   if (tid == 0) { s.n_list = rank; cs.lo = 0xffffu; cs.hi = 0u; }
   __syncthreads();
@@ -477,8 +549,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
   rank = s.n_list;
   const unsigned lo = cs.lo, span = cs.hi - lo;
   // ---- how many of them each 512 elements hold: counter 0 for what lies in front of the first 16-byte border
-  const int head = min(V, (int)(((16u - ((unsigned)(uintptr_t)row & 15u)) & 15u) / sizeof(T)));
-  const int nvec = (V - head) / 8, parts = (nvec + 63) / 64;
+  const int head = data.head, nvec = data.nvec, parts = (nvec + 63) / 64;
   const unsigned short* raw = reinterpret_cast<const unsigned short*>(row);
   auto hit = [&](unsigned x) { return ((O::place(x, flip) - lo) & 0xffffu) <= span; };
   const unsigned drawn = both16(O::bits(lo, flip));
@@ -494,26 +565,31 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
   };
   auto single = [&](unsigned x, int i) { if (hit(x)) atomicAdd(tab + (i < head ? 0 : parts + 1), 1u); };
   if (span == 0)                                   // (one pattern, as good as always)
-    for_row16(
-        row, V,
-        [&](Vec v, int i, bool live) {
-          const Pair16 l = {1, 1};
-          Pair16 others = {0, 0};
+    data.each([&](Vec v, int i, bool live) {
+      Pair16 x[4];
 #pragma unroll
-          for (int w = 0; w < 4; ++w) others += __builtin_elementwise_min(pair16(v[w] ^ drawn), l);
-          hits_of(live ? 8u - others[0] - others[1] : 0u, i, live);
-        },
-        single);
+      for (int w = 0; w < 4; ++w) x[w] = pair16(v[w] ^ drawn);
+      const Pair16 least = __builtin_elementwise_min(__builtin_elementwise_min(x[0], x[1]), __builtin_elementwise_min(x[2], x[3]));
+      unsigned sum = 0;
+      if (__any(live && (least[0] == 0 || least[1] == 0))) {     // (512 elements seldom have one)
+        const Pair16 l = {1, 1};
+        Pair16 others = {0, 0};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) others += __builtin_elementwise_min(x[w], l);
+        const unsigned c = live ? 8u - others[0] - others[1] : 0u;
+#pragma unroll
+        for (int bit = 0; bit < 4; ++bit) sum += (unsigned)__popcll(__ballot(c >> bit & 1u)) << bit;
+      }
+      if (lane == 0 && live) tab[1 + (i >> 6)] = sum;
+    });
   else
-    for_row16(
-        row, V,
-        [&](Vec v, int i, bool live) {
-          unsigned c = 0;
+    data.again(0, [&](Vec v, int i, bool live) {
+      unsigned c = 0;
 #pragma unroll
-          for (int w = 0; w < 4; ++w) c += hit(v[w] & 0xffffu) + hit(v[w] >> 16);
-          hits_of(live ? c : 0u, i, live);
-        },
-        single);
+      for (int w = 0; w < 4; ++w) c += hit(v[w] & 0xffffu) + hit(v[w] >> 16);
+      hits_of(live ? c : 0u, i, live);
+    });
+  data.ends(single);
   __syncthreads();
   // ---- the stretch that the wanted one lies in
   const unsigned each = (parts + 2 + ST - 1) / ST;
@@ -523,7 +599,7 @@ __device__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, fl
     if (i < parts + 2) mine += tab[i];
   }
   double none, all;
-  block_scan(mine, 0.0, before, none, all, s);
+  block_scan(mine, 0.0, before, none, all, s, turn);
   if (before < rank && rank <= before + mine)
     for (unsigned e = 0; e < each; ++e) {
       const int i = (int)(each * tid + e);
@@ -569,7 +645,8 @@ __global__ __launch_bounds__(ST) void sample_kernel(int* __restrict__ out, const
                                                     const int* __restrict__ top_k, const float* __restrict__ top_p,
                                                     const float* __restrict__ min_p,
                                                     const float* __restrict__ uniform) {
-  __shared__ Hist<WIDE> h1, h2;
+  __shared__ Hist<WIDE, BINS1> h1;
+  __shared__ Hist<WIDE, BINS> h2;
   __shared__ unsigned long long list[CAP];
   __shared__ SampleShared s;
   __shared__ float red[16];
@@ -577,6 +654,7 @@ __global__ __launch_bounds__(ST) void sample_kernel(int* __restrict__ out, const
   static_assert(sizeof(T) == 4, "");
   unsigned* const tab = nullptr;
   CountShared cs;
+  Turn turn = 0;
 #include "sampling_row.inc"
 }
 
@@ -596,9 +674,11 @@ __global__ __launch_bounds__(ST) void sample16_kernel(int* __restrict__ out, con
   __shared__ float red[16];
   __shared__ int s_idx;
   static_assert(sizeof(T) == 2, "");
-  Hist<WIDE>&h1 = sh.bins.h1, &h2 = sh.bins.h2;
+  auto &h1 = sh.bins.h1;
+  auto& h2 = sh.bins.h2;
   unsigned long long* const list = sh.bins.list;
   unsigned* const tab = sh.counts;
+  Turn turn = 0;
 #include "sampling_row.inc"
 }
 

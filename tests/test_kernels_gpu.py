@@ -750,6 +750,53 @@ def test_sample_of_counted_patterns_is_the_one_of_the_same_values_in_32_bits(V, 
         assert torch.equal(got, want), (got.tolist(), want.tolist())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,offset", [(8 * 1024 - 1, 1), (131072, 0), (131072 + 8, 0), (131072 + 15, 3), (16 * 8192 - 9, 5)])
+def test_sample_holds_rows_of_whole_and_of_cut_rounds(V, offset, dtype):
+    """16-bit rows stay in registers up to 131072 entries behind the first 16-byte border: rows on either side of it, and of a last round
+    that is nearly empty, draw what the same values in 32 bits draw.  Among the rows: every pattern of one sign (more than the first
+    half of the packed list holds), masked ones, the likely entries at both ends."""
+    B = 6
+    g = torch.Generator(DEV).manual_seed(V)
+    x = (torch.randn(B, V + offset, generator=g, device=DEV) * 2.5).to(dtype)[:, offset:]
+    patterns = torch.arange(V, device=DEV) % 0x7000
+    x[1] = (patterns if dtype == torch.float16 else patterns % 0x4200).to(torch.int16).view(dtype)
+    x[2][: V // 2] = float("-inf")
+    x[3][8:] = torch.finfo(dtype).min
+    x[4][0], x[4][V - 1] = 14.0, 13.5
+    x[5][: V - 20] -= 30.0
+    temperature = torch.full((B,), 0.9, device=DEV)
+    top_k = torch.tensor([0, 0, 50, 5, 2, 12], dtype=torch.int32, device=DEV)
+    top_p = torch.tensor([0.9, 1.0, 0.95, 1.0, 1.0, 0.9], device=DEV)
+    min_p = torch.zeros(B, device=DEV)
+    for u in (1e-6, 0.3, 0.6, 0.97, 1 - 1e-6):
+        uniform = torch.full((B,), u, device=DEV)
+        got = ops.sample(x, temperature, top_k, top_p, min_p, uniform)
+        assert torch.equal(got, ops.sample(x.float(), temperature, top_k, top_p, min_p, uniform)), u
+    assert got[4] == V - 1 and got[5] >= V - 20
+
+
+@pytest.mark.parametrize("base,temperature", [(0.0, 1.0), (100.0, 0.05), (-3000.0, 1.3), (100.0, -0.05), (0.0, 1e-3)])
+def test_sample_lists_a_bin_s_entries_wherever_the_logits_lie(base, temperature):
+    """A bin's entries are looked for among the logits near it: logits of one size behind a large common part, small and negative
+    temperatures.  Weights from the stored logits in 64 bits, drawn at the middle of an entry's stretch (1e-4 of the mass or more, a
+    weight is off by less than 1e-5 of itself: an exponent of at most a hundred, rounded to 32 bits)."""
+    V, kept = 20000, 600
+    g = torch.Generator(DEV).manual_seed(3)
+    steps = torch.linspace(0.0, -60.0, V, device=DEV, dtype=torch.float64)
+    row = (base + temperature * steps[torch.randperm(V, generator=g, device=DEV)]).float()
+    w = torch.exp((row.double() - (row.max() if temperature > 0 else row.min()).double()) / temperature)
+    w, order = w.sort(descending=True, stable=True)
+    cum = w.cumsum(0)
+    ranks = [1, 2, 17, 100, 250, kept]
+    assert all(w[r - 1] / cum[kept - 1] > 1e-4 for r in ranks) and (w[:kept] - w[1:kept + 1] > 1e-4 * w[:kept]).all()
+    n = len(ranks)
+    u = torch.stack([(cum[r - 1] - 0.5 * w[r - 1]) / cum[kept - 1] for r in ranks]).float()
+    full = lambda v, t=torch.float32: torch.full((n,), v, device=DEV, dtype=t)
+    got = ops.sample(row.expand(n, -1).contiguous(), full(temperature), full(kept, torch.int32), full(1.0), full(0.0), u)
+    assert got.tolist() == [order[r - 1].item() for r in ranks]
+
+
 def test_sample_of_rows_without_a_distribution_is_entry_zero():
     """Rows of nothing but minus infinity, with a NaN or with an infinity: token 0, no hang, neighbours unharmed."""
     logits = _rand(4, 5000, dtype=torch.float32, scale=2.0)
