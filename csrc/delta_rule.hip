@@ -11,7 +11,8 @@
 //                     u = b (v - r), o = p + (k.q) u, S = gS + k u^T.  A lane keeps a part (a 4th, 8th or 16th) of one
 //                     column of S in registers; the parts are summed across lanes; q / k / g / v / b / k.q of a
 //                     chunk of rows are staged in LDS with the next chunk's loads in flight (one barrier per chunk).
-//                     A prompt portion and a single decoded row are the same kernel in two lane layouts.
+//                     A prompt portion and a few decoded rows are the same kernel in two lane layouts.
+//   delta_rule_row    both in one for sequences of a row each: per (sequence, head, tile of 64 or 128 value columns)
 #include "common.h"
 #include <math.h>
 #include <type_traits>
@@ -243,6 +244,144 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(float* __restrict
   }
 }
 
+// Steps of one row a sequence.  grid (tiles of 4 LC value columns, H, sequences), 256 threads: lane lc = tid % LC has columns 4 lc .. of
+// the rows i RG + tid / LC of S, so that the workgroup reads whole lines, rows one after the other.  S is on its way while wave 0
+// makes q and k unit vectors and the others the decays, in the operations of delta_rule_prep; the sums over rows are lanes', then
+// waves' through LDS.  (Rows beyond the first of a sequence are walked like it.)
+// Bound by reading and writing the states where there are many.  In a graph, with the write's own, and as two launches that read 64 bytes
+// of a state row at a time: 128 rows of 32 heads of 128 x 128, a decay per channel, 114 us (4.7 TB/s) and 176, 223 of 16 heads of
+// 64 x 128, a decay per head, 41 and 50, 35 of 32 of 64 x 128 16 and 34, one of 8 7.2 and 9.7; from Python, where a launch takes 13 us
+// of the host, 16 and 28 for 33 rows of 16 heads.  Registers for three workgroups a compute unit of 16 pieces a lane, five of eight:
+// with four and six they spill (129 and 46 us in place of 114 and 41).
+// ONCE: states read past the caches, see selective_scan_kernel.
+template <typename T, int LC, int R, bool PH, bool ONCE>
+__global__ __launch_bounds__(256, R > 8 ? 3 : 5) void delta_rule_row_kernel(
+    float* __restrict__ out, const T* __restrict__ x, long x_stride, const T* __restrict__ beta, long beta_stride,
+    const T* __restrict__ dt, long dt_stride, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
+    float* __restrict__ state, const int* __restrict__ slots, const int* __restrict__ qsl, const int* __restrict__ seq_lens, int H,
+    int G, int dim, int vdim, float norm_eps) {
+  constexpr int RG = 256 / LC, DP = RG * R;
+  static_assert(R % 4 == 0 && DP <= 128, "");
+  // (row r at (r % RG) R + r / RG: a lane's are side by side)
+  __shared__ __attribute__((aligned(16))) float ql[DP], kl[DP], gl[PH ? 4 : DP];
+  __shared__ float bkg[3];                         // sigmoid(beta), k.q, the head's decay
+  __shared__ f32x4 sums[2][4][LC];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = blockIdx.y, s = blockIdx.z, grp = h / (H / G);
+  const int q0 = qsl[s], n = qsl[s + 1] - q0;
+  if (n <= 0) return;                              // (the whole workgroup)
+  const int lc = tid % LC, rg = tid / LC, col = (blockIdx.x * LC + lc) * 4;
+  const bool col_ok = col < vdim;                  // (vdim % 4 == 0)
+  // (the workgroup's address and a lane's offset: an address a lane and piece would be as many registers as half of S)
+  float* const st = state + ((long)__builtin_amdgcn_readfirstlane(slots[s]) * H + h) * dim * vdim;
+  const unsigned own = rg * vdim + (col_ok ? col : 0);
+  const bool fresh = seq_lens[s] - n <= 0;         // the rows start the sequence: whatever the slot holds is not ours
+  f32x4 S[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = i * RG + rg;
+    S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (!fresh && col_ok && r < dim) {
+      const f32x4* from = reinterpret_cast<const f32x4*>(st + (long)i * RG * vdim + own);
+      S[i] = ONCE ? __builtin_nontemporal_load(from) : *from;
+    }
+  }
+  const float qscale = 1.0f / sqrtf((float)dim);
+  auto at = [](int r) { return (r % RG) * R + r / RG; };
+#pragma unroll 1
+  for (int t = q0; t < q0 + n; ++t) {
+    const T* xr = x + t * x_stride;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (col_ok)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = ldf(xr + 2 * (long)G * dim + (long)h * vdim + col + e);
+    if (wave == 0) {
+      const T* qs = xr + (long)grp * dim;
+      const T* ks = xr + (long)(G + grp) * dim;
+      float a[2], b[2], sq = 0.f, sk = 0.f;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int i = lane + 64 * e;
+        a[e] = i < dim ? ldf(qs + i) : 0.f;
+        b[e] = i < dim ? ldf(ks + i) : 0.f;
+        sq += a[e] * a[e];
+        sk += b[e] * b[e];
+      }
+      const float iq = 1.0f / sqrtf(wave_sum(sq) + norm_eps) * qscale, ik = 1.0f / sqrtf(wave_sum(sk) + norm_eps);
+      float dot = 0.f;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        a[e] *= iq;
+        b[e] *= ik;
+        dot += a[e] * b[e];
+        if (lane + 64 * e < DP) {
+          ql[at(lane + 64 * e)] = a[e];
+          kl[at(lane + 64 * e)] = b[e];
+        }
+      }
+      dot = wave_sum(dot);
+      if (lane == 0) bkg[1] = dot;
+    } else {
+      const T* dr = dt + t * dt_stride;
+      if constexpr (PH) {
+        if (tid == 64) bkg[2] = expf(-expf(a_log[h]) * softplus_f(ldf(dr + h) + dt_bias[h]));
+      } else {
+        const int i = tid - 64;                    // (DP <= 128)
+        if (i < DP)
+          gl[at(i)] = i < dim ? expf(-expf(a_log[h]) * softplus_f(ldf(dr + (long)h * dim + i) + dt_bias[h * dim + i])) : 0.f;
+      }
+      if (tid == 255) bkg[0] = 1.0f / (1.0f + expf(-ldf(beta + t * beta_stride + h)));
+    }
+    __syncthreads();
+    f32x4 r4[2] = {}, p4[2] = {};
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {
+      const f32x4 kv = *reinterpret_cast<const f32x4*>(kl + rg * R + i), qv = *reinterpret_cast<const f32x4*>(ql + rg * R + i);
+      f32x4 gv;
+      if constexpr (!PH) gv = *reinterpret_cast<const f32x4*>(gl + rg * R + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (!PH) S[i + e] *= gv[e];
+        r4[e & 1] += S[i + e] * kv[e];
+        p4[e & 1] += S[i + e] * qv[e];
+      }
+    }
+    f32x4 r = r4[0] + r4[1], p = p4[0] + p4[1];
+#pragma unroll
+    for (int o = 32; o >= LC; o >>= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        r[e] += __shfl_xor(r[e], o, 64);
+        p[e] += __shfl_xor(p[e], o, 64);
+      }
+    if (lane < LC) {
+      sums[0][wave][lane] = r;
+      sums[1][wave][lane] = p;
+    }
+    __syncthreads();
+    r = (sums[0][0][lc] + sums[0][1][lc]) + (sums[0][2][lc] + sums[0][3][lc]);
+    p = (sums[1][0][lc] + sums[1][1][lc]) + (sums[1][2][lc] + sums[1][3][lc]);
+    const float gs = PH ? bkg[2] : 1.f;
+    if constexpr (PH) { r *= gs; p *= gs; }
+    const f32x4 u = bkg[0] * (v - r);
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {
+      const f32x4 kv = *reinterpret_cast<const f32x4*>(kl + rg * R + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (PH) S[i + e] = gs * S[i + e] + kv[e] * u;
+        else S[i + e] += kv[e] * u;
+      }
+    }
+    if (rg == 0 && col_ok) *reinterpret_cast<f32x4*>(out + ((long)t * H + h) * vdim + col) = p + bkg[1] * u;
+    if (t + 1 < q0 + n) __syncthreads();
+  }
+  if (col_ok)
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (i * RG + rg < dim) *reinterpret_cast<f32x4*>(st + (long)i * RG * vdim + own) = S[i];
+}
+
 }  // namespace
 
 VDAMD_API int vdamd_delta_rule_prep(float* qn, float* kn, float* decay, float* bsig, const void* x, long x_stride,
@@ -303,6 +442,44 @@ VDAMD_API int vdamd_gated_delta_rule(float* out, const void* x, long x_stride, i
 #undef GDR_P
 #undef GDR
 #undef GDR_H
+  });
+  if (rc) return 1;
+  HIP_LAUNCH_CHECK();
+  return 0;
+}
+
+// Sequences of one row each (more are taken too): prep and recurrence in one.  x [T, x_stride] of type dtype with q, k and v in this
+// order; dt [T, H] (per_head) or [T, H * dim]; dim <= 128, vdim a multiple of 4, state and out on 16-byte borders
+VDAMD_API int vdamd_delta_rule_rows(float* out, const void* x, long x_stride, const void* beta, long beta_stride, const void* dt,
+                                    long dt_stride, const float* dt_bias, const float* a_log, float* state, const int* slots,
+                                    const int* qsl, const int* seq_lens, int B, int H, int G, int dim, int vdim, int per_head,
+                                    float norm_eps, int dtype, hipStream_t stream) {
+  if (B <= 0) return 0;
+  if (H <= 0 || H > 65535 || B > 65535 || G <= 0 || H % G || dim <= 0 || dim > 128 || vdim <= 0 || vdim % 4 || (uintptr_t)state % 16 ||
+      (uintptr_t)out % 16)
+    return 1;
+  const long bytes = (long)B * H * dim * vdim * 4;
+  const bool once = bytes > (64l << 20) && bytes <= (320l << 20);
+  const int rc = by_dtype(dtype, [&](auto* tp) {
+    using TT = std::remove_pointer_t<decltype(tp)>;
+#define ROW4(LC_, R_, PH_, ONCE_)                                                                                                  \
+  hipLaunchKernelGGL((delta_rule_row_kernel<TT, LC_, R_, PH_, ONCE_>), dim3((vdim + 4 * LC_ - 1) / (4 * LC_), H, B), dim3(256), 0, \
+                     stream, out, (const TT*)x, x_stride, (const TT*)beta, beta_stride, (const TT*)dt, dt_stride, dt_bias, a_log,  \
+                     state, slots, qsl, seq_lens, H, G, dim, vdim, norm_eps)
+#define ROW3(LC_, R_, PH_)                                                       \
+  do {                                                                           \
+    if (once) ROW4(LC_, R_, PH_, true); else ROW4(LC_, R_, PH_, false);          \
+  } while (0)
+#define ROW2(LC_, R_)                                                            \
+  do {                                                                           \
+    if (per_head) ROW3(LC_, R_, true); else ROW3(LC_, R_, false);                \
+  } while (0)
+    if (vdim > 64) { if (dim > 64) ROW2(32, 16); else ROW2(32, 8); }
+    else if (dim > 64) ROW2(16, 8);
+    else ROW2(16, 4);
+#undef ROW2
+#undef ROW3
+#undef ROW4
   });
   if (rc) return 1;
   HIP_LAUNCH_CHECK();

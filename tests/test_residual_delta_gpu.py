@@ -261,6 +261,38 @@ def test_gated_delta_rule(dtype, heads, qk, dim, vdim):
     assert torch.equal(s1[1], state[1]) and torch.equal(s1[2], state[2])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("heads,qk,dim,vdim", [(4, 2, 1, 4), (2, 2, 64, 64), (3, 3, 65, 68), (4, 1, 128, 132), (2, 1, 127, 60), (1, 1, 16, 256),
+                                               (2, 2, 64, 66), (2, 1, 129, 64)])
+def test_delta_rule_of_a_row_each(heads, qk, dim, vdim, per_head, dtype):
+    """Decoded rows in one launch, tiles of 64 and of 128 columns with remainders of rows and columns, and the sizes that go on in two
+    (columns that are no multiple of four, keys beyond 128): fresh, continued and empty sequences, states left alone between them,
+    and a sequence of three rows under the same hint.  Against the reference in 32 bits."""
+    hip = _hip()
+    g = torch.Generator(device="cuda").manual_seed(dim + vdim)
+    for rows in ([1, 1, 0, 1, 1, 1], [1, 3, 1, 0, 1, 1]):
+        starts = [5, 0, 3, 0, 70, 1]
+        t, n = sum(rows), len(rows)
+        x = (torch.randn(t, 2 * qk * dim + heads * vdim + 3, device="cuda", generator=g) * 0.8).to(dtype)
+        channels = heads if per_head else heads * dim
+        wide = torch.randn(t, heads + channels, device="cuda", generator=g).to(dtype)
+        beta, dtr = wide[:, :heads], wide[:, heads:]
+        dt_bias = torch.randn(channels, device="cuda", generator=g) * 0.5
+        a_log = torch.randn(heads, device="cuda", generator=g) - 1.0
+        state = torch.randn(9, heads, dim, vdim, device="cuda", generator=g) * 0.3
+        s1, after = state.clone(), state.clone()
+        ends = torch.tensor([0] + rows).cumsum(0).to(torch.int32).cuda()
+        lens, slots = _i32(*[s + r for s, r in zip(starts, rows)]), _i32(3, 0, 7, 4, 8, 2)
+        got = hip.gated_delta_rule(x, heads, qk, dim, vdim, beta, dtr, dt_bias, a_log, s1, slots, ends, lens, 1e-6, 1)
+        want = torch_ref.gated_delta_rule(x.float(), heads, qk, dim, vdim, beta.float(), dtr.float(), dt_bias, a_log, after, slots,
+                                          ends, lens, 1e-6)
+        # (sums of dim products, each rounded to 2^-24 of it, in another order, and three rows of them at most)
+        for a, b in ((got, want), (s1, after)):
+            assert (a - b).abs().max() <= 3 * 2 ** -24 * max(dim, 16) * max(1.0, b.abs().max().item())
+        assert torch.equal(s1[[1, 5, 6]], state[[1, 5, 6]])
+
+
 @pytest.mark.parametrize("window", [0, 19, 70])
 def test_windowed_latent_rows_on_the_matrix_cores(window):
     """Latent rows of 64 + 32 values kept as rows and as V^T fragments: the matrix-core kernels with a window, sinks

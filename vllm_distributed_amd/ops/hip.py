@@ -92,6 +92,7 @@ def load() -> ctypes.CDLL:
         "vdamd_sigmoid_mul": [P, L, P, L, P, L, F, I, I, I, P],
         "vdamd_gelu": [P, P, L, I, I, P],
         "vdamd_delta_rule_prep": [P, P, P, P, P, L, P, L, P, L, P, P, I, I, I, I, F, I, P],
+        "vdamd_delta_rule_rows": [P, P, L, P, L, P, L] + [P] * 6 + [I] * 6 + [F, I, P],
         "vdamd_gated_delta_rule": [P, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "vdamd_embed_scaled": [P, P, P, F, I, I, I, I, P],
         "vdamd_layer_norm_to": [P, P, L, P, L, P, P, F, I, I, I, I, I, P],
@@ -2140,13 +2141,21 @@ def gated_delta_rule(x, num_heads: int, num_qk_heads: int, dim: int, vdim: int, 
                            _f32_vec(dt_bias, dt.shape[1], "dt_bias"), _f32_vec(a_log, h, "a_log"), None, None, h, g, dim, vdim,
                            state, _i32(slots, "slots"), _i32(query_start_loc, "query_start_loc"), _i32(seq_lens, "seq_lens"),
                            False, norm_eps, 1.0, max_query_len)
+    out = torch.empty((t, h * vdim), dtype=torch.float32, device=x.device)
+    if max_query_len == 1 and not parts and dim <= 128 and vdim % 4 == 0 and state.data_ptr() % 16 == 0 and b <= 65535:
+        _check(_LIB.vdamd_delta_rule_rows(
+            out.data_ptr(), x.data_ptr(), x.stride(0), beta.data_ptr(), beta.stride(0), dt.data_ptr(), dt.stride(0),
+            _f32_vec(dt_bias, dt.shape[1], "dt_bias").data_ptr(), _f32_vec(a_log, h, "a_log").data_ptr(), state.data_ptr(),
+            _i32(slots, "slots").data_ptr(), _i32(query_start_loc, "query_start_loc").data_ptr(),
+            _i32(seq_lens, "seq_lens").data_ptr(), b, h, g, dim, vdim, int(per_head), float(norm_eps), _dt(x), _stream()),
+            "delta_rule_rows")
+        return out
     dev = x.device
     qn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
     kn = torch.empty((t, g, dim), dtype=torch.float32, device=dev)
     decay = None if per_head else torch.empty((t, h, dim), dtype=torch.float32, device=dev)
     # sigmoid(beta) | k.q of the head's group (| the head's decay)
     bsig = torch.empty((t, 3 if per_head else 2, h), dtype=torch.float32, device=dev)
-    out = torch.empty((t, h * vdim), dtype=torch.float32, device=dev)
     _check(_LIB.vdamd_delta_rule_prep(
         qn.data_ptr(), kn.data_ptr(), _ptr(decay), bsig.data_ptr(), x.data_ptr(), x.stride(0), beta.data_ptr(),
         beta.stride(0), dt.data_ptr(), dt.stride(0), _f32_vec(dt_bias, dt.shape[1], "dt_bias").data_ptr(),
