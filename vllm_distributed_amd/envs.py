@@ -18,9 +18,24 @@ import os
 from typing import Any, Callable, Dict
 
 
+def _reader(name: str, default: Any) -> Callable[[], Any]:
+    """``os.environ.get(name, default)``, at what an unset variable costs every launch: 0.1 us by asking the dictionary behind
+    ``os.environ``, 0.6 by ``get``, which encodes the name and catches an exception."""
+    values, key = getattr(os.environ, "_data", None), getattr(os.environ, "encodekey", None)
+    if not isinstance(values, dict) or key is None:
+        return lambda: os.environ.get(name, default)
+    encoded = key(name)
+
+    def get() -> Any:
+        return os.environ.get(name, default) if encoded in values else default
+    return get
+
+
 def _bool(name: str, default: bool) -> Callable[[], bool]:
+    read = _reader(name, None)
+
     def get() -> bool:
-        v = os.environ.get(name)
+        v = read()
         if v is None:
             return default
         return v.strip().lower() in ("1", "true", "yes", "on")
@@ -28,15 +43,17 @@ def _bool(name: str, default: bool) -> Callable[[], bool]:
 
 
 def _int(name: str, default: int) -> Callable[[], int]:
-    return lambda: int(os.environ.get(name, default))
+    read = _reader(name, default)
+    return lambda: int(read())
 
 
 def _float(name: str, default: float) -> Callable[[], float]:
-    return lambda: float(os.environ.get(name, default))
+    read = _reader(name, default)
+    return lambda: float(read())
 
 
 def _str(name: str, default: Any = None) -> Callable[[], Any]:
-    return lambda: os.environ.get(name, default)
+    return _reader(name, default)
 
 
 environment_variables: Dict[str, Callable[[], Any]] = {
