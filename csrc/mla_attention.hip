@@ -487,6 +487,262 @@ __global__ __launch_bounds__(256, 2) void mla_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// The same rows for FOUR tiles of 16 heads of a token a workgroup.  Groups of 64 keys in LDS, the next one on its way while one is
+// multiplied; eight waves:
+//   * QK: a wave one tile's whole reduction (its Q in registers) for half of the group's keys, so that a key's score is in one
+//     lane.  A tile's two waves trade their maxima through LDS before they form weights, which are then what mla_rows_kernel has (the
+//     largest one exact; each half by a maximum of its own in whole powers of two spares a barrier that turned out to cost nothing, and
+//     is up to 1.13 times as far from 64-bit sums).
+//   * All trade weights through LDS (16 bytes a lane).
+//   * PV: a wave a run of 64 values (half of them and two tiles where there are 256) for all keys and tiles: a value is read and turned
+//     into a fragment, as in mla_rows_kernel, once for the four.
+// The single kernel is bound by turning keys into V^T fragments and by its barriers, 1.25 us per 16 heads and 32 keys of a workgroup;
+// here a group costs 2.15 us for four times the heads and twice the keys (a fragment turned serves four tiles, a key read
+// from LDS a QK of its own still), though 156 KB of LDS leave one workgroup a CU and nothing beside it while it begins and ends.
+// us, single / this (one launch each, 576 of 512 values, 16 bits): 128 heads, 126 rows of 241 keys 56 / 31, 69 of 780 105 / 55, 128 of
+// 600 128 / 53, 30 of 2500 109 / 64, 7 of 9212 109 / 55, a prompt of 174 behind 496 110 / 68, three of 293 169 / 119; 64 heads, two
+// prompts of 200 111 / 63; 80 heads, 100 tokens behind 2900 166 / 118; one row of 3000, 128 heads, 20 / 26.
+// ---------------------------------------------------------------------------------------------------------------
+template <typename T, int DK, int DV>
+__global__ __launch_bounds__(512, 2) void mla_rows4_kernel(
+    T* __restrict__ out, long out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const T* __restrict__ q, long q_stride, const T* __restrict__ k_cache, const int* __restrict__ block_table, int bt_stride,
+    const int* __restrict__ token_seq, const int* __restrict__ seq_lens, float scale_log2e, int Hq, int block_size, int num_splits,
+    MlaExtra ex) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the buffer builtins exist in the device pass only)
+  using V = typename Vec8<T>::type;
+  constexpr int KSTEPS = DK / 32, ROW = DK * 2, PIECES = DK / 8, GROUP = 64;
+  constexpr int NP = 32 * PIECES / 256;            // 16-byte pieces of a half group per thread
+  constexpr int RUNS = DV / 64, TPW = RUNS / 2;    // of values, one a wave; tiles that a wave multiplies it by
+  static_assert(DK % 64 == 0 && (RUNS == 4 || RUNS == 8) && 32 * PIECES % 256 == 0, "unsupported latent width");
+  // (one object for all uses, see mla_rows_kernel): two groups | weights of eight waves | their maxima
+  __shared__ __attribute__((aligned(1024))) char smem[2 * GROUP * ROW + 8 * 64 * 16 + 8 * 16 * 4];
+  char* const s_p = smem + 2 * GROUP * ROW;
+  float* const s_m = reinterpret_cast<float*>(s_p + 8 * 64 * 16);
+
+  const int split = blockIdx.x, t = blockIdx.z;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int tile_n = wid & 3, half = wid >> 2;     // of the scores: the wave's tile and half of the keys
+  const int run_v = wid % RUNS, tile0 = wid / RUNS * TPW;        // of the products with values: the run, the first of the tiles
+  const int seq_len = seq_lens[t];
+  const int* const bt_row = block_table + (long)(token_seq != nullptr ? token_seq[t] : t) * bt_stride;
+  const int win_lo = ex.window > 0 ? max(seq_len - ex.window, 0) : 0;
+  const int g_lo = win_lo / GROUP;
+  const int n_groups = (seq_len + GROUP - 1) / GROUP - g_lo;
+  const int gps = (n_groups + num_splits - 1) / num_splits;
+  const int g_begin = g_lo + split * gps;
+  const int g_end = min(g_begin + gps, g_lo + n_groups);
+
+  auto swz = [](int key) { return ((key >> 1) & 1) | (((key >> 3) & 3) << 1); };
+  // this thread's pieces of its half of a group (four waves bring a half): their places in 32 rows in memory
+  unsigned place[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int c = i * 256 + ((int)threadIdx.x & 255), r = c / PIECES;
+    place[i] = r * ROW + ((c - r * PIECES) ^ swz(r)) * 16;
+  }
+  const int per_block = block_size >> 5, shift = (per_block & (per_block - 1)) == 0 ? __builtin_ctz(per_block) : -1;
+  // the wave's half of a group: which 32 keys (a half that holds no visible key repeats one that does), and their block
+  int half_of = 0, block_of = 0;
+  auto find = [&](int g) {
+    half_of = max(min(2 * g + half, (seq_len - 1) >> 5), win_lo >> 5);
+    block_of = bt_row[shift >= 0 ? half_of >> shift : half_of / per_block];
+  };
+  // what `find` has found: the descriptor, and the places of this thread's pieces (rows that hold no visible key repeat one that does)
+  auto rows_of = [&](unsigned (&at)[NP]) {
+    const int base = half_of * 32, inside = shift >= 0 ? half_of & (per_block - 1) : half_of % per_block;
+    const long first = (long)block_of * block_size + inside * 32;
+    const int lo = max(win_lo - base, 0), hi = min(seq_len - 1 - base, 31);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) at[i] = place[i];
+    if (lo > 0 || hi < 31) {
+      int tid = threadIdx.x & 255;
+      asm volatile("" : "+v"(tid));                // (not worth registers in between)
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int c = i * 256 + tid, r = c / PIECES;
+        at[i] = max(min(r, hi), lo) * ROW + ((c - r * PIECES) ^ swz(r)) * 16;
+      }
+    }
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(k_cache + first * DK), 0, 32 * ROW, 0x00020000);
+  };
+  char* const mine = smem + half * 32 * ROW + tile_n * 1024;
+  if (g_begin < g_end) {
+    find(g_begin);
+    unsigned at[NP];
+    const auto rows = rows_of(at);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (mla_lds_void*)(mine + i * 4096), 16, at[i], 0, 0, 0);
+    if (g_begin + 1 < g_end) find(g_begin + 1);
+  }
+  V qf[KSTEPS];
+  {
+    const int head = (4 * (int)blockIdx.y + tile_n) * 16 + r16;
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+      V z;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) z[j] = (T)0.f;
+      qf[s] = head < Hq ? ld8<T>(q + t * q_stride + (long)head * DK + 32 * s + 8 * g4) : z;
+    }
+  }
+  f32x4 acc[TPW][4];
+  float M[TPW];                                    // the tiles' maxima, which the sums go by
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    M[i] = MLA_NEG_BIG;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float m = MLA_NEG_BIG, l = 0.f;                  // the maximum of the wave's own tile, the sum of its half
+  // K rows of the two interleaved S^T tiles: key_a and 4 behind it (whose pieces are turned alike); of 64 values the two pieces.
+  // V: keys 8 g4 + j of a half, the pieces of those with bit 1 of j clear and set.  All else is in the instructions' offsets.
+  const int key_a = 8 * (r16 >> 2) + (r16 & 3);
+  int k_at[2], v_at[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    k_at[e] = key_a * ROW + (((4 * e + g4) ^ swz(key_a)) << 4);
+    v_at[e] = 8 * g4 * ROW + (((r16 >> 1) ^ (e | g4 << 1)) << 4) + (r16 & 1) * 8 + run_v * 128;
+  }
+
+  for (int g = g_begin; g < g_end; ++g) {
+    const int buf = (g - g_begin) & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                               // the group is in LDS, and nobody reads the other buffer any more
+    const char* const group = smem + buf * GROUP * ROW;
+    const char* const keys = group + half * 32 * ROW;
+    f32x4 s0[2] = {}, s1[2] = {};
+    auto score = [&](int s) {
+      const char* const at = keys + k_at[s & 1] + (s >> 1) * 128;
+      s0[s & 1] = mfma16(*reinterpret_cast<const V*>(at), qf[s], s0[s & 1]);
+      s1[s & 1] = mfma16(*reinterpret_cast<const V*>(at + 4 * ROW), qf[s], s1[s & 1]);
+    };
+    static_assert(KSTEPS == 2 * NP, "a piece every other step");
+    if (g + 1 < g_end) {
+      unsigned at[NP];
+      const auto rows = rows_of(at);
+      // (72 pieces of 1 KB asked for at a time are 0.6 us before the last waves' first product)
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (mla_lds_void*)(mine + (buf ^ 1) * GROUP * ROW + i * 4096), 16, at[i], 0, 0, 0);
+        score(2 * i);
+        score(2 * i + 1);
+        __builtin_amdgcn_sched_barrier(0x18e);     // (what reads LDS and multiplies may move across, the pieces stay apart)
+      }
+      if (g + 2 < g_end) find(g + 2);              // (the table's entry is there when it is wanted)
+    } else {
+#pragma unroll
+      for (int s = 0; s < KSTEPS; ++s) score(s);
+    }
+    const f32x4 sa = s0[0] + s0[1], sb = s1[0] + s1[1];
+    const int key0 = g * GROUP + half * 32, kidx0 = key0 + 8 * g4;
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = (j < 4 ? sa[j & 3] : sb[j & 3]) * scale_log2e;
+    const bool masked = key0 + 32 > seq_len || key0 < win_lo;
+    if (masked)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = (kidx0 + j < seq_len && kidx0 + j >= win_lo) ? p[j] : MLA_NEG_BIG;
+    float tmax = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    if (g4 == 0) s_m[wid * 16 + r16] = tmax;
+    // (not __syncthreads(), which would also wait for the next group's rows)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const float m_new = fmaxf(m, fmaxf(tmax, s_m[(wid ^ 4) * 16 + r16]));
+    float top[TPW];
+#pragma unroll
+    for (int n = 0; n < TPW; ++n) top[n] = fmaxf(M[n], fmaxf(s_m[(tile0 + n) * 16 + r16], s_m[(tile0 + n + 4) * 16 + r16]));
+    V pf;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float e = fast_exp2(p[j] - m_new);
+      p[j] = masked && p[j] <= 0.5f * MLA_NEG_BIG ? 0.f : e;
+      pf[j] = (T)p[j];
+    }
+    const float psum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    l = l * fast_exp2(m - m_new) + psum;
+    m = m_new;
+    *reinterpret_cast<V*>(s_p + (wid * 64 + lane) * 16) = pf;
+#pragma unroll
+    for (int n = 0; n < TPW; ++n) {
+      if (__any(top[n] != M[n])) {
+        const float alpha = fast_exp2(M[n] - top[n]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[n][v] *= alpha;
+        M[n] = top[n];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    V weights[TPW][2];
+#pragma unroll
+    for (int n = 0; n < TPW; ++n)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) weights[n][h] = *reinterpret_cast<const V*>(s_p + ((tile0 + n + 4 * h) * 64 + lane) * 16);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      // a lane's four neighbouring values of each of eight keys, turned into V^T fragments of four tiles of columns
+      u32x2 w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = *reinterpret_cast<const u32x2*>(group + v_at[j >> 1 & 1] + (kk * 32 + j) * ROW);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        union { uint32_t u[4]; V f; } fr;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t a = w[2 * j][v >> 1], b = w[2 * j + 1][v >> 1];
+          fr.u[j] = __builtin_amdgcn_perm(b, a, (v & 1) ? 0x07060302u : 0x05040100u);
+        }
+#pragma unroll
+        for (int n = 0; n < TPW; ++n) acc[n][v] = mfma16(fr.f, weights[n][kk], acc[n][v]);
+      }
+    }
+  }
+
+  // ---- the halves' sums meet
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  __syncthreads();
+  float* const s_l = reinterpret_cast<float*>(s_p);
+  if (g4 == 0) s_l[wid * 16 + r16] = l;
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < TPW; ++n) {
+    const int tile = tile0 + n, qh = (4 * (int)blockIdx.y + tile) * 16 + r16;
+    if (qh >= Hq) continue;
+    float lsum = s_l[tile * 16 + r16] + s_l[(tile + 4) * 16 + r16];
+    // acc[n][v][r]: value 64 run_v + 16 g4 + 4 r + v
+    if (num_splits == 1) {
+      float factor = 1.f;
+      if (ex.sinks != nullptr) mla_add_sink(ex.sinks[qh] * 1.4426950408889634f, M[n], lsum, factor);
+      float inv = lsum > 0.f ? factor / lsum : 0.f;
+      if (ex.gate != nullptr) inv *= 1.f / (1.f + __expf(-(float)((const T*)ex.gate)[t * ex.gate_stride + qh]));
+      T* orow = out + t * out_stride + (long)qh * DV + 64 * run_v + 16 * g4;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        typename Vec4<T>::type o;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (T)(acc[n][v][r] * inv);
+        *reinterpret_cast<typename Vec4<T>::type*>(orow + 4 * r) = o;
+      }
+    } else {
+      const long pidx = ((long)t * Hq + qh) * num_splits + split;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(part_o + pidx * DV + 64 * run_v + 16 * g4 + 4 * r) =
+            f32x4{acc[n][0][r], acc[n][1][r], acc[n][2][r], acc[n][3][r]};
+      if (run_v == 0 && g4 == 0) { part_ml[2 * pidx] = M[n]; part_ml[2 * pidx + 1] = lsum; }
+    }
+  }
+#endif
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // Several query tiles per workgroup over ONE stream of cache fragments, for caches that the kernel over key rows does not read (8
 // bits, blocks that cut a group of 32 keys, narrow values; where it does, it is 1.2 to 4.6 times as fast: 880 prompt tokens of 128
 // heads 902 us here and 584 there).  The kernel over both caches requests every cached
@@ -828,6 +1084,15 @@ int launch_mla(void* out, long out_stride, void* part_o, void* part_ml, const vo
     } else {
       return -4;
     }
+  } else if (mode == 4) {                           // four tiles of a token's heads over the key rows
+    if constexpr (!KV8 && !P2 && DV % 256 == 0 && DK % 64 == 0) {
+      if (block_size % 32) return -1;
+      mla_rows4_kernel<T, DK, DV><<<dim3(num_splits, (q_tiles + 3) / 4, T_), 512, 0, st>>>(
+          (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, (const T*)k_cache, block_table, bt_stride,
+          token_seq, seq_lens, sl2, Hq, block_size, num_splits, ex);
+    } else {
+      return -4;
+    }
   } else {
     mla_attention_kernel<T, DK, DV, KV8, P2><<<dim3(num_splits, q_tiles, T_), 256, 0, st>>>(
         (T*)out, out_stride, (float*)part_o, (float*)part_ml, (const T*)q, q_stride, k_cache, v_cache, block_table,
@@ -875,7 +1140,8 @@ int dispatch_mla(int DK, int DV, int kv_fp8, void* out, long out_stride, void* p
 // mode 0: one workgroup per (token, 16 heads); 1: four consecutive tokens of a sequence per workgroup (needs
 // token_seq; positions inside a sequence must be consecutive); 2: four head tiles of a token per workgroup.
 // mode 3: as mode 0, the values taken from the key rows (16-bit caches, blocks of a multiple of 32 tokens, DV a multiple of 256);
-// past_bytes > 0 (token_seq null): where the rows seen are that many bytes, those of one token alone are read past the caches.
+// mode 4: as mode 3, four head tiles of a token per workgroup (not with precise).
+// past_bytes > 0 (mode 3, token_seq null): where the rows seen are that many bytes, those of one token alone are read past the caches.
 // Supported (DK, DV): (576, 512) DeepSeek-V2 / V3, (320, 256), (96, 64).
 VDAMD_API int vdamd_mla_attention(void* out, long out_stride, void* part_o, void* part_ml, const void* q,
                                   long q_stride, const void* k_cache, const void* v_cache, const int* block_table,

@@ -161,6 +161,34 @@ def test_latent_attention_takes_the_plan(rows_ok, monkeypatch):
         assert handed[-1] == (splits, mode) and (mode == 3) is rows_ok
 
 
+@pytest.mark.parametrize("tokens,heads,keys,captured,shared", [
+    # single / shared, us: 29 / 26, 62 / 43, 39 / 36, 49 / 38, 172 / 115; 20 / 26, 31 / 34, 34 / 37; too few tiles; in a graph (27 / 22)
+    (50, 128, 400, False, True), (20, 128, 1500, False, True), (5, 128, 4000, False, True), (12, 64, 4000, False, True),
+    (100, 80, 3000, False, True), (1, 128, 3000, False, False), (8, 128, 1500, False, False), (8, 64, 4000, False, False),
+    (4000, 48, 4000, False, False), (100, 128, 9000, True, True), (64, 128, 9000, True, False), (100, 128, 100, True, False)])
+def test_latent_heads_shared(tokens, heads, keys, captured, shared, monkeypatch):
+    """The rule, and that the kernel over key rows is the one that it turns: not for precise weights, nor where another was asked for."""
+    import torch
+    assert hip.mla_heads_shared(tokens, heads, keys, captured) is shared
+    handed = []
+
+    class Lib:
+        @staticmethod
+        def vdamd_mla_attention(*args):
+            handed.append(args[18:20])                 # splits, mode
+            return 0
+    monkeypatch.setattr(hip, "_LIB", Lib)
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "mla_supported", lambda *shape: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: captured)
+    kc, vc = torch.zeros(4, 1, 32, 320, dtype=torch.bfloat16), torch.zeros(4, 1, 16, 4, 16, 8, dtype=torch.bfloat16)
+    row = lambda n: torch.zeros(1, heads, n, dtype=torch.bfloat16).expand(tokens, heads, n)
+    q, out, table = row(320), row(256), torch.zeros(tokens, 4, dtype=torch.int32)
+    for mode, precise in ((None, False), (3, False), (3, True), (2, False)):
+        hip.mla_attention(q, kc, vc, table, None, torch.ones(tokens, dtype=torch.int32), 0.1, keys, out=out, mode=mode, precise=precise)
+        assert handed[-1][1] == (mode if mode == 2 else 4 if shared and not precise else 3)
+
+
 @pytest.mark.parametrize("m,n,k,reduced,takes", [
     # the next kernel sums the slabs (library / this, us): 8.5 / 5.5, 16.2 / 11.2; a small W at many rows 8.9 / 9.9, 10.2 / 13.3,
     # 17.7 / 16.5; 32 / 18; a router

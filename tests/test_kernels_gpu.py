@@ -1718,6 +1718,45 @@ def test_latent_attention_of_prompts_and_many_heads_reads_key_rows(dk, dv, hq, w
             assert err(run(None, splits)) <= bound < 2 ** -7
 
 
+@pytest.mark.parametrize("dk,dv,hq,bs,dtype", [(576, 512, 64, 32, torch.float16), (576, 512, 128, 96, torch.bfloat16),
+                                              (576, 512, 81, 64, torch.bfloat16), (320, 256, 70, 96, torch.float16),
+                                              (320, 256, 128, 32, torch.bfloat16)])
+@pytest.mark.parametrize("window", [0, 45])
+@pytest.mark.parametrize("extras", [False, True])
+def test_latent_rows_of_four_head_tiles_a_workgroup(dk, dv, hq, bs, dtype, window, extras):
+    """Lengths around the halves and the whole of a group of 64 keys, decoded rows and prompts that name theirs, whole and in splits
+    that no key falls into, a last workgroup with tiles and heads left over, scores that climb
+    towards the end, and NaN wherever no key is.  Bound as for the single tiles: each weight rounded to half a unit in its last place, the
+    result once, half of it again for the scores and sums in 32 bits."""
+    from vllm_distributed_amd.ops import hip as _hip
+    torch.manual_seed(dk + hq + window)
+    lens = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 500]
+    per = -(-max(lens) // bs)
+    rows = torch.full(torch_ref.k_cache_shape(len(lens) * per, 1, dk, bs), float("nan"), device=DEV).to(dtype)
+    unread = torch.full(torch_ref.v_cache_shape(len(lens) * per, 1, dv, bs), float("nan"), device=DEV).to(dtype)
+    table = torch.randperm(len(lens) * per, device=DEV).int().view(len(lens), per)
+    for b, n in enumerate(lens):
+        at = torch.arange(n, device=DEV)
+        rows[table[b, at // bs].long(), 0, at % bs] = (torch.randn(n, dk, device=DEV) * (0.2 + at.unsqueeze(1) / n)).to(dtype)
+    clean = torch.nan_to_num(rows).float()
+    sinks = torch.randn(hq, device=DEV) if extras else None
+    half = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    bound = half * 2 * 1.5 * clean[..., :dv].abs().max()
+    prompt = [(b, n - i) for b, n in enumerate(lens) for i in reversed(range(min(n, 5)))]
+    for seq, keys in ((None, lens), (torch.tensor([b for b, _ in prompt], dtype=torch.int32, device=DEV), [n for _, n in prompt])):
+        sl = torch.tensor(keys, dtype=torch.int32, device=DEV)
+        q = (2 * torch.randn(len(keys), hq, dk, device=DEV)).to(dtype)
+        gate = torch.randn(len(keys), hq + 3, device=DEV).to(dtype)[:, 3:] if extras else None
+        want = torch_ref.latent_row_attention(q.float(), clean, table, seq, sl, 0.15, dv, window, sinks,
+                                              None if gate is None else gate.float())
+        run = lambda lengths, splits: _hip.mla_attention(q, rows, unread, table, seq, lengths, 0.15, max(lens), splits=splits, mode=4,
+                                                         window=window, sinks=sinks, gate=gate)
+        for splits in (1, 2, 7):
+            err = (run(sl, splits).float() - want).abs().max()
+            assert err <= bound, (splits, err.item(), bound.item())
+            assert run(0 * sl, splits).eq(0).all()
+
+
 @pytest.mark.parametrize("e,k,n_group,topk_group,v3,renorm", [
     (256, 8, 8, 4, True, True), (256, 8, 1, 1, True, True), (160, 6, 8, 3, False, False), (64, 6, 1, 1, False, False),
     (64, 6, 1, 1, False, True), (8, 2, 4, 2, True, True), (128, 1, 1, 1, True, True), (72, 4, 8, 8, False, True)])

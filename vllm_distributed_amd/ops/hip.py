@@ -1353,20 +1353,38 @@ def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows
     if mode is None:
         # (four head tiles per workgroup need enough workgroups left to fill the chip)
         mode = 3 if rows_ok else 1 if by_token else 2 if q_tiles >= 4 and tokens * q_tiles >= 128 else 0
-    if mode in (0, 3) and keys < 384 and not captured:
+    if mode in (0, 3, 4) and keys < 384 and not captured:
         return mode, 1
     if mode == 0:
         return mode, mla_num_splits(tokens, q_tiles, keys)
     if mode == 1:
         wgs = min(tokens, -(-tokens // 4) + seqs - 1) * q_tiles       # (a sequence's tokens start a group of four anywhere)
     else:
-        wgs = tokens * (-(-q_tiles // 4) if mode == 2 else q_tiles)
+        wgs = tokens * (-(-q_tiles // 4) if mode in (2, 4) else q_tiles)
     per, shortest = (512 if mode == 3 else 256) // max(wgs, 1), 64
     if mode == 1 and 128 < wgs < 256:
         per = 2
     if mode == 3 and wgs > 64:
         shortest = 128 if wgs < 256 else 256
+    if mode == 4:
+        shortest = 192
     return mode, max(1, min(per, keys // shortest, 64))
+
+
+def mla_heads_shared(tokens: int, heads: int, keys: int, captured: bool) -> bool:
+    """Whether a step over key rows (``mla_plan``'s 3) goes four tiles of 16 heads a workgroup (4): from 64 heads on, where there is
+    work enough.  Such a workgroup needs the time of two single ones for four tiles of a key, and 6 to 8 us more before its first
+    product and after its last, so the line is at 160000 (tiles - what the last four leave idle) x rows x keys.  us, single / shared:
+    128 heads, 50 rows of 250 keys 29 / 26, 100 of 250 46 / 29, 20 of 1500 62 / 43, 12 of 4000 86 / 49, 5 of 4000 39 / 36, 3 of 9000
+    52 / 39; 64 heads, 12 of 4000 49 / 38, 50 of 1500 78 / 47, 100 of 1500 132 / 67; below the line, 128 heads, one row of 3000 20 / 26,
+    8 of 1500 31 / 34, 20 of 600 34 / 36, and 64 heads, 8 of 4000 34 / 37, 20 of 600 25 / 32.
+    In a graph ``keys`` is a bound that the lengths may be far below, and a split that is empty still costs its partial sums: only
+    steps whose workgroups fill half of the CUs whole (100 rows of 128 heads, 100 keys: 27 / 22)."""
+    q_tiles = -(-heads // 16)
+    fours = -(-q_tiles // 4)
+    if q_tiles < 4 or tokens * keys * (2 * q_tiles - 4 * fours) < 160000:
+        return False
+    return not captured or tokens * fours > 128
 
 
 # latent rows of a decode step that are read past the caches (again and again 57 and 86 MB are slower so, 210 MB 63 -> 57 us)
@@ -1385,7 +1403,8 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     consecutive positions); 2 = four head tiles of a token per workgroup (64 heads per rank and more); 3 = as 0,
     the values read from the key rows (their first ``DV`` values, which is what every writer puts into both caches):
     half the bytes, 1.1 to 4.6 times as fast from one sequence of 32 keys to 256 of 1500 and prompts of 5000, at every width and
-    head count measured, so the others are left with what 3 does not read (``mla_rows_ok``).
+    head count measured, so the others are left with what 3 does not read (``mla_rows_ok``); 4 = four head tiles of a token per
+    workgroup over the key rows, which 3 turns into where that is faster (``mla_heads_shared``; weights not ``precise``).
     ``precise``: the softmax weights enter the PV product with fp32 precision (a high and a low 16-bit part).
     ``window`` > 0: only the last ``window`` of those keys; ``sinks[Hq]`` (fp32): ``exp(sinks[h])`` joins head ``h``'s
     softmax denominator; ``gate[T, Hq]`` (raw, rows may be strided): the output times its sigmoid."""
@@ -1407,6 +1426,8 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
+    if mode == 3 and not precise and hq > 48 and mla_heads_shared(t, hq, keys, torch.cuda.is_current_stream_capturing()):
+        mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], True, 4, keys >= 384)
     # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
     past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
                                          and t * keys * dk * 2 >= LATENT_ONCE_BYTES) else 0
