@@ -1,4 +1,4 @@
-// GEMM for decode batches of 1..512 rows:  y[M][N] = x[M][K] . W[N][K]^T  (bf16 / f16, fp32 accumulate), plain or with
+// GEMM for batches of 1..1280 rows:  y[M][N] = x[M][K] . W[N][K]^T  (bf16 / f16, fp32 accumulate), plain or with
 // SiLU(gate) * up over a [gate ; up] weight.
 //
 // In this range a step is bound by reading W once from HBM while the MFMA work per weight byte is already substantial
@@ -32,6 +32,12 @@
 //   70B down      87 -> 77     89 -> 77     (no) -> 87    133 -> 105     (8192 x 28672)
 //   8B qkv        16 -> 11     16 -> 12     24 -> 16      28 -> 22       (6144 x 4096)
 //   8B gate_up    47 -> 41     68 -> 41     58 -> 51      77 -> 62       (28672 x 4096, with SiLU * up)
+// Above 256 rows W comes once a row tile and its neighbours on an XCD share it; what this kernel has over the library there are the K
+// splits of long reductions, and tiles of 192 rows for what 256 would pad by a third (library -> here):
+//   rows          300          557          768           1024          1280
+//   8B down       76 -> 54     114 -> 74    107 -> 90     132 -> 113    147 -> 133    (4096 x 14336)
+//   7B down       102 -> 65    142 -> 87    183 -> 102    191 -> 129    230 -> 159    (3584 x 18944)
+//   70B down      219 -> 161 (185 in tiles of 256)                                    (8192 x 28672)
 // Row-grouped form (sparse experts, rows sorted by expert): a table names each entry's weight matrix, first row and rows; rows may
 // be read through the sorted list (gate and up with SiLU * up, then down, us, against tiles of 16 to 128 rows with W straight
 // from memory, a gather and the activation kernel; from 72 rows an expert on the large-batch kernel's tiles of 256 are ahead):
@@ -319,6 +325,8 @@ int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os,
   if (bm == BM && bn == BN) return launch<T, BM, BN, WM, WN, XS, WS>(x, xs, w, ws, out, os, bias, partial, M, N, K, ksplit, epi, st);
   MG_CASE(256, 256, 4, 2, 2, 3)
   MG_CASE(256, 128, 2, 4, 3, 4)
+  MG_CASE(192, 256, 2, 4, 2, 3)
+  MG_CASE(192, 128, 4, 2, 3, 4)
   MG_CASE(128, 256, 2, 4, 2, 3)
   MG_CASE(128, 128, 4, 2, 4, 5)
   MG_CASE(64, 128, 2, 2, 3, 3)
@@ -329,7 +337,7 @@ int dispatch(const void* x, long xs, const void* w, long ws, void* out, long os,
 }  // namespace
 
 // out = epilogue(x[M][K] . w[N][K]^T).  K % 64 == 0, N % 16 == 0; strides in elements, multiples of 8; pointers 16-byte
-// aligned.  (bm, bn) is the workgroup tile: (256, 128|256), (128, 128|256), (64, 128).
+// aligned.  (bm, bn) is the workgroup tile: (256 | 192 | 128, 128 | 256), (64, 128).
 // epi 0: out[M][N], with bias[N] (or null, 8-byte aligned) added before the one rounding; partial holds ksplit * M * N floats
 // when ksplit > 1, and out may be null then: the slabs are the result.
 // epi 2: w = [gate ; up], N % 32 == 0, ksplit 1, out[M][N/2] = silu(gate) * up.

@@ -208,6 +208,20 @@ def test_short_batch_products(m, n, k, reduced, takes):
         assert (bm, bn) in hip._MID_TILES and bm >= min(m, 256) and 1 <= ksplit <= k // 64
 
 
+@pytest.mark.parametrize("m,n,k,reduced,takes,rows", [
+    # library / this, us: 114 / 74, 107 / 90, 147 / 133, 45 / 31, 76 / 54, 219 / 161; tiles by the thousand, squarer shapes and more rows
+    # (265 / 287, 165 / 143, 37 / 33, 97 / 101)
+    (557, 4096, 14336, False, True, 192), (768, 4096, 14336, True, True, None), (1280, 4096, 14336, False, True, 256),
+    (557, 2048, 8192, True, True, None), (300, 4096, 14336, False, True, 192), (300, 8192, 28672, False, True, 192),
+    (640, 8192, 28672, False, False, None), (1281, 4096, 14336, False, False, None), (557, 4096, 4096, False, False, None),
+    (557, 10240, 8192, True, False, None)])
+def test_products_of_several_row_tiles(m, n, k, reduced, takes, rows):
+    assert hip.mid_profitable(m, n, k, reduced) is takes
+    if takes:
+        bm, bn, ksplit = hip.mid_choose(m, n, k, reduced)
+        assert bm >= 128 and ksplit > 1 and bm == (rows or bm)
+
+
 def test_gate_up_at_short_batches():
     assert hip.mid_silu_profitable(1, 28672, 4096) and hip.mid_silu_profitable(256, 57344, 8192)
     assert not hip.mid_silu_profitable(257, 57344, 8192) and not hip.mid_silu_profitable(9, 28672, 2048)

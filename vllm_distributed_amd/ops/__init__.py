@@ -16,7 +16,7 @@ from . import torch_ref
 from .torch_ref import k_cache_shape, v_cache_shape  # noqa: F401  (the paged-cache layouts every backend shares)
 
 # rows up to which a projection may leave fp32 partial sums of a split K to the kernel that follows
-SHORT_BATCH = 512
+SHORT_BATCH = 1280
 
 _hip = None
 _hip_error: Optional[BaseException] = None

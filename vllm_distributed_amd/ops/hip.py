@@ -794,7 +794,7 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
 
 
 # ---------------------------------------- split-K LDS-DMA GEMM, 1 <= M <= 512
-MID_MAX_M = 512
+MID_MAX_M = 1280
 
 
 def mid_supported(x: torch.Tensor, w: torch.Tensor, silu_mul: bool = False) -> bool:
@@ -818,10 +818,12 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
-# TB/s of W that those reach.  Fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
+# TB/s of W that those reach.  The tiles of 192 rows, for 129 to 192, 257 to 384 and 513 to 576: fitted on 92 shapes of 130 to 1280 rows,
+# where the choice is 2.3 % above the fastest in the mean, 12 % at most.  The others fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
 # and every split 8.4 % off in the mean, the chosen tile and split 3.3 % above the fastest in the mean, 40 % at most (8192 x
 # 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model)
-_MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (128, 256): (6.5, 0.89, 256, 5.9),
+_MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (192, 256): (6.8, 0.8, 256, 5.9),
+              (192, 128): (4.0, 0.75, 256, 5.4), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
 # K-split counts the choice is made from (VDAMD_MID_KSPLITS=1,2,4,8,16 restricts it, for A/B measurements)
 _MID_KSPLITS = tuple(int(v) for v in os.environ.get("VDAMD_MID_KSPLITS", "1,2,3,4,5,6,7,8,12,16").split(","))
@@ -853,10 +855,11 @@ def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int, reduced
 @functools.lru_cache(maxsize=4096)
 def mid_choose(m: int, n: int, k: int, reduced: bool = True) -> Tuple[int, int, int]:
     """``(bm, bn, ksplit)`` with the smallest modelled time.  The row tile covers all of M up to 256
-    (W is then read from HBM once); splitting K buys parallelism and costs slab traffic."""
+    (W is then read from HBM once), above that whatever pads the last one least may be the faster (557 rows of 4096 x 14336: 71 us in
+    three tiles of 192, 80 of 256); splitting K buys parallelism and costs slab traffic."""
     best = None
     for (bm, bn) in _MID_TILES:
-        if bm < min(m, 256) or (bm > 64 and bm >= 4 * m):
+        if bm < (min(m, 256) if m <= 256 else 192 if m <= 512 else 128) or (bm > 64 and bm >= 4 * m):
             continue
         # (counts that are not powers of two as well: a 70B qkv projection's 80 column tiles fill 240 of the
         # 256 CUs at 3, 160 at 2)
@@ -883,12 +886,15 @@ def mid_profitable(m: int, n: int, k: int, reduced: bool = True) -> bool:
     16.5 / 17.7; 4608 x 3072 18.3 / 32).  With a reduction of its own (4 to 9 us): 48 rows into K >= 2 N, 128 into squarer
     shapes (from 48 when K >= 8192 and N <= 8192); small W stay with the library (3072 x 2048 at 256 rows 21 / 11).
     Outputs wide enough to fill the chip unsplit: always (an LM head of 128256 x 4096 at 1 / 64 / 256 rows 164 / 200 / 252 us,
-    the library 190 / 222 / 309).  Above 256 rows W is read twice: only where the library's tiles leave the chip idle as well
-    (8192 x 28672 at 384 and 512 rows 183 and 186 us / 203 and 316; 4096 x 14336 52 and 57 / 78 and 88)."""
+    the library 190 / 222 / 309).  Above 256 rows W is read once a row tile: only where the library's tiles leave the chip idle as well,
+    which they do for long reductions (8192 x 28672 at 384 and 512 rows 165 and 199 us / 201 and 313; 4096 x 14336 59 and 67 / 80
+    and 91), and above 512 for fewer than 96 tiles of 256 x 256 (4096 x 14336 at 557, 768, 1024 and 1280 rows 74, 90, 113 and 133 /
+    114, 107, 132 and 147; 3584 x 18944 at 768 102 / 183; 2048 x 8192 at 557 31 / 45; with 96 and more 8192 x 28672 at 557, 640 and
+    900 rows 254, 287 and 357 / 258, 265 and 357, and squarer shapes at 557 32.8 / 36.9, 89 / 93, 101 / 97)."""
     if m <= 0 or m > MID_MAX_M or n < 512 or k < 1024:
         return False
     if m > 256:
-        return k >= 2 * n and n * k >= 12 << 20
+        return k >= 2 * n and n * k >= 12 << 20 and (m <= 512 or -(-m // 256) * -(-n // 256) < 96)
     bm, bn, ksplit = mid_choose(m, n, k, reduced)
     if ksplit == 1:
         return _mid_blocks(m, n, bm, bn, 1) >= 192 and k >= 2048
@@ -914,7 +920,7 @@ def mid_silu_profitable(m: int, n: int, k: int) -> bool:
 def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, ksplit: Optional[int] = None,
              bm: Optional[int] = None, bn: Optional[int] = None, variant: Optional[int] = None,
              partials: bool = False, silu_mul: bool = False, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``x [M<=512, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
+    """``x [M<=1280, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
     fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit).  ``silu_mul``:
     ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  ``bias [N]`` is added to the fp32 sums.  Calls written for
     the kernels before this one keep working: a tile wider than those in ``_MID_TILES`` runs as the widest of its rows, and
