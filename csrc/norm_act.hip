@@ -230,8 +230,10 @@ __global__ void embedding_scalar_kernel(T* __restrict__ out, const int* __restri
   for (int i = threadIdx.x; i < H; i += blockDim.x) dst[i] = ok ? src[i] : (T)0.f;
 }
 
-inline int norm_threads(int H) {
-  int t = ((H >> 3) + NORM_MAX_ITERS - 1) / NORM_MAX_ITERS;   // threads so that 4 iterations cover the row
+// Threads for `passes` passes of 8 values over a row: one of a wide workgroup while the loads' latency is what a launch waits for, more
+// once rows in plenty hide it (each function says from where).
+inline int norm_threads(int H, int passes = NORM_MAX_ITERS) {
+  int t = ((H >> 3) + passes - 1) / passes;
   t = (t + 63) / 64 * 64;
   if (t < 64) t = 64;
   if (t > 1024) t = 1024;
@@ -245,7 +247,9 @@ VDAMD_API int vdamd_rms_norm(void* out, const void* x, void* residual, const voi
                              int H, long x_stride, long out_stride, int dtype, hipStream_t s) {
   if (T == 0) return 0;
   if (H % 8 != 0 || H > 8 * 1024 * NORM_MAX_ITERS) return -1;
-  const int threads = norm_threads(H);
+  // us in 4, 2 and 1 passes, with a residual: 148 rows of 4096 5.7, 5.0, 4.8, of 8192 6.5, 5.6, 5.3; 557 7.6, 7.2, 6.9 and 10.0, 9.8, 9.8;
+  // 800 of 5120 and 8192 9.3, 9.2, 9.4 and 12.2, 11.9, 12.6; 4096 of 5120 34, 33, 32; without one, 8192 of 5120 32, 31, 36
+  const int threads = norm_threads(H, T <= 640 ? 1 : 2);
 #define LAUNCH(TY, ADD)                                                                                   \
   hipLaunchKernelGGL((rms_norm_kernel<TY, ADD>), dim3(T), dim3(threads), 0, s, (TY*)out, (const TY*)x,    \
                      (TY*)residual, (const TY*)w, eps, H, x_stride, out_stride)
@@ -262,11 +266,9 @@ VDAMD_API int vdamd_reduce_add_rms_norm(void* out, const float* partial, int ks,
                                         float eps, int T, int H, long out_stride, int dtype, hipStream_t s) {
   if (T == 0) return 0;
   if (H % 8 != 0 || H > 8 * 1024 * NORM_MAX_ITERS || ks < 1 || residual == nullptr) return -1;
-  int threads = norm_threads(H);
-  if (T <= 64) {               // a few rows: one pass of a wider workgroup, the launch is latency-bound
-    threads = ((H >> 3) + 63) / 64 * 64;
-    if (threads > 1024) threads = 1024;
-  }
+  // us in 4 passes and 1: 67 rows of 4096, 8 slabs, 7.3 and 5.4; 148 rows, 5 slabs, 7.9 and 5.9; 148 of 8192, 7 slabs, 12.0 and 9.9, 256
+  // of it 14.9 and 13.9; 557 of 4096, 5 slabs, 13.0 and 12.4; 557 of 8192, 4 and 7 slabs, 19.5 and 20.3, 32.4 and 33.5
+  const int threads = norm_threads(H, T <= 320 || H <= 4096 ? 1 : NORM_MAX_ITERS);
   const long slab = (long)T * H;
   if (dtype == DT_BF16)
     hipLaunchKernelGGL(reduce_add_rms_norm_kernel<bf16_t>, dim3(T), dim3(threads), 0, s, (bf16_t*)out, partial, ks,

@@ -45,6 +45,26 @@ def test_rms_norm_strided_rows():
                                torch_ref.rms_norm(x.float(), w.float(), 1e-6), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("T,H", [(65, 4096), (320, 8200), (321, 4104), (321, 8200), (640, 2056), (641, 5120), (2, 16392), (641, 32768)])
+def test_norms_in_one_and_in_several_passes(T, H):
+    """Rows at the borders of the workgroups' widths, a last pass of one piece: residuals to a rounding and the slabs' sums in 32 bits,
+    norms to a rounding and the 32-bit sum of squares.  A rounding to bfloat16 (8 significant bits) is at most 2^-8 of the value."""
+    half = torch.finfo(torch.bfloat16).eps / 2
+    w, r = _rand(H, scale=0.3) + 1, _rand(T, H)
+    normed = lambda v: v.double() * torch.rsqrt(v.double().pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    close = lambda got, v: ((got.double() - normed(v)).abs() <= (half + H * 2.0 ** -24) * normed(v).abs() + 1e-9).all()
+    assert close(ops.rms_norm(r, w, 1e-5), r)
+    x, rr = _rand(T, H), r.clone()
+    got, kept = ops.fused_add_rms_norm(x.clone(), rr, w, 1e-5)
+    assert torch.equal(kept, (x.float() + r.float()).to(r.dtype)) and close(got, kept)
+    for ks in (1, 3, 8):
+        slabs, rr = torch.randn(ks, T, H, device=DEV), r.clone()
+        got, kept = ops.reduce_add_rms_norm(slabs, rr, w, 1e-5)
+        want = slabs.double().sum(0) + r.double()
+        assert ((kept.double() - want).abs() <= half * want.abs() + 2 * ks * 2.0 ** -24 * (slabs.abs().sum(0) + r.abs())).all()
+        assert close(got, kept)
+
+
 @pytest.mark.parametrize("T,H", [(3, 768), (64, 4096)])
 def test_layer_norm(T, H):
     x, w, b = _rand(T, H, dtype=torch.float16), _rand(H, dtype=torch.float16) + 1, _rand(H, dtype=torch.float16)
