@@ -818,10 +818,11 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # workgroup tile: us of a launch apart from its K tiles, us of one 64-deep K tile of a workgroup, workgroups that run at once,
-# TB/s of W that those reach.  The tiles of 192 rows, for 129 to 192, 257 to 384 and 513 to 576: fitted on 92 shapes of 130 to 1280 rows,
-# where the choice is 2.3 % above the fastest in the mean, 12 % at most.  The others fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
+# TB/s of W that those reach.  Fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
 # and every split 8.4 % off in the mean, the chosen tile and split 3.3 % above the fastest in the mean, 40 % at most (8192 x
-# 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model)
+# 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model).  Tiles of 192 rows,
+# for 129 to 192, 257 to 384 and 513 to 576: fitted on 92 shapes of 130 to 1280 rows, where the choice is 2.3 % above the fastest in the
+# mean, 12 % at most.
 _MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (192, 256): (6.8, 0.8, 256, 5.9),
               (192, 128): (4.0, 0.75, 256, 5.4), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
