@@ -817,6 +817,27 @@ def test_sample_lists_a_bin_s_entries_wherever_the_logits_lie(base, temperature)
     assert got.tolist() == [order[r - 1].item() for r in ranks]
 
 
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sample_at_temperatures_where_the_lowest_value_weighs(dtype, sign):
+    """Temperatures so high that entries of the type's largest size have weights: each draw at the middle of its entry's stretch, the
+    extremes among the drawn ones and at the top of the row.  (Sums of up to 6000 weights, 2^-24 of each: far below half an entry.)"""
+    V, big, temperature = 6000, torch.finfo(dtype).max, 8e37 * sign
+    g = torch.Generator(DEV).manual_seed(11)
+    for extreme, common in ((-big, 0.0), (0.0, big)):
+        row = torch.full((V,), sign * common, device=DEV, dtype=dtype)
+        row[torch.randperm(V, generator=g, device=DEV)[: V // 2]] = sign * extreme
+        w = torch.exp((row.double() - sign * common) / temperature)
+        w, order = w.sort(descending=True, stable=True)
+        cum = w.cumsum(0)
+        ranks = [1, 17, V // 2, V // 2 + 1, V // 2 + 900, V]
+        n = len(ranks)
+        u = torch.stack([(cum[r - 1] - 0.5 * w[r - 1]) / cum[-1] for r in ranks]).float()
+        full = lambda v, t=torch.float32: torch.full((n,), v, device=DEV, dtype=t)
+        got = ops.sample(row.expand(n, -1).contiguous(), full(temperature), full(0, torch.int32), full(1.0), full(0.0), u)
+        assert got.tolist() == [order[r - 1].item() for r in ranks]
+
+
 def test_sample_of_rows_without_a_distribution_is_entry_zero():
     """Rows of nothing but minus infinity, with a NaN or with an infinity: token 0, no hang, neighbours unharmed."""
     logits = _rand(4, 5000, dtype=torch.float32, scale=2.0)
