@@ -838,6 +838,54 @@ def test_sample_at_temperatures_where_the_lowest_value_weighs(dtype, sign):
         assert got.tolist() == [order[r - 1].item() for r in ranks]
 
 
+def test_sample_draws_an_entry_where_a_sum_of_weights_is_rounded():
+    """A draw that falls a last place (2^-52) behind the sum A of the entries in front, where A and the next entry m add up to an odd
+    multiple of it above 2, halfway between two doubles: A + m - m is A + 2^-52.  Entry m is drawn, nothing masked (entry 0)."""
+    scale, limit = torch.tensor(1.4426950408889634), 1 << 24        # (temperature 1: a weight is 2 to the power of the rounded product)
+    at = {0: 0.0}                                  # the logits whose weights are powers of two
+    for e in range(1, 53):
+        x = torch.tensor(-e / 1.4426950408889634)
+        near = torch.stack([x.view(torch.int32) + d for d in range(-4, 5)]).view(torch.float32)
+        hit = near[near * scale == -float(e)]
+        if len(hit):
+            at[e] = hit[0].item()
+    def powers(units):                             # logits whose weights add up to so many 2^-52, none above 2^-29
+        logits = []
+        for e in (e for e in range(29, 53) if e in at):
+            count, units = divmod(units, 1 << (52 - e))
+            logits += [at[e]] * count
+        return logits if units == 0 else None
+    front, owed = [0.0], 0                         # 1 + 1/2 + .. + 2^-28
+    for e in range(1, 29):
+        owed = 2 * owed + 1
+        if e in at:
+            front, owed = front + [at[e]] * owed, 0
+    assert owed == 0
+    x = -torch.linspace(19.45, 20.05, 60000)
+    units = (torch.exp2((x * scale).to(DEV)).cpu().double() * 2.0 ** 52).long()
+    some = lambda lo, hi, odd: [(int(v), x[i].item()) for i, v in enumerate(units) if lo <= v / 2 ** 23 < hi and v % 2 == odd][:400:7]
+    rows, drawn, uniform = [], [], 1.0 - 3 * 2.0 ** -24
+    *weights, (after, after_x) = some(1.407, 1.421, 1)           # (of one bin, the lightest last)
+    for above, above_x in some(1.5, 1.51, 0):
+        a = (2 << 52) - (1 << 24) + above
+        for m, m_x in weights:
+            mass = 2 * round((a + 1) * limit / (limit - 3) / 2)
+            for total in (mass - 2, mass, mass + 2):
+                rest = powers(total - a - m - after)
+                if rest is not None and (a + m) % 4 == 3 and uniform * (total * 2.0 ** -52) == (a + 1) * 2.0 ** -52:
+                    row = torch.full((300,), float("-inf"))
+                    entries = torch.tensor(front + [above_x, after_x] + rest + [m_x])
+                    row[1:1 + len(entries)] = entries
+                    rows.append(row)
+                    drawn.append(len(entries))
+    rows, drawn = rows[:64], drawn[:64]
+    n = len(rows)
+    assert n >= 16
+    full = lambda v, t=torch.float32: torch.full((n,), v, device=DEV, dtype=t)
+    got = ops.sample(torch.stack(rows).to(DEV), full(1.0), full(0, torch.int32), full(1.0), full(0.0), full(uniform))
+    assert got.tolist() == drawn
+
+
 def test_sample_of_rows_without_a_distribution_is_entry_zero():
     """Rows of nothing but minus infinity, with a NaN or with an infinity: token 0, no hang, neighbours unharmed."""
     logits = _rand(4, 5000, dtype=torch.float32, scale=2.0)
