@@ -167,7 +167,8 @@ def test_latent_attention_takes_the_plan(rows_ok, monkeypatch):
     (100, 80, 3000, False, True), (1, 128, 3000, False, False), (8, 128, 1500, False, False), (8, 64, 4000, False, False),
     (4000, 48, 4000, False, False), (100, 128, 9000, True, True), (64, 128, 9000, True, False), (100, 128, 100, True, False)])
 def test_latent_heads_shared(tokens, heads, keys, captured, shared, monkeypatch):
-    """The rule, and that the kernel over key rows is the one that it turns: not for precise weights, nor where another was asked for."""
+    """The rule, and that it decides where no kernel was asked for, weights precise or not; a kernel that was asked for is the one that
+    runs."""
     import torch
     assert hip.mla_heads_shared(tokens, heads, keys, captured) is shared
     handed = []
@@ -184,9 +185,9 @@ def test_latent_heads_shared(tokens, heads, keys, captured, shared, monkeypatch)
     kc, vc = torch.zeros(4, 1, 32, 320, dtype=torch.bfloat16), torch.zeros(4, 1, 16, 4, 16, 8, dtype=torch.bfloat16)
     row = lambda n: torch.zeros(1, heads, n, dtype=torch.bfloat16).expand(tokens, heads, n)
     q, out, table = row(320), row(256), torch.zeros(tokens, 4, dtype=torch.int32)
-    for mode, precise in ((None, False), (3, False), (3, True), (2, False)):
+    for mode, precise in ((None, False), (None, True), (3, False), (3, True), (4, False), (2, False), (0, False)):
         hip.mla_attention(q, kc, vc, table, None, torch.ones(tokens, dtype=torch.int32), 0.1, keys, out=out, mode=mode, precise=precise)
-        assert handed[-1][1] == (mode if mode == 2 else 4 if shared and not precise else 3)
+        assert handed[-1][1] == (mode if mode is not None else 4 if shared and not precise else 3)
 
 
 @pytest.mark.parametrize("m,n,k,reduced,takes", [

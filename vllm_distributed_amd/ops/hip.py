@@ -1411,7 +1411,7 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     the values read from the key rows (their first ``DV`` values, which is what every writer puts into both caches):
     half the bytes, 1.1 to 4.6 times as fast from one sequence of 32 keys to 256 of 1500 and prompts of 5000, at every width and
     head count measured, so the others are left with what 3 does not read (``mla_rows_ok``); 4 = four head tiles of a token per
-    workgroup over the key rows, which 3 turns into where that is faster (``mla_heads_shared``; weights not ``precise``).
+    workgroup over the key rows, the default where that is faster (``mla_heads_shared``; weights not ``precise``).
     ``precise``: the softmax weights enter the PV product with fp32 precision (a high and a low 16-bit part).
     ``window`` > 0: only the last ``window`` of those keys; ``sinks[Hq]`` (fp32): ``exp(sinks[h])`` joins head ``h``'s
     softmax denominator; ``gate[T, Hq]`` (raw, rows may be strided): the output times its sigmoid."""
@@ -1431,9 +1431,11 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         assert gate.dim() == 2 and gate.shape[0] >= t and gate.shape[1] == hq and gate.stride(1) == 1 and gate.dtype == q.dtype
         gate_stride = gate.stride(0)
     keys = min(max_seq_len, int(window) + 3) if window else max_seq_len
+    asked = mode
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
-    if mode == 3 and not precise and hq > 48 and mla_heads_shared(t, hq, keys, torch.cuda.is_current_stream_capturing()):
+    if (asked is None and mode == 3 and not precise and hq > 48
+            and mla_heads_shared(t, hq, keys, torch.cuda.is_current_stream_capturing())):
         mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], True, 4, keys >= 384)
     # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
     past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
