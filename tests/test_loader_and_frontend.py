@@ -870,3 +870,20 @@ def test_eagle3_head_checkpoint_in_the_authors_layout(tmp_path):
     assert llm.engine.core.scheduler.spec_stats["drafted"] > 0
     ref.shutdown()
     llm.shutdown()
+
+
+def test_environment_is_read_from_whatever_os_environ_is(monkeypatch):
+    """Set, unset and changed variables, in ``os.environ`` itself and in a mapping that takes its place."""
+    import os
+    from vllm_distributed_amd import envs
+    for environ in (os.environ, {}, dict(os.environ)):
+        monkeypatch.setattr(os, "environ", environ)
+        for value, flag in (("1", True), ("off", False), ("yes", True)):
+            monkeypatch.setitem(environ, "VDAMD_TRACE", value)
+            monkeypatch.setitem(environ, "VLLM_SERVER_PORT", "1234")
+            monkeypatch.setitem(environ, "VDAMD_OPS_BACKEND", "torch")
+            assert envs.VDAMD_TRACE is flag and envs.VLLM_SERVER_PORT == 1234 and envs.VDAMD_OPS_BACKEND == "torch"
+        for name in ("VDAMD_TRACE", "VLLM_SERVER_PORT"):
+            monkeypatch.delitem(environ, name)
+        assert envs.VDAMD_TRACE is False and envs.VLLM_SERVER_PORT == 30044
+        monkeypatch.undo()
