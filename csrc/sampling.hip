@@ -308,7 +308,16 @@ template <typename T> struct HeldRow {
       if (e * ST < nvec) f(held[e], e * ST + (int)threadIdx.x, e * ST + (int)threadIdx.x < nvec);
     again(HELD * ST, f);
   }
-  // the same, from memory, from the piece `from` on (a multiple of ST)
+  // the thread's piece of a held round, the same round for all lanes (a branch: picked by conditions it is 64 instructions)
+  __device__ __forceinline__ Vec piece(int round) const {
+    switch (round) {
+#define OF(e) case e: return held[e];
+      OF(0) OF(1) OF(2) OF(3) OF(4) OF(5) OF(6) OF(7) OF(8) OF(9) OF(10) OF(11) OF(12) OF(13) OF(14)
+#undef OF
+      default: return held[15];
+    }
+  }
+  // the same as `each`, from memory, from the piece `from` on (a multiple of ST)
   template <typename F> __device__ __forceinline__ void again(int from, F&& f) const {
 #pragma unroll 1
     for (int i0 = from; i0 < nvec; i0 += ST) {
@@ -367,33 +376,54 @@ __device__ __forceinline__ int sample_by_counts(const T* row, int V, float inv_t
     else if ((x & 0x7fffu) > magnitude + 1) nan = 1;
     else count(x);
   };
-  bool some_odd = false;
-  auto ordinary = [&](Vec v) {
+  auto largest = [&](Vec v) {
     const Pair16 most = __builtin_elementwise_max(
         __builtin_elementwise_max(pair16(v[0] & 0x7fff7fffu), pair16(v[1] & 0x7fff7fffu)),
         __builtin_elementwise_max(pair16(v[2] & 0x7fff7fffu), pair16(v[3] & 0x7fff7fffu)));
-    return max((unsigned)most[0], (unsigned)most[1]) < magnitude;
+    return max((unsigned)most[0], (unsigned)most[1]);
   };
-  data.each([&](Vec v, int, bool live) {
-    const bool plain = ordinary(v);
+  // A piece with elements that are counted apart, or NaN, waits until the plain ones are through: here its round is noted, so that the code
+  // for it is there once.  us, 256 rows of 128256 bf16: half masked at random 49, the last half 37, all but 64 39, nothing 36; read again
+  // from memory and walked element by element 57, 46 and 49, with the code for both kinds in every round 54, 44 and 43 (nothing masked 44)
+  unsigned apart_in = 0;
+  data.each([&](Vec v, int i, bool live) {
+    const bool plain = largest(v) < magnitude;
     if (live && plain) {
 #pragma unroll
       for (int w = 0; w < 4; ++w) { count(v[w] & 0xffffu); count(v[w] >> 16); }
     }
-    some_odd = some_odd || !plain;
+    apart_in |= (__any(!plain) ? 1u : 0u) << min((unsigned)(i - tid) / ST, (unsigned)data.HELD);
   });
-  if (__builtin_expect(__any(some_odd), 0))        // (from memory, once more)
-    data.again(0, [&](Vec v, int, bool live) {
-      if (!live || ordinary(v)) return;
-#pragma unroll 1
-      for (int j = 0; j < 8; ++j) {
-        one(v[0] & 0xffffu);
-        v = Vec{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+  auto apart = [&](Vec v) {
+    const unsigned most = largest(v);
+    if (most < magnitude) return;                  // (a lane without a piece has zeros)
+    const Pair16 l = {1, 1};
+    Pair16 not_low = {0, 0}, not_inf = {0, 0};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      not_low += __builtin_elementwise_min(pair16(v[w] ^ both16(lowest)), l);
+      not_inf += __builtin_elementwise_min(pair16(v[w] ^ both16(lowest + 1)), l);
+    }
+    const unsigned lows = 8u - not_low[0] - not_low[1], infs = 8u - not_inf[0] - not_inf[1];
+    low += lows;
+    inf += infs;
+    if (most > magnitude + 1) nan = 1;             // (whatever else is counted: the row has no distribution)
+    if (lows + infs < 8u)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if (((v[w] & 0xffffu) - lowest) > 1u) count(v[w] & 0xffffu);
+        if (((v[w] >> 16) - lowest) > 1u) count(v[w] >> 16);
       }
-    });
+  };
+#pragma unroll 1
+  for (unsigned rounds = apart_in & ((1u << data.HELD) - 1u); rounds; rounds &= rounds - 1u) apart(data.piece(__builtin_ctz(rounds)));
+  if (apart_in >> data.HELD) data.again(data.HELD * ST, [&](Vec v, int, bool) { apart(v); });
   data.ends([&](unsigned x, int) { one(x); });
-  if (low) atomicAdd(&cs.low, low);
-  if (inf) atomicAdd(&cs.inf, inf);
+  if (__any((low | inf) != 0)) {                   // (one atomic a wave)
+    low = (unsigned)wave_scan((int)low);
+    inf = (unsigned)wave_scan((int)inf);
+    if (lane == 63) { atomicAdd(&cs.low, low); atomicAdd(&cs.inf, inf); }
+  }
   if (nan) s.bad = 1;
   __syncthreads();
   // ---- those that occur, in order, as (place, count) words in the counts' stead: 128 stretches of 512 places, eight a lane,

@@ -796,6 +796,34 @@ def test_sample_holds_rows_of_whole_and_of_cut_rounds(V, offset, dtype):
     assert got[4] == V - 1 and got[5] >= V - 20
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [5003, 131072 + 8 * 1024 + 13])
+@pytest.mark.parametrize("temperature", [0.9, -0.9])
+def test_sample_counts_masked_entries_apart(V, dtype, temperature):
+    """Rows of 16 bits with the two values that masks are made of, alone and mixed, in some pieces of 16 bytes and in all, in those
+    held in registers and behind them, beside the largest value and a NaN: what the same values in 32 bits draw."""
+    sign = 1 if temperature > 0 else -1
+    low, inf = -sign * torch.finfo(dtype).max, -sign * float("inf")
+    g = torch.Generator(DEV).manual_seed(V)
+    x = (torch.randn(9, V, generator=g, device=DEV) * 2.5).to(dtype)
+    part = torch.rand(9, V, generator=g, device=DEV)
+    x[0][part[0] < 0.5], x[1][part[1] < 0.5] = low, inf
+    x[2][part[2] < 0.6], x[2][part[2] < 0.3] = low, inf
+    x[3][part[3] < 0.001] = inf
+    x[4][part[4] < 0.999] = low
+    x[5][V - 4000:] = inf
+    x[6][: V // 2], x[6][V - 1] = low, inf
+    x[7][part[7] < 0.5], x[7][V // 3], x[7][V - 2] = inf, -low, -low
+    x[8][part[8] < 0.5], x[8][V // 2] = low, float("nan")
+    full = lambda v, t=torch.float32: torch.full((9,), v, device=DEV, dtype=t)
+    for top_k, top_p in ((0, 1.0), (0, 0.9), (7, 1.0)):
+        for u in (1e-6, 0.4, 0.95, 1 - 1e-6):
+            rest = (full(temperature), full(top_k, torch.int32), full(top_p), full(0.0), full(u))
+            got = ops.sample(x, *rest)
+            assert torch.equal(got, ops.sample(x.float(), *rest)), (top_k, top_p, u)
+            assert got[8] == 0 and got[7] in (V // 3, V - 2)
+
+
 @pytest.mark.parametrize("base,temperature", [(0.0, 1.0), (100.0, 0.05), (-3000.0, 1.3), (100.0, -0.05), (0.0, 1e-3)])
 def test_sample_lists_a_bin_s_entries_wherever_the_logits_lie(base, temperature):
     """A bin's entries are looked for among the logits near it: logits of one size behind a large common part, small and negative
