@@ -230,14 +230,24 @@ __global__ void embedding_scalar_kernel(T* __restrict__ out, const int* __restri
   for (int i = threadIdx.x; i < H; i += blockDim.x) dst[i] = ok ? src[i] : (T)0.f;
 }
 
-// Threads for `passes` passes of 8 values over a row: one of a wide workgroup while the loads' latency is what a launch waits for, more
-// once rows in plenty hide it (each function says from where).
+// Threads for `passes` passes of 8 values over a row
 inline int norm_threads(int H, int passes = NORM_MAX_ITERS) {
   int t = ((H >> 3) + passes - 1) / passes;
   t = (t + 63) / 64 * 64;
   if (t < 64) t = 64;
   if (t > 1024) t = 1024;
   return t;
+}
+
+// The widest workgroup (one pass, two or four) of which all T run at once, and four passes where none do: a row is bound by its loads'
+// latency, which one pass waits for once, but workgroups that wait for a place on the chip cost more than that.  `simd_waves`: of the
+// kernel, by its registers; a workgroup's waves go to the four SIMDs of a unit in turn
+inline int norm_threads_of_rows(int T, int H, int simd_waves) {
+  for (int passes = 1; passes < NORM_MAX_ITERS; passes *= 2) {
+    const int threads = norm_threads(H, passes);
+    if (T <= 256 * (simd_waves / ((threads / 64 + 3) / 4))) return threads;
+  }
+  return norm_threads(H);
 }
 
 }  // namespace
@@ -247,9 +257,9 @@ VDAMD_API int vdamd_rms_norm(void* out, const void* x, void* residual, const voi
                              int H, long x_stride, long out_stride, int dtype, hipStream_t s) {
   if (T == 0) return 0;
   if (H % 8 != 0 || H > 8 * 1024 * NORM_MAX_ITERS) return -1;
-  // us in 4, 2 and 1 passes, with a residual: 148 rows of 4096 5.7, 5.0, 4.8, of 8192 6.5, 5.6, 5.3; 557 7.6, 7.2, 6.9 and 10.0, 9.8, 9.8;
-  // 800 of 5120 and 8192 9.3, 9.2, 9.4 and 12.2, 11.9, 12.6; 4096 of 5120 34, 33, 32; without one, 8192 of 5120 32, 31, 36
-  const int threads = norm_threads(H, T <= 640 ? 1 : 2);
+  // us in 1, 2 and 4 passes: 512 rows of 5120 4.0, 4.3, 5.0, 576 5.0, 4.6, 5.3; 1024 of 4096 5.0, 5.3, 5.7; 896 of 16384 12.4, 12.4,
+  // 11.5; 8192 of 5120 37, 31, 32; with a residual 320 of 4096 3.7, 4.2, 5.2; 512 of 8192 7.3, 7.5, 7.9; 768 of 16384 21.3, 20.9, 19.4
+  const int threads = norm_threads_of_rows(T, H, 8);
 #define LAUNCH(TY, ADD)                                                                                   \
   hipLaunchKernelGGL((rms_norm_kernel<TY, ADD>), dim3(T), dim3(threads), 0, s, (TY*)out, (const TY*)x,    \
                      (TY*)residual, (const TY*)w, eps, H, x_stride, out_stride)
@@ -266,9 +276,9 @@ VDAMD_API int vdamd_reduce_add_rms_norm(void* out, const float* partial, int ks,
                                         float eps, int T, int H, long out_stride, int dtype, hipStream_t s) {
   if (T == 0) return 0;
   if (H % 8 != 0 || H > 8 * 1024 * NORM_MAX_ITERS || ks < 1 || residual == nullptr) return -1;
-  // us in 4 passes and 1: 67 rows of 4096, 8 slabs, 7.3 and 5.4; 148 rows, 5 slabs, 7.9 and 5.9; 148 of 8192, 7 slabs, 12.0 and 9.9, 256
-  // of it 14.9 and 13.9; 557 of 4096, 5 slabs, 13.0 and 12.4; 557 of 8192, 4 and 7 slabs, 19.5 and 20.3, 32.4 and 33.5
-  const int threads = norm_threads(H, T <= 320 || H <= 4096 ? 1 : NORM_MAX_ITERS);
+  // us in 1, 2 and 4 passes: 256 rows of 8192, two slabs, 6.8, 6.7, 7.4, 288 8.8, 7.7, 8.0, 576 13.9, 12.6, 12.6; 512 of 3072, three,
+  // 6.6, 6.5, 7.1, 576 8.1, 7.2, 7.6; 512 of 4096, two, 6.7, 6.8, 7.5, 576 7.8, 7.5, 8.0; 288 of 7168, five, 11.8, 11.1, 11.1
+  const int threads = norm_threads_of_rows(T, H, 5);
   const long slab = (long)T * H;
   if (dtype == DT_BF16)
     hipLaunchKernelGGL(reduce_add_rms_norm_kernel<bf16_t>, dim3(T), dim3(threads), 0, s, (bf16_t*)out, partial, ks,

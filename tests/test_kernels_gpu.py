@@ -45,7 +45,8 @@ def test_rms_norm_strided_rows():
                                torch_ref.rms_norm(x.float(), w.float(), 1e-6), rtol=2e-2, atol=2e-2)
 
 
-@pytest.mark.parametrize("T,H", [(65, 4096), (320, 8200), (321, 4104), (321, 8200), (640, 2056), (641, 5120), (2, 16392), (641, 32768)])
+@pytest.mark.parametrize("T,H", [(65, 4096), (320, 8200), (321, 4104), (321, 8200), (640, 2056), (641, 5120), (2, 16392), (641, 32768),
+                                 (256, 8192), (257, 8192), (513, 5120), (513, 16384), (577, 3080), (1281, 6144)])
 def test_norms_in_one_and_in_several_passes(T, H):
     """Rows at the borders of the workgroups' widths, a last pass of one piece: residuals to a rounding and the slabs' sums in 32 bits,
     norms to a rounding and the 32-bit sum of squares.  A rounding to bfloat16 (8 significant bits) is at most 2^-8 of the value."""
