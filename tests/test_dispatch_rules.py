@@ -223,6 +223,14 @@ def test_products_of_several_row_tiles(m, n, k, reduced, takes, rows):
         assert bm >= 128 and ksplit > 1 and bm == (rows or bm)
 
 
+@pytest.mark.parametrize("m,n,k,slow", [
+    # us: 158 in tiles of 192 x 128 and 106 in 192 x 256, 154 and 100; in 16 splits and in 12 25.7 and 23.2, 21.0 and 18.7
+    (257, 8192, 16384, (192, 128, 2)), (272, 8192, 16384, (192, 128, 2)), (160, 2048, 12288, (192, 128, 16)),
+    (130, 2048, 8192, (192, 128, 16))])
+def test_tiles_that_are_not_chosen(m, n, k, slow):
+    assert hip.mid_profitable(m, n, k, False) and hip.mid_choose(m, n, k, False) != slow
+
+
 def test_gate_up_at_short_batches():
     assert hip.mid_silu_profitable(1, 28672, 4096) and hip.mid_silu_profitable(256, 57344, 8192)
     assert not hip.mid_silu_profitable(257, 57344, 8192) and not hip.mid_silu_profitable(9, 28672, 2048)

@@ -848,7 +848,14 @@ def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int, reduced
     if rounds + (left > 0) > 1:            # a CU's one workgroup fills and drains its ring in every round
         tile *= 1.25 if bn == 128 and slots == 256 else 1.1
     slabs = ((3.0 if reduced else 0.0) + ksplit * m * n * 4 * 0.4e-6) if ksplit > 1 else 0.0
-    return fixed + k / 64 / ksplit * tile + slabs
+    if bm == 192 and ksplit == 16:         # (2048 x 12288 at 160 rows 25.7 us in 16 splits, 23.2 in 12)
+        slabs += 1.5
+    total = fixed + k / 64 / ksplit * tile + slabs
+    # (K in slices of a multiple of 16 KB, few rows in the last of several tiles: 257 rows of 8192 x 16384 in tiles of 192 x 128 and
+    # halves of K 156 us, 384 rows 112, 257 in tiles of 192 x 256 and quarters 107)
+    if bn == 128 and ksplit > 1 and k // ksplit % 8192 == 0 and m > bm and (m - 1) % bm < bm // 2:
+        total *= 1.4
+    return total
 
 
 # The rules below are functions of whole numbers alone, asked several times for every product of a step that runs outside a
