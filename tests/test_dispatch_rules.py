@@ -215,7 +215,10 @@ def test_short_batch_products(m, n, k, reduced, takes):
     (557, 4096, 14336, False, True, 192), (768, 4096, 14336, True, True, None), (1280, 4096, 14336, False, True, 256),
     (557, 2048, 8192, True, True, None), (300, 4096, 14336, False, True, 192), (300, 8192, 28672, False, True, 192),
     (640, 8192, 28672, False, False, None), (1281, 4096, 14336, False, False, None), (557, 4096, 4096, False, False, None),
-    (557, 10240, 8192, True, False, None)])
+    (557, 10240, 8192, True, False, None),
+    # a small W of K = 2 N: 55 / 62 with a reduction of its own, 62 / 61 (and the norm) without; 62 / 50; 76 / 71
+    (769, 3584, 7168, True, False, None), (769, 3584, 7168, False, True, None), (768, 3584, 7168, True, True, None),
+    (769, 4096, 8192, True, True, None)])
 def test_products_of_several_row_tiles(m, n, k, reduced, takes, rows):
     assert hip.mid_profitable(m, n, k, reduced) is takes
     if takes:

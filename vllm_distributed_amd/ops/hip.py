@@ -898,10 +898,14 @@ def mid_profitable(m: int, n: int, k: int, reduced: bool = True) -> bool:
     which they do for long reductions (8192 x 28672 at 384 and 512 rows 165 and 199 us / 201 and 313; 4096 x 14336 59 and 67 / 80
     and 91), and above 512 for fewer than 96 tiles of 256 x 256 (4096 x 14336 at 557, 768, 1024 and 1280 rows 74, 90, 113 and 133 /
     114, 107, 132 and 147; 3584 x 18944 at 768 102 / 183; 2048 x 8192 at 557 31 / 45; with 96 and more 8192 x 28672 at 557, 640 and
-    900 rows 254, 287 and 357 / 258, 265 and 357, and squarer shapes at 557 32.8 / 36.9, 89 / 93, 101 / 97)."""
+    900 rows 254, 287 and 357 / 258, 265 and 357, and squarer shapes at 557 32.8 / 36.9, 89 / 93, 101 / 97).  A reduction of its own leaves
+    little of that above 768 rows where W is small and K hardly more than 2 N: 3584 x 7168 at 769, 1025 and 1150 rows 62, 74 and 75 / 55, 66
+    and 71, with the next kernel's sums 61, 74 and 77 / 62, 74 and 79; 4096 x 8192 71, 85 and 87 / 76, 86 and 87."""
     if m <= 0 or m > MID_MAX_M or n < 512 or k < 1024:
         return False
     if m > 256:
+        if reduced and m > 768 and 2 * k < 5 * n and n * k < 32 << 20:
+            return False
         return k >= 2 * n and n * k >= 12 << 20 and (m <= 512 or -(-m // 256) * -(-n // 256) < 96)
     bm, bn, ksplit = mid_choose(m, n, k, reduced)
     if ksplit == 1:
