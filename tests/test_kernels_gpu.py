@@ -1471,7 +1471,7 @@ def test_grouped_products_of_experts_at_an_odd_place(tile_rows):
         assert torch.equal(hip.grouped_gemm(x, odd, tiles, tile_rows, **kw), hip.grouped_gemm(x, w, tiles, tile_rows, **kw))
 
 
-@pytest.mark.parametrize("m,n,k", [(3, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192)])
+@pytest.mark.parametrize("m,n,k", [(3, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192), (557, 4096, 14336), (1280, 4096, 14336)])
 def test_linear_writes_any_output_of_a_short_batch(m, n, k):
     """Rows that the short-batch kernels cannot write in place (odd strides and places, columns apart) are the library's.
     Bound: the rounding of the result, and K roundings of the sums."""
@@ -1490,7 +1490,8 @@ def test_linear_writes_any_output_of_a_short_batch(m, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", [(16, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192), (100, 2048, 8192)])
+@pytest.mark.parametrize("m,n,k", [(16, 32000, 4096), (300, 4096, 14336), (128, 8192, 8192), (100, 2048, 8192), (557, 4096, 14336),
+                                   (1280, 4096, 14336)])
 def test_linear_adds_a_bias_before_the_one_rounding(m, n, k, dtype):
     """A bias near the negative of a row's products leaves what a rounding in between would swamp.  Bound: one rounding of the
     result, and K roundings of the sums."""
@@ -1641,7 +1642,8 @@ def test_skinny_gemm_with_silu_mul_operand(m):
     torch.testing.assert_close(a.float(), b.float(), rtol=3e-2, atol=0.3)
 
 
-@pytest.mark.parametrize("m,n,k", [(256, 8192, 8192), (64, 8192, 28672), (1, 8192, 28672), (200, 4096, 14336)])
+@pytest.mark.parametrize("m,n,k", [(256, 8192, 8192), (64, 8192, 28672), (1, 8192, 28672), (200, 4096, 14336), (557, 4096, 14336),
+                                   (1280, 4096, 14336)])
 def test_k_split_partial_sums_reduced_by_the_following_norm(m, n, k):
     """A projection left as fp32 K-split slabs + the kernel that sums them, adds the residual and
     normalises, against the fp32 definition; and against the reduce -> add + norm pair it replaces."""
