@@ -134,6 +134,14 @@ def test_latent_plan(tokens, heads, keys, by_token, seqs, rows_ok, captured, pla
     assert hip.mla_plan(tokens, heads, keys, by_token, seqs, rows_ok, None, captured) == plan
 
 
+@pytest.mark.parametrize("tokens,heads,keys,splits", [
+    # whole / in two, us: 29 / 44, 30 / 49, 60 tokens behind 300 25 / 42, 31 / 43; in two / four 43 / 48; in one / three 42 / 34; 68 / 65
+    (50, 128, 400, 1), (64, 128, 400, 1), (60, 128, 560, 1), (100, 64, 500, 1), (32, 128, 800, 2), (20, 128, 600, 3), (50, 128, 1500, 2),
+    (100, 128, 4000, 1)])
+def test_latent_splits_of_four_tiles_a_workgroup(tokens, heads, keys, splits):
+    assert hip.mla_plan(tokens, heads, keys, False, tokens, True, 4, False) == (4, splits)
+
+
 @pytest.mark.parametrize("rows_ok", [True, False])
 def test_latent_attention_takes_the_plan(rows_ok, monkeypatch):
     """What ``mla_plan`` answers is what the kernels are handed; there is no rule beside it."""

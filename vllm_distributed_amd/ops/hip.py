@@ -1385,7 +1385,9 @@ def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows
     if mode == 3 and wgs > 64:
         shortest = 128 if wgs < 256 else 256
     if mode == 4:
-        shortest = 192
+        # (us of a call, 128 heads: 50 and 64 rows of 400 keys in one split 29 and 30, in two 44 and 49, single tiles 34 and 41; 32 rows of
+        # 800 in two and four 43 and 48; 50 of 1500 in one and two 68 and 65; 20 of 600 in one and three 42 and 34)
+        shortest = 192 if wgs <= 48 else 320
     return mode, max(1, min(per, keys // shortest, 64))
 
 
