@@ -198,6 +198,14 @@ def test_latent_heads_shared(tokens, heads, keys, captured, shared, monkeypatch)
         assert handed[-1][1] == (mode if mode is not None else 4 if shared and not precise else 3)
 
 
+@pytest.mark.parametrize("tokens,heads,keys,prompts,shared", [
+    # single / shared, us: 28 / 33, 47 / 53, 44 / 48, 153 / 159; 61 / 50, 37 / 33, 162 / 134; windows
+    (200, 96, 200, 1, False), (400, 128, 100, 4, False), (300, 80, 300, 1, False), (1165, 80, 512, 5, False), (300, 128, 300, 1, True),
+    (300, 64, 300, 1, True), (700, 80, 700, 1, True), (182, 128, 43, 6, False), (2000, 128, 131, 6, True)])
+def test_latent_heads_shared_by_prompts(tokens, heads, keys, prompts, shared):
+    assert hip.mla_heads_shared(tokens, heads, keys, False, prompts) is shared
+
+
 @pytest.mark.parametrize("m,n,k,reduced,takes", [
     # the next kernel sums the slabs (library / this, us): 8.5 / 5.5, 16.2 / 11.2; a small W at many rows 8.9 / 9.9, 10.2 / 13.3,
     # 17.7 / 16.5; 32 / 18; a router

@@ -1391,7 +1391,7 @@ def mla_plan(tokens: int, heads: int, keys: int, by_token: bool, seqs: int, rows
     return mode, max(1, min(per, keys // shortest, 64))
 
 
-def mla_heads_shared(tokens: int, heads: int, keys: int, captured: bool) -> bool:
+def mla_heads_shared(tokens: int, heads: int, keys: int, captured: bool, prompts: int = 0) -> bool:
     """Whether a step over key rows (``mla_plan``'s 3) goes four tiles of 16 heads a workgroup (4): from 64 heads on, where there is
     work enough.  Such a workgroup needs the time of two single ones for four tiles of a key, and 6 to 8 us more before its first
     product and after its last, so the line is at 160000 (tiles - what the last four leave idle) x rows x keys.  us, single / shared:
@@ -1399,10 +1399,23 @@ def mla_heads_shared(tokens: int, heads: int, keys: int, captured: bool) -> bool
     52 / 39; 64 heads, 12 of 4000 49 / 38, 50 of 1500 78 / 47, 100 of 1500 132 / 67; below the line, 128 heads, one row of 3000 20 / 26,
     8 of 1500 31 / 34, 20 of 600 34 / 36, and 64 heads, 8 of 4000 34 / 37, 20 of 600 25 / 32.
     In a graph ``keys`` is a bound that the lengths may be far below, and a split that is empty still costs its partial sums: only
-    steps whose workgroups fill half of the CUs whole (100 rows of 128 heads, 100 keys: 27 / 22)."""
+    steps whose workgroups fill half of the CUs whole (100 rows of 128 heads, 100 keys: 27 / 22; of 20 keys and fewer 12 / 14, 512 rows
+    42 / 57, which no bound tells).
+    The rows of ``prompts`` sequences see fewer keys than the longest of them: half as many where nothing lies in front, and hardly
+    any in short ones (200 tokens of 96 heads 28 / 33, four prompts of 100 of 128 heads 47 / 53).  80 heads, five tiles in eight
+    places, gain less (300 tokens 44 / 48, and 28 / 34 of 320 values; 700 162 / 134; 130 behind 1000 of 320 values 67 / 70), and
+    several prompts may be shorter than the longest tells (five of 30 to 512 153 / 159, 98 / 106)."""
     q_tiles = -(-heads // 16)
     fours = -(-q_tiles // 4)
-    if q_tiles < 4 or tokens * keys * (2 * q_tiles - 4 * fours) < 160000:
+    least = 160000
+    if prompts > 0:
+        new = tokens / prompts
+        keys = keys - new / 2 if new <= keys else keys           # (more rows than keys: a window)
+        if keys < 100:
+            return False
+        if q_tiles % 4 == 1:
+            least = 300000 if prompts == 1 else 1000000
+    if q_tiles < 4 or tokens * keys * (2 * q_tiles - 4 * fours) < least:
         return False
     return not captured or tokens * fours > 128
 
@@ -1448,7 +1461,8 @@ def mla_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], mla_rows_ok(k_cache, dv), mode,
                           keys >= 384 or keys >= 128 and torch.cuda.is_current_stream_capturing())
     if (asked is None and mode == 3 and not precise and hq > 48
-            and mla_heads_shared(t, hq, keys, torch.cuda.is_current_stream_capturing())):
+            and mla_heads_shared(t, hq, keys, torch.cuda.is_current_stream_capturing(),
+                                 block_table.shape[0] if token_seq is not None else 0)):
         mode, best = mla_plan(t, hq, keys, token_seq is not None, block_table.shape[0], True, 4, keys >= 384)
     # (a bound, in a graph a loose one: the kernel asks the lengths, and which pages several rows share)
     past = max(1, LATENT_ONCE_BYTES) if (mode == 3 and hq <= 16 and token_seq is None
