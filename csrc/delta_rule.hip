@@ -11,7 +11,7 @@
 //                     u = b (v - r), o = p + (k.q) u, S = gS + k u^T.  A lane keeps a part (a 4th, 8th or 16th) of one
 //                     column of S in registers; the parts are summed across lanes; q / k / g / v / b / k.q of a
 //                     chunk of rows are staged in LDS with the next chunk's loads in flight (one barrier per chunk).
-//                     A prompt portion and a few decoded rows are the same kernel in two lane layouts.
+//                     A prompt portion and the decoded rows that come here are the same kernel in two lane layouts.
 //   delta_rule_row    both in one for sequences of a row each: per (sequence, head, tile of 64 or 128 value columns)
 #include "common.h"
 #include <math.h>
@@ -83,8 +83,8 @@ __global__ __launch_bounds__(256) void delta_rule_prep_kernel(float* __restrict_
 // grid (tiles of CB = 4 * 64 / P value columns, H, sequences), 4 waves: wave w owns columns w * 64 / P .. of the tile,
 // a lane keeps R rows of one column of S in registers (P R >= dim; groups of four rows, dealt to the parts in turn).
 // Two lane layouts.
-// Launches of decoded rows are bound by reading and writing the states: P = 4, parts 16 lanes apart, so that a wave
-// reads 64 bytes of a state row at a time.  Prompt portions are bound by the chain of dependent steps per row (the
+// Launches of decoded rows that delta_rule_row does not take (value columns no multiple of 4, states on odd borders) are bound by reading
+// and writing the states: P = 4, parts 16 lanes apart, so that a wave reads 64 bytes of a state row at a time; heads of up to 32 keys too.  Prompt portions are bound by the chain of dependent steps per row (the
 // state cannot be written before r = (gS)^T k is summed over the parts): P = 8 or 16 neighbouring lanes per column,
 // short chains, and the sums stay in the vector unit.  The sequence's rows are walked in chunks of C: q, k, g (all of
 // the head, fp32), v (the tile's columns), b and k.q of a chunk are staged in LDS by the whole workgroup - the next
@@ -410,7 +410,7 @@ VDAMD_API int vdamd_gated_delta_rule(float* out, const void* x, long x_stride, i
   if (B <= 0) return 0;
   if (H <= 0 || G <= 0 || H % G || dim <= 0 || dim > 256 || vdim <= 0) return 1;
   if (parts == 0) {
-    // decoded rows: 4.  Prompt portions: as many parts as still leave every compute unit no more than four workgroups
+    // decoded rows that come here: 4.  Prompt portions: as many parts as still leave every compute unit no more than four workgroups
     // (the chain per row gets shorter with more parts, but the workgroups of a head then read q / k / g more often)
     parts = 4;
     if (max_rows != 1)

@@ -92,8 +92,8 @@ constexpr int BINS1 = 8192, SHIFT1 = 17, BINS = 2048, SHIFT2 = 6, CAP = 4096;
 constexpr unsigned NORMAL_END = 0x40000000u;     // bits of 2.0: weights are at most 1; NaN and infinity lie above
 
 // Weights (positive floats) by the leading bits of their representation: how many, and the sum of the bits below -
-// whole numbers, so any order of additions gives the same.  Up to 2^22 elements both share one 64-bit word (19 low bits
-// times 2^22 stays under 2^41), a single LDS atomic per element; WIDE keeps them apart.
+// whole numbers, so any order of additions gives the same.  Up to 2^22 elements both share one 64-bit word (17 low bits
+// times 2^22 stay under 2^39, the count begins at 2^41), a single LDS atomic per element; WIDE keeps them apart.
 template <bool WIDE, int N> struct Hist {
   unsigned long long sum[N];
   unsigned cnt[WIDE ? N : 1];
@@ -349,8 +349,8 @@ template <typename T> struct HeldRow {
 // lane (2 us) and the waves' totals added up by every wave 39, 29 and 18; by bins, as 32-bit rows are, 79, 36 and 18.  The patterns are
 // packed by stretches of 512 places a wave: with 64 places a thread the few threads that have any were 7 us on their own.
 // -1: a pattern occurs 65536 times or more (a count ran over: the counts' sum is then too small), more than 32768 patterns
-// occur or more than 16384 of the likelier sign, or the row is longer than the second pass has counters for.  The type's lowest value and the infinity next to it, which
-// masks fill rows with, are counted apart, in registers.
+// occur or more than 16384 of the likelier sign, or the row is longer than the second pass has counters for.  The type's lowest value and
+// the infinity next to it, which masks fill rows with, are counted apart, in registers.
 template <typename T>
 __device__ __forceinline__ int sample_by_counts(const T* row, int V, float inv_t, unsigned k, float tp, float mp, float u, unsigned* tab,
                                 SampleShared& s, CountShared& cs, Turn& turn) {

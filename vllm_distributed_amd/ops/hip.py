@@ -793,7 +793,7 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     return out
 
 
-# ---------------------------------------- split-K LDS-DMA GEMM, 1 <= M <= 512
+# ---------------------------------------- split-K LDS-DMA GEMM, 1 <= M <= 1280
 MID_MAX_M = 1280
 
 
@@ -821,8 +821,8 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 # TB/s of W that those reach.  Fitted by least squares; against 4294 timings of 21 weight shapes (8 MB to 2.1 GB) at 1 to 512 rows
 # and every split 8.4 % off in the mean, the chosen tile and split 3.3 % above the fastest in the mean, 40 % at most (8192 x
 # 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model).  Tiles of 192 rows,
-# for 129 to 192, 257 to 384 and 513 to 576: fitted on 92 shapes of 130 to 1280 rows, where the choice is 2.3 % above the fastest in the
-# mean, 12 % at most.
+# for 129 to 192, 257 to 384 and 513 to 576: of the 432 products of 130 to 1280 rows there that this kernel takes, the choice is 1.8 %
+# above the fastest in the mean, 14 % at most.
 _MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (192, 256): (6.8, 0.8, 256, 5.9),
               (192, 128): (4.0, 0.75, 256, 5.4), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
@@ -863,8 +863,8 @@ def _mid_estimate(m: int, n: int, k: int, bm: int, bn: int, ksplit: int, reduced
 @functools.lru_cache(maxsize=4096)
 def mid_choose(m: int, n: int, k: int, reduced: bool = True) -> Tuple[int, int, int]:
     """``(bm, bn, ksplit)`` with the smallest modelled time.  The row tile covers all of M up to 256
-    (W is then read from HBM once), above that whatever pads the last one least may be the faster (557 rows of 4096 x 14336: 71 us in
-    three tiles of 192, 80 of 256); splitting K buys parallelism and costs slab traffic."""
+    (W is then read from HBM once), above that whatever pads the last one least may be the faster (557 rows of 4096 x 14336: 75 us in
+    three tiles of 192, 88 of 256); splitting K buys parallelism and costs slab traffic."""
     best = None
     for (bm, bn) in _MID_TILES:
         if bm < (min(m, 256) if m <= 256 else 192 if m <= 512 else 128) or (bm > 64 and bm >= 4 * m):
@@ -932,7 +932,7 @@ def mid_silu_profitable(m: int, n: int, k: int) -> bool:
 def mid_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, ksplit: Optional[int] = None,
              bm: Optional[int] = None, bn: Optional[int] = None, variant: Optional[int] = None,
              partials: bool = False, silu_mul: bool = False, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``x [M<=1280, K] @ w [N, K]^T`` with W streamed once and K split over the chip.  ``partials``: the
+    """``x [M<=1280, K] @ w [N, K]^T`` with W streamed once a tile of rows and K split over the chip.  ``partials``: the
     fp32 K-split slabs ``[ksplit, M, N]`` instead of their sum (None when the shape runs unsplit).  ``silu_mul``:
     ``w`` is ``[gate ; up]`` and ``silu(gate) * up`` (``N/2`` wide) the result.  ``bias [N]`` is added to the fp32 sums.  Calls written for
     the kernels before this one keep working: a tile wider than those in ``_MID_TILES`` runs as the widest of its rows, and
