@@ -493,7 +493,8 @@ __device__ __forceinline__ int sample_by_counts(const T* row, int V, float inv_t
         if (v[j][w] >> 16) word(at++) = (d + 1u) << 16 | v[j][w] >> 16;
       }
     }
-    __syncthreads();
+    // (the first half's words lie where only its own counts were, which nobody reads any more)
+    if (half == 1) __syncthreads();
   }
   const unsigned lows = cs.low;
   // the row's largest entry (its place: the one in front of all); NaN, and an infinity there, are no distribution
