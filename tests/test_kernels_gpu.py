@@ -172,6 +172,36 @@ def test_rope_and_cache_from_k_split_partial_sums(dtype, kv8, hq, hkv, d, bs, ks
     assert kc0.float().abs().sum().item() > 0 and vc0.float().abs().sum().item() > 0
 
 
+@pytest.mark.parametrize("T", [557, 1280])
+def test_rope_and_cache_of_a_projection_in_several_row_tiles(T):
+    """Query, key and value columns of a tensor-parallel rank above 512 rows: the product leaves slabs, which the rotary + cache kernel adds
+    up.  Bounds: a slab's sums run over K products in 32 bits; queries and caches as from the rounded sums but for turned roundings (of
+    8 significant bits: 2^-8 of an element, and of the two that a rotation mixes)."""
+    hq, hkv, d, k, bs = 16, 2, 128, 8192, 64
+    n, nb = (hq + 2 * hkv) * d, T // bs + 2
+    x, w = _rand(T, k), _rand(n, k, scale=k ** -0.5)
+    slabs = ops.linear_partials(x, w)
+    assert slabs is not None and slabs.shape[0] > 1
+    sums, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert ((slabs.double().sum(0) - sums).abs() <= k * 2.0 ** -24 * size).all()
+    cos_sin = torch_ref.build_cos_sin_cache(d, 4096, 1e6).to(DEV)
+    pos = torch.randint(0, 4096, (T,), device=DEV, dtype=torch.int32)
+    slots = torch.randperm(nb * bs, device=DEV)[:T].to(torch.int32)
+    slots[T - 1] = -1
+    got, want = [], []
+    for out in (got, want):
+        kc = torch.zeros(nb, hkv, bs, d, device=DEV, dtype=x.dtype)
+        vc = torch.zeros(nb, hkv, d // 16, bs // 8, 16, 8, device=DEV, dtype=x.dtype)
+        if out is got:
+            q = ops.rope_and_cache_partials(pos, slabs, x.dtype, cos_sin, kc, vc, slots, hq, hkv, d)
+        else:
+            q = ops.rope_and_cache(pos, slabs.sum(0).to(x.dtype), cos_sin, kc, vc, slots, hq, hkv, d)
+        out += [q.float(), kc.float(), vc.float()]
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=2.0 ** -7, atol=2.0 ** -7 * b.abs().max().item())
+        assert (a == b).float().mean().item() > 0.99 and b.abs().sum().item() > 0
+
+
 def test_rotary_and_reshape_unfused():
     T, hq, hkv, d, bs, nb = 19, 4, 2, 64, 16, 8
     q, k, v = _rand(T, hq * d), _rand(T, hkv * d), _rand(T, hkv * d)
