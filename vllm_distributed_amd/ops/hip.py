@@ -822,7 +822,7 @@ def mid_bias_ok(bias: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
 # and every split 8.4 % off in the mean, the chosen tile and split 3.3 % above the fastest in the mean, 40 % at most (8192 x
 # 1024 at 256 rows and above; profiles/mid_gemm_tiles_mi355x.txt, from benchmarks/stream_gemm_sweep.py --model).  Tiles of 192 rows,
 # for 129 to 192, 257 to 384 and 513 to 576: of the 432 products of 130 to 1280 rows there that this kernel takes, the choice is 1.8 %
-# above the fastest in the mean, 14 % at most.
+# above the fastest in the mean, 15 % at most.
 _MID_TILES = {(256, 256): (7.1, 1.21, 256, 5.9), (256, 128): (5.4, 0.76, 256, 4.8), (192, 256): (6.8, 0.8, 256, 5.9),
               (192, 128): (4.0, 0.75, 256, 5.4), (128, 256): (6.5, 0.89, 256, 5.9),
               (128, 128): (4.4, 0.59, 256, 5.9), (64, 128): (4.0, 0.45, 512, 5.9)}
